@@ -17,7 +17,7 @@
  *     results between calls (it remembers, per device, which kernels were granted
  *     large LDS sizes and where its one static scratch array lives).
  *   - Forward outputs are fully overwritten (no zero-initialisation needed).
- *     Only lffn_scatter_add_f32 / _f16 accumulate into their output.
+ *     Only lffn_scatter_add_f32 / _f16 accumulate into their output (others where a flag asks for it).
  *   - Calls are asynchronous on `stream` (NULL = the legacy default stream) and
  *     may be issued from any host thread.
  *   - Return value: LFFN_OK, or a negative LFFN_ERR_* code.  Nothing throws or
@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 7
+#define LFFN_ABI_VERSION 8
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -607,6 +607,35 @@ int lffn_indexed_inner_product_f32(const int32_t *idx, const float *g, const flo
  */
 int lffn_scatter_add_f32(const int32_t *idx, const float *g, const float *w, float *out,
                          int64_t B, int64_t I, int64_t out_size, int64_t Dv, void *stream);
+
+/*
+ * The three operators with a workspace: the same results, for flat row numbers of any origin, faster.
+ *
+ * gather_add and indexed_inner_product look on the device whether the row numbers are those LookupFFN.gather makes
+ * (PL/lookup.py:120-130: code + i*256 in column i, so I tables of 256 rows and source_size = 256*I), and then run the
+ * table-major kernels of lffn_lookup_gather_* / lffn_lookup_inner_f32, otherwise the token-major ones; no
+ * synchronisation.  The size queries give 0 where only the token-major kernel comes into question, and the calls then
+ * take a null workspace.  row_format: 0 fp32, 1 bfloat16, 2 half rows, as in lffn_lookup_gather_ws_plan.
+ *
+ * lffn_scatter_rows lists the (token, weight) pairs row by row and sums each row in registers instead of
+ * adding products to memory with fp32 atomics.  g_format: 0 fp32, 2 half rows of g; out is fp32 and is
+ * overwritten, or added to with accumulate != 0.  The order of additions within a row varies from run to run.  The
+ * size query gives 0 where lffn_scatter_add_f32 / _f16 are to be used (few products, or few for the rows there are).
+ * workspace: 16-byte aligned, contents irrelevant before and after.
+ */
+int lffn_gather_add_workspace_bytes(int64_t B, int64_t I, int64_t source_size, int64_t Dv, int32_t row_format,
+                                    int64_t *bytes);
+int lffn_gather_add_ws_rows(const int32_t *idx, const void *src, const float *w, float *out, void *workspace,
+                            int64_t workspace_bytes, int64_t B, int64_t I, int64_t source_size, int64_t Dv,
+                            int32_t row_format, void *stream);
+int lffn_indexed_inner_product_workspace_bytes(int64_t B, int64_t I, int64_t source_size, int64_t Dv, int64_t *bytes);
+int lffn_indexed_inner_product_ws_f32(const int32_t *idx, const float *g, const float *src, float *out, void *workspace,
+                                      int64_t workspace_bytes, int64_t B, int64_t I, int64_t source_size, int64_t Dv,
+                                      void *stream);
+int lffn_scatter_rows_workspace_bytes(int64_t B, int64_t I, int64_t out_size, int64_t Dv, int64_t *bytes);
+int lffn_scatter_rows(const int32_t *idx, const void *g, const float *w, float *out, void *workspace,
+                      int64_t workspace_bytes, int64_t B, int64_t I, int64_t out_size, int64_t Dv, int32_t g_format,
+                      int32_t accumulate, void *stream);
 
 /*
  * The two backward operators with half (IEEE binary16) inputs, the rest of the reference's

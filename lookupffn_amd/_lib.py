@@ -15,7 +15,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # LOOKUPFFN_HIP_LIB points at another build of the same ABI (e.g. a tuning build)
 LIB_PATH = os.environ.get("LOOKUPFFN_HIP_LIB") or os.path.join(_PKG_DIR, "liblookupffn_hip.so")
 
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 LFFN_OK = 0
 LFFN_ERR_BAD_ARG = -1
@@ -98,6 +98,12 @@ SIGNATURES = {
     "lffn_lookup_scatter_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64)],
     "lffn_lookup_scatter_sorted_f32": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
     "lffn_lookup_backward_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
+    "lffn_gather_add_workspace_bytes": [_i64, _i64, _i64, _i64, _i32, ctypes.POINTER(_i64)],
+    "lffn_gather_add_ws_rows": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp],
+    "lffn_indexed_inner_product_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)],
+    "lffn_indexed_inner_product_ws_f32": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
+    "lffn_scatter_rows_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)],
+    "lffn_scatter_rows": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _vp],
     "lffn_lookup_inner_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
 }
 

@@ -121,6 +121,7 @@ struct GatherArgs {
     int64_t source_size;  // rows of src / out
     int Dv;
     int S;                // structured: table size (power of two); 0 = flat indices
+    TableGuard guard;
 };
 
 // Stage the block's (index, weight) pairs [i0, i0+IC) in LDS, resolving the row
@@ -156,6 +157,7 @@ __global__ __launch_bounds__(256) void gather_add_kernel(GatherArgs a) {
     constexpr int EPV = Row<FMT>::EPV;
     __shared__ int s_row[TPB][IC];
     __shared__ float s_w[TPB][IC];
+    if (table_guard_ends(a.guard)) return;
 
     const int tl = threadIdx.x / LPT;
     const int ll = threadIdx.x % LPT;
@@ -253,6 +255,7 @@ __global__ __launch_bounds__(256) void inner_product_kernel(GatherArgs a, int ch
     constexpr int TPB = 256 / LPT;
     __shared__ int s_row[TPB][IC];
     __shared__ float s_dot[TPB][IC];
+    if (table_guard_ends(a.guard)) return;
 
     const int tl = threadIdx.x / LPT;
     const int ll = threadIdx.x % LPT;
@@ -367,6 +370,30 @@ Tiling pick_tiling(int nvec) {
     return t;
 }
 
+// flags[w] = does workgroup w see a row number outside table i in column i (I tables of 256 rows)?
+__global__ __launch_bounds__(1024) void table_form_kernel(const int32_t *idx, int32_t *flags, int64_t B, int I) {
+    __shared__ int s_bad[16];
+    const int64_t n = B * I, stride = int64_t(TABLE_FLAGS) * 1024;
+    int bad = 0;
+    int64_t e = int64_t(blockIdx.x) * 1024 + threadIdx.x;
+    int i = (int)(e % I);
+    const int step = (int)(stride % I);
+    for (; e < n; e += stride) {
+        bad |= (idx[e] >> 8) ^ i;
+        i += step;
+        if (i >= I) i -= I;
+    }
+    const unsigned long long m = __ballot(bad != 0);
+    if ((threadIdx.x & 63) == 0) s_bad[threadIdx.x >> 6] = m != 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) any |= s_bad[w];
+        flags[blockIdx.x] = any;
+    }
+}
+
 enum class Op { Gather, Inner, Scatter };
 
 template <int FMT, Op OP, int LPT, int NV>
@@ -419,32 +446,64 @@ int check_common(const void *idx, int64_t B, int64_t I, int64_t rows, int64_t Dv
 template <int FMT>
 int gather_entry(const int32_t *idx, const void *src, const float *w, const float *bias, const float *residual,
                  float *out,
-                 int64_t B, int64_t I, int64_t rows, int64_t Dv, int64_t S, void *stream) {
+                 int64_t B, int64_t I, int64_t rows, int64_t Dv, int64_t S, TableGuard guard, void *stream) {
     int rc = check_common(idx, B, I, rows, Dv);
     if (rc != LFFN_OK) return rc;
     LFFN_REQUIRE(src && out && (w || B * I == 0), LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(lffn_aligned16(src) && lffn_aligned16(out) && (!bias || lffn_aligned16(bias)), LFFN_ERR_BAD_ARG);
     GatherArgs a{};
     a.idx = idx; a.src = src; a.w = w; a.g = nullptr; a.bias = bias; a.residual = residual; a.out = out;
-    a.B = B; a.I = (int)I; a.source_size = rows; a.Dv = (int)Dv; a.S = (int)S;
+    a.B = B; a.I = (int)I; a.source_size = rows; a.Dv = (int)Dv; a.S = (int)S; a.guard = guard;
     return launch<FMT, Op::Gather>(a, static_cast<hipStream_t>(stream));
 }
 
 }  // namespace
 
+static thread_local const int32_t *tls_table_flags = nullptr;
+const int32_t *lffn_internal_table_flags() { return tls_table_flags; }
+void lffn_internal_set_table_flags(const int32_t *flags) { tls_table_flags = flags; }
+
+// Flat row numbers, for arrays that are not in table form when flags are given (not exported).
+int lffn_internal_gather_add_flat(const int32_t *idx, const void *src, const float *w, float *out, int64_t B, int64_t I,
+                                  int64_t source_size, int64_t Dv, int fmt, const int32_t *flags, void *stream) {
+    const TableGuard guard{flags, 0};
+    if (fmt == LFFN_ROWS_F16)
+        return gather_entry<LFFN_ROWS_F16>(idx, src, w, nullptr, nullptr, out, B, I, source_size, Dv, 0, guard, stream);
+    return fmt == LFFN_ROWS_BF16
+               ? gather_entry<LFFN_ROWS_BF16>(idx, src, w, nullptr, nullptr, out, B, I, source_size, Dv, 0, guard, stream)
+               : gather_entry<LFFN_ROWS_F32>(idx, src, w, nullptr, nullptr, out, B, I, source_size, Dv, 0, guard, stream);
+}
+
+int lffn_internal_inner_flat(const int32_t *idx, const float *g, const float *src, float *out, int64_t B, int64_t I,
+                             int64_t source_size, int64_t Dv, const int32_t *flags, void *stream) {
+    int rc = check_common(idx, B, I, source_size, Dv);
+    if (rc != LFFN_OK) return rc;
+    LFFN_REQUIRE(g && src && (out || B * I == 0), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(src) && lffn_aligned16(g), LFFN_ERR_BAD_ARG);
+    GatherArgs a{};
+    a.idx = idx; a.src = src; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
+    a.B = B; a.I = (int)I; a.source_size = source_size; a.Dv = (int)Dv; a.S = 0; a.guard = TableGuard{flags, 0};
+    return launch<LFFN_ROWS_F32, Op::Inner>(a, static_cast<hipStream_t>(stream));
+}
+
+int lffn_internal_table_form(const int32_t *idx, int32_t *flags, int64_t B, int64_t I, void *stream) {
+    hipLaunchKernelGGL(table_form_kernel, dim3(TABLE_FLAGS), dim3(1024), 0, static_cast<hipStream_t>(stream), idx, flags, B, (int)I);
+    return lffn_launch_status();
+}
+
 extern "C" int lffn_gather_add_f32(const int32_t *idx, const float *src, const float *w, float *out,
                                    int64_t B, int64_t I, int64_t source_size, int64_t Dv, void *stream) {
-    return gather_entry<LFFN_ROWS_F32>(idx, src, w, nullptr, nullptr, out, B, I, source_size, Dv, 0, stream);
+    return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, LFFN_ROWS_F32, nullptr, stream);
 }
 
 extern "C" int lffn_gather_add_bf16(const int32_t *idx, const uint16_t *src, const float *w, float *out,
                                     int64_t B, int64_t I, int64_t source_size, int64_t Dv, void *stream) {
-    return gather_entry<LFFN_ROWS_BF16>(idx, src, w, nullptr, nullptr, out, B, I, source_size, Dv, 0, stream);
+    return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, LFFN_ROWS_BF16, nullptr, stream);
 }
 
 extern "C" int lffn_gather_add_f16(const int32_t *idx, const uint16_t *src, const float *w, float *out,
                                    int64_t B, int64_t I, int64_t source_size, int64_t Dv, void *stream) {
-    return gather_entry<LFFN_ROWS_F16>(idx, src, w, nullptr, nullptr, out, B, I, source_size, Dv, 0, stream);
+    return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, LFFN_ROWS_F16, nullptr, stream);
 }
 
 // Token-major kernel on table-local codes (offset i*S and bias folded in): the
@@ -454,9 +513,9 @@ int lffn_internal_lookup_gather_token_major(const int32_t *code, const float *sc
                                             const float *bias, const float *residual, float *out, int64_t B,
                                             int64_t T, int64_t S, int64_t Do, int fmt, void *stream) {
     const int64_t rows = T * S > 0 ? T * S : 1;
-    if (fmt == LFFN_ROWS_F16) return gather_entry<LFFN_ROWS_F16>(code, tables, score, bias, residual, out, B, T, rows, Do, S, stream);
-    return fmt == LFFN_ROWS_BF16 ? gather_entry<LFFN_ROWS_BF16>(code, tables, score, bias, residual, out, B, T, rows, Do, S, stream)
-                                 : gather_entry<LFFN_ROWS_F32>(code, tables, score, bias, residual, out, B, T, rows, Do, S, stream);
+    if (fmt == LFFN_ROWS_F16) return gather_entry<LFFN_ROWS_F16>(code, tables, score, bias, residual, out, B, T, rows, Do, S, lffn_table_guard(), stream);
+    return fmt == LFFN_ROWS_BF16 ? gather_entry<LFFN_ROWS_BF16>(code, tables, score, bias, residual, out, B, T, rows, Do, S, lffn_table_guard(), stream)
+                                 : gather_entry<LFFN_ROWS_F32>(code, tables, score, bias, residual, out, B, T, rows, Do, S, lffn_table_guard(), stream);
 }
 
 // Atomic scatter-add on table-local codes (row = code & (S-1) + t*S), into a buffer
@@ -475,20 +534,13 @@ int lffn_internal_lookup_inner_token_major(const int32_t *code, const float *g, 
                                            void *stream) {
     GatherArgs a{};
     a.idx = code; a.src = tables; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
-    a.B = B; a.I = (int)T; a.source_size = T * S; a.Dv = (int)Do; a.S = (int)S;
+    a.B = B; a.I = (int)T; a.source_size = T * S; a.Dv = (int)Do; a.S = (int)S; a.guard = lffn_table_guard();
     return launch<LFFN_ROWS_F32, Op::Inner>(a, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int lffn_indexed_inner_product_f32(const int32_t *idx, const float *g, const float *src, float *out,
                                               int64_t B, int64_t I, int64_t source_size, int64_t Dv, void *stream) {
-    int rc = check_common(idx, B, I, source_size, Dv);
-    if (rc != LFFN_OK) return rc;
-    LFFN_REQUIRE(g && src && (out || B * I == 0), LFFN_ERR_BAD_ARG);
-    LFFN_REQUIRE(lffn_aligned16(src) && lffn_aligned16(g), LFFN_ERR_BAD_ARG);
-    GatherArgs a{};
-    a.idx = idx; a.src = src; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
-    a.B = B; a.I = (int)I; a.source_size = source_size; a.Dv = (int)Dv; a.S = 0;
-    return launch<LFFN_ROWS_F32, Op::Inner>(a, static_cast<hipStream_t>(stream));
+    return lffn_internal_inner_flat(idx, g, src, out, B, I, source_size, Dv, nullptr, stream);
 }
 
 extern "C" int lffn_scatter_add_f32(const int32_t *idx, const float *g, const float *w, float *out,

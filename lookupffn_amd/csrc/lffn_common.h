@@ -34,6 +34,17 @@ int lffn_internal_lookup_gather_token_major(const int32_t *code, const float *sc
                                             const float *bias, const float *residual, float *out, int64_t B,
                                             int64_t T, int64_t S, int64_t Do, int fmt, void *stream);
 
+// gather.hip: the token-major operators on flat row numbers; with flags (see TableGuard) the launch is for arrays
+// that are not in table form.  table_form writes those flags (TABLE_FLAGS words).
+__attribute__((visibility("hidden")))
+int lffn_internal_gather_add_flat(const int32_t *idx, const void *src, const float *w, float *out, int64_t B, int64_t I,
+                                  int64_t source_size, int64_t Dv, int fmt, const int32_t *flags, void *stream);
+__attribute__((visibility("hidden")))
+int lffn_internal_inner_flat(const int32_t *idx, const float *g, const float *src, float *out, int64_t B, int64_t I,
+                             int64_t source_size, int64_t Dv, const int32_t *flags, void *stream);
+__attribute__((visibility("hidden")))
+int lffn_internal_table_form(const int32_t *idx, int32_t *flags, int64_t B, int64_t I, void *stream);
+
 // gather.hip: atomic scatter-add on table-local codes (not exported)
 __attribute__((visibility("hidden")))
 int lffn_internal_lookup_scatter_atomic(const int32_t *code, const float *score, const float *g, float *out,
@@ -50,6 +61,39 @@ __attribute__((visibility("hidden")))
 int lffn_internal_lookup_gather_pair(const int32_t *code, const float *score, const void *tables,
                                      const float *bias, const float *residual, float *out, int64_t B, int64_t T,
                                      int64_t S, int64_t Do, bool bf16, int np, void *stream);
+
+// Flat row numbers in table form.  weighted_gather_add and its backward take any row numbers, but the layer they come
+// from numbers rows as code + i * 256 in column i of I tables of 256 rows (PL/lookup.py:120-130), and for such numbers
+// the table-major kernels are several times faster than the token-major ones (gather, 4096 x 128 rows of 512 columns:
+// 122 -> 47 us).  Whether an index array has that form is only known on the device, and asking for it on the host would
+// wait for the stream.  So table_form_kernel (gather.hip) leaves one word per workgroup, not zero where a row number is
+// outside its column's table, both forms are launched, and the form that does not apply ends at once: the kernels
+// below take a TableGuard.  (A row number's low 8 bits are then its code: the table-major kernels, which mask
+// the codes they are given, take the index array as it is.)
+constexpr int TABLE_FLAGS = 256;          // words; a wavefront reads them as one 16-byte vector per lane
+struct TableGuard {
+    const int32_t *flags;                 // null: no guard
+    int32_t run_on_tables;                // this launch is for arrays in table form (1) or for the others (0)
+};
+__device__ __forceinline__ bool table_guard_ends(const TableGuard &g) {
+    if (!g.flags) return false;
+    const int4 v = reinterpret_cast<const int4 *>(g.flags)[threadIdx.x & 63];
+    const bool other = __ballot((v.x | v.y | v.z | v.w) != 0) != 0;
+    return other == (g.run_on_tables != 0);
+}
+// The flags under which the calling thread's launches of table-major kernels run (null: no guard): set for the
+// duration of one entry point by TableGuardScope, read where the kernels' arguments are filled in.  (gather.hip; functions,
+// because a thread_local variable shared between the library's objects goes through an initialisation symbol that
+// hidden visibility leaves unresolved.)
+__attribute__((visibility("hidden"))) const int32_t *lffn_internal_table_flags();
+__attribute__((visibility("hidden"))) void lffn_internal_set_table_flags(const int32_t *flags);
+struct TableGuardScope {
+    explicit TableGuardScope(const int32_t *flags) { lffn_internal_set_table_flags(flags); }
+    ~TableGuardScope() { lffn_internal_set_table_flags(nullptr); }
+    TableGuardScope(const TableGuardScope &) = delete;
+    TableGuardScope &operator=(const TableGuardScope &) = delete;
+};
+static inline TableGuard lffn_table_guard() { return TableGuard{lffn_internal_table_flags(), 1}; }
 
 // Dynamic LDS beyond the default limit has to be granted to a kernel once per device
 // (hipFuncAttributeMaxDynamicSharedMemorySize).  `granted` is the caller's record for ONE kernel

@@ -54,6 +54,7 @@ struct LdsGatherArgs {
     // and, when nparts > 1, writes its sums without bias and residual to part_out[p][B][Do].
     int nparts, part_tables;
     float *part_out;
+    TableGuard guard;
 };
 
 // Copy this lane's four vectors of a table slice straight from global memory into
@@ -117,6 +118,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_lds_kernel(LdsGatherArgs a) 
     constexpr int EPV = BF16 ? 8 : 4;
     static_assert(MAX_S * SEG_VECS == 4 * WG, "a lane copies four vectors of a slice");
     extern __shared__ uint4 lds[];                // 2 buffers of S * SEG_VECS vectors
+    if (table_guard_ends(a.guard)) return;
 
     const int xcd = blockIdx.x % XCDS;
     const int unit = xcd * a.per_xcd + blockIdx.x / XCDS;
@@ -318,6 +320,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_lds_kernel(LdsGatherArgs a) 
 
 template <bool BF16, int NP, bool FULL>
 int launch_lds_full(LdsGatherArgs a, hipStream_t stream) {
+    a.guard = lffn_table_guard();
     a.ntiles = (int)((a.B + 64 * NP - 1) / (64 * NP));
     const int units = a.ntiles * a.nslices * a.nparts;
     a.per_xcd = (units + XCDS - 1) / XCDS;
@@ -471,7 +474,9 @@ SplitPlan plan_split(int64_t B, int64_t T, int64_t S, int64_t Do) {
 }
 
 __global__ __launch_bounds__(256) void gather_parts_reduce_kernel(const float *parts, int nparts, const float *bias,
-                                                                  const float *residual, float *out, int64_t B, int Do) {
+                                                                  const float *residual, float *out, int64_t B, int Do,
+                                                                  TableGuard guard) {
+    if (table_guard_ends(guard)) return;
     const int64_t n4 = B * Do / 4;
     const int q = Do / 4;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n4; i += int64_t(gridDim.x) * 256) {
@@ -633,7 +638,7 @@ int lookup_gather_entry(const int32_t *code, const float *score, const void *tab
                 if (rc != LFFN_OK) return rc;
                 const int64_t blocks = (B * Do / 4 + 255) / 256;
                 hipLaunchKernelGGL(gather_parts_reduce_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, st,
-                                   a.part_out, sp.nparts, bias, residual, out, B, (int)Do);
+                                   a.part_out, sp.nparts, bias, residual, out, B, (int)Do, lffn_table_guard());
                 return lffn_launch_status();
             }
         }
@@ -937,4 +942,73 @@ extern "C" int lffn_lookup_gather_records_f32(const uint32_t *records, int64_t r
                                               int64_t S, int64_t Do, int32_t tokens_per_workgroup, void *stream) {
     return lffn_lookup_gather_records_rows(records, record_stride, tables, bias, residual, out, B, T, S, Do, LFFN_ROWS_F32,
                                            tokens_per_workgroup, stream);
+}
+
+namespace {
+
+constexpr int64_t FLAG_BYTES = TABLE_FLAGS * 4;
+
+// Microseconds the table-major forms are predicted to take for 256-row tables with a workspace; 1e300 where the
+// token-major kernel would run.
+double table_major_us(int fmt, int64_t B, int64_t T, int64_t Do) {
+    if (fmt == LFFN_ROWS_F16) {
+        const GatherPlan qp = plan_quad(fmt, B, T, MAX_S, Do);
+        return qp.kind == 3 ? qp.us : 1e300;
+    }
+    const bool bf16 = fmt == LFFN_ROWS_BF16;
+    const GatherPlan qp = bf16 ? choose_quad<true>(B, T, MAX_S, Do) : choose_quad<false>(B, T, MAX_S, Do);
+    if (qp.kind == 3) return qp.us;
+    const int64_t each = bf16 ? gather_pieces<true>(B, T, MAX_S, Do) : gather_pieces<false>(B, T, MAX_S, Do);
+    const GatherPlan plan = bf16 ? plan_gather<true>(each, T, MAX_S, Do) : plan_gather<false>(each, T, MAX_S, Do);
+    if (each < B) return plan.kind ? double((B + each - 1) / each) * (plan.us + 4.0) : 1e300;
+    const SplitPlan sp = bf16 ? plan_split<true>(B, T, MAX_S, Do) : plan_split<false>(B, T, MAX_S, Do);
+    if (sp.nparts > 1 && sp.us < 0.85 * plan.us) return sp.us;
+    return plan.kind ? plan.us : 1e300;
+}
+
+// Row numbers that can be in table form, and a table-major form that pays for looking (4 us for the flags, 4 us for the
+// launches that end at once) with a margin of a fifth for its own prediction.
+bool try_tables(int fmt, int64_t B, int64_t I, int64_t source_size, int64_t Dv) {
+    if (B < 1 || I < 2 || I % 2 != 0 || source_size != I * MAX_S || Dv < 64 || Dv % 64 != 0 || B * I >= (int64_t(1) << 31)) return false;
+    const double token_major_us = double(B) * double(I) * double(Dv) * (fmt == LFFN_ROWS_F32 ? 4 : 2) / 9e6 + 5.0;
+    return table_major_us(fmt, B, I, Dv) + 8.0 < 0.8 * token_major_us;
+}
+
+}  // namespace
+
+extern "C" int lffn_gather_add_workspace_bytes(int64_t B, int64_t I, int64_t source_size, int64_t Dv, int32_t row_format,
+                                               int64_t *bytes) {
+    LFFN_REQUIRE(bytes && row_format >= 0 && row_format <= 2, LFFN_ERR_BAD_ARG);
+    *bytes = 0;
+    if (!try_tables(row_format, B, I, source_size, Dv)) return LFFN_OK;
+    const int rc = lffn_lookup_gather_workspace_bytes(B, I, MAX_S, Dv, row_format, bytes);
+    *bytes += FLAG_BYTES;
+    return rc;
+}
+
+extern "C" int lffn_gather_add_ws_rows(const int32_t *idx, const void *src, const float *w, float *out, void *workspace,
+                                       int64_t workspace_bytes, int64_t B, int64_t I, int64_t source_size, int64_t Dv,
+                                       int32_t row_format, void *stream) {
+    LFFN_REQUIRE(row_format >= 0 && row_format <= 2 && workspace_bytes >= 0 && (workspace || workspace_bytes == 0), LFFN_ERR_BAD_ARG);
+    int64_t need = 0;
+    lffn_gather_add_workspace_bytes(B, I, source_size, Dv, row_format, &need);
+    if (need == 0 || workspace_bytes < need)
+        return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, row_format, nullptr, stream);
+    LFFN_REQUIRE(idx && src && w && out && lffn_aligned16(workspace), LFFN_ERR_BAD_ARG);
+    int32_t *flags = static_cast<int32_t *>(workspace);
+    int rc = lffn_internal_table_form(idx, flags, B, I, stream);
+    if (rc != LFFN_OK) return rc;
+    {
+        TableGuardScope scope(flags);
+        char *ws = need > FLAG_BYTES ? static_cast<char *>(workspace) + FLAG_BYTES : nullptr;
+        const int64_t ws_bytes = need - FLAG_BYTES;
+        if (row_format == LFFN_ROWS_F16)
+            rc = lookup_gather_entry_f16(idx, w, src, nullptr, nullptr, out, B, I, MAX_S, Dv, -1, 0, stream, ws, ws_bytes);
+        else if (row_format == LFFN_ROWS_BF16)
+            rc = lookup_gather_entry<true>(idx, w, src, nullptr, nullptr, out, B, I, MAX_S, Dv, -1, 0, stream, ws, ws_bytes);
+        else
+            rc = lookup_gather_entry<false>(idx, w, src, nullptr, nullptr, out, B, I, MAX_S, Dv, -1, 0, stream, ws, ws_bytes);
+    }
+    if (rc != LFFN_OK) return rc;
+    return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, row_format, flags, stream);
 }

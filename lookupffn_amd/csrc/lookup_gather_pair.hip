@@ -49,6 +49,7 @@ struct PairArgs {
     int ntiles, nslices, per_xcd;
     int row_bytes;         // Do * element size
     int touch;             // 1: with the team touch (decided by the host, see launch_pair)
+    TableGuard guard;
 };
 
 // global_load_lds_dwordx4: lane i of the wavefront writes its 16 bytes at the LDS
@@ -109,6 +110,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_pair_kernel(PairArgs a) {
     constexpr int NQ = WIDE ? (NP + 1) / 2 : (NP + 3) / 4;
     extern __shared__ uint4 lds[];                // 2 buffers of S * ROW_VECS vectors
 
+    if (table_guard_ends(a.guard)) return;
     const int xcd = blockIdx.x % XCDS;
     const int unit = xcd * a.per_xcd + blockIdx.x / XCDS;
     if (unit >= a.ntiles * a.nslices) return;     // uniform over the workgroup
@@ -312,6 +314,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_pair_kernel(PairArgs a) {
 
 template <bool BF16, int NP, bool FULL, bool TOUCH>
 int launch_pair_full(PairArgs a, hipStream_t stream) {
+    a.guard = lffn_table_guard();
     a.ntiles = (int)((a.B + 128 * NP - 1) / (128 * NP));
     const int units = a.ntiles * a.nslices;
     a.per_xcd = (units + XCDS - 1) / XCDS;

@@ -77,6 +77,7 @@ struct QuadArgs {
     int row_bytes;         // Do * bytes per element
     const uint32_t *stream;     // [T/2][Bpad][3] record words written by pack_pairs_kernel
     int64_t Bpad;               // record slots per table pair: every tile's tile_tokens (lffn_internal_quad_record_stride)
+    TableGuard guard;
 };
 
 // global_load_lds_dwordx4 / _dword with a scalar base and a 32-bit lane offset: lane i of the
@@ -130,7 +131,9 @@ __device__ __forceinline__ unsigned with_row(unsigned base, unsigned packed) {
 // contiguous bytes).  Slots of tokens from B on are left as they are: the gather reads them (their row
 // numbers are bytes, always inside the LDS buffer) and does not store their sums.
 __global__ __launch_bounds__(256) void pack_pairs_kernel(const int32_t *code, const float *score, uint32_t *stream,
-                                                         int64_t B, int64_t Bpad, int T, int S, int tile_tokens) {
+                                                         int64_t B, int64_t Bpad, int T, int S, int tile_tokens,
+                                                         TableGuard guard) {
+    if (table_guard_ends(guard)) return;
     __shared__ PairRecord tile[32][64 + 1];
     const int npairs = T / 2;
     const int64_t tok0 = int64_t(blockIdx.x) * 64;
@@ -206,6 +209,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
     const int xcd = blockIdx.x % XCDS;
     const int unit = xcd * a.per_xcd + blockIdx.x / XCDS;
     if (unit >= a.ntiles * a.nslices) return;     // uniform over the workgroup
+    if (table_guard_ends(a.guard)) return;
     const int slice = unit / a.ntiles;
     const int tile = unit % a.ntiles;
 
@@ -440,6 +444,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
 
 template <int FMT, int NP, bool TOUCH>
 int launch_quad(QuadArgs a, hipStream_t stream) {
+    a.guard = lffn_table_guard();
     a.ntiles = (int)((a.B + a.tile_tokens - 1) / a.tile_tokens);
     const int units = a.ntiles * a.nslices;
     a.per_xcd = (units + XCDS - 1) / XCDS;
@@ -537,7 +542,7 @@ int lffn_internal_lookup_gather_quad(const int32_t *code, const float *score, co
     const int64_t stride = lffn_internal_quad_record_stride(B, fmt, tokens);
     const dim3 grid((unsigned)((B + 63) / 64), (unsigned)((T / 2 + 31) / 32));
     hipLaunchKernelGGL(pack_pairs_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), code, score, recs, B,
-                       stride, (int)T, (int)S, tokens);
+                       stride, (int)T, (int)S, tokens, lffn_table_guard());
     if (hipGetLastError() != hipSuccess) return LFFN_ERR_LAUNCH;
     return lffn_internal_lookup_gather_quad_records(recs, stride, tables, bias, residual, out, B, T, S, Do, fmt, tokens, stream);
 }

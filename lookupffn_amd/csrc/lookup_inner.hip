@@ -49,6 +49,7 @@ struct InnerArgs {
     int T, S, Do;
     int ntiles, nslices, per_xcd;
     int row_bytes;
+    TableGuard guard;
 };
 
 // global_load_lds_dwordx4: lane i of the wavefront writes its 16 bytes at the LDS
@@ -90,6 +91,7 @@ __global__ __launch_bounds__(WG) void lookup_inner_lds_kernel(InnerArgs a) {
     static_assert(MAX_S * SEG_VECS == 4 * WG, "a lane copies four vectors of a slice");
     constexpr int NQ = (NP + 3) / 4;              // four 8-bit codes per register
     extern __shared__ uint4 lds[];                // 2 buffers of S * SEG_VECS vectors
+    if (table_guard_ends(a.guard)) return;
 
     const int xcd = blockIdx.x % XCDS;
     const int unit = xcd * a.per_xcd + blockIdx.x / XCDS;
@@ -223,12 +225,14 @@ __global__ __launch_bounds__(WG) void lookup_inner_lds_kernel(InnerArgs a) {
     __builtin_amdgcn_s_waitcnt(0x0F70);         // nothing may still be writing this workgroup's LDS when it ends
 }
 
-__global__ __launch_bounds__(256) void fill_zero_f32_kernel(float *p, int64_t n) {
+__global__ __launch_bounds__(256) void fill_zero_f32_kernel(float *p, int64_t n, TableGuard guard) {
+    if (table_guard_ends(guard)) return;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) p[i] = 0.f;
 }
 
 template <int NP, bool FULL>
 int launch_inner_full(InnerArgs a, hipStream_t stream) {
+    a.guard = lffn_table_guard();
     a.ntiles = (int)((a.B + 64 * NP - 1) / (64 * NP));
     const int units = a.ntiles * a.nslices;
     a.per_xcd = (units + XCDS - 1) / XCDS;
@@ -292,7 +296,7 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
     const int64_t n = B * T;
     const int64_t blocks = (n + 255) / 256;
     hipLaunchKernelGGL(fill_zero_f32_kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, st,
-                       grad_score, n);
+                       grad_score, n, lffn_table_guard());
     int rc = lffn_launch_status();
     if (rc != LFFN_OK) return rc;
 
@@ -316,4 +320,50 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
         case 8: return launch_inner<8>(a, st);
         default: return launch_inner<4>(a, st);
     }
+}
+
+namespace {
+
+// The four-lanes-per-token form for row numbers in table form (256-row tables): its steps (table pair x slice, about
+// 1.3 us each, rounds of 256 workgroups) against the token-major kernel's 9.4 TB/s, with 6 us for the flags and the
+// launch that ends at once and a margin for the prediction.
+bool inner_try_tables(int64_t B, int64_t I, int64_t source_size, int64_t Dv) {
+    if (B < 1 || I < 2 || I % 2 != 0 || source_size != I * MAX_S || Dv < 64 || Dv % 64 != 0 || Dv > (1 << 20) ||
+        B * I >= (int64_t(1) << 31) || 2 * MAX_S * Dv * 4 >= (int64_t(1) << 32))
+        return false;
+    const int64_t tiles = (B + 1023) / 1024, pairs = I / 2;
+    const int c = tiles * ((pairs + 3) / 4) >= 200 ? 4 : (tiles * ((pairs + 1) / 2) >= 96 ? 2 : 0);
+    if (!c) return false;
+    const int64_t rounds = (tiles * ((pairs + c - 1) / c) + 255) / 256;
+    const double us = double(rounds) * double(Dv / 32) * c * 1.3 + 6.0;
+    return us + 6.0 < 0.8 * (double(B) * double(I) * double(Dv) * 4 / 9.4e6);
+}
+
+}  // namespace
+
+extern "C" int lffn_indexed_inner_product_workspace_bytes(int64_t B, int64_t I, int64_t source_size, int64_t Dv,
+                                                          int64_t *bytes) {
+    LFFN_REQUIRE(bytes, LFFN_ERR_BAD_ARG);
+    *bytes = inner_try_tables(B, I, source_size, Dv) ? TABLE_FLAGS * 4 : 0;
+    return LFFN_OK;
+}
+
+extern "C" int lffn_indexed_inner_product_ws_f32(const int32_t *idx, const float *g, const float *src, float *out,
+                                                 void *workspace, int64_t workspace_bytes, int64_t B, int64_t I,
+                                                 int64_t source_size, int64_t Dv, void *stream) {
+    LFFN_REQUIRE(workspace_bytes >= 0 && (workspace || workspace_bytes == 0), LFFN_ERR_BAD_ARG);
+    if (workspace_bytes < TABLE_FLAGS * 4 || !inner_try_tables(B, I, source_size, Dv))
+        return lffn_internal_inner_flat(idx, g, src, out, B, I, source_size, Dv, nullptr, stream);
+    LFFN_REQUIRE(idx && g && src && out && lffn_aligned16(workspace) && lffn_aligned16(src) && lffn_aligned16(g), LFFN_ERR_BAD_ARG);
+    int32_t *flags = static_cast<int32_t *>(workspace);
+    int rc = lffn_internal_table_form(idx, flags, B, I, stream);
+    if (rc != LFFN_OK) return rc;
+    bool taken;
+    {
+        TableGuardScope scope(flags);
+        int rc_quad = LFFN_OK;
+        taken = lffn_internal_lookup_inner_quad_try(idx, g, Dv, 32, src, out, B, I, MAX_S, Dv, stream, &rc_quad);
+        if (taken && rc_quad != LFFN_OK) return rc_quad;
+    }
+    return lffn_internal_inner_flat(idx, g, src, out, B, I, source_size, Dv, taken ? flags : nullptr, stream);
 }

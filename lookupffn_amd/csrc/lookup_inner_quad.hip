@@ -62,6 +62,7 @@ struct InnerQuadArgs {
     int ntiles, nchunks, nslices, per_xcd;
     int group_tiles;       // tiles per tile group (see the unit order in the kernel)
     int row_bytes;         // Do * 4
+    TableGuard guard;
 };
 
 // global_load_lds_dwordx4 with a scalar base and a 32-bit lane offset: lane i of the wavefront writes
@@ -121,6 +122,7 @@ __global__ __launch_bounds__(WG) void lookup_inner_quad_kernel(InnerQuadArgs a) 
     static_assert(C >= 1 && C <= 4, "row numbers of a chunk: two registers per lane");
     constexpr int W = (C + 1) / 2;                // words of row numbers per pass: two pairs (4 bytes) a word
     extern __shared__ uint4 lds[];                // 2 buffers of BUF_BYTES, the touches' sink
+    if (table_guard_ends(a.guard)) return;
 
     const int xcd = blockIdx.x % XCDS;
     const int unit = xcd * a.per_xcd + blockIdx.x / XCDS;
@@ -359,6 +361,7 @@ __global__ __launch_bounds__(WG) void lookup_inner_quad_kernel(InnerQuadArgs a) 
 
 template <int NP, int C>
 int launch_inner_quad(InnerQuadArgs a, hipStream_t stream) {
+    a.guard = lffn_table_guard();
     a.ntiles = (int)((a.B + 256 * NP - 1) / (256 * NP));
     a.nchunks = (a.T / 2 + C - 1) / C;
     // tile groups: with per_xcd units on an XCD, group_tiles tiles and per_xcd / group_tiles chunks meet there;

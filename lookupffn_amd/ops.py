@@ -784,6 +784,23 @@ def _check_gather_args(indexes, rows, vector_dim):
     assert rows >= 1
 
 
+_WORKSPACE_BYTES = {}
+
+
+def _workspace(device, query, *sizes):
+    """A workspace of the size that the library's query asks for (None for 0), from torch's allocator; the answer to a
+    query depends on the sizes alone and is kept."""
+    key = (query, sizes)
+    n = _WORKSPACE_BYTES.get(key)
+    if n is None:
+        nbytes = ctypes.c_int64(0)
+        _lib.check(getattr(_lib.load(), query)(*sizes, ctypes.byref(nbytes)), query)
+        n = nbytes.value
+        if len(_WORKSPACE_BYTES) < 4096:
+            _WORKSPACE_BYTES[key] = n
+    return torch.empty(n, dtype=torch.uint8, device=device) if n > 0 else None
+
+
 _L.define("gather_add(Tensor indexes, Tensor source, Tensor weights) -> Tensor")
 
 
@@ -796,19 +813,15 @@ def _gather_add_impl(indexes, source, weights):
     S, Dv = source.shape
     _check_gather_args(indexes, S, Dv)
     out = torch.empty(B, Dv, dtype=torch.float32, device=source.device)
-    lib = _lib.load()
-    if source.dtype == torch.float32:
-        fn, name = lib.lffn_gather_add_f32, "lffn_gather_add_f32"
-    elif source.dtype == torch.bfloat16:
-        fn, name = lib.lffn_gather_add_bf16, "lffn_gather_add_bf16"
-    elif source.dtype == torch.float16:
-        fn, name = lib.lffn_gather_add_f16, "lffn_gather_add_f16"
-    else:
+    fmt = row_format(source.dtype)
+    if fmt is None:
         raise NotImplementedError(f"gather_add: source dtype {source.dtype} (float32, bfloat16 and float16 rows are built)")
+    ws = _workspace(source.device, "lffn_gather_add_workspace_bytes", B, I, S, Dv, fmt)
     with _dev_guard(source):
-        rc = fn(_lib.ptr(indexes), _lib.ptr(source), _lib.ptr(weights), _lib.ptr(out), B, I, S, Dv,
-                _lib.stream_of(source))
-    _lib.check(rc, f"{name}(B={B}, I={I}, S={S}, Dv={Dv})")
+        rc = _lib.load().lffn_gather_add_ws_rows(_lib.ptr(indexes), _lib.ptr(source), _lib.ptr(weights), _lib.ptr(out),
+                                                 _lib.ptr(ws), 0 if ws is None else ws.numel(), B, I, S, Dv, fmt,
+                                                 _lib.stream_of(source))
+    _lib.check(rc, f"lffn_gather_add_ws_rows(B={B}, I={I}, S={S}, Dv={Dv}, row_format={fmt})")
     return out
 
 
@@ -977,12 +990,17 @@ def _inner_impl(indexes, source_1, source_2):
     _check_gather_args(indexes, S, Dv)
     out = torch.empty(B, I, dtype=torch.float32, device=source_2.device)
     lib = _lib.load()
-    fn, name = ((lib.lffn_indexed_inner_product_f16, "lffn_indexed_inner_product_f16")
-                if source_2.dtype == torch.float16 else
-                (lib.lffn_indexed_inner_product_f32, "lffn_indexed_inner_product_f32"))
     with _dev_guard(source_2):
-        rc = fn(_lib.ptr(indexes), _lib.ptr(source_1), _lib.ptr(source_2), _lib.ptr(out), B, I, S, Dv,
-                _lib.stream_of(source_2))
+        if source_2.dtype == torch.float16:
+            name = "lffn_indexed_inner_product_f16"
+            rc = lib.lffn_indexed_inner_product_f16(_lib.ptr(indexes), _lib.ptr(source_1), _lib.ptr(source_2), _lib.ptr(out),
+                                                    B, I, S, Dv, _lib.stream_of(source_2))
+        else:
+            name = "lffn_indexed_inner_product_ws_f32"
+            ws = _workspace(source_2.device, "lffn_indexed_inner_product_workspace_bytes", B, I, S, Dv)
+            rc = lib.lffn_indexed_inner_product_ws_f32(_lib.ptr(indexes), _lib.ptr(source_1), _lib.ptr(source_2), _lib.ptr(out),
+                                                       _lib.ptr(ws), 0 if ws is None else ws.numel(), B, I, S, Dv,
+                                                       _lib.stream_of(source_2))
     _lib.check(rc, f"{name}(B={B}, I={I}, S={S}, Dv={Dv})")
     return out
 
@@ -1008,8 +1026,16 @@ def _scatter_impl(indexes, source, weights, output_size):
     Dv = source.shape[1]
     assert source.shape[0] == B
     _check_gather_args(indexes, output_size, Dv)
-    out = torch.zeros(output_size, Dv, dtype=torch.float32, device=source.device)
     lib = _lib.load()
+    ws = _workspace(source.device, "lffn_scatter_rows_workspace_bytes", B, I, output_size, Dv)
+    if ws is not None:        # the pairs listed row by row, rows summed in registers: every row is written
+        out = torch.empty(output_size, Dv, dtype=torch.float32, device=source.device)
+        with _dev_guard(source):
+            rc = lib.lffn_scatter_rows(_lib.ptr(indexes), _lib.ptr(source), _lib.ptr(weights), _lib.ptr(out), _lib.ptr(ws),
+                                       ws.numel(), B, I, output_size, Dv, row_format(source.dtype), 0, _lib.stream_of(source))
+        _lib.check(rc, f"lffn_scatter_rows(B={B}, I={I}, out={output_size}, Dv={Dv})")
+        return out
+    out = torch.zeros(output_size, Dv, dtype=torch.float32, device=source.device)
     fn, name = ((lib.lffn_scatter_add_f16, "lffn_scatter_add_f16") if source.dtype == torch.float16 else
                 (lib.lffn_scatter_add_f32, "lffn_scatter_add_f32"))
     with _dev_guard(source):

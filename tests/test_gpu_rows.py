@@ -1,0 +1,112 @@
+"""weighted_gather_add and its backward on flat row numbers at the sizes where the choice of kernels, the row lists or the
+tiles can go wrong, against float64 sums of the same values.
+
+Bounds: an fp32 sum of n products is within n * 2^-24 of the sum of their magnitudes; the comparisons below use that sum
+itself (the operator on absolute values in float64) as the scale of every element."""
+import pytest
+import torch
+
+import lookupffn_amd
+from lookupffn_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _inputs(B, I, rows, Dv, form, dtype=torch.float32, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed + B + I + Dv)
+    if form == "tables":
+        idx = torch.randint(0, 256, (B, I), generator=g, device=DEV, dtype=torch.int32)
+        idx += 256 * torch.arange(I, device=DEV, dtype=torch.int32)[None]
+    elif form == "one row":
+        idx = torch.full((B, I), rows - 1, device=DEV, dtype=torch.int32)
+    else:
+        idx = torch.randint(0, rows, (B, I), generator=g, device=DEV, dtype=torch.int32)
+    if form == "tables but one":
+        idx = torch.randint(0, 256, (B, I), generator=g, device=DEV, dtype=torch.int32)
+        idx += 256 * torch.arange(I, device=DEV, dtype=torch.int32)[None]
+        idx[B - 1, I - 1] = 3
+    src = torch.randn(rows, Dv, generator=g, device=DEV).to(dtype)
+    w = torch.randn(B, I, generator=g, device=DEV).to(dtype)
+    grad = torch.randn(B, Dv, generator=g, device=DEV).to(dtype)
+    return idx, src, w, grad
+
+
+def _reference(idx, src, w, grad):
+    """(out, grad_weights, grad_source) in float64 by columns of the index array."""
+    src, w, grad = src.double(), w.double(), grad.double()
+    out, gw, gs = torch.zeros_like(grad), torch.empty_like(w), torch.zeros_like(src)
+    for i in range(idx.shape[1]):
+        rows = idx[:, i].long()
+        out += w[:, i, None] * src[rows]
+        gw[:, i] = (grad * src[rows]).sum(1)
+        gs.index_add_(0, rows, w[:, i, None] * grad)
+    return out, gw, gs
+
+
+def _close(got, want, scale, terms):
+    # + 2^-23: the result's own rounding
+    assert ((got.double() - want).abs() <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
+
+
+SHAPES = [
+    # (tokens, columns, rows, Dv): table-major forms with ragged tiles, a table split, the smallest sorted lists, rows that
+    # are no multiple of 256, more tokens than one chunk, a single 64-column slice pair
+    (4096, 128, 128 * 256, 512), (2103, 64, 64 * 256, 768), (1031, 32, 32 * 256, 1024), (4099, 130, 130 * 256, 64),
+    (257, 126, 1000, 192), (100, 8, 77, 8192), (16500, 8, 8 * 256, 128), (1, 6, 24, 1 << 20), (513, 62, 62 * 256, 320),
+]
+
+
+@pytest.mark.parametrize("form", ["tables", "any", "tables but one", "one row"])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_weighted_gather_add_and_gradients(shape, form):
+    B, I, rows, Dv = shape
+    if form.startswith("tables") and rows != 256 * I:
+        pytest.skip("not tables of 256 rows")
+    idx, src, w, grad = _inputs(B, I, rows, Dv, form)
+    src.requires_grad_(), w.requires_grad_()
+    out = lookupffn_amd.weighted_gather_add(idx, src, w)
+    out.backward(grad)
+    want = _reference(idx, src.detach(), w.detach(), grad)
+    scale = _reference(idx, src.detach().abs(), w.detach().abs(), grad.abs())
+    counts = torch.bincount(idx.reshape(-1), minlength=rows).max().item()
+    for got, x, s, terms in zip((out.detach(), w.grad, src.grad), want, scale, (I, Dv, counts)):
+        _close(got, x, s, terms)
+
+
+@pytest.mark.parametrize("shape", [(4096, 128, 128 * 256, 512), (100, 8, 77, 8192), (3000, 62, 62 * 256, 192)], ids=str)
+@pytest.mark.parametrize("form", ["tables", "any"])
+def test_half_rows_and_gradients(shape, form):
+    B, I, rows, Dv = shape
+    if form == "tables" and rows != 256 * I:
+        pytest.skip("not tables of 256 rows")
+    idx, src, w, grad = _inputs(B, I, rows, Dv, form, torch.float16)
+    src.requires_grad_(), w.requires_grad_()
+    out = lookupffn_amd.weighted_gather_add(idx, src, w)
+    out.backward(grad)
+    want = _reference(idx, src.detach(), w.detach(), grad)
+    scale = _reference(idx, src.detach().abs(), w.detach().abs(), grad.abs())
+    counts = torch.bincount(idx.reshape(-1), minlength=rows).max().item()
+    for got, x, s, terms in zip((out.detach(), w.grad, src.grad), want, scale, (I, Dv, counts)):
+        assert got.dtype == torch.float16
+        # fp32 sums, then one rounding to half (2^-11 of the value, 2^-25 below the normal range)
+        assert ((got.double() - x).abs() <= s * terms * 2.0 ** -24 + x.abs() * 2.0 ** -10.9 + 2.0 ** -24).all()
+
+
+def test_scatter_rows_accumulates_and_clamps():
+    B, I, rows, Dv = 700, 64, 300, 256
+    idx, _, w, grad = _inputs(B, I, rows, Dv, "any")
+    idx[3, 5], idx[4, 6] = -7, rows + 1000          # clamped into range, as every operator does
+    start = torch.randn(rows, Dv, device=DEV)
+    out = start.clone()
+    lib = _lib.load()
+    ws = ops._workspace(out.device, "lffn_scatter_rows_workspace_bytes", B, I, rows, Dv)
+    assert ws is not None
+    rc = lib.lffn_scatter_rows(idx.data_ptr(), grad.data_ptr(), w.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), B, I, rows,
+                               Dv, 0, 1, _lib.stream_of(out))
+    assert rc == 0
+    clamped = idx.clamp(0, rows - 1)
+    src = torch.zeros(rows, Dv, device=DEV)
+    want = _reference(clamped, src, w, grad)[2] + start.double()
+    scale = _reference(clamped, src, w.abs(), grad.abs())[2] + start.abs().double()
+    _close(out, want, scale, torch.bincount(clamped.reshape(-1)).max().item() + 1)
