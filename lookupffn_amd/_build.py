@@ -1,7 +1,8 @@
-"""Builds liblookupffn_hip.so (the C-ABI kernel library) for gfx950 with hipcc.
+"""Builds liblookupffn_hip.so (the C-ABI kernel library) for gfx950 with hipcc, and _host.so (the layer's host path in C++,
+csrc/host.cpp, against the installed torch) with g++.
 
 Run as ``python -m lookupffn_amd._build``.  hipcc cross-compiles, so no GPU is
-needed.  The library lands next to this file so that it is found in-tree.
+needed.  Both land next to this file so that they are found in-tree.
 """
 from __future__ import annotations
 
@@ -9,12 +10,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "liblookupffn_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 SOURCES = ["fht.hip", "code_score.hip", "gather.hip", "lookup_gather.hip", "lookup_gather_pair.hip", "lookup_gather_quad.hip", "lookup_scatter.hip", "lookup_scatter_sorted.hip", "lookup_inner.hip", "lookup_inner_quad.hip", "bh4_block.hip", "bh4_wgrad.hip", "layer_norm.hip"]
 
 HIPCC_FLAGS = [
@@ -34,6 +37,22 @@ def _hipcc() -> str:
     if not os.path.exists(exe):
         raise RuntimeError("hipcc not found: the kernel library can only be built in a ROCm image")
     return exe
+
+
+def _build_host() -> None:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    tmp = HOST_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *[a for d in includes for a in ("-isystem", d)], os.path.join(CSRC, "host.cpp"), "-o", tmp,
+           "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{res.stderr[-8000:]}")
+    os.replace(tmp, HOST_PATH)
 
 
 def build_library(verbose: bool = False) -> str:
@@ -56,8 +75,10 @@ def build_library(verbose: bool = False) -> str:
             print(err, file=sys.stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=5) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(compile_one, srcs))
+        host.result()
     tmp = LIB_PATH + ".tmp"
     res = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp],
                          capture_output=True, text=True)

@@ -155,6 +155,29 @@ def load() -> ctypes.CDLL:
         return _lib
 
 
+_host = None
+
+
+def host():
+    """The layer's host path (csrc/host.cpp, built next to the kernel library), bound to the loaded kernel library; raise
+    if it is absent."""
+    global _host
+    if _host is None:
+        load()
+        with _lock:
+            if _host is None:
+                path = os.path.join(_PKG_DIR, "_host.so")
+                if not os.path.exists(path):
+                    raise LookupFFNLibraryError(f"{path} is missing: build it with `python -m lookupffn_amd._build`")
+                try:
+                    from . import _host as module
+                except ImportError as e:
+                    raise LookupFFNLibraryError(f"cannot load {path}: {e}") from e
+                module.bind_library(LIB_PATH)
+                _host = module
+    return _host
+
+
 def exported_symbols():
     return ["lffn_version", "lffn_error_string", *SIGNATURES.keys()]
 

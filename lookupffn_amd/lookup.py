@@ -3,10 +3,9 @@ PL/lookup.py (PL/ = src/roberta/models/prenorm_lookup/), with the same
 constructor arguments, ``config`` attribute names, parameter names and shapes
 (so a reference state_dict loads unchanged), on the gfx950 kernels.
 
-Inference (no gradient needed) with ``block_size == 1`` and 8-bit codes runs as
-LayerNorm -> one fused projection+hash kernel -> one gather kernel.  Every other
-case runs the same operator sequence as the reference, each operator on its
-kernel and differentiable.
+A LookupFFN call on fp32 tokens with 8-bit codes and diagonal or 64 x 64 blocks, with or without
+gradient, goes through the host path in csrc/host.cpp.  Every other case runs the same operator
+sequence as the reference, each operator on its kernel and differentiable.
 """
 from __future__ import annotations
 
@@ -17,7 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import ops
+from . import _lib, ops
 from .bh4 import bh4
 from .compute_code_score import compute_code_score
 from .gather import gather, lookup_gather
@@ -373,6 +372,8 @@ class LookupFFN(nn.Module):
         state = super().__getstate__() if hasattr(super(), "__getstate__") else self.__dict__.copy()
         state = dict(state)
         state.pop("_inference_cache", None)
+        state.pop("_handle", None)
+        state.pop("_handle_key", None)
         return state
 
     def extra_repr(self):
@@ -435,52 +436,48 @@ class LookupFFN(nn.Module):
                       if form == "diag" else None),
                 pbias=None if p.bias is None else p.bias.detach(), tables=self.tables.detach(),
                 obias=self.bias.detach(), decay=float(p.decay_coeff), res_coef=float(1 - p.decay_coeff))
-            if state["one_launch"]:
-                state["block"] = ops.fused_layer_block(state["ln_w"], state["ln_b"], state["eps"], state["diag"], state["pbias"],
-                                                       state["tables"], state["obias"], state["decay"], state["res_coef"])
         self._inference_cache = (key, state)
         return state
 
-    def _forward_inference(self, x, residual, st):
-        """No gradient wanted and parameters the inference kernels are built for: the entry points
-        are called without the operator dispatcher or autograd (same kernels, same results)."""
-        x = x.contiguous()
-        if residual is not None:
-            # forward() hands over fp32 of shape [tokens, output_size]; anything else is a caller's mistake
-            if (residual.dtype != torch.float32 or residual.device != x.device
-                    or tuple(residual.shape) != (x.shape[0], self.output_size)):
-                raise ValueError("residual: fp32 [tokens, output_size] on the input's device")
-            residual = residual.contiguous()
-        if st["one_launch"] and x.shape[0] <= self.FUSED_LAYER_MAX_TOKENS:
-            # small batches: the whole layer in one launch
-            return ops.lookup_ffn_fused_block(st["block"], x, residual)
-        if self.num_table % 2 == 0:
-            # many tokens: the projection kernel writes the gather kernel's record stream directly
-            plan = ops.lookup_gather_records_plan(x.shape[0], self.num_table, self.table_size, self.output_size,
-                                                  ops.row_format(st["tables"].dtype))
-            records = None
-            if plan is not None and st["form"] == "diag" and st["diag"].shape[2] >= 16:
-                records = ops.ln_project_hash_records_direct(x, st["ln_w"], st["ln_b"], st["eps"], st["diag"], st["pbias"],
-                                                             self.num_table, st["decay"], st["res_coef"], plan)
-            elif plan is not None and st["form"] == "block":
-                records = ops.ln_bh4_block_hash_records_direct(x, st["ln_w"], st["ln_b"], st["eps"], self.hash.folded_weight(),
-                                                               st["pbias"], self.num_table, st["decay"], st["res_coef"], plan)
-            if records is not None:
-                return ops.lookup_gather_records_direct(records, plan, st["tables"], st["obias"], residual, x.shape[0])
-        if st["form"] == "diag":
-            code, score, _ = ops.ln_project_hash_direct(x, st["ln_w"], st["ln_b"], st["eps"], st["diag"], st["pbias"],
-                                                        self.num_table, st["decay"], st["res_coef"], False)
-        else:
-            code, score = ops.ln_bh4_block_hash_direct(x, st["ln_w"], st["ln_b"], st["eps"], self.hash.folded_weight(),
-                                                       st["pbias"], self.num_table, st["decay"], st["res_coef"])
-        return ops.lookup_gather_direct(code, score, st["tables"], st["obias"], residual)
+    def _forward_host(self, x, residual):
+        """The layer through the host path (csrc/host.cpp), or None when the call or the parameters are not of a kind it is
+        built for.  Its handle holds for as long as the parameters it names are the layer's, with the storage and dtype
+        they had (and, without gradient, the folded 64 x 64 blocks the weights they were folded from)."""
+        if not (x.is_cuda and x.dtype == torch.float32 and self.tables.is_cuda):
+            return None
+        st = self._inference_state()
+        if st is None:
+            return None
+        fold = st["form"] == "block" and self._no_gradient_wanted(x)
+        if fold:
+            self.hash.folded_weight()
+        key = (st, self.hash._folded if fold else None)
+        known = self.__dict__.get("_handle_key")
+        if known is None or known[0] is not st or (fold and known[1] is not key[1]):
+            self._handle, self._handle_key = self._make_handle(st, key[1]), key
+        return _lib.host().forward(self._handle, x.contiguous(), None if residual is None else residual.contiguous(),
+                                   self.FUSED_LAYER_MAX_TOKENS)
+
+    def _make_handle(self, st, folded):
+        ln, p = self.LayerNorm, self.hash.projection
+        block = st["form"] == "block"
+        R, J, D = p.num_repeat, p.weight.shape[1], p.padded_in_dim
+        trainable = (self.tables.dtype == torch.float32 and self.hidden_size % 4 == 0 and self.hidden_size <= 1024
+                     and (block or (256 <= D and J <= 4)))
+        watched = ((ln._parameters, "weight"), (ln._parameters, "bias"), (p._parameters, "weight"), (p._parameters, "bias"),
+                   (self._parameters, "tables"), (self._parameters, "bias"))
+        return _lib.host().make_layer(
+            (int(block), int(st["one_launch"]), self.hidden_size, D, R, J, self.num_table, self.table_size, self.output_size,
+             ops.row_format(self.tables.dtype), ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS, ops.PROJECT_BWD_PARTIALS,
+             ops.COLUMN_SUM_CHUNK_ROWS, int(trainable)),
+            (st["eps"], st["decay"], st["res_coef"]), watched,
+            None if folded is None else (self.hash.__dict__, "_folded", folded, folded[1], p.weight._version))
 
     def _forward(self, hidden_states, residual=None):
-        if (hidden_states.is_cuda and hidden_states.dtype == torch.float32 and not torch.compiler.is_compiling()
-                and self._no_gradient_wanted(hidden_states)):
-            st = self._inference_state()
-            if st is not None:
-                return self._forward_inference(hidden_states, residual, st)
+        if not torch.compiler.is_compiling():
+            out = self._forward_host(hidden_states, residual)
+            if out is not None:
+                return out
         ln = self.LayerNorm
         ln_fusable = (ln.elementwise_affine and ln.weight is not None and ln.bias is not None
                       and ln.weight.dtype == torch.float32
@@ -521,10 +518,13 @@ class LookupFFN(nn.Module):
     def forward(self, hidden_states, residual=None):
         """PL/lookup.py:110-118.  ``residual`` (not in the reference; shape [..., output_size]) is
         added to the result inside the gather kernel: the encoder layer's "FFN(x) + x"."""
-        if hidden_states.dim() == 2 and residual is None:
-            # already [tokens, hidden]: nothing to reshape (at a few hundred tokens the layer is one launch of
-            # a few microseconds and every view made here shows in its time)
-            return self._forward(hidden_states, None)
+        handle = self.__dict__.get("_handle")
+        if handle is not None and not torch.compiler.is_compiling():
+            # (before anything else: at a few hundred tokens the layer is one launch of a few microseconds, and every view
+            # made here shows in its time)
+            out = _lib.host().forward(handle, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS)
+            if out is not None:
+                return out
         shape = hidden_states.shape[:-1]
         dim = hidden_states.shape[-1]
         tokens = math.prod(shape)

@@ -456,73 +456,6 @@ def _lookup_ffn_fused_impl(x, ln_w, ln_b, eps, diag, pbias, tables, obias, resid
 _L.impl("lookup_ffn_fused", _lookup_ffn_fused_impl, "CUDA")
 
 
-# The inference path of the layer calls the implementations below directly: outside torch.compile
-# the dispatcher adds nothing but a few microseconds per call, which is the larger part of a step
-# at small batches.
-def ln_project_hash_direct(*args):
-    return _ln_project_hash_impl(*args)
-
-
-def ln_bh4_block_hash_direct(*args):
-    return _ln_bh4_block_hash_impl(*args)
-
-
-def lookup_gather_direct(*args):
-    return _lookup_gather_impl(*args)
-
-
-def lookup_ffn_fused_direct(x, ln_w, ln_b, eps, diag, pbias, tables, obias, residual, decay, residual_coef):
-    """lookup_ffn_fused for a caller that has already checked the parameters (LookupFFN caches that):
-    no dispatcher, no per-call checks beyond x itself.  The layer's launch is a few microseconds, so
-    at small batches the host side of a call is most of its time."""
-    if torch.compiler.is_compiling():
-        return torch.ops.lookupffn.lookup_ffn_fused(x, ln_w, ln_b, eps, diag, pbias, tables, obias, residual,
-                                                    decay, residual_coef)
-    assert x.dtype == torch.float32 and x.is_cuda and x.is_contiguous() and x.device == tables.device
-    B, H = x.shape
-    R, J, D = diag.shape
-    T, S, Do = tables.shape
-    assert H == ln_w.numel() and (residual is None or (residual.dtype == torch.float32 and residual.is_contiguous()
-                                                        and tuple(residual.shape) == (B, Do)))
-    out = torch.empty((B, Do), dtype=torch.float32, device=x.device)
-    with _dev_guard(x):
-        rc = _lib.load().lffn_lookup_ffn_fused_f32(
-            x.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), eps, diag.data_ptr(),
-            None if pbias is None else pbias.data_ptr(), tables.data_ptr(),
-            None if obias is None else obias.data_ptr(), None if residual is None else residual.data_ptr(),
-            out.data_ptr(), B, H, D, R, J, T, S, Do, decay, residual_coef, _lib.stream_of(x))
-    if rc != 0:
-        _lib.check(rc, f"lffn_lookup_ffn_fused_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T}, S={S}, Do={Do})")
-    return out
-
-
-def fused_layer_block(ln_w, ln_b, eps, diag, pbias, tables, obias, decay, residual_coef):
-    """The parameter block of lffn_lookup_ffn_fused_layer_f32 for a set of (checked, contiguous, fp32, same-device)
-    parameters, with the entry point and a byref to the block: what lookup_ffn_fused_block takes.  The tensors
-    must outlive the block (LookupFFN keeps both in one cache entry)."""
-    R, J, D = diag.shape
-    T, S, Do = tables.shape
-    blk = _lib.FusedLayer(ln_w.data_ptr(), ln_b.data_ptr(), diag.data_ptr(), None if pbias is None else pbias.data_ptr(),
-                          tables.data_ptr(), None if obias is None else obias.data_ptr(), ln_w.numel(), D, R, J, T, S, Do,
-                          eps, decay, residual_coef)
-    return (_lib.load().lffn_lookup_ffn_fused_layer_f32, ctypes.byref(blk), blk, ln_w.numel(), Do, tables.device)
-
-
-def lookup_ffn_fused_block(block, x, residual):
-    """lookup_ffn_fused_direct through the parameter block: six arguments cross the foreign-function interface
-    instead of twenty-one."""
-    fn, ref, _keep, H, Do, device = block
-    if x.dtype != torch.float32 or x.dim() != 2 or x.shape[1] != H or x.device != device or not x.is_contiguous():
-        raise ValueError("x: contiguous fp32 [B, H] on the parameters' device")
-    B = x.shape[0]
-    out = torch.empty((B, Do), dtype=torch.float32, device=device)
-    with _dev_guard(x):
-        rc = fn(ref, x.data_ptr(), None if residual is None else residual.data_ptr(), out.data_ptr(), B, _lib.stream_of(x))
-    if rc != 0:
-        _lib.check(rc, f"lffn_lookup_ffn_fused_layer_f32(B={B}, H={H}, Do={Do})")
-    return out
-
-
 @torch.library.register_fake("lookupffn::lookup_ffn_fused")
 def _(x, ln_w, ln_b, eps, diag, pbias, tables, obias, residual, decay, residual_coef):
     return x.new_empty(x.shape[0], tables.shape[2])
