@@ -282,6 +282,10 @@ typedef struct lffn_fused_layer {
 } lffn_fused_layer;
 int lffn_lookup_ffn_fused_layer_f32(const lffn_fused_layer *layer, const float *x, const float *residual_in,
                                     float *out, int64_t B, void *stream);
+/* The same for rows in any format (row_format 0: fp32, 1: bfloat16, 2: half; layer->tables points to rows of
+ * that format): products and sums in fp32. */
+int lffn_lookup_ffn_fused_layer_rows(const lffn_fused_layer *layer, int32_t row_format, const float *x,
+                                     const float *residual_in, float *out, int64_t B, void *stream);
 
 /*
  * Weight gradient of the BH4 module with 64 x 64 blocks, all stages in one launch, in the

@@ -115,6 +115,7 @@ class FusedLayer(ctypes.Structure):
 
 
 SIGNATURES["lffn_lookup_ffn_fused_layer_f32"] = [ctypes.POINTER(FusedLayer), _vp, _vp, _vp, _i64, _vp]
+SIGNATURES["lffn_lookup_ffn_fused_layer_rows"] = [ctypes.POINTER(FusedLayer), ctypes.c_int32, _vp, _vp, _vp, _i64, _vp]
 
 _lib = None
 _lock = threading.Lock()

@@ -21,6 +21,7 @@
 // (fast_hadamard_transform/extension/cuda_kernel.cu:235-251), so results agree
 // bit for bit with a scalar butterfly in that order.
 #include "lffn_common.h"
+#include "token_gather.h"
 
 #include <type_traits>
 
@@ -257,16 +258,7 @@ struct ProjectArgs {
     int mix;              // 1: out = decay*y + residual*x (+ bias); 0: out = y
     int vec_in;           // x rows are 16-byte aligned and H % 4 == 0
     int vec_ln;           // and so are ln_w and ln_b: the LayerNorm parameters load as float4
-    // GATHER only: the table rows the codes select are added up in the same kernel
-    const float *tables;  // [T, S, Do]
-    const float *obias;   // [Do] or null
-    const float *gres;    // [B, Do] or null: added to the result
-    float *gout;          // [B, Do]
-    int S, Do;
 };
-
-constexpr int FUSED_MAX_T = 512;   // (code, score) pairs a wavefront keeps in LDS for its token
-constexpr int FUSED_MAX_NC = 4;    // column passes of 256 the one-launch layer's gather keeps in flight together
 
 // Part of the score recurrence over the four values of one float4:
 // s <- s + a_c, p <- p * f_c with a_c = |z_c| and f_c = 1 + exp(-2|z_c|), c ascending.
@@ -278,93 +270,23 @@ __device__ __forceinline__ void score_chain(const float (&a)[4], const float (&f
     }
 }
 
-// The gather-add of one token inside the one-launch layer (PL/lookup.py:120-130, 108): this
-// wavefront adds the rows of tables [t_lo, t_hi) that the (code, score) pairs in `mine` select,
-// eight tables at a time and all NC column passes of 256 columns of those eight rows in flight
-// together (the token's chain of dependent memory round trips is what a small batch waits for:
-// 8 * NC row loads per round trip instead of 8); the four wavefronts' partial sums meet in LDS and
-// wavefront 0 adds bias and residual and writes the row.  Loads are unconditional at clamped
-// columns, so that none of them waits for another; what a clamped lane loaded is never stored.
-template <int NC>
-__device__ __forceinline__ void fused_gather(const ProjectArgs &a, const uint2 *mine, float4 (*part)[FUSED_MAX_NC][64],
-                                             int64_t row, int col0, int t_lo, int t_hi, int wave, int lane) {
-    int gc[NC];
-    bool on[NC];
-    float4 acc[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        on[c] = col0 + 256 * c + 4 * lane < a.Do;
-        gc[c] = on[c] ? col0 + 256 * c + 4 * lane : 0;
-        acc[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    for (int t0 = t_lo; t0 < t_hi; t0 += 8) {
-        float4 rv[8][NC];
-        float sv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int tt = min(t0 + u, t_hi - 1);
-            const uint2 pr = mine[tt];
-            sv[u] = t0 + u < t_hi ? __uint_as_float(pr.y) : 0.f;
-            const float *rowp = a.tables + ((size_t)tt * a.S + pr.x) * a.Do;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) rv[u][c] = *reinterpret_cast<const float4 *>(rowp + gc[c]);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                acc[c].x = fmaf(sv[u], rv[u][c].x, acc[c].x);
-                acc[c].y = fmaf(sv[u], rv[u][c].y, acc[c].y);
-                acc[c].z = fmaf(sv[u], rv[u][c].z, acc[c].z);
-                acc[c].w = fmaf(sv[u], rv[u][c].w, acc[c].w);
-            }
-    }
-#pragma unroll
-    for (int c = 0; c < NC; ++c) part[wave][c][lane] = acc[c];
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            if (!on[c]) continue;
-            float4 o = part[0][c][lane];
-#pragma unroll
-            for (int w = 1; w < 4; ++w) {
-                const float4 q = part[w][c][lane];
-                o.x += q.x; o.y += q.y; o.z += q.z; o.w += q.w;
-            }
-            if (a.obias) {
-                const float4 bb = *reinterpret_cast<const float4 *>(a.obias + gc[c]);
-                o.x += bb.x; o.y += bb.y; o.z += bb.z; o.w += bb.w;
-            }
-            if (a.gres) {
-                const float4 rr = *reinterpret_cast<const float4 *>(a.gres + row * a.Do + gc[c]);
-                o.x += rr.x; o.y += rr.y; o.z += rr.z; o.w += rr.w;
-            }
-            *reinterpret_cast<float4 *>(a.gout + row * a.Do + gc[c]) = o;
-        }
-    }
-    __syncthreads();                                         // `part` is free again
-}
-
-template <int LOGD, bool HASH, bool GATHER = false>
+template <int LOGD, bool HASH>
 __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
     using C = FhtCfg<LOGD>;
     constexpr int D = C::D, NJ = C::NJ, LPR = C::LPR, RPW = C::RPW;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int lr = lane % LPR;
-    // GATHER: one token per workgroup; its four wavefronts each compute the token's codes (no
-    // hand-over needed) and then share the gather, a quarter of the tables each
     // Records are written 12 bytes at a time, a token's slot next to its neighbours': a 128-byte line holds
     // about ten consecutive tokens' records of a table pair, and consecutive workgroups run on different
     // XCDs, whose L2s would each write back a sliver of every line.  So with records every XCD takes a
     // contiguous range of rows (workgroup b runs on XCD b % 8 and is that XCD's workgroup number b / 8).
-    const int64_t blk = (HASH && !GATHER && a.records)
+    const int64_t blk = (HASH && a.records)
                             ? int64_t(blockIdx.x % 8) * a.blocks_per_xcd + blockIdx.x / 8 : int64_t(blockIdx.x);
-    const int64_t row = GATHER ? int64_t(blockIdx.x) : (blk * 4 + wave) * RPW + lane / LPR;
+    const int64_t row = (blk * 4 + wave) * RPW + lane / LPR;
     const bool live = row < a.B;
     int64_t rec_slot = 0;                  // where this row's records go within a table pair's
-    if constexpr (HASH && !GATHER) {
+    if constexpr (HASH) {
         if (a.records && live) rec_slot = lffn_quad_record_slot(row, a.rec_tile);
     }
 
@@ -448,7 +370,7 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
                     v[j][3] = v[j][3] * w.w;
                 }
             }
-            if constexpr ((LOGD == 10 || LOGD == 9) && !GATHER) {
+            if constexpr (LOGD == 10 || LOGD == 9) {
                 __shared__ float xl[4 * XlCfg<LOGD>::ROW];
                 fht_rows_xl<LOGD>(v, lr, xl + wave * XlCfg<LOGD>::ROW);
             } else {
@@ -501,30 +423,7 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
                 const int nib_hi = __float_as_int(lane_xor<1>(__int_as_float(nib)));
                 score_chain(az, fz, s_run, p_run);                 // an odd lane continues from there
                 const int t = col >> 3;
-                if constexpr (GATHER) {
-                    __shared__ uint2 pairs[4][FUSED_MAX_T];
-                    static_assert(RPW == 1, "one token per wavefront");
-                    if ((lr & 1) && t < a.T)
-                        pairs[wave][t] = make_uint2((unsigned)((nib_hi << 4) | nib), __float_as_uint(s_run / p_run));
-                    if (r == a.R - 1 && j == NJ - 1) {
-                        // Small batches: the gather-add of the token's T rows follows in the same
-                        // workgroup: wavefront w takes tables [w*T/4, (w+1)*T/4) (fused_gather).
-                        // No codes or scores go to memory and nothing else is launched.
-                        __shared__ float4 part[4][FUSED_MAX_NC][64];
-                        __syncthreads();                         // the odd lanes' pairs are visible to the whole wavefront
-                        const int tq = (a.T + 3) / 4;
-                        const int t_lo = min(wave * tq, a.T), t_hi = min(t_lo + tq, a.T);
-                        // up to four column passes of 256 in flight together; wider rows in rounds of 1024
-                        for (int col0 = 0; col0 < a.Do; col0 += 256 * FUSED_MAX_NC) {
-                            switch (min(FUSED_MAX_NC, (a.Do - col0 + 255) / 256)) {
-                                case 1: fused_gather<1>(a, pairs[wave], part, row, col0, t_lo, t_hi, wave, lane); break;
-                                case 2: fused_gather<2>(a, pairs[wave], part, row, col0, t_lo, t_hi, wave, lane); break;
-                                case 3: fused_gather<3>(a, pairs[wave], part, row, col0, t_lo, t_hi, wave, lane); break;
-                                default: fused_gather<4>(a, pairs[wave], part, row, col0, t_lo, t_hi, wave, lane); break;
-                            }
-                        }
-                    }
-                } else if (a.records) {
+                if (a.records) {
                     // Tables t - 1 (even) and t sit in lanes 4m + 1 and 4m + 3: the latter fetches the
                     // former's code and score (quad_perm [1,1,1,1]) and writes the pair's record.
                     const int code_here = (nib_hi << 4) | nib;
@@ -547,6 +446,174 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
             }
         }
     }
+}
+
+// The whole layer for small batches in one launch: LayerNorm, projection and hash of a token, then its gather-add
+// (token_gather.h), one token per workgroup of eight or four wavefronts.  Codes and scores stay in LDS and are bit-identical to
+// project_kernel's (the same operations in the same order).
+//
+// What a small batch waits for is a chain of memory round trips (rows of the input, parameters, table rows), so: the
+// input row, the LayerNorm parameters, the diagonals and the bias are requested together before the first is used; the
+// repeats run side by side, one per wavefront (512 tables of 1024 columns: four); and the wavefronts split the rows.  Rows in
+// fp32, bfloat16 or half (FMT).  128 tables of 768 columns, 16 tokens: 12.3 -> 11.4 us (fp32), 34.4 -> 11.6 us (bfloat16,
+// before in two launches); 512 tables of 1024 columns 39.7 -> 29.4 us and 87.1 -> 24.5 us.
+struct TokenLayerArgs {
+    ProjectArgs p;
+    TokenGatherArgs g;
+};
+
+constexpr int TOKEN_STAGES = 4;     // diagonals requested together
+
+template <int LOGD, int FMT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs args) {
+    using C = FhtCfg<LOGD>;
+    constexpr int D = C::D, NJ = C::NJ;
+    static_assert(C::LPR == 64, "one token per wavefront");
+    __shared__ uint2 pairs[TOKEN_MAX_T];
+    const ProjectArgs &a = args.p;
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int64_t row = blockIdx.x;
+    if (wave < a.R) {                                          // uniform over the wavefront
+        float orig[NJ][4], lw[NJ][4], lb[NJ][4];
+        float4 dg[TOKEN_STAGES][NJ], pb[NJ];
+        auto fetch_diag = [&](int r, int s0) {
+#pragma unroll
+            for (int s = 0; s < TOKEN_STAGES; ++s)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+                    if (s0 + s < a.J)
+                        dg[s][j] = *reinterpret_cast<const float4 *>(a.diag + ((int64_t)r * a.J + s0 + s) * D + 256 * j + 4 * lane);
+        };
+        auto fetch_bias = [&](int r) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int col = r * D + 256 * j + 4 * lane;
+                pb[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (a.pbias && col < a.out_cols) pb[j] = *reinterpret_cast<const float4 *>(a.pbias + col);
+            }
+        };
+        auto fetch_row = [&](const float *p, bool vec, float (&v)[NJ][4]) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int e0 = 256 * j + 4 * lane;
+                float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (vec) {
+                    if (e0 < a.H) t = *reinterpret_cast<const float4 *>(p + e0);
+                } else {
+                    if (e0 + 0 < a.H) t.x = p[e0 + 0];
+                    if (e0 + 1 < a.H) t.y = p[e0 + 1];
+                    if (e0 + 2 < a.H) t.z = p[e0 + 2];
+                    if (e0 + 3 < a.H) t.w = p[e0 + 3];
+                }
+                v[j][0] = t.x; v[j][1] = t.y; v[j][2] = t.z; v[j][3] = t.w;
+            }
+        };
+        fetch_row(a.x + row * a.H, a.vec_in, orig);
+        if (a.ln_w) {
+            fetch_row(a.ln_w, a.vec_ln, lw);
+            fetch_row(a.ln_b, a.vec_ln, lb);
+        }
+        fetch_diag(wave, 0);
+        fetch_bias(wave);
+        __builtin_amdgcn_sched_barrier(0);                     // (the loads stay ahead of the reductions below)
+
+        if (a.ln_w) {
+            // LayerNorm as in project_kernel
+            float s1 = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s1 += orig[j][c];
+            const float mean = lane_group_sum<64>(s1) / float(a.H);
+            float s2 = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float dlt = (256 * j + 4 * lane + c < a.H) ? orig[j][c] - mean : 0.f;
+                    s2 += dlt * dlt;
+                }
+            const float rstd = 1.0f / sqrtf(lane_group_sum<64>(s2) / float(a.H) + a.ln_eps);
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (256 * j + 4 * lane + c < a.H) orig[j][c] = (orig[j][c] - mean) * rstd * lw[j][c] + lb[j][c];
+        }
+
+        for (int r = wave; r < a.R; r += WAVES) {
+            float v[NJ][4];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[j][c] = orig[j][c];
+            if (r != wave) {
+                fetch_diag(r, 0);
+                fetch_bias(r);
+            }
+            for (int s0 = 0; s0 < a.J; s0 += TOKEN_STAGES) {
+                if (s0) fetch_diag(r, s0);
+#pragma unroll
+                for (int s = 0; s < TOKEN_STAGES; ++s) {
+                    if (s0 + s < a.J) {                        // uniform
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) {
+                            v[j][0] = v[j][0] * dg[s][j].x; v[j][1] = v[j][1] * dg[s][j].y;
+                            v[j][2] = v[j][2] * dg[s][j].z; v[j][3] = v[j][3] * dg[s][j].w;
+                        }
+                        fht_rows<LOGD>(v, lane);
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                float z[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float m0 = a.decay * v[j][c];
+                    const float m1 = a.residual * orig[j][c];
+                    z[c] = m0 + m1;
+                }
+                if (a.pbias) { z[0] = z[0] + pb[j].x; z[1] = z[1] + pb[j].y; z[2] = z[2] + pb[j].z; z[3] = z[3] + pb[j].w; }
+                // code and score as in project_kernel: the odd lane of a pair continues the even lane's sum and product
+                const int nib = (z[0] > 0.f ? 8 : 0) | (z[1] > 0.f ? 4 : 0) | (z[2] > 0.f ? 2 : 0) | (z[3] > 0.f ? 1 : 0);
+                float az[4], fz[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    az[c] = fabsf(z[c]);
+                    fz[c] = 1.0f + exp_minus_2a(az[c]);
+                }
+                float s_loc = 0.f, p_loc = 1.f;
+                score_chain(az, fz, s_loc, p_loc);
+                float s_run = lane_xor<1>(s_loc);
+                float p_run = lane_xor<1>(p_loc);
+                const int nib_hi = __float_as_int(lane_xor<1>(__int_as_float(nib)));
+                score_chain(az, fz, s_run, p_run);
+                const int t = (r * D + 256 * j + 4 * lane) >> 3;
+                if ((lane & 1) && t < a.T)
+                    pairs[t] = make_uint2((unsigned)((nib_hi << 4) | nib), __float_as_uint(s_run / p_run));
+            }
+        }
+    }
+    __syncthreads();
+    token_gather<WAVES, FMT>(args.g, pairs, row, wave, lane);
+}
+
+template <int FMT, int WAVES>
+int launch_token_layer_waves(const TokenLayerArgs &a, int64_t D, hipStream_t st) {
+    const dim3 grid((unsigned)a.p.B), block(64 * WAVES);
+    switch (lffn_log2(D)) {
+        case 8: hipLaunchKernelGGL((token_layer_kernel<8, FMT, WAVES>), grid, block, 0, st, a); break;
+        case 9: hipLaunchKernelGGL((token_layer_kernel<9, FMT, WAVES>), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((token_layer_kernel<10, FMT, WAVES>), grid, block, 0, st, a); break;
+    }
+    return lffn_launch_status();
+}
+
+template <int FMT>
+int launch_token_layer(const TokenLayerArgs &a, int64_t D, hipStream_t st) {
+    return a.p.B <= TOKEN_WIDE_MAX ? launch_token_layer_waves<FMT, 8>(a, D, st) : launch_token_layer_waves<FMT, 4>(a, D, st);
 }
 
 template <bool HASH>
@@ -982,47 +1049,49 @@ static int project_hash_impl(const float *x, const float *ln_w, const float *ln_
     return launch_project<true>(a, lffn_log2(D), static_cast<hipStream_t>(stream));
 }
 
+extern "C" int lffn_lookup_ffn_fused_layer_rows(const lffn_fused_layer *layer, int32_t row_format, const float *x,
+                                                const float *residual_in, float *out, int64_t B, void *stream) {
+    LFFN_REQUIRE(layer && row_format >= 0 && row_format <= 2, LFFN_ERR_BAD_ARG);
+    const lffn_fused_layer &l = *layer;
+    LFFN_REQUIRE(x && l.diag && l.tables && out, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE((l.ln_weight != nullptr) == (l.ln_bias != nullptr) && l.ln_eps >= 0.f, LFFN_ERR_BAD_ARG);
+    int rc = check_dims(B, l.H, l.D, l.R, l.J);
+    if (rc != LFFN_OK) return rc;
+    LFFN_REQUIRE(l.D >= 256 && l.T <= TOKEN_MAX_T && l.S >= 256 && l.S * l.T <= 0x7fffffff, LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(l.Do >= 4 && l.Do % 4 == 0 && l.Do <= (1 << 20), LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(l.T >= 1 && l.T * 8 <= l.R * l.D, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(l.diag) && (!l.proj_bias || lffn_aligned16(l.proj_bias)) && lffn_aligned16(l.tables) &&
+                     (!l.out_bias || lffn_aligned16(l.out_bias)) && (!residual_in || lffn_aligned16(residual_in)) &&
+                     lffn_aligned16(out),
+                 LFFN_ERR_BAD_ARG);
+    if (B == 0) return LFFN_OK;
+    TokenLayerArgs args{};
+    ProjectArgs &a = args.p;
+    a.x = x; a.diag = l.diag; a.pbias = l.proj_bias; a.ln_w = l.ln_weight; a.ln_b = l.ln_bias; a.ln_eps = l.ln_eps;
+    a.B = B; a.H = (int)l.H; a.R = (int)l.R; a.J = (int)l.J;
+    a.out_cols = (int)(l.T * 8); a.T = (int)l.T;
+    a.decay = l.decay; a.residual = l.residual;
+    a.vec_in = (lffn_aligned16(x) && l.H % 4 == 0) ? 1 : 0;
+    a.vec_ln = (l.H % 4 == 0 && l.ln_weight && lffn_aligned16(l.ln_weight) && lffn_aligned16(l.ln_bias)) ? 1 : 0;
+    args.g = TokenGatherArgs{l.tables, l.out_bias, residual_in, out, (int)l.T, (int)l.S, (int)l.Do};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (row_format == LFFN_ROWS_BF16) return launch_token_layer<LFFN_ROWS_BF16>(args, l.D, st);
+    if (row_format == LFFN_ROWS_F16) return launch_token_layer<LFFN_ROWS_F16>(args, l.D, st);
+    return launch_token_layer<LFFN_ROWS_F32>(args, l.D, st);
+}
+
+extern "C" int lffn_lookup_ffn_fused_layer_f32(const lffn_fused_layer *layer, const float *x, const float *residual_in,
+                                               float *out, int64_t B, void *stream) {
+    return lffn_lookup_ffn_fused_layer_rows(layer, LFFN_ROWS_F32, x, residual_in, out, B, stream);
+}
+
 extern "C" int lffn_lookup_ffn_fused_f32(const float *x, const float *ln_weight, const float *ln_bias, float ln_eps,
                                          const float *diag, const float *proj_bias, const float *tables,
                                          const float *out_bias, const float *residual_in, float *out, int64_t B,
                                          int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t S,
                                          int64_t Do, float decay, float residual, void *stream) {
-    LFFN_REQUIRE(x && diag && tables && out, LFFN_ERR_BAD_ARG);
-    LFFN_REQUIRE((ln_weight != nullptr) == (ln_bias != nullptr) && ln_eps >= 0.f, LFFN_ERR_BAD_ARG);
-    int rc = check_dims(B, H, D, R, J);
-    if (rc != LFFN_OK) return rc;
-    LFFN_REQUIRE(D >= 256 && T <= FUSED_MAX_T && S >= 256 && S * T <= 0x7fffffff, LFFN_ERR_UNSUPPORTED);
-    LFFN_REQUIRE(Do >= 4 && Do % 4 == 0 && Do <= (1 << 20), LFFN_ERR_UNSUPPORTED);
-    LFFN_REQUIRE(T >= 1 && T * 8 <= R * D, LFFN_ERR_BAD_ARG);
-    LFFN_REQUIRE(lffn_aligned16(diag) && (!proj_bias || lffn_aligned16(proj_bias)) && lffn_aligned16(tables) &&
-                     (!out_bias || lffn_aligned16(out_bias)) && (!residual_in || lffn_aligned16(residual_in)) &&
-                     lffn_aligned16(out),
-                 LFFN_ERR_BAD_ARG);
-    if (B == 0) return LFFN_OK;
-    ProjectArgs a{};
-    a.x = x; a.diag = diag; a.pbias = proj_bias; a.ln_w = ln_weight; a.ln_b = ln_bias; a.ln_eps = ln_eps;
-    a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J;
-    a.out_stride = (int)(T * 8); a.out_cols = (int)(T * 8); a.T = (int)T;
-    a.decay = decay; a.residual = residual; a.mix = 1;
-    a.vec_in = (lffn_aligned16(x) && H % 4 == 0) ? 1 : 0;
-    a.vec_ln = (H % 4 == 0 && ln_weight && lffn_aligned16(ln_weight) && lffn_aligned16(ln_bias)) ? 1 : 0;
-    a.tables = tables; a.obias = out_bias; a.gres = residual_in; a.gout = out; a.S = (int)S; a.Do = (int)Do;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const dim3 grid((unsigned)B);                       // one token per workgroup
-    switch (lffn_log2(D)) {
-        case 8: hipLaunchKernelGGL((project_kernel<8, true, true>), grid, dim3(256), 0, st, a); break;
-        case 9: hipLaunchKernelGGL((project_kernel<9, true, true>), grid, dim3(256), 0, st, a); break;
-        default: hipLaunchKernelGGL((project_kernel<10, true, true>), grid, dim3(256), 0, st, a); break;
-    }
-    return lffn_launch_status();
-}
-
-extern "C" int lffn_lookup_ffn_fused_layer_f32(const lffn_fused_layer *layer, const float *x, const float *residual_in,
-                                               float *out, int64_t B, void *stream) {
-    LFFN_REQUIRE(layer, LFFN_ERR_BAD_ARG);
-    return lffn_lookup_ffn_fused_f32(x, layer->ln_weight, layer->ln_bias, layer->ln_eps, layer->diag, layer->proj_bias,
-                                     layer->tables, layer->out_bias, residual_in, out, B, layer->H, layer->D, layer->R,
-                                     layer->J, layer->T, layer->S, layer->Do, layer->decay, layer->residual, stream);
+    const lffn_fused_layer l{ln_weight, ln_bias, diag, proj_bias, tables, out_bias, H, D, R, J, T, S, Do, ln_eps, decay, residual};
+    return lffn_lookup_ffn_fused_layer_f32(&l, x, residual_in, out, B, stream);
 }
 
 extern "C" int lffn_fht_f16(const uint16_t *in, uint16_t *out, int64_t B, int64_t D, void *stream) {

@@ -380,9 +380,10 @@ class LookupFFN(nn.Module):
         return (f"hidden_size={self.hidden_size}, num_table={self.num_table}, "
                 f"table_size={self.table_size}, output_size={self.output_size}")
 
-    # Up to this many tokens the one-launch form of the layer (a wavefront per token: LayerNorm,
-    # projection, hash and the token's gather-add) beats the projection kernel followed by the
-    # table-major gather, which stages every table slice in LDS and needs many tokens to pay for it.
+    # Up to this many tokens (half as many more for 16-bit rows) the one-launch form of the layer (a workgroup per
+    # token: LayerNorm, projection, hash and the token's gather-add) beats the projection kernel followed by the
+    # table-major gather, which stages every table slice in LDS and needs many tokens to pay for it: 512 tokens, 128
+    # tables of 768 fp32 columns 34 us against 37, 768 tokens 49 against 46.
     FUSED_LAYER_MAX_TOKENS = 512
 
     def _no_gradient_wanted(self, x):
@@ -391,8 +392,11 @@ class LookupFFN(nn.Module):
 
     def can_fuse_layer(self, x):
         """The one-launch form applies: few tokens, fp32 on the GPU, no gradient wanted, and parameters
-        of the kind it is built for (diagonal BH4, 8-bit codes, 256-entry fp32 tables)."""
-        if not (x.shape[0] <= self.FUSED_LAYER_MAX_TOKENS and x.is_cuda and x.dtype == torch.float32
+        of the kind it is built for (diagonal BH4, 8-bit codes, 256-entry tables)."""
+        most = self.FUSED_LAYER_MAX_TOKENS
+        if self.tables.dtype != torch.float32:
+            most += most // 2
+        if not (x.shape[0] <= most and x.is_cuda and x.dtype == torch.float32
                 and self._no_gradient_wanted(x)):
             return False
         st = self._inference_state()
@@ -430,7 +434,7 @@ class LookupFFN(nn.Module):
             state = dict(
                 form=form,
                 one_launch=(form == "diag" and p.padded_in_dim >= 256 and self.num_table <= 512
-                            and self.table_size == 256 and self.tables.dtype == torch.float32),
+                            and self.table_size == 256),
                 ln_w=ln.weight.detach(), ln_b=ln.bias.detach(), eps=float(ln.eps),
                 diag=(p.weight.detach().reshape(p.num_repeat, p.weight.shape[1], p.padded_in_dim)
                       if form == "diag" else None),

@@ -3,11 +3,15 @@ tiles can go wrong, against float64 sums of the same values.
 
 Bounds: an fp32 sum of n products is within n * 2^-24 of the sum of their magnitudes; the comparisons below use that sum
 itself (the operator on absolute values in float64) as the scale of every element."""
+import ctypes
+
+import numpy as np
 import pytest
 import torch
 
 import lookupffn_amd
 from lookupffn_amd import _lib, ops
+from tests import _cabi as cabi
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -110,3 +114,34 @@ def test_scatter_rows_accumulates_and_clamps():
     want = _reference(clamped, src, w, grad)[2] + start.double()
     scale = _reference(clamped, src, w.abs(), grad.abs())[2] + start.abs().double()
     _close(out, want, scale, torch.bincount(clamped.reshape(-1)).max().item() + 1)
+
+
+# The layer in one launch: column passes of 256 below, at and past their edges and past the four that go together, table
+# counts around the eight wavefronts' shares, one to three repeats, more stages than are requested together
+@pytest.mark.parametrize("B,H,D,R,J,T,Do", [(1, 256, 256, 1, 4, 1, 64), (3, 250, 256, 2, 5, 63, 260), (5, 512, 512, 1, 1, 64, 512),
+                                            (2, 768, 1024, 1, 4, 128, 1284), (9, 1024, 1024, 4, 4, 512, 1024),
+                                            (260, 512, 512, 1, 4, 33, 256), (257, 1024, 1024, 4, 4, 480, 1088)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_one_launch_layer_on_rows_of_every_format(B, H, D, R, J, T, Do, dtype):
+    gen = torch.Generator().manual_seed(B + H + T)
+    rand = lambda *s: torch.randn(*s, generator=gen)
+    x, res = rand(B, H), rand(B, Do)
+    lw, lb = 1 + 0.1 * rand(H), 0.1 * rand(H)
+    diag = torch.sign(rand(R, J, D)) / D ** 0.5
+    pbias, obias = 0.01 * rand(T * 8), 0.001 * rand(Do)
+    tables = (0.02 * rand(T, 256, Do)).to(dtype)
+    code, score, _ = cabi.ln_project_hash(x.numpy(), lw.numpy(), lb.numpy(), 1e-5, diag.numpy(), pbias.numpy(), T)
+    rows = tables.double()[torch.arange(T)[None], torch.from_numpy(code).long()]             # [B, T, Do]
+    products = rows * torch.from_numpy(score).double()[:, :, None]
+    want = products.sum(1) + obias.double() + res.double()
+    dev = {k: v.cuda() for k, v in dict(lw=lw, lb=lb, diag=diag, pbias=pbias, tables=tables, obias=obias, x=x, res=res).items()}
+    p = lambda k: dev[k].data_ptr()
+    block = _lib.FusedLayer(p("lw"), p("lb"), p("diag"), p("pbias"), p("tables"), p("obias"), H, D, R, J, T, 256, Do, 1e-5,
+                            float(np.float32(0.7)), float(np.float32(1 - 0.7)))
+    out = torch.full((B, Do), float("nan"), device="cuda")
+    fmt = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    _lib.check(_lib.load().lffn_lookup_ffn_fused_layer_rows(ctypes.byref(block), fmt, p("x"), p("res"), out.data_ptr(), B,
+                                                            torch.cuda.current_stream().cuda_stream), "fused")
+    # fp32 sums of T products, exact in the rows: each of T + 8 additions rounds by 2^-24 of a partial sum
+    bound = (T + 8) * 2.0 ** -24 * (products.abs().sum(1) + obias.abs() + res.abs())
+    assert ((out.cpu().double() - want).abs() <= bound).all()
