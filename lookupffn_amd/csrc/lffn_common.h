@@ -34,6 +34,12 @@ int lffn_internal_lookup_gather_token_major(const int32_t *code, const float *sc
                                             const float *bias, const float *residual, float *out, int64_t B,
                                             int64_t T, int64_t S, int64_t Do, int fmt, void *stream);
 
+// gather.hip: the same for a caller that leaves the choice of kernel open: few tokens take a workgroup each (not exported)
+__attribute__((visibility("hidden")))
+int lffn_internal_lookup_gather_tokens(const int32_t *code, const float *score, const void *tables, const float *bias,
+                                       const float *residual, float *out, int64_t B, int64_t T, int64_t S, int64_t Do,
+                                       int fmt, void *stream);
+
 // gather.hip: the token-major operators on flat row numbers; with flags (see TableGuard) the launch is for arrays
 // that are not in table form.  table_form writes those flags (TABLE_FLAGS words).
 __attribute__((visibility("hidden")))

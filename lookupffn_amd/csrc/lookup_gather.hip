@@ -660,6 +660,8 @@ int lookup_gather_entry(const int32_t *code, const float *score, const void *tab
             quad_ws = workspace;
         }
     }
+    if (plan.kind == 0 && kind_req < 0)
+        return lffn_internal_lookup_gather_tokens(code, score, tables, bias, residual, out, B, T, S, Do, BF16, stream);
     if (plan.kind == 0)
         return lffn_internal_lookup_gather_token_major(code, score, tables, bias, residual, out, B, T, S, Do, BF16, stream);
     if (plan.kind == 3)
@@ -721,6 +723,8 @@ int lookup_gather_entry_f16(const int32_t *code, const float *score, const void 
     if (tile)
         return lffn_internal_lookup_gather_quad(code, score, tables, bias, residual, out, B, T, S, Do, LFFN_ROWS_F16, tile,
                                                 workspace, stream);
+    if (kind_req < 0)
+        return lffn_internal_lookup_gather_tokens(code, score, tables, bias, residual, out, B, T, S, Do, LFFN_ROWS_F16, stream);
     return lffn_internal_lookup_gather_token_major(code, score, tables, bias, residual, out, B, T, S, Do, LFFN_ROWS_F16, stream);
 }
 

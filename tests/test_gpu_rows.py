@@ -145,3 +145,22 @@ def test_one_launch_layer_on_rows_of_every_format(B, H, D, R, J, T, Do, dtype):
     # fp32 sums of T products, exact in the rows: each of T + 8 additions rounds by 2^-24 of a partial sum
     bound = (T + 8) * 2.0 ** -24 * (products.abs().sum(1) + obias.abs() + res.abs())
     assert ((out.cpu().double() - want).abs() <= bound).all()
+
+
+# The gather by a workgroup per token: both widths of workgroup, table counts around the wavefronts' shares, column passes, table
+# sizes other than 256, and the largest batch of it
+@pytest.mark.parametrize("B,T,S,Do", [(1, 1, 16, 64), (7, 65, 256, 320), (256, 32, 128, 256), (257, 30, 256, 1088), (512, 512, 256, 64),
+                                      (1024, 8, 256, 768)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_gather_of_few_tokens(B, T, S, Do, dtype):
+    gen = torch.Generator().manual_seed(B + T)
+    code = torch.randint(0, S, (B, T), generator=gen, dtype=torch.int32)
+    score = torch.randn(B, T, generator=gen)
+    tables = torch.randn(T, S, Do, generator=gen).to(dtype)
+    bias, res = torch.randn(Do, generator=gen), torch.randn(B, Do, generator=gen)
+    want, scale = bias.double() + res.double(), bias.abs().double() + res.abs().double()
+    for t in range(T):
+        products = tables[t].double()[code[:, t].long()] * score[:, t].double()[:, None]
+        want, scale = want + products, scale + products.abs()
+    got = ops.lookup_gather(code.cuda(), score.cuda(), tables.cuda(), bias.cuda(), res.cuda())
+    assert ((got.cpu().double() - want).abs() <= (T + 8) * 2.0 ** -24 * scale).all()      # T + 8 additions in fp32
