@@ -51,11 +51,9 @@ constexpr int PAD = 4;          // floats of padding per LDS row
 // index o'.  MODE 2: natural [o'][i] order (turns a gradient w.r.t. the folded weights into the
 // gradient w.r.t. the weights: H64 is symmetric).
 template <int MODE>
-__global__ __launch_bounds__(256) void bh4_fold_kernel(const float *w, float *wf, int64_t nblk) {
-    const int64_t gid = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (gid >= nblk * BS) return;
-    const int64_t blk = gid / BS;
-    const int i = (int)(gid % BS);
+__global__ __launch_bounds__(64) void bh4_fold_kernel(const float *w, float *wf) {
+    const int64_t blk = blockIdx.x;               // one block per workgroup: there are few
+    const int i = threadIdx.x;
     const float *src = w + blk * (BS * BS) + i;
     float v[BS];
 #pragma unroll
@@ -138,21 +136,27 @@ __device__ __forceinline__ float from_row_below(float v) {
 // HV = 16-token halves per workgroup: 2 (32 tokens, one workgroup per CU at D = 1024) or 1 (16
 // tokens, half the LDS, so that two workgroups share a CU and the load, hand-over and hash phases
 // of one run under the products of the other).
-template <int NB, bool HASH, int NH, bool BWD = false, int HV = 2>
-__global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kernel(BlockArgs a) {
+// BG = groups the blocks are split into: 1, or 4 for the wide form of small batches, in which 16 wavefronts share
+// 16 tokens and wavefront group bg has blocks bg, bg + 4, ...  The butterflies across a wavefront's own blocks (strides
+// 4 and up) stay between accumulators, the last two (strides 2 and 1) are a pass over the LDS tile: the same additions in the
+// same order, so the results are those of the other forms bit for bit.
+template <int NB, bool HASH, int NH, bool BWD = false, int HV = 2, int BG = 1>
+__global__ __launch_bounds__(256 * BG * HV / NH, BG > 1 ? 4 : (HV == 1 ? 2 : 1)) void bh4_block_kernel(BlockArgs a) {
     static_assert(!(HASH && BWD), "one form at a time");
     static_assert(NH <= HV, "a wavefront cannot hold more halves than the tile has");
+    static_assert(BG == 1 || (BG == 4 && HV == 1 && NB >= 4), "the wide form: 16 tokens, four groups of blocks");
     constexpr int TOK = 16 * HV;                  // tokens per workgroup
-    constexpr int NWAVE = 4 * (HV / NH);
+    constexpr int NWAVE = 4 * (HV / NH) * BG;
+    constexpr int NBW = NB / BG;                  // blocks of a wavefront: bg + BG * n, n < NBW
     const float *__restrict__ x = a.x;
     const float *__restrict__ wf = a.wf;
     const int64_t B = a.B;
     const int H = a.H, R = a.R, J = a.J;
     constexpr int D = BS * NB;
     constexpr int LDR = D + PAD;
-    constexpr int G = NB >= 2 ? 2 : 1;            // blocks worked on together
+    constexpr int G = NBW >= 2 ? 2 : 1;           // blocks worked on together
     constexpr int NS = 2 * G;                     // register slots: block n sits in slot n % NS
-    constexpr bool AHEAD = NB >= NS;              // first blocks of a stage fetched during the previous one
+    constexpr bool AHEAD = BG > 1 || NB >= NS;    // first blocks of a stage fetched during the previous one
     extern __shared__ __attribute__((aligned(16))) float xs[];   // TOK rows of LDR floats, then the row statistics
     float *stats = xs + TOK * LDR;                // [TOK][2]: mean and 1/sigma of LayerNorm
     float *lnw_s = stats + 2 * TOK;               // [D] LayerNorm weight and bias (hash form, for the epilogue)
@@ -162,7 +166,8 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int ow = wave & 3;                      // output columns [16*ow, 16*ow + 16) of each block
-    const int hg = wave >> 2;                     // NH == 1: the token half of this wavefront
+    const int hg = BG > 1 ? 0 : wave >> 2;        // NH == 1: the token half of this wavefront
+    const int bg = BG > 1 ? wave >> 2 : 0;        // group of blocks of this wavefront
     const int c = lane & 15;                      // A operand: output column; B operand and result: token
     const int kq = lane >> 4;                     // k index inside an MFMA; result: output columns 4*kq .. 4*kq+3
     const int64_t tok_base = int64_t(blockIdx.x) * TOK;
@@ -178,21 +183,45 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
 
     // this lane's weight fragment of block n, quarter q (input columns 16*kq + 4*q .. +3 of output
     // column 16*wave + c): wf[..][n][wave][q][lane][0..3]
-    const int w_lane_off = ow * 1024 + lane * 4;
+    const int w_lane_off = bg * (BS * BS) + ow * 1024 + lane * 4;
     // this lane's token values of block n, half h: xs[(16*h + c) * LDR + 64*n + 16*kq ..]
-    const int x_lane_off = c * LDR + 16 * kq;
+    const int x_lane_off = c * LDR + bg * BS + 16 * kq;
     // where this lane's results of block n, half h go: xs[(16*h + c) * LDR + 64*n + 16*wave + 4*kq ..]
-    const int y_lane_off = c * LDR + 16 * ow + 4 * kq;
+    const int y_lane_off = c * LDR + bg * BS + 16 * ow + 4 * kq;
 
     auto load_w = [&](const float *wst, int n, int q) {
-        return *reinterpret_cast<const float4 *>(wst + n * (BS * BS) + q * 256);
+        return *reinterpret_cast<const float4 *>(wst + n * BG * (BS * BS) + q * 256);
     };
     auto read_x = [&](int h, int n, int q) {
-        return *reinterpret_cast<const float4 *>(xs + h * 16 * LDR + x_lane_off + n * BS + q * 4);
+        return *reinterpret_cast<const float4 *>(xs + h * 16 * LDR + x_lane_off + n * BG * BS + q * 4);
     };
 
-    for (int r = 0; r < R; ++r) {
-        __syncthreads();                          // the previous repeat's last stage has been read
+    // A workgroup takes one repeat of its tokens, and the repeats come one after the other in the grid: their 1 MB of weights
+    // stay in the L2 for the launch's workgroups, and few tokens with several repeats are as many workgroups more (32768
+    // tokens, D = 512, two repeats: the layer 355 -> 320 us against a loop over the repeats; 64 tokens, D = 1024, four: 240 -> 138).
+    const int r = blockIdx.y;
+    // Wide form: strides 2 and 1 of the butterflies across the blocks, on the LDS tile, 16 bytes of blocks 4 n .. 4 n + 3 per
+    // thread and step; the tile's result is also written to rows of D floats at `save` if there is one.
+    auto last_strides = [&](float *save) {
+        if constexpr (BG > 1) {
+            for (int e = tid; e < TOK * 16 * NBW; e += 64 * NWAVE) {
+                const int row = e / (16 * NBW), n = (e / 16) % NBW, c4 = (e % 16) * 4;
+                float *p = xs + row * LDR + n * BG * BS + c4;
+                f32x4 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4 *>(p + k * BS);
+                const f32x4 s0 = v[0] + v[2], s1 = v[1] + v[3], d0 = v[0] - v[2], d1 = v[1] - v[3];
+                v[0] = s0 + s1; v[1] = s0 - s1; v[2] = d0 + d1; v[3] = d0 - d1;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(p + k * BS) = v[k];
+                if (save && tok_base + row < B) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(save + size_t(row) * D + (n * BG + k) * BS + c4) = v[k];
+                }
+            }
+        }
+    };
+    {
         {
             // A wavefront loads TOK/NWAVE rows, 16 bytes per lane and 1 KB of a row per instruction, all
             // loads in flight before the first use (one at a time, each would pay the full
@@ -283,7 +312,31 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
         for (int si = 0; si < J; ++si) {
             const int s = BWD ? J - 1 - si : si;                  // the backward walks the stages down
             const float *wst = wf + (size_t)((r * J + s) * NB) * (BS * BS) + w_lane_off;
-            if constexpr (BWD) {
+            if constexpr (BWD && BG > 1) {
+                // the same in the wide form, in two passes over the tile
+                if constexpr (NBW > 1) {
+                    const int row = tid / 64, k = (tid / 16) % 4, c4 = (tid % 16) * 4;
+                    static_assert(TOK * 64 == 64 * NWAVE, "a thread per row, first block and 16 bytes");
+                    float *p = xs + row * LDR + k * BS + c4;
+                    f32x4 v[NBW];
+#pragma unroll
+                    for (int m = 0; m < NBW; ++m) v[m] = *reinterpret_cast<const f32x4 *>(p + m * BG * BS);
+#pragma unroll
+                    for (int h = NBW / 2; h >= 1; h >>= 1)
+#pragma unroll
+                        for (int m = 0; m < NBW; ++m)
+                            if ((m & h) == 0) {
+                                const f32x4 lo = v[m], hi = v[m + h];
+                                v[m] = lo + hi;
+                                v[m + h] = lo - hi;
+                            }
+#pragma unroll
+                    for (int m = 0; m < NBW; ++m) *reinterpret_cast<f32x4 *>(p + m * BG * BS) = v[m];
+                    __syncthreads();
+                }
+                last_strides(a.stage_save + ((size_t(r) * J + s) * B + tok_base) * D);
+                __syncthreads();
+            } else if constexpr (BWD) {
                 // butterflies across the blocks on the LDS tile, 16 bytes of every block per thread;
                 // the result is this stage's P, kept for the weight gradient
                 for (int e = tid; e < TOK * 16; e += 64 * NWAVE) {
@@ -312,9 +365,9 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
                 }
                 __syncthreads();
             }
-            f32x4 acc[NH][NB];
+            f32x4 acc[NH][NBW];
 #pragma unroll
-            for (int n = 0; n < NB; ++n)
+            for (int n = 0; n < NBW; ++n)
 #pragma unroll
                 for (int t = 0; t < NH; ++t) acc[t][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
             if constexpr (!AHEAD) {
@@ -335,10 +388,10 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
             // pair of blocks are spread between the products instead of queueing in a burst at the
             // LDS and the texture unit, and two blocks are worked on together (2*NH independent
             // accumulation chains).
-            static_for<NB / G>([&](auto p_c) {
+            static_for<NBW / G>([&](auto p_c) {
                 constexpr int n0 = decltype(p_c)::value * G;
                 constexpr int n1 = n0 + G - 1;                  // == n0 when G == 1
-                constexpr bool more = n0 + G < NB;              // another pair follows in this stage
+                constexpr bool more = n0 + G < NBW;             // another pair follows in this stage
                 constexpr int m0 = (n0 + G) % NS, m1 = (n1 + G) % NS;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
@@ -402,9 +455,9 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
             // H_NB across the blocks (the backward did it before the product)
             if constexpr (!BWD) {
 #pragma unroll
-                for (int h = NB / 2; h >= 1; h >>= 1) {
+                for (int h = NBW / 2; h >= 1; h >>= 1) {
 #pragma unroll
-                    for (int n = 0; n < NB; ++n) {
+                    for (int n = 0; n < NBW; ++n) {
                         if ((n & h) == 0) {
 #pragma unroll
                             for (int t = 0; t < NH; ++t) {
@@ -418,12 +471,26 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
             }
 
             __syncthreads();                      // every wavefront has read this stage's input
-            if (si + 1 < J) {
+            if constexpr (BG > 1 && !BWD) {
+                // strides 2 and 1 of the butterflies: blocks 4 n .. 4 n + 3, which four wavefronts hold
 #pragma unroll
-                for (int n = 0; n < NB; ++n)
+                for (int n = 0; n < NBW; ++n) *reinterpret_cast<f32x4 *>(xs + y_lane_off + n * BG * BS) = acc[0][n];
+                __syncthreads();
+                last_strides(a.stage_save && si + 1 < J ? a.stage_save + ((size_t(r) * (J - 1) + s) * B + tok_base) * D : nullptr);
+                __syncthreads();
+                if (si + 1 == J) {                // the results go on from the accumulators, and the tile is free
+#pragma unroll
+                    for (int n = 0; n < NBW; ++n) acc[0][n] = *reinterpret_cast<const f32x4 *>(xs + y_lane_off + n * BG * BS);
+                    __syncthreads();
+                }
+            }
+            if (si + 1 < J) {
+                if constexpr (BG > 1 && !BWD) continue;
+#pragma unroll
+                for (int n = 0; n < NBW; ++n)
 #pragma unroll
                     for (int t = 0; t < NH; ++t)
-                        *reinterpret_cast<f32x4 *>(xs + (hg * NH + t) * 16 * LDR + y_lane_off + n * BS) = acc[t][n];
+                        *reinterpret_cast<f32x4 *>(xs + (hg * NH + t) * 16 * LDR + y_lane_off + n * BG * BS) = acc[t][n];
                 if (!BWD && a.stage_save) {
                     // the input of stage s+1, kept for the weight gradient of the backward
 #pragma unroll
@@ -432,7 +499,7 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
                         if (tok < B) {
                             float *o = a.stage_save + ((size_t(r) * (J - 1) + s) * B + tok) * D + 16 * ow + 4 * kq;
 #pragma unroll
-                            for (int n = 0; n < NB; ++n) *reinterpret_cast<f32x4 *>(o + n * BS) = acc[t][n];
+                            for (int n = 0; n < NBW; ++n) *reinterpret_cast<f32x4 *>(o + n * BS) = acc[t][n];
                         }
                     }
                 }
@@ -445,8 +512,8 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
                     const int64_t tok = tok_base + 16 * (hg * NH + t) + c;
                     if (tok < B) {
 #pragma unroll
-                        for (int n = 0; n < NB; ++n) {
-                            const int xc = n * BS + 16 * ow + 4 * kq;
+                        for (int n = 0; n < NBW; ++n) {
+                            const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq;
                             if (xc < H) {
                                 f32x4 o = acc[t][n];
                                 if (r * D + xc < ncols) {
@@ -465,9 +532,9 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
                 for (int t = 0; t < NH; ++t) {
                     const int64_t tok = tok_base + 16 * (hg * NH + t) + c;
                     if (tok < B) {
-                        float *o = a.out + tok * ld_out + (size_t)r * D + 16 * ow + 4 * kq;
+                        float *o = a.out + tok * ld_out + (size_t)r * D + bg * BS + 16 * ow + 4 * kq;
 #pragma unroll
-                        for (int n = 0; n < NB; ++n) *reinterpret_cast<f32x4 *>(o + n * BS) = acc[t][n];
+                        for (int n = 0; n < NBW; ++n) *reinterpret_cast<f32x4 *>(o + n * BG * BS) = acc[t][n];
                     }
                 }
             } else {
@@ -483,7 +550,7 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
                 bool livev[NH];
                 float meanv[NH], rstdv[NH];
                 // the tokens' input values for every block, all requested before the first use
-                float4 xin[NH][NB];
+                float4 xin[NH][NBW];
 #pragma unroll
                 for (int t = 0; t < NH; ++t) {
                     const int trow = 16 * (hg * NH + t) + c + opq;     // token within the tile
@@ -492,16 +559,16 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
                     meanv[t] = a.ln_w ? stats[2 * trow] : 0.f;
                     rstdv[t] = a.ln_w ? stats[2 * trow + 1] : 1.f;
 #pragma unroll
-                    for (int n = 0; n < NB; ++n) {
-                        const int xc = n * BS + 16 * ow + 4 * kq + opq;
+                    for (int n = 0; n < NBW; ++n) {
+                        const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq + opq;
                         xin[t][n] = (livev[t] && xc < H) ? *reinterpret_cast<const float4 *>(x + tokv[t] * H + xc)
                                                          : make_float4(0.f, 0.f, 0.f, 0.f);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int n = 0; n < NB; ++n) {
-                    const int xc = n * BS + 16 * ow + 4 * kq + opq;        // column of the padded input
+                for (int n = 0; n < NBW; ++n) {
+                    const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq + opq;    // column of the padded input
                     const int col = r * D + xc;                            // column of z
                     const bool in_cols = col < ncols;                      // whole groups of 8: all or nothing
                     float4 lw = make_float4(0.f, 0.f, 0.f, 0.f), lb = lw, bb = lw;
@@ -603,24 +670,33 @@ __global__ __launch_bounds__(256 * HV / NH, HV == 1 ? 2 : 1) void bh4_block_kern
     }
 }
 
-template <int NB, bool HASH, int NH, bool BWD = false, int HV = 2>
+template <int NB, bool HASH, int NH, bool BWD = false, int HV = 2, int BG = 1>
 int launch_block(const BlockArgs &a, hipStream_t st) {
     constexpr int TOK = 16 * HV;
     const size_t lds_bytes = (size_t(TOK) * (BS * NB + PAD) + 2 * TOK + (HASH ? 2 * BS * NB : 0)) * sizeof(float);
-    auto kern = bh4_block_kernel<NB, HASH, NH, BWD, HV>;
+    auto kern = bh4_block_kernel<NB, HASH, NH, BWD, HV, BG>;
     static LdsGrant granted;      // one record per kernel instantiation
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(kern), lds_bytes, granted)) return LFFN_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((a.B + TOK - 1) / TOK)), dim3(256 * HV / NH), lds_bytes, st, a);
+    const dim3 grid((unsigned)((a.B + TOK - 1) / TOK), (unsigned)a.R);
+    hipLaunchKernelGGL(kern, grid, dim3(256 * BG * HV / NH), lds_bytes, st, a);
     return lffn_launch_status();
 }
+
+// The wide form where its 16-token workgroups leave no compute unit a second one: there the 4 or 8 wavefronts of the other
+// forms wait for every latency of their own.  512 columns, 64 tables, 385 tokens: backward 29.2 -> 22.3 us; 1024 columns,
+// 128 tables, 16 tokens: 47.6 -> 42.0 us; a training step of 4096 tokens 498 -> 472 us, of 8192 (512 workgroups) 660 -> 663.
+// Forward at D = 256 the same (64 tokens 22.8 -> 13.1 us; layer at 4096 tokens 34.3 -> 24.9 us, at 8192 44.3 either way); at D = 512
+// and 1024 the 16-token form of 4 wavefronts is as fast with any number of tokens (23 and 42 us for 16 tokens).
+constexpr int64_t WIDE_WORKGROUPS = 256;
+bool wide(const BlockArgs &a) { return (a.B + 15) / 16 * a.R <= WIDE_WORKGROUPS; }
 
 int dispatch_block_bwd(const BlockArgs &a, int64_t D, hipStream_t st) {
     switch (D / BS) {
         case 1: return launch_block<1, false, 2, true>(a, st);
         case 2: return launch_block<2, false, 2, true>(a, st);
-        case 4: return launch_block<4, false, 2, true>(a, st);
-        case 8: return launch_block<8, false, 2, true>(a, st);
-        default: return launch_block<16, false, 1, true>(a, st);
+        case 4: return wide(a) ? launch_block<4, false, 1, true, 1, 4>(a, st) : launch_block<4, false, 2, true>(a, st);
+        case 8: return wide(a) ? launch_block<8, false, 1, true, 1, 4>(a, st) : launch_block<8, false, 2, true>(a, st);
+        default: return wide(a) ? launch_block<16, false, 1, true, 1, 4>(a, st) : launch_block<16, false, 1, true>(a, st);
     }
 }
 
@@ -633,7 +709,7 @@ int dispatch_block(const BlockArgs &a, int64_t D, hipStream_t st) {
         // (kept on 32 tokens); the plain form is as fast or faster with 32 tokens everywhere.
         case 1: return HASH ? launch_block<1, HASH, 1, false, 1>(a, st) : launch_block<1, HASH, 2>(a, st);
         case 2: return HASH ? launch_block<2, HASH, 1, false, 1>(a, st) : launch_block<2, HASH, 2>(a, st);
-        case 4: return launch_block<4, HASH, 2>(a, st);
+        case 4: return wide(a) ? launch_block<4, HASH, 1, false, 1, 4>(a, st) : launch_block<4, HASH, 2>(a, st);
         case 8: return HASH ? launch_block<8, HASH, 1, false, 1>(a, st) : launch_block<8, HASH, 2>(a, st);
         // measured at 16384 x 1024: the plain form 110 us with 4 wavefronts, 118 us with 8 (the
         // second fetch of the weight fragments costs more than the other phases gain); the hash
@@ -655,8 +731,7 @@ extern "C" int lffn_bh4_fold_f32(const float *w, float *w_folded, int64_t R, int
     LFFN_REQUIRE(w && w_folded && w != w_folded, LFFN_ERR_BAD_ARG);
     const int64_t nblk = R * stages * num_block;
     LFFN_REQUIRE(nblk <= (int64_t(1) << 24), LFFN_ERR_UNSUPPORTED);
-    hipLaunchKernelGGL(bh4_fold_kernel<0>, dim3((unsigned)((nblk * BS + 255) / 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), w, w_folded, nblk);
+    hipLaunchKernelGGL(bh4_fold_kernel<0>, dim3((unsigned)nblk), dim3(BS), 0, static_cast<hipStream_t>(stream), w, w_folded);
     return lffn_launch_status();
 }
 
@@ -666,11 +741,11 @@ extern "C" int lffn_bh4_fold_mode_f32(const float *w, float *out, int64_t num_bl
     LFFN_REQUIRE(block_size == BS && mode >= 0 && mode <= 2, LFFN_ERR_UNSUPPORTED);
     if (num_blocks == 0) return LFFN_OK;
     LFFN_REQUIRE(w && out && w != out, LFFN_ERR_BAD_ARG);
-    const dim3 grid((unsigned)((num_blocks * BS + 255) / 256));
+    const dim3 grid((unsigned)num_blocks);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (mode == 0) hipLaunchKernelGGL(bh4_fold_kernel<0>, grid, dim3(256), 0, st, w, out, num_blocks);
-    else if (mode == 1) hipLaunchKernelGGL(bh4_fold_kernel<1>, grid, dim3(256), 0, st, w, out, num_blocks);
-    else hipLaunchKernelGGL(bh4_fold_kernel<2>, grid, dim3(256), 0, st, w, out, num_blocks);
+    if (mode == 0) hipLaunchKernelGGL(bh4_fold_kernel<0>, grid, dim3(BS), 0, st, w, out);
+    else if (mode == 1) hipLaunchKernelGGL(bh4_fold_kernel<1>, grid, dim3(BS), 0, st, w, out);
+    else hipLaunchKernelGGL(bh4_fold_kernel<2>, grid, dim3(BS), 0, st, w, out);
     return lffn_launch_status();
 }
 

@@ -30,7 +30,16 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BS = 64;
-constexpr int CHUNK = 512;        // tokens per workgroup
+// Tokens per workgroup: 512, or fewer where that leaves the chip idle (a batch of 385 tokens at 512 columns is 32
+// workgroups of 512; chunk_tokens).  More chunks are more atomic additions to the result, which at thousands of tokens
+// cost more than they bring (256 tokens instead of 512 at 16384 x 1024 measured slower).
+constexpr int CHUNK = 512, MIN_CHUNK = 64;
+constexpr int64_t CHUNK_WORKGROUPS = 512;
+int chunk_tokens(int64_t B, int64_t blocks) {
+    int chunk = CHUNK;
+    while (chunk > MIN_CHUNK && (B + chunk - 1) / chunk * blocks < CHUNK_WORKGROUPS) chunk /= 2;
+    return chunk;
+}
 constexpr int DEPTH = 4;          // token quads whose loads are in flight per wavefront
 
 __global__ __launch_bounds__(256) void bh4_wgrad_kernel(const float *__restrict__ stage_grads,
@@ -38,7 +47,7 @@ __global__ __launch_bounds__(256) void bh4_wgrad_kernel(const float *__restrict_
                                                         const float *__restrict__ stage_inputs,
                                                         float *__restrict__ g, int64_t B, int H, int D, int J,
                                                         const float *__restrict__ ln_w, const float *__restrict__ ln_b,
-                                                        const float *__restrict__ row_stats) {
+                                                        const float *__restrict__ row_stats, int chunk) {
     __shared__ float red[4][BS * BS / 4];          // a quarter of each wavefront's 64x64 tile
     const int n = blockIdx.y;
     const int s = blockIdx.z;                      // stage r * J + j
@@ -53,8 +62,8 @@ __global__ __launch_bounds__(256) void bh4_wgrad_kernel(const float *__restrict_
     const int wave = threadIdx.x >> 6;
     const int c = lane & 15;
     const int kq = lane >> 4;
-    const int64_t tok_lo = int64_t(blockIdx.x) * CHUNK + wave * (CHUNK / 4);
-    const int64_t tok_hi = min<int64_t>(tok_lo + CHUNK / 4, B);
+    const int64_t tok_lo = int64_t(blockIdx.x) * chunk + wave * (chunk / 4);
+    const int64_t tok_hi = min<int64_t>(tok_lo + chunk / 4, B);
     const int ucol = n * BS + 4 * c;
     const bool u_live = ucol < Hu;                 // Hu % 4 == 0: the four columns are all in or all out
     // LayerNorm on load (stage 0 only): this lane's four columns of the weight and bias
@@ -144,11 +153,12 @@ int wgrad_entry(const float *stage_grads, const float *x, const float *ln_weight
                  LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(!ln_weight || (ln_bias && row_stats && lffn_aligned16(ln_weight) && lffn_aligned16(ln_bias) &&
                                 (uintptr_t)row_stats % 8 == 0), LFFN_ERR_BAD_ARG);
-    const int64_t chunks = (B + CHUNK - 1) / CHUNK;
+    const int chunk = chunk_tokens(B, D / BS * R * J);
+    const int64_t chunks = (B + chunk - 1) / chunk;
     LFFN_REQUIRE(chunks <= 0x7fffffff && D / BS <= 65535, LFFN_ERR_UNSUPPORTED);
     hipLaunchKernelGGL(bh4_wgrad_kernel, dim3((unsigned)chunks, (unsigned)(D / BS), (unsigned)(R * J)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), stage_grads, x, stage_inputs, g_folded, B, (int)H, (int)D, (int)J,
-                       ln_weight, ln_bias, row_stats);
+                       ln_weight, ln_bias, row_stats, chunk);
     return lffn_launch_status();
 }
 

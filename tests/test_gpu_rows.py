@@ -164,3 +164,33 @@ def test_gather_of_few_tokens(B, T, S, Do, dtype):
         want, scale = want + products, scale + products.abs()
     got = ops.lookup_gather(code.cuda(), score.cuda(), tables.cuda(), bias.cuda(), res.cuda())
     assert ((got.cpu().double() - want).abs() <= (T + 8) * 2.0 ** -24 * scale).all()      # T + 8 additions in fp32
+
+
+# 64 x 64 blocks: few tokens and many take different forms of the kernel, which do the same additions in the same order
+@pytest.mark.parametrize("D,R", [(256, 1), (256, 2), (512, 1), (1024, 1)])
+def test_block_kernel_forms_agree(D, R):
+    rng = np.random.RandomState(D + R)
+    B, few, J, T = 16 * (256 // R) + 5, 37, 3, R * D // 8
+    w = (rng.randn(R, J, D // 64, 64, 64) / np.sqrt(64 * D)).astype(np.float32)
+    x, bias = rng.randn(B, D - 4).astype(np.float32), (0.05 * rng.randn(T * 8)).astype(np.float32)
+    lw, lb = (1 + 0.1 * rng.randn(D - 4)).astype(np.float32), (0.1 * rng.randn(D - 4)).astype(np.float32)
+    many = cabi.ln_bh4_block_train(x, lw, lb, 1e-5, w, bias, T)
+    for a, b in zip(many, cabi.ln_bh4_block_train(x[:few], lw, lb, 1e-5, w, bias, T)):
+        assert np.array_equal(a[:, :, :few] if a.ndim == 4 else a[:few], b)
+    assert np.array_equal(cabi.bh4_block(x, w)[0][:few], cabi.bh4_block(x[:few], w)[0])
+    g = rng.randn(B, T * 8).astype(np.float32)
+    for a, b in zip(cabi.bh4_block_bwd(g, w, D - 4), cabi.bh4_block_bwd(g[:few], w, D - 4)):
+        assert np.array_equal(a[..., :few, :], b)
+
+
+@pytest.mark.parametrize("B", [1, 63, 64, 65, 385, 1100])
+def test_block_weight_gradient_over_chunks(B):
+    """Chunks of 64 to 512 tokens: sums of B products in fp32, per element within B * 2^-24 of the sum of their magnitudes."""
+    rng = np.random.RandomState(B)
+    J, D = 2, 128
+    sg, x, si = (rng.randn(*s).astype(np.float32) for s in ((J, B, D), (B, D), (1, J - 1, B, D)))
+    u = np.stack([x, si[0, 0]]).astype(np.float64).reshape(J, B, D // 64, 64)
+    p = sg.astype(np.float64).reshape(J, B, D // 64, 64)
+    want, scale = np.einsum("jbno,jbni->jnoi", p, u), np.einsum("jbno,jbni->jnoi", np.abs(p), np.abs(u))
+    got = cabi.bh4_block_wgrad(sg, x, si, 1, J)
+    assert (np.abs(got - want) <= (B + 4) * 2.0 ** -24 * scale).all()
