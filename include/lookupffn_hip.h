@@ -660,6 +660,10 @@ int lffn_indexed_inner_product_f16(const int32_t *idx, const uint16_t *g, const 
 int lffn_scatter_add_f16(const int32_t *idx, const uint16_t *g, const float *w, float *out,
                          int64_t B, int64_t I, int64_t out_size, int64_t Dv, void *stream);
 
+/* Tokens up to which lffn_lookup_scatter_f32 sums every row of the gradient from a list of its tokens (tables of at most 256
+ * rows); up to there it is also faster than lffn_lookup_scatter_sorted_f32. */
+#define LFFN_SCATTER_LIST_TOKENS 2048
+
 /*
  * The scatter-add as the layer's backward issues it: table-local codes, the
  * gradient of the whole [T, S, Do] table array in one call,

@@ -478,6 +478,74 @@ __global__ __launch_bounds__(64 * WAVES) void token_gather_kernel(TokenCodes a) 
     token_gather<WAVES, FMT>(a.g, pairs, row, threadIdx.x >> 6, threadIdx.x & 63);
 }
 
+// The score gradient for small batches: grad_score[b,t] = <g[b,:], tables[t][code[b,t]][:]>, a token per workgroup of eight
+// wavefronts, which take an eighth of the tables each, eight rows together.  128 tables of 768 columns: 64 tokens 28.8 -> 7.0 us, 384
+// 32.1 -> 22.3 (1024 columns 34.0 -> 30.2, and at 512 tokens 35.7 -> 38.3: hence the limit); 512 tables of 1024 187 -> 31 and 193 -> 119.
+constexpr int64_t TOKEN_INNER_MAX = 384;
+struct TokenInner {
+    const int32_t *code;
+    const float *g;
+    const float *tables;
+    float *out;
+    int T, S, Do;
+    TableGuard guard;
+};
+
+template <int NC>
+__global__ __launch_bounds__(512) void token_inner_kernel(TokenInner a) {
+    if (table_guard_ends(a.guard)) return;
+    const int64_t row = blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int share = (a.T + 7) / 8, t_lo = min(wave * share, a.T), t_hi = min(t_lo + share, a.T);
+    const float *grow = a.g + row * a.Do;
+    for (int t0 = t_lo; t0 < t_hi; t0 += 8) {
+        float d[8];
+        const float *rows[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int t = min(t0 + u, t_hi - 1);
+            rows[u] = a.tables + ((size_t)t * a.S + (a.code[row * a.T + t] & (a.S - 1))) * a.Do;
+            d[u] = 0.f;
+        }
+        for (int col0 = 0; col0 < a.Do; col0 += 256 * NC) {
+            float4 gv[NC], rv[8][NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int col = col0 + 256 * c + 4 * lane;
+                gv[c] = col < a.Do ? *reinterpret_cast<const float4 *>(grow + col) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const int col = col0 + 256 * c + 4 * lane;
+                    rv[u][c] = *reinterpret_cast<const float4 *>(rows[u] + (col < a.Do ? col : 0));
+                }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int c = 0; c < NC; ++c)
+                    if (col0 + 256 * c + 4 * lane < a.Do) {
+                        d[u] = fmaf(gv[c].x, rv[u][c].x, d[u]); d[u] = fmaf(gv[c].y, rv[u][c].y, d[u]);
+                        d[u] = fmaf(gv[c].z, rv[u][c].z, d[u]); d[u] = fmaf(gv[c].w, rv[u][c].w, d[u]);
+                    }
+        }
+        // eight sums over 64 lanes: three exchanges halve the number of sums a lane works on, three more finish the one left
+        float q[4], h[2];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = ((lane & 1) ? d[u + 4] : d[u]) + lane_xor<1>((lane & 1) ? d[u] : d[u + 4]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) h[u] = ((lane & 2) ? q[u + 2] : q[u]) + lane_xor<2>((lane & 2) ? q[u] : q[u + 2]);
+        float v = ((lane & 4) ? h[1] : h[0]) + lane_xor<4>((lane & 4) ? h[0] : h[1]);
+        v += lane_xor<8>(v);
+        v += lane_xor<16>(v);
+        v += lane_xor<32>(v);
+        const int t = t0 + 4 * (lane & 1) + (lane & 2) + ((lane >> 2) & 1);
+        if (lane < 8 && t < t_hi) a.out[row * a.T + t] = v;
+    }
+}
+
 template <int FMT, int WAVES>
 int launch_token_gather(const TokenCodes &a, int64_t B, hipStream_t st) {
     hipLaunchKernelGGL((token_gather_kernel<FMT, WAVES>), dim3((unsigned)B), dim3(64 * WAVES), 0, st, a);
@@ -573,6 +641,21 @@ int lffn_internal_lookup_scatter_atomic(const int32_t *code, const float *score,
     a.idx = code; a.src = nullptr; a.w = score; a.g = g; a.bias = nullptr; a.out = out;
     a.B = B; a.I = (int)T; a.source_size = T * S; a.Dv = (int)Do; a.S = (int)S;
     return launch<LFFN_ROWS_F32, Op::Scatter>(a, static_cast<hipStream_t>(stream));
+}
+
+bool lffn_internal_lookup_inner_tokens_try(const int32_t *code, const float *g, const float *tables, float *out, int64_t B,
+                                           int64_t T, int64_t S, int64_t Do, void *stream, int *rc) {
+    if (B > TOKEN_INNER_MAX || T < 1 || T * S > 0x7fffffff) return false;
+    const TokenInner a{code, g, tables, out, (int)T, (int)S, (int)Do, lffn_table_guard()};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    switch ((Do + 255) / 256) {
+        case 1: hipLaunchKernelGGL(token_inner_kernel<1>, dim3((unsigned)B), dim3(512), 0, st, a); break;
+        case 2: hipLaunchKernelGGL(token_inner_kernel<2>, dim3((unsigned)B), dim3(512), 0, st, a); break;
+        case 3: hipLaunchKernelGGL(token_inner_kernel<3>, dim3((unsigned)B), dim3(512), 0, st, a); break;
+        default: hipLaunchKernelGGL(token_inner_kernel<4>, dim3((unsigned)B), dim3(512), 0, st, a); break;
+    }
+    *rc = lffn_launch_status();
+    return true;
 }
 
 // Token-major inner product on table-local codes: the fallback of lookup_inner.hip.

@@ -285,6 +285,7 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
     // fetched once per chunk and slice), and the form below when even 2 leaves most of it idle.
     {
         int rc = LFFN_OK;
+        if (lffn_internal_lookup_inner_tokens_try(code, g, tables, grad_score, B, T, S, Do, stream, &rc)) return rc;
         if (lffn_internal_lookup_inner_quad_try(code, g, Do, 32, tables, grad_score, B, T, S, Do, stream, &rc)) return rc;
     }
 

@@ -989,6 +989,8 @@ def _(indexes, source, weights, output_size):
 # Below this many multiply-adds (B * T * Do) the LDS-accumulating scatter is the faster one
 # (measured: 16384 x 32 x 768 and 16384 x 128 x 256 favour the sorted form, 2048 x 128 x 768 does not).
 SORTED_SCATTER_MIN_WORK = 4 * 10 ** 8
+# and up to this many tokens (LFFN_SCATTER_LIST_TOKENS of the C header) the one that sums rows from lists of their tokens is
+LIST_SCATTER_MAX_TOKENS = 2048
 
 _L.define("lookup_scatter(Tensor code, Tensor score, Tensor g, int S) -> Tensor")
 
@@ -1007,7 +1009,7 @@ def _lookup_scatter_impl(code, score, g, S):
     ws_bytes = ctypes.c_int64(0)
     _lib.check(lib.lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)), "lffn_lookup_scatter_workspace_bytes")
     with _dev_guard(g):
-        if ws_bytes.value > 0 and B * T * Do >= SORTED_SCATTER_MIN_WORK:
+        if ws_bytes.value > 0 and B > LIST_SCATTER_MAX_TOKENS and B * T * Do >= SORTED_SCATTER_MIN_WORK:
             # sort the tokens of every table by code, then sum rows in registers: no atomics
             ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=g.device)
             rc = lib.lffn_lookup_scatter_sorted_f32(_lib.ptr(code), _lib.ptr(score), _lib.ptr(g), _lib.ptr(out), _lib.ptr(ws),
@@ -1034,7 +1036,7 @@ _L.define("lookup_backward(Tensor code, Tensor score, Tensor g, Tensor tables) -
 def lookup_backward_is_fused(B, T, S, Do):
     """Both gradients of the gather go through one call (lffn_lookup_backward_f32: the sorted scatter and the
     score gradient sharing one slice-major copy of g) for this shape."""
-    if B * T * Do < SORTED_SCATTER_MIN_WORK or Do % 64 != 0:
+    if B <= LIST_SCATTER_MAX_TOKENS or B * T * Do < SORTED_SCATTER_MIN_WORK or Do % 64 != 0:
         return False
     ws_bytes = ctypes.c_int64(0)
     _lib.check(_lib.load().lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)),

@@ -194,3 +194,28 @@ def test_block_weight_gradient_over_chunks(B):
     want, scale = np.einsum("jbno,jbni->jnoi", p, u), np.einsum("jbno,jbni->jnoi", np.abs(p), np.abs(u))
     got = cabi.bh4_block_wgrad(sg, x, si, 1, J)
     assert (np.abs(got - want) <= (B + 4) * 2.0 ** -24 * scale).all()
+
+
+# Both gradients of the layer's gather for few tokens and just past it: row groups of 32 and smaller tables, column passes, every token
+# on one row, adding to what is there
+@pytest.mark.parametrize("B,T,S,Do", [(1, 1, 256, 64), (5, 9, 16, 320), (64, 3, 32, 1088), (384, 65, 256, 768), (385, 8, 128, 256),
+                                      (2048, 3, 256, 64), (2049, 3, 256, 64)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_gather_gradients_of_few_tokens(B, T, S, Do, skew):
+    rng = np.random.RandomState(B + T + S)
+    code = np.full((B, T), S - 1, np.int32) if skew else rng.randint(0, S, (B, T)).astype(np.int32)
+    score, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    tables, init = rng.randn(T, S, Do).astype(np.float32), rng.randn(T, S, Do).astype(np.float32)
+    want, scale = np.zeros((T, S, Do)), np.zeros((T, S, Do))
+    for t in range(T):
+        products = score[:, t, None].astype(np.float64) * g
+        np.add.at(want[t], code[:, t], products)
+        np.add.at(scale[t], code[:, t], np.abs(products))
+    # products rounded to fp32, summed in fp64, the sum (and the one onto `init`) rounded to fp32
+    assert (np.abs(cabi.lookup_scatter(code, score, g, S) - want) <= 2 * 2.0 ** -24 * scale).all()
+    got = cabi.lookup_scatter(code, score, g, S, accumulate=True, init=init)
+    assert (np.abs(got - want - init) <= 3 * 2.0 ** -24 * (scale + np.abs(init))).all()
+    rows = tables[np.arange(T)[None], code].astype(np.float64)                               # [B, T, Do]
+    inner = np.einsum("btd,bd->bt", rows, g.astype(np.float64))
+    bound = (Do + 8) * 2.0 ** -24 * np.einsum("btd,bd->bt", np.abs(rows), np.abs(g).astype(np.float64))
+    assert (np.abs(cabi.lookup_inner(code, g, tables) - inner) <= bound).all()
