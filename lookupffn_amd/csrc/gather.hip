@@ -463,9 +463,13 @@ int gather_entry(const int32_t *idx, const void *src, const float *w, const floa
 struct TokenCodes {
     const int32_t *code;
     const float *score;
-    TokenGatherArgs g;
+    TokenGatherArgs g;    // S == 0: flat row numbers, clamped into [0, last_row]
+    int last_row;
     TableGuard guard;
 };
+
+__device__ __forceinline__ int token_row(int raw, int S, int last_row) { return S ? raw & (S - 1) : min(max(raw, 0), last_row); }
+
 
 template <int FMT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void token_gather_kernel(TokenCodes a) {
@@ -473,63 +477,79 @@ __global__ __launch_bounds__(64 * WAVES) void token_gather_kernel(TokenCodes a) 
     __shared__ uint2 pairs[TOKEN_MAX_T];
     const int64_t row = blockIdx.x;
     for (int t = threadIdx.x; t < a.g.T; t += 64 * WAVES)
-        pairs[t] = make_uint2((unsigned)a.code[row * a.g.T + t] & (unsigned)(a.g.S - 1), __float_as_uint(a.score[row * a.g.T + t]));
+        pairs[t] = make_uint2((unsigned)token_row(a.code[row * a.g.T + t], a.g.S, a.last_row), __float_as_uint(a.score[row * a.g.T + t]));
     __syncthreads();
     token_gather<WAVES, FMT>(a.g, pairs, row, threadIdx.x >> 6, threadIdx.x & 63);
 }
 
-// The score gradient for small batches: grad_score[b,t] = <g[b,:], tables[t][code[b,t]][:]>, a token per workgroup of eight
+// The score gradient (and the inner product on flat row numbers) for small batches:
+// grad_score[b,t] = <g[b,:], tables[t][code[b,t]][:]>, a token per workgroup of eight
 // wavefronts, which take an eighth of the tables each, eight rows together.  128 tables of 768 columns: 64 tokens 28.8 -> 7.0 us, 384
 // 32.1 -> 22.3 (1024 columns 34.0 -> 30.2, and at 512 tokens 35.7 -> 38.3: hence the limit); 512 tables of 1024 187 -> 31 and 193 -> 119.
 constexpr int64_t TOKEN_INNER_MAX = 384;
 struct TokenInner {
     const int32_t *code;
-    const float *g;
-    const float *tables;
+    const void *g;
+    const void *tables;
     float *out;
-    int T, S, Do;
+    int T, S, Do;         // S == 0: flat row numbers, clamped into [0, last_row]
+    int last_row;
     TableGuard guard;
 };
 
-template <int NC>
+// d + <g, v> over four columns, column ascending, products and sums in fp32
+template <int FMT>
+__device__ __forceinline__ float dot_quad(const RowQuad<FMT> &g, const RowQuad<FMT> &v, float d) {
+    if constexpr (FMT == LFFN_ROWS_F32) {
+        d = fmaf(g.x, v.x, d); d = fmaf(g.y, v.y, d); d = fmaf(g.z, v.z, d); d = fmaf(g.w, v.w, d);
+    } else {
+        static_assert(FMT == LFFN_ROWS_F16, "fp32 or half");
+        const half2_t a = __builtin_bit_cast(half2_t, g.x), b = __builtin_bit_cast(half2_t, g.y);
+        const half2_t x = __builtin_bit_cast(half2_t, v.x), y = __builtin_bit_cast(half2_t, v.y);
+        d = fmaf((float)a.x, (float)x.x, d); d = fmaf((float)a.y, (float)x.y, d);
+        d = fmaf((float)b.x, (float)y.x, d); d = fmaf((float)b.y, (float)y.y, d);
+    }
+    return d;
+}
+
+template <int FMT, int NC>
 __global__ __launch_bounds__(512) void token_inner_kernel(TokenInner a) {
+    using Quad = RowQuad<FMT>;
+    constexpr int ESZ = FMT == LFFN_ROWS_F32 ? 4 : 2;
     if (table_guard_ends(a.guard)) return;
     const int64_t row = blockIdx.x;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int share = (a.T + 7) / 8, t_lo = min(wave * share, a.T), t_hi = min(t_lo + share, a.T);
-    const float *grow = a.g + row * a.Do;
+    const char *grow = static_cast<const char *>(a.g) + row * a.Do * ESZ;
     for (int t0 = t_lo; t0 < t_hi; t0 += 8) {
         float d[8];
-        const float *rows[8];
+        const char *rows[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int t = min(t0 + u, t_hi - 1);
-            rows[u] = a.tables + ((size_t)t * a.S + (a.code[row * a.T + t] & (a.S - 1))) * a.Do;
+            rows[u] = static_cast<const char *>(a.tables) + ((size_t)t * a.S + token_row(a.code[row * a.T + t], a.S, a.last_row)) * a.Do * ESZ;
             d[u] = 0.f;
         }
         for (int col0 = 0; col0 < a.Do; col0 += 256 * NC) {
-            float4 gv[NC], rv[8][NC];
+            Quad gv[NC], rv[8][NC];
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
                 const int col = col0 + 256 * c + 4 * lane;
-                gv[c] = col < a.Do ? *reinterpret_cast<const float4 *>(grow + col) : make_float4(0.f, 0.f, 0.f, 0.f);
+                gv[c] = *reinterpret_cast<const Quad *>(grow + (col < a.Do ? col : 0) * ESZ);
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u)
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
                     const int col = col0 + 256 * c + 4 * lane;
-                    rv[u][c] = *reinterpret_cast<const float4 *>(rows[u] + (col < a.Do ? col : 0));
+                    rv[u][c] = *reinterpret_cast<const Quad *>(rows[u] + (col < a.Do ? col : 0) * ESZ);
                 }
 #pragma unroll
             for (int u = 0; u < 8; ++u)
 #pragma unroll
                 for (int c = 0; c < NC; ++c)
-                    if (col0 + 256 * c + 4 * lane < a.Do) {
-                        d[u] = fmaf(gv[c].x, rv[u][c].x, d[u]); d[u] = fmaf(gv[c].y, rv[u][c].y, d[u]);
-                        d[u] = fmaf(gv[c].z, rv[u][c].z, d[u]); d[u] = fmaf(gv[c].w, rv[u][c].w, d[u]);
-                    }
+                    if (col0 + 256 * c + 4 * lane < a.Do) d[u] = dot_quad<FMT>(gv[c], rv[u][c], d[u]);
         }
         // eight sums over 64 lanes: three exchanges halve the number of sums a lane works on, three more finish the one left
         float q[4], h[2];
@@ -546,10 +566,30 @@ __global__ __launch_bounds__(512) void token_inner_kernel(TokenInner a) {
     }
 }
 
+template <int FMT>
+void launch_token_inner(const TokenInner &a, int64_t B, void *stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const dim3 grid((unsigned)B), block(512);
+    switch ((a.Do + 255) / 256) {
+        case 1: hipLaunchKernelGGL((token_inner_kernel<FMT, 1>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((token_inner_kernel<FMT, 2>), grid, block, 0, st, a); break;
+        case 3: hipLaunchKernelGGL((token_inner_kernel<FMT, 3>), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((token_inner_kernel<FMT, 4>), grid, block, 0, st, a); break;
+    }
+}
+
 template <int FMT, int WAVES>
 int launch_token_gather(const TokenCodes &a, int64_t B, hipStream_t st) {
     hipLaunchKernelGGL((token_gather_kernel<FMT, WAVES>), dim3((unsigned)B), dim3(64 * WAVES), 0, st, a);
     return lffn_launch_status();
+}
+
+int launch_token_gather(const TokenCodes &a, int64_t B, int fmt, void *stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool wide = B <= TOKEN_WIDE_MAX;
+    if (fmt == LFFN_ROWS_F16) return wide ? launch_token_gather<LFFN_ROWS_F16, 8>(a, B, st) : launch_token_gather<LFFN_ROWS_F16, 4>(a, B, st);
+    if (fmt == LFFN_ROWS_BF16) return wide ? launch_token_gather<LFFN_ROWS_BF16, 8>(a, B, st) : launch_token_gather<LFFN_ROWS_BF16, 4>(a, B, st);
+    return wide ? launch_token_gather<LFFN_ROWS_F32, 8>(a, B, st) : launch_token_gather<LFFN_ROWS_F32, 4>(a, B, st);
 }
 
 // Up to this many tokens (layer, 128 tables of 768 columns, 64 tokens: fp32 27.6 -> 15.6 us, bfloat16 34.4 -> 14.7; 512 tables of
@@ -584,6 +624,10 @@ int lffn_internal_inner_flat(const int32_t *idx, const float *g, const float *sr
     GatherArgs a{};
     a.idx = idx; a.src = src; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
     a.B = B; a.I = (int)I; a.source_size = source_size; a.Dv = (int)Dv; a.S = 0; a.guard = TableGuard{flags, 0};
+    if (B >= 1 && B <= TOKEN_INNER_MAX && I >= 1) {
+        launch_token_inner<LFFN_ROWS_F32>(TokenInner{idx, g, src, out, (int)I, 0, (int)Dv, (int)(source_size - 1), a.guard}, B, stream);
+        return lffn_launch_status();
+    }
     return launch<LFFN_ROWS_F32, Op::Inner>(a, static_cast<hipStream_t>(stream));
 }
 
@@ -622,15 +666,23 @@ int lffn_internal_lookup_gather_token_major(const int32_t *code, const float *sc
 int lffn_internal_lookup_gather_tokens(const int32_t *code, const float *score, const void *tables, const float *bias,
                                        const float *residual, float *out, int64_t B, int64_t T, int64_t S, int64_t Do,
                                        int fmt, void *stream) {
-    if (B <= token_gather_max(fmt, Do) && T >= 1 && T <= TOKEN_MAX_T && S > 0 && B * T * S > 0) {
-        const TokenCodes a{code, score, TokenGatherArgs{tables, bias, residual, out, (int)T, (int)S, (int)Do}, lffn_table_guard()};
-        hipStream_t st = static_cast<hipStream_t>(stream);
-        const bool wide = B <= TOKEN_WIDE_MAX;
-        if (fmt == LFFN_ROWS_F16) return wide ? launch_token_gather<LFFN_ROWS_F16, 8>(a, B, st) : launch_token_gather<LFFN_ROWS_F16, 4>(a, B, st);
-        if (fmt == LFFN_ROWS_BF16) return wide ? launch_token_gather<LFFN_ROWS_BF16, 8>(a, B, st) : launch_token_gather<LFFN_ROWS_BF16, 4>(a, B, st);
-        return wide ? launch_token_gather<LFFN_ROWS_F32, 8>(a, B, st) : launch_token_gather<LFFN_ROWS_F32, 4>(a, B, st);
-    }
+    if (B <= token_gather_max(fmt, Do) && T >= 1 && T <= TOKEN_MAX_T && S > 0 && B * T * S > 0)
+        return launch_token_gather(TokenCodes{code, score, TokenGatherArgs{tables, bias, residual, out, (int)T, (int)S, (int)Do}, 0,
+                                              lffn_table_guard()}, B, fmt, stream);
     return lffn_internal_lookup_gather_token_major(code, score, tables, bias, residual, out, B, T, S, Do, fmt, stream);
+}
+
+// weighted_gather_add on flat row numbers where the choice of kernel is open: as above for few tokens
+int lffn_internal_gather_add_tokens(const int32_t *idx, const void *src, const float *w, float *out, int64_t B, int64_t I,
+                                    int64_t source_size, int64_t Dv, int fmt, const int32_t *flags, void *stream) {
+    if (B >= 1 && B <= token_gather_max(fmt, Dv) && I >= 1 && I <= TOKEN_MAX_T) {
+        const int rc = check_common(idx, B, I, source_size, Dv);
+        if (rc != LFFN_OK) return rc;
+        LFFN_REQUIRE(src && w && out && lffn_aligned16(src) && lffn_aligned16(out), LFFN_ERR_BAD_ARG);
+        return launch_token_gather(TokenCodes{idx, w, TokenGatherArgs{src, nullptr, nullptr, out, (int)I, 0, (int)Dv},
+                                              (int)(source_size - 1), TableGuard{flags, 0}}, B, fmt, stream);
+    }
+    return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, fmt, flags, stream);
 }
 
 // Atomic scatter-add on table-local codes (row = code & (S-1) + t*S), into a buffer
@@ -646,14 +698,7 @@ int lffn_internal_lookup_scatter_atomic(const int32_t *code, const float *score,
 bool lffn_internal_lookup_inner_tokens_try(const int32_t *code, const float *g, const float *tables, float *out, int64_t B,
                                            int64_t T, int64_t S, int64_t Do, void *stream, int *rc) {
     if (B > TOKEN_INNER_MAX || T < 1 || T * S > 0x7fffffff) return false;
-    const TokenInner a{code, g, tables, out, (int)T, (int)S, (int)Do, lffn_table_guard()};
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    switch ((Do + 255) / 256) {
-        case 1: hipLaunchKernelGGL(token_inner_kernel<1>, dim3((unsigned)B), dim3(512), 0, st, a); break;
-        case 2: hipLaunchKernelGGL(token_inner_kernel<2>, dim3((unsigned)B), dim3(512), 0, st, a); break;
-        case 3: hipLaunchKernelGGL(token_inner_kernel<3>, dim3((unsigned)B), dim3(512), 0, st, a); break;
-        default: hipLaunchKernelGGL(token_inner_kernel<4>, dim3((unsigned)B), dim3(512), 0, st, a); break;
-    }
+    launch_token_inner<LFFN_ROWS_F32>(TokenInner{code, g, tables, out, (int)T, (int)S, (int)Do, 0, lffn_table_guard()}, B, stream);
     *rc = lffn_launch_status();
     return true;
 }
@@ -695,6 +740,10 @@ extern "C" int lffn_indexed_inner_product_f16(const int32_t *idx, const uint16_t
     GatherArgs a{};
     a.idx = idx; a.src = src; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
     a.B = B; a.I = (int)I; a.source_size = source_size; a.Dv = (int)Dv; a.S = 0;
+    if (B >= 1 && B <= TOKEN_INNER_MAX && I >= 1) {
+        launch_token_inner<LFFN_ROWS_F16>(TokenInner{idx, g, src, out, (int)I, 0, (int)Dv, (int)(source_size - 1), TableGuard{}}, B, stream);
+        return lffn_launch_status();
+    }
     return launch<LFFN_ROWS_F16, Op::Inner>(a, static_cast<hipStream_t>(stream));
 }
 

@@ -41,10 +41,14 @@ int lffn_internal_lookup_gather_tokens(const int32_t *code, const float *score, 
                                        int fmt, void *stream);
 
 // gather.hip: the token-major operators on flat row numbers; with flags (see TableGuard) the launch is for arrays
-// that are not in table form.  table_form writes those flags (TABLE_FLAGS words).
+// that are not in table form; gather_add_tokens takes few tokens a workgroup each, where the choice of kernel is open.
+// table_form writes those flags (TABLE_FLAGS words).
 __attribute__((visibility("hidden")))
 int lffn_internal_gather_add_flat(const int32_t *idx, const void *src, const float *w, float *out, int64_t B, int64_t I,
                                   int64_t source_size, int64_t Dv, int fmt, const int32_t *flags, void *stream);
+__attribute__((visibility("hidden")))
+int lffn_internal_gather_add_tokens(const int32_t *idx, const void *src, const float *w, float *out, int64_t B, int64_t I,
+                                    int64_t source_size, int64_t Dv, int fmt, const int32_t *flags, void *stream);
 __attribute__((visibility("hidden")))
 int lffn_internal_inner_flat(const int32_t *idx, const float *g, const float *src, float *out, int64_t B, int64_t I,
                              int64_t source_size, int64_t Dv, const int32_t *flags, void *stream);

@@ -997,7 +997,7 @@ extern "C" int lffn_gather_add_ws_rows(const int32_t *idx, const void *src, cons
     int64_t need = 0;
     lffn_gather_add_workspace_bytes(B, I, source_size, Dv, row_format, &need);
     if (need == 0 || workspace_bytes < need)
-        return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, row_format, nullptr, stream);
+        return lffn_internal_gather_add_tokens(idx, src, w, out, B, I, source_size, Dv, row_format, nullptr, stream);
     LFFN_REQUIRE(idx && src && w && out && lffn_aligned16(workspace), LFFN_ERR_BAD_ARG);
     int32_t *flags = static_cast<int32_t *>(workspace);
     int rc = lffn_internal_table_form(idx, flags, B, I, stream);
@@ -1014,5 +1014,5 @@ extern "C" int lffn_gather_add_ws_rows(const int32_t *idx, const void *src, cons
             rc = lookup_gather_entry<false>(idx, w, src, nullptr, nullptr, out, B, I, MAX_S, Dv, -1, 0, stream, ws, ws_bytes);
     }
     if (rc != LFFN_OK) return rc;
-    return lffn_internal_gather_add_flat(idx, src, w, out, B, I, source_size, Dv, row_format, flags, stream);
+    return lffn_internal_gather_add_tokens(idx, src, w, out, B, I, source_size, Dv, row_format, flags, stream);
 }

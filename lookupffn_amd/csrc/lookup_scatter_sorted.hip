@@ -695,13 +695,14 @@ struct RowsWorkspace {
     int64_t count, rank, off8, pairs, g_packed, total;
 };
 
-// Worth it from 6e6 products on (five launches, about 30 us of them whatever the size, against 79 G atomics/s) and while
+// Worth it from 3e6 products on (five launches, about 30 us of them whatever the size, against 79 G atomics/s; forward and backward at 512
+// tokens of 32 x 256, 4e6 products: fp32 75 -> 71 us, half 155 -> 99; at 128 x 512, 64 tokens 104 -> 73 and 219 -> 99) and while
 // the list that every slice reads is in proportion: at least one pair for every four rows of the output.
 bool rows_supported(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
     if (B < 1 || I < 1 || rows < 1 || Dv < SC || Dv % SC != 0 || Dv > (1 << 20)) return false;
     const int64_t Bc = B < CHUNK ? B : CHUNK, tables = (rows + VT - 1) / VT;
     return Bc * I < (int64_t(1) << 31) - 8 * 256 && rows <= (int64_t(1) << 30) && B * I * 4 >= rows &&
-           double(B) * double(I) * double(Dv) >= 6e6 && tables * ((Dv / SC + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff &&
+           double(B) * double(I) * double(Dv) >= 3e6 && tables * ((Dv / SC + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff &&
            Bc * Dv / 1024 < (int64_t(1) << 30);
 }
 

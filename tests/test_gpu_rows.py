@@ -219,3 +219,19 @@ def test_gather_gradients_of_few_tokens(B, T, S, Do, skew):
     inner = np.einsum("btd,bd->bt", rows, g.astype(np.float64))
     bound = (Do + 8) * 2.0 ** -24 * np.einsum("btd,bd->bt", np.abs(rows), np.abs(g).astype(np.float64))
     assert (np.abs(cabi.lookup_inner(code, g, tables) - inner) <= bound).all()
+
+
+# Flat row numbers, few tokens: numbers outside the source are clamped, any source size, more columns than go together
+@pytest.mark.parametrize("B,I,rows,Dv", [(1, 1, 1, 64), (3, 70, 999, 320), (256, 16, 100, 1088), (385, 9, 4000, 128), (513, 9, 4000, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_operators_on_flat_rows_of_few_tokens(B, I, rows, Dv, dtype):
+    gen = torch.Generator().manual_seed(B + I)
+    idx = torch.randint(-3, rows + 3, (B, I), generator=gen, dtype=torch.int32)
+    src, g, w = (torch.randn(*s, generator=gen).to(dtype) for s in ((rows, Dv), (B, Dv), (B, I)))
+    picked = src.double()[idx.long().clamp(0, rows - 1)]                                     # [B, I, Dv]
+    want, scale = ((f(picked) * f(w.double())[:, :, None]).sum(1) for f in (lambda t: t, torch.abs))
+    got = ops.gather_add(idx.cuda(), src.cuda(), w.float().cuda()).cpu().double()
+    assert ((got - want).abs() <= (I + 8) * 2.0 ** -24 * scale).all()
+    want, scale = ((f(picked) * f(g.double())[:, None]).sum(2) for f in (lambda t: t, torch.abs))
+    got = ops.indexed_inner_product(idx.cuda(), g.cuda(), src.cuda()).cpu().double()
+    assert ((got - want).abs() <= (Dv + 8) * 2.0 ** -24 * scale).all()
