@@ -691,6 +691,116 @@ __global__ __launch_bounds__(256) void rows_place_kernel(RowsArgs a) {
     }
 }
 
+// The rows' sums where rows have few pairs or none (SPARSE_PAIRS on average or fewer): a wavefront adds up a row at a time over
+// all its columns from g as it lies and writes it whole.  The slice-by-slice accumulation above reads every row's list once per 32
+// columns, which for rows of a few pairs is most of its time.  All five launches, 64 tokens: 128 tables of 768 columns 55 -> 29 us,
+// 512 of 1024 217 -> 125 us (537 MB written: 4.3 TB/s); 8 pairs a row, 2048 tokens of 128 x 512: 92 -> 60 us; 16 pairs a row 128 us
+// either way, hence the limit.  A row of more than LONG_ROW pairs goes to the whole workgroup; with half of all pairs on one row a single
+// compute unit's reads of g bound it (512 tokens of 128 x 768: 516 us by slices, 1283 so; fp32 atomics on one row are slower yet).
+constexpr int64_t SPARSE_PAIRS = 8;
+constexpr int LONG_ROW = 32;
+constexpr int ROW_GROUP = 32;                         // rows of a workgroup
+
+// acc += the pairs [i0, n) of a row, 64 at a time with `step` from one 64 to the next: a pair per lane, read from there
+template <typename G, int NC, int U>
+__device__ __forceinline__ void add_pairs(float4 (&acc)[NC], const G *g, const uint2 *list, int i0, int n, int step, int Dv, int col0,
+                                          int lane) {
+    for (int base = i0; base < n; base += step) {
+        const int m = min(64, n - base);
+        const uint2 mine = list[base + min(lane, m - 1)];
+        for (int k = 0; k < m; k += U) {
+            float4 v[U][NC];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const G *p = g + (size_t)(unsigned)__builtin_amdgcn_readlane((int)mine.x, min(k + u, m - 1)) * Dv;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) v[u][c] = load4(p + (col0 + 256 * c < Dv ? col0 + 256 * c : 0));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k + u < m) {                              // uniform
+                    const float s = __int_as_float(__builtin_amdgcn_readlane((int)mine.y, k + u));
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) {
+                        acc[c].x = fmaf(s, v[u][c].x, acc[c].x); acc[c].y = fmaf(s, v[u][c].y, acc[c].y);
+                        acc[c].z = fmaf(s, v[u][c].z, acc[c].z); acc[c].w = fmaf(s, v[u][c].w, acc[c].w);
+                    }
+                }
+        }
+    }
+}
+
+template <typename G, int NC>
+__global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, int accumulate) {
+    __shared__ float4 part[4][NC][64];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t first = int64_t(blockIdx.x) * ROW_GROUP;
+    const int nrows = (int)min<int64_t>(ROW_GROUP, a.rows - first);
+    const G *g = static_cast<const G *>(a.g);
+    // counts and list positions of the workgroup's rows, a row per lane
+    const int64_t my_row = first + min(lane, nrows - 1);
+    const int my_count = a.count[my_row], my_off = a.off8[(my_row / VT) * (VT + 1) + my_row % VT];
+    auto list_of = [&](int r) { return a.pairs + (int64_t)__builtin_amdgcn_readlane(my_off, r) * 8; };
+    auto store = [&](int r, int col, float4 v) {
+        float4 *dst = reinterpret_cast<float4 *>(out + (first + r) * a.Dv + col);
+        if (accumulate) {
+            const float4 old = *dst;
+            v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+        }
+        *dst = v;
+    };
+    for (int col0 = 4 * lane; col0 - 4 * lane < a.Dv; col0 += 256 * NC) {
+        for (int r = wave; r < nrows; r += 4) {
+            const int n = __builtin_amdgcn_readlane(my_count, r);
+            if (n > LONG_ROW) continue;
+            float4 acc[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+            add_pairs<G, NC, 4>(acc, g, list_of(r), 0, n, 64, a.Dv, col0, lane);
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                if (col0 + 256 * c < a.Dv) store(r, col0 + 256 * c, acc[c]);
+        }
+        for (int r = 0; r < nrows; ++r) {                     // (the counts are the same for every wavefront)
+            const int n = __builtin_amdgcn_readlane(my_count, r);
+            if (n <= LONG_ROW) continue;
+            float4 acc[NC];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+            add_pairs<G, NC, 8>(acc, g, list_of(r), 64 * wave, n, 256, a.Dv, col0, lane);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) part[wave][c][lane] = acc[c];
+            __syncthreads();
+            if (wave == 0) {
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    float4 v = part[0][c][lane];
+#pragma unroll
+                    for (int w = 1; w < 4; ++w) {
+                        const float4 q = part[w][c][lane];
+                        v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
+                    }
+                    if (col0 + 256 * c < a.Dv) store(r, col0 + 256 * c, v);
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+template <typename G>
+int launch_rows_sum(const RowsArgs &a, float *out, int accumulate, hipStream_t st) {
+    const dim3 grid((unsigned)((a.rows + ROW_GROUP - 1) / ROW_GROUP));
+    switch ((a.Dv + 255) / 256) {
+        case 1: hipLaunchKernelGGL((rows_sum_kernel<G, 1>), grid, dim3(256), 0, st, a, out, accumulate); break;
+        case 2: hipLaunchKernelGGL((rows_sum_kernel<G, 2>), grid, dim3(256), 0, st, a, out, accumulate); break;
+        case 3: hipLaunchKernelGGL((rows_sum_kernel<G, 3>), grid, dim3(256), 0, st, a, out, accumulate); break;
+        default: hipLaunchKernelGGL((rows_sum_kernel<G, 4>), grid, dim3(256), 0, st, a, out, accumulate); break;
+    }
+    return lffn_launch_status();
+}
+
 struct RowsWorkspace {
     int64_t count, rank, off8, pairs, g_packed, total;
 };
@@ -752,7 +862,8 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         a.tables = (int)((out_size + VT - 1) / VT);
         const int64_t blocks = (a.n + 255) / 256;
         a.place_blocks = (int)(blocks < 4096 ? blocks : 4096);
-        const int64_t pack_blocks = (a.B * (Dv / 4) + 1023) / 1024;
+        const bool sparse = a.n <= SPARSE_PAIRS * out_size;      // (no slice-major copy of g)
+        const int64_t pack_blocks = sparse ? 0 : (a.B * (Dv / 4) + 1023) / 1024;
         const int64_t zero4 = l.rank / 16;                      // the counters and the list's end
         hipLaunchKernelGGL(rows_zero_kernel, dim3((unsigned)((zero4 + 255) / 256 < 1024 ? (zero4 + 255) / 256 : 1024)), dim3(256), 0, st,
                            reinterpret_cast<int4 *>(base), zero4);
@@ -763,6 +874,12 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         else hipLaunchKernelGGL(rows_place_kernel<float>, grid, dim3(256), 0, st, a);
         int rc = lffn_launch_status();
         if (rc != LFFN_OK) return rc;
+        if (sparse) {
+            const int add = (accumulate || c0 > 0) ? 1 : 0;
+            rc = g_format == LFFN_ROWS_F16 ? launch_rows_sum<_Float16>(a, out, add, st) : launch_rows_sum<float>(a, out, add, st);
+            if (rc != LFFN_OK) return rc;
+            continue;
+        }
         SortedArgs ma{};
         ma.pairs = a.pairs; ma.off8 = a.off8; ma.g = a.g_packed; ma.out = out; ma.stride = 0; ma.rows = out_size;
         ma.last_token = (unsigned)(a.B - 1);

@@ -235,3 +235,23 @@ def test_operators_on_flat_rows_of_few_tokens(B, I, rows, Dv, dtype):
     want, scale = ((f(picked) * f(g.double())[:, None]).sum(2) for f in (lambda t: t, torch.abs))
     got = ops.indexed_inner_product(idx.cuda(), g.cuda(), src.cuda()).cpu().double()
     assert ((got - want).abs() <= (Dv + 8) * 2.0 ** -24 * scale).all()
+
+
+# Rows' gradient where rows have few pairs: groups of 32 rows and what is left of one, empty rows, rows of 1, 32, 33 and hundreds of pairs,
+# column passes, the average at and past the limit of 8 pairs a row
+@pytest.mark.parametrize("B,I,rows,Dv", [(700, 32, 4007, 320), (512, 32, 2048, 192), (600, 32, 2048, 192), (96, 40, 3000, 1088)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_rows_gradient_of_few_pairs(B, I, rows, Dv, dtype):
+    gen = torch.Generator().manual_seed(B + I)
+    idx = torch.randint(40, rows, (B, I), generator=gen, dtype=torch.int32)
+    flat = idx.view(-1)
+    flat[:600], flat[600:632], flat[632:665], flat[665] = 1, 2, 3, rows - 1
+    g, w = torch.randn(B, Dv, generator=gen).to(dtype), torch.randn(B, I, generator=gen).to(dtype)
+    want, scale = torch.zeros(rows, Dv, dtype=torch.double), torch.zeros(rows, Dv, dtype=torch.double)
+    for i in range(I):
+        products = w[:, i].double()[:, None] * g.double()
+        want.index_add_(0, idx[:, i].long(), products)
+        scale.index_add_(0, idx[:, i].long(), products.abs())
+    got = ops.scatter_add(idx.cuda(), g.cuda(), w.float().cuda(), rows).cpu().double()
+    n = torch.bincount(flat.long(), minlength=rows).double()[:, None]
+    assert ((got - want).abs() <= (n + 4) * 2.0 ** -24 * scale).all()                # n additions in fp32
