@@ -8,12 +8,15 @@
 //
 // Python builds a handle (make_layer) when the parameters are of a kind the kernels are built for, and calls
 // forward(handle, x, residual, ...).  The answer is None whenever anything is not as the handle expects: another parameter
-// object, storage or dtype, an input of another type, dtype, device or layout, a gradient wanted that this path does not
+// object, storage, dtype, sizes or strides, an input of another type, dtype, device or layout, a gradient wanted that this path does not
 // compute.  Then the Python path runs, with its own checks and errors.
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -94,6 +97,11 @@ struct Watched {
     PyObject *dict, *key, *object;
     const void *data;
     at::ScalarType dtype;
+    std::vector<int64_t> sizes, strides;
+
+    bool same(const Tensor &t) const {
+        return t.data_ptr() == data && t.scalar_type() == dtype && t.sizes().equals(sizes) && t.strides().equals(strides);
+    }
 };
 
 struct Layer {
@@ -370,7 +378,16 @@ bool plain(PyObject *o) {
     const Tensor &t = THPVariable_Unpack(o);
     constexpr c10::DispatchKeySet other({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
                                          c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
-    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(other);
+    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(other) && !t._fw_grad(/*level=*/0).defined();
+}
+
+// Somebody watches the operators that are called: a tracer, a mode of torch.overrides or torch.utils._python_dispatch, a
+// transform of torch.func.  They see them on the Python path.
+bool watched_over() {
+    return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize);
 }
 
 PyObject *bind_library(PyObject *, PyObject *path) {
@@ -409,8 +426,14 @@ PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
         TORCH_CHECK(o && (o == Py_None || THPVariable_Check(o)), "make_layer: a parameter is missing");
         if (o != Py_None) l->p[i] = THPVariable_Unpack(o);
         for (PyObject *k : {dict, key, o}) Py_INCREF(k);
-        l->watched.push_back(Watched{dict, key, o, l->p[i].defined() ? l->p[i].data_ptr() : nullptr,
-                                     l->p[i].defined() ? l->p[i].scalar_type() : at::kFloat});
+        Watched w{dict, key, o, nullptr, at::kFloat, {}, {}};
+        if (const Tensor &t = l->p[i]; t.defined()) {
+            w.data = t.data_ptr();
+            w.dtype = t.scalar_type();
+            w.sizes = t.sizes().vec();
+            w.strides = t.strides().vec();
+        }
+        l->watched.push_back(std::move(w));
     }
     if (args[3] != Py_None) {
         l->folded_dict = PyTuple_GET_ITEM(args[3], 0);
@@ -436,7 +459,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     Layer *l = static_cast<Layer *>(PyCapsule_GetPointer(args[0], CAPSULE));
     if (!l) return nullptr;
     const Config &c = l->c;
-    if (!plain(args[1])) Py_RETURN_NONE;
+    if (watched_over() || !plain(args[1])) Py_RETURN_NONE;
     const Tensor &x = THPVariable_Unpack(args[1]);
     const at::Device dev = l->p[4].device();
     const int64_t dims = x.dim();
@@ -463,7 +486,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (PyDict_GetItem(w.dict, w.key) != w.object) Py_RETURN_NONE;
         const Tensor &p = l->p[i];
         if (!p.defined()) continue;
-        if (p.data_ptr() != w.data || p.scalar_type() != w.dtype) Py_RETURN_NONE;
+        if (!w.same(p)) Py_RETURN_NONE;
         if (grad_mode) grads = grads || p.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;

@@ -459,6 +459,8 @@ class LookupFFN(nn.Module):
         known = self.__dict__.get("_handle_key")
         if known is None or known[0] is not st or (fold and known[1] is not key[1]):
             self._handle, self._handle_key = self._make_handle(st, key[1]), key
+        if self._handle is None:
+            return None
         return _lib.host().forward(self._handle, x.contiguous(), None if residual is None else residual.contiguous(),
                                    self.FUSED_LAYER_MAX_TOKENS)
 
@@ -470,6 +472,8 @@ class LookupFFN(nn.Module):
                      and (block or (256 <= D and J <= 4)))
         watched = ((ln._parameters, "weight"), (ln._parameters, "bias"), (p._parameters, "weight"), (p._parameters, "bias"),
                    (self._parameters, "tables"), (self._parameters, "bias"))
+        if not all(name in parameters for parameters, name in watched):
+            return None                   # a reparametrised weight is no parameter but computed on every access
         return _lib.host().make_layer(
             (int(block), int(st["one_launch"]), self.hidden_size, D, R, J, self.num_table, self.table_size, self.output_size,
              ops.row_format(self.tables.dtype), ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS, ops.PROJECT_BWD_PARTIALS,

@@ -771,3 +771,55 @@ def test_layer_under_autocast_float16(projection, bs):
             # same rows gathered; the scores come from float16 z, so they differ at half precision
             assert relmax(npf(out16)[agree], npf(out32)[agree]) <= 2e-2
             assert relmax(npf(gx16)[agree], npf(gx32)[agree]) <= 5e-2
+
+
+@pytest.mark.parametrize("block", [1, 64])
+def test_host_path_leaves_to_python_what_it_does_not_compute(block):
+    """A reparametrised weight, a tangent on the input, modes that watch operators and hooks on saved tensors: as on the
+    operators' own path, or refused as there."""
+    import torch.autograd.forward_ad as fwAD
+    from torch.nn.utils import parametrize
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    torch.manual_seed(41)
+    layer = lookupffn_amd.LookupFFN(_config(hidden_size=256, ffn_num_table=32, block_size=block), 256).to(DEV)
+    x = torch.randn(20, 256, device=DEV)
+    plain = layer(x)
+    plain.sum().backward()
+    grad = layer.hash.projection.weight.grad.clone()
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        assert torch.equal(layer(x), plain)
+    assert any("lookupffn" in n for n in Seen.names)
+
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
+        out = layer(x)
+    assert packed and torch.equal(out, plain)
+
+    with fwAD.dual_level(), pytest.raises(Exception):
+        layer(fwAD.make_dual(x, torch.ones_like(x)))
+
+    class Twice(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+
+        def right_inverse(self, w):
+            return w / 2
+
+    layer.zero_grad()
+    parametrize.register_parametrization(layer.hash.projection, "weight", Twice())
+    out = layer(x)
+    assert torch.equal(out, plain)
+    out.sum().backward()
+    got = layer.hash.projection.parametrizations.weight.original.grad
+    assert relmax(npf(got), npf(2 * grad)) <= 1e-5
+    with torch.no_grad():
+        assert relmax(npf(layer.eval()(x)), npf(plain)) <= 1e-5
