@@ -363,6 +363,16 @@ constexpr double QUAD_MARGIN = 0.92;      // the form must promise this much to 
 // indexed by LFFN_ROWS_*: fp32, bfloat16, half
 constexpr double QUAD_US_PER_PAIR[3] = {0.53, 0.56, 0.61};
 constexpr double QUAD_US_PER_PAIR_PASS[3] = {0.165, 0.36, 0.275};
+// Workgroups of 1024 tokens below which the form is not asked for, whatever it promises: it leaves compute units idle, and
+// the others then copy at a rate its costs do not describe.  Layer, us, other form -> this one: fp32 6144 x 128 x 768 (144 workgroups)
+// 125 -> 100, 10240 x 128 x 512 (160) 131 -> 102, but 4096 x 128 x 1024 (128) 94 -> 98 and 5120 x 128 x 768 (120) 96 -> 99;
+// bfloat16 12288 x 128 x 768 (144) 176 -> 139, 10240 x 512 x 1024 (160) 670 -> 507, but 8192 x 64 x 512 (64) 68 -> 74; half, whose other form is
+// the token-major one, 6144 x 128 x 768 (72) 124 -> 117, 4096 x 512 x 1024 (64) 540 -> 460.  fp32 tables beyond the memory-side cache,
+// whose copies cost half as much again: 5120 x 512 x 768 (120) 351 -> 457 and 6144 (144) 391 -> 453, so a round of them has to be
+// three quarters full.
+// With the records written by the projection kernel; where they are packed from codes and scores, 16-bit rows stay at 192.
+constexpr int64_t QUAD_MIN_WORKGROUPS[3] = {144, 96, 64};
+constexpr int64_t QUAD_MIN_WORKGROUPS_FULL = 192;
 constexpr double QUAD_US_PER_PAIR_MIN = 1.19;
 
 template <bool BF16>
@@ -409,7 +419,10 @@ GatherPlan plan_quad(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, bool 
         2 * S * Do * esz >= (int64_t(1) << 32))
         return best;
     const int64_t nslices = Do / cols;
-    if (((B + 1023) / 1024) * nslices < 192 || B * nslices > (int64_t(1) << 30)) return best;
+    const bool full = fmt == LFFN_ROWS_F32 ? double(T) * double(S) * double(Do) * 4 > 200e6 : pack;
+    if (((B + 1023) / 1024) * nslices < (full ? QUAD_MIN_WORKGROUPS_FULL : QUAD_MIN_WORKGROUPS[fmt]) ||
+        B * nslices > (int64_t(1) << 30))
+        return best;
     const double per_pass = QUAD_US_PER_PAIR_PASS[fmt], fixed = QUAD_US_PER_PAIR[fmt];
     for (int np : {4, 5, 6, 7, 8}) {
         if (!lffn_internal_quad_np_built(fmt, np)) continue;
