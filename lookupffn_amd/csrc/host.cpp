@@ -7,8 +7,8 @@
 // training forward records one autograd node whose backward launches the whole chain.
 //
 // Python builds a handle (make_layer) when the parameters are of a kind the kernels are built for, and calls
-// forward(handle, x, residual, ...).  The answer is None whenever anything is not as the handle expects: another parameter
-// object, storage, dtype, sizes or strides, an input of another type, dtype, device or layout, a gradient wanted that this path does not
+// forward(handle, layer, x, residual, ...).  The answer is None whenever anything is not as the handle expects: a module or a
+// parameter of another kind, another parameter object (each looked up through the layer's modules on every call), storage, dtype, sizes or strides, an input of another type, dtype, device or layout, a gradient wanted that this path does not
 // compute.  Then the Python path runs, with its own checks and errors.
 #include <Python.h>
 
@@ -92,9 +92,9 @@ struct RecordPlan {
     int32_t tokens = 0;
 };
 
-// A parameter, where Python finds it, and what it was when the handle was made.
+// A parameter, and what it was when the handle was made.
 struct Watched {
-    PyObject *dict, *key, *object;
+    PyObject *object;
     const void *data;
     at::ScalarType dtype;
     std::vector<int64_t> sizes, strides;
@@ -104,8 +104,42 @@ struct Watched {
     }
 };
 
+// What the layer holds at this moment: it, its LayerNorm, its hash and the hash's projection as Python finds them on every
+// access, and the parameters in them (in the order of Input below).  Borrowed references.
+struct Parts {
+    std::array<PyObject *, 4> modules;
+    std::array<PyObject *, 6> params;
+};
+
+PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES;   // interned
+
+PyObject *dict_of(PyObject *o) {
+    PyObject **d = o ? _PyObject_GetDictPtr(o) : nullptr;
+    return d ? *d : nullptr;
+}
+
+PyObject *item(PyObject *dict, PyObject *key) { return dict && PyDict_Check(dict) ? PyDict_GetItem(dict, key) : nullptr; }
+
+// False when something is not where a LookupFFN has it (a reparametrised weight is no parameter but computed on every access).
+bool find_parts(PyObject *layer, Parts &found) {
+    PyObject *own = dict_of(layer), *modules = item(own, KEY_MODULES);
+    PyObject *norm = item(modules, KEY_LAYER_NORM), *hash = item(modules, KEY_HASH);
+    PyObject *projection = item(item(dict_of(hash), KEY_MODULES), KEY_PROJECTION);
+    PyObject *of_layer = item(own, KEY_PARAMETERS), *of_norm = item(dict_of(norm), KEY_PARAMETERS),
+             *of_projection = item(dict_of(projection), KEY_PARAMETERS);
+    found.modules = {layer, norm, hash, projection};
+    found.params = {item(of_norm, KEY_WEIGHT),       item(of_norm, KEY_BIAS),      item(of_projection, KEY_WEIGHT),
+                    item(of_projection, KEY_BIAS), item(of_layer, KEY_TABLES), item(of_layer, KEY_BIAS)};
+    for (PyObject *o : found.modules)
+        if (!o) return false;
+    for (PyObject *o : found.params)
+        if (!o) return false;
+    return true;
+}
+
 struct Layer {
     Config c{};
+    std::array<PyTypeObject *, 4> types;  // of the modules
     std::vector<Watched> watched;
     // lnw, lnb, weight, pbias, tables, obias (pbias may be undefined)
     std::array<Tensor, 6> p;
@@ -361,11 +395,8 @@ const char *CAPSULE = "lookupffn_amd.layer";
 void free_layer(PyObject *capsule) {
     Layer *l = static_cast<Layer *>(PyCapsule_GetPointer(capsule, CAPSULE));
     if (!l) return;
-    for (Watched &w : l->watched) {
-        Py_XDECREF(w.dict);
-        Py_XDECREF(w.key);
-        Py_XDECREF(w.object);
-    }
+    for (Watched &w : l->watched) Py_XDECREF(w.object);
+    for (PyTypeObject *t : l->types) Py_XDECREF(t);
     Py_XDECREF(l->folded_dict);
     Py_XDECREF(l->folded_key);
     Py_XDECREF(l->folded_object);
@@ -408,25 +439,31 @@ PyObject *bind_library(PyObject *, PyObject *path) {
     END_HANDLE_TH_ERRORS
 }
 
-// make_layer(config: 15 ints, floats: 3, watched: [(dict, key)] * 6, folded: (dict, key, object, tensor, version) or None)
+// make_layer(config: 15 ints, floats: 3, layer, folded: (dict, key, object, tensor, version) or None) -> handle, or None when the
+// layer has not the parameters it was made with
 PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 4, "make_layer: 4 arguments");
+    Parts parts;
+    if (!find_parts(args[2], parts)) Py_RETURN_NONE;
+    for (PyObject *o : parts.params)
+        if (o != Py_None && !THPVariable_Check(o)) Py_RETURN_NONE;
     auto l = std::make_unique<Layer>();
     int64_t *ints = &l->c.form;
-    TORCH_CHECK(PyTuple_GET_SIZE(args[0]) == 15 && PyTuple_GET_SIZE(args[1]) == 3 && PyTuple_GET_SIZE(args[2]) == 6, "make_layer: sizes");
+    TORCH_CHECK(PyTuple_GET_SIZE(args[0]) == 15 && PyTuple_GET_SIZE(args[1]) == 3, "make_layer: sizes");
     for (int i = 0; i < 15; ++i) ints[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(args[0], i));
     double *floats = &l->c.eps;
     for (int i = 0; i < 3; ++i) floats[i] = PyFloat_AsDouble(PyTuple_GET_ITEM(args[1], i));
     if (PyErr_Occurred()) return nullptr;
+    for (int i = 0; i < 4; ++i) {
+        l->types[i] = Py_TYPE(parts.modules[i]);
+        Py_INCREF(l->types[i]);
+    }
     for (int i = 0; i < 6; ++i) {
-        PyObject *pair = PyTuple_GET_ITEM(args[2], i);
-        PyObject *dict = PyTuple_GET_ITEM(pair, 0), *key = PyTuple_GET_ITEM(pair, 1);
-        PyObject *o = PyDict_GetItemWithError(dict, key);
-        TORCH_CHECK(o && (o == Py_None || THPVariable_Check(o)), "make_layer: a parameter is missing");
+        PyObject *o = parts.params[i];
         if (o != Py_None) l->p[i] = THPVariable_Unpack(o);
-        for (PyObject *k : {dict, key, o}) Py_INCREF(k);
-        Watched w{dict, key, o, nullptr, at::kFloat, {}, {}};
+        Py_INCREF(o);
+        Watched w{o, nullptr, at::kFloat, {}, {}};
         if (const Tensor &t = l->p[i]; t.defined()) {
             w.data = t.data_ptr();
             w.dtype = t.scalar_type();
@@ -452,15 +489,15 @@ PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// forward(handle, x, residual or None, tokens up to which the one-launch form is taken) -> tensor or None
+// forward(handle, layer, x, residual or None, tokens up to which the one-launch form is taken) -> tensor or None
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(n == 4, "forward: 4 arguments");
+    TORCH_CHECK(n == 5, "forward: 5 arguments");
     Layer *l = static_cast<Layer *>(PyCapsule_GetPointer(args[0], CAPSULE));
     if (!l) return nullptr;
     const Config &c = l->c;
-    if (watched_over() || !plain(args[1])) Py_RETURN_NONE;
-    const Tensor &x = THPVariable_Unpack(args[1]);
+    if (watched_over() || !plain(args[2])) Py_RETURN_NONE;
+    const Tensor &x = THPVariable_Unpack(args[2]);
     const at::Device dev = l->p[4].device();
     const int64_t dims = x.dim();
     if (dims < 1 || x.size(dims - 1) != c.H || x.numel() == 0 || x.scalar_type() != at::kFloat || !x.is_contiguous() || x.device() != dev ||
@@ -471,9 +508,9 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
     sizes[dims - 1] = c.Do;
     Tensor residual;
-    if (args[2] != Py_None) {
-        if (!plain(args[2])) Py_RETURN_NONE;
-        residual = THPVariable_Unpack(args[2]);
+    if (args[3] != Py_None) {
+        if (!plain(args[3])) Py_RETURN_NONE;
+        residual = THPVariable_Unpack(args[3]);
         if (residual.scalar_type() != at::kFloat || residual.device() != dev || !residual.is_contiguous() || !residual.sizes().equals(sizes) ||
             reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 != 0)
             Py_RETURN_NONE;
@@ -481,9 +518,13 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     bool grads = false;
     const bool grad_mode = at::GradMode::is_enabled();
     if (grad_mode) grads = x.requires_grad() || (residual.defined() && residual.requires_grad());
+    Parts parts;
+    if (!find_parts(args[1], parts)) Py_RETURN_NONE;
+    for (size_t i = 0; i < l->types.size(); ++i)
+        if (Py_TYPE(parts.modules[i]) != l->types[i]) Py_RETURN_NONE;
     for (size_t i = 0; i < l->watched.size(); ++i) {
         const Watched &w = l->watched[i];
-        if (PyDict_GetItem(w.dict, w.key) != w.object) Py_RETURN_NONE;
+        if (parts.params[i] != w.object) Py_RETURN_NONE;
         const Tensor &p = l->p[i];
         if (!p.defined()) continue;
         if (!w.same(p)) Py_RETURN_NONE;
@@ -495,7 +536,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         Py_RETURN_NONE;
     Tensor out = empty_f32(sizes, dev);
     if (grads) train(*l, x, residual, out, B);
-    else infer(*l, x, f32(residual), out, B, PyLong_AsLongLong(args[3]));
+    else infer(*l, x, f32(residual), out, B, PyLong_AsLongLong(args[4]));
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -511,4 +552,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host() {
+    const std::pair<PyObject **, const char *> keys[] = {
+        {&KEY_MODULES, "_modules"}, {&KEY_PARAMETERS, "_parameters"}, {&KEY_LAYER_NORM, "LayerNorm"}, {&KEY_HASH, "hash"},
+        {&KEY_PROJECTION, "projection"}, {&KEY_WEIGHT, "weight"}, {&KEY_BIAS, "bias"}, {&KEY_TABLES, "tables"},
+    };
+    for (const auto &[key, name] : keys)
+        if (!(*key = PyUnicode_InternFromString(name))) return nullptr;
+    return PyModule_Create(&module);
+}

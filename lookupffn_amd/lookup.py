@@ -445,8 +445,8 @@ class LookupFFN(nn.Module):
 
     def _forward_host(self, x, residual):
         """The layer through the host path (csrc/host.cpp), or None when the call or the parameters are not of a kind it is
-        built for.  Its handle holds for as long as the parameters it names are the layer's, with the storage and dtype
-        they had (and, without gradient, the folded 64 x 64 blocks the weights they were folded from)."""
+        built for.  Its handle holds for as long as the parameters it names are those of the layer, its LayerNorm and its
+        projection, with the storage and dtype they had (and, without gradient, the folded 64 x 64 blocks the weights they were folded from)."""
         if not (x.is_cuda and x.dtype == torch.float32 and self.tables.is_cuda):
             return None
         st = self._inference_state()
@@ -461,24 +461,20 @@ class LookupFFN(nn.Module):
             self._handle, self._handle_key = self._make_handle(st, key[1]), key
         if self._handle is None:
             return None
-        return _lib.host().forward(self._handle, x.contiguous(), None if residual is None else residual.contiguous(),
+        return _lib.host().forward(self._handle, self, x.contiguous(), None if residual is None else residual.contiguous(),
                                    self.FUSED_LAYER_MAX_TOKENS)
 
     def _make_handle(self, st, folded):
-        ln, p = self.LayerNorm, self.hash.projection
+        p = self.hash.projection
         block = st["form"] == "block"
         R, J, D = p.num_repeat, p.weight.shape[1], p.padded_in_dim
         trainable = (self.tables.dtype == torch.float32 and self.hidden_size % 4 == 0 and self.hidden_size <= 1024
                      and (block or (256 <= D and J <= 4)))
-        watched = ((ln._parameters, "weight"), (ln._parameters, "bias"), (p._parameters, "weight"), (p._parameters, "bias"),
-                   (self._parameters, "tables"), (self._parameters, "bias"))
-        if not all(name in parameters for parameters, name in watched):
-            return None                   # a reparametrised weight is no parameter but computed on every access
         return _lib.host().make_layer(
             (int(block), int(st["one_launch"]), self.hidden_size, D, R, J, self.num_table, self.table_size, self.output_size,
              ops.row_format(self.tables.dtype), ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS, ops.PROJECT_BWD_PARTIALS,
              ops.COLUMN_SUM_CHUNK_ROWS, int(trainable)),
-            (st["eps"], st["decay"], st["res_coef"]), watched,
+            (st["eps"], st["decay"], st["res_coef"]), self,
             None if folded is None else (self.hash.__dict__, "_folded", folded, folded[1], p.weight._version))
 
     def _forward(self, hidden_states, residual=None):
@@ -530,7 +526,7 @@ class LookupFFN(nn.Module):
         if handle is not None and not torch.compiler.is_compiling():
             # (before anything else: at a few hundred tokens the layer is one launch of a few microseconds, and every view
             # made here shows in its time)
-            out = _lib.host().forward(handle, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS)
+            out = _lib.host().forward(handle, self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS)
             if out is not None:
                 return out
         shape = hidden_states.shape[:-1]

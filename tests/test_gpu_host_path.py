@@ -1,0 +1,87 @@
+"""The layer's host path (csrc/host.cpp) takes what it computes with from the layer on every call: a layer that was called before
+and then changed is compared with one that was changed before its first call."""
+import copy
+from argparse import Namespace
+
+import pytest
+import torch
+
+import lookupffn_amd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _layer(block=1, seed=0, hidden=256, tables=32, out=256):
+    torch.manual_seed(seed)
+    cfg = Namespace(hidden_size=hidden, ffn_num_table=tables, ffn_table_size=256, layer_norm_eps=1e-5, projection_type="bh4",
+                    block_size=block)
+    layer = lookupffn_amd.LookupFFN(cfg, out).to(DEV)
+    with torch.no_grad():
+        for q in (layer.LayerNorm.weight, layer.LayerNorm.bias, layer.hash.projection.bias):
+            q.add_(0.1 * torch.randn_like(q))
+    return layer
+
+
+def _pass(layer, x, train):
+    """The result and, in training, the gradient of every parameter."""
+    if not train:
+        with torch.no_grad():
+            return [layer.eval()(x)]
+    layer.train().zero_grad(set_to_none=True)
+    out = layer(x)
+    out.sum().backward()
+    return [out.detach()] + [q.grad for q in layer.parameters()]
+
+
+def _assert_same(got, want):
+    # (the two may take different kernels, whose fp32 sums of up to a few hundred terms are in another order)
+    assert len(got) == len(want)
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-5 * b.abs().max().item())
+
+
+class Shifted(torch.nn.Module):
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+        self.shift = torch.nn.Parameter(torch.full((inner.out_dim,), 0.3, device=DEV))
+
+    def forward(self, x):
+        return self.inner(x) + self.shift
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("block", [1, 64])
+@pytest.mark.parametrize("which", ["LayerNorm", "hash", "projection", "wrapped projection"])
+def test_replaced_modules_are_seen(block, train, which):
+    layer, fresh, other = _layer(block), _layer(block), _layer(block, seed=1)
+    x = torch.randn(40, 256, device=DEV)
+    before = [_pass(layer, x, train) for _ in range(2)][0]
+    for m in (layer, fresh):
+        donor = copy.deepcopy(other)
+        if which == "LayerNorm":
+            m.LayerNorm = donor.LayerNorm
+        elif which == "hash":
+            m.hash = donor.hash
+        elif which == "projection":
+            m.hash.projection = donor.hash.projection
+        else:
+            m.hash.projection = Shifted(m.hash.projection)
+    got = _pass(layer, x, train)
+    assert not torch.allclose(got[0], before[0], rtol=1e-2)
+    _assert_same(got, _pass(fresh, x, train))
+
+
+@pytest.mark.parametrize("block", [1, 64])
+def test_a_copy_with_parameters_of_its_own_uses_them(block):
+    """A replica as DataParallel makes one shares the instance dictionary's entries but has other tensors as its parameters."""
+    layer, other = _layer(block).eval(), _layer(block, seed=1).eval()
+    x = torch.randn(40, 256, device=DEV)
+    with torch.no_grad():
+        layer(x), layer(x)
+        replica = layer._replicate_for_data_parallel()
+        replica._parameters = dict(other._parameters)
+        replica._modules["LayerNorm"], replica._modules["hash"] = other.LayerNorm, other.hash
+        _assert_same([replica(x)], [other(x)])
+        assert torch.equal(layer(x), copy.deepcopy(layer)(x))
