@@ -424,6 +424,14 @@ class LookupFFN(nn.Module):
                                     and q.device == self.tables.device) for q in small)
               and self.tables.is_cuda and self.tables.is_contiguous()
               and ops.row_format(self.tables.dtype) is not None and self.output_size % 64 == 0)
+        if ok:
+            # sizes that do not fit together are for the general path to refuse: the kernels take them from the layer
+            R, D, bs = p.num_repeat, p.padded_in_dim, p.block_size
+            ok = (ln.weight.numel() == ln.bias.numel() == self.hidden_size <= D
+                  and p.weight.dim() == 5 and p.weight.shape == (R, p.weight.shape[1], D // bs, bs, bs)
+                  and 8 * self.num_table <= R * D and (p.bias is None or p.bias.numel() == 8 * self.num_table)
+                  and self.tables.shape == (self.num_table, self.table_size, self.output_size)
+                  and self.bias.numel() == self.output_size)
         form = None
         if ok and p.block_size == 1 and 8 <= p.padded_in_dim <= 1024:
             form = "diag"

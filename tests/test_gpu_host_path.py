@@ -85,3 +85,32 @@ def test_a_copy_with_parameters_of_its_own_uses_them(block):
         replica._modules["LayerNorm"], replica._modules["hash"] = other.LayerNorm, other.hash
         _assert_same([replica(x)], [other(x)])
         assert torch.equal(layer(x), copy.deepcopy(layer)(x))
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("block", [1, 64])
+@pytest.mark.parametrize("which", ["LayerNorm", "tables", "rows", "bias", "projection.bias", "projection"])
+def test_parameters_that_do_not_fit_together_are_refused(block, train, which):
+    """Each is one that the kernels, which take their sizes from the layer, would read beyond the end of."""
+    layer = _layer(block)
+    x = torch.randn(40, 256, device=DEV)
+    _pass(layer, x, train), _pass(layer, x, train)
+    zeros = lambda *shape: torch.nn.Parameter(torch.zeros(*shape, device=DEV))
+    if which == "LayerNorm":
+        layer.LayerNorm = torch.nn.LayerNorm(128).to(DEV)
+    elif which == "tables":
+        layer.tables = zeros(16, 256, 256)
+    elif which == "rows":
+        layer.tables = zeros(32, 128, 256)
+    elif which == "bias":
+        layer.bias = zeros(64)
+    elif which == "projection.bias":
+        layer.hash.projection.bias = zeros(128)
+    else:
+        layer.hash.projection = lookupffn_amd.BH4(128, 128, block).to(DEV)
+    if which == "rows":          # a table of half as many rows is in order, and its rows are taken by the code's low bits
+        assert torch.equal(_pass(layer, x, train)[0], layer.bias.detach().expand(40, 256))
+        return
+    with pytest.raises((AssertionError, RuntimeError)):
+        _pass(layer, x, train)
+        torch.cuda.synchronize()
