@@ -80,7 +80,8 @@ void check(int rc, const char *what) { TORCH_CHECK(rc == LFFN_OK, what, ": ", li
 
 enum Form { DIAG = 0, BLOCK = 1 };
 
-// Sizes and constants of a layer; the thresholds are the Python operators' own.
+// Sizes and constants of a layer; the thresholds are the Python operators' own.  The last three are what the modules hold
+// at the call.
 struct Config {
     int64_t form, one_launch, H, D, R, J, T, S, Do, fmt;
     int64_t sorted_min_work, ln_partials, project_partials, sum_chunk_rows, trainable;
@@ -105,13 +106,15 @@ struct Watched {
 };
 
 // What the layer holds at this moment: it, its LayerNorm, its hash and the hash's projection as Python finds them on every
-// access, and the parameters in them (in the order of Input below).  Borrowed references.
+// access, the parameters in them (in the order of Input below) and their constants.  Borrowed references.
 struct Parts {
     std::array<PyObject *, 4> modules;
     std::array<PyObject *, 6> params;
+    double eps, decay;
 };
 
-PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES;   // interned
+PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES, *KEY_EPS,
+    *KEY_DECAY;                           // interned
 
 PyObject *dict_of(PyObject *o) {
     PyObject **d = o ? _PyObject_GetDictPtr(o) : nullptr;
@@ -119,6 +122,16 @@ PyObject *dict_of(PyObject *o) {
 }
 
 PyObject *item(PyObject *dict, PyObject *key) { return dict && PyDict_Check(dict) ? PyDict_GetItem(dict, key) : nullptr; }
+
+bool number(PyObject *o, double &value) {
+    if (!o || !(PyFloat_Check(o) || PyLong_Check(o))) return false;
+    value = PyFloat_AsDouble(o);
+    if (value == -1.0 && PyErr_Occurred()) {             // an integer beyond double
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
 
 // False when something is not where a LookupFFN has it (a reparametrised weight is no parameter but computed on every access).
 bool find_parts(PyObject *layer, Parts &found) {
@@ -134,7 +147,7 @@ bool find_parts(PyObject *layer, Parts &found) {
         if (!o) return false;
     for (PyObject *o : found.params)
         if (!o) return false;
-    return true;
+    return number(item(dict_of(norm), KEY_EPS), found.eps) && number(item(dict_of(projection), KEY_DECAY), found.decay);
 }
 
 struct Layer {
@@ -146,7 +159,6 @@ struct Layer {
     Tensor folded;                       // BLOCK inference: the folded weights and the weight's version they belong to
     uint32_t folded_version = 0;
     PyObject *folded_dict = nullptr, *folded_key = nullptr, *folded_object = nullptr;
-    lffn_fused_layer block{};
     std::array<RecordPlan, 8> plans;     // a few batch sizes in turn; guarded by the interpreter lock
     int next_plan = 0;
 };
@@ -189,14 +201,15 @@ void gather(const Config &c, const Tensor &codes, const Tensor &scores, const Te
              wp, ws_bytes, B, c.T, c.S, c.Do, st);
 }
 
-void infer(Layer &l, const Tensor &x, const float *residual, Tensor &out, int64_t B, int64_t fused_max) {
-    const Config &c = l.c;
+void infer(Layer &l, const Config &c, const Tensor &x, const float *residual, Tensor &out, int64_t B, int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     // (rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half
     // as many tokens more: 768 tokens, 128 tables of 768 columns 34 us against 55 in two launches, 512 of 1024 113 against 120)
     if (c.one_launch && B <= (c.fmt == 0 ? fused_max : fused_max + fused_max / 2)) {
-        CALL(lffn_lookup_ffn_fused_layer_rows, &l.block, (int32_t)c.fmt, f32(x), residual, f32(out), B, st);
+        const lffn_fused_layer layer{f32(l.p[0]), f32(l.p[1]), f32(l.p[2]), f32(l.p[3]), f32(l.p[4]), f32(l.p[5]), c.H, c.D, c.R, c.J, c.T,
+                                     c.S, c.Do, (float)c.eps, (float)c.decay, (float)c.residual};
+        CALL(lffn_lookup_ffn_fused_layer_rows, &layer, (int32_t)c.fmt, f32(x), residual, f32(out), B, st);
         return;
     }
     const float eps = (float)c.eps, decay = (float)c.decay, res = (float)c.residual;
@@ -348,8 +361,7 @@ struct LookupFFNBackward : public torch::autograd::Node {
     }
 };
 
-void train(Layer &l, const Tensor &x, const Tensor &residual, Tensor &out, int64_t B) {
-    const Config &c = l.c;
+void train(Layer &l, const Config &c, const Tensor &x, const Tensor &residual, Tensor &out, int64_t B) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     auto node = std::shared_ptr<LookupFFNBackward>(new LookupFFNBackward(), torch::autograd::deleteNode);
@@ -439,21 +451,19 @@ PyObject *bind_library(PyObject *, PyObject *path) {
     END_HANDLE_TH_ERRORS
 }
 
-// make_layer(config: 15 ints, floats: 3, layer, folded: (dict, key, object, tensor, version) or None) -> handle, or None when the
+// make_layer(config: 15 ints, layer, folded: (dict, key, object, tensor, version) or None) -> handle, or None when the
 // layer has not the parameters it was made with
 PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(n == 4, "make_layer: 4 arguments");
+    TORCH_CHECK(n == 3, "make_layer: 3 arguments");
     Parts parts;
-    if (!find_parts(args[2], parts)) Py_RETURN_NONE;
+    if (!find_parts(args[1], parts)) Py_RETURN_NONE;
     for (PyObject *o : parts.params)
         if (o != Py_None && !THPVariable_Check(o)) Py_RETURN_NONE;
     auto l = std::make_unique<Layer>();
     int64_t *ints = &l->c.form;
-    TORCH_CHECK(PyTuple_GET_SIZE(args[0]) == 15 && PyTuple_GET_SIZE(args[1]) == 3, "make_layer: sizes");
+    TORCH_CHECK(PyTuple_GET_SIZE(args[0]) == 15, "make_layer: sizes");
     for (int i = 0; i < 15; ++i) ints[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(args[0], i));
-    double *floats = &l->c.eps;
-    for (int i = 0; i < 3; ++i) floats[i] = PyFloat_AsDouble(PyTuple_GET_ITEM(args[1], i));
     if (PyErr_Occurred()) return nullptr;
     for (int i = 0; i < 4; ++i) {
         l->types[i] = Py_TYPE(parts.modules[i]);
@@ -472,17 +482,14 @@ PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
         }
         l->watched.push_back(std::move(w));
     }
-    if (args[3] != Py_None) {
-        l->folded_dict = PyTuple_GET_ITEM(args[3], 0);
-        l->folded_key = PyTuple_GET_ITEM(args[3], 1);
-        l->folded_object = PyTuple_GET_ITEM(args[3], 2);
+    if (args[2] != Py_None) {
+        l->folded_dict = PyTuple_GET_ITEM(args[2], 0);
+        l->folded_key = PyTuple_GET_ITEM(args[2], 1);
+        l->folded_object = PyTuple_GET_ITEM(args[2], 2);
         for (PyObject *k : {l->folded_dict, l->folded_key, l->folded_object}) Py_INCREF(k);
-        l->folded = THPVariable_Unpack(PyTuple_GET_ITEM(args[3], 3));
-        l->folded_version = (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(args[3], 4));
+        l->folded = THPVariable_Unpack(PyTuple_GET_ITEM(args[2], 3));
+        l->folded_version = (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(args[2], 4));
     }
-    const Config &c = l->c;
-    l->block = lffn_fused_layer{f32(l->p[0]), f32(l->p[1]), f32(l->p[2]), f32(l->p[3]), f32(l->p[4]), f32(l->p[5]), c.H, c.D, c.R, c.J, c.T,
-                                c.S, c.Do, (float)c.eps, (float)c.decay, (float)c.residual};
     PyObject *capsule = PyCapsule_New(l.get(), CAPSULE, free_layer);
     if (capsule) l.release();
     return capsule;
@@ -495,7 +502,12 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     TORCH_CHECK(n == 5, "forward: 5 arguments");
     Layer *l = static_cast<Layer *>(PyCapsule_GetPointer(args[0], CAPSULE));
     if (!l) return nullptr;
-    const Config &c = l->c;
+    Parts parts;
+    if (!find_parts(args[1], parts)) Py_RETURN_NONE;
+    Config c = l->c;
+    c.eps = parts.eps;
+    c.decay = parts.decay;
+    c.residual = 1.0 - parts.decay;
     if (watched_over() || !plain(args[2])) Py_RETURN_NONE;
     const Tensor &x = THPVariable_Unpack(args[2]);
     const at::Device dev = l->p[4].device();
@@ -518,8 +530,6 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     bool grads = false;
     const bool grad_mode = at::GradMode::is_enabled();
     if (grad_mode) grads = x.requires_grad() || (residual.defined() && residual.requires_grad());
-    Parts parts;
-    if (!find_parts(args[1], parts)) Py_RETURN_NONE;
     for (size_t i = 0; i < l->types.size(); ++i)
         if (Py_TYPE(parts.modules[i]) != l->types[i]) Py_RETURN_NONE;
     for (size_t i = 0; i < l->watched.size(); ++i) {
@@ -535,8 +545,8 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         (!l->folded.defined() || PyDict_GetItem(l->folded_dict, l->folded_key) != l->folded_object || l->p[2]._version() != l->folded_version))
         Py_RETURN_NONE;
     Tensor out = empty_f32(sizes, dev);
-    if (grads) train(*l, x, residual, out, B);
-    else infer(*l, x, f32(residual), out, B, PyLong_AsLongLong(args[4]));
+    if (grads) train(*l, c, x, residual, out, B);
+    else infer(*l, c, x, f32(residual), out, B, PyLong_AsLongLong(args[4]));
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -556,6 +566,7 @@ PyMODINIT_FUNC PyInit__host() {
     const std::pair<PyObject **, const char *> keys[] = {
         {&KEY_MODULES, "_modules"}, {&KEY_PARAMETERS, "_parameters"}, {&KEY_LAYER_NORM, "LayerNorm"}, {&KEY_HASH, "hash"},
         {&KEY_PROJECTION, "projection"}, {&KEY_WEIGHT, "weight"}, {&KEY_BIAS, "bias"}, {&KEY_TABLES, "tables"},
+        {&KEY_EPS, "eps"}, {&KEY_DECAY, "decay_coeff"},
     };
     for (const auto &[key, name] : keys)
         if (!(*key = PyUnicode_InternFromString(name))) return nullptr;

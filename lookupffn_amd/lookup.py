@@ -405,7 +405,7 @@ class LookupFFN(nn.Module):
     def _inference_state(self):
         """What the inference kernels take from the parameters, or None when the parameters are not of
         a kind those kernels are built for; worked out once and kept until a parameter is replaced,
-        moved or cast (in-place updates keep the storage, so the cached views stay good).  A launch
+        moved or cast or a constant changed (in-place updates keep the storage, so the cached views stay good).  A launch
         is a few microseconds: re-deriving this on every call cost more than the kernels at small
         batches.  Keys: form ("diag": one kernel for LayerNorm + diagonal BH4 + hash; "block": the
         matrix-core kernel for 64 x 64 blocks), one_launch (the whole layer in one kernel is possible),
@@ -414,6 +414,7 @@ class LookupFFN(nn.Module):
         ln = self.LayerNorm
         params = (ln.weight, ln.bias, getattr(p, "weight", None), getattr(p, "bias", None), self.tables, self.bias)
         key = tuple((id(q), q.data_ptr(), q.dtype) if q is not None else None for q in params)
+        key += (getattr(ln, "eps", None), getattr(p, "decay_coeff", None))
         cached = getattr(self, "_inference_cache", None)
         if cached is not None and cached[0] == key:
             return cached[1]
@@ -482,7 +483,7 @@ class LookupFFN(nn.Module):
             (int(block), int(st["one_launch"]), self.hidden_size, D, R, J, self.num_table, self.table_size, self.output_size,
              ops.row_format(self.tables.dtype), ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS, ops.PROJECT_BWD_PARTIALS,
              ops.COLUMN_SUM_CHUNK_ROWS, int(trainable)),
-            (st["eps"], st["decay"], st["res_coef"]), self,
+            self,
             None if folded is None else (self.hash.__dict__, "_folded", folded, folded[1], p.weight._version))
 
     def _forward(self, hidden_states, residual=None):

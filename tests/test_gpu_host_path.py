@@ -114,3 +114,19 @@ def test_parameters_that_do_not_fit_together_are_refused(block, train, which):
     with pytest.raises((AssertionError, RuntimeError)):
         _pass(layer, x, train)
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("block", [1, 64])
+def test_changed_constants_are_seen(block, train):
+    """A schedule on decay_coeff, another eps: the values the modules hold at the call."""
+    layer, fresh = _layer(block), _layer(block)
+    x = 0.01 * torch.randn(40, 256, device=DEV)                   # (small enough for eps to show)
+    last = _pass(layer, x, train)
+    for eps, decay in ((1e-3, 0.7), (1e-3, 0.4), (1, 1)):
+        for m in (layer, fresh):
+            m.LayerNorm.eps, m.hash.projection.decay_coeff = eps, decay
+        got = _pass(layer, x, train)
+        assert not torch.allclose(got[0], last[0], rtol=1e-2)
+        _assert_same(got, _pass(copy.deepcopy(fresh), x, train))
+        last = got
