@@ -415,14 +415,15 @@ void free_layer(PyObject *capsule) {
     delete l;
 }
 
-// An ordinary tensor: no subclass, no transform of torch.func around it, nothing lazy.
-bool plain(PyObject *o) {
-    if (!THPVariable_CheckExact(o)) return false;
-    const Tensor &t = THPVariable_Unpack(o);
+// An ordinary tensor: no transform of torch.func around it, nothing lazy, no tangent.
+bool ordinary(const Tensor &t) {
     constexpr c10::DispatchKeySet other({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
                                          c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
     return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(other) && !t._fw_grad(/*level=*/0).defined();
 }
+
+// and of no subclass
+bool plain(PyObject *o) { return THPVariable_CheckExact(o) && ordinary(THPVariable_Unpack(o)); }
 
 // Somebody watches the operators that are called: a tracer, a mode of torch.overrides or torch.utils._python_dispatch, a
 // transform of torch.func.  They see them on the Python path.
@@ -459,7 +460,7 @@ PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
     Parts parts;
     if (!find_parts(args[1], parts)) Py_RETURN_NONE;
     for (PyObject *o : parts.params)
-        if (o != Py_None && !THPVariable_Check(o)) Py_RETURN_NONE;
+        if (o != Py_None && !(THPVariable_Check(o) && ordinary(THPVariable_Unpack(o)))) Py_RETURN_NONE;
     auto l = std::make_unique<Layer>();
     int64_t *ints = &l->c.form;
     TORCH_CHECK(PyTuple_GET_SIZE(args[0]) == 15, "make_layer: sizes");
@@ -537,7 +538,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (parts.params[i] != w.object) Py_RETURN_NONE;
         const Tensor &p = l->p[i];
         if (!p.defined()) continue;
-        if (!w.same(p)) Py_RETURN_NONE;
+        if (!ordinary(p) || !w.same(p)) Py_RETURN_NONE;
         if (grad_mode) grads = grads || p.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;

@@ -5,6 +5,7 @@ from argparse import Namespace
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 import lookupffn_amd
 
@@ -130,3 +131,23 @@ def test_changed_constants_are_seen(block, train):
         assert not torch.allclose(got[0], last[0], rtol=1e-2)
         _assert_same(got, _pass(copy.deepcopy(fresh), x, train))
         last = got
+
+
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("block", [1, 64])
+@pytest.mark.parametrize("name", ["tables", "bias", "LayerNorm.weight", "LayerNorm.bias", "hash.projection.weight",
+                                  "hash.projection.bias"])
+def test_a_tangent_on_a_parameter_is_refused(block, name, first):
+    """As one on the input is, rather than dropped: the layer's autograd functions have no forward mode."""
+    layer = _layer(block)
+    x = torch.randn(20, 256, device=DEV)
+    if not first:
+        want = layer(x).detach()
+        assert torch.equal(layer(x), want)
+    params = dict(layer.named_parameters())
+    with fwAD.dual_level():
+        params[name] = fwAD.make_dual(params[name].detach(), torch.ones_like(params[name]))
+        with pytest.raises((NotImplementedError, RuntimeError)):
+            torch.func.functional_call(layer, params, (x,))
+    if not first:
+        assert torch.equal(layer(x), want)
