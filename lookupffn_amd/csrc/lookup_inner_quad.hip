@@ -54,7 +54,7 @@ constexpr int TOUCH_AHEAD = 3;              // steps between the one being read 
 struct InnerQuadArgs {
     const int32_t *code;   // [B, T]
     const float *g;        // token b, slice s (32 columns) at g + b * g_token_stride + s * g_slice_stride
-    int64_t g_token_stride, g_slice_stride;     // floats: Do and 32 for [B, Do]; 32 and B * 32 for [Do/32][B][32]
+    int64_t g_token_stride, g_slice_stride;     // floats: Do and 32 for [B, Do]; 32 and (B + 1) * 32 for [Do/32][B + 1][32]
     const char *tables;    // [T, S, Do] fp32
     float *out;            // [B, T]
     int64_t B;

@@ -11,7 +11,7 @@
 //
 // lookup_sort_pack_kernel: two jobs in one launch, by workgroup number.  The sort occupies one
 // workgroup per table (128 of the 256 compute units at 128 tables) and is bound by latency; the
-// copy of g to a slice-major layout [Do/32][B][32] (in which the 128-byte row pieces of a slice
+// copy of g to a slice-major layout [Do/32][B + 1][32] (in which the 128-byte row pieces of a slice
 // are contiguous: with rows 4*Do bytes apart the pieces of one slice fall on a quarter of the L2
 // channels) is pure memory traffic and depends on nothing: its workgroups fill the rest of the
 // chip while the sort runs (23 + 25 us as two launches at 16384 tokens x 128 tables x 768).
@@ -21,9 +21,10 @@
 // ranks inside a 64-token batch from ballots over the code bits) and writes (token, score)
 // pairs bucket by bucket: into LDS first (a 16-bit token and a score per entry: at most 18432
 // entries, 108 KB), from where the list goes to memory in whole lines; written straight
-// from the ranks, every wavefront store was 64 separate 8-byte requests.  Every bucket is padded to a multiple of eight entries with
-// (first token of the bucket, 0.0f), so that eight consecutive entries always belong to
-// one code, and the bucket boundaries are stored in units of eight entries.
+// from the ranks, every wavefront store was 64 separate 8-byte requests.  Every bucket is padded to a multiple of eight entries,
+// so that eight consecutive entries always belong to one code, and the bucket boundaries are stored in units of eight entries.
+// The padding names token B, whose row of the copy of g is zero (a token of the bucket with weight 0 would make a row of an
+// infinite gradient NaN).
 //
 // lookup_scatter_sorted_kernel: one workgroup per (table, 32-column slice).  The sorted
 // list is cut into equal pieces, one per wavefront, whatever the bucket sizes (a skewed code
@@ -57,7 +58,7 @@ struct PrepArgs {
     const float *g;        // [B, Do]
     uint16_t *code_t;      // [T, Bp]
     float *score_t;        // [T, Bp]
-    float *g_packed;       // [Do / SC][B][SC]
+    float *g_packed;       // [Do / SC][B + 1][SC], the last row zero
     int64_t B, Bp;
     int T, S, Do, tiles_t;
 };
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(256) void lookup_prep_kernel(PrepArgs a) {
 
 constexpr int PACK_TOKENS = 32;      // rows of g per workgroup of the slice-major copy
 
-// PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy)
+// PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy); row B is the padding's
 __device__ __forceinline__ void pack_rows(const PrepArgs &a, int64_t blk) {
     const int64_t b0 = blk * PACK_TOKENS;
     const int q = a.Do / 4;
@@ -121,8 +122,8 @@ __device__ __forceinline__ void pack_rows(const PrepArgs &a, int64_t blk) {
             const int e = e0 + i * SORT_WG;
             const int64_t b = b0 + e / q;
             const int col = (e % q) * 4;
-            if (e < PACK_TOKENS * q && b < a.B)
-                *reinterpret_cast<float4 *>(a.g_packed + ((size_t)(col / SC) * a.B + b) * SC + col % SC) = v[i];
+            if (e < PACK_TOKENS * q && b <= a.B)
+                *reinterpret_cast<float4 *>(a.g_packed + ((size_t)(col / SC) * (a.B + 1) + b) * SC + col % SC) = v[i];
         }
     }
 }
@@ -143,8 +144,7 @@ __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
     int *hist = sm;                    // [SORT_WAVES][S]: counts, then running write positions
     int *count = hist + SORT_WAVES * S;
     int *start = count + S;            // padded bucket starts (entries)
-    int *first = start + S;            // lowest token of the bucket
-    int *total = first + S;
+    int *total = start + S;
     float *sc_s = reinterpret_cast<float *>(total + 4);                       // [stride] scores of the sorted list
     unsigned short *tok_s = reinterpret_cast<unsigned short *>(sc_s + a.stride);   // [stride] tokens
 
@@ -152,7 +152,6 @@ __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
     const uint16_t *code = a.code + (size_t)t * a.Bp;
     const float *score = a.score + (size_t)t * a.Bp;
     for (int q = tid; q < SORT_WAVES * S; q += SORT_WG) hist[q] = 0;
-    for (int q = tid; q < S; q += SORT_WG) first[q] = 0x7fffffff;
     __syncthreads();
 
     // A wavefront takes up to SORT_DEPTH batches of 64 consecutive tokens (the launch keeps B within 1024 * SORT_DEPTH).
@@ -189,10 +188,7 @@ __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
         const int rank = __popcll(m & ((1ull << lane) - 1ull));
         const int cnt = __popcll(m);
         rk[k] = rank | (cnt << 8);
-        if (live && rank == 0) {
-            myh[c] += cnt;
-            atomicMin(&first[c], (int)(lo + 64 * k + lane));
-        }
+        if (live && rank == 0) myh[c] += cnt;
     }
     __syncthreads();
     for (int c = tid; c < S; c += SORT_WG) {
@@ -259,10 +255,10 @@ __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
         const int n = count[c], o = start[c];
         for (int p = n; p < ((n + 7) & ~7); ++p) {
             if (a.stage) {
-                tok_s[o + p] = (unsigned short)first[c];
+                tok_s[o + p] = (unsigned short)a.B;
                 sc_s[o + p] = 0.f;
             } else {
-                out[o + p] = make_uint2((unsigned)first[c], 0u);
+                out[o + p] = make_uint2((unsigned)a.B, 0u);
             }
         }
     }
@@ -281,10 +277,10 @@ __global__ __launch_bounds__(SORT_WG) void lookup_sort_pack_kernel(SortArgs sa, 
 struct SortedArgs {
     const uint2 *pairs;    // table t's list starts at t * stride
     const int32_t *off8;   // [T, S + 1] bucket starts inside that list, in units of eight entries
-    const float *g;        // [Do / SC][B][SC]
+    const float *g;        // [Do / SC][B + 1][SC]
     float *out;            // [rows, Do]; table t's rows from t * S on
     int64_t stride, rows;
-    unsigned last_token;   // B - 1
+    unsigned last_token;   // B: the padding's
     int T, S, Do, nslices, accumulate;
 };
 
@@ -460,7 +456,7 @@ inline Workspace workspace_layout(int64_t B, int64_t T, int64_t S, int64_t Do) {
     w.code_t = w.off8 + round16(T * (S + 1) * 4);
     w.score_t = w.code_t + round16(T * Bp * 2);
     w.g_packed = w.score_t + round16(T * Bp * 4);
-    w.total = w.g_packed + round16(Bc * Do * 4);
+    w.total = w.g_packed + round16((Bc + 1) * Do * 4);
     return w;
 }
 
@@ -500,7 +496,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         pa.tiles_t = (int)((T + 63) / 64);
         // (score gradient only: the codes and scores need no transposing or sorting, only g its slice-major copy)
         const int64_t transpose_blocks = grad_tables ? (Bp / 64) * pa.tiles_t : 0;
-        const int64_t pack_blocks = (Bc + PACK_TOKENS - 1) / PACK_TOKENS;
+        const int64_t pack_blocks = (Bc + 1 + PACK_TOKENS - 1) / PACK_TOKENS;
         const int64_t nsort = grad_tables ? T : 0;
         LFFN_REQUIRE(transpose_blocks <= 0x7fffffff && nsort + pack_blocks <= 0x7fffffff, LFFN_ERR_UNSUPPORTED);
         int rc = LFFN_OK;
@@ -513,9 +509,9 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         sa.code = pa.code_t; sa.score = pa.score_t; sa.pairs = pairs; sa.off8 = off8;
         sa.B = Bc; sa.Bp = Bp; sa.stride = stride; sa.T = (int)T; sa.S = (int)S; sa.nbits = lffn_log2(S);
         // histograms and bucket tables, then the sorted list itself (4 + 2 bytes per entry; tokens of a chunk fit 16 bits)
-        static_assert(CHUNK <= 65536, "tokens of a chunk are staged as 16-bit values");
+        static_assert(CHUNK < 65536, "tokens of a chunk and the padding's are staged as 16-bit values");
         static_assert(CHUNK <= int64_t(SORT_WG) * SORT_DEPTH, "a wavefront of the sort holds its tokens in registers");
-        const size_t tables_lds = (size_t(SORT_WAVES) * S + 3 * S + 4 + 4) * sizeof(int);
+        const size_t tables_lds = (size_t(SORT_WAVES) * S + 2 * S + 4 + 4) * sizeof(int);
         const size_t staged_lds = tables_lds + size_t(stride) * 6 + 16;
         sa.stage = staged_lds <= 160 * 1024 ? 1 : 0;            // 512-row tables: the list goes straight to memory
         const size_t sort_lds = nsort ? (sa.stage ? staged_lds : tables_lds) : 0;
@@ -528,8 +524,8 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         if (rc != LFFN_OK) return rc;
 
         if (grad_score) {
-            // token b's 32 columns of slice s sit at g_packed + (s * Bc + b) * 32
-            if (!lffn_internal_lookup_inner_quad_try(pa.code, pa.g_packed, SC, Bc * SC, tables, grad_score + c0 * T, Bc, T, S,
+            // token b's 32 columns of slice s sit at g_packed + (s * (Bc + 1) + b) * 32
+            if (!lffn_internal_lookup_inner_quad_try(pa.code, pa.g_packed, SC, (Bc + 1) * SC, tables, grad_score + c0 * T, Bc, T, S,
                                                      Do, stream, &rc))
                 rc = lffn_lookup_inner_f32(pa.code, pa.g, tables, grad_score + c0 * T, Bc, T, S, Do, stream);
             if (rc != LFFN_OK) return rc;
@@ -538,7 +534,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
 
         SortedArgs ma{};
         ma.pairs = pairs; ma.off8 = off8; ma.g = pa.g_packed; ma.out = grad_tables; ma.stride = stride; ma.rows = T * S;
-        ma.last_token = (unsigned)(Bc - 1);
+        ma.last_token = (unsigned)Bc;
         ma.T = (int)T; ma.S = (int)S; ma.Do = (int)Do; ma.nslices = (int)(Do / SC);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
         rc = launch_sorted(ma, st);
@@ -590,7 +586,8 @@ extern "C" int lffn_lookup_backward_f32(const int32_t *code, const float *score,
 //   rows_rank_kernel    a pair's place among the pairs of its row: the value its atomic add on the row's counter returns
 //   rows_claim_kernel   one workgroup per 256 rows (a "table" of the accumulation) scans their padded counts and takes that
 //                       much of the list; which table's part comes first does not matter
-//   rows_place_kernel   pairs into the list (and a row's padding by its first pair); other workgroups copy g slice-major
+//   rows_place_kernel   pairs into the list (and a row's padding, which names the zero row, by its first pair); other workgroups copy
+//                       g slice-major
 // The order inside a row is the order of arrival: sums differ from run to run in their last bit, as they did with
 // atomics.  Measured at 4096 x 128 x 512, 32768 rows: see launch_rows.
 namespace {
@@ -605,7 +602,7 @@ struct RowsArgs {
     int32_t *rank;         // [B * I]
     int32_t *off8;         // [tables, VT + 1]
     uint2 *pairs;
-    float *g_packed;       // [Dv / SC][B][SC]
+    float *g_packed;       // [Dv / SC][B + 1][SC], the last row zero
     int64_t B, n, rows;
     int I, Dv, tables, place_blocks;
 };
@@ -666,27 +663,28 @@ __global__ __launch_bounds__(256) void rows_place_kernel(RowsArgs a) {
             list[rank] = make_uint2(token, __float_as_uint(a.w[e]));
             if (rank == 0) {
                 const int c = a.count[row];
-                for (int p = c; p < ((c + 7) & ~7); ++p) list[p] = make_uint2(token, 0u);
+                for (int p = c; p < ((c + 7) & ~7); ++p) list[p] = make_uint2((unsigned)a.B, 0u);
             }
         }
         return;
     }
-    // four 16-byte pieces of g per thread
+    // four 16-byte pieces of g per thread, zeros past its end
     const int q = a.Dv / 4;
     const int64_t n = a.B * q, first = (int64_t(blockIdx.x) - a.place_blocks) * 1024 + threadIdx.x;
     float4 v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int64_t e = min(first + 256 * i, n - 1);
-        v[i] = load4(static_cast<const G *>(a.g) + e * 4);
+        const int64_t e = first + 256 * i;
+        v[i] = load4(static_cast<const G *>(a.g) + min(e, n - 1) * 4);
+        if (e >= n) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int64_t e = first + 256 * i;
-        if (e < n) {
+        if (e < n + q) {
             const int64_t b = e / q;
             const int col = (int)(e - b * q) * 4;
-            *reinterpret_cast<float4 *>(a.g_packed + ((size_t)(col / SC) * a.B + b) * SC + col % SC) = v[i];
+            *reinterpret_cast<float4 *>(a.g_packed + ((size_t)(col / SC) * (a.B + 1) + b) * SC + col % SC) = v[i];
         }
     }
 }
@@ -813,7 +811,7 @@ bool rows_supported(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
     const int64_t Bc = B < CHUNK ? B : CHUNK, tables = (rows + VT - 1) / VT;
     return Bc * I < (int64_t(1) << 31) - 8 * 256 && rows <= (int64_t(1) << 30) && B * I * 4 >= rows &&
            double(B) * double(I) * double(Dv) >= 3e6 && tables * ((Dv / SC + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff &&
-           Bc * Dv / 1024 < (int64_t(1) << 30);
+           (Bc + 1) * Dv / 1024 < (int64_t(1) << 30);
 }
 
 RowsWorkspace rows_layout(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
@@ -825,7 +823,7 @@ RowsWorkspace rows_layout(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
     w.pairs = w.off8 + round16(tables * (VT + 1) * 4);
     w.g_packed = w.pairs + (n + 7 * (n < rows ? n : rows)) * 8 + 8;
     w.g_packed = round16(w.g_packed);
-    w.total = w.g_packed + Bc * Dv * 4;
+    w.total = w.g_packed + (Bc + 1) * Dv * 4;
     return w;
 }
 
@@ -863,7 +861,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         const int64_t blocks = (a.n + 255) / 256;
         a.place_blocks = (int)(blocks < 4096 ? blocks : 4096);
         const bool sparse = a.n <= SPARSE_PAIRS * out_size;      // (no slice-major copy of g)
-        const int64_t pack_blocks = sparse ? 0 : (a.B * (Dv / 4) + 1023) / 1024;
+        const int64_t pack_blocks = sparse ? 0 : ((a.B + 1) * (Dv / 4) + 1023) / 1024;
         const int64_t zero4 = l.rank / 16;                      // the counters and the list's end
         hipLaunchKernelGGL(rows_zero_kernel, dim3((unsigned)((zero4 + 255) / 256 < 1024 ? (zero4 + 255) / 256 : 1024)), dim3(256), 0, st,
                            reinterpret_cast<int4 *>(base), zero4);
@@ -882,7 +880,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         }
         SortedArgs ma{};
         ma.pairs = a.pairs; ma.off8 = a.off8; ma.g = a.g_packed; ma.out = out; ma.stride = 0; ma.rows = out_size;
-        ma.last_token = (unsigned)(a.B - 1);
+        ma.last_token = (unsigned)a.B;
         ma.T = a.tables; ma.S = VT; ma.Do = (int)Dv; ma.nslices = (int)(Dv / SC);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
         rc = launch_sorted(ma, st);

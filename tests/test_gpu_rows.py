@@ -255,3 +255,40 @@ def test_rows_gradient_of_few_pairs(B, I, rows, Dv, dtype):
     got = ops.scatter_add(idx.cuda(), g.cuda(), w.float().cuda(), rows).cpu().double()
     n = torch.bincount(flat.long(), minlength=rows).double()[:, None]
     assert ((got - want).abs() <= (n + 4) * 2.0 ** -24 * scale).all()                # n additions in fp32
+
+
+def _assert_same_infinities(got, want):
+    got = torch.as_tensor(got).double()
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+
+
+# Lists are padded to multiples of eight pairs: the padding adds nothing, not 0 * infinity.  By slices and by wavefronts, tokens that
+# fill the copy of the gradient's last workgroup and a whole chunk of them
+@pytest.mark.parametrize("B,I,rows,Dv", [(513, 62, 300, 320), (1024, 64, 300, 64), (16384, 8, 300, 64), (512, 32, 2048, 192)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_rows_gradient_of_an_infinite_gradient(B, I, rows, Dv, dtype):
+    gen = torch.Generator().manual_seed(B)
+    idx = torch.randint(0, rows, (B, I), generator=gen, dtype=torch.int32)
+    g, w = torch.randn(B, Dv, generator=gen).to(dtype), (0.1 + torch.rand(B, I, generator=gen)).to(dtype)
+    g[0, 3], g[7, 5], g[B - 1, 0] = float("inf"), float("inf"), -float("inf")
+    want = torch.zeros(rows, Dv, dtype=torch.double)
+    for i in range(I):
+        want.index_add_(0, idx[:, i].long(), w[:, i].double()[:, None] * g.double())
+    src = torch.zeros(rows, Dv, dtype=dtype, device=DEV).requires_grad_()
+    lookupffn_amd.weighted_gather_add(idx.to(DEV), src, w.to(DEV)).backward(g.to(DEV))
+    _assert_same_infinities(src.grad.cpu(), want)
+
+
+@pytest.mark.parametrize("B", [2500, 2560, 16384, 16385])
+@pytest.mark.parametrize("S", [256, 512])
+def test_tables_gradient_of_an_infinite_gradient(B, S):
+    T, Do = 3, 64
+    gen = torch.Generator().manual_seed(B)
+    code = torch.randint(0, S, (B, T), generator=gen, dtype=torch.int32)
+    score, g = 0.1 + torch.rand(B, T, generator=gen), torch.randn(B, Do, generator=gen)
+    g[0, 3], g[64, 5], g[B - 1, 0] = float("inf"), float("inf"), -float("inf")
+    want = torch.zeros(T, S, Do, dtype=torch.double)
+    for t in range(T):
+        want[t].index_add_(0, code[:, t].long(), score[:, t].double()[:, None] * g.double())
+    _assert_same_infinities(cabi.lookup_scatter_sorted(code.numpy(), score.numpy(), g.numpy(), S), want)
