@@ -259,6 +259,15 @@ void column_sums(const Config &c, const float *a, float *out_a, int64_t na, cons
 // Inputs of the node, in the order of its gradients.
 enum Input { X, LN_W, LN_B, WEIGHT, PBIAS, TABLES, OBIAS, RESIDUAL, INPUTS };
 
+// What a graph through the layer's gradients (create_graph) ends in: the kernels compute them without one.
+struct NoSecondDerivative : public torch::autograd::Node {
+    std::string name() const override { return "LookupFFNNoSecondDerivative"; }
+    variable_list apply(variable_list &&) override {
+        TORCH_CHECK(false, "LookupFFN: the gradients of the layer cannot be differentiated (a graph through them was asked for with "
+                           "create_graph)");
+    }
+};
+
 struct LookupFFNBackward : public torch::autograd::Node {
     Config c{};
     int64_t B = 0;
@@ -271,6 +280,19 @@ struct LookupFFNBackward : public torch::autograd::Node {
     }
 
     variable_list apply(variable_list &&grads) override {
+        const bool graph = at::GradMode::is_enabled();
+        variable_list out = gradients(grads);
+        if (!graph) return out;
+        auto end = std::shared_ptr<NoSecondDerivative>(new NoSecondDerivative(), torch::autograd::deleteNode);
+        torch::autograd::edge_list edges = next_edges();                     // they depend on the inputs and on the gradient
+        for (auto &e : torch::autograd::collect_next_edges(grads[0])) edges.push_back(std::move(e));
+        end->set_next_edges(std::move(edges));
+        for (int i = 0; i < INPUTS; ++i)
+            if (i != RESIDUAL && out[i].defined()) torch::autograd::set_history(out[i], end);
+        return out;
+    }
+
+    variable_list gradients(const variable_list &grads) {
         variable_list out(INPUTS);
         if (!grads[0].defined()) return out;
         at::AutoGradMode no_grad(false);

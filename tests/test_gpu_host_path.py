@@ -151,3 +151,24 @@ def test_a_tangent_on_a_parameter_is_refused(block, name, first):
             torch.func.functional_call(layer, params, (x,))
     if not first:
         assert torch.equal(layer(x), want)
+
+
+@pytest.mark.parametrize("block", [1, 64])
+def test_a_graph_through_the_gradients_ends_in_an_error(block):
+    """create_graph: the gradients are the ones of an ordinary backward; a penalty on one of them raises, where it would
+    have added nothing.  The residual's gradient is the result's and can be differentiated."""
+    layer = _layer(block)
+    x, res = torch.randn(20, 256, device=DEV, requires_grad=True), torch.randn(20, 256, device=DEV, requires_grad=True)
+    inputs = [x, *layer.parameters()]
+    want = torch.autograd.grad(layer(x).square().sum(), inputs)
+    out = layer(x)
+    got = torch.autograd.grad(out.square().sum(), inputs, create_graph=True)
+    for a, b in zip(got, want):
+        assert a.requires_grad and torch.equal(a.detach(), b)
+        with pytest.raises(RuntimeError, match="differentiated"):
+            (out.sum() + a.square().sum()).backward(retain_graph=True)
+        with pytest.raises(RuntimeError, match="differentiated"):
+            torch.autograd.grad(a.sum(), inputs, allow_unused=True, retain_graph=True)
+    g, = torch.autograd.grad(layer(x, res).square().sum(), res, create_graph=True)
+    g.sum().backward()
+    assert torch.allclose(res.grad, torch.full_like(res, 2.0))
