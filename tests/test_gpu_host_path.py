@@ -172,3 +172,27 @@ def test_a_graph_through_the_gradients_ends_in_an_error(block):
     g, = torch.autograd.grad(layer(x, res).square().sum(), res, create_graph=True)
     g.sum().backward()
     assert torch.allclose(res.grad, torch.full_like(res, 2.0))
+
+
+@pytest.mark.parametrize("how", ["class", "layer", "patched"])
+def test_an_overridden_forward_is_called_every_time(how, monkeypatch):
+    calls, base = [], lookupffn_amd.LookupFFN._forward
+
+    def override(self, x, residual=None):
+        calls.append((tuple(x.shape), residual is not None))
+        return base(self, x, residual)
+
+    layer = _layer().eval()
+    x = torch.randn(2, 20, 256, device=DEV)
+    with torch.no_grad():
+        want = layer(x)
+        if how == "class":
+            layer.__class__ = type("Sub", (lookupffn_amd.LookupFFN,), {"_forward": override})
+        elif how == "layer":
+            layer._forward = lambda x, residual=None: override(layer, x, residual)
+        else:
+            monkeypatch.setattr(lookupffn_amd.LookupFFN, "_forward", override)
+        for _ in range(3):
+            assert torch.equal(layer(x), want)
+        layer(x, x)
+    assert calls == 3 * [((40, 256), False)] + [((40, 256), True)]
