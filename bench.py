@@ -521,17 +521,19 @@ def main():
     with torch.no_grad():
         fused_layer = layer.can_fuse_layer(x)      # few tokens: the layer is one launch, gather included
     # many tokens, diagonal BH4, fp32 tables: the projection kernel writes the gather's record stream itself
-    st = layer._inference_state()
+    proj, ln = layer.hash.projection, layer.LayerNorm
+    with torch.no_grad():
+        diag = None if block else proj.weight.reshape(proj.num_repeat, proj.weight.shape[1], proj.padded_in_dim)
+    coefs = float(proj.decay_coeff), float(1 - proj.decay_coeff)
     rec_plan = None
-    if not fused_layer and T % 2 == 0 and st is not None:
+    if not fused_layer and T % 2 == 0:
         rec_plan = ops.lookup_gather_records_plan(B, T, S, Do, fmt)
 
     def records_front():
         if block:
-            return ops.ln_bh4_block_hash_records_direct(x, st["ln_w"], st["ln_b"], st["eps"], layer.hash.folded_weight(),
-                                                        st["pbias"], T, st["decay"], st["res_coef"], rec_plan)
-        return ops.ln_project_hash_records_direct(x, st["ln_w"], st["ln_b"], st["eps"], st["diag"], st["pbias"],
-                                                  T, st["decay"], st["res_coef"], rec_plan)
+            return ops.ln_bh4_block_hash_records_direct(x, ln.weight, ln.bias, float(ln.eps), layer.hash.folded_weight(), proj.bias, T,
+                                                        *coefs, rec_plan)
+        return ops.ln_project_hash_records_direct(x, ln.weight, ln.bias, float(ln.eps), diag, proj.bias, T, *coefs, rec_plan)
 
     def step(events=None):
         # exactly what LookupFFN.forward runs in eval mode (checked below), with an
@@ -548,7 +550,7 @@ def main():
                 records = records_front()
                 if events is not None:
                     events[0].record()
-                out = ops.lookup_gather_records_direct(records, rec_plan, st["tables"], st["obias"], None, B)
+                out = ops.lookup_gather_records_direct(records, rec_plan, layer.tables, layer.bias, None, B)
                 if events is not None:
                     events[1].record()
                 return out
@@ -680,7 +682,7 @@ def main():
         else:
             if rec_plan is not None:
                 records = front()
-                gather_only = lambda: ops.lookup_gather_records_direct(records, rec_plan, st["tables"], st["obias"], None, B)
+                gather_only = lambda: ops.lookup_gather_records_direct(records, rec_plan, layer.tables, layer.bias, None, B)
             else:
                 code, score = hash_front()
                 gather_only = lambda: ops.lookup_gather(code, score, layer.tables, layer.bias)

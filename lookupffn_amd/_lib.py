@@ -174,7 +174,10 @@ def host():
                     from . import _host as module
                 except ImportError as e:
                     raise LookupFFNLibraryError(f"cannot load {path}: {e}") from e
-                module.bind_library(LIB_PATH)
+                from . import ops
+                from .lookup import BH4
+                module.bind(LIB_PATH, torch.nn.LayerNorm, BH4, (ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS,
+                                                               ops.PROJECT_BWD_PARTIALS, ops.COLUMN_SUM_CHUNK_ROWS))
                 _host = module
     return _host
 

@@ -6,10 +6,9 @@
 // checks what can have changed since the layer's parameters were last looked at, allocates its result and launches; a
 // training forward records one autograd node whose backward launches the whole chain.
 //
-// Python builds a handle (make_layer) when the parameters are of a kind the kernels are built for, and calls
-// forward(handle, layer, x, residual, ...).  The answer is None whenever anything is not as the handle expects: a module or a
-// parameter of another kind, another parameter object (each looked up through the layer's modules on every call), storage, dtype, sizes or strides, an input of another type, dtype, device or layout, a gradient wanted that this path does not
-// compute.  Then the Python path runs, with its own checks and errors.
+// forward(layer, x, residual, ...) looks its modules and parameters up on every call and keeps nothing of them.  The answer is
+// None whenever anything is not of a kind the kernels are built for: another module, sizes that do not fit together, a dtype,
+// device or layout, a gradient wanted that this path does not compute.  Then the Python path runs, with its own checks and errors.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -21,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -41,7 +41,7 @@ using at::Tensor;
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
-// The kernel library is the one Python has loaded (bind_library gets its path): its entry points by name.
+// The kernel library is the one Python has loaded (bind gets its path): its entry points by name.
 #define LFFN_ENTRIES(X)                     \
     X(lffn_error_string)                    \
     X(lffn_lookup_ffn_fused_layer_rows)     \
@@ -80,48 +80,45 @@ void check(int rc, const char *what) { TORCH_CHECK(rc == LFFN_OK, what, ": ", li
 
 enum Form { DIAG = 0, BLOCK = 1 };
 
-// Sizes and constants of a layer; the thresholds are the Python operators' own.  The last three are what the modules hold
-// at the call.
+// Sizes and constants of a layer.
 struct Config {
-    int64_t form, one_launch, H, D, R, J, T, S, Do, fmt;
-    int64_t sorted_min_work, ln_partials, project_partials, sum_chunk_rows, trainable;
+    int64_t form, H, D, R, J, T, S, Do, fmt;
+    bool one_launch, trainable;
     double eps, decay, residual;
 };
 
+// The Python operators' own (bind).
+struct Thresholds {
+    int64_t sorted_min_work, ln_partials, project_partials, sum_chunk_rows;
+} limits;
+PyTypeObject *layer_norm_type, *bh4_type;
+
+// Which form the gather takes for a batch, a function of the sizes alone.
 struct RecordPlan {
-    int64_t B = -1, stride = 0, bytes = 0, ws_bytes = 0;
+    std::array<int64_t, 6> sizes{-1};    // B, T, S, Do, row format, records possible
+    int64_t stride = 0, bytes = 0, ws_bytes = 0;
     int32_t tokens = 0;
 };
 
-// A parameter, and what it was when the handle was made.
-struct Watched {
-    PyObject *object;
-    const void *data;
-    at::ScalarType dtype;
-    std::vector<int64_t> sizes, strides;
-
-    bool same(const Tensor &t) const {
-        return t.data_ptr() == data && t.scalar_type() == dtype && t.sizes().equals(sizes) && t.strides().equals(strides);
-    }
-};
-
-// What the layer holds at this moment: it, its LayerNorm, its hash and the hash's projection as Python finds them on every
-// access, the parameters in them (in the order of Input below) and their constants.  Borrowed references.
+// What the layer holds at this moment: its hash, the hash's projection and its LayerNorm as Python finds them on every access, the
+// parameters in them (in the order of Input below) and their constants.  Borrowed references.
 struct Parts {
-    std::array<PyObject *, 4> modules;
+    PyObject *norm, *hash, *projection;
     std::array<PyObject *, 6> params;
     double eps, decay;
+    int64_t num_table, output_size;
 };
 
 PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES, *KEY_EPS,
-    *KEY_DECAY;                           // interned
+    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_FOLDED;      // interned
 
 PyObject *dict_of(PyObject *o) {
     PyObject **d = o ? _PyObject_GetDictPtr(o) : nullptr;
     return d ? *d : nullptr;
 }
 
-PyObject *item(PyObject *dict, PyObject *key) { return dict && PyDict_Check(dict) ? PyDict_GetItem(dict, key) : nullptr; }
+// (keys are strings: looking one up raises nothing)
+PyObject *item(PyObject *dict, PyObject *key) { return dict && PyDict_Check(dict) ? PyDict_GetItemWithError(dict, key) : nullptr; }
 
 bool number(PyObject *o, double &value) {
     if (!o || !(PyFloat_Check(o) || PyLong_Check(o))) return false;
@@ -133,35 +130,31 @@ bool number(PyObject *o, double &value) {
     return true;
 }
 
+bool whole(PyObject *o, int64_t &value) {
+    if (!o || !PyLong_Check(o)) return false;
+    int overflow = 0;
+    value = PyLong_AsLongLongAndOverflow(o, &overflow);
+    return !overflow;
+}
+
 // False when something is not where a LookupFFN has it (a reparametrised weight is no parameter but computed on every access).
 bool find_parts(PyObject *layer, Parts &found) {
     PyObject *own = dict_of(layer), *modules = item(own, KEY_MODULES);
-    PyObject *norm = item(modules, KEY_LAYER_NORM), *hash = item(modules, KEY_HASH);
-    PyObject *projection = item(item(dict_of(hash), KEY_MODULES), KEY_PROJECTION);
-    PyObject *of_layer = item(own, KEY_PARAMETERS), *of_norm = item(dict_of(norm), KEY_PARAMETERS),
-             *of_projection = item(dict_of(projection), KEY_PARAMETERS);
-    found.modules = {layer, norm, hash, projection};
-    found.params = {item(of_norm, KEY_WEIGHT),       item(of_norm, KEY_BIAS),      item(of_projection, KEY_WEIGHT),
+    found.norm = item(modules, KEY_LAYER_NORM);
+    found.hash = item(modules, KEY_HASH);
+    PyObject *norm = dict_of(found.norm), *hash = dict_of(found.hash);
+    found.projection = item(item(hash, KEY_MODULES), KEY_PROJECTION);
+    if (!found.norm || !found.projection || !PyObject_TypeCheck(found.norm, layer_norm_type) || !PyObject_TypeCheck(found.projection, bh4_type))
+        return false;
+    PyObject *projection = dict_of(found.projection), *of_layer = item(own, KEY_PARAMETERS), *of_norm = item(norm, KEY_PARAMETERS),
+             *of_projection = item(projection, KEY_PARAMETERS);
+    found.params = {item(of_norm, KEY_WEIGHT),       item(of_norm, KEY_BIAS),    item(of_projection, KEY_WEIGHT),
                     item(of_projection, KEY_BIAS), item(of_layer, KEY_TABLES), item(of_layer, KEY_BIAS)};
-    for (PyObject *o : found.modules)
-        if (!o) return false;
     for (PyObject *o : found.params)
-        if (!o) return false;
-    return number(item(dict_of(norm), KEY_EPS), found.eps) && number(item(dict_of(projection), KEY_DECAY), found.decay);
+        if (!o || !THPVariable_Check(o)) return false;
+    return number(item(norm, KEY_EPS), found.eps) && number(item(projection, KEY_DECAY), found.decay) &&
+           whole(item(own, KEY_NUM_TABLE), found.num_table) && whole(item(own, KEY_OUTPUT_SIZE), found.output_size);
 }
-
-struct Layer {
-    Config c{};
-    std::array<PyTypeObject *, 4> types;  // of the modules
-    std::vector<Watched> watched;
-    // lnw, lnb, weight, pbias, tables, obias (pbias may be undefined)
-    std::array<Tensor, 6> p;
-    Tensor folded;                       // BLOCK inference: the folded weights and the weight's version they belong to
-    uint32_t folded_version = 0;
-    PyObject *folded_dict = nullptr, *folded_key = nullptr, *folded_object = nullptr;
-    std::array<RecordPlan, 8> plans;     // a few batch sizes in turn; guarded by the interpreter lock
-    int next_plan = 0;
-};
 
 float *f32(const Tensor &t) { return t.defined() ? static_cast<float *>(t.data_ptr()) : nullptr; }
 
@@ -170,17 +163,21 @@ hipStream_t stream_on(const at::Device &d) { return c10::hip::getCurrentHIPStrea
 Tensor empty_f32(at::IntArrayRef sizes, const at::Device &d) { return at::empty(sizes, at::TensorOptions().dtype(at::kFloat).device(d)); }
 Tensor empty_bytes(int64_t n, const at::Device &d) { return at::empty({n}, at::TensorOptions().dtype(at::kByte).device(d)); }
 
-const RecordPlan &plan_for(Layer &l, int64_t B) {
-    for (const RecordPlan &p : l.plans)
-        if (p.B == B) return p;
-    RecordPlan &p = l.plans[l.next_plan];
-    l.next_plan = (l.next_plan + 1) % (int)l.plans.size();
-    const Config &c = l.c;
-    p = RecordPlan{};
-    if (c.T % 2 == 0 && (c.form == BLOCK || c.D >= 16))
-        CALL(lffn_lookup_gather_records_plan_rows, B, c.T, c.S, c.Do, (int32_t)c.fmt, &p.tokens, &p.stride, &p.bytes);
-    if (p.bytes == 0) CALL(lffn_lookup_gather_workspace_bytes, B, c.T, c.S, c.Do, (int32_t)c.fmt, &p.ws_bytes);
-    p.B = B;
+RecordPlan plan_for(const Config &c, int64_t B) {
+    // (the last plans by their sizes, guarded by the interpreter lock)
+    static std::array<RecordPlan, 64> known;
+    const std::array<int64_t, 6> sizes{B, c.T, c.S, c.Do, c.fmt, c.T % 2 == 0 && (c.form == BLOCK || c.D >= 16)};
+    size_t slot = 0;
+    for (int64_t n : sizes) slot = slot * 31 + (size_t)n;
+    RecordPlan &p = known[(slot ^ slot >> 12) % known.size()];
+    if (p.sizes != sizes) {
+        RecordPlan made;
+        if (sizes[5])
+            CALL(lffn_lookup_gather_records_plan_rows, B, c.T, c.S, c.Do, (int32_t)c.fmt, &made.tokens, &made.stride, &made.bytes);
+        if (made.bytes == 0) CALL(lffn_lookup_gather_workspace_bytes, B, c.T, c.S, c.Do, (int32_t)c.fmt, &made.ws_bytes);
+        made.sizes = sizes;
+        p = made;
+    }
     return p;
 }
 
@@ -201,51 +198,55 @@ void gather(const Config &c, const Tensor &codes, const Tensor &scores, const Te
              wp, ws_bytes, B, c.T, c.S, c.Do, st);
 }
 
-void infer(Layer &l, const Config &c, const Tensor &x, const float *residual, Tensor &out, int64_t B, int64_t fused_max) {
+// The layer's parameters: LayerNorm's, the projection's, tables and output bias.
+using Params = std::array<Tensor, 6>;
+
+void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor &x, const float *residual, Tensor &out, int64_t B,
+           int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     // (rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half
     // as many tokens more: 768 tokens, 128 tables of 768 columns 34 us against 55 in two launches, 512 of 1024 113 against 120)
     if (c.one_launch && B <= (c.fmt == 0 ? fused_max : fused_max + fused_max / 2)) {
-        const lffn_fused_layer layer{f32(l.p[0]), f32(l.p[1]), f32(l.p[2]), f32(l.p[3]), f32(l.p[4]), f32(l.p[5]), c.H, c.D, c.R, c.J, c.T,
+        const lffn_fused_layer layer{f32(p[0]), f32(p[1]), f32(p[2]), f32(p[3]), f32(p[4]), f32(p[5]), c.H, c.D, c.R, c.J, c.T,
                                      c.S, c.Do, (float)c.eps, (float)c.decay, (float)c.residual};
         CALL(lffn_lookup_ffn_fused_layer_rows, &layer, (int32_t)c.fmt, f32(x), residual, f32(out), B, st);
         return;
     }
     const float eps = (float)c.eps, decay = (float)c.decay, res = (float)c.residual;
-    const RecordPlan plan = plan_for(l, B);
+    const RecordPlan plan = plan_for(c, B);
     if (plan.bytes > 0) {
         // many tokens: the projection kernel writes the gather kernel's record stream directly
         Tensor records = empty_bytes(plan.bytes, dev);
         uint32_t *rp = static_cast<uint32_t *>(records.data_ptr());
         if (c.form == DIAG)
-            CALL(lffn_ln_project_hash_records_f32, f32(x), f32(l.p[0]), f32(l.p[1]), eps, f32(l.p[2]), f32(l.p[3]), rp, plan.stride,
+            CALL(lffn_ln_project_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, decay, res, st);
         else
-            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(l.p[0]), f32(l.p[1]), eps, f32(l.folded), f32(l.p[3]), rp, plan.stride,
+            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
-        CALL(lffn_lookup_gather_records_rows, rp, plan.stride, l.p[4].data_ptr(), f32(l.p[5]), residual, f32(out), B, c.T, c.S, c.Do,
+        CALL(lffn_lookup_gather_records_rows, rp, plan.stride, p[4].data_ptr(), f32(p[5]), residual, f32(out), B, c.T, c.S, c.Do,
              (int32_t)c.fmt, plan.tokens, st);
         return;
     }
     Tensor codes = at::empty({B, c.T}, at::TensorOptions().dtype(at::kInt).device(dev)), scores = empty_f32({B, c.T}, dev);
     int32_t *cp = static_cast<int32_t *>(codes.data_ptr());
     if (c.form == DIAG)
-        CALL(lffn_ln_project_hash_f32, f32(x), f32(l.p[0]), f32(l.p[1]), eps, f32(l.p[2]), f32(l.p[3]), nullptr, cp, f32(scores), B, c.H,
+        CALL(lffn_ln_project_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), nullptr, cp, f32(scores), B, c.H,
              c.D, c.R, c.J, c.T, decay, res, st);
     else
-        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(l.p[0]), f32(l.p[1]), eps, f32(l.folded), f32(l.p[3]), cp, f32(scores), B, c.H, c.D,
+        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), B, c.H, c.D,
              c.R, c.J, c.T, 64, decay, res, st);
-    gather(c, codes, scores, l.p[4], l.p[5], residual, out, B, plan.ws_bytes, st);
+    gather(c, codes, scores, p[4], p[5], residual, out, B, plan.ws_bytes, st);
 }
 
 // Column sums of one or two [P, n] arrays of partial sums, fixed order of additions; many rows go through a first
 // pass over chunks of rows on many workgroups.
-void column_sums(const Config &c, const float *a, float *out_a, int64_t na, const float *b, float *out_b, int64_t nb, int64_t P,
+void column_sums(const float *a, float *out_a, int64_t na, const float *b, float *out_b, int64_t nb, int64_t P,
                  const at::Device &dev, void *st) {
     Tensor mid;
-    if (P > 4 * c.sum_chunk_rows) {
-        int64_t chunks = (P + c.sum_chunk_rows - 1) / c.sum_chunk_rows;
+    if (P > 4 * limits.sum_chunk_rows) {
+        int64_t chunks = (P + limits.sum_chunk_rows - 1) / limits.sum_chunk_rows;
         const int64_t each = (P + chunks - 1) / chunks;
         chunks = (P + each - 1) / each;                    // no empty chunk
         mid = empty_f32({chunks * (na + nb)}, dev);
@@ -311,7 +312,7 @@ struct LookupFFNBackward : public torch::autograd::Node {
         if (need[RESIDUAL]) out[RESIDUAL] = grads[0];
         if (need[OBIAS]) {
             out[OBIAS] = empty_f32({Do}, dev);
-            column_sums(c, f32(g), f32(out[OBIAS]), Do, nullptr, nullptr, 0, B, dev, st);
+            column_sums(f32(g), f32(out[OBIAS]), Do, nullptr, nullptr, 0, B, dev, st);
         }
         const bool need_ln = need[X] || need[LN_W] || need[LN_B];
         const bool need_score = need_ln || need[WEIGHT] || need[PBIAS];
@@ -322,7 +323,7 @@ struct LookupFFNBackward : public torch::autograd::Node {
         if (need_score || need[TABLES]) {
             int64_t ws_bytes = 0;
             CALL(lffn_lookup_scatter_workspace_bytes, B, T, S, Do, &ws_bytes);
-            if (B <= LFFN_SCATTER_LIST_TOKENS || B * T * Do < c.sorted_min_work) ws_bytes = 0;
+            if (B <= LFFN_SCATTER_LIST_TOKENS || B * T * Do < limits.sorted_min_work) ws_bytes = 0;
             if (need[TABLES] && ws_bytes > 0) {
                 Tensor ws = empty_bytes(ws_bytes, dev);
                 if (need_score)
@@ -340,14 +341,14 @@ struct LookupFFNBackward : public torch::autograd::Node {
         const float decay = (float)c.decay, res = (float)c.residual, eps = (float)c.eps;
         Tensor g_h = empty_f32({R, B, H}, dev);            // gradient of the LayerNorm output, one slab per repeat
         if (c.form == DIAG) {
-            const int64_t n = std::max<int64_t>(1, std::min(c.project_partials, (B + 3) / 4));
+            const int64_t n = std::max<int64_t>(1, std::min(limits.project_partials, (B + 3) / 4));
             Tensor parts = empty_f32({n * R * (J + 1) * D}, dev);
             float *pd = f32(parts), *pb = pd + n * R * J * D;
             CALL(lffn_ln_project_hash_bwd_f32, f32(x_), f32(lw), f32(lb), eps, f32(w), f32(z_), f32(g_score), f32(g_h), pd, pb, B, H, D, R, J,
                  T, n, decay, res, st);
             if (need[WEIGHT] || need[PBIAS]) {
                 Tensor g_w = at::empty_like(w), g_b = empty_f32({R * D}, dev);
-                column_sums(c, pd, f32(g_w), R * J * D, pb, f32(g_b), R * D, n, dev, st);
+                column_sums(pd, f32(g_w), R * J * D, pb, f32(g_b), R * D, n, dev, st);
                 if (need[WEIGHT]) out[WEIGHT] = g_w;
                 if (need[PBIAS]) out[PBIAS] = g_b.narrow(0, 0, T * 8);
             }
@@ -367,14 +368,14 @@ struct LookupFFNBackward : public torch::autograd::Node {
             }
             if (need[PBIAS]) {
                 out[PBIAS] = empty_f32({T * 8}, dev);
-                column_sums(c, f32(g_z), f32(out[PBIAS]), T * 8, nullptr, nullptr, 0, B, dev, st);
+                column_sums(f32(g_z), f32(out[PBIAS]), T * 8, nullptr, nullptr, 0, B, dev, st);
             }
         }
         if (need_ln) {
-            const int64_t n = std::max<int64_t>(1, std::min(c.ln_partials, (B + 3) / 4));
+            const int64_t n = std::max<int64_t>(1, std::min(limits.ln_partials, (B + 3) / 4));
             Tensor parts = empty_f32({2 * n * H}, dev), g_x = at::empty_like(x_), g_lw = empty_f32({H}, dev), g_lb = empty_f32({H}, dev);
             CALL(lffn_layer_norm_bwd_f32, f32(x_), f32(lw), eps, f32(g_h), f32(g_x), f32(parts), f32(parts) + n * H, B, H, R, n, st);
-            column_sums(c, f32(parts), f32(g_lw), H, f32(parts) + n * H, f32(g_lb), H, n, dev, st);
+            column_sums(f32(parts), f32(g_lw), H, f32(parts) + n * H, f32(g_lb), H, n, dev, st);
             if (need[X]) out[X] = g_x;
             if (need[LN_W]) out[LN_W] = g_lw;
             if (need[LN_B]) out[LN_B] = g_lb;
@@ -383,7 +384,7 @@ struct LookupFFNBackward : public torch::autograd::Node {
     }
 };
 
-void train(Layer &l, const Config &c, const Tensor &x, const Tensor &residual, Tensor &out, int64_t B) {
+void train(const Config &c, const Params &p, const Tensor &x, const Tensor &residual, Tensor &out, int64_t B) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     auto node = std::shared_ptr<LookupFFNBackward>(new LookupFFNBackward(), torch::autograd::deleteNode);
@@ -392,28 +393,28 @@ void train(Layer &l, const Config &c, const Tensor &x, const Tensor &residual, T
     int32_t *cp = static_cast<int32_t *>(codes.data_ptr());
     const float eps = (float)c.eps, decay = (float)c.decay, res = (float)c.residual;
     if (c.form == DIAG) {
-        CALL(lffn_ln_project_hash_f32, f32(x), f32(l.p[0]), f32(l.p[1]), eps, f32(l.p[2]), f32(l.p[3]), f32(z), cp, f32(scores), B, c.H, c.D,
+        CALL(lffn_ln_project_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), f32(z), cp, f32(scores), B, c.H, c.D,
              c.R, c.J, c.T, decay, res, st);
     } else {
         stage = empty_f32({c.R, c.J - 1, B, c.D}, dev);
         stats = empty_f32({B, 2}, dev);
-        Tensor folded = at::empty_like(l.p[2]);
-        CALL(lffn_bh4_fold_mode_f32, f32(l.p[2]), f32(folded), c.R * c.J * (c.D / 64), 64, 0, st);
-        CALL(lffn_ln_bh4_block_hash_train_f32, f32(x), f32(l.p[0]), f32(l.p[1]), eps, f32(folded), f32(l.p[3]), cp, f32(scores), f32(z),
+        Tensor folded = at::empty_like(p[2]);
+        CALL(lffn_bh4_fold_mode_f32, f32(p[2]), f32(folded), c.R * c.J * (c.D / 64), 64, 0, st);
+        CALL(lffn_ln_bh4_block_hash_train_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), f32(z),
              c.J > 1 ? f32(stage) : nullptr, f32(stats), B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
     }
     int64_t ws_bytes = 0;
     CALL(lffn_lookup_gather_workspace_bytes, B, c.T, c.S, c.Do, (int32_t)c.fmt, &ws_bytes);
-    gather(c, codes, scores, l.p[4], l.p[5], f32(residual), out, B, ws_bytes, st);
+    gather(c, codes, scores, p[4], p[5], f32(residual), out, B, ws_bytes, st);
 
     node->c = c;
     node->B = B;
-    node->set_next_edges(torch::autograd::collect_next_edges(x, l.p[0], l.p[1], l.p[2], l.p[3], l.p[4], l.p[5], residual));
+    node->set_next_edges(torch::autograd::collect_next_edges(x, p[0], p[1], p[2], p[3], p[4], p[5], residual));
     node->x = SavedVariable(x, false);                      // (every one an input of the node or no part of the graph)
-    node->ln_w = SavedVariable(l.p[0], false);
-    node->ln_b = SavedVariable(l.p[1], false);
-    node->weight = SavedVariable(l.p[2], false);
-    node->tables = SavedVariable(l.p[4], false);
+    node->ln_w = SavedVariable(p[0], false);
+    node->ln_b = SavedVariable(p[1], false);
+    node->weight = SavedVariable(p[2], false);
+    node->tables = SavedVariable(p[4], false);
     node->codes = SavedVariable(codes, false);
     node->scores = SavedVariable(scores, false);
     node->z = SavedVariable(z, false);
@@ -424,25 +425,17 @@ void train(Layer &l, const Config &c, const Tensor &x, const Tensor &residual, T
 
 // ---------------------------------------------------------------- Python
 
-const char *CAPSULE = "lookupffn_amd.layer";
+// Tangents exist inside a forward-mode level only (asking a tensor for its own takes a lock).
+bool forward_mode() { return torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr; }
 
-void free_layer(PyObject *capsule) {
-    Layer *l = static_cast<Layer *>(PyCapsule_GetPointer(capsule, CAPSULE));
-    if (!l) return;
-    for (Watched &w : l->watched) Py_XDECREF(w.object);
-    for (PyTypeObject *t : l->types) Py_XDECREF(t);
-    Py_XDECREF(l->folded_dict);
-    Py_XDECREF(l->folded_key);
-    Py_XDECREF(l->folded_object);
-    delete l;
-}
-
-// An ordinary tensor: no transform of torch.func around it, nothing lazy, no tangent.
+// An ordinary tensor: no transform of torch.func around it, nothing lazy.
 bool ordinary(const Tensor &t) {
     constexpr c10::DispatchKeySet other({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Python,
                                          c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
-    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(other) && !t._fw_grad(/*level=*/0).defined();
+    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(other);
 }
+
+bool has_tangent(const Tensor &t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
 
 // and of no subclass
 bool plain(PyObject *o) { return THPVariable_CheckExact(o) && ordinary(THPVariable_Unpack(o)); }
@@ -456,9 +449,12 @@ bool watched_over() {
            c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize);
 }
 
-PyObject *bind_library(PyObject *, PyObject *path) {
+// bind(path of the kernel library, nn.LayerNorm, BH4, the operators' thresholds)
+PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    const char *p = PyUnicode_AsUTF8(path);
+    TORCH_CHECK(n == 4 && PyType_Check(args[1]) && PyType_Check(args[2]) && PyTuple_Check(args[3]) && PyTuple_GET_SIZE(args[3]) == 4,
+                "bind: a path, two types and four numbers");
+    const char *p = PyUnicode_AsUTF8(args[0]);
     if (!p) return nullptr;
     void *h = dlopen(p, RTLD_NOW | RTLD_NOLOAD);
     if (!h) h = dlopen(p, RTLD_NOW);
@@ -469,114 +465,115 @@ PyObject *bind_library(PyObject *, PyObject *path) {
     TORCH_CHECK(found.name, p, " has no ", #name);
     LFFN_ENTRIES(X)
 #undef X
+    Thresholds t{};
+    for (int i = 0; i < 4; ++i)
+        TORCH_CHECK(whole(PyTuple_GET_ITEM(args[3], i), (&t.sorted_min_work)[i]), "bind: a threshold is no integer");
+    Py_INCREF(args[1]);
+    Py_INCREF(args[2]);
     lib = found;
+    limits = t;
+    layer_norm_type = reinterpret_cast<PyTypeObject *>(args[1]);
+    bh4_type = reinterpret_cast<PyTypeObject *>(args[2]);
     Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS
 }
 
-// make_layer(config: 15 ints, layer, folded: (dict, key, object, tensor, version) or None) -> handle, or None when the
-// layer has not the parameters it was made with
-PyObject *make_layer(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    HANDLE_TH_ERRORS
-    TORCH_CHECK(n == 3, "make_layer: 3 arguments");
-    Parts parts;
-    if (!find_parts(args[1], parts)) Py_RETURN_NONE;
-    for (PyObject *o : parts.params)
-        if (o != Py_None && !(THPVariable_Check(o) && ordinary(THPVariable_Unpack(o)))) Py_RETURN_NONE;
-    auto l = std::make_unique<Layer>();
-    int64_t *ints = &l->c.form;
-    TORCH_CHECK(PyTuple_GET_SIZE(args[0]) == 15, "make_layer: sizes");
-    for (int i = 0; i < 15; ++i) ints[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(args[0], i));
-    if (PyErr_Occurred()) return nullptr;
-    for (int i = 0; i < 4; ++i) {
-        l->types[i] = Py_TYPE(parts.modules[i]);
-        Py_INCREF(l->types[i]);
-    }
-    for (int i = 0; i < 6; ++i) {
-        PyObject *o = parts.params[i];
-        if (o != Py_None) l->p[i] = THPVariable_Unpack(o);
-        Py_INCREF(o);
-        Watched w{o, nullptr, at::kFloat, {}, {}};
-        if (const Tensor &t = l->p[i]; t.defined()) {
-            w.data = t.data_ptr();
-            w.dtype = t.scalar_type();
-            w.sizes = t.sizes().vec();
-            w.strides = t.strides().vec();
-        }
-        l->watched.push_back(std::move(w));
-    }
-    if (args[2] != Py_None) {
-        l->folded_dict = PyTuple_GET_ITEM(args[2], 0);
-        l->folded_key = PyTuple_GET_ITEM(args[2], 1);
-        l->folded_object = PyTuple_GET_ITEM(args[2], 2);
-        for (PyObject *k : {l->folded_dict, l->folded_key, l->folded_object}) Py_INCREF(k);
-        l->folded = THPVariable_Unpack(PyTuple_GET_ITEM(args[2], 3));
-        l->folded_version = (uint32_t)PyLong_AsUnsignedLong(PyTuple_GET_ITEM(args[2], 4));
-    }
-    PyObject *capsule = PyCapsule_New(l.get(), CAPSULE, free_layer);
-    if (capsule) l.release();
-    return capsule;
-    END_HANDLE_TH_ERRORS
+// The layer's sizes from those of its parameters; false when they do not fit together or are not of a kind the kernels are built for.
+bool configure(const Parts &parts, const Params &p, const at::Device &dev, Config &c) {
+    for (int i = 0; i < 6; ++i)
+        if (!ordinary(p[i]) || p[i].device() != dev || !p[i].is_contiguous() || (i != 4 && p[i].scalar_type() != at::kFloat)) return false;
+    const Tensor &lw = p[0], &lb = p[1], &w = p[2], &pb = p[3], &tables = p[4], &ob = p[5];
+    if (w.dim() != 5 || tables.dim() != 3) return false;
+    const auto fmt = tables.scalar_type();
+    if (fmt != at::kFloat && fmt != at::kBFloat16 && fmt != at::kHalf) return false;
+    const int64_t bs = w.size(4);
+    c.form = bs == 64 ? BLOCK : DIAG;
+    c.fmt = fmt == at::kFloat ? 0 : fmt == at::kBFloat16 ? 1 : 2;
+    c.H = lw.numel();
+    c.R = w.size(0); c.J = w.size(1); c.D = w.size(2) * bs;
+    c.T = tables.size(0); c.S = tables.size(1); c.Do = tables.size(2);
+    c.eps = parts.eps; c.decay = parts.decay; c.residual = 1.0 - parts.decay;
+    if ((bs != 1 && bs != 64) || w.size(3) != bs || c.D < (bs == 64 ? 64 : 8) || c.D > 1024 || c.J < 1 || c.T < 1 || c.Do < 1) return false;
+    // (8 T values for T tables are codes of 8 bits)
+    if (c.T != parts.num_table || c.Do != parts.output_size || c.Do % 64 != 0 || c.S < 1 || (c.S & (c.S - 1)) != 0) return false;
+    // the projection as BH4 makes it for a hidden size of H and T codes: D the next power of two, as few repeats as give 8 T outputs
+    if (c.H > c.D || 2 * c.H <= c.D || (c.D & (c.D - 1)) != 0 || c.R != (8 * c.T + c.D - 1) / c.D) return false;
+    if (lb.numel() != c.H || pb.numel() != 8 * c.T || ob.numel() != c.Do || (c.form == BLOCK && c.H % 4 != 0)) return false;
+    c.one_launch = c.form == DIAG && c.D >= 256 && c.T <= 512 && c.S == 256;
+    c.trainable = c.fmt == 0 && c.H % 4 == 0 && (c.form == BLOCK || (c.D >= 256 && c.J <= 4));
+    return true;
 }
 
-// forward(handle, layer, x, residual or None, tokens up to which the one-launch form is taken) -> tensor or None
+// hash._folded = ((version, address, device), folded weights), as Hashing.folded_weight keeps them: the weights if they are w's.
+Tensor folded_of(PyObject *hash, const Tensor &w) {
+    PyObject *kept = item(dict_of(hash), KEY_FOLDED);
+    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 2) return {};
+    PyObject *key = PyTuple_GET_ITEM(kept, 0), *folded = PyTuple_GET_ITEM(kept, 1);
+    int64_t version = 0, address = 0;
+    if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
+        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(folded))
+        return {};
+    const Tensor &f = THPVariable_Unpack(folded);
+    const bool same = w._version() == (uint32_t)version && w.data_ptr() == reinterpret_cast<void *>(address) && f.device() == w.device() &&
+                      f.numel() == w.numel();
+    return same ? f : Tensor();
+}
+
+// forward(layer, x, residual or None, tokens up to which the one-launch form is taken) -> a tensor; None: not for this path;
+// False: the folded weights (Hashing.folded_weight) are not up to date
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(n == 5, "forward: 5 arguments");
-    Layer *l = static_cast<Layer *>(PyCapsule_GetPointer(args[0], CAPSULE));
-    if (!l) return nullptr;
-    Parts parts;
-    if (!find_parts(args[1], parts)) Py_RETURN_NONE;
-    Config c = l->c;
-    c.eps = parts.eps;
-    c.decay = parts.decay;
-    c.residual = 1.0 - parts.decay;
-    if (watched_over() || !plain(args[2])) Py_RETURN_NONE;
-    const Tensor &x = THPVariable_Unpack(args[2]);
-    const at::Device dev = l->p[4].device();
+    TORCH_CHECK(n == 4, "forward: 4 arguments");
+    if (watched_over() || !plain(args[1])) Py_RETURN_NONE;
+    Tensor x = THPVariable_Unpack(args[1]);
+    const at::Device dev = x.device();
     const int64_t dims = x.dim();
-    if (dims < 1 || x.size(dims - 1) != c.H || x.numel() == 0 || x.scalar_type() != at::kFloat || !x.is_contiguous() || x.device() != dev ||
-        c10::hip::current_device() != dev.index())
+    Parts parts;
+    if (dims < 1 || x.numel() == 0 || x.scalar_type() != at::kFloat || c10::hip::current_device() != dev.index() ||
+        !find_parts(args[0], parts))
         Py_RETURN_NONE;
+    Params params;
+    for (int i = 0; i < 6; ++i) params[i] = THPVariable_Unpack(parts.params[i]);
+    Config c{};
+    if (!configure(parts, params, dev, c) || x.size(dims - 1) != c.H) Py_RETURN_NONE;
     const int64_t B = x.numel() / c.H;
-    if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 != 0) Py_RETURN_NONE;
     c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
     sizes[dims - 1] = c.Do;
     Tensor residual;
-    if (args[3] != Py_None) {
-        if (!plain(args[3])) Py_RETURN_NONE;
-        residual = THPVariable_Unpack(args[3]);
-        if (residual.scalar_type() != at::kFloat || residual.device() != dev || !residual.is_contiguous() || !residual.sizes().equals(sizes) ||
-            reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 != 0)
-            Py_RETURN_NONE;
+    if (args[2] != Py_None) {
+        if (!plain(args[2])) Py_RETURN_NONE;
+        residual = THPVariable_Unpack(args[2]);
+        if (residual.device() != dev || residual.numel() != B * c.Do) Py_RETURN_NONE;
+    }
+    if (forward_mode()) {
+        bool any = has_tangent(x) || has_tangent(residual);
+        for (const Tensor &t : params) any = any || has_tangent(t);
+        if (any) Py_RETURN_NONE;
     }
     bool grads = false;
-    const bool grad_mode = at::GradMode::is_enabled();
-    if (grad_mode) grads = x.requires_grad() || (residual.defined() && residual.requires_grad());
-    for (size_t i = 0; i < l->types.size(); ++i)
-        if (Py_TYPE(parts.modules[i]) != l->types[i]) Py_RETURN_NONE;
-    for (size_t i = 0; i < l->watched.size(); ++i) {
-        const Watched &w = l->watched[i];
-        if (parts.params[i] != w.object) Py_RETURN_NONE;
-        const Tensor &p = l->p[i];
-        if (!p.defined()) continue;
-        if (!ordinary(p) || !w.same(p)) Py_RETURN_NONE;
-        if (grad_mode) grads = grads || p.requires_grad();
+    if (at::GradMode::is_enabled()) {
+        grads = x.requires_grad() || (residual.defined() && residual.requires_grad());
+        for (const Tensor &t : params) grads = grads || t.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;
-    if (!grads && c.form == BLOCK &&
-        (!l->folded.defined() || PyDict_GetItem(l->folded_dict, l->folded_key) != l->folded_object || l->p[2]._version() != l->folded_version))
+    Tensor folded;
+    if (!grads && c.form == BLOCK && !(folded = folded_of(parts.hash, params[2])).defined()) Py_RETURN_FALSE;
+    // any layout of x and any shape and type of the residual, as the Python path makes them
+    x = x.contiguous();
+    if (residual.defined() && !(residual.scalar_type() == at::kFloat && residual.is_contiguous() && residual.sizes().equals(sizes)))
+        residual = residual.reshape(sizes).to(at::kFloat).contiguous();
+    if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 != 0 ||
+        (residual.defined() && reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 != 0))
         Py_RETURN_NONE;
     Tensor out = empty_f32(sizes, dev);
-    if (grads) train(*l, c, x, residual, out, B);
-    else infer(*l, c, x, f32(residual), out, B, PyLong_AsLongLong(args[4]));
+    if (grads) train(c, params, x, residual, out, B);
+    else infer(c, params, folded, x, f32(residual), out, B, PyLong_AsLongLong(args[3]));
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {
-    {"bind_library", bind_library, METH_O, nullptr},
-    {"make_layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(make_layer)), METH_FASTCALL, nullptr},
+    {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(bind)), METH_FASTCALL, nullptr},
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(forward)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
@@ -589,7 +586,8 @@ PyMODINIT_FUNC PyInit__host() {
     const std::pair<PyObject **, const char *> keys[] = {
         {&KEY_MODULES, "_modules"}, {&KEY_PARAMETERS, "_parameters"}, {&KEY_LAYER_NORM, "LayerNorm"}, {&KEY_HASH, "hash"},
         {&KEY_PROJECTION, "projection"}, {&KEY_WEIGHT, "weight"}, {&KEY_BIAS, "bias"}, {&KEY_TABLES, "tables"},
-        {&KEY_EPS, "eps"}, {&KEY_DECAY, "decay_coeff"},
+        {&KEY_EPS, "eps"}, {&KEY_DECAY, "decay_coeff"}, {&KEY_NUM_TABLE, "num_table"},
+        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_FOLDED, "_folded"},
     };
     for (const auto &[key, name] : keys)
         if (!(*key = PyUnicode_InternFromString(name))) return nullptr;

@@ -367,15 +367,6 @@ class LookupFFN(nn.Module):
         self.tables = nn.Parameter(0.02 * torch.randn(self.num_table, self.table_size, self.output_size))
         self.bias = nn.Parameter(0.001 * torch.randn(self.output_size))
 
-    def __getstate__(self):
-        # the cached parameter views are derived data: not pickled with the module
-        state = super().__getstate__() if hasattr(super(), "__getstate__") else self.__dict__.copy()
-        state = dict(state)
-        state.pop("_inference_cache", None)
-        state.pop("_handle", None)
-        state.pop("_handle_key", None)
-        return state
-
     def extra_repr(self):
         return (f"hidden_size={self.hidden_size}, num_table={self.num_table}, "
                 f"table_size={self.table_size}, output_size={self.output_size}")
@@ -399,98 +390,33 @@ class LookupFFN(nn.Module):
         if not (x.shape[0] <= most and x.is_cuda and x.dtype == torch.float32
                 and self._no_gradient_wanted(x)):
             return False
-        st = self._inference_state()
-        return st is not None and st["one_launch"]
-
-    def _inference_state(self):
-        """What the inference kernels take from the parameters, or None when the parameters are not of
-        a kind those kernels are built for; worked out once and kept until a parameter is replaced,
-        moved or cast or a constant changed (in-place updates keep the storage, so the cached views stay good).  A launch
-        is a few microseconds: re-deriving this on every call cost more than the kernels at small
-        batches.  Keys: form ("diag": one kernel for LayerNorm + diagonal BH4 + hash; "block": the
-        matrix-core kernel for 64 x 64 blocks), one_launch (the whole layer in one kernel is possible),
-        and the detached parameter views."""
-        p = self.hash.projection
-        ln = self.LayerNorm
-        params = (ln.weight, ln.bias, getattr(p, "weight", None), getattr(p, "bias", None), self.tables, self.bias)
-        key = tuple((id(q), q.data_ptr(), q.dtype) if q is not None else None for q in params)
-        key += (getattr(ln, "eps", None), getattr(p, "decay_coeff", None))
-        cached = getattr(self, "_inference_cache", None)
-        if cached is not None and cached[0] == key:
-            return cached[1]
-        small = (ln.weight, ln.bias, getattr(p, "weight", None), getattr(p, "bias", None), self.bias)
-        ok = (isinstance(p, BH4) and self.hash.code_length == 8 and ln.elementwise_affine
-              and ln.weight is not None and ln.bias is not None and p.in_dim == self.hidden_size
-              and all(q is None or (q.dtype == torch.float32 and q.is_cuda and q.is_contiguous()
-                                    and q.device == self.tables.device) for q in small)
-              and self.tables.is_cuda and self.tables.is_contiguous()
-              and ops.row_format(self.tables.dtype) is not None and self.output_size % 64 == 0)
-        if ok:
-            # sizes that do not fit together are for the general path to refuse: the kernels take them from the layer
-            R, D, bs = p.num_repeat, p.padded_in_dim, p.block_size
-            ok = (ln.weight.numel() == ln.bias.numel() == self.hidden_size <= D
-                  and p.weight.dim() == 5 and p.weight.shape == (R, p.weight.shape[1], D // bs, bs, bs)
-                  and 8 * self.num_table <= R * D and (p.bias is None or p.bias.numel() == 8 * self.num_table)
-                  and self.tables.shape == (self.num_table, self.table_size, self.output_size)
-                  and self.bias.numel() == self.output_size)
-        form = None
-        if ok and p.block_size == 1 and 8 <= p.padded_in_dim <= 1024:
-            form = "diag"
-        elif ok and p.block_size == 64 and 64 <= p.padded_in_dim <= 1024 and p.in_dim % 4 == 0:
-            form = "block"
-        state = None
-        if form is not None:
-            state = dict(
-                form=form,
-                one_launch=(form == "diag" and p.padded_in_dim >= 256 and self.num_table <= 512
-                            and self.table_size == 256),
-                ln_w=ln.weight.detach(), ln_b=ln.bias.detach(), eps=float(ln.eps),
-                diag=(p.weight.detach().reshape(p.num_repeat, p.weight.shape[1], p.padded_in_dim)
-                      if form == "diag" else None),
-                pbias=None if p.bias is None else p.bias.detach(), tables=self.tables.detach(),
-                obias=self.bias.detach(), decay=float(p.decay_coeff), res_coef=float(1 - p.decay_coeff))
-        self._inference_cache = (key, state)
-        return state
+        p, ln = self.hash.projection, self.LayerNorm
+        if not (isinstance(p, BH4) and p.block_size == 1 and self.hash.code_length == 8 and isinstance(ln, nn.LayerNorm)):
+            return False
+        small = (ln.weight, ln.bias, p.weight, p.bias, self.bias)
+        return (256 <= p.padded_in_dim <= 1024 and self.num_table <= 512 and self.table_size == 256 and self.output_size % 64 == 0
+                and self.tables.is_cuda and ops.row_format(self.tables.dtype) is not None
+                and all(q is not None and q.is_cuda and q.dtype == torch.float32 for q in small))
 
     def _forward_host(self, x, residual):
         """The layer through the host path (csrc/host.cpp), or None when the call or the parameters are not of a kind it is
-        built for.  Its handle holds for as long as the parameters it names are those of the layer, its LayerNorm and its
-        projection, with the storage and dtype they had (and, without gradient, the folded 64 x 64 blocks the weights they were folded from)."""
-        if not (x.is_cuda and x.dtype == torch.float32 and self.tables.is_cuda):
-            return None
-        st = self._inference_state()
-        if st is None:
-            return None
-        fold = st["form"] == "block" and self._no_gradient_wanted(x)
-        if fold:
+        built for.  x [..., hidden] and residual [..., output_size] as the caller has them."""
+        forward = _lib.host().forward
+        out = forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
+        if out is False:                  # the 64 x 64 blocks have changed since they were folded
             self.hash.folded_weight()
-        key = (st, self.hash._folded if fold else None)
-        known = self.__dict__.get("_handle_key")
-        if known is None or known[0] is not st or (fold and known[1] is not key[1]):
-            self._handle, self._handle_key = self._make_handle(st, key[1]), key
-        if self._handle is None:
-            return None
-        return _lib.host().forward(self._handle, self, x.contiguous(), None if residual is None else residual.contiguous(),
-                                   self.FUSED_LAYER_MAX_TOKENS)
-
-    def _make_handle(self, st, folded):
-        p = self.hash.projection
-        block = st["form"] == "block"
-        R, J, D = p.num_repeat, p.weight.shape[1], p.padded_in_dim
-        trainable = (self.tables.dtype == torch.float32 and self.hidden_size % 4 == 0 and self.hidden_size <= 1024
-                     and (block or (256 <= D and J <= 4)))
-        return _lib.host().make_layer(
-            (int(block), int(st["one_launch"]), self.hidden_size, D, R, J, self.num_table, self.table_size, self.output_size,
-             ops.row_format(self.tables.dtype), ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS, ops.PROJECT_BWD_PARTIALS,
-             ops.COLUMN_SUM_CHUNK_ROWS, int(trainable)),
-            self,
-            None if folded is None else (self.hash.__dict__, "_folded", folded, folded[1], p.weight._version))
+            out = forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
+        return None if out is False else out
 
     def _forward(self, hidden_states, residual=None):
         if not torch.compiler.is_compiling():
             out = self._forward_host(hidden_states, residual)
             if out is not None:
                 return out
+        return self._forward_operators(hidden_states, residual)
+
+    def _forward_operators(self, hidden_states, residual):
+        """The reference's operator sequence, x [tokens, hidden] and fp32 residual [tokens, output_size]."""
         ln = self.LayerNorm
         ln_fusable = (ln.elementwise_affine and ln.weight is not None and ln.bias is not None
                       and ln.weight.dtype == torch.float32
@@ -531,12 +457,13 @@ class LookupFFN(nn.Module):
     def forward(self, hidden_states, residual=None):
         """PL/lookup.py:110-118.  ``residual`` (not in the reference; shape [..., output_size]) is
         added to the result inside the gather kernel: the encoder layer's "FFN(x) + x"."""
-        handle = self.__dict__.get("_handle")
-        if (handle is not None and type(self)._forward is _LAYER_FORWARD and "_forward" not in self.__dict__
-                and not torch.compiler.is_compiling()):
+        own = type(self)._forward is _LAYER_FORWARD and "_forward" not in self.__dict__
+        if own and not torch.compiler.is_compiling():
             # (before anything else: at a few hundred tokens the layer is one launch of a few microseconds, and every view
             # made here shows in its time)
-            out = _lib.host().forward(handle, self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS)
+            out = _lib.host().forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS)
+            if out is False:
+                out = self._forward_host(hidden_states, residual)
             if out is not None:
                 return out
         shape = hidden_states.shape[:-1]

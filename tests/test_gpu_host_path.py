@@ -196,3 +196,51 @@ def test_an_overridden_forward_is_called_every_time(how, monkeypatch):
             assert torch.equal(layer(x), want)
         layer(x, x)
     assert calls == 3 * [((40, 256), False)] + [((40, 256), True)]
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("block", [1, 64])
+def test_nothing_of_a_layer_is_held_between_calls(block, train):
+    """Replaced parameters are freed at once, and torch.utils.swap_tensors, which wants no other reference, works."""
+    layer = _layer(block)
+    x = torch.randn(40, 256, device=DEV)
+    _pass(layer, x, train), _pass(layer, x, train)
+    layer.zero_grad(set_to_none=True)
+    for name in ("tables", "bias"):
+        torch.utils.swap_tensors(getattr(layer, name), torch.nn.Parameter(torch.ones_like(getattr(layer, name))))
+    for m in (layer.LayerNorm, layer.hash.projection):
+        torch.utils.swap_tensors(m.weight, torch.nn.Parameter(m.weight.detach().clone()))
+    with torch.no_grad():
+        code, score = layer.hash(layer.LayerNorm(x))
+    _assert_same([_pass(layer, x, train)[0]], [(score.sum(1) + 1)[:, None].expand(40, 256)])
+    layer.zero_grad(set_to_none=True)
+    before, size = torch.cuda.memory_allocated(), layer.tables.numel() * 4
+    layer.tables = None
+    assert torch.cuda.memory_allocated() <= before - size
+
+
+def test_inputs_as_a_caller_has_them():
+    """Layouts of the input, shapes and types of the residual: the gradients and results of contiguous fp32 ones."""
+    layer = _layer(out=128)
+    x, res = torch.randn(6, 10, 256, device=DEV), torch.randn(6, 10, 128, device=DEV)
+    g = torch.randn(6, 10, 128, device=DEV)
+
+    def run(x, res):
+        leaves = [t.detach().clone(memory_format=torch.preserve_format).requires_grad_() for t in (x, res)]
+        out = layer(*leaves)
+        assert out.shape == x.shape[:-1] + (128,) and out.is_contiguous()
+        return [out.detach(), *torch.autograd.grad(out, [*leaves, layer.tables], g.reshape(out.shape))]
+
+    want = run(x, res)
+    strided = torch.empty(10, 6, 256, device=DEV).transpose(0, 1).copy_(x)
+    for a, b in ((strided, res), (x, res.reshape(60, 128)), (x, res.double()), (strided, res.to(torch.float64).reshape(-1))):
+        got = run(a, b)
+        assert got[2].shape == b.shape and got[2].dtype == b.dtype
+        for p, q in zip(got, want):
+            assert torch.equal(p.reshape(q.shape).float(), q)
+    half = run(x, res.to(torch.bfloat16))
+    _assert_same(half[:1], run(x, res.to(torch.bfloat16).float())[:1])
+    with torch.no_grad():
+        assert torch.allclose(layer(strided, res), want[0], rtol=1e-4, atol=1e-5)
+        with pytest.raises(RuntimeError):
+            layer(x, res[:5])
