@@ -472,7 +472,7 @@ class LookupFFN(nn.Module):
         hidden_states = hidden_states.reshape(tokens, dim)
         if residual is not None:
             residual = residual.reshape(tokens, self.output_size).float()
-        outputs = self._forward(hidden_states, residual)
+        outputs = (self._forward_operators if own else self._forward)(hidden_states, residual)
         return outputs.reshape(*shape, self.output_size)
 
     def gather(self, indexes, weights, tables):

@@ -8,6 +8,7 @@ import torch
 import torch.autograd.forward_ad as fwAD
 
 import lookupffn_amd
+from lookupffn_amd import _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -244,3 +245,40 @@ def test_inputs_as_a_caller_has_them():
         assert torch.allclose(layer(strided, res), want[0], rtol=1e-4, atol=1e-5)
         with pytest.raises(RuntimeError):
             layer(x, res[:5])
+
+
+@pytest.mark.parametrize("kind", ["taken", "dense projection", "fp64", "watched", "overridden"])
+def test_the_host_path_is_tried_once_a_call(kind, monkeypatch):
+    layer = _layer().eval()
+    x = torch.randn(20, 256, device=DEV)
+    if kind == "dense projection":
+        layer.hash.projection = torch.nn.Linear(256, 256).to(DEV)
+    elif kind == "fp64":
+        layer, x = layer.double(), x.double()
+    elif kind == "overridden":
+        layer.__class__ = type("Sub", (lookupffn_amd.LookupFFN,), {"_forward": lambda self, *a: super(type(self), self)._forward(*a)})
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    tries, real = [], _lib.host().forward
+
+    class Counted:
+        @staticmethod
+        def forward(*args):
+            out = real(*args)
+            tries.append(out is not None)
+            return out
+
+    monkeypatch.setattr(_lib, "host", lambda: Counted)
+    with torch.no_grad():
+        for _ in range(2):
+            if kind == "watched":
+                with Watch():
+                    layer(x)
+            elif kind == "fp64":                       # (which the operators refuse)
+                with pytest.raises((AssertionError, RuntimeError)):
+                    layer(x)
+            else:
+                layer(x)
+    assert tries == 2 * [kind in ("taken", "overridden")]
