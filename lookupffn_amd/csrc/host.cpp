@@ -30,6 +30,7 @@
 #include <array>
 #include <atomic>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -164,8 +165,10 @@ Tensor empty_f32(at::IntArrayRef sizes, const at::Device &d) { return at::empty(
 Tensor empty_bytes(int64_t n, const at::Device &d) { return at::empty({n}, at::TensorOptions().dtype(at::kByte).device(d)); }
 
 RecordPlan plan_for(const Config &c, int64_t B) {
-    // (the last plans by their sizes, guarded by the interpreter lock)
+    // the last plans by their sizes
     static std::array<RecordPlan, 64> known;
+    static std::mutex lock;
+    const std::lock_guard<std::mutex> guard(lock);
     const std::array<int64_t, 6> sizes{B, c.T, c.S, c.Do, c.fmt, c.T % 2 == 0 && (c.form == BLOCK || c.D >= 16)};
     size_t slot = 0;
     for (int64_t n : sizes) slot = slot * 31 + (size_t)n;
@@ -519,6 +522,12 @@ Tensor folded_of(PyObject *hash, const Tensor &w) {
     return same ? f : Tensor();
 }
 
+// Other threads run while this one allocates and launches: either may wait (for memory, for room in a full queue).
+struct WithoutInterpreter {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutInterpreter() { PyEval_RestoreThread(state); }
+};
+
 // forward(layer, x, residual or None, tokens up to which the one-launch form is taken) -> a tensor; None: not for this path;
 // False: the folded weights (Hashing.folded_weight) are not up to date
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -558,16 +567,24 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (grads && !c.trainable) Py_RETURN_NONE;
     Tensor folded;
     if (!grads && c.form == BLOCK && !(folded = folded_of(parts.hash, params[2])).defined()) Py_RETURN_FALSE;
-    // any layout of x and any shape and type of the residual, as the Python path makes them
-    x = x.contiguous();
-    if (residual.defined() && !(residual.scalar_type() == at::kFloat && residual.is_contiguous() && residual.sizes().equals(sizes)))
-        residual = residual.reshape(sizes).to(at::kFloat).contiguous();
-    if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 != 0 ||
-        (residual.defined() && reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 != 0))
-        Py_RETURN_NONE;
-    Tensor out = empty_f32(sizes, dev);
-    if (grads) train(c, params, x, residual, out, B);
-    else infer(c, params, folded, x, f32(residual), out, B, PyLong_AsLongLong(args[3]));
+    const int64_t fused_max = PyLong_AsLongLong(args[3]);
+    if (fused_max == -1 && PyErr_Occurred()) return nullptr;
+    Tensor out;
+    {
+        // (from here on only what is owned here is used: x, the residual, the parameters and the folded weights)
+        const WithoutInterpreter unlocked;
+        // any layout of x and any shape and type of the residual, as the Python path makes them
+        x = x.contiguous();
+        if (residual.defined() && !(residual.scalar_type() == at::kFloat && residual.is_contiguous() && residual.sizes().equals(sizes)))
+            residual = residual.reshape(sizes).to(at::kFloat).contiguous();
+        if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
+            (!residual.defined() || reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0)) {
+            out = empty_f32(sizes, dev);
+            if (grads) train(c, params, x, residual, out, B);
+            else infer(c, params, folded, x, f32(residual), out, B, fused_max);
+        }
+    }
+    if (!out.defined()) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }

@@ -1,6 +1,9 @@
 """The layer's host path (csrc/host.cpp) takes what it computes with from the layer on every call: a layer that was called before
 and then changed is compared with one that was changed before its first call."""
 import copy
+import sys
+import threading
+import time
 from argparse import Namespace
 
 import pytest
@@ -282,3 +285,62 @@ def test_the_host_path_is_tried_once_a_call(kind, monkeypatch):
             else:
                 layer(x)
     assert tries == 2 * [kind in ("taken", "overridden")]
+
+
+def test_other_threads_run_while_a_call_waits():
+    """An allocation that has to go to the driver takes long enough for a thread that waits for the interpreter to get it."""
+    layer = _layer(hidden=1024).eval()
+    x = torch.randn(8192, 1024, device=DEV)
+    count, stop, interval = [0], threading.Event(), sys.getswitchinterval()
+
+    def spin():
+        while not stop.is_set():
+            count[0] += 1
+            time.sleep(0)
+
+    thread, moved = threading.Thread(target=spin), []
+    with torch.no_grad():
+        layer(x)
+        try:
+            sys.setswitchinterval(1.0)           # (nothing but a release gives the interpreter away)
+            thread.start()
+            for _ in range(20):
+                torch.cuda.synchronize()
+                torch.cuda.empty_cache()
+                before = count[0]
+                layer(x)
+                moved.append(count[0] > before)
+        finally:
+            stop.set()
+            sys.setswitchinterval(interval)
+            thread.join()
+    assert sum(moved) >= 10
+
+
+def test_threads_and_streams_of_their_own():
+    """Calls of several threads on one layer, each on a stream of its own, inference and training: every one's result."""
+    layer = _layer()
+    inputs = [torch.randn(40 * (i + 1), 256, device=DEV) for i in range(4)]
+    with torch.no_grad():
+        want = [layer(x) for x in inputs]
+    torch.cuda.synchronize()
+    failed = []
+
+    def work(i):
+        x = inputs[i].clone().requires_grad_()
+        with torch.cuda.stream(torch.cuda.Stream()):
+            torch.cuda.synchronize()
+            for _ in range(30):
+                with torch.no_grad():
+                    out = layer(x)
+                grad, = torch.autograd.grad(layer(x).sum(), x)
+                torch.cuda.current_stream().synchronize()
+                if not (torch.equal(out, want[i]) and torch.isfinite(grad).all()):
+                    failed.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
