@@ -46,7 +46,7 @@ def _build_host() -> None:
                 "/opt/rocm/include", sysconfig.get_paths()["include"]]
     tmp = HOST_PATH + ".tmp"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f'-DLFFN_TORCH_VERSION="{torch.__version__}"',
            *[a for d in includes for a in ("-isystem", d)], os.path.join(CSRC, "host.cpp"), "-o", tmp,
            "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
     res = subprocess.run(cmd, capture_output=True, text=True)

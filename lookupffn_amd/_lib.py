@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch
 
@@ -156,29 +157,37 @@ def load() -> ctypes.CDLL:
         return _lib
 
 
-_host = None
+HOST_PATH = os.path.join(_PKG_DIR, "_host.so")
+_host = None                    # False: not to be had
+
+
+def _load_host():
+    if not os.path.exists(HOST_PATH):
+        raise ImportError(f"{HOST_PATH} is missing")
+    from . import _host as module
+    if module.torch_version != str(torch.__version__):
+        raise ImportError(f"{HOST_PATH} was built against torch {module.torch_version}, this is {torch.__version__}")
+    from . import ops
+    from .lookup import BH4
+    module.bind(LIB_PATH, torch.nn.LayerNorm, BH4, (ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS,
+                                                   ops.PROJECT_BWD_PARTIALS, ops.COLUMN_SUM_CHUNK_ROWS))
+    return module
 
 
 def host():
-    """The layer's host path (csrc/host.cpp, built next to the kernel library), bound to the loaded kernel library; raise
-    if it is absent."""
+    """The layer's host path (csrc/host.cpp, built next to the kernel library), bound to the loaded kernel library.  False where
+    it is missing or was built against another torch: the layer then calls the same kernels from Python."""
     global _host
     if _host is None:
         load()
         with _lock:
             if _host is None:
-                path = os.path.join(_PKG_DIR, "_host.so")
-                if not os.path.exists(path):
-                    raise LookupFFNLibraryError(f"{path} is missing: build it with `python -m lookupffn_amd._build`")
                 try:
-                    from . import _host as module
+                    _host = _load_host()
                 except ImportError as e:
-                    raise LookupFFNLibraryError(f"cannot load {path}: {e}") from e
-                from . import ops
-                from .lookup import BH4
-                module.bind(LIB_PATH, torch.nn.LayerNorm, BH4, (ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS,
-                                                               ops.PROJECT_BWD_PARTIALS, ops.COLUMN_SUM_CHUNK_ROWS))
-                _host = module
+                    warnings.warn(f"lookupffn_amd: the host path of LookupFFN is not available ({e}): its calls cost more host time.  "
+                                  "Build it with `python -m lookupffn_amd._build`", RuntimeWarning)
+                    _host = False
     return _host
 
 

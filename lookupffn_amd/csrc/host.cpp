@@ -608,5 +608,7 @@ PyMODINIT_FUNC PyInit__host() {
     };
     for (const auto &[key, name] : keys)
         if (!(*key = PyUnicode_InternFromString(name))) return nullptr;
-    return PyModule_Create(&module);
+    PyObject *made = PyModule_Create(&module);
+    if (made && PyModule_AddStringConstant(made, "torch_version", LFFN_TORCH_VERSION) != 0) Py_CLEAR(made);
+    return made;
 }

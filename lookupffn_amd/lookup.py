@@ -401,11 +401,13 @@ class LookupFFN(nn.Module):
     def _forward_host(self, x, residual):
         """The layer through the host path (csrc/host.cpp), or None when the call or the parameters are not of a kind it is
         built for.  x [..., hidden] and residual [..., output_size] as the caller has them."""
-        forward = _lib.host().forward
-        out = forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
+        host = _lib.host()
+        if not host:
+            return None
+        out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         if out is False:                  # the 64 x 64 blocks have changed since they were folded
             self.hash.folded_weight()
-            out = forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
+            out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         return None if out is False else out
 
     def _forward(self, hidden_states, residual=None):
@@ -461,7 +463,8 @@ class LookupFFN(nn.Module):
         if own and not torch.compiler.is_compiling():
             # (before anything else: at a few hundred tokens the layer is one launch of a few microseconds, and every view
             # made here shows in its time)
-            out = _lib.host().forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS)
+            host = _lib.host()
+            out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS) if host else None
             if out is False:
                 out = self._forward_host(hidden_states, residual)
             if out is not None:

@@ -7,6 +7,8 @@ No kernel is launched here.
 import ctypes
 import os
 import re
+import sys
+import warnings
 from argparse import Namespace
 
 import pytest
@@ -399,3 +401,21 @@ def test_attention_fused_equals_literal_formula_on_cpu():
         emb.word_embeddings.weight[ids] + emb.token_type_embeddings.weight[0] + emb.position_embeddings.weight[pos + 2],
         (64,), emb.LayerNorm.weight, emb.LayerNorm.bias, 1e-5)
     assert torch.allclose(out, want, atol=1e-6)
+
+
+@pytest.mark.parametrize("why", ["missing", "does not load", "another torch"])
+def test_a_host_path_that_is_not_to_be_had_is_said_once_and_done_without(why, monkeypatch):
+    assert _lib.host()                                       # built next to the kernel library
+    monkeypatch.setattr(_lib, "_host", None)
+    if why == "missing":
+        monkeypatch.setattr(_lib, "HOST_PATH", "/nonexistent/_host.so")
+    elif why == "does not load":
+        monkeypatch.delattr(lookupffn_amd, "_host", raising=False)
+        monkeypatch.setitem(sys.modules, "lookupffn_amd._host", None)
+    else:
+        monkeypatch.setattr(torch, "__version__", "0.0")
+    with pytest.warns(RuntimeWarning, match="host path"):
+        assert _lib.host() is False
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host() is False

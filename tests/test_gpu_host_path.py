@@ -344,3 +344,13 @@ def test_threads_and_streams_of_their_own():
     for t in threads:
         t.join()
     assert not failed
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("block", [1, 64])
+def test_a_layer_without_the_host_path_gives_the_same(block, train, monkeypatch):
+    layer = _layer(block)
+    x = torch.randn(40, 256, device=DEV)
+    want = [t.clone() for t in _pass(layer, x, train)]
+    monkeypatch.setattr(_lib, "_host", False)
+    _assert_same(_pass(layer, x, train), want)
