@@ -507,10 +507,11 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._folded = ((version, address, device), folded weights), as Hashing.folded_weight keeps them: the weights if they are w's.
+// hash._folded = ((version, address, device), folded weights, what they were folded from), as Hashing.folded_weight keeps them: the
+// folded weights if they are w's.
 Tensor folded_of(PyObject *hash, const Tensor &w) {
     PyObject *kept = item(dict_of(hash), KEY_FOLDED);
-    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 2) return {};
+    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3) return {};
     PyObject *key = PyTuple_GET_ITEM(kept, 0), *folded = PyTuple_GET_ITEM(kept, 1);
     int64_t version = 0, address = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||

@@ -187,14 +187,21 @@ class Hashing(nn.Module):
         version counter, which in-place writes through ``.data`` (``w.data.add_(...)``, some
         hand-written optimizers) do not advance: after such a write call
         ``invalidate_folded_weight()``; switching the module between train() and eval() drops
-        the cached copy as well."""
+        the cached copy as well.  The weights it was folded from stay allocated with it, so that no
+        other weight takes their address."""
         w = self.projection.weight
         key = (w._version, w.data_ptr(), w.device)
         cached = getattr(self, "_folded", None)
         if cached is None or cached[0] != key:
-            cached = (key, ops.bh4_fold(w.detach().contiguous()))
+            alias = w.detach()
+            cached = (key, ops.bh4_fold(alias.contiguous()), alias)
             self._folded = cached
         return cached[1]
+
+    def __getstate__(self):
+        state = self.__dict__.copy()
+        state.pop("_folded", None)        # derived from the weight, and names its address
+        return state
 
     def invalidate_folded_weight(self):
         """Forget the folded copy of the BH4 weights: the next block-64 inference call folds again."""

@@ -354,3 +354,25 @@ def test_a_layer_without_the_host_path_gives_the_same(block, train, monkeypatch)
     want = [t.clone() for t in _pass(layer, x, train)]
     monkeypatch.setattr(_lib, "_host", False)
     _assert_same(_pass(layer, x, train), want)
+
+
+def test_folded_blocks_are_those_of_the_weight_the_layer_has():
+    """A weight that takes the address and the version number of one that was freed is another weight."""
+    layer, fresh = _layer(64).eval(), _layer(64).eval()
+    x = torch.randn(40, 256, device=DEV)
+    p = layer.hash.projection
+    new = torch.randn(p.weight.shape) / 128
+    with torch.no_grad():
+        layer(x)
+        address, p.weight = p.weight.data_ptr(), None
+        tries = [new.to(DEV)]
+        while tries[-1].data_ptr() != address and len(tries) < 64:
+            tries.append(new.to(DEV))
+        p.weight = torch.nn.Parameter(tries[-1])
+        fresh.hash.projection.weight = torch.nn.Parameter(new.to(DEV))
+        assert torch.equal(layer(x), fresh(x))
+        for a, b in zip(layer.hash(x), fresh.hash(x)):
+            assert torch.equal(a, b)
+        twin = copy.deepcopy(layer)
+        assert "_folded" not in twin.hash.__dict__            # (it names an address of the other layer's)
+        assert torch.equal(twin(x), layer(x))
