@@ -136,54 +136,76 @@ __global__ __launch_bounds__(WG) void lookup_scatter_lds_kernel(ScatterArgs a) {
 
 // The same for few tokens.  Most rows of the gradient are then zero and the rest sums of a few products, and the kernel above
 // spends its time clearing and emptying 128 KB of LDS with one workgroup on a compute unit.  Here a workgroup owns 32 rows of a
-// table: it lists the (token, score) pairs of each row, and a wavefront adds up a row's products in registers (in fp64, as
-// above) and writes the whole row: plain streaming stores from many wavefronts.  A row's pairs are listed in any order, which
+// table, every groups-th: it lists the (token, score) pairs of each row, and a wavefront adds up a row's products in registers (in
+// fp64, as above) and writes the whole row: plain streaming stores from many wavefronts.  A row's pairs are listed in any order, which
 // fp64 sums do not show but for ties of the final rounding.  128 tables of 768 columns: 64 tokens 35.8 -> 18.2 us (100 MB
 // written: 5.5 TB/s), 1024 tokens 76.5 -> 35.5, 2048 112 -> 77 (the sorted form 102), 3072 131 against the sorted form's 112; 512
-// tables of 1024 columns: 64 tokens 179 -> 100, 2048 430 (sorted 453).  32 tables of 256 columns: 7.0 -> 7.7, 2048 18.7 -> 18.9.
+// tables of 1024 columns: 64 tokens 179 -> 100, 2048 430 (sorted 453).
+//
+// Rows of many pairs would leave that to one wavefront, a chain of loads (2048 tokens of which half fall on one row of 128 tables of
+// 768 columns: 264 us).  A row of more than LONG_ROW pairs, and of four times the average, is summed by all workgroups of its
+// table, a slice of the columns each: every one of them lists it beside its own short rows.  Half on one row 83 us, all on one 426 ->
+// 69, codes with Zipf's distribution 219 -> 95-100 (112 above, whatever the distribution); evenly spread codes as before (77).
 constexpr int ROWS_PER_WG = 32;
 constexpr int LIST_MAX_B = LFFN_SCATTER_LIST_TOKENS;
 constexpr int LIST_BATCHES = LIST_MAX_B / 256;
+constexpr int LONG_ROW = 32;
+constexpr int SLICE_QUADS = 16;                    // fewest columns of a slice, in fours
 
 template <int NC>
-__global__ __launch_bounds__(256) void lookup_scatter_list_kernel(ScatterArgs a, int groups) {
-    __shared__ int count[ROWS_PER_WG], start[ROWS_PER_WG + 1], cursor[ROWS_PER_WG];
-    __shared__ uint2 list[LIST_MAX_B];
+__global__ __launch_bounds__(256) void lookup_scatter_list_kernel(ScatterArgs a, int groups, int long_from) {
+    __shared__ int count[MAX_S], start[MAX_S], cursor[MAX_S], wave_sum[4], long_row[LIST_MAX_B / LONG_ROW], nlong;
+    __shared__ double part[4][256];                // (columns by threads: no bank conflicts)
+    extern __shared__ double lds[];
+    uint2 *list = reinterpret_cast<uint2 *>(lds);  // [B]: the listed rows have no token in common
     const int unit = (int)(blockIdx.x % XCDS) * a.per_xcd + (int)(blockIdx.x / XCDS);     // neighbouring tables on one XCD
     if (unit >= a.T * groups) return;              // uniform over the workgroup
-    const int t = unit / groups, row0 = (unit % groups) * ROWS_PER_WG;
+    const int t = unit / groups, group = unit % groups;
     const int nrows = min(ROWS_PER_WG, a.S);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto mine = [&](int r) { return (r & (groups - 1)) == group; };     // its rows: group + groups * i
     int row[LIST_BATCHES];
 #pragma unroll
     for (int k = 0; k < LIST_BATCHES; ++k) {
         const int64_t b = tid + 256 * k;
-        row[k] = b < a.B ? (a.code[b * a.T + t] & (a.S - 1)) - row0 : -1;
+        row[k] = b < a.B ? a.code[b * a.T + t] & (a.S - 1) : -1;
     }
-    if (tid < ROWS_PER_WG) count[tid] = 0;
+    count[tid] = 0;
+    if (tid == 0) nlong = 0;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < LIST_BATCHES; ++k)
-        if ((unsigned)row[k] < (unsigned)nrows) atomicAdd(&count[row[k]], 1);
+        if (row[k] >= 0) atomicAdd(&count[row[k]], 1);
     __syncthreads();
-    if (tid <= ROWS_PER_WG) {
-        int n = 0;
-        for (int r = 0; r < tid; ++r) n += count[r];
-        start[tid] = n;
-        if (tid < ROWS_PER_WG) cursor[tid] = n;
+    {   // a row per thread: where its list starts, if it is listed here
+        const int n = count[tid], listed = mine(tid) || n > long_from ? n : 0;
+        int inc = listed;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(inc, d);
+            if (lane >= d) inc += v;
+        }
+        if (lane == 63) wave_sum[wave] = inc;
+        if (n > long_from) long_row[atomicAdd(&nlong, 1)] = tid;
+        __syncthreads();
+        int before = inc - listed;
+        for (int w = 0; w < wave; ++w) before += wave_sum[w];
+        start[tid] = before;
+        cursor[tid] = listed ? before : -1;
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < LIST_BATCHES; ++k)
-        if ((unsigned)row[k] < (unsigned)nrows) {
+        if (row[k] >= 0 && (mine(row[k]) || count[row[k]] > long_from)) {
             const int b = tid + 256 * k;
             list[atomicAdd(&cursor[row[k]], 1)] = make_uint2((unsigned)b, __float_as_uint(a.score[(int64_t)b * a.T + t]));
         }
     __syncthreads();
-    for (int r = wave; r < nrows; r += 4) {
-        const int n0 = __builtin_amdgcn_readfirstlane(start[r]), n1 = __builtin_amdgcn_readfirstlane(start[r + 1]);
-        float *dst = a.out + ((size_t)t * a.S + row0 + r) * a.Do;
+    for (int i = wave; i < nrows; i += 4) {
+        const int r = group + groups * i;
+        const int n0 = __builtin_amdgcn_readfirstlane(start[r]), n1 = n0 + __builtin_amdgcn_readfirstlane(count[r]);
+        if (n1 - n0 > long_from) continue;
+        float *dst = a.out + ((size_t)t * a.S + r) * a.Do;
         for (int col0 = 0; col0 < a.Do; col0 += 256 * NC) {
             double acc[NC][4];
             int col[NC];
@@ -226,6 +248,50 @@ __global__ __launch_bounds__(256) void lookup_scatter_list_kernel(ScatterArgs a,
             }
         }
     }
+    // long rows: this workgroup's columns, in fours, a thread each; what threads that leaves share out the pairs
+    const int quads = a.Do / 4, slices = min(groups, max(1, quads / SLICE_QUADS));
+    if (group >= slices) return;                   // uniform
+    const int q_end = (int)((int64_t)quads * (group + 1) / slices);
+    for (int i = 0; i < nlong; ++i) {
+        const int r = long_row[i], n0 = start[r], n = count[r];
+        for (int q0 = (int)((int64_t)quads * group / slices); q0 < q_end; q0 += 64) {
+            const int width = min(64, q_end - q0), shares = 256 / width, share = tid / width, q = q0 + tid % width;
+            double acc[4] = {0.0, 0.0, 0.0, 0.0};
+            if (share < shares)
+                for (int k = share; k < n; k += 8 * shares) {
+                    float4 gv[8];
+                    float sv[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const uint2 pr = list[n0 + min(k + u * shares, n - 1)];
+                        sv[u] = __uint_as_float(pr.y);
+                        gv[u] = *reinterpret_cast<const float4 *>(a.g + (size_t)pr.x * a.Do + 4 * q);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (k + u * shares < n) {
+                            acc[0] += (double)(sv[u] * gv[u].x); acc[1] += (double)(sv[u] * gv[u].y);
+                            acc[2] += (double)(sv[u] * gv[u].z); acc[3] += (double)(sv[u] * gv[u].w);
+                        }
+                }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[e][tid] = acc[e];
+            __syncthreads();
+            if (tid < width) {
+                for (int w = 1; w < shares; ++w)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[e] += part[e][tid + w * width];
+                float4 v = make_float4((float)acc[0], (float)acc[1], (float)acc[2], (float)acc[3]);
+                float4 *dst = reinterpret_cast<float4 *>(a.out + ((size_t)t * a.S + r) * a.Do + 4 * q);
+                if (a.accumulate) {
+                    const float4 old = *dst;
+                    v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
+                }
+                *dst = v;
+            }
+            __syncthreads();
+        }
+    }
 }
 
 int launch_list(const ScatterArgs &args, hipStream_t st) {
@@ -233,11 +299,13 @@ int launch_list(const ScatterArgs &args, hipStream_t st) {
     const int groups = a.S > ROWS_PER_WG ? a.S / ROWS_PER_WG : 1;
     a.per_xcd = (a.T * groups + XCDS - 1) / XCDS;
     const dim3 grid((unsigned)(a.per_xcd * XCDS));
+    const size_t lds_bytes = (size_t)a.B * sizeof(uint2);
+    const int average = (int)((a.B + a.S - 1) / a.S), long_from = 4 * average > LONG_ROW ? 4 * average : LONG_ROW;
     switch ((a.Do + 255) / 256) {
-        case 1: hipLaunchKernelGGL(lookup_scatter_list_kernel<1>, grid, dim3(256), 0, st, a, groups); break;
-        case 2: hipLaunchKernelGGL(lookup_scatter_list_kernel<2>, grid, dim3(256), 0, st, a, groups); break;
-        case 3: hipLaunchKernelGGL(lookup_scatter_list_kernel<3>, grid, dim3(256), 0, st, a, groups); break;
-        default: hipLaunchKernelGGL(lookup_scatter_list_kernel<4>, grid, dim3(256), 0, st, a, groups); break;
+        case 1: hipLaunchKernelGGL(lookup_scatter_list_kernel<1>, grid, dim3(256), lds_bytes, st, a, groups, long_from); break;
+        case 2: hipLaunchKernelGGL(lookup_scatter_list_kernel<2>, grid, dim3(256), lds_bytes, st, a, groups, long_from); break;
+        case 3: hipLaunchKernelGGL(lookup_scatter_list_kernel<3>, grid, dim3(256), lds_bytes, st, a, groups, long_from); break;
+        default: hipLaunchKernelGGL(lookup_scatter_list_kernel<4>, grid, dim3(256), lds_bytes, st, a, groups, long_from); break;
     }
     return lffn_launch_status();
 }
@@ -280,7 +348,10 @@ extern "C" int lffn_lookup_scatter_f32(const int32_t *code, const float *score, 
     a.nslices = (int)(Do / COLS);
     a.per_xcd = (int)((units + XCDS - 1) / XCDS);
     a.accumulate = accumulate;
-    if (B <= LIST_MAX_B && T * S <= (int64_t(1) << 30)) return launch_list(a, st);
+    // The LDS form takes its time per round of one workgroup on each of 256 compute units: with a single round it is the faster one
+    // (32 tables of 256 columns: 64 tokens 7.0 us against 7.7, 512 9.4 against 10.8).  So it is where a table is one workgroup of the
+    // list form and has many tokens (128 tables of 32 x 768: 512 tokens 36.5 against 35, 1024 60.5 against 60.3, 2048 96 against 134).
+    if (units > 256 && B <= (S > ROWS_PER_WG ? LIST_MAX_B : 512) && T * S <= (int64_t(1) << 30)) return launch_list(a, st);
     const size_t lds_bytes = size_t(S) * COLS * 8 + size_t(WAVES) * 64 * 8;
     static LdsGrant granted;      // one record per kernel instantiation
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_lds_kernel), lds_bytes, granted)) return LFFN_ERR_LAUNCH;

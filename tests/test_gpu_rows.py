@@ -292,3 +292,25 @@ def test_tables_gradient_of_an_infinite_gradient(B, S):
     for t in range(T):
         want[t].index_add_(0, code[:, t].long(), score[:, t].double()[:, None] * g.double())
     _assert_same_infinities(cabi.lookup_scatter_sorted(code.numpy(), score.numpy(), g.numpy(), S), want)
+
+
+# Rows of few tokens' gradients at and past the length from which a table's workgroups share a row out by columns: one slice of
+# columns, uneven ones, several passes of one, tables of one and of several workgroups
+@pytest.mark.parametrize("T,S,Do", [(3, 256, 64), (2, 256, 320), (1, 64, 832), (2, 256, 4672), (2, 16, 256)])
+def test_gather_gradients_of_long_rows(T, S, Do):
+    rng = np.random.RandomState(T + Do)
+    lengths = [64, 65, 66, 200, 1]                                    # of rows 0, 1, 2, 9 and S - 1
+    filled = np.repeat(np.array([0, 1, 2, 9, S - 1], np.int32), lengths)
+    code = np.stack([rng.permutation(np.concatenate([filled, rng.randint(10, S, 700)])) for _ in range(T)], 1).astype(np.int32)
+    B = len(code)
+    score, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    init = rng.randn(T, S, Do).astype(np.float32)
+    want, scale = np.zeros((T, S, Do)), np.zeros((T, S, Do))
+    for t in range(T):
+        products = score[:, t, None].astype(np.float64) * g
+        np.add.at(want[t], code[:, t], products)
+        np.add.at(scale[t], code[:, t], np.abs(products))
+    # products rounded to fp32, summed in fp64, the sum (and the one onto `init`) rounded to fp32
+    assert (np.abs(cabi.lookup_scatter(code, score, g, S) - want) <= 2 * 2.0 ** -24 * scale).all()
+    got = cabi.lookup_scatter(code, score, g, S, accumulate=True, init=init)
+    assert (np.abs(got - want - init) <= 3 * 2.0 ** -24 * (scale + np.abs(init))).all()
