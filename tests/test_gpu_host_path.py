@@ -376,3 +376,33 @@ def test_folded_blocks_are_those_of_the_weight_the_layer_has():
         twin = copy.deepcopy(layer)
         assert "_folded" not in twin.hash.__dict__            # (it names an address of the other layer's)
         assert torch.equal(twin(x), layer(x))
+
+
+# The backward exists twice, as one node in C++ and as the operators' autograd functions: at sizes where the forms of a kernel change
+# (few tokens' gradients to 384, one-launch column sums to 1024 rows, lists to 2048, the sorted scatter and its chunks), for every
+# gradient and for each one alone
+@pytest.mark.parametrize("block,B,H,T,out", [(1, 1, 256, 32, 64), (64, 1, 256, 32, 64), (1, 384, 252, 34, 320), (64, 385, 512, 64, 512),
+                                             (64, 1025, 700, 33, 192), (1, 2048, 1024, 128, 256), (1, 2049, 768, 128, 768),
+                                             (64, 4097, 768, 128, 768), (1, 16385, 512, 32, 768)])
+def test_both_backward_chains_agree(block, B, H, T, out, monkeypatch):
+    layer = _layer(block, hidden=H, tables=T, out=out).train()
+    gen = torch.Generator(device=DEV).manual_seed(B)
+    x, res, g = (torch.randn(B, n, device=DEV, generator=gen) for n in (H, out, out))
+
+    def run(wanted):
+        leaves = dict(x=x.clone(), residual=res.clone(), **dict(layer.named_parameters()))
+        for name, t in leaves.items():
+            t.requires_grad_(wanted in (name, "all"))
+        result = layer(leaves["x"], leaves["residual"])
+        names = [name for name, t in leaves.items() if t.requires_grad]
+        return dict(zip(["out", *names], [result.detach(), *torch.autograd.grad(result, [leaves[n] for n in names], g)]))
+
+    wanted = ["all"] + (["x", "residual"] + [n for n, _ in layer.named_parameters()] if B < 5000 else [])
+    host = [run(w) for w in wanted]
+    monkeypatch.setattr(_lib, "_host", False)
+    for w, got in zip(wanted, host):
+        want = run(w)
+        assert got.keys() == want.keys()
+        for name in want:
+            # the same kernels; sums over the tokens that workgroups add up in the order they end differ in fp32's last bits
+            assert (got[name] - want[name]).abs().max() <= 2e-6 * want[name].abs().max() + 1e-30, (w, name)
