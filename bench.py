@@ -3,14 +3,14 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload cfg2|cfg1|cfg3|cfg3bf16|cfg3f16|cfg2b64|cmp512|cfg4|cfg5]
 
 A step is one forward pass of the layer over one batch of synthetic tokens that
-is already resident in HBM: fused LayerNorm+projection+hash kernel -> gather-add
-kernel (+bias), i.e. LookupFFN.forward in eval mode.  Prints ONE JSON line:
+is already resident in HBM: LookupFFN.forward in eval mode, whose kernels are a fused
+LayerNorm+projection+hash and a gather-add (+bias).  Prints ONE JSON line:
 
   value        whole-layer forward tokens/s (BASELINE.json's metric, config 2 by default)
   roofline     the gather-add kernel against the bound that binds it.  The table-major
                kernels serve every row read from LDS, so the bound is the LDS read
                path: achieved = B*T*Do*e row bytes per launch / the kernel's average
-               duration (HIP events on the launch stream, inside the timed region),
+               duration (HIP events around launches of it alone, after the timed region),
                peak = 256 B/clk/CU x 256 CUs x 2.4 GHz.  Beside it: the compulsory
                HBM bytes (tables + codes + scores + output, each once) and the
                fabric traffic measured with rocprofv3 --pmc, as fractions of 8 TB/s,
@@ -529,41 +529,43 @@ def main():
     if not fused_layer and T % 2 == 0:
         rec_plan = ops.lookup_gather_records_plan(B, T, S, Do, fmt)
 
-    def records_front():
-        if block:
-            return ops.ln_bh4_block_hash_records_direct(x, ln.weight, ln.bias, float(ln.eps), layer.hash.folded_weight(), proj.bias, T,
-                                                        *coefs, rec_plan)
-        return ops.ln_project_hash_records_direct(x, ln.weight, ln.bias, float(ln.eps), diag, proj.bias, T, *coefs, rec_plan)
+    # The stages on their own, by the entry points of the C ABI that LookupFFN.forward goes through
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    records = torch.empty(rec_plan[2] // 4, dtype=torch.int32, device=dev) if rec_plan is not None else None
+    staged_out = torch.empty(B, Do, dtype=torch.float32, device=dev)
 
-    def step(events=None):
-        # exactly what LookupFFN.forward runs in eval mode (checked below), with an
-        # event pair around the gather launch
+    def records_front():
+        sizes = (B, H, proj.padded_in_dim, proj.num_repeat, proj.weight.shape[1], T)
+        head = (x.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(), float(ln.eps))
+        tail = (proj.bias.data_ptr(), records.data_ptr(), rec_plan[1], rec_plan[0])
+        if block:
+            _lib.check(lib.lffn_ln_bh4_block_hash_records_f32(*head, layer.hash.folded_weight().data_ptr(), *tail, *sizes, 64, *coefs,
+                                                              stream), "lffn_ln_bh4_block_hash_records_f32")
+        else:
+            _lib.check(lib.lffn_ln_project_hash_records_f32(*head, diag.data_ptr(), *tail, *sizes, *coefs, stream),
+                       "lffn_ln_project_hash_records_f32")
+
+    def records_gather():
+        _lib.check(lib.lffn_lookup_gather_records_rows(records.data_ptr(), rec_plan[1], layer.tables.data_ptr(), layer.bias.data_ptr(), None,
+                                                       staged_out.data_ptr(), B, T, S, Do, fmt, rec_plan[0], stream),
+                   "lffn_lookup_gather_records_rows")
+        return staged_out
+
+    def step():
         with torch.no_grad():
-            if fused_layer:
-                if events is not None:
-                    events[0].record()
-                out = layer._forward(x)
-                if events is not None:
-                    events[1].record()
-                return out
-            if rec_plan is not None:
-                records = records_front()
-                if events is not None:
-                    events[0].record()
-                out = ops.lookup_gather_records_direct(records, rec_plan, layer.tables, layer.bias, None, B)
-                if events is not None:
-                    events[1].record()
-                return out
-            code, score = hash_front()
-            if events is not None:
-                events[0].record()
-            out = ops.lookup_gather(code, score, layer.tables, layer.bias)
-            if events is not None:
-                events[1].record()
-        return out
+            return layer(x)
 
     with torch.no_grad():
-        assert torch.equal(step(), layer(x)), "bench step and LookupFFN.forward disagree"
+        if fused_layer:
+            front, gather_only = None, step
+        elif rec_plan is not None:
+            front, gather_only = records_front, records_gather
+            front()
+        else:
+            front = hash_front
+            code, score = front()
+            gather_only = lambda: ops.lookup_gather(code, score, layer.tables, layer.bias)
+        assert torch.equal(gather_only(), step()), "the stages and LookupFFN.forward disagree"
 
     if args.calibrate_copy:
         calibrate_copy(dev)
@@ -573,8 +575,6 @@ def main():
     settle_steps, settle_ms = (0, 0.0) if args.no_settle else settle(step)
     for _ in range(args.warmup):
         step()
-    torch.cuda.synchronize()
-    evs = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(args.steps)]
     torch.cuda.synchronize()
     if args.graph:
         side = torch.cuda.Stream()
@@ -588,27 +588,28 @@ def main():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(graph_out, step()), "graph replay and eager step disagree"
-        t0 = time.perf_counter()
-        for i in range(args.steps):
-            graph.replay()
-        torch.cuda.synchronize()
-        sec = time.perf_counter() - t0
-        timed_evs = evs
-        for i in range(args.steps):                       # the gather's duration: eager, with events
-            step(evs[i])
-        torch.cuda.synchronize()
+        run = graph.replay
     else:
-        # one launch of a few microseconds per step: an event pair around every launch would be a third
-        # of the step, so every eighth step carries one
-        stride = 8 if fused_layer else 1
-        timed_evs = evs[::stride]
-        t0 = time.perf_counter()
-        for i in range(args.steps):
-            out = step(evs[i] if i % stride == 0 else None)
-        torch.cuda.synchronize()
-        t1 = time.perf_counter()
-        sec = t1 - t0
-    gather_ms = sum(a.elapsed_time(b) for a, b in timed_evs) / len(timed_evs)
+        run = step
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    for i in range(args.steps):
+        run()
+    torch.cuda.synchronize()
+    sec = time.perf_counter() - t0
+
+    # the stages (outside the timed region)
+    def timed(fn, n=50):
+        fn(); torch.cuda.synchronize()
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(n):
+            fn()
+        b.record(); torch.cuda.synchronize()
+        return a.elapsed_time(b) / n
+    with torch.no_grad():
+        hash_ms = None if front is None else timed(front)
+        gather_ms = timed(gather_only)
     logical_gbps = gather_bytes / (gather_ms * 1e-3) / 1e9
     row_bytes = B * T * Do * esz                                          # one row per (token, table)
     compulsory = T * S * Do * esz + B * T * 8 + B * Do * 4                # tables, codes + scores, output: each once
@@ -647,22 +648,6 @@ def main():
                     "traffic": traffic, "avg_kernel_ms": gather_ms, "hbm": hbm,
                     "logical_gbps": logical_gbps, "algorithmic_bytes": gather_bytes}
 
-    # stage breakdown (outside the timed region)
-    def timed(fn, n=20):
-        fn(); torch.cuda.synchronize()
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        a.record()
-        for _ in range(n):
-            fn()
-        b.record(); torch.cuda.synchronize()
-        return a.elapsed_time(b) / n
-    def front():
-        if rec_plan is not None:
-            return records_front()
-        return hash_front()
-    with torch.no_grad():
-        hash_ms = None if fused_layer else timed(front)
-
     # Warm and cold medians of single launches (outside the timed region).  Warm: back to
     # back, the tables still in the caches from the launch before.  Cold: a 1 GiB fill
     # between the launches pushes the tables out of the L2s and the 256 MB Infinity Cache.
@@ -677,15 +662,6 @@ def main():
             ts.append(a.elapsed_time(b))
         return statistics.median(ts)
     with torch.no_grad():
-        if fused_layer:
-            gather_only = step
-        else:
-            if rec_plan is not None:
-                records = front()
-                gather_only = lambda: ops.lookup_gather_records_direct(records, rec_plan, layer.tables, layer.bias, None, B)
-            else:
-                code, score = hash_front()
-                gather_only = lambda: ops.lookup_gather(code, score, layer.tables, layer.bias)
         warm_gather, warm_step = single(gather_only, 25), single(step, 25)
         flush = torch.zeros(1 << 28, dtype=torch.float32, device=dev)
         cold_gather, cold_step = single(gather_only, 15, flush), single(step, 15, flush)

@@ -766,9 +766,8 @@ def _(indexes, source, weights):
     return weights.new_empty(indexes.shape[0], source.shape[1])
 
 
-# The inference path of the layer at many tokens: the projection kernel writes the gather kernel's record
-# stream itself (no [B, T] codes and scores, no packing kernel).  Plain functions, no operator: the
-# records are a private hand-over between the two kernels.
+# The layer in inference at many tokens: the projection kernel writes the gather kernel's record stream itself (no [B, T]
+# codes and scores, no packing kernel).  The records are a private hand-over between the two kernels.
 _RECORDS_PLANS = {}
 
 
@@ -794,68 +793,6 @@ def lookup_gather_records_plan(B, T, S, Do, fmt=ROWS_F32):
     if len(_RECORDS_PLANS) < 4096:
         _RECORDS_PLANS[key] = plan
     return plan
-
-
-def _require(cond, what):
-    """Argument checks of the *_direct helpers (no operator dispatcher in front of them): a real exception,
-    also under ``python -O``."""
-    if not cond:
-        raise ValueError(what)
-
-
-def ln_project_hash_records_direct(x, ln_w, ln_b, eps, diag, pbias, T, decay, residual, plan):
-    """LayerNorm + diagonal BH4 + mix + 8-bit hash of x [B, H], written as the record stream of `plan`
-    (from lookup_gather_records_plan) instead of codes and scores.  The caller has checked the parameters
-    (fp32, contiguous, on x's device)."""
-    _require(x.dtype == torch.float32 and x.is_cuda and x.is_contiguous() and x.dim() == 2, "x: contiguous fp32 [B, H] on the GPU")
-    B, H = x.shape
-    R, J, D = diag.shape
-    _require(H == ln_w.numel() and T * 8 <= R * D and T % 2 == 0 and plan[1] >= B, "shapes do not fit the record plan")
-    records = torch.empty(plan[2] // 4, dtype=torch.int32, device=x.device)
-    with _dev_guard(x):
-        rc = _lib.load().lffn_ln_project_hash_records_f32(
-            x.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), eps, diag.data_ptr(), None if pbias is None else pbias.data_ptr(),
-            records.data_ptr(), plan[1], plan[0], B, H, D, R, J, T, decay, residual, _lib.stream_of(x))
-    if rc != 0:
-        _lib.check(rc, f"lffn_ln_project_hash_records_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
-    return records
-
-
-def ln_bh4_block_hash_records_direct(x, ln_w, ln_b, eps, w_folded, pbias, T, decay, residual, plan):
-    """The same for BH4 with 64 x 64 blocks (folded weights [R, J, D/64, 64, 64]) on the matrix cores."""
-    _require(x.dtype == torch.float32 and x.is_cuda and x.is_contiguous() and x.dim() == 2, "x: contiguous fp32 [B, H] on the GPU")
-    B, H = x.shape
-    R, J, NB, bs, _ = w_folded.shape
-    D = NB * bs
-    _require(H == ln_w.numel() and T * 8 <= R * D and T % 2 == 0 and plan[1] >= B, "shapes do not fit the record plan")
-    records = torch.empty(plan[2] // 4, dtype=torch.int32, device=x.device)
-    with _dev_guard(x):
-        rc = _lib.load().lffn_ln_bh4_block_hash_records_f32(
-            x.data_ptr(), ln_w.data_ptr(), ln_b.data_ptr(), eps, w_folded.data_ptr(), None if pbias is None else pbias.data_ptr(),
-            records.data_ptr(), plan[1], plan[0], B, H, D, R, J, T, bs, decay, residual, _lib.stream_of(x))
-    if rc != 0:
-        _lib.check(rc, f"lffn_ln_bh4_block_hash_records_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
-    return records
-
-
-def lookup_gather_records_direct(records, plan, tables, bias, residual, B):
-    """out[b] = residual[b] + bias + sum_t score * row, from the record stream written for `plan` (which was
-    made for the tables' row format)."""
-    T, S, Do = tables.shape
-    fmt = row_format(tables.dtype)
-    _require(fmt is not None and tables.is_contiguous() and records.numel() * 4 >= plan[2],
-             "tables: contiguous float32, bfloat16 or float16; records: at least the plan's bytes")
-    _require(residual is None or (residual.dtype == torch.float32 and residual.is_contiguous()
-                                  and residual.device == tables.device and tuple(residual.shape) == (B, Do)),
-             "residual: contiguous fp32 [B, Do] on the tables' device")
-    out = torch.empty(B, Do, dtype=torch.float32, device=tables.device)
-    with _dev_guard(tables):
-        rc = _lib.load().lffn_lookup_gather_records_rows(
-            records.data_ptr(), plan[1], tables.data_ptr(), None if bias is None else bias.data_ptr(),
-            None if residual is None else residual.data_ptr(), out.data_ptr(), B, T, S, Do, fmt, plan[0], _lib.stream_of(tables))
-    if rc != 0:
-        _lib.check(rc, f"lffn_lookup_gather_records_rows(B={B}, T={T}, S={S}, Do={Do}, row_format={fmt})")
-    return out
 
 
 _L.define("lookup_gather(Tensor code, Tensor score, Tensor tables, Tensor? bias, Tensor? residual=None) -> Tensor")

@@ -96,7 +96,7 @@ MANY_TOKEN_LAYERS = [((32, 512), 768, 128, 768, 1, torch.float32), ((32, 512), 1
 
 @pytest.mark.parametrize("shape,H,T,Do,bs,tdtype", MANY_TOKEN_LAYERS)
 def test_layer_forward_eval_many_tokens_matches_oracle(shape, H, T, Do, bs, tdtype):
-    """LookupFFN.eval() at 16384 tokens: the record-stream path of LookupFFN._forward_inference, on a sample of
+    """LookupFFN.eval() at 16384 tokens: the record-stream path of LookupFFN.forward, on a sample of
     tokens against the oracle."""
     from lookupffn_amd import ops
     torch.manual_seed(H + T + bs)
@@ -559,9 +559,8 @@ def test_training_step_of_a_large_batch_is_the_sum_of_its_halves(bs):
 
 
 def test_one_launch_layer_follows_its_parameters():
-    """Small batches take the one-launch form, which keeps views of the parameters between calls:
-    they must follow in-place updates, a loaded state dict, a replaced parameter and a cast, and
-    the result must stay that of the two-kernel form (same kernels' arithmetic, same codes)."""
+    """Small batches take the one-launch form: the result must follow in-place updates, a loaded state
+    dict, a replaced parameter and a cast, and stay that of the two-kernel form (same kernels' arithmetic, same codes)."""
     torch.manual_seed(33)
     cfg = _config(hidden_size=256, ffn_num_table=32, block_size=1)
     layer = lookupffn_amd.LookupFFN(cfg, 256).eval().to(DEV)
