@@ -158,7 +158,7 @@ def load() -> ctypes.CDLL:
 
 
 HOST_PATH = os.path.join(_PKG_DIR, "_host.so")
-_host = None                    # False: not to be had
+loaded_host = None                    # False: not to be had
 
 
 def _load_host():
@@ -177,18 +177,18 @@ def _load_host():
 def host():
     """The layer's host path (csrc/host.cpp, built next to the kernel library), bound to the loaded kernel library.  False where
     it is missing or was built against another torch: the layer then calls the same kernels from Python."""
-    global _host
-    if _host is None:
+    global loaded_host
+    if loaded_host is None:
         load()
         with _lock:
-            if _host is None:
+            if loaded_host is None:
                 try:
-                    _host = _load_host()
+                    loaded_host = _load_host()
                 except ImportError as e:
                     warnings.warn(f"lookupffn_amd: the host path of LookupFFN is not available ({e}): its calls cost more host time.  "
                                   "Build it with `python -m lookupffn_amd._build`", RuntimeWarning)
-                    _host = False
-    return _host
+                    loaded_host = False
+    return loaded_host
 
 
 def exported_symbols():

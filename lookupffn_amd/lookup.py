@@ -15,6 +15,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.compiler import is_compiling
 
 from . import _lib, ops
 from .bh4 import bh4
@@ -418,7 +419,7 @@ class LookupFFN(nn.Module):
         return None if out is False else out
 
     def _forward(self, hidden_states, residual=None):
-        if not torch.compiler.is_compiling():
+        if not is_compiling():
             out = self._forward_host(hidden_states, residual)
             if out is not None:
                 return out
@@ -467,10 +468,12 @@ class LookupFFN(nn.Module):
         """PL/lookup.py:110-118.  ``residual`` (not in the reference; shape [..., output_size]) is
         added to the result inside the gather kernel: the encoder layer's "FFN(x) + x"."""
         own = type(self)._forward is _LAYER_FORWARD and "_forward" not in self.__dict__
-        if own and not torch.compiler.is_compiling():
+        if own and not is_compiling():
             # (before anything else: at a few hundred tokens the layer is one launch of a few microseconds, and every view
             # made here shows in its time)
-            host = _lib.host()
+            host = _lib.loaded_host
+            if host is None:
+                host = _lib.host()
             out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS) if host else None
             if out is False:
                 out = self._forward_host(hidden_states, residual)

@@ -406,7 +406,7 @@ def test_attention_fused_equals_literal_formula_on_cpu():
 @pytest.mark.parametrize("why", ["missing", "does not load", "another torch"])
 def test_a_host_path_that_is_not_to_be_had_is_said_once_and_done_without(why, monkeypatch):
     assert _lib.host()                                       # built next to the kernel library
-    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(_lib, "loaded_host", None)
     if why == "missing":
         monkeypatch.setattr(_lib, "HOST_PATH", "/nonexistent/_host.so")
     elif why == "does not load":

@@ -273,7 +273,7 @@ def test_the_host_path_is_tried_once_a_call(kind, monkeypatch):
             tries.append(out is not None)
             return out
 
-    monkeypatch.setattr(_lib, "host", lambda: Counted)
+    monkeypatch.setattr(_lib, "loaded_host", Counted)
     with torch.no_grad():
         for _ in range(2):
             if kind == "watched":
@@ -352,7 +352,7 @@ def test_a_layer_without_the_host_path_gives_the_same(block, train, monkeypatch)
     layer = _layer(block)
     x = torch.randn(40, 256, device=DEV)
     want = [t.clone() for t in _pass(layer, x, train)]
-    monkeypatch.setattr(_lib, "_host", False)
+    monkeypatch.setattr(_lib, "loaded_host", False)
     _assert_same(_pass(layer, x, train), want)
 
 
@@ -399,7 +399,7 @@ def test_both_backward_chains_agree(block, B, H, T, out, monkeypatch):
 
     wanted = ["all"] + (["x", "residual"] + [n for n, _ in layer.named_parameters()] if B < 5000 else [])
     host = [run(w) for w in wanted]
-    monkeypatch.setattr(_lib, "_host", False)
+    monkeypatch.setattr(_lib, "loaded_host", False)
     for w, got in zip(wanted, host):
         want = run(w)
         assert got.keys() == want.keys()
