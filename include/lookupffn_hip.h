@@ -660,8 +660,8 @@ int lffn_indexed_inner_product_f16(const int32_t *idx, const uint16_t *g, const 
 int lffn_scatter_add_f16(const int32_t *idx, const uint16_t *g, const float *w, float *out,
                          int64_t B, int64_t I, int64_t out_size, int64_t Dv, void *stream);
 
-/* Tokens up to which lffn_lookup_scatter_f32 sums every row of the gradient from a list of its tokens (tables of at most 256
- * rows); up to there it is also faster than lffn_lookup_scatter_sorted_f32. */
+/* Tokens up to which lffn_lookup_scatter_f32 is faster than lffn_lookup_scatter_sorted_f32 (tables of at most 256 rows): up to
+ * there it sums every row of the gradient from a list of its tokens, where that is faster than summing in LDS. */
 #define LFFN_SCATTER_LIST_TOKENS 2048
 
 /*
@@ -670,7 +670,7 @@ int lffn_scatter_add_f16(const int32_t *idx, const uint16_t *g, const float *w, 
  *   grad_tables[t, s, :] (+)= sum_{b : (code[b,t] & (S-1)) == s} score[b,t] * g[b,:]
  * code: [B, T] int32; score: [B, T]; g: [B, Do]; grad_tables: [T, S, Do].
  * accumulate == 0: grad_tables is overwritten (it needs no zero-fill); otherwise
- * added to.  For S <= 256 the sums are formed in LDS (no global atomics); the
+ * added to.  For S <= 256 the sums are formed in LDS or in registers (no global atomics); the
  * order of additions is still free, as with the reference's atomics.
  * Replaces WeightedVectorGatherAdd.backward's weighted_vector_scatter_add call
  * (PL/gather/cuda/kernel.py:200) together with the index offset of PL/lookup.py:126.

@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256 * BG * HV / NH, BG > 1 ? 4 : (HV == 1 ? 2 : 1))
 
     // A workgroup takes one repeat of its tokens, and the repeats come one after the other in the grid: their 1 MB of weights
     // stay in the L2 for the launch's workgroups, and few tokens with several repeats are as many workgroups more (32768
-    // tokens, D = 512, two repeats: the layer 355 -> 320 us against a loop over the repeats; 64 tokens, D = 1024, four: 240 -> 138).
+    // tokens, D = 512, two repeats: the layer 357 -> 336 us against a loop over the repeats; 64 tokens, D = 1024, four: 240 -> 138).
     const int r = blockIdx.y;
     // Wide form: strides 2 and 1 of the butterflies across the blocks, on the LDS tile, 16 bytes of blocks 4 n .. 4 n + 3 per
     // thread and step; the tile's result is also written to rows of D floats at `save` if there is one.

@@ -694,7 +694,7 @@ __global__ __launch_bounds__(256) void rows_place_kernel(RowsArgs a) {
 // columns, which for rows of a few pairs is most of its time.  All five launches, 64 tokens: 128 tables of 768 columns 55 -> 29 us,
 // 512 of 1024 217 -> 125 us (537 MB written: 4.3 TB/s); 8 pairs a row, 2048 tokens of 128 x 512: 92 -> 60 us; 16 pairs a row 128 us
 // either way, hence the limit.  A row of more than LONG_ROW pairs goes to the whole workgroup; with half of all pairs on one row a single
-// compute unit's reads of g bound it (512 tokens of 128 x 768: 516 us by slices, 1283 so; fp32 atomics on one row are slower yet).
+// compute unit's reads of g bound it (512 tokens of 128 x 768: 516 us by slices, 1275 so, 3437 by fp32 atomics; with a tenth 288 and 1174).
 constexpr int64_t SPARSE_PAIRS = 8;
 constexpr int LONG_ROW = 32;
 constexpr int ROW_GROUP = 32;                         // rows of a workgroup
