@@ -3,7 +3,7 @@
 // A layer call at a few hundred tokens is one launch of a few microseconds, a training step of that size about twenty;
 // through the interpreter (argument checks, the operator dispatcher, foreign-function calls, two autograd functions) a call
 // took 15 us and a step 400 us whatever the kernels took (17 tokens, and 385 tokens at hidden 512).  Here a call
-// checks what can have changed since the layer's parameters were last looked at, allocates its result and launches; a
+// looks up what the layer holds, allocates its result and launches; a
 // training forward records one autograd node whose backward launches the whole chain.
 //
 // forward(layer, x, residual, ...) looks its modules and parameters up on every call and keeps nothing of them.  The answer is
@@ -28,11 +28,9 @@
 #include <dlfcn.h>
 
 #include <array>
-#include <atomic>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <vector>
 
 #include "../../include/lookupffn_hip.h"
 
