@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 8
+#define LFFN_ABI_VERSION 9
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -735,6 +735,29 @@ int lffn_lookup_backward_f32(const int32_t *code, const float *score, const floa
  */
 int lffn_lookup_inner_f32(const int32_t *code, const float *g, const float *tables, float *grad_score,
                           int64_t B, int64_t T, int64_t S, int64_t Do, void *stream);
+
+/* ------------------------------------------------- the encoder around the layer */
+
+/*
+ * out[s][m, :] = x[m, :] . w[s]^T + bias[s] (+ residual[m, :]) for s < sets, one launch: torch.nn.Linear of
+ * the encoder's attention (PL/layer.py:23-26, 28), query, key and value together.  x: [M, K]; w[s]: [N, K];
+ * bias[s]: [N] or NULL; residual: [M, N] or NULL; out[s]: [M, N], fp32.  w, bias and out are HOST arrays of
+ * `sets` device pointers, read before the call returns.  1 <= sets <= 3; K a multiple of 32; K, N <= 2^20;
+ * x and w[s] 16-byte aligned.  fp32 accuracy (2e-7 of the result's norm against 64 bits); infinities and
+ * NaN as in an fp32 sum of products.  No output may overlap an input.
+ */
+int lffn_linear_f32(const float *x, const float *const *w, const float *const *bias, const float *residual,
+                    float *const *out, int64_t sets, int64_t M, int64_t N, int64_t K, void *stream);
+
+/*
+ * out[b, i, h, :] = sum_j p_j v[b, j, h, :],  p = softmax_j(q[b, i, h, :] . k[b, j, h, :] / 8 - 1000 (1 - mask[b, j]))
+ * for heads of 64 columns, the encoder's attention (PL/layer.py:33-47), fp32.  q, k, v, out:
+ * [B, L, heads, 64], 16-byte aligned; mask: [B, L], any numbers.  L <= LFFN_ATTENTION_MAX_KEYS.  A query
+ * whose keys are all masked by an infinity gets zeros.
+ */
+#define LFFN_ATTENTION_MAX_KEYS 2048
+int lffn_attention_f32(const float *q, const float *k, const float *v, const float *mask, float *out, int64_t B,
+                       int64_t L, int64_t heads, void *stream);
 
 #ifdef __cplusplus
 }

@@ -1041,6 +1041,67 @@ def _(code, g, tables):
     return g.new_empty(code.shape[0], code.shape[1])
 
 
+# ----------------------------------------------------------------------------- the encoder around the layer
+
+_L.define("linear(Tensor x, Tensor[] w, Tensor?[] bias, Tensor? residual) -> Tensor")
+
+
+def _linear_impl(x, w, bias, residual):
+    """x [M, K]; w: up to three [N, K]; bias of each [N] or None -> [len(w), M, N] (+ residual [M, N])."""
+    _lib.require_gpu(x, *w, *bias, residual)
+    sets, (M, K), N = len(w), x.shape, w[0].shape[0]
+    assert 1 <= sets <= 3 and len(bias) == sets
+    for t in (x, *w, *(b for b in bias if b is not None), *(() if residual is None else (residual,))):
+        assert t.dtype == torch.float32 and t.is_contiguous()
+    assert all(t.shape == (N, K) for t in w) and all(b is None or b.shape == (N,) for b in bias)
+    assert residual is None or residual.shape == (M, N)
+    out = torch.empty(sets, M, N, dtype=torch.float32, device=x.device)
+    pointers = ctypes.c_void_p * sets
+    first = out.data_ptr()
+    with _dev_guard(x):
+        rc = _lib.load().lffn_linear_f32(_lib.ptr(x), pointers(*(t.data_ptr() for t in w)), pointers(*(_lib.ptr(b) for b in bias)),
+                                         _lib.ptr(residual), pointers(*(first + 4 * s * M * N for s in range(sets))), sets, M, N, K,
+                                         _lib.stream_of(x))
+    _lib.check(rc, f"lffn_linear_f32(sets={sets}, M={M}, N={N}, K={K})")
+    return out
+
+
+_L.impl("linear", _linear_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::linear")
+def _(x, w, bias, residual):
+    return x.new_empty(len(w), x.shape[0], w[0].shape[0])
+
+
+ATTENTION_MAX_KEYS = 2048       # LFFN_ATTENTION_MAX_KEYS
+
+_L.define("attention(Tensor q, Tensor k, Tensor v, Tensor mask) -> Tensor")
+
+
+def _attention_impl(q, k, v, mask):
+    """q, k, v [B, L, heads, 64], mask [B, L] -> [B, L, heads, 64]."""
+    _lib.require_gpu(q, k, v, mask)
+    B, L, heads, columns = q.shape
+    assert columns == 64 and k.shape == q.shape and v.shape == q.shape and mask.shape == (B, L)
+    for t in (q, k, v, mask):
+        assert t.dtype == torch.float32 and t.is_contiguous()
+    out = torch.empty_like(q)
+    with _dev_guard(q):
+        rc = _lib.load().lffn_attention_f32(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(mask), _lib.ptr(out), B, L, heads,
+                                            _lib.stream_of(q))
+    _lib.check(rc, f"lffn_attention_f32(B={B}, L={L}, heads={heads})")
+    return out
+
+
+_L.impl("attention", _attention_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::attention")
+def _(q, k, v, mask):
+    return torch.empty_like(q)
+
+
 fht = torch.ops.lookupffn.fht
 bh4_diag = torch.ops.lookupffn.bh4_diag
 bh4_fold = torch.ops.lookupffn.bh4_fold
@@ -1067,3 +1128,5 @@ scatter_add = torch.ops.lookupffn.scatter_add
 lookup_scatter = torch.ops.lookupffn.lookup_scatter
 lookup_backward = torch.ops.lookupffn.lookup_backward
 lookup_inner = torch.ops.lookupffn.lookup_inner
+linear = torch.ops.lookupffn.linear
+attention = torch.ops.lookupffn.attention
