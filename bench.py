@@ -28,6 +28,7 @@ One GPU only: this path has no multi-GPU form in this build.
 from __future__ import annotations
 
 import argparse
+import ctypes
 import statistics
 import json
 import math
@@ -539,8 +540,10 @@ def main():
         head = (x.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(), float(ln.eps))
         tail = (proj.bias.data_ptr(), records.data_ptr(), rec_plan[1], rec_plan[0])
         if block:
-            _lib.check(lib.lffn_ln_bh4_block_hash_records_f32(*head, layer.hash.folded_weight().data_ptr(), *tail, *sizes, 64, *coefs,
-                                                              stream), "lffn_ln_bh4_block_hash_records_f32")
+            front = _lib.BlockFront(ln.weight.data_ptr(), ln.bias.data_ptr(), layer.hash.split_weight().data_ptr(), proj.bias.data_ptr(),
+                                    None, None, records.data_ptr(), rec_plan[1], *sizes[1:], rec_plan[0], float(ln.eps),
+                                    *coefs)
+            _lib.check(lib.lffn_bh4_block_front_split_f32(ctypes.byref(front), x.data_ptr(), B, stream), "lffn_bh4_block_front_split_f32")
         else:
             _lib.check(lib.lffn_ln_project_hash_records_f32(*head, diag.data_ptr(), *tail, *sizes, *coefs, stream),
                        "lffn_ln_project_hash_records_f32")
@@ -683,7 +686,7 @@ def main():
                  "synthetic (seeded N(0,1) tokens, seeded +-1/sqrt(D) sign diagonals, N(0,0.02) tables)"),
         "config": {"workload": wl["desc"], "tokens": B, "d_model": H, "fht_dim": layer.hash.projection.padded_in_dim,
                    "tables": T, "table_size": S, "d_out": Do,
-                   "step": ("one kernel: LayerNorm + BH4(block 64)x4 on fp32 MFMA + mix + hash (weights folded once, "
+                   "step": ("one kernel: LayerNorm + BH4(block 64)x4 on fp16 MFMA, two terms a number, + mix + hash (weights folded once, "
                             "outside the step)" + (", written as the gather's record stream" if rec_plan is not None else "") +
                             "; one kernel: gather-add + bias") if block else
                            ("one kernel: LayerNorm + BH4(block 1)x4 + mix + hash + gather-add + bias" if fused_layer else

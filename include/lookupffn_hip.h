@@ -736,6 +736,43 @@ int lffn_lookup_backward_f32(const int32_t *code, const float *score, const floa
 int lffn_lookup_inner_f32(const int32_t *code, const float *g, const float *tables, float *grad_score,
                           int64_t B, int64_t T, int64_t S, int64_t Do, void *stream);
 
+/* ------------------------- 64 x 64 blocks on the fp16 matrix cores: inference and backward */
+
+/*
+ * The kernels of lffn_ln_bh4_block_hash_f32 (inference) and lffn_bh4_block_bwd_f32 with every number as two
+ * half-precision terms, which is faster and closer to 64 bits (csrc/bh4_split.hip); what the layer runs.  They are
+ * rounded differently: a code may differ where its z is within 1e-6 of the row's size of zero.
+ *
+ * lffn_bh4_fold_split_f32: the 64-point transform of lffn_bh4_fold_mode_f32 (transposed == 0: mode 0, else
+ * mode 1) of stages x num_block blocks, split.  w: [stages, num_block, 64, 64], num_block a power of two up to
+ * 16, stages = R * J; w_split: stages * (num_block * 4096 + 4) floats, 16-byte aligned.
+ */
+int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t stages, int64_t num_block, int64_t block_size,
+                            int32_t transposed, void *stream);
+
+/*
+ * The hashing front end: lffn_ln_bh4_block_hash_f32 (codes and scores) or, with records set,
+ * lffn_ln_bh4_block_hash_records_f32.  The struct is read before the call returns.
+ */
+typedef struct lffn_block_front {
+    const float *ln_weight, *ln_bias;       /* [H], both NULL for no LayerNorm */
+    const float *w_split;                   /* lffn_bh4_fold_split_f32, transposed == 0 */
+    const float *proj_bias;                 /* [T*8] or NULL */
+    int32_t *codes;                         /* [B, T] */
+    float *scores;                          /* [B, T] */
+    uint32_t *records;                      /* or NULL: instead of codes and scores */
+    int64_t record_stride;
+    int64_t H, D, R, J, T;
+    int32_t tokens_per_workgroup;
+    float ln_eps, decay, residual;
+} lffn_block_front;
+int lffn_bh4_block_front_split_f32(const lffn_block_front *front, const float *x, int64_t B, void *stream);
+
+/* lffn_bh4_block_bwd_f32 with weights of lffn_bh4_fold_split_f32, transposed != 0. */
+int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float *g_x, float *stage_grads, int64_t B,
+                                 int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t block_size, float decay,
+                                 float residual, void *stream);
+
 /* ------------------------------------------------- the encoder around the layer */
 
 /*

@@ -105,6 +105,8 @@ SIGNATURES = {
     "lffn_indexed_inner_product_ws_f32": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _vp],
     "lffn_scatter_rows_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)],
     "lffn_scatter_rows": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _vp],
+    "lffn_bh4_fold_split_f32": [_vp, _vp, _i64, _i64, _i64, _i32, _vp],
+    "lffn_bh4_block_bwd_split_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp],
     "lffn_linear_f32": [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp, ctypes.POINTER(_vp), _i64, _i64, _i64, _i64, _vp],
     "lffn_attention_f32": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "lffn_lookup_inner_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
@@ -117,6 +119,15 @@ class FusedLayer(ctypes.Structure):
                 ("ln_eps", _f32), ("decay", _f32), ("residual", _f32)]
 
 
+class BlockFront(ctypes.Structure):
+    """struct lffn_block_front of include/lookupffn_hip.h."""
+    _fields_ = [("ln_weight", _vp), ("ln_bias", _vp), ("w_split", _vp), ("proj_bias", _vp), ("codes", _vp), ("scores", _vp),
+                ("records", _vp), ("record_stride", _i64),
+                ("H", _i64), ("D", _i64), ("R", _i64), ("J", _i64), ("T", _i64), ("tokens_per_workgroup", _i32),
+                ("ln_eps", _f32), ("decay", _f32), ("residual", _f32)]
+
+
+SIGNATURES["lffn_bh4_block_front_split_f32"] = [ctypes.POINTER(BlockFront), _vp, _i64, _vp]
 SIGNATURES["lffn_lookup_ffn_fused_layer_f32"] = [ctypes.POINTER(FusedLayer), _vp, _vp, _vp, _i64, _vp]
 SIGNATURES["lffn_lookup_ffn_fused_layer_rows"] = [ctypes.POINTER(FusedLayer), ctypes.c_int32, _vp, _vp, _vp, _i64, _vp]
 

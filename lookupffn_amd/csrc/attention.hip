@@ -39,18 +39,13 @@ struct AttentionArgs {
 // Piece `piece` of row `row` of a plane: rows of 128 bytes, turned so that 16 rows' reads of one piece fall on different banks.
 __device__ __forceinline__ int at_piece(int row, int piece) { return row * 8 + (piece ^ ((row >> 1) & 7)); }
 
-__device__ __forceinline__ uint32_t pack_lo(float a, float b, uint32_t hi) {
-    const f16x2_t h = __builtin_bit_cast(f16x2_t, hi);
-    const f32x2_t v = {a - (float)h[0], b - (float)h[1]};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-}
 // eight numbers as hi and the rest
 __device__ __forceinline__ void split8(const float (&v)[8], uint4 &hi, uint4 &lo) {
     uint32_t h[4], l[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         h[e] = split_hi(v[2 * e], v[2 * e + 1], 1.f);
-        l[e] = pack_lo(v[2 * e], v[2 * e + 1], h[e]);
+        l[e] = split_rest(v[2 * e], v[2 * e + 1], h[e]);
     }
     hi = make_uint4(h[0], h[1], h[2], h[3]);
     lo = make_uint4(l[0], l[1], l[2], l[3]);

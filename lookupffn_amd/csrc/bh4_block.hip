@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256 * BG * HV / NH, BG > 1 ? 4 : (HV == 1 ? 2 : 1))
                 for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(p + k * BS) = v[k];
                 if (save && tok_base + row < B) {
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(save + size_t(row) * D + (n * BG + k) * BS + c4) = v[k];
+                    for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(v[k], reinterpret_cast<f32x4 *>(save + size_t(row) * D + (n * BG + k) * BS + c4));
                 }
             }
         }
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256 * BG * HV / NH, BG > 1 ? 4 : (HV == 1 ? 2 : 1))
 #pragma unroll
                     for (int n = 0; n < NB; ++n) {
                         *reinterpret_cast<f32x4 *>(xs + row * LDR + n * BS + c4) = pv[n];
-                        if (tok < B) *reinterpret_cast<f32x4 *>(ps + n * BS) = pv[n];
+                        if (tok < B) __builtin_nontemporal_store(pv[n], reinterpret_cast<f32x4 *>(ps + n * BS));
                     }
                 }
                 __syncthreads();
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256 * BG * HV / NH, BG > 1 ? 4 : (HV == 1 ? 2 : 1))
                         if (tok < B) {
                             float *o = a.stage_save + ((size_t(r) * (J - 1) + s) * B + tok) * D + 16 * ow + 4 * kq;
 #pragma unroll
-                            for (int n = 0; n < NBW; ++n) *reinterpret_cast<f32x4 *>(o + n * BS) = acc[t][n];
+                            for (int n = 0; n < NBW; ++n) __builtin_nontemporal_store(acc[t][n], reinterpret_cast<f32x4 *>(o + n * BS));
                         }
                     }
                 }
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256 * BG * HV / NH, BG > 1 ? 4 : (HV == 1 ? 2 : 1))
                             z[0] = z[0] + bb.x; z[1] = z[1] + bb.y; z[2] = z[2] + bb.z; z[3] = z[3] + bb.w;
                         }
                         if (a.z_out && in_cols && livev[t])
-                            *reinterpret_cast<float4 *>(a.z_out + tokv[t] * ncols + col) = make_float4(z[0], z[1], z[2], z[3]);
+                            __builtin_nontemporal_store((f32x4){z[0], z[1], z[2], z[3]}, reinterpret_cast<f32x4 *>(a.z_out + tokv[t] * ncols + col));
                         // columns 8g .. 8g+3 sit in the lane with even kq (the high nibble),
                         // 8g+4 .. 8g+7 in lane + 16, which continues the sum and the product
                         // (d = 0..7 in order, compute_code_score/torch_extension.cc:31-37)

@@ -1,0 +1,717 @@
+// BH4 with 64 x 64 blocks (PL/bh4/kernel.py:23-36) for inference and for the backward, on the fp16 matrix cores: the stages of
+// bh4_block.hip, (H_NB (x) I_64) * blockdiag(H_64 W[r,s,n]) each, with the weights and the tokens' rows as two half-precision terms
+// a number (split_mfma.h).
+//
+// The hash form runs the layer's whole front end for 8-bit codes: LayerNorm while the tile is loaded, the stages, z = decay * y +
+// residual * LN(x) + bias on the accumulators (x is read again and normalised with the kept statistics), codes and scores.  A
+// wavefront owns 16 output columns of every block, products on v_mfma_f32_16x16x32_f16 with the weights as A and the tokens as B, so
+// that a lane ends up with four consecutive columns of one token in every block: the butterflies across blocks are register adds.
+// Between two stages a token's row is scaled by a power of two, its largest to [2^14, 2^15), split, and written to the tile (hi and
+// lo, 4 bytes a number, as much as it was in fp32); both terms are then normal half-precision numbers or smaller than 2^-38 of the
+// row's largest, so neither needs a factor, the six instructions of a block add into one accumulator, and nothing overflows however a
+// stage amplifies.  A row's scale depends on that row alone: its results do not depend on its neighbours.
+//
+// What bounds it: the forward the weights' way from the L2 (2.1 GB in 128 us at 32768 tokens, D = 512, two repeats; 16 tokens a
+// workgroup) and the vector work (LayerNorm 18, a stage 9, hash 18 instructions a number), the backward the gradients it writes to
+// memory (0.8 GB in 205 us).  Products on the fp32 matrix cores (bh4_block.hip) take 16/3 of the time of these.  32768 tokens, D = 512,
+// two repeats: forward 235 -> 128-144 us, backward 280 -> 205; 16384, D = 1024 125 -> 75, 128 -> 103; 385, D = 512 18.5 -> 12.3, 18.7 ->
+// 12.2.  Tried: 32 tokens a workgroup in 4 wavefronts (124-149 us from build to build) and 8 (151), 64 in 8 (145), four blocks' weights
+// ahead instead of two (134).  Error of the last stage against 64 bits 2.4e-7 (fp32 matrix cores 3.2e-7), input gradient 2.2e-7 (3.1e-7).
+//
+// The training forward stays on the fp32 matrix cores: a projected value within rounding of zero takes either sign, with the sign the
+// derivative of its score turns round, and a training step's gradients should not change with the kernel.
+#include "split_mfma.h"
+
+// the mix and the score keep the reference's operation order: no fused multiply-add
+#pragma clang fp contract(off)
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int BS = 64;          // block size this file is built for
+constexpr int PAD = 4;          // floats of padding per row of the fp32 tile
+constexpr float TOP = 16384.f;  // what the largest of a row is scaled to at least (and less than twice that)
+
+__device__ __forceinline__ float wave_most(float v) {
+    v = fmaxf(v, lane_xor<1>(v));
+    v = fmaxf(v, lane_xor<2>(v));
+    v = fmaxf(v, lane_xor<4>(v));
+    v = fmaxf(v, lane_xor<8>(v));
+    v = fmaxf(v, lane_xor<16>(v));
+    return fmaxf(v, lane_xor<32>(v));
+}
+
+// The 64-point transform of every block (bh4_block.hip: bh4_fold_kernel), split, ready for the product kernel.  One workgroup per stage, a wavefront per
+// block: the 16 output (forward; transposed: input) columns that a product wavefront has of every block are scaled together by a
+// power of two, their largest in the stage to [2^14, 2^15), so that lo needs no factor.  Per block and product wavefront four
+// fragments of 64 lanes x 8 numbers: hi of the first and the second eight columns of a lane's sixteen, then lo of them; behind all
+// blocks the inverse scales, [stage][4].
+template <bool TRANSPOSED>
+__global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, uint32_t *out, float *inverse) {
+    __shared__ float most_s[16][4];
+    const int num_block = blockDim.x / 64, wave = threadIdx.x >> 6;
+    const int64_t blk = int64_t(blockIdx.x) * num_block + wave;
+    const int i = threadIdx.x & 63;
+    const float *src = w + blk * (BS * BS) + i;
+    float v[BS];
+#pragma unroll
+    for (int o = 0; o < BS; ++o) v[o] = src[o * BS];
+#pragma unroll
+    for (int h = BS / 2; h >= 1; h >>= 1) {
+#pragma unroll
+        for (int o = 0; o < BS; ++o) {
+            if ((o & h) == 0) {
+                const float lo = v[o], hi = v[o + h];
+                v[o] = lo + hi;
+                v[o + h] = lo - hi;
+            }
+        }
+    }
+    if constexpr (!TRANSPOSED) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float most = 0.f;
+#pragma unroll
+            for (int o = 16 * g; o < 16 * g + 16; ++o) most = fmaxf(most, fabsf(v[o]));
+            most = wave_most(most);
+            if (i == 0) most_s[wave][g] = most;
+        }
+    } else {
+        float most = 0.f;
+#pragma unroll
+        for (int o = 0; o < BS; ++o) most = fmaxf(most, fabsf(v[o]));
+        most = fmaxf(most, lane_xor<1>(most));
+        most = fmaxf(most, lane_xor<2>(most));
+        most = fmaxf(most, lane_xor<4>(most));
+        most = fmaxf(most, lane_xor<8>(most));
+        if (i % 16 == 0) most_s[wave][i / 16] = most;
+    }
+    __syncthreads();
+    float scale[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        float most = 0.f;
+        for (int n = 0; n < num_block; ++n) most = fmaxf(most, most_s[n][g]);
+        const PowerOfTwo p = scale_to_one(most);
+        scale[g] = p.scale * TOP;
+        if (threadIdx.x == 0) inverse[blockIdx.x * 4 + g] = p.inverse * (1 / TOP);
+    }
+    // eight consecutive k of a row of the A operand as hi and lo: fragment (row / 16, (k % 16) / 8), lane 16 (k / 16) + row % 16
+    uint4 *const dst = reinterpret_cast<uint4 *>(out + blk * (BS * BS));
+    auto store8 = [&](int row, int k, const float (&x)[8]) {
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            h[e] = split_hi(x[2 * e], x[2 * e + 1], 1.f);
+            l[e] = split_rest(x[2 * e], x[2 * e + 1], h[e]);
+        }
+        const int at = ((row / 16) * 4 + (k % 16) / 8) * 64 + 16 * (k / 16) + row % 16;
+        dst[at] = make_uint4(h[0], h[1], h[2], h[3]);
+        dst[at + 128] = make_uint4(l[0], l[1], l[2], l[3]);
+    };
+    if constexpr (TRANSPOSED) {
+        const float f = i < 32 ? (i < 16 ? scale[0] : scale[1]) : (i < 48 ? scale[2] : scale[3]);
+#pragma unroll
+        for (int k = 0; k < BS; k += 8) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = v[k + e] * f;
+            store8(i, k, x);
+        }
+    } else {
+        // a lane has a column of the block: sixteen rows at a time turned round through the wavefront's own 16 x 65 floats of LDS
+        extern __shared__ float turn[];
+        float *const t = turn + wave * (16 * 65);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+#pragma unroll
+            for (int o = 0; o < 16; ++o) t[o * 65 + i] = v[16 * g + o] * scale[g];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int row = i % 16, k = 16 * (i / 16) + 8 * m;
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = t[row * 65 + k + e];
+                store8(16 * g + row, k, x);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+}
+
+struct SplitArgs {
+    const float *x;        // [B, H]
+    const float *ln_w;     // [H] LayerNorm weight, or null: no LayerNorm
+    const float *ln_b;     // [H]
+    float ln_eps;
+    const float *w;        // split weights
+    const float *wscale;   // their inverse scales [R*J][4]
+    const float *pbias;    // [T*8] or null
+    int32_t *codes;        // [B, T]
+    float *scores;         // [B, T]
+    uint32_t *records;     // instead of codes and scores: the record stream of the four-lanes-per-token gather,
+    int64_t rec_stride;    // [T/2][rec_stride][3] (lffn_quad_record_slot)
+    int rec_tile;          // tokens per workgroup of the gather the records are written for
+    const float *gz;       // backward: [B, T*8] gradient of z
+    float *g_x;            // backward: [R, B, H]
+    float *stage_grads;    // backward: [R, J, B, D] gradient before the product of each stage
+    int64_t B;
+    int H, R, J, T;
+    float decay, residual;
+};
+
+// Largest over the four rows of 16 lanes (row swaps on the vector ALU: an LDS permute would be waited for).
+__device__ __forceinline__ float rows_most(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+__device__ __forceinline__ f32x4 mfma16(uint4 a, uint4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
+// hi and lo of four numbers
+__device__ __forceinline__ void split4(f32x4 v, uint2 &hi, uint2 &lo) {
+    hi = make_uint2(split_hi(v.x, v.y, 1.f), split_hi(v.z, v.w, 1.f));
+    lo = make_uint2(split_rest(v.x, v.y, hi.x), split_rest(v.z, v.w, hi.y));
+}
+
+// A workgroup has 16 tokens: 4 wavefronts (BG = 1) of 16 output columns of every block each, or 16 for small batches (BG = 4), in
+// which wavefront group bg has blocks bg, bg + 4, ...: the butterflies across a wavefront's own blocks (strides 4 and up) stay
+// between accumulators, the last two (strides 2 and 1) are a pass over the tile in LDS.
+// Both do the same operations in the same order: the results are those of the other form bit for bit.
+//
+// BWD: the backward through the stages with the same machinery.  With G_{s+1} the gradient of a stage's output, the gradient of its
+// input is  W'_s^T (H_NB (x) I_64) G_{s+1}  (H_64 is symmetric and already inside W' = H_64 W): the butterflies across blocks run
+// BEFORE the product, which takes the folded weights in transposed fragment order, and nothing follows it.  The butterflied
+// gradient P_s = (H_NB (x) I) G_{s+1} is also written to memory: the gradient w.r.t. the folded weights is the per-block product
+// P_s^T U_s over all tokens (U_s = the stage's input, which the forward saved), formed by the caller.  First gradient: decay * grad z;
+// result: grad x of this repeat = G_0[:, :H] + residual * grad z[:, :H].
+template <int NB, bool BWD, int BG>
+__global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split_kernel(SplitArgs a) {
+    static_assert(BG == 1 || (BG == 4 && NB >= 4), "the wide form: four groups of blocks");
+    constexpr int TOK = 16;                       // tokens per workgroup
+    constexpr int NWAVE = 4 * BG;
+    constexpr int NBW = NB / BG;                  // blocks of a wavefront: bg + BG * n, n < NBW
+    const float *__restrict__ x = a.x;
+    const int64_t B = a.B;
+    const int H = a.H, R = a.R, J = a.J;
+    constexpr int D = BS * NB;
+    constexpr int LDP = 2 * D + 16;               // bytes of a tile row: 16 rows' reads of a fragment fall on different banks
+    constexpr int LDR = D + PAD;
+    constexpr int AHEAD = NBW < 2 ? NBW : 2;     // blocks whose weights are on their way
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    char *const tile = lds;                       // [2][TOK] rows of LDP bytes: hi, lo
+    float *const wide_tile = reinterpret_cast<float *>(lds + 2 * TOK * LDP);          // wide form: [TOK][LDR] in fp32
+    float *const stats = wide_tile + (BG > 1 ? TOK * LDR : 0);                        // [TOK][2]: LayerNorm's mean and 1/sigma
+    float *const unscale = stats + 2 * TOK;       // [TOK] 1 / scale of a token's row
+    float *const most_s = unscale + TOK;          // [TOK][4] largest of a token's row in a wavefront's columns
+    float *const lnw_s = most_s + 4 * TOK;        // hash form: [D] each LayerNorm's weight and bias, the projection's bias
+    float *const lnb_s = lnw_s + D, *const pbias_s = lnb_s + D;
+    float *const xs = reinterpret_cast<float *>(lds);      // hash form, after the last stage: codes and scores
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ow = wave & 3;                      // output columns [16*ow, 16*ow + 16) of each block
+    const int bg = wave >> 2;                     // group of blocks of this wavefront
+    const int c = lane & 15;                      // A operand: output column; B operand and result: token
+    const int kq = lane >> 4;                     // operands: columns 16*kq .. + 15 of the block; result: output columns 4*kq .. + 3
+    const int64_t tok_base = int64_t(blockIdx.x) * TOK;
+    if (!BWD) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        for (int e = tid * 4; e < D; e += 256 * NWAVE) {
+            const f32x4 one = {1.f, 1.f, 1.f, 1.f};
+            *reinterpret_cast<f32x4 *>(lnw_s + e) = e >= H ? zero : a.ln_w ? *reinterpret_cast<const f32x4 *>(a.ln_w + e) : one;
+            *reinterpret_cast<f32x4 *>(lnb_s + e) = e < H && a.ln_w ? *reinterpret_cast<const f32x4 *>(a.ln_b + e) : zero;
+            const int col = blockIdx.y * D + e;
+            *reinterpret_cast<f32x4 *>(pbias_s + e) = a.pbias && col < a.T * 8 ? *reinterpret_cast<const f32x4 *>(a.pbias + col) : zero;
+        }
+        __syncthreads();
+    }
+
+    // A workgroup takes one repeat of its tokens, and the repeats come one after the other in the grid: their weights
+    // stay in the L2 for the launch's workgroups, and few tokens with several repeats are as many workgroups more.
+    const int r = blockIdx.y;
+    f32x4 acc[NBW];
+
+    // this wavefront's weights of a block: four fragments of 1 KB (WSPLIT: hi, hi, lo, lo; else 16 numbers a lane)
+    uint4 wq[AHEAD][4];
+    auto load_w = [&](int s, int n) {
+        if (n >= NBW) {                           // the next stage's first blocks (after the last stage: a harmless re-read)
+            n -= NBW;
+            s = BWD ? max(s - 1, 0) : min(s + 1, J - 1);
+        }
+        const float *p = a.w + (size_t)((r * J + s) * NB + n * BG + bg) * (BS * BS) + ow * 1024 + lane * 4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) wq[n % AHEAD][q] = *reinterpret_cast<const uint4 *>(p + q * 256);
+    };
+    // this lane's token values of block n: 16 numbers as hi and lo fragments
+    auto read_x = [&](int n, uint4 (&f)[4]) {
+        const char *p = tile + c * LDP + (n * BG + bg) * 128 + kq * 32;
+        f[0] = *reinterpret_cast<const uint4 *>(p);
+        f[1] = *reinterpret_cast<const uint4 *>(p + 16);
+        f[2] = *reinterpret_cast<const uint4 *>(p + TOK * LDP);
+        f[3] = *reinterpret_cast<const uint4 *>(p + TOK * LDP + 16);
+    };
+    // four numbers of a token's row into the tile
+    auto put = [&](int row, int col, f32x4 v) {
+        uint2 hi, lo;
+        split4(v, hi, lo);
+        char *p = tile + row * LDP + col * 2;
+        *reinterpret_cast<uint2 *>(p) = hi;
+        *reinterpret_cast<uint2 *>(p + TOK * LDP) = lo;
+    };
+
+    // What the accumulators are to be multiplied with: the inverse scales of this wavefront's weights and of the lane's tokens.
+    float inv_w = 1.f, inv_x = 1.f;
+
+    // acc = (blocks of the stage's weights) x (the tile's tokens)
+    auto product = [&](int s) {
+        inv_w = a.wscale[(r * J + s) * 4 + ow];
+        inv_x = unscale[c];
+        uint4 xv[2][4];
+        read_x(0, xv[0]);
+        static_for<NBW>([&](auto n_c) {
+            constexpr int n = decltype(n_c)::value;
+            if constexpr (n > 0) load_w(s, n - 1 + AHEAD);
+            if constexpr (n + 1 < NBW) read_x(n + 1, xv[(n + 1) % 2]);
+            __builtin_amdgcn_sched_barrier(0);
+            // the small terms first
+            const uint4 (&w)[4] = wq[n % AHEAD], (&x4)[4] = xv[n % 2];
+            acc[n] = mfma16(w[2], x4[0], (f32x4){0.f, 0.f, 0.f, 0.f});
+            acc[n] = mfma16(w[0], x4[2], acc[n]);
+            acc[n] = mfma16(w[3], x4[1], acc[n]);
+            acc[n] = mfma16(w[1], x4[3], acc[n]);
+            acc[n] = mfma16(w[0], x4[0], acc[n]);
+            acc[n] = mfma16(w[1], x4[1], acc[n]);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        load_w(s, NBW - 1 + AHEAD);
+    };
+
+    // H_NB across the blocks of the accumulators, from stride NB / 2 down (wide form: down to BG)
+    auto butterflies = [&]() {
+#pragma unroll
+        for (int h = NBW / 2; h >= 1; h >>= 1) {
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) {
+                if ((n & h) == 0) {
+                    const f32x4 lo = acc[n], hi = acc[n + h];
+                    acc[n] = lo + hi;
+                    acc[n + h] = lo - hi;
+                }
+            }
+        }
+    };
+
+    // The accumulators (after butterflies()) become the next product's tile, and the rows of D floats at `save` where they are kept:
+    // a token's row is scaled by the power of two that takes its largest to [2^14, 2^15).
+    auto hand_over = [&](float *save) {
+        if constexpr (BG > 1) {
+            // strides 2 and 1, which take four wavefronts' accumulators: a pass over the tile in fp32, 16 bytes of blocks
+            // 4 n .. 4 n + 3 per thread; the 16 NBW threads of a row are neighbours in a wavefront
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+                *reinterpret_cast<f32x4 *>(wide_tile + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n] * inv_w;
+            if (bg == 0 && ow == 0 && kq == 0) unscale[c] = inv_x;
+            __syncthreads();
+            if (tid < TOK * 16 * NBW) {
+                const int row = tid / (16 * NBW), n = (tid / 16) % NBW, c4 = (tid % 16) * 4;
+                const float *p = wide_tile + row * LDR + n * BG * BS + c4;
+                const float inv = unscale[row];
+                f32x4 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4 *>(p + k * BS);
+                const f32x4 s0 = v[0] + v[2], s1 = v[1] + v[3], d0 = v[0] - v[2], d1 = v[1] - v[3];
+                v[0] = s0 + s1; v[1] = s0 - s1; v[2] = d0 + d1; v[3] = d0 - d1;
+                float most = 0.f;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) most = fmaxf(most, fabsf(v[k][e]));
+                most = fmaxf(most, lane_xor<1>(most));
+                most = fmaxf(most, lane_xor<2>(most));
+                most = fmaxf(most, lane_xor<4>(most));
+                most = fmaxf(most, lane_xor<8>(most));
+                if constexpr (NBW > 1) most = fmaxf(most, lane_xor<16>(most));
+                if constexpr (NBW > 2) most = fmaxf(most, lane_xor<32>(most));
+                const PowerOfTwo s = scale_to_one(most);
+                if (tid % (16 * NBW) == 0) unscale[row] = inv * (s.inverse * (1 / TOP));
+                const bool live = BWD && tok_base + row < B;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    put(row, (n * BG + k) * BS + c4, v[k] * (s.scale * TOP));
+                    if (live) __builtin_nontemporal_store(v[k] * inv, reinterpret_cast<f32x4 *>(save + size_t(row) * D + (n * BG + k) * BS + c4));
+                }
+            }
+            __syncthreads();
+        } else {
+            float most = 0.f;
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) most = fmaxf(most, fabsf(acc[n][e]));
+            most = rows_most(most) * inv_w;
+            if (kq == 0) most_s[c * 4 + ow] = most;
+            __syncthreads();                      // every wavefront has read this stage's input and left its largest
+            const float4 m = *reinterpret_cast<const float4 *>(most_s + c * 4);
+            const PowerOfTwo s = scale_to_one(fmaxf(fmaxf(m.x, m.y), fmaxf(m.z, m.w)));
+            if (kq == 0 && ow == 0) unscale[c] = inv_x * (s.inverse * (1 / TOP));
+            const float scale = inv_w * (s.scale * TOP);
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) put(c, n * BS + 16 * ow + 4 * kq, acc[n] * scale);
+            if (BWD && tok_base + c < B) {
+                float *o = save + size_t(c) * D + 16 * ow + 4 * kq;
+                const float f = inv_w * inv_x;
+#pragma unroll
+                for (int n = 0; n < NBW; ++n) __builtin_nontemporal_store(acc[n] * f, reinterpret_cast<f32x4 *>(o + n * BS));
+            }
+            __syncthreads();
+        }
+    };
+    // wide form, after the last stage: the accumulators of strides 2 and 1 as well
+    auto last_strides = [&]() {
+        if constexpr (BG > 1) {
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+                *reinterpret_cast<f32x4 *>(wide_tile + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n];
+            __syncthreads();
+            if (tid < TOK * 16 * NBW) {
+                const int row = tid / (16 * NBW), n = (tid / 16) % NBW, c4 = (tid % 16) * 4;
+                float *p = wide_tile + row * LDR + n * BG * BS + c4;
+                f32x4 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4 *>(p + k * BS);
+                const f32x4 s0 = v[0] + v[2], s1 = v[1] + v[3], d0 = v[0] - v[2], d1 = v[1] - v[3];
+                v[0] = s0 + s1; v[1] = s0 - s1; v[2] = d0 + d1; v[3] = d0 - d1;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(p + k * BS) = v[k];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+                acc[n] = *reinterpret_cast<const f32x4 *>(wide_tile + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq);
+        }
+    };
+
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) load_w(BWD ? J - 1 : 0, n);
+    if constexpr (BWD) {
+        const int ncols = a.T * 8;
+#pragma unroll
+        for (int n = 0; n < NBW; ++n) {
+            const int gcol = r * D + (n * BG + bg) * BS + 16 * ow + 4 * kq;
+            f32x4 g = {0.f, 0.f, 0.f, 0.f};
+            if (tok_base + c < B && gcol < ncols) g = *reinterpret_cast<const f32x4 *>(a.gz + (tok_base + c) * ncols + gcol);
+            acc[n] = a.decay * g;
+        }
+#pragma unroll 1
+        for (int s = J - 1; s >= 0; --s) {
+            butterflies();
+            hand_over(a.stage_grads + ((size_t(r) * J + s) * B + tok_base) * D);
+            product(s);
+        }
+    } else {
+        // Sixteen lanes have a row (wide form: a wavefront, its sixteens every fourth 64 columns), 16 bytes a lane of every 64
+        // columns, all loads in flight before the first use.  Columns at or beyond H are zero.  Sums are taken over every fourth 64
+        // columns of a lane, then those, then the sixteen lanes, in either form.
+        constexpr int QG = BG > 1 ? 4 : 1, NQ = NB / QG, SG = NB < 4 ? NB : 4, LANES = 16 * QG;
+        const int l = tid & 15, g = QG > 1 ? (tid >> 4) & 3 : 0;
+        auto row_sum = [&](const float (&part)[NQ]) {
+            float sum[SG] = {};
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) sum[QG > 1 ? 0 : i % SG] += part[i];
+            float v = sum[0];
+            if constexpr (QG > 1) {
+                v += lane_xor<16>(v);
+                v += lane_xor<32>(v);
+            } else {
+                if constexpr (SG > 1) v += sum[1];
+                if constexpr (SG > 2) v += sum[2] + sum[3];
+            }
+            return lane_group_sum<16>(v);
+        };
+#pragma unroll
+        for (int row = tid / LANES; row < TOK; row += 64 * NWAVE / LANES) {
+            const int64_t tok = tok_base + row;
+            const float *px = x + min(tok, B - 1) * H;
+            f32x4 v[NQ];
+            float part[NQ];
+            auto column = [&](int i) { return (g + i * QG) * 64 + 4 * l; };
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) v[i] = *reinterpret_cast<const f32x4 *>(px + min(column(i), H - 4));
+            if (tok >= B || H < D) {
+#pragma unroll
+                for (int i = 0; i < NQ; ++i)
+                    if (tok >= B || column(i) >= H) v[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+            if (a.ln_w) {
+                // LayerNorm over the H valid columns (biased variance, two passes, eps inside the
+                // square root: torch.nn.LayerNorm, PL/lookup.py:84,99)
+#pragma unroll
+                for (int i = 0; i < NQ; ++i) part[i] = (v[i].x + v[i].y) + (v[i].z + v[i].w);
+                const float mean = row_sum(part) / float(H);
+#pragma unroll
+                for (int i = 0; i < NQ; ++i) {
+                    v[i] = v[i] - mean;
+                    const f32x4 sq = v[i] * v[i];
+                    part[i] = (sq.x + sq.y) + (sq.z + sq.w);
+                }
+                if (H < D) {
+#pragma unroll
+                    for (int i = 0; i < NQ; ++i)
+                        if (column(i) >= H) part[i] = 0.f;
+                }
+                const float rstd = 1.0f / sqrtf(row_sum(part) / float(H) + a.ln_eps);
+#pragma unroll
+                for (int i = 0; i < NQ; ++i)          // (weight and bias are zero beyond column H)
+                    v[i] = v[i] * rstd * *reinterpret_cast<const f32x4 *>(lnw_s + column(i)) +
+                           *reinterpret_cast<const f32x4 *>(lnb_s + column(i));
+                if (tid % LANES == 0) {
+                    stats[2 * row] = mean;
+                    stats[2 * row + 1] = rstd;
+                }
+            }
+            float most = 0.f;
+#pragma unroll
+            for (int i = 0; i < NQ; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) most = fmaxf(most, fabsf(v[i][e]));
+            most = fmaxf(most, lane_xor<1>(most));
+            most = fmaxf(most, lane_xor<2>(most));
+            most = fmaxf(most, lane_xor<4>(most));
+            most = fmaxf(most, lane_xor<8>(most));
+            if constexpr (QG > 1) {
+                most = fmaxf(most, lane_xor<16>(most));
+                most = fmaxf(most, lane_xor<32>(most));
+            }
+            const PowerOfTwo s = scale_to_one(most);
+            if (tid % LANES == 0) unscale[row] = s.inverse * (1 / TOP);
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) put(row, column(i), v[i] * (s.scale * TOP));
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int s = 0; s < J; ++s) {
+            product(s);
+            butterflies();
+            if (s + 1 < J) hand_over(nullptr);
+        }
+        last_strides();
+    }
+    const int64_t token = tok_base + c;
+    if constexpr (BWD) {
+        // grad x of this repeat: the first H columns, plus the residual path of the mix
+        const int ncols = a.T * 8;
+        if (token < B) {
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) {
+                const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq;
+                if (xc < H) {
+                    f32x4 o = acc[n] * (inv_w * inv_x);
+                    if (r * D + xc < ncols) o = o + a.residual * *reinterpret_cast<const f32x4 *>(a.gz + token * ncols + r * D + xc);
+                    *reinterpret_cast<f32x4 *>(a.g_x + (size_t(r) * B + token) * H + xc) = o;
+                }
+            }
+        }
+    } else {
+        __syncthreads();                          // the tile has been read: it takes the codes and scores
+        const int ncols = a.T * 8;
+        constexpr int CROW = D / 8 + 1;                // padded: tokens down a column hit different banks
+        int *cs = reinterpret_cast<int *>(xs);         // [TOK][CROW] codes of this repeat
+        float *ss = xs + TOK * CROW;                   // [TOK][CROW] scores
+        // the addresses below do not change from stage to stage; computed from an opaque
+        // zero they are formed here instead of being kept in registers through the stages
+        int opq = 0;
+        asm volatile("" : "+v"(opq));
+        const float mean = a.ln_w ? stats[2 * (c + opq)] : 0.f, rstd = a.ln_w ? stats[2 * (c + opq) + 1] : 1.f;
+        // the token's input values for every block, all requested before the first use (tokens and columns beyond the end: the last
+        // ones again, whose results go nowhere)
+        f32x4 xin[NBW];
+        const float *px = x + min(token + opq, B - 1) * H;
+#pragma unroll
+        for (int n = 0; n < NBW; ++n) xin[n] = *reinterpret_cast<const f32x4 *>(px + min((n * BG + bg) * BS + 16 * ow + 4 * kq, H - 4));
+        __builtin_amdgcn_sched_barrier(0);
+        // z of the lane's four columns of block n
+        auto form_z = [&](int n) {
+            const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq + opq;    // column of the padded input
+            // (without LayerNorm or bias: 0, 1, 1, 0 and 0; the weight is zero beyond column H)
+            const f32x4 xv = (xin[n] - mean) * rstd * *reinterpret_cast<const f32x4 *>(lnw_s + xc) +
+                             *reinterpret_cast<const f32x4 *>(lnb_s + xc);
+            const f32x4 z = a.decay * (inv_w * inv_x) * acc[n] + a.residual * xv +      // (decay times a power of two: as decay * y)
+                            *reinterpret_cast<const f32x4 *>(pbias_s + xc);
+            return z;
+        };
+        // Columns 8 g .. 8 g + 3 sit in the lane with even kq, 8 g + 4 .. 8 g + 7 in lane + 16.  Two groups of four are taken at a
+        // time and exchanged between the lanes' rows, so that an even row has all eight columns of the first and an odd row of the
+        // second: code, sum and product in column order (compute_code_score/torch_extension.cc:31-37), one division a lane.
+        constexpr int ITEMS = NBW;
+#pragma unroll
+        for (int i = 0; i < ITEMS; i += 2) {
+            const int i1 = i + 1 < ITEMS ? i + 1 : i;              // (a single one: with itself, the odd rows' copy is not used)
+            const f32x4 za = form_z(i), zb = form_z(i1);
+            float z[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const auto pair = __builtin_amdgcn_permlane16_swap(__float_as_uint(za[e]), __float_as_uint(zb[e]), false, false);
+                z[e] = __uint_as_float(pair[0]);
+                z[e + 4] = __uint_as_float(pair[1]);
+            }
+            int code = 0;
+            float sum = fabsf(z[0]), prod = 1.0f + exp_minus_2a(fabsf(z[0]));
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                asm("v_cmp_lt_f32 vcc, 0, %1\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(code) : "v"(z[e]) : "vcc");
+#pragma unroll
+            for (int e = 1; e < 8; ++e) {
+                sum = sum + fabsf(z[e]);
+                prod = prod * (1.0f + exp_minus_2a(fabsf(z[e])));
+            }
+            // staged in LDS, written out row by row below: straight from here a store would scatter 4-byte pieces over 32 rows
+            const bool odd = kq & 1;
+            const int at = c * CROW + ((odd ? i1 : i) * BG + bg) * 8 + 2 * ow + (kq >> 1);
+            if (ITEMS > 1 || !odd) {
+                cs[at] = code;
+                ss[at] = sum / prod;
+            }
+        }
+        __syncthreads();
+        if (a.records) {
+            // records: per table pair three words per token, the workgroup's TOK tokens (whole
+            // groups of 16: 192 contiguous bytes each) side by side; a token whose index has bit 1
+            // set takes the pair's tables in the order (2k+1, 2k)
+            static_assert((64 * NWAVE) % TOK == 0, "a thread stays on one token");
+            const int row = tid % TOK;
+            const int64_t tok = tok_base + row;
+            const int64_t slot = tok < B ? lffn_quad_record_slot(tok, a.rec_tile) : 0;
+            for (int kk = tid / TOK; kk < D / 16; kk += 64 * NWAVE / TOK) {
+                const int pair = r * (D / 16) + kk;
+                if (tok < B && 2 * pair + 1 < a.T) {
+                    const int ca = cs[row * CROW + 2 * kk], cb = cs[row * CROW + 2 * kk + 1];
+                    const float sa = ss[row * CROW + 2 * kk], sb = ss[row * CROW + 2 * kk + 1];
+                    const bool second_first = (tok & 2) != 0;
+                    uint32_t *dst = a.records + ((size_t)pair * a.rec_stride + slot) * LFFN_RECORD_WORDS;
+                    dst[0] = __float_as_uint(second_first ? sb : sa);
+                    dst[1] = __float_as_uint(second_first ? sa : sb);
+                    dst[2] = second_first ? (unsigned)(cb | (ca << 8)) : (unsigned)(ca | (cb << 8));
+                }
+            }
+        } else {
+            // every wavefront writes the D/8 codes and scores of TOK/NWAVE tokens
+#pragma unroll 1
+            for (int i = 0; i < TOK / NWAVE; ++i) {
+                const int row = wave * (TOK / NWAVE) + i;
+                const int64_t tok = tok_base + row;
+                if (tok >= B) break;
+#pragma unroll
+                for (int e0 = 0; e0 < D / 8; e0 += 64) {
+                    const int e = e0 + lane;
+                    const int tt = r * (D / 8) + e;
+                    if (e < D / 8 && tt < a.T) {
+                        a.codes[tok * a.T + tt] = cs[row * CROW + e];
+                        a.scores[tok * a.T + tt] = ss[row * CROW + e];
+                    }
+                }
+            }
+        }
+    }
+}
+
+template <int NB, bool BWD, int BG>
+int launch_form(const SplitArgs &a, hipStream_t st) {
+    constexpr int TOK = 16, D = BS * NB;
+    constexpr size_t lds_bytes = 2 * TOK * (2 * D + 16) + (BG > 1 ? TOK * (D + PAD) * 4 : 0) + 7 * TOK * 4 + (BWD ? 0 : 3 * D * 4);
+    static_assert(lds_bytes <= 160 * 1024);
+    auto kern = bh4_split_kernel<NB, BWD, BG>;
+    static LdsGrant granted;      // one record per kernel instantiation
+    if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(kern), lds_bytes, granted)) return LFFN_ERR_LAUNCH;
+    const dim3 grid((unsigned)((a.B + TOK - 1) / TOK), (unsigned)a.R);
+    hipLaunchKernelGGL(kern, grid, dim3(256 * BG), lds_bytes, st, a);
+    return lffn_launch_status();
+}
+
+// The wide form where its workgroups leave no compute unit a second one: there 4 wavefronts wait for every latency of their own.
+// Forward / backward, 4 -> 16 wavefronts: 2103 tokens, D = 1024 23.7 -> 20.9 / 31.2 -> 21.5 us; 385, D = 512 12.3 both / 15.3 ->
+// 12.2; 600, D = 256, four repeats 9.6 -> 9.7 / 10.4 -> 9.4.  Two rounds of it: 4096, D = 512, two repeats 19.1 -> 26.8 / 30.7 -> 29.7.
+constexpr int64_t WIDE_WORKGROUPS = 256;
+
+template <int NB, bool BWD>
+int launch_block(const SplitArgs &a, hipStream_t st) {
+    if constexpr (NB >= 4)
+        if ((a.B + 15) / 16 * a.R <= WIDE_WORKGROUPS) return launch_form<NB, BWD, 4>(a, st);
+    return launch_form<NB, BWD, 1>(a, st);
+}
+
+template <bool BWD>
+int dispatch_block(const SplitArgs &a, int64_t D, hipStream_t st) {
+    switch (D / BS) {
+        case 1: return launch_block<1, BWD>(a, st);
+        case 2: return launch_block<2, BWD>(a, st);
+        case 4: return launch_block<4, BWD>(a, st);
+        case 8: return launch_block<8, BWD>(a, st);
+        default: return launch_block<16, BWD>(a, st);
+    }
+}
+
+}  // namespace
+
+extern "C" int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t stages, int64_t num_block, int64_t block_size,
+                                       int32_t transposed, void *stream) {
+    LFFN_REQUIRE(stages >= 0 && stages <= (1 << 20) && num_block >= 1, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(block_size == BS && lffn_is_pow2(num_block) && num_block <= 16, LFFN_ERR_UNSUPPORTED);
+    if (stages == 0) return LFFN_OK;
+    LFFN_REQUIRE(w && w_split && w != w_split && lffn_aligned16(w_split), LFFN_ERR_BAD_ARG);
+    float *inverse = w_split + stages * num_block * (BS * BS);
+    auto kern = transposed ? bh4_fold_split_kernel<true> : bh4_fold_split_kernel<false>;
+    const size_t lds = transposed ? 0 : num_block * 16 * 65 * sizeof(float);
+    static LdsGrant granted;
+    if (lds > 65000 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(kern), lds, granted)) return LFFN_ERR_LAUNCH;
+    hipLaunchKernelGGL(kern, dim3((unsigned)stages), dim3((unsigned)(BS * num_block)), lds, static_cast<hipStream_t>(stream), w,
+                       reinterpret_cast<uint32_t *>(w_split), inverse);
+    return lffn_launch_status();
+}
+
+extern "C" int lffn_bh4_block_front_split_f32(const lffn_block_front *f, const float *x, int64_t B, void *stream) {
+    LFFN_REQUIRE(f, LFFN_ERR_BAD_ARG);
+    const int64_t H = f->H, D = f->D, R = f->R, J = f->J, T = f->T;
+    LFFN_REQUIRE(B >= 0 && R >= 1 && J >= 1 && D >= 1 && H >= 1 && H <= D && T >= 1, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(H % 4 == 0 && J <= 64, LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(lffn_is_pow2(D) && D >= BS && D <= 1024, LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(R <= 4096 && B <= (int64_t(1) << 31) - 1 && T <= (1 << 24), LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(T * 8 <= R * D, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(!f->ln_weight || (f->ln_bias && f->ln_eps >= 0.f), LFFN_ERR_BAD_ARG);
+    if (B == 0) return LFFN_OK;
+    LFFN_REQUIRE(x && f->w_split && (f->records || (f->codes && f->scores)), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(!f->records || (T % 2 == 0 && lffn_record_layout_ok(B, f->record_stride, f->tokens_per_workgroup) &&
+                                 (uintptr_t)f->records % 4 == 0), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(x) && lffn_aligned16(f->w_split) && lffn_aligned16(f->proj_bias) && lffn_aligned16(f->ln_weight) &&
+                     lffn_aligned16(f->ln_bias), LFFN_ERR_BAD_ARG);
+    SplitArgs a{};
+    a.x = x; a.ln_w = f->ln_weight; a.ln_b = f->ln_bias; a.ln_eps = f->ln_eps; a.w = f->w_split;
+    a.wscale = f->w_split + R * J * D * BS; a.pbias = f->proj_bias; a.codes = f->codes; a.scores = f->scores;
+    a.records = f->records; a.rec_stride = f->record_stride; a.rec_tile = f->tokens_per_workgroup;
+    a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = f->decay; a.residual = f->residual;
+    return dispatch_block<false>(a, D, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float *g_x, float *stage_grads, int64_t B,
+                                            int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t block_size, float decay,
+                                            float residual, void *stream) {
+    LFFN_REQUIRE(B >= 0 && R >= 1 && J >= 1 && D >= 1 && H >= 1 && H <= D && T >= 1, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(H % 4 == 0 && J <= 64, LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(block_size == BS && lffn_is_pow2(D) && D >= BS && D <= 1024, LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(R <= 4096 && B <= (int64_t(1) << 31) - 1 && T <= (1 << 24), LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(T * 8 <= R * D, LFFN_ERR_BAD_ARG);
+    if (B == 0) return LFFN_OK;
+    LFFN_REQUIRE(g_z && w_split_t && g_x && stage_grads, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(g_z) && lffn_aligned16(w_split_t) && lffn_aligned16(g_x) && lffn_aligned16(stage_grads), LFFN_ERR_BAD_ARG);
+    SplitArgs a{};
+    a.gz = g_z; a.w = w_split_t; a.wscale = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_grads = stage_grads;
+    a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = decay; a.residual = residual;
+    return dispatch_block<true>(a, D, static_cast<hipStream_t>(stream));
+}

@@ -46,15 +46,15 @@ using torch::autograd::variable_list;
     X(lffn_lookup_ffn_fused_layer_rows)     \
     X(lffn_lookup_gather_records_plan_rows) \
     X(lffn_ln_project_hash_records_f32)     \
-    X(lffn_ln_bh4_block_hash_records_f32)   \
     X(lffn_lookup_gather_records_rows)      \
     X(lffn_ln_project_hash_f32)             \
-    X(lffn_ln_bh4_block_hash_f32)           \
     X(lffn_lookup_gather_workspace_bytes)   \
     X(lffn_lookup_gather_ws_f32)            \
     X(lffn_lookup_gather_ws_bf16)           \
     X(lffn_lookup_gather_ws_f16)            \
     X(lffn_ln_bh4_block_hash_train_f32)     \
+    X(lffn_bh4_block_front_split_f32)       \
+    X(lffn_bh4_fold_split_f32)              \
     X(lffn_bh4_fold_mode_f32)               \
     X(lffn_lookup_scatter_workspace_bytes)  \
     X(lffn_lookup_backward_f32)             \
@@ -63,7 +63,7 @@ using torch::autograd::variable_list;
     X(lffn_lookup_scatter_sorted_f32)       \
     X(lffn_ln_project_hash_bwd_f32)         \
     X(lffn_code_score_bwd_f32)              \
-    X(lffn_bh4_block_bwd_f32)               \
+    X(lffn_bh4_block_bwd_split_f32)         \
     X(lffn_ln_bh4_block_wgrad_f32)          \
     X(lffn_layer_norm_bwd_f32)              \
     X(lffn_sum_partials_f32)
@@ -109,7 +109,7 @@ struct Parts {
 };
 
 PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES, *KEY_EPS,
-    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_FOLDED;      // interned
+    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_SPLIT;      // interned
 
 PyObject *dict_of(PyObject *o) {
     PyObject **d = o ? _PyObject_GetDictPtr(o) : nullptr;
@@ -202,7 +202,28 @@ void gather(const Config &c, const Tensor &codes, const Tensor &scores, const Te
 // The layer's parameters: LayerNorm's, the projection's, tables and output bias.
 using Params = std::array<Tensor, 6>;
 
-void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor &x, const float *residual, Tensor &out, int64_t B,
+// The 64 x 64 blocks' kernel with the layer's parameters, its outputs open.
+lffn_block_front block_front(const Config &c, const Params &p, const Tensor &split) {
+    lffn_block_front f{};
+    f.ln_weight = f32(p[0]);
+    f.ln_bias = f32(p[1]);
+    f.w_split = f32(split);
+    f.proj_bias = f32(p[3]);
+    f.H = c.H;
+    f.D = c.D;
+    f.R = c.R;
+    f.J = c.J;
+    f.T = c.T;
+    f.ln_eps = (float)c.eps;
+    f.decay = (float)c.decay;
+    f.residual = (float)c.residual;
+    return f;
+}
+
+// Floats of the split weights (lffn_bh4_fold_split_f32).
+int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 4); }
+
+void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &x, const float *residual, Tensor &out, int64_t B,
            int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
@@ -223,9 +244,13 @@ void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor 
         if (c.form == DIAG)
             CALL(lffn_ln_project_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, decay, res, st);
-        else
-            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), rp, plan.stride,
-                 plan.tokens, B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
+        else {
+            lffn_block_front front = block_front(c, p, split);
+            front.records = rp;
+            front.record_stride = plan.stride;
+            front.tokens_per_workgroup = plan.tokens;
+            CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
+        }
         CALL(lffn_lookup_gather_records_rows, rp, plan.stride, p[4].data_ptr(), f32(p[5]), residual, f32(out), B, c.T, c.S, c.Do,
              (int32_t)c.fmt, plan.tokens, st);
         return;
@@ -235,9 +260,12 @@ void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor 
     if (c.form == DIAG)
         CALL(lffn_ln_project_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), nullptr, cp, f32(scores), B, c.H,
              c.D, c.R, c.J, c.T, decay, res, st);
-    else
-        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), B, c.H, c.D,
-             c.R, c.J, c.T, 64, decay, res, st);
+    else {
+        lffn_block_front front = block_front(c, p, split);
+        front.codes = cp;
+        front.scores = f32(scores);
+        CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
+    }
     gather(c, codes, scores, p[4], p[5], residual, out, B, plan.ws_bytes, st);
 }
 
@@ -355,11 +383,11 @@ struct LookupFFNBackward : public torch::autograd::Node {
             }
         } else {
             const Tensor stage = stage_in.unpack(self), st_ = stats.unpack(self);
-            Tensor g_z = empty_f32({B, T * 8}, dev), stage_g = empty_f32({R * J, B, D}, dev), folded = at::empty_like(w);
+            Tensor g_z = empty_f32({B, T * 8}, dev), stage_g = empty_f32({R * J, B, D}, dev), split = empty_f32({split_words(c)}, dev);
             CALL(lffn_code_score_bwd_f32, f32(z_), f32(g_score), f32(g_z), B * T, 8, st);
             const int64_t blocks = R * J * (D / 64);
-            CALL(lffn_bh4_fold_mode_f32, f32(w), f32(folded), blocks, 64, 1, st);
-            CALL(lffn_bh4_block_bwd_f32, f32(g_z), f32(folded), f32(g_h), f32(stage_g), B, H, D, R, J, T, 64, decay, res, st);
+            CALL(lffn_bh4_fold_split_f32, f32(w), f32(split), R * J, D / 64, 64, 1, st);
+            CALL(lffn_bh4_block_bwd_split_f32, f32(g_z), f32(split), f32(g_h), f32(stage_g), B, H, D, R, J, T, 64, decay, res, st);
             if (need[WEIGHT]) {
                 Tensor g_folded = at::zeros({R * J, D / 64, 64, 64}, at::TensorOptions().dtype(at::kFloat).device(dev));
                 CALL(lffn_ln_bh4_block_wgrad_f32, f32(stage_g), f32(x_), f32(lw), f32(lb), f32(st_), J > 1 ? f32(stage) : nullptr, f32(g_folded),
@@ -505,19 +533,19 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._folded = ((version, address, device), folded weights, what they were folded from), as Hashing.folded_weight keeps them: the
-// folded weights if they are w's.
-Tensor folded_of(PyObject *hash, const Tensor &w) {
-    PyObject *kept = item(dict_of(hash), KEY_FOLDED);
+// hash._split = ((version, address, device), split weights, what they were made from), as Hashing.split_weight keeps them: the
+// split weights if they are w's.
+Tensor split_of(PyObject *hash, const Tensor &w, int64_t words) {
+    PyObject *kept = item(dict_of(hash), KEY_SPLIT);
     if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3) return {};
-    PyObject *key = PyTuple_GET_ITEM(kept, 0), *folded = PyTuple_GET_ITEM(kept, 1);
+    PyObject *key = PyTuple_GET_ITEM(kept, 0), *split = PyTuple_GET_ITEM(kept, 1);
     int64_t version = 0, address = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
-        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(folded))
+        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(split))
         return {};
-    const Tensor &f = THPVariable_Unpack(folded);
+    const Tensor &f = THPVariable_Unpack(split);
     const bool same = w._version() == (uint32_t)version && w.data_ptr() == reinterpret_cast<void *>(address) && f.device() == w.device() &&
-                      f.numel() == w.numel();
+                      f.numel() == words;
     return same ? f : Tensor();
 }
 
@@ -528,7 +556,7 @@ struct WithoutInterpreter {
 };
 
 // forward(layer, x, residual or None, tokens up to which the one-launch form is taken) -> a tensor; None: not for this path;
-// False: the folded weights (Hashing.folded_weight) are not up to date
+// False: the split weights (Hashing.split_weight) are not up to date
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 4, "forward: 4 arguments");
@@ -564,13 +592,13 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         for (const Tensor &t : params) grads = grads || t.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;
-    Tensor folded;
-    if (!grads && c.form == BLOCK && !(folded = folded_of(parts.hash, params[2])).defined()) Py_RETURN_FALSE;
+    Tensor split;
+    if (!grads && c.form == BLOCK && !(split = split_of(parts.hash, params[2], split_words(c))).defined()) Py_RETURN_FALSE;
     const int64_t fused_max = PyLong_AsLongLong(args[3]);
     if (fused_max == -1 && PyErr_Occurred()) return nullptr;
     Tensor out;
     {
-        // (from here on only what is owned here is used: x, the residual, the parameters and the folded weights)
+        // (from here on only what is owned here is used: x, the residual, the parameters and the split weights)
         const WithoutInterpreter unlocked;
         // any layout of x and any shape and type of the residual, as the Python path makes them
         x = x.contiguous();
@@ -580,7 +608,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
             (!residual.defined() || reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0)) {
             out = empty_f32(sizes, dev);
             if (grads) train(c, params, x, residual, out, B);
-            else infer(c, params, folded, x, f32(residual), out, B, fused_max);
+            else infer(c, params, split, x, f32(residual), out, B, fused_max);
         }
     }
     if (!out.defined()) Py_RETURN_NONE;
@@ -603,7 +631,7 @@ PyMODINIT_FUNC PyInit__host() {
         {&KEY_MODULES, "_modules"}, {&KEY_PARAMETERS, "_parameters"}, {&KEY_LAYER_NORM, "LayerNorm"}, {&KEY_HASH, "hash"},
         {&KEY_PROJECTION, "projection"}, {&KEY_WEIGHT, "weight"}, {&KEY_BIAS, "bias"}, {&KEY_TABLES, "tables"},
         {&KEY_EPS, "eps"}, {&KEY_DECAY, "decay_coeff"}, {&KEY_NUM_TABLE, "num_table"},
-        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_FOLDED, "_folded"},
+        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_SPLIT, "_split"},
     };
     for (const auto &[key, name] : keys)
         if (!(*key = PyUnicode_InternFromString(name))) return nullptr;

@@ -36,6 +36,15 @@ __device__ __forceinline__ uint32_t split_lo(float a, float b, float scale, uint
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
 }
 
+// lo without the factor, of two numbers that are large enough for it to be among half's normal numbers (their largest 2^6 and more)
+__device__ __forceinline__ uint32_t split_rest(float a, float b, uint32_t hi) {
+    f32x2_t v;
+    // a - hi (exact), the half-precision operand widened inside the instruction: the compiler forms a conversion and a subtraction
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(v[0]) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(v[1]) : "v"(hi), "v"(b));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+}
+
 __device__ __forceinline__ f32x16_t mfma_f16(uint4 a, uint4 b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
@@ -52,7 +61,7 @@ struct PowerOfTwo {
 };
 __device__ __forceinline__ PowerOfTwo scale_to_one(float most) {
     uint32_t e = (__float_as_uint(most) >> 23) & 0xFFu;
-    e = e == 0 || e == 255 ? 127 : min(max(e, 2u), 252u);
+    e = e == 0 || e == 255 ? 127 : min(max(e, 16u), 252u);          // (times or by 2^15 still a normal number)
     return {__uint_as_float((254 - e) << 23), __uint_as_float(e << 23)};
 }
 

@@ -121,7 +121,7 @@ class BlockProjectHash(torch.autograd.Function):
         B, H = x.shape
         T = g_score.shape[1]
         g_z = ops.code_score_bwd(z.reshape(B, T, 8), g_score.contiguous()).reshape(B, T * 8)
-        g_x, stage_g = ops.bh4_block_bwd(g_z, ops.bh4_fold_mode(w, 1), H, ctx.decay, 1 - ctx.decay)
+        g_x, stage_g = ops.bh4_block_bwd_split(g_z, ops.bh4_fold_split(w, True), R, J, NB * bs, H, ctx.decay, 1 - ctx.decay)
         g_w = None
         if ctx.needs_input_grad[1]:
             # stage 0 reads x (zero beyond its H columns), stage j the saved input of that stage
@@ -190,27 +190,35 @@ class Hashing(nn.Module):
         ``invalidate_folded_weight()``; switching the module between train() and eval() drops
         the cached copy as well.  The weights it was folded from stay allocated with it, so that no
         other weight takes their address."""
+        return self._kept("_folded", ops.bh4_fold)
+
+    def split_weight(self):
+        """folded_weight() as the block kernels multiply it (ops.bh4_fold_split), kept in the same way."""
+        return self._kept("_split", lambda w: ops.bh4_fold_split(w, False))
+
+    def _kept(self, name, make):
         w = self.projection.weight
         key = (w._version, w.data_ptr(), w.device)
-        cached = getattr(self, "_folded", None)
+        cached = getattr(self, name, None)
         if cached is None or cached[0] != key:
             alias = w.detach()
-            cached = (key, ops.bh4_fold(alias.contiguous()), alias)
-            self._folded = cached
+            cached = (key, make(alias.contiguous()), alias)
+            setattr(self, name, cached)
         return cached[1]
 
     def __getstate__(self):
         state = self.__dict__.copy()
-        state.pop("_folded", None)        # derived from the weight, and names its address
+        for name in ("_folded", "_split"):
+            state.pop(name, None)         # derived from the weight, and names its address
         return state
 
     def invalidate_folded_weight(self):
-        """Forget the folded copy of the BH4 weights: the next block-64 inference call folds again."""
-        self._folded = None
+        """Forget the folded copies of the BH4 weights: the next block-64 inference call folds again."""
+        self._folded = self._split = None
 
     def train(self, mode=True):
         if mode != self.training:
-            self._folded = None           # weights usually change between an eval and the next one
+            self.invalidate_folded_weight()          # weights usually change between an eval and the next one
         return super().train(mode)
 
     def forward_block(self, x, layer_norm=None):
@@ -222,8 +230,8 @@ class Hashing(nn.Module):
             lw = None if layer_norm is None else layer_norm.weight
             lb = None if layer_norm is None else layer_norm.bias
             eps = 0.0 if layer_norm is None else float(layer_norm.eps)
-            return ops.ln_bh4_block_hash(x, lw, lb, eps, self.folded_weight(), p.bias, self.num_table,
-                                         float(p.decay_coeff), float(1 - p.decay_coeff))
+            return ops.bh4_block_front(x, lw, lb, eps, self.split_weight(), p.num_repeat, p.weight.shape[1], p.padded_in_dim, p.bias,
+                                       self.num_table, float(p.decay_coeff), float(1 - p.decay_coeff))
         if layer_norm is not None:
             x = layer_norm(x)
         y = ops.bh4_block(x, self.folded_weight())
@@ -345,7 +353,7 @@ class LnBlockProjectHash(torch.autograd.Function):
         T = g_score.shape[1]
         need = ctx.needs_input_grad
         g_z = ops.code_score_bwd(z.reshape(B, T, 8), g_score.contiguous()).reshape(B, T * 8)
-        g_h, stage_g = ops.bh4_block_bwd(g_z, ops.bh4_fold_mode(w, 1), H, ctx.decay, 1 - ctx.decay)
+        g_h, stage_g = ops.bh4_block_bwd_split(g_z, ops.bh4_fold_split(w, True), R, J, NB * bs, H, ctx.decay, 1 - ctx.decay)
         g_w = None
         if need[4]:
             g_folded = ops.ln_bh4_block_wgrad(stage_g.reshape(R * J, B, NB * bs), x, ln_weight, ln_bias, stats, stage_in,
@@ -414,7 +422,7 @@ class LookupFFN(nn.Module):
             return None
         out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         if out is False:                  # the 64 x 64 blocks have changed since they were folded
-            self.hash.folded_weight()
+            self.hash.split_weight()
             out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         return None if out is False else out
 

@@ -398,6 +398,94 @@ def _(g_z, w_folded_t, H, decay, residual):
     return g_z.new_empty(R, g_z.shape[0], H), g_z.new_empty(R, J, g_z.shape[0], NB * bs)
 
 
+# ----------------------------------------------------------------------------- bh4_block with split weights
+
+_L.define("bh4_fold_split(Tensor w, bool transposed) -> Tensor")
+
+
+def split_words(w_shape):
+    """Words of the split form of weights [R, J, D/64, 64, 64]."""
+    R, J, NB, _, _ = w_shape
+    return R * J * (NB * 4096 + 4)
+
+
+def _bh4_fold_split_impl(w: torch.Tensor, transposed: bool) -> torch.Tensor:
+    """The folded weights as the block kernels multiply them, two half-precision terms a number: what bh4_block_front takes and,
+    transposed, bh4_block_bwd_split."""
+    _lib.require_gpu(w)
+    assert w.dim() == 5 and w.shape[3] == w.shape[4] == 64 and w.dtype == torch.float32 and w.is_contiguous()
+    R, J, NB, bs, _ = w.shape
+    out = torch.empty(split_words(w.shape), dtype=torch.float32, device=w.device)
+    with _dev_guard(w):
+        rc = _lib.load().lffn_bh4_fold_split_f32(_lib.ptr(w), _lib.ptr(out), R * J, NB, bs, int(transposed), _lib.stream_of(w))
+    _lib.check(rc, f"lffn_bh4_fold_split_f32(stages={R * J}, num_block={NB}, transposed={transposed})")
+    return out
+
+
+_L.impl("bh4_fold_split", _bh4_fold_split_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::bh4_fold_split")
+def _(w, transposed):
+    return w.new_empty(split_words(w.shape))
+
+
+_L.define("bh4_block_front(Tensor x, Tensor? ln_w, Tensor? ln_b, float eps, Tensor w_split, int R, int J, int D, Tensor? bias, int T, "
+          "float decay, float residual) -> (Tensor, Tensor)")
+
+
+def _bh4_block_front_impl(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
+    """(LayerNorm ->) 64 x 64 blocks -> mix -> hash -> (codes [B,T], scores [B,T])."""
+    _lib.require_gpu(x, ln_w, ln_b, w_split, bias)
+    for t in (x, ln_w, ln_b, w_split, bias):
+        assert t is None or (t.dtype == torch.float32 and t.is_contiguous())
+    B, H = x.shape
+    assert H <= D and T * 8 <= R * D and w_split.numel() == split_words((R, J, D // 64, 64, 64)) and (ln_w is None) == (ln_b is None)
+    assert ln_w is None or (ln_w.numel() == H and ln_b.numel() == H)
+    assert bias is None or bias.numel() == T * 8
+    codes = torch.empty(B, T, dtype=torch.int32, device=x.device)
+    scores = torch.empty(B, T, dtype=torch.float32, device=x.device)
+    front = _lib.BlockFront(_lib.ptr(ln_w), _lib.ptr(ln_b), _lib.ptr(w_split), _lib.ptr(bias), codes.data_ptr(), scores.data_ptr(), None,
+                            0, H, D, R, J, T, 0, eps, decay, residual)
+    with _dev_guard(x):
+        rc = _lib.load().lffn_bh4_block_front_split_f32(ctypes.byref(front), _lib.ptr(x), B, _lib.stream_of(x))
+    _lib.check(rc, f"lffn_bh4_block_front_split_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
+    return codes, scores
+
+
+_L.impl("bh4_block_front", _bh4_block_front_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::bh4_block_front")
+def _(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
+    return torch.empty(x.shape[0], T, dtype=torch.int32, device=x.device), x.new_empty(x.shape[0], T)
+
+
+_L.define("bh4_block_bwd_split(Tensor g_z, Tensor w_split_t, int R, int J, int D, int H, float decay, float residual) -> (Tensor, Tensor)")
+
+
+def _bh4_block_bwd_split_impl(g_z, w_split_t, R, J, D, H, decay, residual):
+    """bh4_block_bwd -> (g_x [R,B,H], stage_grads [R,J,B,D])."""
+    _lib.require_gpu(g_z, w_split_t)
+    assert g_z.dim() == 2 and g_z.dtype == torch.float32 and g_z.is_contiguous() and g_z.shape[1] % 8 == 0
+    assert w_split_t.dtype == torch.float32 and w_split_t.is_contiguous() and w_split_t.numel() == split_words((R, J, D // 64, 64, 64))
+    B, T = g_z.shape[0], g_z.shape[1] // 8
+    g_x, stage_g = g_z.new_empty(R, B, H), g_z.new_empty(R, J, B, D)
+    with _dev_guard(g_z):
+        rc = _lib.load().lffn_bh4_block_bwd_split_f32(_lib.ptr(g_z), _lib.ptr(w_split_t), _lib.ptr(g_x), _lib.ptr(stage_g), B, H, D, R,
+                                                      J, T, 64, decay, residual, _lib.stream_of(g_z))
+    _lib.check(rc, f"lffn_bh4_block_bwd_split_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
+    return g_x, stage_g
+
+
+_L.impl("bh4_block_bwd_split", _bh4_block_bwd_split_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::bh4_block_bwd_split")
+def _(g_z, w_split_t, R, J, D, H, decay, residual):
+    return g_z.new_empty(R, g_z.shape[0], H), g_z.new_empty(R, J, g_z.shape[0], D)
+
+
 _L.define("bh4_block_wgrad(Tensor stage_grads, Tensor x, Tensor stage_inputs, int R, int J) -> Tensor")
 
 
@@ -1107,6 +1195,9 @@ bh4_diag = torch.ops.lookupffn.bh4_diag
 bh4_fold = torch.ops.lookupffn.bh4_fold
 bh4_block = torch.ops.lookupffn.bh4_block
 mix_code_score = torch.ops.lookupffn.mix_code_score
+bh4_fold_split = torch.ops.lookupffn.bh4_fold_split
+bh4_block_front = torch.ops.lookupffn.bh4_block_front
+bh4_block_bwd_split = torch.ops.lookupffn.bh4_block_bwd_split
 bh4_fold_mode = torch.ops.lookupffn.bh4_fold_mode
 bh4_block_hash_train = torch.ops.lookupffn.bh4_block_hash_train
 bh4_block_bwd = torch.ops.lookupffn.bh4_block_bwd

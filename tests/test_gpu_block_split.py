@@ -1,0 +1,121 @@
+"""64 x 64 blocks on the fp16 matrix cores (csrc/bh4_split.hip) against 64 bits."""
+import math
+
+import pytest
+import torch
+
+from lookupffn_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _randn(gen, *shape):
+    return torch.randn(*shape, generator=gen, device=DEV)
+
+
+def _hadamard(n):
+    h = torch.ones(1, 1, dtype=torch.float64)
+    while h.shape[0] < n:
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    return h
+
+
+def _blocks(w, u):
+    n, D = u.shape
+    return torch.matmul(w.contiguous().unsqueeze(0), u.reshape(n, D // 64, 64, 1)).reshape(n, D)
+
+
+def _rel(a, b):
+    return ((a.double().cpu() - b).norm() / b.norm()).item()
+
+
+# Four stages of sums over 64: a product is off by 2^-22 at most, a sum by 2^-24 in each of 6 instructions; then butterflies, log2 D
+# additions.  Per stage 2^-22 + sqrt(6 + 4) 2^-24 at worst, of either sign from stage to stage: 2 * 4.3e-7.
+REL = 8.6e-7
+
+
+# every number of blocks, both forms of the kernel (few and many workgroups), rows around the 16 of a tile, columns short of D, codes
+# short of them
+@pytest.mark.parametrize("B,H,D,R,T", [(1, 64, 64, 2, 16), (33, 100, 128, 2, 30), (70, 256, 256, 1, 32), (4200, 200, 256, 1, 32),
+                                       (31, 512, 512, 2, 100), (2300, 500, 512, 2, 128), (17, 768, 1024, 1, 128), (4100, 1024, 1024, 1, 128)])
+@pytest.mark.parametrize("with_ln", [True, False])
+def test_against_64_bits(B, H, D, R, T, with_ln):
+    gen = torch.Generator(device=DEV).manual_seed(B + D)
+    J, NB = 4, D // 64
+    x, w = 1.5 * _randn(gen, B, H) + 0.3, _randn(gen, R, J, NB, 64, 64) / math.sqrt(64 * D)
+    lw, lb = (1 + 0.1 * _randn(gen, H), 0.1 * _randn(gen, H)) if with_ln else (None, None)
+    bias = 0.05 * _randn(gen, T * 8) if with_ln else None
+    split = ops.bh4_fold_split(w, False)
+    codes, scores = ops.bh4_block_front(x, lw, lb, 1e-5, split, R, J, D, bias, T, 0.7, 0.3)
+    few = min(B, 20)
+    for a, b in zip(ops.bh4_block_front(x[:few], lw, lb, 1e-5, split, R, J, D, bias, T, 0.7, 0.3), (codes, scores)):
+        assert torch.equal(a, b[:few])                # whichever form, whatever the neighbours
+    some = list(range(min(B, 40))) + [B - 1]
+    h = x[some].double().cpu()
+    if with_ln:
+        h = torch.nn.functional.layer_norm(h, (H,), lw.double().cpu(), lb.double().cpu(), 1e-5)
+    h = torch.cat([h, torch.zeros(len(some), D - H, dtype=torch.float64)], 1)
+    w64, HD, HN = w.double().cpu(), _hadamard(D), _hadamard(NB)
+    z = []
+    for r in range(R):
+        u = h
+        for j in range(J):
+            u = _blocks(w64[r, j], u) @ HD
+        z.append(0.7 * u + 0.3 * h)
+    z = torch.cat(z, 1)[:, :T * 8] + (bias.double().cpu() if with_ln else 0)
+    z8, size = z.view(len(some), T, 8), z.pow(2).mean().sqrt()
+    code = ((z8 > 0) * (2 ** torch.arange(7, -1, -1))).sum(-1)
+    same = code == codes[some].cpu()
+    # six standard deviations of an error of REL (and LayerNorm's, as large)
+    assert (z8.abs().amin(-1)[~same] <= 12 * REL * size).all() and same.double().mean() >= 0.999
+    score = z8.abs().sum(-1) / (1 + torch.exp(-2 * z8.abs())).prod(-1)
+    # a score moves at most 2.2 times as far as a z of its eight (1 + 1.25 sum / product for small ones), 8^0.5 of them together
+    assert ((scores[some].double().cpu() - score)[same].norm() / score.norm()) <= 6.3 * 2 * REL
+
+    g_z = _randn(gen, B, T * 8)
+    split_t = ops.bh4_fold_split(w, True)
+    g_x, stage_g = ops.bh4_block_bwd_split(g_z, split_t, R, J, D, H, 0.7, 0.3)
+    g_few, stage_few = ops.bh4_block_bwd_split(g_z[:few], split_t, R, J, D, H, 0.7, 0.3)
+    assert torch.equal(g_few, g_x[:, :few]) and torch.equal(stage_few, stage_g[:, :, :few])
+    g_pad = torch.cat([g_z[some].double().cpu(), torch.zeros(len(some), R * D - T * 8, dtype=torch.float64)], 1)
+    for r in range(R):
+        g = g_pad[:, r * D:(r + 1) * D]
+        G = 0.7 * g
+        for j in range(J - 1, -1, -1):
+            assert _rel(stage_g[r, j][some], torch.matmul(HN, G.view(-1, NB, 64)).reshape(-1, D)) <= REL
+            G = _blocks(w64[r, j].transpose(-1, -2), G @ HD)
+        assert _rel(g_x[r][some], (G + 0.3 * g)[:, :H]) <= REL
+
+
+@pytest.mark.parametrize("B", [40, 9000])
+def test_scales_and_rows_of_their_own(B):
+    """Any size of gradients and weights, rows of very different sizes side by side, and a row that is not finite stays alone."""
+    gen = torch.Generator(device=DEV).manual_seed(B)
+    D, J, T = 256, 4, 32
+    g, w = _randn(gen, B, D), _randn(gen, 1, J, D // 64, 64, 64) / math.sqrt(64 * D)
+    back = lambda g, w: ops.bh4_block_bwd_split(g, ops.bh4_fold_split(w, True), 1, J, D, D, 1.0, 0.0)[0][0]
+    want, HD = g[:40].double().cpu(), _hadamard(D)
+    for j in range(J - 1, -1, -1):
+        want = _blocks(w[0, j].double().cpu().transpose(-1, -2), want @ HD)
+    for sg, sw in ((1e20, 1e-6), (1e-25, 1e6), (1e-8, 1e-4), (1e-3, 1e8)):
+        assert _rel(back(g * sg, w * sw)[:40].double() / (sg * sw ** 4), want) <= REL
+    base = back(g, w)
+    y = g.clone()
+    y[3] *= 1e-15
+    y[5] *= 1e15
+    y[7] = 0
+    y[11, 3], y[12, 9] = float("nan"), float("inf")
+    got = back(y, w)
+    rows = [i for i in range(40) if i not in (3, 5, 7, 11, 12)]
+    assert torch.equal(got[rows], base[rows])
+    assert _rel(got[3].double() * 1e15, want[3]) <= REL and _rel(got[5].double() * 1e-15, want[5]) <= REL
+    assert torch.equal(got[7], torch.zeros_like(got[7])) and got[11].isnan().all() and got[12].isnan().all()
+    # the forward: a power of two changes no code
+    front = lambda x: ops.bh4_block_front(x, None, None, 0.0, ops.bh4_fold_split(w, False), 1, J, D, None, T, 1.0, 0.0)[0]
+    codes = front(g)
+    for s in (2.0 ** 60, 2.0 ** -60):
+        assert torch.equal(front(g * s), codes)
+    got = front(y)
+    assert torch.equal(got[rows + [7]], torch.cat([codes[rows], torch.zeros_like(codes[:1])]))
+    assert not got[11].any() and not got[12].any()                  # NaN is not above zero
