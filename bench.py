@@ -118,6 +118,10 @@ def gather_form(B, T, S, Do, fmt):
 
     from lookupffn_amd import _lib
     lib = _lib.load()
+    plan = _lib.GatherParts()
+    _lib.check(lib.lffn_lookup_gather_parts_plan(B, T, S, Do, fmt, 1, ctypes.byref(plan)), "parts plan")
+    if plan.parts:
+        return f"record stream (four lanes per token), {plan.tokens_per_workgroup} tokens and 1/{plan.parts} of the tables per workgroup"
     tok, stride, nbytes = ctypes.c_int32(0), ctypes.c_int64(0), ctypes.c_int64(0)
     _lib.check(lib.lffn_lookup_gather_records_plan_rows(B, T, S, Do, fmt, ctypes.byref(tok), ctypes.byref(stride),
                                                         ctypes.byref(nbytes)), "records plan")

@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 9
+#define LFFN_ABI_VERSION 10
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -413,6 +413,32 @@ int lffn_lookup_gather_records_rows(const uint32_t *records, int64_t record_stri
                                     const float *bias, const float *residual, float *out, int64_t B, int64_t T,
                                     int64_t S, int64_t Do, int32_t row_format, int32_t tokens_per_workgroup,
                                     void *stream);
+
+/*
+ * The same gather for a few thousand tokens, which have too few (token tile, column slice) pairs to fill the chip:
+ * `parts` workgroups share a pair, each adding its range of the tables into a partial output, and a second kernel
+ * adds the partials in table order with bias and residual (reproducible; equal to the other forms' results up to
+ * the association of the fp32 sums).
+ * lffn_lookup_gather_parts_plan: host-side query; packed != 0: the caller's records are written by a projection
+ * kernel, 0: they are packed from codes and scores.  plan->parts == 0 when another form is the one to use; otherwise
+ * tokens_per_workgroup and record_stride as lffn_lookup_gather_records_plan's and bytes, the scratch the call wants:
+ * the records (6 * T * record_stride bytes) and behind them the partial outputs.
+ * lffn_lookup_gather_parts_rows: code and score both NULL: the records lie in the workspace, written for the plan's
+ * tokens_per_workgroup and record_stride; otherwise they are packed there first (8-byte aligned, T even).  Any tile
+ * that the format is built for and any number of parts that leaves none empty runs.  workspace: 16-byte aligned
+ * device memory of `bytes`, contents undefined afterwards.  bias and residual may be NULL, residual may be out.
+ * Same replacement as lffn_lookup_gather_f32 (PL/lookup.py:120-130, 108).
+ */
+typedef struct lffn_gather_parts {
+    int32_t tokens_per_workgroup, parts;
+    int64_t record_stride, bytes;
+} lffn_gather_parts;
+int lffn_lookup_gather_parts_plan(int64_t B, int64_t T, int64_t S, int64_t Do, int32_t row_format, int32_t packed,
+                                  lffn_gather_parts *plan);
+int lffn_lookup_gather_parts_rows(const lffn_gather_parts *plan, const int32_t *code, const float *score,
+                                  const void *tables, const float *bias, const float *residual, float *out, void *workspace,
+                                  int64_t workspace_bytes, int64_t B, int64_t T, int64_t S, int64_t Do, int32_t row_format,
+                                  void *stream);
 
 /* ---------------------------------------------------------------- code + score */
 

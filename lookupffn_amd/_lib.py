@@ -16,7 +16,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # LOOKUPFFN_HIP_LIB points at another build of the same ABI (e.g. a tuning build)
 LIB_PATH = os.environ.get("LOOKUPFFN_HIP_LIB") or os.path.join(_PKG_DIR, "liblookupffn_hip.so")
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 LFFN_OK = 0
 LFFN_ERR_BAD_ARG = -1
@@ -89,6 +89,8 @@ SIGNATURES = {
     "lffn_lookup_gather_records_f32": [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
     "lffn_lookup_gather_records_plan_rows": [_i64, _i64, _i64, _i64, ctypes.c_int32, ctypes.POINTER(ctypes.c_int32),
                                              ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)],
+    "lffn_lookup_gather_parts_plan": [_i64, _i64, _i64, _i64, ctypes.c_int32, ctypes.c_int32, _vp],
+    "lffn_lookup_gather_parts_rows": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
     "lffn_lookup_gather_records_rows": [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, ctypes.c_int32, ctypes.c_int32, _vp],
     "lffn_lookup_gather_plan": [_i64, _i64, _i64, _i64, ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)],
     "lffn_indexed_inner_product_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
@@ -117,6 +119,11 @@ class FusedLayer(ctypes.Structure):
     _fields_ = [("ln_weight", _vp), ("ln_bias", _vp), ("diag", _vp), ("proj_bias", _vp), ("tables", _vp), ("out_bias", _vp),
                 ("H", _i64), ("D", _i64), ("R", _i64), ("J", _i64), ("T", _i64), ("S", _i64), ("Do", _i64),
                 ("ln_eps", _f32), ("decay", _f32), ("residual", _f32)]
+
+
+class GatherParts(ctypes.Structure):
+    """struct lffn_gather_parts of include/lookupffn_hip.h."""
+    _fields_ = [("tokens_per_workgroup", ctypes.c_int32), ("parts", ctypes.c_int32), ("record_stride", _i64), ("bytes", _i64)]
 
 
 class BlockFront(ctypes.Structure):

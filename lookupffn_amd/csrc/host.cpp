@@ -47,6 +47,8 @@ using torch::autograd::variable_list;
     X(lffn_lookup_gather_records_plan_rows) \
     X(lffn_ln_project_hash_records_f32)     \
     X(lffn_lookup_gather_records_rows)      \
+    X(lffn_lookup_gather_parts_plan)        \
+    X(lffn_lookup_gather_parts_rows)        \
     X(lffn_ln_project_hash_f32)             \
     X(lffn_lookup_gather_workspace_bytes)   \
     X(lffn_lookup_gather_ws_f32)            \
@@ -97,6 +99,7 @@ struct RecordPlan {
     std::array<int64_t, 6> sizes{-1};    // B, T, S, Do, row format, records possible
     int64_t stride = 0, bytes = 0, ws_bytes = 0;
     int32_t tokens = 0;
+    lffn_gather_parts parts{};           // parts > 0: the tables shared out over several workgroups
 };
 
 // What the layer holds at this moment: its hash, the hash's projection and its LayerNorm as Python finds them on every access, the
@@ -162,20 +165,26 @@ hipStream_t stream_on(const at::Device &d) { return c10::hip::getCurrentHIPStrea
 Tensor empty_f32(at::IntArrayRef sizes, const at::Device &d) { return at::empty(sizes, at::TensorOptions().dtype(at::kFloat).device(d)); }
 Tensor empty_bytes(int64_t n, const at::Device &d) { return at::empty({n}, at::TensorOptions().dtype(at::kByte).device(d)); }
 
-RecordPlan plan_for(const Config &c, int64_t B) {
+RecordPlan plan_for(const Config &c, int64_t B, bool records) {
     // the last plans by their sizes
     static std::array<RecordPlan, 64> known;
     static std::mutex lock;
     const std::lock_guard<std::mutex> guard(lock);
-    const std::array<int64_t, 6> sizes{B, c.T, c.S, c.Do, c.fmt, c.T % 2 == 0 && (c.form == BLOCK || c.D >= 16)};
+    const std::array<int64_t, 6> sizes{B, c.T, c.S, c.Do, c.fmt, records && c.T % 2 == 0 && (c.form == BLOCK || c.D >= 16)};
     size_t slot = 0;
     for (int64_t n : sizes) slot = slot * 31 + (size_t)n;
     RecordPlan &p = known[(slot ^ slot >> 12) % known.size()];
     if (p.sizes != sizes) {
         RecordPlan made;
-        if (sizes[5])
+        CALL(lffn_lookup_gather_parts_plan, B, c.T, c.S, c.Do, (int32_t)c.fmt, (int32_t)sizes[5], &made.parts);
+        if (made.parts.parts) {
+            made.tokens = made.parts.tokens_per_workgroup;
+            made.stride = made.parts.record_stride;
+            made.ws_bytes = made.parts.bytes;
+            if (sizes[5]) made.bytes = made.parts.bytes;
+        } else if (sizes[5])
             CALL(lffn_lookup_gather_records_plan_rows, B, c.T, c.S, c.Do, (int32_t)c.fmt, &made.tokens, &made.stride, &made.bytes);
-        if (made.bytes == 0) CALL(lffn_lookup_gather_workspace_bytes, B, c.T, c.S, c.Do, (int32_t)c.fmt, &made.ws_bytes);
+        if (made.bytes == 0 && made.ws_bytes == 0) CALL(lffn_lookup_gather_workspace_bytes, B, c.T, c.S, c.Do, (int32_t)c.fmt, &made.ws_bytes);
         made.sizes = sizes;
         p = made;
     }
@@ -184,11 +193,17 @@ RecordPlan plan_for(const Config &c, int64_t B) {
 
 // Codes and scores [B, T] -> the gather, by whichever form the shape gets.
 void gather(const Config &c, const Tensor &codes, const Tensor &scores, const Tensor &tables, const Tensor &obias, const float *residual,
-            Tensor &out, int64_t B, int64_t ws_bytes, void *st) {
+            Tensor &out, int64_t B, const RecordPlan &plan, void *st) {
+    const int64_t ws_bytes = plan.ws_bytes;
     Tensor ws;
     if (ws_bytes > 0) ws = empty_bytes(ws_bytes, out.device());
     void *wp = ws_bytes > 0 ? ws.data_ptr() : nullptr;
     const int32_t *cp = static_cast<const int32_t *>(codes.data_ptr());
+    if (plan.parts.parts) {
+        CALL(lffn_lookup_gather_parts_rows, &plan.parts, cp, f32(scores), tables.data_ptr(), f32(obias), residual, f32(out), wp, ws_bytes,
+             B, c.T, c.S, c.Do, (int32_t)c.fmt, st);
+        return;
+    }
     if (c.fmt == 0)
         CALL(lffn_lookup_gather_ws_f32, cp, f32(scores), f32(tables), f32(obias), residual, f32(out), wp, ws_bytes, B, c.T, c.S, c.Do, st);
     else if (c.fmt == 1)
@@ -236,9 +251,9 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
         return;
     }
     const float eps = (float)c.eps, decay = (float)c.decay, res = (float)c.residual;
-    const RecordPlan plan = plan_for(c, B);
+    const RecordPlan plan = plan_for(c, B, true);
     if (plan.bytes > 0) {
-        // many tokens: the projection kernel writes the gather kernel's record stream directly
+        // some thousand tokens and more: the projection kernel writes the gather kernel's record stream directly
         Tensor records = empty_bytes(plan.bytes, dev);
         uint32_t *rp = static_cast<uint32_t *>(records.data_ptr());
         if (c.form == DIAG)
@@ -251,7 +266,11 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
             front.tokens_per_workgroup = plan.tokens;
             CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
         }
-        CALL(lffn_lookup_gather_records_rows, rp, plan.stride, p[4].data_ptr(), f32(p[5]), residual, f32(out), B, c.T, c.S, c.Do,
+        if (plan.parts.parts)
+            CALL(lffn_lookup_gather_parts_rows, &plan.parts, nullptr, nullptr, p[4].data_ptr(), f32(p[5]), residual, f32(out), rp, plan.bytes,
+                 B, c.T, c.S, c.Do, (int32_t)c.fmt, st);
+        else
+            CALL(lffn_lookup_gather_records_rows, rp, plan.stride, p[4].data_ptr(), f32(p[5]), residual, f32(out), B, c.T, c.S, c.Do,
              (int32_t)c.fmt, plan.tokens, st);
         return;
     }
@@ -266,7 +285,7 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
         front.scores = f32(scores);
         CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
     }
-    gather(c, codes, scores, p[4], p[5], residual, out, B, plan.ws_bytes, st);
+    gather(c, codes, scores, p[4], p[5], residual, out, B, plan, st);
 }
 
 // Column sums of one or two [P, n] arrays of partial sums, fixed order of additions; many rows go through a first
@@ -432,9 +451,7 @@ void train(const Config &c, const Params &p, const Tensor &x, const Tensor &resi
         CALL(lffn_ln_bh4_block_hash_train_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), f32(z),
              c.J > 1 ? f32(stage) : nullptr, f32(stats), B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
     }
-    int64_t ws_bytes = 0;
-    CALL(lffn_lookup_gather_workspace_bytes, B, c.T, c.S, c.Do, (int32_t)c.fmt, &ws_bytes);
-    gather(c, codes, scores, p[4], p[5], f32(residual), out, B, ws_bytes, st);
+    gather(c, codes, scores, p[4], p[5], f32(residual), out, B, plan_for(c, B, false), st);
 
     node->c = c;
     node->B = B;

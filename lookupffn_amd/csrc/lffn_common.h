@@ -157,7 +157,22 @@ int64_t lffn_internal_quad_record_stride(int64_t B, int fmt, int64_t tokens);
 __attribute__((visibility("hidden")))
 int lffn_internal_lookup_gather_quad_records(const uint32_t *records, int64_t record_stride, const void *tables,
                                              const float *bias, const float *residual, float *out, int64_t B,
-                                             int64_t T, int64_t S, int64_t Do, int fmt, int tokens, void *stream);
+                                             int64_t T, int64_t S, int64_t Do, int fmt, int tokens, int parts, void *stream);
+__attribute__((visibility("hidden")))
+int lffn_internal_quad_pack(const int32_t *code, const float *score, uint32_t *records, int64_t stride, int64_t B, int64_t T,
+                            int64_t S, int tokens, void *stream);
+// How many table pairs ahead the tiles of a slice touch its blocks by turns; 0: not at all.  The fewer tiles share a block, the more
+// different blocks an XCD's workgroups read at a time, 1 MB of its 4 MB of L2 per pair with two tiles, and what is touched
+// too early is gone again.  us with tables in / beyond the memory-side cache, no touch | 2 ahead | 3 ahead:
+//   1 tile   1000 x 128 x 768 in 8 parts  29, 39 | 37, 45 | 39, 47
+//   2 tiles  2103 x 128 x 768 in 5        37, 53 | 39, 51 | 43, 52
+//   3 tiles  6000 x 128 x 768 in 3        60, 87 | 63, 78 | 65, 79
+//   4 tiles  4096 x 128 x 512 in 4        37, 56 | 36, 47 | 36, 45
+//   5 tiles  6000 x 128 x 768 in 2        65, 100 | 59, 79 | 59, 75
+//  10 tiles 16384 x 128 x 768 in 1       111, 171 | 103, 130 | 102, 113
+static inline int lffn_quad_touch_ahead(int64_t tiles) { return tiles < 2 ? 0 : tiles < 4 ? 2 : 3; }
+// table pairs per part when `parts` workgroups share a tile and slice; the last part may get fewer
+static inline int64_t lffn_quad_part_pairs(int64_t T, int64_t parts) { return parts > 0 ? (T / 2 + parts - 1) / parts : 0; }
 
 // The record stream of the four-lanes-per-token gather (lookup_gather_quad.hip), as its writers address it.
 // A record is three words: score of the pair's first table, score of its second, row of the first | row of
@@ -301,6 +316,7 @@ constexpr int TOUCH_SINK_BYTES = 256;
 // s_waitcnt immediates (vmcnt in bits 3:0, the other counters left alone)
 constexpr int WAIT_VMCNT_0 = 0x0F70;
 constexpr int WAIT_VMCNT_1 = 0x0F71;
+constexpr int WAIT_VMCNT_2 = 0x0F72;
 __device__ __forceinline__ void l2_touch(const char *base, uint32_t lane_offset, uint32_t lds_byte_addr) {
     // M0 is put back: the compiler reserves it for its own use and does not honour a clobber
     // declaration of it, so the statement must leave it as it found it

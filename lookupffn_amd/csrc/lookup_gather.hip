@@ -563,6 +563,132 @@ GatherPlan choose_quad(int64_t B, int64_t T, int64_t S, int64_t Do, bool pack = 
     return qp.us < QUAD_MARGIN * other ? qp : none;
 }
 
+// The four-lanes-per-token kernel with the table pairs of a (tile, slice) shared out over `parts` workgroups, one round
+// of at most 256 of them: what fills the chip where the tokens alone do not.  Microseconds, fitted to 600 measurements
+// of 75 random shapes (300 .. 12288 tokens, 8 .. 512 tables, 128 .. 1024 columns) in turn on the tables of twelve layers, as a
+// model uses them (off by 7, 6 and 6 % root mean square for the three row formats), all of them with the records there:
+//   * a start and end of the launch;
+//   * per pair of tables the largest of: the copy to LDS (`pair_min`); the adds (`pair` and `pass`, as above); and the
+//     fetch of the blocks that the workgroups read at that moment (one per slice and part, 64 KB each) into the L2s, where
+//     they are touched ahead (lffn_quad_touch_ahead) and where they are not: a latency and a rate;
+//   * the partial sums, written and read once, and the second launch.
+struct PartsPlan {
+    int tile = 0, parts = 0;
+    double us = 1e300;
+};
+struct PartsCost {
+    double start, pair_min, pair, pass, fetch, fetch_block, touched, touched_block, reduce, reduce_mb;
+};
+constexpr PartsCost PARTS_COST[3] = {{3.3, 1.35, 0.78, 0.158, 1.70, 0.0066, 1.18, 0.0064, 3.9, 0.155},
+                                     {4.6, 0.97, 0.74, 0.323, 2.00, 0.0043, 0.79, 0.0060, 5.0, 0.136},
+                                     {8.9, 1.45, 0.75, 0.213, 1.87, 0.0059, 0.80, 0.0031, 0.0, 0.137}};
+constexpr double PARTS_BIG_BYTES = 240e6;                // tables beyond the memory-side cache by themselves
+constexpr double PARTS_BIG_FETCH = 1.74, PARTS_BIG_FETCH_BLOCK = 0.0062, PARTS_BIG_TOUCHED = 0.87, PARTS_BIG_TOUCHED_BLOCK = 0.015;
+constexpr int MAX_PARTS = 32;
+constexpr double PARTS_MARGIN = 1.0;                     // the other plans' times are those of tables in the memory-side cache
+// What plan_quad's time leaves out: the start and end of its launch (16384 x 128 x 768: 101 us promised, 108 measured)
+constexpr double QUAD_START_US = 8.0;
+
+PartsPlan plan_parts(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, bool pack) {
+    PartsPlan best;
+    const int esz = fmt == LFFN_ROWS_F32 ? 4 : 2;
+    const int64_t nslices = Do * esz / 128;
+    const int64_t max_tile = fmt == LFFN_ROWS_F32 ? 2048 : 1024;
+    if (S != MAX_S || T < 4 || T % 2 != 0 || Do * esz % 128 != 0 || B > 256 * max_tile || 2 * nslices > 256 ||
+        2 * S * Do * esz >= (int64_t(1) << 32))
+        return best;
+    const PartsCost &c = PARTS_COST[fmt];
+    const bool big = double(T) * double(S) * double(Do) * esz > PARTS_BIG_BYTES;
+    const double out_mb = double(B) * double(Do) * 4e-6;
+    const double pack_us = pack ? 4.2 + double(B) * double(T) * 14.0 / 9e6 : 0.0;
+    for (int64_t tiles = (B + max_tile - 1) / max_tile; 2 * tiles * nslices <= 256; ++tiles) {
+        int64_t tile = ((B + tiles - 1) / tiles + 15) & ~int64_t(15);
+        if (tile <= 768) tile = 784;                     // four passes are the fewest that are built
+        if ((tiles - 1) * tile >= B) break;              // more tiles than the tokens fill
+        const int64_t np = (tile + 255) / 256;
+        const double passes = double(np - 1) + double(tile - 256 * (np - 1)) / 256.0;
+        const double adds = c.pair + c.pass * passes;
+        for (int64_t parts = 2; parts <= MAX_PARTS && tiles * nslices * parts <= 256; ++parts) {
+            const int64_t pairs = lffn_quad_part_pairs(T, parts);
+            if ((parts - 1) * pairs >= T / 2) continue;  // the last part would be empty
+            const double blocks = double(nslices * parts);
+            double pair_us = lffn_quad_touch_ahead(tiles) < 3
+                                 ? (big ? PARTS_BIG_FETCH + PARTS_BIG_FETCH_BLOCK * blocks : c.fetch + c.fetch_block * blocks)
+                                 : (big ? PARTS_BIG_TOUCHED + PARTS_BIG_TOUCHED_BLOCK * blocks : c.touched + c.touched_block * blocks);
+            if (pair_us < adds) pair_us = adds;
+            if (pair_us < c.pair_min) pair_us = c.pair_min;
+            const double us = pack_us + c.start + double(pairs) * pair_us + c.reduce + c.reduce_mb * double(2 * parts + 1) * out_mb;
+            if (us < best.us) { best.tile = (int)tile; best.parts = (int)parts; best.us = us; }
+        }
+    }
+    return best;
+}
+
+// plan_parts if it promises to beat the other forms, parts = 0 otherwise.  Layer gather from records, tables of twelve layers in
+// turn | of one layer again and again, us, other form -> this one: fp32 2674 x 128 x 768 65 -> 56 | 54 -> 42, 3763 x 128 x 512 56 -> 46 | 49 -> 35,
+// 6000 x 128 x 768 103 -> 75 | 88 -> 59, 8954 x 256 x 384 160 -> 85 | 143 -> 73, 8621 x 512 x 512 325 -> 177; bfloat16 1800 x 128 x 1024
+// 54 -> 45 | 55 -> 41; half 3022 x 256 x 768 126 -> 68 | 126 -> 58, 8000 x 128 x 1024 242 -> 86.  Left where they are: fp32 2103 x 128 x 768
+// 57 -> 52 | 48 -> 39 (no faster in the layer, whose tables are half in the cache), 1024 x 128 x 1024 48 -> 47, 2136 x 64 x 768 33 -> 35.
+PartsPlan choose_parts(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, bool pack) {
+    const PartsPlan p = plan_parts(fmt, B, T, S, Do, pack);
+    if (p.parts == 0) return p;
+    // What the token-major kernel reads of small tables or short rows comes at 12 or 15 TB/s, not at the 9 that the other plans
+    // count with (half: 12767 x 64 x 256 33 us, 18271 x 32 x 384 33; bfloat16 4720 x 64 x 512 30, 6656 x 128 x 256 33): those
+    // calls stay there.
+    const double row_bytes = double(Do) * (fmt == LFFN_ROWS_F32 ? 4 : 2), table_bytes = double(T) * double(S) * row_bytes;
+    const double rate = row_bytes <= 512.0 || table_bytes <= 10e6 ? 15e6 : (table_bytes <= 20e6 ? 12e6 : 9e6);
+    if (p.us >= PARTS_MARGIN * (double(B) * double(T) * row_bytes / rate + 5.0)) return PartsPlan{};
+    double other;
+    if (fmt == LFFN_ROWS_F16) {
+        const GatherPlan qp = plan_quad(fmt, B, T, S, Do, pack);
+        other = double(B) * double(T) * double(Do) * 2 / 9e6 + 5.0;
+        if (qp.kind == 3 && qp.us < QUAD_MARGIN * other) other = qp.us + QUAD_START_US;
+    } else {
+        const bool bf16 = fmt == LFFN_ROWS_BF16;
+        const GatherPlan qp = bf16 ? choose_quad<true>(B, T, S, Do, pack) : choose_quad<false>(B, T, S, Do, pack);
+        if (qp.kind == 3) {
+            other = qp.us + QUAD_START_US;
+        } else {
+            const int64_t each = bf16 ? gather_pieces<true>(B, T, S, Do) : gather_pieces<false>(B, T, S, Do);
+            other = bf16 ? plan_gather<true>(each < B ? each : B, T, S, Do).us : plan_gather<false>(each < B ? each : B, T, S, Do).us;
+            if (each < B) {
+                other = double((B + each - 1) / each) * (other + 4.0);
+            } else {
+                const SplitPlan sp = bf16 ? plan_split<true>(B, T, S, Do) : plan_split<false>(B, T, S, Do);
+                // (plan_split counts 4 TB/s for the partial sums; they come at 6, and 2 us less for the launch)
+                if (sp.nparts > 1 && sp.us < 0.85 * other) other = sp.us - double(2 * sp.nparts + 1) * double(B) * double(Do) * 4.0 / 12e6 - 2.0;
+            }
+        }
+    }
+    return p.us < PARTS_MARGIN * other ? p : PartsPlan{};
+}
+
+// the records, then one [B, Do] of partial sums per part
+int64_t parts_bytes(const lffn_gather_parts &p, int64_t B, int64_t T, int64_t Do) {
+    return (T / 2) * LFFN_RECORD_WORDS * 4 * p.record_stride + (p.parts > 1 ? p.parts * B * Do * 4 : 0);
+}
+
+int gather_parts(const lffn_gather_parts &p, const int32_t *code, const float *score, const void *tables, const float *bias,
+                 const float *residual, float *out, void *workspace, int64_t B, int64_t T, int64_t S, int64_t Do, int fmt,
+                 void *stream) {
+    uint32_t *records = static_cast<uint32_t *>(workspace);
+    if (code) {
+        const int rc = lffn_internal_quad_pack(code, score, records, p.record_stride, B, T, S, p.tokens_per_workgroup, stream);
+        if (rc != LFFN_OK) return rc;
+    }
+    if (p.parts == 1)
+        return lffn_internal_lookup_gather_quad_records(records, p.record_stride, tables, bias, residual, out, B, T, S, Do, fmt,
+                                                        p.tokens_per_workgroup, 1, stream);
+    float *partials = reinterpret_cast<float *>(records + (T / 2) * LFFN_RECORD_WORDS * p.record_stride);
+    const int rc = lffn_internal_lookup_gather_quad_records(records, p.record_stride, tables, nullptr, nullptr, partials, B, T, S,
+                                                            Do, fmt, p.tokens_per_workgroup, p.parts, stream);
+    if (rc != LFFN_OK) return rc;
+    const int64_t blocks = (B * Do / 4 + 255) / 256;
+    hipLaunchKernelGGL(gather_parts_reduce_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), partials, p.parts, bias, residual, out, B, (int)Do, lffn_table_guard());
+    return lffn_launch_status();
+}
+
 // four lanes per token: a tile (tokens per workgroup: whole groups of 16, its last pass not empty) whose number
 // of passes is built for the row format, 256-row tables, an even number of them, whole 128-byte slices, 32-bit
 // offsets inside a table pair
@@ -951,7 +1077,7 @@ extern "C" int lffn_lookup_gather_records_rows(const uint32_t *records, int64_t 
                  LFFN_ERR_BAD_ARG);
     if (B == 0) return LFFN_OK;
     return lffn_internal_lookup_gather_quad_records(records, record_stride, tables, bias, residual, out, B, T, S, Do,
-                                                    row_format, tokens_per_workgroup, stream);
+                                                    row_format, tokens_per_workgroup, 1, stream);
 }
 
 extern "C" int lffn_lookup_gather_records_f32(const uint32_t *records, int64_t record_stride, const float *tables,
@@ -961,6 +1087,41 @@ extern "C" int lffn_lookup_gather_records_f32(const uint32_t *records, int64_t r
                                            tokens_per_workgroup, stream);
 }
 
+extern "C" int lffn_lookup_gather_parts_plan(int64_t B, int64_t T, int64_t S, int64_t Do, int32_t row_format, int32_t packed,
+                                             lffn_gather_parts *plan) {
+    LFFN_REQUIRE(plan && row_format >= 0 && row_format <= 2, LFFN_ERR_BAD_ARG);
+    *plan = lffn_gather_parts{};
+    if (B < 1 || T < 1 || Do < 1 || !lffn_is_pow2(S) || Do % 64 != 0 || B * T >= (int64_t(1) << 31)) return LFFN_OK;
+    const PartsPlan p = choose_parts(row_format, B, T, S, Do, packed == 0);
+    if (p.parts == 0) return LFFN_OK;
+    plan->tokens_per_workgroup = p.tile;
+    plan->parts = p.parts;
+    plan->record_stride = lffn_internal_quad_record_stride(B, row_format, p.tile);
+    plan->bytes = parts_bytes(*plan, B, T, Do);
+    return LFFN_OK;
+}
+
+extern "C" int lffn_lookup_gather_parts_rows(const lffn_gather_parts *plan, const int32_t *code, const float *score,
+                                             const void *tables, const float *bias, const float *residual, float *out,
+                                             void *workspace, int64_t workspace_bytes, int64_t B, int64_t T, int64_t S,
+                                             int64_t Do, int32_t row_format, void *stream) {
+    LFFN_REQUIRE(plan && B >= 0 && T >= 0 && Do >= 1 && row_format >= 0 && row_format <= 2, LFFN_ERR_BAD_ARG);
+    const int tokens = plan->tokens_per_workgroup, parts = plan->parts;
+    LFFN_REQUIRE(tokens > 0 && tokens % 16 == 0 && parts >= 1 && !code == !score, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_is_pow2(S) && Do % 64 == 0 && quad_plan_is_valid(row_format, tokens, B, T, S, Do) && parts <= T / 2 &&
+                     (parts - 1) * lffn_quad_part_pairs(T, parts) < T / 2,
+                 LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(plan->record_stride % 4 == 0 && plan->record_stride <= (int64_t(1) << 31) &&
+                     lffn_record_layout_ok(B, plan->record_stride, tokens),
+                 LFFN_ERR_BAD_ARG);
+    if (B == 0) return LFFN_OK;
+    LFFN_REQUIRE(tables && out && workspace && workspace_bytes >= parts_bytes(*plan, B, T, Do), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(tables) && lffn_aligned16(out) && lffn_aligned16(workspace) && (!bias || lffn_aligned16(bias)) &&
+                     (!residual || lffn_aligned16(residual)) && (uintptr_t)code % 8 == 0 && (uintptr_t)score % 8 == 0,
+                 LFFN_ERR_BAD_ARG);
+    return gather_parts(*plan, code, score, tables, bias, residual, out, workspace, B, T, S, Do, row_format, stream);
+}
+
 namespace {
 
 constexpr int64_t FLAG_BYTES = TABLE_FLAGS * 4;
@@ -968,6 +1129,8 @@ constexpr int64_t FLAG_BYTES = TABLE_FLAGS * 4;
 // Microseconds the table-major forms are predicted to take for 256-row tables with a workspace; 1e300 where the
 // token-major kernel would run.
 double table_major_us(int fmt, int64_t B, int64_t T, int64_t Do) {
+    const PartsPlan pp = choose_parts(fmt, B, T, MAX_S, Do, true);
+    if (pp.parts) return pp.us;
     if (fmt == LFFN_ROWS_F16) {
         const GatherPlan qp = plan_quad(fmt, B, T, MAX_S, Do);
         return qp.kind == 3 ? qp.us : 1e300;
@@ -998,7 +1161,11 @@ extern "C" int lffn_gather_add_workspace_bytes(int64_t B, int64_t I, int64_t sou
     LFFN_REQUIRE(bytes && row_format >= 0 && row_format <= 2, LFFN_ERR_BAD_ARG);
     *bytes = 0;
     if (!try_tables(row_format, B, I, source_size, Dv)) return LFFN_OK;
-    const int rc = lffn_lookup_gather_workspace_bytes(B, I, MAX_S, Dv, row_format, bytes);
+    int rc = lffn_lookup_gather_workspace_bytes(B, I, MAX_S, Dv, row_format, bytes);      // (row numbers that cannot be packed)
+    if (rc != LFFN_OK) return rc;
+    lffn_gather_parts plan;
+    rc = lffn_lookup_gather_parts_plan(B, I, MAX_S, Dv, row_format, 0, &plan);
+    if (plan.bytes > *bytes) *bytes = plan.bytes;
     *bytes += FLAG_BYTES;
     return rc;
 }
@@ -1019,7 +1186,11 @@ extern "C" int lffn_gather_add_ws_rows(const int32_t *idx, const void *src, cons
         TableGuardScope scope(flags);
         char *ws = need > FLAG_BYTES ? static_cast<char *>(workspace) + FLAG_BYTES : nullptr;
         const int64_t ws_bytes = need - FLAG_BYTES;
-        if (row_format == LFFN_ROWS_F16)
+        lffn_gather_parts plan;
+        lffn_lookup_gather_parts_plan(B, I, MAX_S, Dv, row_format, 0, &plan);
+        if (plan.parts && (uintptr_t)idx % 8 == 0 && (uintptr_t)w % 8 == 0)
+            rc = lffn_lookup_gather_parts_rows(&plan, idx, w, src, nullptr, nullptr, out, ws, ws_bytes, B, I, MAX_S, Dv, row_format, stream);
+        else if (row_format == LFFN_ROWS_F16)
             rc = lookup_gather_entry_f16(idx, w, src, nullptr, nullptr, out, B, I, MAX_S, Dv, -1, 0, stream, ws, ws_bytes);
         else if (row_format == LFFN_ROWS_BF16)
             rc = lookup_gather_entry<true>(idx, w, src, nullptr, nullptr, out, B, I, MAX_S, Dv, -1, 0, stream, ws, ws_bytes);

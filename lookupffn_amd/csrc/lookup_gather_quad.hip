@@ -43,6 +43,8 @@
 // (bfloat16: a shift or a mask per value), 8 v_fma_mix_f32 (half: the instruction widens its operand).
 #include "lffn_common.h"
 
+#include <climits>
+
 namespace {
 
 constexpr int WG = 1024;
@@ -53,7 +55,6 @@ constexpr int BUF_BYTES = MAX_S * 256;      // one table pair: S rows of 2 x 128
 constexpr int SLICE_BYTES = 128;            // a slice of a row: 32 fp32 columns or 64 16-bit columns
 constexpr int FMT_F32 = LFFN_ROWS_F32, FMT_BF16 = LFFN_ROWS_BF16, FMT_F16 = LFFN_ROWS_F16;
 constexpr int fmt_bytes(int fmt) { return fmt == FMT_F32 ? 4 : 2; }
-constexpr int QUAD_TOUCH_AHEAD = 3;         // pairs between the one being read and the one being touched
 
 // (code, score) of one token and one table pair in the order the token's quad takes the pair's tables
 // (tokens whose index has bit 1 set take table 2k+1 first): three words, word 0 = score of the first
@@ -67,12 +68,14 @@ constexpr int REC_WORDS = LFFN_RECORD_WORDS;
 
 struct QuadArgs {
     const char *tables;    // [T, S, Do] fp32, bfloat16 or half
-    const float *bias;     // [Do] or null
-    const float *residual; // [B, Do] or null: added to the result (may be the output buffer)
-    float *out;            // [B, Do]
+    const float *bias;     // [Do] or null (null with several parts)
+    const float *residual; // [B, Do] or null: added to the result (may be the output buffer; null with several parts)
+    float *out;            // [parts, B, Do]
     int64_t B;
     int T, S, Do;          // T even, S = 256
     int ntiles, nslices, per_xcd;
+    int touch_ahead;       // pairs between the one being read and the one being touched; 0: none is touched
+    int parts, part_pairs; // part p adds the table pairs [p * part_pairs, min((p + 1) * part_pairs, T / 2)): one at least
     int tile_tokens;       // tokens per tile: a multiple of 16 in ((NP - 1) * 256, NP * 256]
     int row_bytes;         // Do * bytes per element
     const uint32_t *stream;     // [T/2][Bpad][3] record words written by pack_pairs_kernel
@@ -126,22 +129,23 @@ __device__ __forceinline__ unsigned with_row(unsigned base, unsigned packed) {
 }
 
 // Packs the caller's [B, T] codes and scores into the record stream [T/2][Bpad][3].  A workgroup takes 64
-// tokens x 32 table pairs: it reads them pair-fastest (a token's 32 pairs are 256 contiguous bytes),
+// tokens x 16 table pairs: it reads them pair-fastest (a token's 16 pairs are 128 contiguous bytes),
 // turns them round in LDS and writes them token-fastest (16 consecutive tokens' records of a pair are 192
 // contiguous bytes).  Slots of tokens from B on are left as they are: the gather reads them (their row
 // numbers are bytes, always inside the LDS buffer) and does not store their sums.
+constexpr int PACK_PAIRS = 16;
 __global__ __launch_bounds__(256) void pack_pairs_kernel(const int32_t *code, const float *score, uint32_t *stream,
                                                          int64_t B, int64_t Bpad, int T, int S, int tile_tokens,
                                                          TableGuard guard) {
     if (table_guard_ends(guard)) return;
-    __shared__ PairRecord tile[32][64 + 1];
+    __shared__ PairRecord tile[PACK_PAIRS][64 + 1];
     const int npairs = T / 2;
     const int64_t tok0 = int64_t(blockIdx.x) * 64;
-    const int k0 = blockIdx.y * 32;
+    const int k0 = blockIdx.y * PACK_PAIRS;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < PACK_PAIRS / 4; ++i) {
         const int item = threadIdx.x + 256 * i;
-        const int kk = item & 31, row = item >> 5;
+        const int kk = item % PACK_PAIRS, row = item / PACK_PAIRS;
         const int64_t b = tok0 + row;
         PairRecord r{0.f, 0.f, 0u};
         if (b < B && k0 + kk < npairs) {
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(256) void pack_pairs_kernel(const int32_t *code, co
     const int row = threadIdx.x & 63;
     const int64_t slot = tok0 + row < B ? lffn_quad_record_slot(tok0 + row, tile_tokens) : 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < PACK_PAIRS / 4; ++i) {
         const int kk = (threadIdx.x >> 6) + 4 * i;
         if (tok0 + row < B && k0 + kk < npairs) {
             uint32_t *dst = stream + (int64_t(k0 + kk) * Bpad + slot) * REC_WORDS;
@@ -208,10 +212,13 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
 
     const int xcd = blockIdx.x % XCDS;
     const int unit = xcd * a.per_xcd + blockIdx.x / XCDS;
-    if (unit >= a.ntiles * a.nslices) return;     // uniform over the workgroup
+    if (unit >= a.ntiles * a.nslices * a.parts) return;     // uniform over the workgroup
     if (table_guard_ends(a.guard)) return;
-    const int slice = unit / a.ntiles;
+    // the tiles of a (slice, part) are neighbours on one XCD: they read the same blocks of the tables in step
     const int tile = unit % a.ntiles;
+    const int slice = unit / a.ntiles / a.parts;
+    const int part = unit / a.ntiles % a.parts;
+    const int first_pair = part * a.part_pairs;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -262,10 +269,10 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
     // 2k+1; rows are Do*4 bytes apart, the second table S rows further down.  The four vectors of a lane
     // are 64 rows apart: one lane offset, four uniform bases.
     const size_t table_bytes = (size_t)a.S * a.row_bytes;
-    const char *slice_base = a.tables + (size_t)slice * SLICE_BYTES;
     const size_t pair_stride = 2 * table_bytes;
+    const char *slice_base = a.tables + (size_t)slice * SLICE_BYTES + (size_t)first_pair * pair_stride;
     const size_t quarter = (size_t)(WG / 16) * a.row_bytes;
-    const int npairs = a.T / 2;
+    const int npairs = min(a.part_pairs, a.T / 2 - first_pair);
     const uint32_t copy_off = ((tid & 15) < 8 ? 0u : (uint32_t)table_bytes) + (uint32_t)(tid >> 4) * (uint32_t)a.row_bytes +
                               (uint32_t)(tid & 7) * 16u;
     const uint32_t copy_dst = (uint32_t)wave * (64 * 16);       // LDS byte offset of this wavefront's first vector in a buffer
@@ -281,14 +288,14 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
     // every step (as the team touch of lookup_gather.hip does) stalls its own copies once per step.  Here
     // the workgroups that share the slice (one per token tile, all on this XCD, in step with each other)
     // take turns instead: in step k the workgroup whose tile number is k mod ntiles touches ALL 2*S lines
-    // of pair k + QUAD_TOUCH_AHEAD (lanes 0..2S-1 one 128-byte line each), the others touch nothing
+    // of pair k + touch_ahead (lanes 0..2S-1 one 128-byte line each), the others touch nothing
     // (their instruction reads a line of the pair they are on: a hit).  Every CU then takes the latency
     // once in ntiles steps.
     const int my_line = tid < 2 * a.S ? tid : 0;
     const bool line_second = my_line >= a.S;
     const uint32_t touch_off_on = (line_second ? (uint32_t)table_bytes : 0u) +
                                   (uint32_t)(my_line - (line_second ? a.S : 0)) * (uint32_t)a.row_bytes;
-    int turn = 0;                                   // k mod ntiles, kept without a division
+    int turn = a.touch_ahead ? 0 : INT_MIN / 2;     // k mod ntiles, kept without a division; never a tile's
     const uint32_t touch_dst = lds0 + 2u * BUF_BYTES;
 
     // This wavefront's records of a table pair: 16 per pass, record r = pass r/16, quad r%16, 12 bytes each,
@@ -296,8 +303,9 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
     // LDS.  12 NPW lanes copy 16 bytes each: one instruction up to five passes, two beyond.
     const uint32_t rec_lds = lds0 + 2u * BUF_BYTES + TOUCH_SINK_BYTES + (uint32_t)wave * (WAVE_RECS * REC_WORDS * 4);
     const int wave_slot = 16 * ((NP - 1) * wave + min(wave, n_last));
-    const char *rec_base = reinterpret_cast<const char *>(a.stream + (int64_t(tile) * a.tile_tokens + wave_slot) * REC_WORDS);
     const size_t pair_rec_bytes = (size_t)a.Bpad * (REC_WORDS * 4);
+    const char *rec_base = reinterpret_cast<const char *>(a.stream + (int64_t(tile) * a.tile_tokens + wave_slot) * REC_WORDS) +
+                           (size_t)first_pair * pair_rec_bytes;
     auto copy_records_to_lds = [&](int k, auto npw_c) {
         constexpr int NV = 12 * decltype(npw_c)::value;         // 16-byte vectors
         const char *src = rec_base + (size_t)k * pair_rec_bytes;
@@ -376,7 +384,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
         copy_pair_to_lds(slice_base + (size_t)kn * pair_stride, lds0 + (uint32_t)((k + 1) & 1) * BUF_BYTES);
         if constexpr (TOUCH) {
             const bool mine = turn == tile;                              // uniform
-            const int kt = mine ? min(k + QUAD_TOUCH_AHEAD, npairs - 1) : k;
+            const int kt = mine ? min(k + a.touch_ahead, npairs - 1) : k;
             l2_touch(slice_base + (size_t)kt * pair_stride, mine ? touch_off_on : 0u, touch_dst);
             turn = turn + 1 == a.ntiles ? 0 : turn + 1;
         }
@@ -422,6 +430,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
     else run_pairs(std::integral_constant<int, NP - 1>{});
     __builtin_amdgcn_s_waitcnt(WAIT_VMCNT_0);         // nothing may still be writing this workgroup's LDS when it ends
 
+    float *out = a.out + (size_t)part * a.B * a.Do;
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         const int64_t tok = tok0 + p * 256;
@@ -436,7 +445,7 @@ __global__ __launch_bounds__(WG) void lookup_gather_quad_kernel(QuadArgs a) {
                         const float4 rr = *reinterpret_cast<const float4 *>(a.residual + off);
                         v.x += rr.x; v.y += rr.y; v.z += rr.z; v.w += rr.w;
                     }
-                    *reinterpret_cast<float4 *>(a.out + off) = v;
+                    *reinterpret_cast<float4 *>(out + off) = v;
                 }
         }
     }
@@ -446,7 +455,8 @@ template <int FMT, int NP, bool TOUCH>
 int launch_quad(QuadArgs a, hipStream_t stream) {
     a.guard = lffn_table_guard();
     a.ntiles = (int)((a.B + a.tile_tokens - 1) / a.tile_tokens);
-    const int units = a.ntiles * a.nslices;
+    a.touch_ahead = lffn_quad_touch_ahead(a.ntiles);
+    const int units = a.ntiles * a.nslices * a.parts;
     a.per_xcd = (units + XCDS - 1) / XCDS;
     // two buffers, the touches' scratch, every wavefront's records of one table pair
     const size_t lds_bytes = size_t(2) * BUF_BYTES + TOUCH_SINK_BYTES + size_t(NWAVES) * 16 * NP * REC_WORDS * 4;
@@ -491,18 +501,23 @@ int64_t lffn_internal_quad_record_stride(int64_t B, int fmt, int64_t tokens) {
 }
 
 // Run the gather from a record stream [T/2][record_stride][3] (pack_pairs_kernel's layout; the projection
-// kernels of fht.hip and bh4_block.hip write the same) with `tokens` tokens per workgroup, the tile size
+// kernels of fht.hip, bh4_block.hip and bh4_split.hip write the same) with `tokens` tokens per workgroup, the tile size
 // the stream was written for.  The caller has checked that the
 // shape qualifies: S = 256 (a table pair fills an LDS buffer), T even, Do a multiple of the slice's columns
 // (32 for fp32 rows, 64 for 16-bit rows), 2*S*Do*element bytes < 2^32 (32-bit lane offsets from a table
 // pair's base), a tile size the format is built for.  record_stride: at least
 // lffn_internal_quad_record_stride(B, fmt, tokens); what the records of tokens from B on hold does not matter
 // (their row numbers are bytes, always inside the LDS buffer, and their sums are not stored).
+// parts > 1: the table pairs are shared out over that many workgroups per (tile, slice), part p's sums without bias
+// and residual (both null) go to out + p * B * Do; every part has to get a pair.
 int lffn_internal_lookup_gather_quad_records(const uint32_t *records, int64_t record_stride, const void *tables,
                                              const float *bias, const float *residual, float *out, int64_t B,
-                                             int64_t T, int64_t S, int64_t Do, int fmt, int tokens, void *stream) {
+                                             int64_t T, int64_t S, int64_t Do, int fmt, int tokens, int parts, void *stream) {
     const int np = lffn_internal_quad_passes(fmt, tokens);
     if (!records || S != MAX_S || T % 2 != 0 || np == 0 || tokens <= 256 * (np - 1)) return LFFN_ERR_BAD_ARG;
+    const int64_t part_pairs = lffn_quad_part_pairs(T, parts);
+    if (parts < 1 || (parts > 1 && (bias || residual)) || (parts - 1) * part_pairs >= T / 2) return LFFN_ERR_BAD_ARG;
+    if ((B + tokens - 1) / tokens * (Do * fmt_bytes(fmt) / SLICE_BYTES) * parts > (int64_t(1) << 30)) return LFFN_ERR_UNSUPPORTED;
     // 16-byte copies: the stream and every table pair's part of it on 16-byte boundaries
     if (record_stride < lffn_internal_quad_record_stride(B, fmt, tokens) || record_stride % 4 != 0 ||
         !lffn_aligned16(records))
@@ -515,6 +530,7 @@ int lffn_internal_lookup_gather_quad_records(const uint32_t *records, int64_t re
     a.nslices = (int)(Do * esz / SLICE_BYTES);
     a.row_bytes = (int)(Do * esz);
     a.tile_tokens = tokens;
+    a.parts = parts; a.part_pairs = (int)part_pairs;
     a.Bpad = record_stride;
     a.stream = records;
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -531,6 +547,16 @@ int lffn_internal_lookup_gather_quad_records(const uint32_t *records, int64_t re
     }
 }
 
+// Pack the (code, score) pairs into a record stream [T/2][stride][3] for tiles of `tokens` tokens.  Codes and scores on
+// 8-byte boundaries, T even.
+int lffn_internal_quad_pack(const int32_t *code, const float *score, uint32_t *records, int64_t stride, int64_t B, int64_t T,
+                            int64_t S, int tokens, void *stream) {
+    const dim3 grid((unsigned)((B + 63) / 64), (unsigned)((T / 2 + PACK_PAIRS - 1) / PACK_PAIRS));
+    hipLaunchKernelGGL(pack_pairs_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), code, score, records, B,
+                       stride, (int)T, (int)S, tokens, lffn_table_guard());
+    return lffn_launch_status();
+}
+
 // Pack the (code, score) pairs into the record stream in `workspace` (at least
 // lffn_internal_quad_stream_bytes(B, T) bytes, 16-byte aligned) and run the gather from it.
 int lffn_internal_lookup_gather_quad(const int32_t *code, const float *score, const void *tables,
@@ -540,9 +566,7 @@ int lffn_internal_lookup_gather_quad(const int32_t *code, const float *score, co
     if (B == 0) return LFFN_OK;
     uint32_t *recs = static_cast<uint32_t *>(workspace);
     const int64_t stride = lffn_internal_quad_record_stride(B, fmt, tokens);
-    const dim3 grid((unsigned)((B + 63) / 64), (unsigned)((T / 2 + 31) / 32));
-    hipLaunchKernelGGL(pack_pairs_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), code, score, recs, B,
-                       stride, (int)T, (int)S, tokens, lffn_table_guard());
-    if (hipGetLastError() != hipSuccess) return LFFN_ERR_LAUNCH;
-    return lffn_internal_lookup_gather_quad_records(recs, stride, tables, bias, residual, out, B, T, S, Do, fmt, tokens, stream);
+    const int rc = lffn_internal_quad_pack(code, score, recs, stride, B, T, S, tokens, stream);
+    if (rc != LFFN_OK) return rc;
+    return lffn_internal_lookup_gather_quad_records(recs, stride, tables, bias, residual, out, B, T, S, Do, fmt, tokens, 1, stream);
 }

@@ -857,6 +857,7 @@ def _(indexes, source, weights):
 # The layer in inference at many tokens: the projection kernel writes the gather kernel's record stream itself (no [B, T]
 # codes and scores, no packing kernel).  The records are a private hand-over between the two kernels.
 _RECORDS_PLANS = {}
+_PARTS_PLANS = {}
 
 
 ROWS_F32, ROWS_BF16, ROWS_F16 = 0, 1, 2      # the C ABI's row_format values
@@ -883,6 +884,21 @@ def lookup_gather_records_plan(B, T, S, Do, fmt=ROWS_F32):
     return plan
 
 
+def _gather_parts_plan(B, T, S, Do, fmt):
+    """The plan of the gather whose tables are shared out over several workgroups, from codes and scores, when it is the
+    form to use for this shape and row format, else None.  Host-side query, cached."""
+    key = (B, T, S, Do, fmt)
+    hit = _PARTS_PLANS.get(key, False)
+    if hit is not False:
+        return hit
+    plan = _lib.GatherParts()
+    _lib.check(_lib.load().lffn_lookup_gather_parts_plan(B, T, S, Do, fmt, 0, ctypes.byref(plan)), "lffn_lookup_gather_parts_plan")
+    plan = plan if plan.parts else None
+    if len(_PARTS_PLANS) < 4096:
+        _PARTS_PLANS[key] = plan
+    return plan
+
+
 _L.define("lookup_gather(Tensor code, Tensor score, Tensor tables, Tensor? bias, Tensor? residual=None) -> Tensor")
 
 
@@ -904,6 +920,15 @@ def _lookup_gather_impl(code, score, tables, bias, residual=None):
     fmt = row_format(tables.dtype)
     if fmt is None:
         raise NotImplementedError(f"lookup_gather: table dtype {tables.dtype} (float32, bfloat16 and float16 are built)")
+    plan = _gather_parts_plan(B, T, S, Do, fmt)
+    if plan is not None and code.data_ptr() % 8 == 0 and score.data_ptr() % 8 == 0:
+        ws = torch.empty(plan.bytes, dtype=torch.uint8, device=tables.device)
+        with _dev_guard(tables):
+            rc = lib.lffn_lookup_gather_parts_rows(ctypes.byref(plan), _lib.ptr(code), _lib.ptr(score), _lib.ptr(tables), _lib.ptr(bias),
+                                                   _lib.ptr(residual), _lib.ptr(out), _lib.ptr(ws), plan.bytes, B, T, S, Do, fmt,
+                                                   _lib.stream_of(tables))
+        _lib.check(rc, f"lffn_lookup_gather_parts_rows(B={B}, T={T}, S={S}, Do={Do}, row_format={fmt})")
+        return out
     # many tokens: the four-lanes-per-token form, which wants a workspace for its record stream; a few
     # thousand: the table-split form, which wants one for its partial outputs
     ws_bytes = ctypes.c_int64(0)
