@@ -18,7 +18,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "liblookupffn_hip.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 HOST_PATH = os.path.join(PKG_DIR, "_host.so")
-SOURCES = ["fht.hip", "code_score.hip", "gather.hip", "lookup_gather.hip", "lookup_gather_pair.hip", "lookup_gather_quad.hip", "lookup_scatter.hip", "lookup_scatter_sorted.hip", "lookup_inner.hip", "lookup_inner_quad.hip", "bh4_block.hip", "bh4_split.hip", "bh4_wgrad.hip", "layer_norm.hip", "linear.hip", "attention.hip"]
+SOURCES = ["fht.hip", "code_score.hip", "gather.hip", "lookup_gather.hip", "lookup_gather_pair.hip", "lookup_gather_quad.hip", "lookup_scatter.hip", "lookup_scatter_sorted.hip", "lookup_inner.hip", "lookup_inner_quad.hip", "bh4_block.hip", "bh4_split.hip", "bh4_wgrad.hip", "fht_bwd.hip", "layer_norm.hip", "linear.hip", "attention.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
