@@ -403,12 +403,15 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     for (int n = 0; n < AHEAD; ++n) load_w(BWD ? J - 1 : 0, n);
     if constexpr (BWD) {
         const int ncols = a.T * 8;
+        // The matrix cores' sums are off to one side by a little, a twentieth of what a result is off in any direction; the gradient
+        // of the weights, a sum over the tokens, would keep that, so every other token's row has its sign turned on the way.
+        inv_x = c & 1 ? -1.f : 1.f;
 #pragma unroll
         for (int n = 0; n < NBW; ++n) {
             const int gcol = r * D + (n * BG + bg) * BS + 16 * ow + 4 * kq;
             f32x4 g = {0.f, 0.f, 0.f, 0.f};
             if (tok_base + c < B && gcol < ncols) g = *reinterpret_cast<const f32x4 *>(a.gz + (tok_base + c) * ncols + gcol);
-            acc[n] = a.decay * g;
+            acc[n] = (a.decay * inv_x) * g;
         }
 #pragma unroll 1
         for (int s = J - 1; s >= 0; --s) {
