@@ -30,15 +30,18 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BS = 64;
-// Tokens per workgroup: 512, or fewer where that leaves the chip idle (a batch of 385 tokens at 512 columns is 32
-// workgroups of 512; chunk_tokens).  More chunks are more atomic additions to the result, which at thousands of tokens
-// cost more than they bring (256 tokens instead of 512 at 16384 x 1024 measured slower).
-constexpr int CHUNK = 512, MIN_CHUNK = 64;
-constexpr int64_t CHUNK_WORKGROUPS = 512;
+// Tokens per workgroup.  Every workgroup ends in 4096 atomic additions to the result, which at a thousand workgroups and more are
+// what a smaller chunk costs, and too few workgroups leave the chip idle.  us at chunks of 1024 | 512 | 256 | 128 | 64 tokens:
+//   32768 tokens, D = 512, two repeats of four stages (2048 workgroups of 1024)  239 | 266 | 320 | 397 | 886
+//   16384, D = 1024, one repeat (1024)                                           129 | 135 | 177 | 217 | 341
+//   16384, D = 512 (512)                                                          65 |  61 |  79 | 115 | 183
+//    4096, D = 512 (128)                                                          48 |  28 |  23 |  30 |  46
+//    1024, D = 512 (32)                                                           37 |  20 |  13 |  10 |  12
 int chunk_tokens(int64_t B, int64_t blocks) {
-    int chunk = CHUNK;
-    while (chunk > MIN_CHUNK && (B + chunk - 1) / chunk * blocks < CHUNK_WORKGROUPS) chunk /= 2;
-    return chunk;
+    constexpr struct { int chunk, workgroups; } options[] = {{1024, 1024}, {512, 512}, {256, 256}, {128, 256}};
+    for (const auto &o : options)
+        if ((B + o.chunk - 1) / o.chunk * blocks >= o.workgroups) return o.chunk;
+    return 64;
 }
 constexpr int DEPTH = 4;          // token quads whose loads are in flight per wavefront
 
