@@ -465,7 +465,7 @@ struct TokenLayerArgs {
 
 constexpr int TOKEN_STAGES = 4;     // diagonals requested together
 
-template <int LOGD, int FMT, int WAVES>
+template <int LOGD, int FMT, int WAVES, bool PARTS>
 __global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs args) {
     using C = FhtCfg<LOGD>;
     constexpr int D = C::D, NJ = C::NJ;
@@ -598,23 +598,28 @@ __global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs 
         }
     }
     __syncthreads();
-    token_gather<WAVES, FMT>(args.g, pairs, row, wave, lane);
+    token_gather<WAVES, FMT, PARTS>(args.g, pairs, row, wave, lane);
 }
 
-template <int FMT, int WAVES>
-int launch_token_layer_waves(const TokenLayerArgs &a, int64_t D, hipStream_t st) {
-    const dim3 grid((unsigned)a.p.B), block(64 * WAVES);
+template <int FMT, int WAVES, bool PARTS = false>
+int launch_token_layer_waves(const TokenLayerArgs &a, int64_t D, int parts, hipStream_t st) {
+    const dim3 grid((unsigned)a.p.B, (unsigned)parts), block(64 * WAVES);
     switch (lffn_log2(D)) {
-        case 8: hipLaunchKernelGGL((token_layer_kernel<8, FMT, WAVES>), grid, block, 0, st, a); break;
-        case 9: hipLaunchKernelGGL((token_layer_kernel<9, FMT, WAVES>), grid, block, 0, st, a); break;
-        default: hipLaunchKernelGGL((token_layer_kernel<10, FMT, WAVES>), grid, block, 0, st, a); break;
+        case 8: hipLaunchKernelGGL((token_layer_kernel<8, FMT, WAVES, PARTS>), grid, block, 0, st, a); break;
+        case 9: hipLaunchKernelGGL((token_layer_kernel<9, FMT, WAVES, PARTS>), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((token_layer_kernel<10, FMT, WAVES, PARTS>), grid, block, 0, st, a); break;
     }
     return lffn_launch_status();
 }
 
 template <int FMT>
-int launch_token_layer(const TokenLayerArgs &a, int64_t D, hipStream_t st) {
-    return a.p.B <= TOKEN_WIDE_MAX ? launch_token_layer_waves<FMT, 8>(a, D, st) : launch_token_layer_waves<FMT, 4>(a, D, st);
+int launch_token_layer(TokenLayerArgs a, int64_t D, hipStream_t st) {
+    if (a.p.B > TOKEN_WIDE_MAX) return launch_token_layer_waves<FMT, 4>(a, D, 1, st);
+    // several workgroups of a token read its input: not where another may have written the result there
+    const char *x = reinterpret_cast<const char *>(a.p.x), *out = reinterpret_cast<const char *>(a.g.gout);
+    const bool apart = out + a.p.B * a.g.Do * 4 <= x || x + a.p.B * a.p.H * 4 <= out;
+    const int parts = apart ? token_parts(a.g, a.p.B) : 1;
+    return parts > 1 ? launch_token_layer_waves<FMT, 8, true>(a, D, parts, st) : launch_token_layer_waves<FMT, 8>(a, D, 1, st);
 }
 
 template <bool HASH>

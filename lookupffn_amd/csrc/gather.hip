@@ -471,7 +471,7 @@ struct TokenCodes {
 __device__ __forceinline__ int token_row(int raw, int S, int last_row) { return S ? raw & (S - 1) : min(max(raw, 0), last_row); }
 
 
-template <int FMT, int WAVES>
+template <int FMT, int WAVES, bool PARTS>
 __global__ __launch_bounds__(64 * WAVES) void token_gather_kernel(TokenCodes a) {
     if (table_guard_ends(a.guard)) return;
     __shared__ uint2 pairs[TOKEN_MAX_T];
@@ -479,7 +479,7 @@ __global__ __launch_bounds__(64 * WAVES) void token_gather_kernel(TokenCodes a) 
     for (int t = threadIdx.x; t < a.g.T; t += 64 * WAVES)
         pairs[t] = make_uint2((unsigned)token_row(a.code[row * a.g.T + t], a.g.S, a.last_row), __float_as_uint(a.score[row * a.g.T + t]));
     __syncthreads();
-    token_gather<WAVES, FMT>(a.g, pairs, row, threadIdx.x >> 6, threadIdx.x & 63);
+    token_gather<WAVES, FMT, PARTS>(a.g, pairs, row, threadIdx.x >> 6, threadIdx.x & 63);
 }
 
 // The score gradient (and the inner product on flat row numbers) for small batches:
@@ -579,8 +579,14 @@ void launch_token_inner(const TokenInner &a, int64_t B, void *stream) {
 }
 
 template <int FMT, int WAVES>
-int launch_token_gather(const TokenCodes &a, int64_t B, hipStream_t st) {
-    hipLaunchKernelGGL((token_gather_kernel<FMT, WAVES>), dim3((unsigned)B), dim3(64 * WAVES), 0, st, a);
+int launch_token_gather(TokenCodes a, int64_t B, hipStream_t st) {
+    if constexpr (WAVES == 8) {
+        if (const int parts = token_parts(a.g, B); parts > 1) {
+            hipLaunchKernelGGL((token_gather_kernel<FMT, WAVES, true>), dim3((unsigned)B, (unsigned)parts), dim3(64 * WAVES), 0, st, a);
+            return lffn_launch_status();
+        }
+    }
+    hipLaunchKernelGGL((token_gather_kernel<FMT, WAVES, false>), dim3((unsigned)B), dim3(64 * WAVES), 0, st, a);
     return lffn_launch_status();
 }
 

@@ -21,7 +21,21 @@ struct TokenGatherArgs {
     const float *gres;    // [B, Do] or null: added to the result
     float *gout;          // [B, Do]
     int T, S, Do;
+    int part_cols = 0;    // columns of workgroup blockIdx.y of a token: a multiple of 256, or 0 for all of them
 };
+
+// Workgroups for a token, and the columns of each: as many as there are 256-column passes while the batch leaves compute units
+// idle.  What comes before the gather is repeated by each; the sums of a column are the same.  One compute unit takes in a token's
+// rows at some 60 bytes a clock, 393 KB of them at 128 tables of 768 fp32 columns: layer, us, 17 tokens 11.7 -> 9.3, 64 tokens 12.7 -> 11.5, 85
+// tokens 13.2 -> 12.6; 512 tables of 1024 columns, 17 tokens 29.5 -> 14.9, 64 tokens 47 -> 28.
+inline int token_parts(TokenGatherArgs &a, int64_t B) {
+    const int passes = (a.Do + 255) / 256;
+    const int64_t most = TOKEN_WIDE_MAX / (B > 0 ? B : 1);
+    const int parts = (int)(most < passes ? most : passes);
+    if (parts < 2) return 1;
+    a.part_cols = (passes + parts - 1) / parts * 256;
+    return (a.Do + a.part_cols - 1) / a.part_cols;
+}
 
 // four columns of a row as they are loaded, and their products with a score added up
 template <int FMT>
@@ -44,7 +58,7 @@ __device__ __forceinline__ void add_quad(float4 &acc, const RowQuad<FMT> &v, flo
 
 // Columns [col0, col0 + 256 NC).  Loads are unconditional at clamped columns, so that none of them waits for another; what
 // a clamped lane loaded is never stored.  Called by all wavefronts of the workgroup, with `pairs` visible to them.
-template <int WAVES, int NC, int FMT>
+template <int WAVES, int NC, int FMT, int ROWS>
 __device__ __forceinline__ void token_gather_columns(const TokenGatherArgs &a, const uint2 *pairs,
                                                      float4 (*part)[TOKEN_MAX_NC][64], int64_t row, int col0, int wave,
                                                      int lane) {
@@ -67,11 +81,11 @@ __device__ __forceinline__ void token_gather_columns(const TokenGatherArgs &a, c
     if (writes && a.gres) rr = *reinterpret_cast<const float4 *>(a.gres + row * a.Do + wcol);
     const int share = (a.T + WAVES - 1) / WAVES;
     const int t_lo = min(wave * share, a.T), t_hi = min(t_lo + share, a.T);
-    for (int t0 = t_lo; t0 < t_hi; t0 += 8) {
-        Quad rv[8][NC];
-        float sv[8];
+    for (int t0 = t_lo; t0 < t_hi; t0 += ROWS) {
+        Quad rv[ROWS][NC];
+        float sv[ROWS];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < ROWS; ++u) {
             const int tt = min(t0 + u, t_hi - 1);
             const uint2 pr = pairs[tt];
             sv[u] = t0 + u < t_hi ? __uint_as_float(pr.y) : 0.f;
@@ -80,7 +94,7 @@ __device__ __forceinline__ void token_gather_columns(const TokenGatherArgs &a, c
             for (int c = 0; c < NC; ++c) rv[u][c] = *reinterpret_cast<const Quad *>(rowp + gc[c] * ESZ);
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+        for (int u = 0; u < ROWS; ++u)
 #pragma unroll
             for (int c = 0; c < NC; ++c)
                 if (t0 + u < t_hi) add_quad<FMT>(acc[c], rv[u][c], sv[u]);    // (uniform; a row past the end may hold anything)
@@ -101,16 +115,27 @@ __device__ __forceinline__ void token_gather_columns(const TokenGatherArgs &a, c
     }
 }
 
-template <int WAVES, int FMT>
+// PARTS: workgroup blockIdx.y has the token's columns from blockIdx.y * part_cols on, one or two passes at a time: their registers allow
+// sixteen rows of a wavefront in flight.
+template <int WAVES, int FMT, bool PARTS>
 __device__ __forceinline__ void token_gather(const TokenGatherArgs &a, const uint2 *pairs, int64_t row, int wave, int lane) {
     __shared__ float4 part[WAVES][TOKEN_MAX_NC][64];
+    if constexpr (PARTS) {
+        const int first = blockIdx.y * a.part_cols, stop = min(a.Do, first + a.part_cols);
+        for (int col0 = first; col0 < stop; col0 += 512) {
+            if (col0 > first) __syncthreads();         // `part` has been read
+            if (stop - col0 > 256) token_gather_columns<WAVES, 2, FMT, 16>(a, pairs, part, row, col0, wave, lane);
+            else token_gather_columns<WAVES, 1, FMT, 16>(a, pairs, part, row, col0, wave, lane);
+        }
+        return;
+    }
     for (int col0 = 0; col0 < a.Do; col0 += 256 * TOKEN_MAX_NC) {
         if (col0) __syncthreads();                     // `part` has been read
         switch (min(TOKEN_MAX_NC, (a.Do - col0 + 255) / 256)) {
-            case 1: token_gather_columns<WAVES, 1, FMT>(a, pairs, part, row, col0, wave, lane); break;
-            case 2: token_gather_columns<WAVES, 2, FMT>(a, pairs, part, row, col0, wave, lane); break;
-            case 3: token_gather_columns<WAVES, 3, FMT>(a, pairs, part, row, col0, wave, lane); break;
-            default: token_gather_columns<WAVES, 4, FMT>(a, pairs, part, row, col0, wave, lane); break;
+            case 1: token_gather_columns<WAVES, 1, FMT, 8>(a, pairs, part, row, col0, wave, lane); break;
+            case 2: token_gather_columns<WAVES, 2, FMT, 8>(a, pairs, part, row, col0, wave, lane); break;
+            case 3: token_gather_columns<WAVES, 3, FMT, 8>(a, pairs, part, row, col0, wave, lane); break;
+            default: token_gather_columns<WAVES, 4, FMT, 8>(a, pairs, part, row, col0, wave, lane); break;
         }
     }
 }

@@ -1,0 +1,62 @@
+"""A token's columns shared out over several workgroups (csrc/token_gather.h): as from one, bit for bit."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+from lookupffn_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+DEV, S = "cuda:0", 256
+
+
+def _layer(H, D, R, T, Do, dtype, seed=0):
+    gen = torch.Generator(device=DEV).manual_seed(H + T + Do + seed)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    t = dict(ln_weight=1 + 0.1 * rand(H), ln_bias=0.1 * rand(H), diag=rand(R, 4, D) / math.sqrt(D), proj_bias=0.1 * rand(T * 8),
+             tables=(0.02 * rand(T, S, Do)).to(dtype), out_bias=rand(Do))
+    layer = _lib.FusedLayer(*(t[k].data_ptr() for k in ("ln_weight", "ln_bias", "diag", "proj_bias", "tables", "out_bias")),
+                            H, D, R, 4, T, S, Do, 1e-5, 0.7, 0.3)
+    return t, layer, rand
+
+
+def _run(layer, fmt, x, residual, out):
+    _lib.check(_lib.load().lffn_lookup_ffn_fused_layer_rows(ctypes.byref(layer), fmt, x.data_ptr(), _lib.ptr(residual), out.data_ptr(),
+                                                            x.shape[0], _lib.stream_of(x)), "fused layer")
+    return out
+
+
+# 256 tokens have one workgroup each; fewer share out 2 to 10 passes of 256 columns, the last of them short, one and two passes to a workgroup
+@pytest.mark.parametrize("H,D,R,T,Do,fmt", [(768, 1024, 1, 128, 768, 0), (500, 512, 2, 100, 260, 0), (256, 256, 1, 32, 516, 1),
+                                            (1024, 1024, 2, 200, 1284, 2), (768, 1024, 1, 65, 2560, 0), (512, 512, 1, 64, 512, 2)])
+def test_layer(H, D, R, T, Do, fmt):
+    _, layer, rand = _layer(H, D, R, T, Do, [torch.float32, torch.bfloat16, torch.float16][fmt])
+    x, residual = rand(256, H), rand(256, Do)
+    want = _run(layer, fmt, x, residual, torch.full((256, Do), float("nan"), device=DEV))
+    assert torch.isfinite(want).all()
+    for B in (1, 17, 51, 64, 85, 86, 127, 128, 129):
+        assert torch.equal(_run(layer, fmt, x[:B].clone(), residual[:B].clone(), torch.full((B, Do), float("nan"), device=DEV)), want[:B])
+        again = residual[:B].clone()                      # the result in the residual's place
+        assert torch.equal(_run(layer, fmt, x[:B].clone(), again, again), want[:B])
+
+
+def test_result_in_the_input():
+    """In the input's place a token's workgroup reads all it needs before it writes: one to a token then."""
+    _, layer, rand = _layer(1024, 1024, 1, 128, 1024, torch.float32)
+    x = rand(40, 1024)
+    want = _run(layer, 0, x, x, torch.empty_like(x))
+    assert torch.equal(_run(layer, 0, x, x, x), want)
+
+
+@pytest.mark.parametrize("T,Do,fmt", [(128, 768, 0), (30, 1024, 1), (300, 576, 2)])
+def test_gather_operators(T, Do, fmt):
+    t, _, _ = _layer(64, 64, 1, T, Do, [torch.float32, torch.bfloat16, torch.float16][fmt])
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    code = torch.randint(0, S, (256, T), generator=gen, device=DEV, dtype=torch.int32)
+    score, tables = torch.rand(256, T, generator=gen, device=DEV), t["tables"]
+    rows = (code + torch.arange(T, device=DEV, dtype=torch.int32) * S)[:, torch.randperm(T, generator=gen, device=DEV)].contiguous()
+    want = ops.lookup_gather(code, score, tables, t["out_bias"]), ops.gather_add(rows, tables.view(T * S, Do), score)
+    for B in (1, 63, 85, 128):
+        assert torch.equal(ops.lookup_gather(code[:B], score[:B], tables, t["out_bias"]), want[0][:B])
+        assert torch.equal(ops.gather_add(rows[:B], tables.view(T * S, Do), score[:B]), want[1][:B])
