@@ -455,9 +455,9 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
 //
 // What a small batch waits for is a chain of memory round trips (rows of the input, parameters, table rows), so: the
 // input row, the LayerNorm parameters, the diagonals and the bias are requested together before the first is used; the
-// repeats run side by side, one per wavefront (512 tables of 1024 columns: four); and the wavefronts split the rows.  Rows in
-// fp32, bfloat16 or half (FMT).  128 tables of 768 columns, 16 tokens: 12.3 -> 11.4 us (fp32), 34.4 -> 11.6 us (bfloat16,
-// before in two launches); 512 tables of 1024 columns 39.7 -> 29.4 us and 87.1 -> 24.5 us.
+// repeats run side by side, one per wavefront (512 tables of 1024 columns: four) or, where the wavefronts are enough, one per
+// 256 points of them (SHARED: project_shared); and the wavefronts split the rows.  Rows in fp32, bfloat16 or half (FMT).  With PARTS
+// several workgroups have a token (token_gather.h).
 struct TokenLayerArgs {
     ProjectArgs p;
     TokenGatherArgs g;
@@ -465,7 +465,139 @@ struct TokenLayerArgs {
 
 constexpr int TOKEN_STAGES = 4;     // diagonals requested together
 
-template <int LOGD, int FMT, int WAVES, bool PARTS>
+// Mix, bias, code and score of a lane's four columns, from column `col` of the result on, as in project_kernel: the odd lane of a pair
+// continues the even lane's sum and product.
+__device__ __forceinline__ void hash_quad(const ProjectArgs &a, const float (&y)[4], const float (&orig)[4], float4 pb, int col, int lane,
+                                          uint2 *pairs) {
+    float z[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const float m0 = a.decay * y[c];
+        const float m1 = a.residual * orig[c];
+        z[c] = m0 + m1;
+    }
+    if (a.pbias) { z[0] = z[0] + pb.x; z[1] = z[1] + pb.y; z[2] = z[2] + pb.z; z[3] = z[3] + pb.w; }
+    const int nib = (z[0] > 0.f ? 8 : 0) | (z[1] > 0.f ? 4 : 0) | (z[2] > 0.f ? 2 : 0) | (z[3] > 0.f ? 1 : 0);
+    float az[4], fz[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        az[c] = fabsf(z[c]);
+        fz[c] = 1.0f + exp_minus_2a(az[c]);
+    }
+    float s_loc = 0.f, p_loc = 1.f;
+    score_chain(az, fz, s_loc, p_loc);
+    float s_run = lane_xor<1>(s_loc);
+    float p_run = lane_xor<1>(p_loc);
+    const int nib_hi = __float_as_int(lane_xor<1>(__int_as_float(nib)));
+    score_chain(az, fz, s_run, p_run);
+    const int t = col >> 3;
+    if ((lane & 1) && t < a.T) pairs[t] = make_uint2((unsigned)((nib_hi << 4) | nib), __float_as_uint(s_run / p_run));
+}
+
+// The projection and hash of a token with a wavefront for every 256 points of every repeat (NJ of them a repeat, all of which the
+// workgroup must have): value c of lane l is element 256 j + 4 l + c as in project_kernel, so the strides of 256 and up are between the
+// wavefronts, a trip through LDS, and the others are a quarter or half of one wavefront's work.  The same operations in the same
+// order, the same bits.  A token waits for this chain: layer, us, 128 tables of 768 columns, 1024 points: 17 tokens 9.3 -> 6.7, 256 tokens
+// 21.4 -> 18.7, 512 tokens 34.0 -> 31.5; 256 half-precision tables of 768, two repeats: 17 tokens 11.1 -> 9.0.
+template <int LOGD, int WAVES>
+__device__ __forceinline__ void project_shared(const ProjectArgs &a, uint2 *pairs, int64_t row, int wave, int lane) {
+    using C = FhtCfg<LOGD>;
+    constexpr int D = C::D, NJ = C::NJ;
+    static_assert(C::LPR == 64 && (NJ == 2 || NJ == 4), "512 or 1024 points");
+    __shared__ float4 turn[2][WAVES][64];
+    const int r = wave / NJ, own = wave % NJ;
+    const bool works = r < a.R;                                // uniform over the wavefront; the others only keep the barriers
+    const int col = r * D + 256 * own + 4 * lane;
+    float v[1][4], orig[4];
+    float4 dg[TOKEN_STAGES], pb = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto fetch_diag = [&](int s0) {
+#pragma unroll
+        for (int s = 0; s < TOKEN_STAGES; ++s)
+            if (s0 + s < a.J) dg[s] = *reinterpret_cast<const float4 *>(a.diag + ((int64_t)r * a.J + s0 + s) * D + 256 * own + 4 * lane);
+    };
+    if (works) {
+        float in[NJ][4], lw[4], lb[4];
+        auto fetch = [&](const float *p, bool vec, int e0, float (&t)[4]) {
+            float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (vec) {
+                if (e0 < a.H) w = *reinterpret_cast<const float4 *>(p + e0);
+            } else {
+                if (e0 + 0 < a.H) w.x = p[e0 + 0];
+                if (e0 + 1 < a.H) w.y = p[e0 + 1];
+                if (e0 + 2 < a.H) w.z = p[e0 + 2];
+                if (e0 + 3 < a.H) w.w = p[e0 + 3];
+            }
+            t[0] = w.x; t[1] = w.y; t[2] = w.z; t[3] = w.w;
+        };
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) fetch(a.x + row * a.H, a.vec_in, 256 * j + 4 * lane, in[j]);
+        if (a.ln_w) {
+            fetch(a.ln_w, a.vec_ln, 256 * own + 4 * lane, lw);
+            fetch(a.ln_b, a.vec_ln, 256 * own + 4 * lane, lb);
+        }
+        fetch_diag(0);
+        if (a.pbias && col < a.out_cols) pb = *reinterpret_cast<const float4 *>(a.pbias + col);
+        __builtin_amdgcn_sched_barrier(0);                     // (the loads stay ahead of the reductions below)
+        float mean = 0.f, rstd = 1.f;
+        if (a.ln_w) {
+            // LayerNorm's sums as in project_kernel, of the whole row by every wavefront
+            float s1 = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s1 += in[j][c];
+            mean = lane_group_sum<64>(s1) / float(a.H);
+            float s2 = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float dlt = (256 * j + 4 * lane + c < a.H) ? in[j][c] - mean : 0.f;
+                    s2 += dlt * dlt;
+                }
+            rstd = 1.0f / sqrtf(lane_group_sum<64>(s2) / float(a.H) + a.ln_eps);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float t = in[0][c];
+#pragma unroll
+            for (int j = 1; j < NJ; ++j) t = own == j ? in[j][c] : t;
+            if (a.ln_w && 256 * own + 4 * lane + c < a.H) t = (t - mean) * rstd * lw[c] + lb[c];
+            orig[c] = t;
+            v[0][c] = t;
+        }
+    }
+    for (int s0 = 0; s0 < a.J; s0 += TOKEN_STAGES) {
+        if (s0 && works) fetch_diag(s0);
+#pragma unroll
+        for (int s = 0; s < TOKEN_STAGES; ++s) {
+            if (s0 + s < a.J) {                                // uniform
+                float4 (&buffer)[WAVES][64] = turn[s & 1];     // (the other one is still being read)
+                if (works)
+                    buffer[wave][lane] = make_float4(v[0][0] * dg[s].x, v[0][1] * dg[s].y, v[0][2] * dg[s].z, v[0][3] * dg[s].w);
+                __syncthreads();
+                if (works) {
+                    float4 q[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) q[j] = buffer[r * NJ + j][lane];
+                    auto add = [](float4 x, float4 y) { return make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w); };
+                    auto sub = [](float4 x, float4 y) { return make_float4(x.x - y.x, x.y - y.y, x.z - y.z, x.w - y.w); };
+                    float4 x = q[0], y = q[1];
+                    if constexpr (NJ == 4) {                   // stride 512
+                        x = own < 2 ? add(q[0], q[2]) : sub(q[0], q[2]);
+                        y = own < 2 ? add(q[1], q[3]) : sub(q[1], q[3]);
+                    }
+                    x = own & 1 ? sub(x, y) : add(x, y);       // stride 256
+                    v[0][0] = x.x; v[0][1] = x.y; v[0][2] = x.z; v[0][3] = x.w;
+                    fht_rows<8, true>(v, lane);
+                }
+            }
+        }
+    }
+    if (works) hash_quad(a, v[0], orig, pb, col, lane, pairs);
+}
+
+template <int LOGD, int FMT, int WAVES, bool PARTS, bool SHARED>
 __global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs args) {
     using C = FhtCfg<LOGD>;
     constexpr int D = C::D, NJ = C::NJ;
@@ -475,7 +607,9 @@ __global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int64_t row = blockIdx.x;
-    if (wave < a.R) {                                          // uniform over the wavefront
+    if constexpr (SHARED) {
+        project_shared<LOGD, WAVES>(a, pairs, row, __builtin_amdgcn_readfirstlane(wave), lane);
+    } else if (wave < a.R) {                                   // uniform over the wavefront
         float orig[NJ][4], lw[NJ][4], lb[NJ][4];
         float4 dg[TOKEN_STAGES][NJ], pb[NJ];
         auto fetch_diag = [&](int r, int s0) {
@@ -569,31 +703,7 @@ __global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs 
             }
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                float z[4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const float m0 = a.decay * v[j][c];
-                    const float m1 = a.residual * orig[j][c];
-                    z[c] = m0 + m1;
-                }
-                if (a.pbias) { z[0] = z[0] + pb[j].x; z[1] = z[1] + pb[j].y; z[2] = z[2] + pb[j].z; z[3] = z[3] + pb[j].w; }
-                // code and score as in project_kernel: the odd lane of a pair continues the even lane's sum and product
-                const int nib = (z[0] > 0.f ? 8 : 0) | (z[1] > 0.f ? 4 : 0) | (z[2] > 0.f ? 2 : 0) | (z[3] > 0.f ? 1 : 0);
-                float az[4], fz[4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    az[c] = fabsf(z[c]);
-                    fz[c] = 1.0f + exp_minus_2a(az[c]);
-                }
-                float s_loc = 0.f, p_loc = 1.f;
-                score_chain(az, fz, s_loc, p_loc);
-                float s_run = lane_xor<1>(s_loc);
-                float p_run = lane_xor<1>(p_loc);
-                const int nib_hi = __float_as_int(lane_xor<1>(__int_as_float(nib)));
-                score_chain(az, fz, s_run, p_run);
-                const int t = (r * D + 256 * j + 4 * lane) >> 3;
-                if ((lane & 1) && t < a.T)
-                    pairs[t] = make_uint2((unsigned)((nib_hi << 4) | nib), __float_as_uint(s_run / p_run));
+                hash_quad(a, v[j], orig[j], pb[j], r * D + 256 * j + 4 * lane, lane, pairs);
             }
         }
     }
@@ -601,13 +711,24 @@ __global__ __launch_bounds__(64 * WAVES) void token_layer_kernel(TokenLayerArgs 
     token_gather<WAVES, FMT, PARTS>(args.g, pairs, row, wave, lane);
 }
 
+template <int LOGD, int FMT, int WAVES, bool PARTS>
+void launch_token_layer_points(const TokenLayerArgs &a, int parts, hipStream_t st) {
+    const dim3 grid((unsigned)a.p.B, (unsigned)parts), block(64 * WAVES);
+    if constexpr (FhtCfg<LOGD>::NJ > 1) {
+        if (a.p.R * FhtCfg<LOGD>::NJ <= WAVES) {
+            hipLaunchKernelGGL((token_layer_kernel<LOGD, FMT, WAVES, PARTS, true>), grid, block, 0, st, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((token_layer_kernel<LOGD, FMT, WAVES, PARTS, false>), grid, block, 0, st, a);
+}
+
 template <int FMT, int WAVES, bool PARTS = false>
 int launch_token_layer_waves(const TokenLayerArgs &a, int64_t D, int parts, hipStream_t st) {
-    const dim3 grid((unsigned)a.p.B, (unsigned)parts), block(64 * WAVES);
     switch (lffn_log2(D)) {
-        case 8: hipLaunchKernelGGL((token_layer_kernel<8, FMT, WAVES, PARTS>), grid, block, 0, st, a); break;
-        case 9: hipLaunchKernelGGL((token_layer_kernel<9, FMT, WAVES, PARTS>), grid, block, 0, st, a); break;
-        default: hipLaunchKernelGGL((token_layer_kernel<10, FMT, WAVES, PARTS>), grid, block, 0, st, a); break;
+        case 8: launch_token_layer_points<8, FMT, WAVES, PARTS>(a, parts, st); break;
+        case 9: launch_token_layer_points<9, FMT, WAVES, PARTS>(a, parts, st); break;
+        default: launch_token_layer_points<10, FMT, WAVES, PARTS>(a, parts, st); break;
     }
     return lffn_launch_status();
 }

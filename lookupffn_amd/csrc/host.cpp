@@ -242,9 +242,12 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
            int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
-    // (rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half
-    // as many tokens more: 768 tokens, 128 tables of 768 columns 34 us against 55 in two launches, 512 of 1024 113 against 120)
-    if (c.one_launch && B <= (c.fmt == 0 ? fused_max : fused_max + fused_max / 2)) {
+    // Rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half as many tokens
+    // more, and so are tables of which a token's rows are few.  One launch, two, us: fp32 768 tokens, 128 tables of 768 columns
+    // 45, 46, 128 of 512 32, 35, but 128 of 1024 60, 57 and 512 of 1024 218, 187; bfloat16 1152 tokens, 128 of 768 37, 56.
+    if (c.fmt != 0) fused_max += fused_max / 2;
+    if (c.T * c.Do <= 128 * 768) fused_max += fused_max / 2;
+    if (c.one_launch && B <= fused_max) {
         const lffn_fused_layer layer{f32(p[0]), f32(p[1]), f32(p[2]), f32(p[3]), f32(p[4]), f32(p[5]), c.H, c.D, c.R, c.J, c.T,
                                      c.S, c.Do, (float)c.eps, (float)c.decay, (float)c.residual};
         CALL(lffn_lookup_ffn_fused_layer_rows, &layer, (int32_t)c.fmt, f32(x), residual, f32(out), B, st);
