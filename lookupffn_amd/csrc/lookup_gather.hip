@@ -585,7 +585,8 @@ constexpr PartsCost PARTS_COST[3] = {{3.3, 1.35, 0.78, 0.158, 1.70, 0.0066, 1.18
 constexpr double PARTS_BIG_BYTES = 240e6;                // tables beyond the memory-side cache by themselves
 constexpr double PARTS_BIG_FETCH = 1.74, PARTS_BIG_FETCH_BLOCK = 0.0062, PARTS_BIG_TOUCHED = 0.87, PARTS_BIG_TOUCHED_BLOCK = 0.015;
 constexpr int MAX_PARTS = 32;
-constexpr double PARTS_MARGIN = 1.0;                     // the other plans' times are those of tables in the memory-side cache
+constexpr double PARTS_TOKEN_MARGIN = 0.92;              // of what the token-major kernel promises; of the other forms, whose times
+                                                         // are those of tables in the memory-side cache, all
 // What plan_quad's time leaves out: the start and end of its launch (16384 x 128 x 768: 101 us promised, 108 measured)
 constexpr double QUAD_START_US = 8.0;
 
@@ -627,8 +628,8 @@ PartsPlan plan_parts(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, bool 
 // plan_parts if it promises to beat the other forms, parts = 0 otherwise.  Layer gather from records, tables of twelve layers in
 // turn | of one layer again and again, us, other form -> this one: fp32 2674 x 128 x 768 65 -> 56 | 54 -> 42, 3763 x 128 x 512 56 -> 46 | 49 -> 35,
 // 6000 x 128 x 768 103 -> 75 | 88 -> 59, 8954 x 256 x 384 160 -> 85 | 143 -> 73, 8621 x 512 x 512 325 -> 177; bfloat16 1800 x 128 x 1024
-// 54 -> 45 | 55 -> 41; half 3022 x 256 x 768 126 -> 68 | 126 -> 58, 8000 x 128 x 1024 242 -> 86.  Left where they are: fp32 2103 x 128 x 768
-// 57 -> 52 | 48 -> 39 (no faster in the layer, whose tables are half in the cache), 1024 x 128 x 1024 48 -> 47, 2136 x 64 x 768 33 -> 35.
+// 54 -> 45 | 55 -> 41; half 3022 x 256 x 768 126 -> 68 | 126 -> 58, 8000 x 128 x 1024 242 -> 86.  Left where they are: fp32 1024 x 128 x 1024
+// 48 -> 47 | 37 -> 35, 512 x 128 x 384 16 -> 22.
 PartsPlan choose_parts(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, bool pack) {
     const PartsPlan p = plan_parts(fmt, B, T, S, Do, pack);
     if (p.parts == 0) return p;
@@ -637,7 +638,7 @@ PartsPlan choose_parts(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, boo
     // calls stay there.
     const double row_bytes = double(Do) * (fmt == LFFN_ROWS_F32 ? 4 : 2), table_bytes = double(T) * double(S) * row_bytes;
     const double rate = row_bytes <= 512.0 || table_bytes <= 10e6 ? 15e6 : (table_bytes <= 20e6 ? 12e6 : 9e6);
-    if (p.us >= PARTS_MARGIN * (double(B) * double(T) * row_bytes / rate + 5.0)) return PartsPlan{};
+    if (p.us >= PARTS_TOKEN_MARGIN * (double(B) * double(T) * row_bytes / rate + 5.0)) return PartsPlan{};
     double other;
     if (fmt == LFFN_ROWS_F16) {
         const GatherPlan qp = plan_quad(fmt, B, T, S, Do, pack);
@@ -655,12 +656,16 @@ PartsPlan choose_parts(int fmt, int64_t B, int64_t T, int64_t S, int64_t Do, boo
                 other = double((B + each - 1) / each) * (other + 4.0);
             } else {
                 const SplitPlan sp = bf16 ? plan_split<true>(B, T, S, Do) : plan_split<false>(B, T, S, Do);
-                // (plan_split counts 4 TB/s for the partial sums; they come at 6, and 2 us less for the launch)
-                if (sp.nparts > 1 && sp.us < 0.85 * other) other = sp.us - double(2 * sp.nparts + 1) * double(B) * double(Do) * 4.0 / 12e6 - 2.0;
+                if (sp.nparts > 1 && sp.us < 0.85 * other) {
+                    other = sp.us;
+                    // (plan_split counts 4 TB/s for the partial sums, of tables in the cache; they come at 6, and the launch in 2 us
+                    // less.  For records, which are there, the two errors are of one size; packing them has to be worth it.)
+                    if (pack) other -= double(2 * sp.nparts + 1) * double(B) * double(Do) * 4.0 / 12e6 + 2.0;
+                }
             }
         }
     }
-    return p.us < PARTS_MARGIN * other ? p : PartsPlan{};
+    return p.us < other ? p : PartsPlan{};
 }
 
 // the records, then one [B, Do] of partial sums per part
