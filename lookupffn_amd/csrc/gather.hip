@@ -484,9 +484,14 @@ __global__ __launch_bounds__(64 * WAVES) void token_gather_kernel(TokenCodes a) 
 
 // The score gradient (and the inner product on flat row numbers) for small batches:
 // grad_score[b,t] = <g[b,:], tables[t][code[b,t]][:]>, a token per workgroup of eight
-// wavefronts, which take an eighth of the tables each, eight rows together.  128 tables of 768 columns: 64 tokens 28.8 -> 7.0 us, 384
-// 32.1 -> 22.3 (1024 columns 34.0 -> 30.2, and at 512 tokens 35.7 -> 38.3: hence the limit); 512 tables of 1024 187 -> 31 and 193 -> 119.
-constexpr int64_t TOKEN_INNER_MAX = 384;
+// wavefronts, which take an eighth of the tables each, eight rows together.  Up to so many tokens times columns: tables of four
+// layers in turn, us, without -> with it: 128 tables of 768 columns 300 tokens 36 -> 22, 512 38 -> 29, 640 38 -> 37, 800 40 -> 47; 64 of 512
+// 385 tokens 16 -> 9, 640 17 -> 13, 800 17 -> 16, 1000 17 -> 19; 128 of 1024 385 41 -> 32, 512 42 -> 38, 640 43 -> 48 (64 of them 512 19 -> 20); 32
+// of 256 1500 9.6 -> 8.9.  Half rows are half of that: 128 of 1024 768 33 -> 29, 1000 34 -> 37; 128 of 512 1500 32 -> 27.
+bool token_inner(int64_t B, int64_t Do, int fmt) {
+    if (B <= 384) return B >= 1;                  // (wider rows: 512 tables of 1024 187 -> 31 at 64 tokens, 193 -> 119 at 384)
+    return B <= 1536 && B * Do <= (fmt == LFFN_ROWS_F16 ? 768 * 1024 : 384 * 1024);
+}
 struct TokenInner {
     const int32_t *code;
     const void *g;
@@ -630,7 +635,7 @@ int lffn_internal_inner_flat(const int32_t *idx, const float *g, const float *sr
     GatherArgs a{};
     a.idx = idx; a.src = src; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
     a.B = B; a.I = (int)I; a.source_size = source_size; a.Dv = (int)Dv; a.S = 0; a.guard = TableGuard{flags, 0};
-    if (B >= 1 && B <= TOKEN_INNER_MAX && I >= 1) {
+    if (token_inner(B, Dv, LFFN_ROWS_F32) && I >= 1) {
         launch_token_inner<LFFN_ROWS_F32>(TokenInner{idx, g, src, out, (int)I, 0, (int)Dv, (int)(source_size - 1), a.guard}, B, stream);
         return lffn_launch_status();
     }
@@ -703,7 +708,7 @@ int lffn_internal_lookup_scatter_atomic(const int32_t *code, const float *score,
 
 bool lffn_internal_lookup_inner_tokens_try(const int32_t *code, const float *g, const float *tables, float *out, int64_t B,
                                            int64_t T, int64_t S, int64_t Do, void *stream, int *rc) {
-    if (B > TOKEN_INNER_MAX || T < 1 || T * S > 0x7fffffff) return false;
+    if (!token_inner(B, Do, LFFN_ROWS_F32) || T < 1 || T * S > 0x7fffffff) return false;
     launch_token_inner<LFFN_ROWS_F32>(TokenInner{code, g, tables, out, (int)T, (int)S, (int)Do, 0, lffn_table_guard()}, B, stream);
     *rc = lffn_launch_status();
     return true;
@@ -746,7 +751,7 @@ extern "C" int lffn_indexed_inner_product_f16(const int32_t *idx, const uint16_t
     GatherArgs a{};
     a.idx = idx; a.src = src; a.w = nullptr; a.g = g; a.bias = nullptr; a.out = out;
     a.B = B; a.I = (int)I; a.source_size = source_size; a.Dv = (int)Dv; a.S = 0;
-    if (B >= 1 && B <= TOKEN_INNER_MAX && I >= 1) {
+    if (token_inner(B, Dv, LFFN_ROWS_F16) && I >= 1) {
         launch_token_inner<LFFN_ROWS_F16>(TokenInner{idx, g, src, out, (int)I, 0, (int)Dv, (int)(source_size - 1), TableGuard{}}, B, stream);
         return lffn_launch_status();
     }

@@ -60,3 +60,20 @@ def test_gather_operators(T, Do, fmt):
     for B in (1, 63, 85, 128):
         assert torch.equal(ops.lookup_gather(code[:B], score[:B], tables, t["out_bias"]), want[0][:B])
         assert torch.equal(ops.gather_add(rows[:B], tables.view(T * S, Do), score[:B]), want[1][:B])
+
+
+# either side of the line up to which the score gradient takes a token per workgroup
+@pytest.mark.parametrize("T,Do,half", [(128, 1024, False), (30, 512, False), (64, 256, False), (60, 768, True), (33, 512, True)])
+def test_inner_product_by_token_and_not(T, Do, half):
+    """Sums of Do products, in any order: off by (Do + 1) 2^-24 of the magnitudes at most."""
+    gen = torch.Generator(device=DEV).manual_seed(T + Do)
+    last = min(1536, (768 if half else 384) * 1024 // Do)
+    tables, g = 0.02 * torch.randn(T * S, Do, generator=gen, device=DEV), torch.randn(last + 1, Do, generator=gen, device=DEV)
+    if half:
+        tables, g = tables.half(), g.half()
+    rows = torch.randint(0, S, (last + 1, T), generator=gen, device=DEV, dtype=torch.int32) + torch.arange(T, device=DEV, dtype=torch.int32) * S
+    for B in (last, last + 1):
+        got = ops.indexed_inner_product(rows[:B].contiguous(), g[:B].contiguous(), tables)
+        for t in range(0, T, 7):
+            term = tables[rows[:B, t].long()].double() * g[:B].double()
+            assert ((got[:, t].double() - term.sum(-1)).abs() <= (Do + 1) * 2.0 ** -24 * term.abs().sum(-1)).all()
