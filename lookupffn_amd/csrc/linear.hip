@@ -37,9 +37,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N, THREADS = 64 * WAVES_M * WAVES_N;
     constexpr int BUF = 2 * (BM + BN) * 4;               // 16-byte pieces of a step's buffer
     constexpr int RSTEP = THREADS / 4;
-    constexpr int NC = (BM + BN) / RSTEP;                // pieces of eight numbers a thread brings a step
+    constexpr int NP = (BM + BN) / RSTEP;                // pieces of eight numbers a thread brings a step,
+    constexpr bool REST = (BM + BN) % RSTEP != 0;        // and half a piece, of the last RSTEP / 2 rows
+    constexpr int NC = NP + REST;
     constexpr int NR = 2 * (WM + WN);                    // fragments of half a step
-    static_assert(BM % RSTEP == 0 && BN % RSTEP == 0 && NC <= 3);
+    static_assert(BM % RSTEP == 0 && (BN % RSTEP == 0 || BN % RSTEP == RSTEP / 2) && NC <= 3);
     extern __shared__ __attribute__((aligned(16))) uint4 lds[];
     float *const inverse = reinterpret_cast<float *>(lds + 3 * BUF);      // [BM + BN] the rows' scales
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -61,8 +63,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     int dst[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
-        const int row = row0 + RSTEP * i;
-        if (RSTEP * i < BM) {
+        const int row = i < NP ? row0 + RSTEP * i : RSTEP * NP + (tid >> 3);
+        if (i == NP) {
+            src[i] = uint32_t(min(row - BM, N - 1 - n0)) * K + (tid & 7) * 4;
+            dst[i] = 2 * BM * 4 + (row - BM) * 4 + (((tid & 7) >> 1) ^ ((row >> 2) & 3));
+        } else if (RSTEP * i < BM) {
             src[i] = uint32_t(min(int64_t(row), M - 1 - m0)) * K + chunk * 8;
             dst[i] = row * 4 + (chunk ^ ((row >> 2) & 3));
         } else {
@@ -83,18 +88,19 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
         const int k = min(k0, K - BK);                  // (beyond the end: the last step again, never used)
         const float *const p = (RSTEP * i < BM ? xa : wb) + k;
         *reinterpret_cast<float4 *>(&v[i][0]) = *reinterpret_cast<const float4 *>(p + src[i]);
-        *reinterpret_cast<float4 *>(&v[i][4]) = *reinterpret_cast<const float4 *>(p + src[i] + 4);
+        if (i < NP) *reinterpret_cast<float4 *>(&v[i][4]) = *reinterpret_cast<const float4 *>(p + src[i] + 4);
     };
     uint32_t h[4];
     auto place = [&](uint4 *buf, int i, int p) {
         const int plane = (RSTEP * i < BM ? BM : BN) * 4;
         uint32_t o[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < (i < NP ? 4 : 2); ++e) {
             if (p == 0) o[e] = h[e] = split_hi(v[i][2 * e], v[i][2 * e + 1], scale[i]);
             else o[e] = split_lo(v[i][2 * e], v[i][2 * e + 1], scale[i], h[e]);
         }
-        buf[dst[i] + p * plane] = make_uint4(o[0], o[1], o[2], o[3]);
+        if (i < NP) buf[dst[i] + p * plane] = make_uint4(o[0], o[1], o[2], o[3]);
+        else reinterpret_cast<uint2 *>(buf + dst[i] + p * plane)[tid & 1] = make_uint2(o[0], o[1]);
     };
     uint4 fa[2][WM][2], fb[2][WN][2];                   // [half of the step][tile][hi, lo]
     auto read = [&](const uint4 *buf, int kk, int n) {
@@ -113,12 +119,17 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     for (int i = 0; i < NC; ++i) {
         float most = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(v[i][e]));
+        for (int e = 0; e < (i < NP ? 8 : 4); ++e) most = fmaxf(most, fabsf(v[i][e]));
         most = fmaxf(most, lane_xor<1>(most));
         most = fmaxf(most, lane_xor<2>(most));
+        if (i == NP) most = fmaxf(most, lane_xor<4>(most));
         const PowerOfTwo s = scale_to_one(most);
         scale[i] = s.scale;
-        if (chunk == 0) inverse[row0 + RSTEP * i] = s.inverse;
+        if (i < NP) {
+            if (chunk == 0) inverse[row0 + RSTEP * i] = s.inverse;
+        } else if ((tid & 7) == 0) {
+            inverse[RSTEP * NP + (tid >> 3)] = s.inverse;
+        }
         place(lds, i, 0);
         place(lds, i, 1);
         fetch(i, BK);
@@ -264,12 +275,16 @@ extern "C" int lffn_linear_f32(const float *x, const float *const *w, const floa
     a.K = (int)K;
     a.sets = (int)sets;
     // Time of each form in ns for K = 768, the same share of it for any other: a round of 256 tiles (one a compute unit) of 128 x 256
-    // takes 43 us, of 128 x 128 27.5; tiles of 64 x 64 share compute units, 13 us at least and 8.6 per 256 tiles.  Measured at 16 to
-    // 16384 rows of 512 to 1024: the form this picks is the fastest or within 3 % of it.
+    // takes 43 us, of 128 x 192 36, of 128 x 128 27.5; tiles of 64 x 64 share compute units, 13 us at least and 8.6 per 256 tiles.
+    // The middle one is the least a column when it fills its rounds and the widest does not: one matrix of 768 x 768 and 16384 rows is
+    // two whole rounds of it against one and a half of 128 x 256 (84 against 94 us), three and 4096 rows one and a half against 1.1
+    // (73 against 82 to 88).  Measured at 16 to 16384 rows of 512 to 1024: the form this picks is the fastest or within 3 % of it.
     auto tiles = [&](int64_t bm, int64_t bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn) * sets; };
-    const int64_t wide = (tiles(128, 256) + 255) / 256 * 43000, square = (tiles(128, 128) + 255) / 256 * 27500;
+    auto rounds = [&](int64_t bn) { return (tiles(128, bn) + 255) / 256; };
+    const int64_t wide = rounds(256) * 43000, middle = rounds(192) * 36000, square = rounds(128) * 27500;
     int64_t small = tiles(64, 64) * 8600 / 256 + 4000;
     if (small < 13000) small = 13000;
-    if (small <= wide && small <= square) return launch<2, 2, 1, 1>(a, stream);
-    return square < wide ? launch<4, 2, 1, 2>(a, stream) : launch<2, 4, 2, 2>(a, stream);
+    if (small <= wide && small <= middle && small <= square) return launch<2, 2, 1, 1>(a, stream);
+    if (square < wide && square <= middle) return launch<4, 2, 1, 2>(a, stream);
+    return middle < wide ? launch<4, 2, 1, 3>(a, stream) : launch<2, 4, 2, 2>(a, stream);
 }

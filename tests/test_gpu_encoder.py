@@ -63,6 +63,20 @@ def test_linear_keeps_scales_and_infinities(M):
     assert (((got[keep].double() - exact).abs() / exact.norm(dim=1, keepdim=True))[finite]).max() <= 1e-6
 
 
+# tiles of 128 x 192: whole rounds and a remainder of rows, a last tile of 124 and of one column, one and three matrices, one step of k
+@pytest.mark.parametrize("M,N,K,sets", [(6145, 768, 768, 1), (6145, 700, 32, 1), (6700, 577, 96, 1), (2103, 768, 64, 3)])
+def test_linear_in_tiles_of_192_columns(M, N, K, sets):
+    x, w, b = _randn(M, K), [_randn(N, K, seed=s) / K ** 0.5 for s in range(sets)], [_randn(N, seed=9 + s) for s in range(sets)]
+    w[-1][N - 1] *= 1e9                     # the rows of half a piece have scales of their own
+    x[M - 1, K - 1] = float("inf")
+    got = ops.linear(x, w, b, None)
+    for s in range(sets):
+        want = x.double().cpu() @ w[s].double().cpu().T + b[s].double().cpu()
+        assert _rel(got[s][:-1, :-1], want[:-1, :-1]) <= LINEAR_REL and _rel(got[s][:-1, -1], want[:-1, -1]) <= LINEAR_REL
+        assert torch.equal(got[s][-1].double().cpu(), want[-1])
+    assert torch.equal(got, ops.linear(x, w, b, None))
+
+
 def _exact_attention(q, k, v, mask):
     q, k, v = (t.double().cpu().permute(0, 2, 1, 3) for t in (q, k, v))
     bias = -1000 * (1 - mask.double().cpu()[:, None, None])
