@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 10
+#define LFFN_ABI_VERSION 11
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -811,6 +811,18 @@ int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float
  */
 int lffn_linear_f32(const float *x, const float *const *w, const float *const *bias, const float *residual,
                     float *const *out, int64_t sets, int64_t M, int64_t N, int64_t K, void *stream);
+
+/*
+ * lffn_linear_f32 of LayerNorm(x) over its rows (PL/layer.py:23-25 and the norm before them), without a
+ * residual: one launch norms the rows and splits them and the rows of every w into what the products read,
+ * the next forms the products.  norm_weight, norm_bias: [K] or NULL, 16-byte aligned.  K <= 2048.  workspace: 16-byte aligned,
+ * lffn_linear_norm_workspace_bytes (0: sizes that are not supported).  Below some 2000 rows the norm and
+ * lffn_linear_f32 by themselves are faster.
+ */
+int lffn_linear_norm_workspace_bytes(int64_t sets, int64_t M, int64_t N, int64_t K, int64_t *bytes);
+int lffn_linear_norm_f32(const float *x, const float *norm_weight, const float *norm_bias, float eps, const float *const *w,
+                         const float *const *bias, float *const *out, void *workspace, int64_t workspace_bytes,
+                         int64_t sets, int64_t M, int64_t N, int64_t K, void *stream);
 
 /*
  * out[b, i, h, :] = sum_j p_j v[b, j, h, :],  p = softmax_j(q[b, i, h, :] . k[b, j, h, :] / 8 - 1000 (1 - mask[b, j]))

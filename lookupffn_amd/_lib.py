@@ -16,7 +16,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # LOOKUPFFN_HIP_LIB points at another build of the same ABI (e.g. a tuning build)
 LIB_PATH = os.environ.get("LOOKUPFFN_HIP_LIB") or os.path.join(_PKG_DIR, "liblookupffn_hip.so")
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 LFFN_OK = 0
 LFFN_ERR_BAD_ARG = -1
@@ -110,6 +110,9 @@ SIGNATURES = {
     "lffn_bh4_fold_split_f32": [_vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "lffn_bh4_block_bwd_split_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp],
     "lffn_linear_f32": [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp, ctypes.POINTER(_vp), _i64, _i64, _i64, _i64, _vp],
+    "lffn_linear_norm_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)],
+    "lffn_linear_norm_f32": [_vp, _vp, _vp, ctypes.c_float, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp, _i64,
+                             _i64, _i64, _i64, _i64, _vp],
     "lffn_attention_f32": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "lffn_lookup_inner_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
 }

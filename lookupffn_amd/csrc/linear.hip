@@ -15,6 +15,13 @@
 // kilobyte, reads 4 to 7) and the splitting take as long as those beside them.  The library's fp32 product takes 426 us
 // (136 TFLOP/s, 0.87 of the fp32 matrix cores' peak).  Error against 64 bits 2.0e-7 of the result (library 5.0e-7; 16 rows, where
 // it splits k, 2.5e-7); as six products of three bfloat16 terms 1.6e-7, but 313 us.
+//
+// lffn_linear_norm_f32 takes the splitting out of the loop: a row of x is split for nine tiles, a row of w for 128, each time anew.
+// LayerNorm's kernel writes its rows split instead (split_rows_kernel), with the rows of every w beside them, and a tile's numbers go
+// into LDS as they come.  LayerNorm and the three matrices, us before -> now: 16384 x 768 254 -> 230, 32768 x 768 486 -> 434, 4096 x
+// 1024 124 -> 107, 16384 x 512 131 -> 118, 2103 x 768 43 -> 42, 1024 x 768 31 -> 31, 512 x 768 24 -> 31 (its form is the one with
+// tiles of 64 x 64 and no extra traffic for w): from 2048 rows on it is never slower.  Splitting w alone gives nothing, the launch
+// costs what it saves (16384 x 768: 233 -> 228, one matrix 82 -> 84).
 #include "split_mfma.h"
 
 
@@ -26,13 +33,111 @@ struct LinearArgs {
     const float *x;              // [M, K]
     const float *residual;       // [M, N] or null
     const float *w[3], *b[3];    // [N, K], [N] or null, of every set
+    const uint4 *split;          // rows of x and of every w by split_rows_kernel, [M + sets N][K / 8][hi, lo]
+    const float *split_inverse;  // [M + sets N]
     float *out[3];               // [M, N]
     int64_t M;
     int N, K, sets;
 };
 
-// WAVES_M x WAVES_N wavefronts of WM x WN tiles of 32 x 32 each.
-template <int WAVES_M, int WAVES_N, int WM, int WN>
+struct SplitArgs {
+    const float *x, *weight, *bias;      // [M, K], [K] or null: LayerNorm of the rows of x
+    const float *w[3];                   // [N, K]
+    uint4 *split;
+    float *inverse;
+    int64_t M, rows;                     // M + sets N
+    int N, K;
+    float eps;
+};
+
+__device__ __forceinline__ float wave_max(float v) {
+    v = fmaxf(v, lane_xor<1>(v));
+    v = fmaxf(v, lane_xor<2>(v));
+    v = fmaxf(v, lane_xor<4>(v));
+    v = fmaxf(v, lane_xor<8>(v));
+    v = fmaxf(v, lane_xor<16>(v));
+    return fmaxf(v, lane_xor<32>(v));
+}
+
+// Rows of LayerNorm(x) and of every w as the products want them, eight hi and eight lo in the place of eight numbers, scaled by a
+// power of two by their largest finite number.  A wavefront a row, NV x 16 bytes a lane; two lanes with the halves of eight numbers
+// exchange them, so that one stores the hi and the other the lo and a row is written as it is read.  One launch in the place of
+// LayerNorm's, 50 MB in and 50 out as that one (16384 x 768: 22 us with three matrices of 768 rows, PyTorch's LayerNorm 29).
+template <int NV>
+__global__ __launch_bounds__(256) void split_rows_kernel(SplitArgs a) {
+    const int lane = threadIdx.x & 63, quads = a.K >> 2;
+    const int64_t row = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (row >= a.rows) return;
+    const bool norm = row < a.M;
+    const int64_t wrow = row - a.M;
+    const float4 *const from = reinterpret_cast<const float4 *>(norm ? a.x + row * a.K : a.w[wrow / a.N] + wrow % a.N * a.K);
+    float v[NV][4];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int q = i * 64 + lane;
+        const float4 u = q < quads ? from[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[i][0] = u.x, v[i][1] = u.y, v[i][2] = u.z, v[i][3] = u.w;
+    }
+    if (norm) {
+        float sum = 0.f, squares = 0.f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+        const float mean = lane_group_sum<64>(sum) / a.K;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[i][e] -= mean;
+                if (i * 64 + lane < quads) squares = fmaf(v[i][e], v[i][e], squares);
+            }
+        const float factor = 1.f / sqrtf(lane_group_sum<64>(squares) / a.K + a.eps);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int q = i * 64 + lane;
+            const bool live = q < quads;
+            const float4 m = live && a.weight ? reinterpret_cast<const float4 *>(a.weight)[q] : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float4 b = live && a.bias ? reinterpret_cast<const float4 *>(a.bias)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[i][0] = fmaf(v[i][0] * factor, m.x, b.x);
+            v[i][1] = fmaf(v[i][1] * factor, m.y, b.y);
+            v[i][2] = fmaf(v[i][2] * factor, m.z, b.z);
+            v[i][3] = fmaf(v[i][3] * factor, m.w, b.w);
+        }
+    }
+    float most = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i * 64 + lane < quads && is_finite(v[i][e])) most = fmaxf(most, fabsf(v[i][e]));
+    const PowerOfTwo s = scale_to_one(wave_max(most));
+    uint4 *const to = a.split + row * quads;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int q = i * 64 + lane;                    // (quads is even: both lanes of a pair are in or neither)
+        const uint32_t h0 = split_hi(v[i][0], v[i][1], s.scale), h1 = split_hi(v[i][2], v[i][3], s.scale);
+        const uint32_t l0 = split_lo(v[i][0], v[i][1], s.scale, h0), l1 = split_lo(v[i][2], v[i][3], s.scale, h1);
+        const bool odd = lane & 1;
+        const uint32_t o0 = __float_as_uint(lane_xor<1>(__uint_as_float(odd ? h0 : l0)));
+        const uint32_t o1 = __float_as_uint(lane_xor<1>(__uint_as_float(odd ? h1 : l1)));
+        if (q < quads) to[q] = odd ? make_uint4(o0, o1, l0, l1) : make_uint4(h0, h1, o0, o1);
+    }
+    if (lane == 0) a.inverse[row] = s.inverse;
+}
+
+// Four numbers of eight that are split, hi at p and lo 16 bytes on, as they were but for the last bits.
+__device__ __forceinline__ float4 joined(const float *p, float inverse) {
+    const uint2 h = *reinterpret_cast<const uint2 *>(p), l = *reinterpret_cast<const uint2 *>(p + 4);
+    float y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float hi = __builtin_bit_cast(f16x2_t, e < 2 ? h.x : h.y)[e & 1], lo = __builtin_bit_cast(f16x2_t, e < 2 ? l.x : l.y)[e & 1];
+        y[e] = (is_finite(hi) ? fmaf(lo, 1 / SPLIT_LO, hi) : hi) * inverse;
+    }
+    return make_float4(y[0], y[1], y[2], y[3]);
+}
+
+// WAVES_M x WAVES_N wavefronts of WM x WN tiles of 32 x 32 each.  SPLIT: x and w come split.
+template <int WAVES_M, int WAVES_N, int WM, int WN, bool SPLIT>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(LinearArgs a) {
     constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N, THREADS = 64 * WAVES_M * WAVES_N;
     constexpr int BUF = 2 * (BM + BN) * 4;               // 16-byte pieces of a step's buffer
@@ -59,6 +164,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     // a thread's pieces of a step: eight numbers each of rows tid / 4 + RSTEP i, those of x before those of w
     const int chunk = tid & 3, row0 = tid >> 2;
     const float *const xa = a.x + m0 * K, *const wb = w + int64_t(n0) * K;
+    // (split or not, eight numbers are 32 bytes)
+    const float *const xf = SPLIT ? reinterpret_cast<const float *>(a.split) + m0 * K : xa;
+    const float *const wf = SPLIT ? reinterpret_cast<const float *>(a.split) + (M + int64_t(set) * N + n0) * K : wb;
     uint32_t src[NC];
     int dst[NC];
 #pragma unroll
@@ -86,7 +194,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     float v[NC][8], scale[NC];
     auto fetch = [&](int i, int k0) {
         const int k = min(k0, K - BK);                  // (beyond the end: the last step again, never used)
-        const float *const p = (RSTEP * i < BM ? xa : wb) + k;
+        const float *const p = (RSTEP * i < BM ? xf : wf) + k;
         *reinterpret_cast<float4 *>(&v[i][0]) = *reinterpret_cast<const float4 *>(p + src[i]);
         if (i < NP) *reinterpret_cast<float4 *>(&v[i][4]) = *reinterpret_cast<const float4 *>(p + src[i] + 4);
     };
@@ -94,6 +202,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     auto place = [&](uint4 *buf, int i, int p) {
         const int plane = (RSTEP * i < BM ? BM : BN) * 4;
         uint32_t o[4];
+        if (SPLIT) {                                    // it comes as it goes; of the half piece a thread has one term
+            const uint4 u = *reinterpret_cast<const uint4 *>(&v[i][i < NP ? 4 * p : 0]);
+            if (i < NP) buf[dst[i] + p * plane] = u;
+            else if (p == 0) buf[dst[i] + (tid & 1) * plane] = u;
+            return;
+        }
 #pragma unroll
         for (int e = 0; e < (i < NP ? 4 : 2); ++e) {
             if (p == 0) o[e] = h[e] = split_hi(v[i][2 * e], v[i][2 * e + 1], scale[i]);
@@ -117,6 +231,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     for (int i = 0; i < NC; ++i) fetch(i, 0);
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
+        if constexpr (SPLIT) {
+            const int row = i < NP ? row0 + RSTEP * i : RSTEP * NP + (tid >> 3);
+            if ((i < NP ? chunk : tid & 7) == 0)
+                inverse[row] = a.split_inverse[RSTEP * i < BM ? min(m0 + row, M - 1) : M + int64_t(set) * N + min(n0 + row - BM, N - 1)];
+            place(lds, i, 0);
+            place(lds, i, 1);
+            fetch(i, BK);
+            continue;
+        }
         float most = 0.f;
 #pragma unroll
         for (int e = 0; e < (i < NP ? 8 : 4); ++e) most = fmaxf(most, fabsf(v[i][e]));
@@ -218,11 +341,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
 #pragma unroll 1
         for (int t = 0; t < WM * WN; ++t) {
             const int n = wn * 32 * WN + t % WN * 32 + r, ml = wm * 32 * WM + t / WN * 32;
-            const float *pa = xa + uint32_t(min(ml + r, rows - 1)) * K + 4 * half, *pb = wb + uint32_t(min(n, cols - 1)) * K + 4 * half;
+            const float *pa = xf + uint32_t(min(ml + r, rows - 1)) * K + (SPLIT ? 2 : 4) * half, *pb = wb + uint32_t(min(n, cols - 1)) * K + 4 * half;
             f32x16_t y = {};
 #pragma unroll 2
             for (int k = 0; k < K; k += 8) {
-                const float4 u = *reinterpret_cast<const float4 *>(pa + k), z = *reinterpret_cast<const float4 *>(pb + k);
+                const float4 u = SPLIT ? joined(pa + k, inverse[ml + r]) : *reinterpret_cast<const float4 *>(pa + k), z = *reinterpret_cast<const float4 *>(pb + k);
                 y = __builtin_amdgcn_mfma_f32_32x32x2f32(u.x, z.x, y, 0, 0, 0);
                 y = __builtin_amdgcn_mfma_f32_32x32x2f32(u.y, z.y, y, 0, 0, 0);
                 y = __builtin_amdgcn_mfma_f32_32x32x2f32(u.z, z.z, y, 0, 0, 0);
@@ -238,16 +361,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     }
 }
 
-template <int WAVES_M, int WAVES_N, int WM, int WN>
+template <int WAVES_M, int WAVES_N, int WM, int WN, bool SPLIT>
 int launch(const LinearArgs &a, void *stream) {
     constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N;
     constexpr size_t lds = 3 * 2 * (BM + BN) * 64 + (BM + BN) * 4;
     static LdsGrant granted;
-    if (lds > 65536 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(&linear_kernel<WAVES_M, WAVES_N, WM, WN>), lds, granted))
+    if (lds > 65536 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(&linear_kernel<WAVES_M, WAVES_N, WM, WN, SPLIT>), lds, granted))
         return LFFN_ERR_LAUNCH;
     const int64_t tiles = (a.M + BM - 1) / BM * ((a.N + BN - 1) / BN) * a.sets;
     LFFN_REQUIRE(tiles <= INT32_MAX, LFFN_ERR_UNSUPPORTED);
-    linear_kernel<WAVES_M, WAVES_N, WM, WN><<<dim3(tiles), dim3(64 * WAVES_M * WAVES_N), lds, static_cast<hipStream_t>(stream)>>>(a);
+    linear_kernel<WAVES_M, WAVES_N, WM, WN, SPLIT><<<dim3(tiles), dim3(64 * WAVES_M * WAVES_N), lds, static_cast<hipStream_t>(stream)>>>(a);
     return lffn_launch_status();
 }
 
@@ -284,7 +407,58 @@ extern "C" int lffn_linear_f32(const float *x, const float *const *w, const floa
     const int64_t wide = rounds(256) * 43000, middle = rounds(192) * 36000, square = rounds(128) * 27500;
     int64_t small = tiles(64, 64) * 8600 / 256 + 4000;
     if (small < 13000) small = 13000;
-    if (small <= wide && small <= middle && small <= square) return launch<2, 2, 1, 1>(a, stream);
-    if (square < wide && square <= middle) return launch<4, 2, 1, 2>(a, stream);
-    return middle < wide ? launch<4, 2, 1, 3>(a, stream) : launch<2, 4, 2, 2>(a, stream);
+    if (small <= wide && small <= middle && small <= square) return launch<2, 2, 1, 1, false>(a, stream);
+    if (square < wide && square <= middle) return launch<4, 2, 1, 2, false>(a, stream);
+    return middle < wide ? launch<4, 2, 1, 3, false>(a, stream) : launch<2, 4, 2, 2, false>(a, stream);
+}
+
+extern "C" int lffn_linear_norm_workspace_bytes(int64_t sets, int64_t M, int64_t N, int64_t K, int64_t *bytes) {
+    LFFN_REQUIRE(bytes, LFFN_ERR_BAD_ARG);
+    const bool taken = sets >= 1 && sets <= 3 && M >= 0 && M <= INT64_C(1) << 32 && N >= 1 && N <= (1 << 20) && K >= BK && K <= 2048 && K % BK == 0;
+    *bytes = taken ? (M + sets * N) * (K + 1) * (int64_t)sizeof(float) : 0;
+    return LFFN_OK;
+}
+
+extern "C" int lffn_linear_norm_f32(const float *x, const float *norm_weight, const float *norm_bias, float eps, const float *const *w,
+                                    const float *const *bias, float *const *out, void *workspace, int64_t workspace_bytes, int64_t sets,
+                                    int64_t M, int64_t N, int64_t K, void *stream) {
+    LFFN_REQUIRE(x && w && bias && out, LFFN_ERR_BAD_ARG);
+    int64_t need = 0;
+    lffn_linear_norm_workspace_bytes(sets, M, N, K, &need);
+    LFFN_REQUIRE(need > 0, LFFN_ERR_UNSUPPORTED);
+    LFFN_REQUIRE(workspace && workspace_bytes >= need && lffn_aligned16(workspace), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(x) && lffn_aligned16(norm_weight) && lffn_aligned16(norm_bias), LFFN_ERR_BAD_ARG);
+    LinearArgs a{};
+    SplitArgs p{};
+    for (int64_t s = 0; s < sets; ++s) {
+        LFFN_REQUIRE(w[s] && out[s] && lffn_aligned16(w[s]), LFFN_ERR_BAD_ARG);
+        p.w[s] = a.w[s] = w[s];
+        a.b[s] = bias[s];
+        a.out[s] = out[s];
+    }
+    if (M == 0) return LFFN_OK;
+    p.x = x;
+    p.weight = norm_weight;
+    p.bias = norm_bias;
+    p.eps = eps;
+    a.split = p.split = static_cast<uint4 *>(workspace);
+    a.M = p.M = M;
+    p.rows = M + sets * N;
+    a.split_inverse = p.inverse = static_cast<float *>(workspace) + p.rows * K;
+    a.N = p.N = (int)N;
+    a.K = p.K = (int)K;
+    a.sets = (int)sets;
+    const dim3 grid((unsigned)((p.rows + 3) / 4)), block(256);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (K <= 256) split_rows_kernel<1><<<grid, block, 0, st>>>(p);
+    else if (K <= 512) split_rows_kernel<2><<<grid, block, 0, st>>>(p);
+    else if (K <= 768) split_rows_kernel<3><<<grid, block, 0, st>>>(p);
+    else if (K <= 1024) split_rows_kernel<4><<<grid, block, 0, st>>>(p);
+    else split_rows_kernel<8><<<grid, block, 0, st>>>(p);
+    if (const int rc = lffn_launch_status(); rc != LFFN_OK) return rc;
+    // as above, with the splitting out of the loop: a round of 128 x 256 40 us, of 128 x 192 32, of 128 x 128 23.5 (K = 768)
+    auto rounds = [&](int64_t bn) { return ((M + 127) / 128 * ((N + bn - 1) / bn) * sets + 255) / 256; };
+    const int64_t wide = rounds(256) * 40000, middle = rounds(192) * 32000, square = rounds(128) * 23500;
+    if (square < wide && square <= middle) return launch<4, 2, 1, 2, true>(a, stream);
+    return middle < wide ? launch<4, 2, 1, 3, true>(a, stream) : launch<2, 4, 2, 2, true>(a, stream);
 }

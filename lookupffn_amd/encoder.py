@@ -105,7 +105,7 @@ class Attention(nn.Module):
     def _kernels_apply(self, x, mask):
         """The products and the softmax go to this package's kernels (csrc/linear.hip, csrc/attention.hip): fp32 on the GPU without
         gradients, heads of 64 columns, and every part of the module the one it was built with.  Against the library's fp32
-        products and attention the encoder layer takes, 32 x 512 tokens of 768, 631 us instead of 1271, 4 x 128 tokens 86 instead of
+        products and attention the encoder layer takes, 32 x 512 tokens of 768, 619 us instead of 1279, 4 x 128 tokens 86 instead of
         164, 16 tokens 86 instead of 166, and its attention half is half as far from 64 bits (5e-7 against 9e-7)."""
         linears = (self.query, self.key, self.value, self.dense)
         if not (x.is_cuda and x.dim() == 3 and x.dtype == torch.float32 and x.numel() > 0 and type(x) in (torch.Tensor, nn.Parameter)
@@ -121,14 +121,26 @@ class Attention(nn.Module):
                          and (x.requires_grad or mask.requires_grad or any(p.requires_grad for p in self.parameters())))
                 and _nobody_watches())
 
+    def _norm_applies(self, x):
+        """The LayerNorm is the one the module was built with and there are rows enough that its kernel splits them, and the weights,
+        once for all tiles."""
+        norm, shape = self.LayerNorm, x.shape[2:]
+        return (x.shape[0] * x.shape[1] >= ops.LINEAR_NORM_MIN_ROWS and shape[0] <= ops.LINEAR_NORM_MAX_COLUMNS
+                and _plain(norm, nn.LayerNorm) and norm.normalized_shape == tuple(shape) and _kernel_operand(x, x.shape, x.device)
+                and all(p is None or _kernel_operand(p, shape, x.device) for p in (norm.weight, norm.bias)))
+
     def _forward_kernels(self, hidden_states, attention_mask, residual=None):
-        h = self.LayerNorm(hidden_states)
-        if not _kernel_operand(h, hidden_states.shape, hidden_states.device):        # another LayerNorm may return anything
-            out = self._attend(h, attention_mask)
-            return out if residual is None else out + residual
-        B, L, hidden = h.shape
-        q, k, v, dense = self.query, self.key, self.value, self.dense
-        qkv = ops.linear(h.view(B * L, hidden), (q.weight, k.weight, v.weight), (q.bias, k.bias, v.bias), None)
+        B, L, hidden = hidden_states.shape
+        q, k, v, dense, norm = self.query, self.key, self.value, self.dense, self.LayerNorm
+        weights, biases = (q.weight, k.weight, v.weight), (q.bias, k.bias, v.bias)
+        if self._norm_applies(hidden_states):
+            qkv = ops.linear_norm(hidden_states.view(B * L, hidden), norm.weight, norm.bias, float(norm.eps), weights, biases)
+        else:
+            h = norm(hidden_states)
+            if not _kernel_operand(h, hidden_states.shape, hidden_states.device):        # another LayerNorm may return anything
+                out = self._attend(h, attention_mask)
+                return out if residual is None else out + residual
+            qkv = ops.linear(h.view(B * L, hidden), weights, biases, None)
         qkv = qkv.view(3, B, L, self.num_attention_heads, 64)
         ctx = ops.attention(qkv[0], qkv[1], qkv[2], attention_mask.float().contiguous())
         if residual is not None:

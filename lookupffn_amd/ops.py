@@ -1187,6 +1187,42 @@ def _(x, w, bias, residual):
     return x.new_empty(len(w), x.shape[0], w[0].shape[0])
 
 
+LINEAR_NORM_MAX_COLUMNS = 2048  # a row is in a wavefront's registers
+LINEAR_NORM_MIN_ROWS = 2048     # below, splitting the weights beforehand costs more than it saves (1024 x 768: even; 512: 24 -> 31 us)
+
+_L.define("linear_norm(Tensor x, Tensor? norm_weight, Tensor? norm_bias, float eps, Tensor[] w, Tensor?[] bias) -> Tensor")
+
+
+def _linear_norm_impl(x, norm_weight, norm_bias, eps, w, bias):
+    """linear(LayerNorm(x), w, bias, None): x [M, K]; norm_weight, norm_bias: [K] or None."""
+    _lib.require_gpu(x, norm_weight, norm_bias, *w, *bias)
+    sets, (M, K), N = len(w), x.shape, w[0].shape[0]
+    assert 1 <= sets <= 3 and len(bias) == sets
+    for t in (x, *w, *(t for t in (norm_weight, norm_bias, *bias) if t is not None)):
+        assert t.dtype == torch.float32 and t.is_contiguous()
+    assert all(t.shape == (N, K) for t in w) and all(b is None or b.shape == (N,) for b in bias)
+    assert all(t is None or t.shape == (K,) for t in (norm_weight, norm_bias))
+    out = torch.empty(sets, M, N, dtype=torch.float32, device=x.device)
+    pointers = ctypes.c_void_p * sets
+    first = out.data_ptr()
+    with _dev_guard(x):
+        ws = _workspace(x.device, "lffn_linear_norm_workspace_bytes", sets, M, N, K)
+        rc = _lib.load().lffn_linear_norm_f32(
+            _lib.ptr(x), _lib.ptr(norm_weight), _lib.ptr(norm_bias), eps, pointers(*(t.data_ptr() for t in w)),
+            pointers(*(_lib.ptr(b) for b in bias)), pointers(*(first + 4 * s * M * N for s in range(sets))), _lib.ptr(ws),
+            0 if ws is None else ws.nbytes, sets, M, N, K, _lib.stream_of(x))
+    _lib.check(rc, f"lffn_linear_norm_f32(sets={sets}, M={M}, N={N}, K={K})")
+    return out
+
+
+_L.impl("linear_norm", _linear_norm_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::linear_norm")
+def _(x, norm_weight, norm_bias, eps, w, bias):
+    return x.new_empty(len(w), x.shape[0], w[0].shape[0])
+
+
 ATTENTION_MAX_KEYS = 2048       # LFFN_ATTENTION_MAX_KEYS
 
 _L.define("attention(Tensor q, Tensor k, Tensor v, Tensor mask) -> Tensor")
@@ -1245,4 +1281,5 @@ lookup_scatter = torch.ops.lookupffn.lookup_scatter
 lookup_backward = torch.ops.lookupffn.lookup_backward
 lookup_inner = torch.ops.lookupffn.lookup_inner
 linear = torch.ops.lookupffn.linear
+linear_norm = torch.ops.lookupffn.linear_norm
 attention = torch.ops.lookupffn.attention

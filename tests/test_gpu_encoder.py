@@ -77,6 +77,57 @@ def test_linear_in_tiles_of_192_columns(M, N, K, sets):
     assert torch.equal(got, ops.linear(x, w, b, None))
 
 
+# rows and columns around the tiles of 128, 192 and 256 columns (the last three: one size that gets each), K around the 256 numbers of a
+# wavefront's load, LayerNorm with and without weights
+@pytest.mark.parametrize("M,N,K,sets", [(1, 1, 32, 1), (129, 200, 288, 3), (300, 64, 2048, 2), (300, 130, 1056, 1), (127, 577, 736, 3),
+                                        (4000, 768, 768, 3), (8192, 512, 512, 1), (16333, 512, 512, 3)])
+def test_linear_of_a_norm(M, N, K, sets):
+    x, w, b = 3 * _randn(M, K) + 1, [_randn(N, K, seed=s) / K ** 0.5 for s in range(sets)], [_randn(N, seed=9 + s) for s in range(sets)]
+    x[M // 2] *= 1e6
+    w[-1][N - 1] *= 1e9                     # rows have scales of their own
+    nw, nb = (None, None) if M == 300 else (1 + 0.1 * _randn(K, seed=5), _randn(K, seed=6))
+    bias = [b[0], None, b[-1]][:sets]
+    got = ops.linear_norm(x, nw, nb, 1e-5, w, bias)
+    rows = sorted(set(torch.randperm(M)[:512].tolist() + [0, M // 2, M - 1]))
+    h = torch.nn.functional.layer_norm(x[rows].double().cpu(), (K,), *(t if t is None else t.double().cpu() for t in (nw, nb)), 1e-5)
+    for s in range(sets):
+        want = h @ w[s].double().cpu().T + (0 if bias[s] is None else bias[s].double().cpu())
+        # the norm's mean and variance are sums of K / 64 + 6 additions of 2^-24, either sign: 2^-22 beside the products' bound
+        last = [N - 1]
+        assert _rel(got[s][rows][:, last], want[:, last]) <= LINEAR_REL + 2.0 ** -22
+        assert N == 1 or _rel(got[s][rows][:, :-1], want[:, :-1]) <= LINEAR_REL + 2.0 ** -22
+    assert torch.equal(got, ops.linear_norm(x, nw, nb, 1e-5, w, bias))
+
+
+@pytest.mark.parametrize("M", [130, 4000])
+def test_linear_of_a_norm_keeps_infinities(M):
+    N = K = 768
+    x, w, nw, nb = _randn(M, K), _randn(N, K, seed=1), 1 + 0.1 * _randn(K, seed=5), _randn(K, seed=6)
+    x[3, 5], x[9, 1] = float("inf"), float("nan")
+    x[20] = 0                               # no variance
+    w[5, 9], w[7, 11] = float("inf"), float("nan")
+    w[8, :700] = 1e-30
+    want = torch.nn.functional.linear(torch.nn.functional.layer_norm(x, (K,), nw, nb), w).cpu()
+    got = ops.linear_norm(x, nw, nb, 1e-5, [w], [None])[0].cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isposinf(), want.isposinf())
+    assert torch.equal(got.isneginf(), want.isneginf())
+    finite = want.isfinite()
+    h = torch.nn.functional.layer_norm(x.double().cpu(), (K,), nw.double().cpu(), nb.double().cpu())
+    # of |h| |w|: 2^-22 for the split and for the norm, 2^-24 in each of 3 K / 16 instructions, either sign: 12 * 2^-24
+    bound = h.norm(dim=1, keepdim=True) * w.double().cpu().norm(dim=1) * (2 * 2.0 ** -22 + 12 * 2.0 ** -24)
+    assert ((got.double() - h @ w.double().cpu().T).abs() <= bound)[finite].all()
+    # infinities in the norm's own weights reach every product of their column
+    nw[40] = float("inf")
+    want = torch.nn.functional.linear(torch.nn.functional.layer_norm(x, (K,), nw, nb), w).cpu()
+    got = ops.linear_norm(x, nw, nb, 1e-5, [w], [None])[0].cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isposinf(), want.isposinf())
+    assert torch.equal(got.isneginf(), want.isneginf())
+    # equal numbers whose square fp32 does not hold: their variance is none (the library's is inf - inf)
+    x[:], nw[40] = 1e30, 1
+    got = ops.linear_norm(x, nw, nb, 1e-5, [w[9:]], [None])[0]
+    assert _rel(got, (nb.double().cpu() @ w[9:].double().cpu().T).expand(M, -1)) <= LINEAR_REL
+
+
 def _exact_attention(q, k, v, mask):
     q, k, v = (t.double().cpu().permute(0, 2, 1, 3) for t in (q, k, v))
     bias = -1000 * (1 - mask.double().cpu()[:, None, None])
@@ -129,6 +180,29 @@ def layer():
 def _by_library(layer, x, mask):
     att = layer.attention
     return layer.dropout(att._attend(att.LayerNorm(x), mask)) + x
+
+
+# another norm is called, the layer's own is not; either way the layer is what the library's products give
+@pytest.mark.parametrize("form", ["own", "hook", "subclass", "no weights", "too few rows"])
+def test_the_norm_in_the_products(layer, form, monkeypatch):
+    att = layer.attention
+    torch.nn.init.normal_(att.LayerNorm.weight, 1, 0.1)
+    rows = 40 if form == "too few rows" else 600
+    x, mask = _randn(4, rows, 256), torch.ones(4, rows, device=DEV)
+    norms, calls = [], []
+    if form == "hook":
+        att.LayerNorm.register_forward_hook(lambda *a: norms.append(1))
+    if form == "subclass":
+        forward = lambda self, h: norms.append(1) or 2 * torch.nn.LayerNorm.forward(self, h)
+        att.LayerNorm = type("Norm", (torch.nn.LayerNorm,), {"forward": forward})(256).to(DEV)
+    if form == "no weights":
+        att.LayerNorm = torch.nn.LayerNorm(256, eps=1e-3, elementwise_affine=False)
+    monkeypatch.setattr(encoder.ops, "linear_norm", lambda *a: calls.append(1) or torch.ops.lookupffn.linear_norm(*a))
+    with torch.no_grad():
+        got = att(x, mask)
+        assert bool(calls) == (form in ("own", "no weights")) and bool(norms) == (form in ("hook", "subclass"))
+        want = att._attend(att.LayerNorm(x), mask)
+    assert _rel(got, want.double().cpu()) <= 1e-6
 
 
 @pytest.mark.parametrize("form", ["plain", "strided", "bool mask", "half mask", "strided mask", "no bias", "one token", "zero dropout"])
