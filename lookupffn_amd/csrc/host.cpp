@@ -55,6 +55,8 @@ using torch::autograd::variable_list;
     X(lffn_lookup_gather_ws_bf16)           \
     X(lffn_lookup_gather_ws_f16)            \
     X(lffn_ln_bh4_block_hash_train_f32)     \
+    X(lffn_ln_bh4_block_hash_f32)           \
+    X(lffn_ln_bh4_block_hash_records_f32)   \
     X(lffn_bh4_block_front_split_f32)       \
     X(lffn_bh4_fold_split_f32)              \
     X(lffn_bh4_fold_mode_f32)               \
@@ -109,10 +111,11 @@ struct Parts {
     std::array<PyObject *, 6> params;
     double eps, decay;
     int64_t num_table, output_size;
+    bool training;                       // the hash's train() or eval()
 };
 
 PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES, *KEY_EPS,
-    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_SPLIT;      // interned
+    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_FOLDED, *KEY_SPLIT, *KEY_TRAINING;      // interned
 
 PyObject *dict_of(PyObject *o) {
     PyObject **d = o ? _PyObject_GetDictPtr(o) : nullptr;
@@ -154,7 +157,9 @@ bool find_parts(PyObject *layer, Parts &found) {
                     item(of_projection, KEY_BIAS), item(of_layer, KEY_TABLES), item(of_layer, KEY_BIAS)};
     for (PyObject *o : found.params)
         if (!o || !THPVariable_Check(o)) return false;
-    return number(item(norm, KEY_EPS), found.eps) && number(item(projection, KEY_DECAY), found.decay) &&
+    PyObject *mode = item(hash, KEY_TRAINING);
+    found.training = mode == Py_True;
+    return (found.training || mode == Py_False) && number(item(norm, KEY_EPS), found.eps) && number(item(projection, KEY_DECAY), found.decay) &&
            whole(item(own, KEY_NUM_TABLE), found.num_table) && whole(item(own, KEY_OUTPUT_SIZE), found.output_size);
 }
 
@@ -238,8 +243,10 @@ lffn_block_front block_front(const Config &c, const Params &p, const Tensor &spl
 // Floats of the split weights (lffn_bh4_fold_split_f32).
 int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 4); }
 
-void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &x, const float *residual, Tensor &out, int64_t B,
-           int64_t fused_max) {
+// as_training: 64 x 64 blocks go through the training forward's kernel (block_weight: folded), so that a module in train() computes the
+// same codes with and without gradients (a checkpointed pass runs both); else through the faster one of inference (block_weight: split).
+void infer(const Config &c, const Params &p, const Tensor &block_weight, bool as_training, const Tensor &x, const float *residual,
+           Tensor &out, int64_t B, int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     // Rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half as many tokens
@@ -262,8 +269,11 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
         if (c.form == DIAG)
             CALL(lffn_ln_project_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, decay, res, st);
+        else if (as_training)
+            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(block_weight), f32(p[3]), rp, plan.stride,
+                 plan.tokens, B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
         else {
-            lffn_block_front front = block_front(c, p, split);
+            lffn_block_front front = block_front(c, p, block_weight);
             front.records = rp;
             front.record_stride = plan.stride;
             front.tokens_per_workgroup = plan.tokens;
@@ -282,8 +292,11 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
     if (c.form == DIAG)
         CALL(lffn_ln_project_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), nullptr, cp, f32(scores), B, c.H,
              c.D, c.R, c.J, c.T, decay, res, st);
+    else if (as_training)
+        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(block_weight), f32(p[3]), cp, f32(scores), B, c.H, c.D,
+             c.R, c.J, c.T, 64, decay, res, st);
     else {
-        lffn_block_front front = block_front(c, p, split);
+        lffn_block_front front = block_front(c, p, block_weight);
         front.codes = cp;
         front.scores = f32(scores);
         CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
@@ -553,17 +566,17 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._split = ((version, address, device), split weights, what they were made from), as Hashing.split_weight keeps them: the
-// split weights if they are w's.
-Tensor split_of(PyObject *hash, const Tensor &w, int64_t words) {
-    PyObject *kept = item(dict_of(hash), KEY_SPLIT);
+// hash._folded or hash._split = ((version, address, device), folded or split weights, what they were made from), as
+// Hashing.block_weight keeps them: those weights if they are w's.
+Tensor weight_of(PyObject *hash, PyObject *name, const Tensor &w, int64_t words) {
+    PyObject *kept = item(dict_of(hash), name);
     if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3) return {};
-    PyObject *key = PyTuple_GET_ITEM(kept, 0), *split = PyTuple_GET_ITEM(kept, 1);
+    PyObject *key = PyTuple_GET_ITEM(kept, 0), *made = PyTuple_GET_ITEM(kept, 1);
     int64_t version = 0, address = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
-        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(split))
+        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(made))
         return {};
-    const Tensor &f = THPVariable_Unpack(split);
+    const Tensor &f = THPVariable_Unpack(made);
     const bool same = w._version() == (uint32_t)version && w.data_ptr() == reinterpret_cast<void *>(address) && f.device() == w.device() &&
                       f.numel() == words;
     return same ? f : Tensor();
@@ -576,7 +589,7 @@ struct WithoutInterpreter {
 };
 
 // forward(layer, x, residual or None, tokens up to which the one-launch form is taken) -> a tensor; None: not for this path;
-// False: the split weights (Hashing.split_weight) are not up to date
+// False: the blocks' weights (Hashing.block_weight) are not up to date
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 4, "forward: 4 arguments");
@@ -612,13 +625,17 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         for (const Tensor &t : params) grads = grads || t.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;
-    Tensor split;
-    if (!grads && c.form == BLOCK && !(split = split_of(parts.hash, params[2], split_words(c))).defined()) Py_RETURN_FALSE;
+    Tensor block_weight;
+    if (!grads && c.form == BLOCK) {
+        block_weight = parts.training ? weight_of(parts.hash, KEY_FOLDED, params[2], params[2].numel())
+                                      : weight_of(parts.hash, KEY_SPLIT, params[2], split_words(c));
+        if (!block_weight.defined()) Py_RETURN_FALSE;
+    }
     const int64_t fused_max = PyLong_AsLongLong(args[3]);
     if (fused_max == -1 && PyErr_Occurred()) return nullptr;
     Tensor out;
     {
-        // (from here on only what is owned here is used: x, the residual, the parameters and the split weights)
+        // (from here on only what is owned here is used: x, the residual, the parameters and the blocks' weights)
         const WithoutInterpreter unlocked;
         // any layout of x and any shape and type of the residual, as the Python path makes them
         x = x.contiguous();
@@ -628,7 +645,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
             (!residual.defined() || reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0)) {
             out = empty_f32(sizes, dev);
             if (grads) train(c, params, x, residual, out, B);
-            else infer(c, params, split, x, f32(residual), out, B, fused_max);
+            else infer(c, params, block_weight, parts.training, x, f32(residual), out, B, fused_max);
         }
     }
     if (!out.defined()) Py_RETURN_NONE;
@@ -651,7 +668,7 @@ PyMODINIT_FUNC PyInit__host() {
         {&KEY_MODULES, "_modules"}, {&KEY_PARAMETERS, "_parameters"}, {&KEY_LAYER_NORM, "LayerNorm"}, {&KEY_HASH, "hash"},
         {&KEY_PROJECTION, "projection"}, {&KEY_WEIGHT, "weight"}, {&KEY_BIAS, "bias"}, {&KEY_TABLES, "tables"},
         {&KEY_EPS, "eps"}, {&KEY_DECAY, "decay_coeff"}, {&KEY_NUM_TABLE, "num_table"},
-        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_SPLIT, "_split"},
+        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_FOLDED, "_folded"}, {&KEY_SPLIT, "_split"}, {&KEY_TRAINING, "training"},
     };
     for (const auto &[key, name] : keys)
         if (!(*key = PyUnicode_InternFromString(name))) return nullptr;

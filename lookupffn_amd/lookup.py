@@ -173,8 +173,8 @@ class Hashing(nn.Module):
         return code, score
 
     def can_fuse_block(self, x):
-        """Two kernels for 64 x 64 blocks without gradient: all BH4 stages on the matrix
-        cores, then mix + bias + code + score."""
+        """64 x 64 blocks without gradient: all BH4 stages on the matrix cores, mix + bias + code + score
+        in the same kernel for 8-bit codes (forward_block)."""
         p = self.projection
         needs_grad = torch.is_grad_enabled() and (
             x.requires_grad or any(q.requires_grad for q in self.parameters()))
@@ -193,8 +193,12 @@ class Hashing(nn.Module):
         return self._kept("_folded", ops.bh4_fold)
 
     def split_weight(self):
-        """folded_weight() as the block kernels multiply it (ops.bh4_fold_split), kept in the same way."""
+        """folded_weight() as the inference kernel multiplies it (ops.bh4_fold_split), kept in the same way."""
         return self._kept("_split", lambda w: ops.bh4_fold_split(w, False))
+
+    def block_weight(self):
+        """What forward_block's kernel for 8-bit codes takes in this mode."""
+        return self.folded_weight() if self.training else self.split_weight()
 
     def _kept(self, name, make):
         w = self.projection.weight
@@ -223,13 +227,20 @@ class Hashing(nn.Module):
 
     def forward_block(self, x, layer_norm=None):
         """8-bit codes: one kernel, (LayerNorm ->) BH4 on the matrix cores -> mix -> bias ->
-        code + score.  Other code lengths: the BH4 kernel, then mix + hash in a second one."""
+        code + score.  In eval() on the fp16 matrix cores; in train() the kernel of the training
+        forward, whose codes are the same bit for bit: a value within rounding of zero takes either
+        sign, and what a module in train() computes must not depend on whether gradients are recorded
+        (a checkpointed pass runs once without and once with them).  Other code lengths: the BH4
+        kernel, then mix + hash in a second one."""
         p = self.projection
         x = x.contiguous()
         if self.code_length == 8:
             lw = None if layer_norm is None else layer_norm.weight
             lb = None if layer_norm is None else layer_norm.bias
             eps = 0.0 if layer_norm is None else float(layer_norm.eps)
+            if self.training:
+                return ops.ln_bh4_block_hash(x, lw, lb, eps, self.folded_weight(), p.bias, self.num_table,
+                                             float(p.decay_coeff), float(1 - p.decay_coeff))
             return ops.bh4_block_front(x, lw, lb, eps, self.split_weight(), p.num_repeat, p.weight.shape[1], p.padded_in_dim, p.bias,
                                        self.num_table, float(p.decay_coeff), float(1 - p.decay_coeff))
         if layer_norm is not None:
@@ -425,7 +436,7 @@ class LookupFFN(nn.Module):
             return None
         out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         if out is False:                  # the 64 x 64 blocks have changed since they were folded
-            self.hash.split_weight()
+            self.hash.block_weight()
             out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         return None if out is False else out
 

@@ -1,0 +1,59 @@
+"""A module in train() computes the same whether gradients are recorded or not."""
+import math
+from argparse import Namespace
+
+import pytest
+import torch
+from torch.utils.checkpoint import checkpoint
+
+import lookupffn_amd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _layer(hidden, tables, block, out, training=True):
+    torch.manual_seed(hidden + tables)
+    cfg = Namespace(hidden_size=hidden, ffn_num_table=tables, ffn_table_size=256, layer_norm_eps=1e-5, projection_type="bh4", block_size=block)
+    layer = lookupffn_amd.LookupFFN(cfg, out).to(DEV).train(training)
+    with torch.no_grad():
+        layer.hash.projection.bias.normal_(std=0.05)
+        if block == 1:
+            layer.hash.projection.weight.copy_(layer.hash.projection.weight.sign() / math.sqrt(layer.hash.projection.padded_in_dim))
+    return layer
+
+
+def _same_rows(a, b):
+    # sums over the tables in another order, either sign: 1e-6 of the results' size; another table row moves one by some 0.1
+    return (a - b).abs().max().item() <= 1e-5 * b.pow(2).mean().sqrt().item()
+
+
+# every form of the fp32 block kernel and of the diagonal one: few and many workgroups, one and several repeats, short rows.  The last
+# size has 17 million projected values, a few of them within rounding of zero.
+@pytest.mark.parametrize("tokens,hidden,tables,block", [(17, 256, 128, 64), (300, 512, 64, 64), (2103, 500, 128, 64), (3000, 1024, 32, 64),
+                                                        (65, 64, 32, 64), (40, 256, 32, 1), (1500, 768, 128, 1), (16384, 512, 128, 64)])
+def test_a_layer_in_train_with_and_without_gradients(tokens, hidden, tables, block):
+    layer = _layer(hidden, tables, block, 64)
+    x = torch.randn(tokens, hidden, device=DEV)
+    code, score = layer.hash(x)
+    out = layer(x)
+    assert score.requires_grad and out.requires_grad
+    with torch.no_grad():
+        plain = layer.hash(x)
+        assert torch.equal(code, plain[0]) and torch.equal(score, plain[1])
+        assert _same_rows(layer(x), out)
+        assert _same_rows(layer._forward_operators(x, None), out)
+    again = checkpoint(layer, x.clone().requires_grad_(), use_reentrant=True)
+    assert again.requires_grad and _same_rows(again, out)
+
+
+@pytest.mark.parametrize("training", [True, False])
+def test_the_blocks_weights_are_those_of_the_mode(training):
+    layer = _layer(256, 32, 64, 64, training)
+    x = torch.randn(50, 256, device=DEV)
+    with torch.no_grad():
+        for change in (lambda: None, lambda: layer.hash.projection.weight.mul_(1.5), lambda: layer.train(not training).train(training)):
+            change()
+            assert _same_rows(layer(x), layer._forward_operators(x, None))
+            kept = layer.hash.__dict__.get("_folded" if training else "_split")
+            assert kept is not None and kept[1] is layer.hash.block_weight()
