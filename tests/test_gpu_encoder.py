@@ -205,7 +205,7 @@ def test_the_norm_in_the_products(layer, form, monkeypatch):
     assert _rel(got, want.double().cpu()) <= 1e-6
 
 
-@pytest.mark.parametrize("form", ["plain", "strided", "bool mask", "half mask", "strided mask", "no bias", "one token", "zero dropout"])
+@pytest.mark.parametrize("form", ["plain", "strided", "bool mask", "half mask", "strided mask", "no bias", "one token"])
 def test_the_kernels_agree_with_the_library_path(layer, form, monkeypatch):
     x, mask = _randn(3, 77, 256), (torch.arange(77, device=DEV)[None] < torch.tensor([[77], [50], [39]], device=DEV)).float()
     if form == "strided":
@@ -220,9 +220,6 @@ def test_the_kernels_agree_with_the_library_path(layer, form, monkeypatch):
         layer.attention.key.bias = None
     if form == "one token":
         x, mask = x[:1, :1], mask[:1, :1]
-    if form == "zero dropout":
-        layer.train()
-        layer.dropout.p = layer.attention.dropout.p = 0.0
     calls = []
     monkeypatch.setattr(encoder.ops, "attention", lambda *a: calls.append(1) or torch.ops.lookupffn.attention(*a))
     with torch.no_grad():
@@ -235,7 +232,7 @@ def test_the_kernels_agree_with_the_library_path(layer, form, monkeypatch):
 
 
 @pytest.mark.parametrize("form", ["hook", "pre-hook", "global hook", "other linear", "own forward", "own attention", "subclass", "gradient", "autocast",
-                                  "dropout", "double", "heads", "wide mask", "vmap", "tangent", "misaligned"])
+                                  "dropout", "train", "double", "heads", "wide mask", "vmap", "tangent", "misaligned"])
 def test_other_calls_keep_the_library_path(layer, form, monkeypatch):
     calls, seen = [], []
     monkeypatch.setattr(encoder.ops, "attention", lambda *a: calls.append(1) or torch.ops.lookupffn.attention(*a))
@@ -274,6 +271,10 @@ def test_other_calls_keep_the_library_path(layer, form, monkeypatch):
         layer.requires_grad_(False)
     if form == "dropout":
         layer.train()
+    if form == "train":                     # (as with gradients)
+        layer.train()
+        layer.dropout.p = layer.attention.dropout.p = 0.0
+        run = lambda: layer._attention_and_residual(x, mask)
     if form == "double":
         att.double()
         x = x.double()
@@ -303,7 +304,7 @@ def test_other_calls_keep_the_library_path(layer, form, monkeypatch):
         if handle is not None:
             handle.remove()
     assert not calls
-    assert seen or form in ("gradient", "autocast", "dropout", "double", "heads", "wide mask", "vmap", "tangent", "misaligned")
+    assert seen or form in ("gradient", "autocast", "dropout", "train", "double", "heads", "wide mask", "vmap", "tangent", "misaligned")
 
 
 def test_encoder_layer_in_a_graph(layer):

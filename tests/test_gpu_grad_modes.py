@@ -57,3 +57,18 @@ def test_the_blocks_weights_are_those_of_the_mode(training):
             assert _same_rows(layer(x), layer._forward_operators(x, None))
             kept = layer.hash.__dict__.get("_folded" if training else "_split")
             assert kept is not None and kept[1] is layer.hash.block_weight()
+
+
+def test_an_encoder_layer_in_train_with_and_without_gradients():
+    torch.manual_seed(1)
+    cfg = Namespace(hidden_size=256, num_attention_heads=4, attention_head_size=64, attention_probs_dropout_prob=0.0, hidden_dropout_prob=0.0,
+                    layer_norm_eps=1e-5, ffn_num_table=64, ffn_table_size=256, projection_type="bh4", block_size=1)
+    layer = lookupffn_amd.EncoderLayer(cfg).to(DEV).train()
+    x, mask = torch.randn(8, 300, 256, device=DEV), torch.ones(8, 300, device=DEV)
+    mask[3, 200:] = 0
+    half, out = layer.attention(x, mask), layer(x, mask)
+    with torch.no_grad():
+        assert torch.equal(layer.attention(x, mask), half)
+        assert _same_rows(layer(x, mask), out)
+    again = checkpoint(layer, x.clone().requires_grad_(), mask, use_reentrant=True)
+    assert again.requires_grad and _same_rows(again, out)
