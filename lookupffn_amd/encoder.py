@@ -23,11 +23,13 @@ from . import ops
 from .lookup import LookupFFN
 
 _GLOBAL_HOOKS = torch.nn.modules.module
+_FORWARDS = {kind: kind.forward for kind in (nn.Linear, nn.LayerNorm, nn.Dropout)}       # (and Attention, below)
 
 
 def _plain(module, kind):
-    """module is a `kind` itself and nothing watches its calls: what it computes may be computed without calling it."""
-    return (type(module) is kind and "forward" not in module.__dict__
+    """module is a `kind` itself, the class as it was written, and nothing watches its calls: what it computes may be computed
+    without calling it."""
+    return (type(module) is kind and "forward" not in module.__dict__ and kind.forward is _FORWARDS[kind]
             and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks))
 
 
@@ -112,7 +114,7 @@ class Attention(nn.Module):
         linears = (self.query, self.key, self.value, self.dense)
         if not (x.is_cuda and x.dim() == 3 and x.dtype == torch.float32 and x.numel() > 0 and type(x) in (torch.Tensor, nn.Parameter)
                 and self.fused and not self.training and type(self) is Attention
-                and not {"attention", "transpose_for_scores"} & self.__dict__.keys()):
+                and not any(name in self.__dict__ or getattr(Attention, name) is not method for name, method in _OWN_METHODS)):
             return False
         hidden = x.shape[2]
         return (self.attention_head_size == 64 and self.all_head_size == hidden and x.shape[1] <= ops.ATTENTION_MAX_KEYS
@@ -164,6 +166,11 @@ class Attention(nn.Module):
         if self._kernels_apply(hidden_states, attention_mask):
             return self._forward_kernels(hidden_states, attention_mask)
         return self._attend(self.LayerNorm(hidden_states), attention_mask)
+
+
+# What the kernels stand in for: a class or a module with another one has it called.
+_FORWARDS[Attention] = Attention.forward
+_OWN_METHODS = tuple((name, getattr(Attention, name)) for name in ("attention", "transpose_for_scores", "_attend"))
 
 
 class EncoderLayer(nn.Module):
