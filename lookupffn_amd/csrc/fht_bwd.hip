@@ -36,6 +36,16 @@ struct Tile {
     static_assert(LOGD >= 8 && LOGD <= 10, "256, 512 and 1024 points");
 };
 
+// exp(-2 a), a >= 0: the instruction's 2^t with what rounding takes from t = -2 a log2 e put back to first order (t grows with a, and a
+// rounded t alone is off by 9e-7 of the result at a = 8).  Beyond 128 the result is 0; there a is held, so that no infinity meets it.
+// (84 -> 86 us of the kernel; expf 89.  Gradients of z of 0.5 to 3: rms error 1.45e-7 -> 1.39e-7.)
+__device__ __forceinline__ float exp_minus_twice(float a) {
+    constexpr float C = -2.885390081777927f, C_REST = float(-2.8853900817779268 - double(C)), LN2 = 0.6931471805599453f;
+    a = fminf(a, 128.f);
+    const float t = a * C, rest = fmaf(a, C_REST, fmaf(a, C, -t)), e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e * LN2, rest, e);
+}
+
 __device__ __forceinline__ uint32_t max_u32(uint32_t a, uint32_t b) { return a > b ? a : b; }
 __device__ __forceinline__ uint32_t magnitude(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
 
@@ -305,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void project_hash_bwd_mfma_kernel(ProjectBw
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const float az = fabsf(z[4 * q + c]);
-                ez[c] = exp_minus_2a(az);
+                ez[c] = exp_minus_twice(az);
                 sum += az;
                 product *= 1.0f + ez[c];
             }

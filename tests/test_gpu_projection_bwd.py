@@ -95,3 +95,25 @@ def test_sizes_and_rows_of_their_own(D):
     want = _reference(x, diag, z, g)[0]
     for i in (4, 9):
         assert ((got.view(41, D)[i].double() - want[i]).norm() / want[i].norm()).item() <= REL
+
+
+@pytest.mark.parametrize("D", [256, 512, 1024])
+def test_the_scores_gradient_far_from_zero(D):
+    """One small value beside seven large ones: its gradient is exp(-2 |z|) times their sum, as exact far from zero as near it."""
+    B, T = 400, D // 8
+    x, diag, _, g_score, _, _ = _inputs(B, D, D, 1, T)
+    gen = torch.Generator(device=DEV).manual_seed(D)
+    z = torch.full((B, T, 8), 1e14, device=DEV)
+    z[:, :, 3] = (0.5 + 14.5 * torch.rand(B, T, generator=gen, device=DEV)) * torch.randn(B, T, generator=gen, device=DEV).sign()
+    z[z == 0] = 1.0
+    g_x, _, _ = ops.project_hash_bwd(x, diag, z.view(B, T * 8), g_score, 0.0, 1.0)          # the gradient of z itself
+    got, z3 = g_x.view(B, T, 8)[:, :, 3].double(), z[:, :, 3].double()
+    e = torch.exp(-2 * z3.abs())
+    want = z3.sign() * (1 + 2 * (7 * z[0, 0, 0].double() + z3.abs()) * e / (1 + e)) * (g_score.double() / (1 + e))
+    # an ulp (2^-23) each for 2^t and the reciprocal, half of one for its correction, 1 + e twice, e / (1 + e), the sum's two last
+    # additions, its product, 1 + it, the division and the last product: at most 2 * 2^-23 + 10 * 2^-24
+    assert ((got - want) / want).abs().max() <= 14 * 2.0 ** -24
+    # infinities, NaN and a sum beyond fp32 stay in their own row (a transform takes them through it)
+    z[5, 7, 2], z[6, 1, 4], z[8, 0] = float("inf"), float("nan"), 3e38
+    finite = torch.isfinite(ops.project_hash_bwd(x, diag, z.view(B, T * 8), g_score, 0.0, 1.0)[0].view(B, D)).all(-1)
+    assert (~finite).nonzero().flatten().tolist() == [5, 6, 8]
