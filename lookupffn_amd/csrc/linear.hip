@@ -7,8 +7,11 @@
 // step's products need one barrier and its first operands are there when it starts.  The products, the splitting and the LDS
 // traffic are spread through each other by scheduling groups: a matrix instruction covers five vector ones.
 //
-// Every row of x and w is scaled by a power of two of its own, taken from its first 32 numbers, and the results are scaled back:
-// any size of numbers goes, and a row that grows past its beginning 30000 times comes out infinite and is done again in fp32.
+// Every row of x and w is scaled by a power of two of its own and the results are scaled back: any size of numbers goes.  The scale comes
+// from 32 numbers spread over the row.  A tile with a row that is 128 times larger elsewhere comes out infinite and is done once more with
+// the scales of the rows' largest numbers; what is not finite then, a third time in fp32, for which infinities and NaN are numbers like
+// others.  16384 x 768 x 768 with a residual, us: 84, where every row outgrows its sample 208, with an infinity in every tile 470.  (The
+// largest numbers looked for beforehand, one more pass over the rows for every tile: 97; 16 rows 13 -> 16, with the sample 13.)
 //
 // What bounds it: power.  16384 x 768 x 768, three matrices: 222 us, 261 TFLOP/s of fp32 product (783 of fp16) at 1.67 GHz; with
 // zeros for numbers the same kernel runs at 2.37 GHz, 194 us.  Of its clocks 62 % are matrix instructions; LDS (writes 13 clocks per
@@ -34,7 +37,7 @@ struct LinearArgs {
     const float *residual;       // [M, N] or null
     const float *w[3], *b[3];    // [N, K], [N] or null, of every set
     const uint4 *split;          // rows of x and of every w by split_rows_kernel, [M + sets N][K / 8][hi, lo]
-    const float *split_inverse;  // [M + sets N]
+    const int *split_exponent;   // [M + sets N]
     float *out[3];               // [M, N]
     int64_t M;
     int N, K, sets;
@@ -44,11 +47,23 @@ struct SplitArgs {
     const float *x, *weight, *bias;      // [M, K], [K] or null: LayerNorm of the rows of x
     const float *w[3];                   // [N, K]
     uint4 *split;
-    float *inverse;
+    int *exponent;
     int64_t M, rows;                     // M + sets N
     int N, K;
     float eps;
 };
+
+// A row's scale: its largest number, or that of a sample of it, to [2^top, 2^(top + 1)); the way back is added to the results'
+// exponents.  A number is then held to 22 bits down to 2^-(14 + top) of that largest one and a smaller one to 2^-(36 + top) of it.
+// A row of zeros, or of less than 2^-103, is scaled as one of 2^-103, so that a sample of zeros hides no small numbers behind it: they
+// outgrow it.
+constexpr int TOP = 13;             // the row's largest number: lo, times 2048, stays below 2^13
+constexpr int TOP_OF_SAMPLE = 8;    // a sample's, which the row may outgrow 128 times
+__device__ __forceinline__ float row_scale(float most, int top, int &exponent) {
+    const int bits = __float_as_uint(most) >> 23, e = bits == 255 ? 127 : max(bits, 24);     // (times 2048 still a number)
+    exponent = e - 127 - top;
+    return __uint_as_float((254 - e + top) << 23);
+}
 
 __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, lane_xor<1>(v));
@@ -109,29 +124,30 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (i * 64 + lane < quads && is_finite(v[i][e])) most = fmaxf(most, fabsf(v[i][e]));
-    const PowerOfTwo s = scale_to_one(wave_max(most));
+    int exponent;
+    const float scale = row_scale(wave_max(most), TOP, exponent);
     uint4 *const to = a.split + row * quads;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int q = i * 64 + lane;                    // (quads is even: both lanes of a pair are in or neither)
-        const uint32_t h0 = split_hi(v[i][0], v[i][1], s.scale), h1 = split_hi(v[i][2], v[i][3], s.scale);
-        const uint32_t l0 = split_lo(v[i][0], v[i][1], s.scale, h0), l1 = split_lo(v[i][2], v[i][3], s.scale, h1);
+        const uint32_t h0 = split_hi(v[i][0], v[i][1], scale), h1 = split_hi(v[i][2], v[i][3], scale);
+        const uint32_t l0 = split_lo(v[i][0], v[i][1], scale, h0), l1 = split_lo(v[i][2], v[i][3], scale, h1);
         const bool odd = lane & 1;
         const uint32_t o0 = __float_as_uint(lane_xor<1>(__uint_as_float(odd ? h0 : l0)));
         const uint32_t o1 = __float_as_uint(lane_xor<1>(__uint_as_float(odd ? h1 : l1)));
         if (q < quads) to[q] = odd ? make_uint4(o0, o1, l0, l1) : make_uint4(h0, h1, o0, o1);
     }
-    if (lane == 0) a.inverse[row] = s.inverse;
+    if (lane == 0) a.exponent[row] = exponent;
 }
 
 // Four numbers of eight that are split, hi at p and lo 16 bytes on, as they were but for the last bits.
-__device__ __forceinline__ float4 joined(const float *p, float inverse) {
+__device__ __forceinline__ float4 joined(const float *p, int exponent) {
     const uint2 h = *reinterpret_cast<const uint2 *>(p), l = *reinterpret_cast<const uint2 *>(p + 4);
     float y[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const float hi = __builtin_bit_cast(f16x2_t, e < 2 ? h.x : h.y)[e & 1], lo = __builtin_bit_cast(f16x2_t, e < 2 ? l.x : l.y)[e & 1];
-        y[e] = (is_finite(hi) ? fmaf(lo, 1 / SPLIT_LO, hi) : hi) * inverse;
+        y[e] = __builtin_amdgcn_ldexpf(is_finite(hi) ? fmaf(lo, 1 / SPLIT_LO, hi) : hi, exponent);
     }
     return make_float4(y[0], y[1], y[2], y[3]);
 }
@@ -148,9 +164,8 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     constexpr int NR = 2 * (WM + WN);                    // fragments of half a step
     static_assert(BM % RSTEP == 0 && (BN % RSTEP == 0 || BN % RSTEP == RSTEP / 2) && NC <= 3);
     extern __shared__ __attribute__((aligned(16))) uint4 lds[];
-    float *const inverse = reinterpret_cast<float *>(lds + 3 * BUF);      // [BM + BN] the rows' scales
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave % WAVES_M, wn = wave / WAVES_M;
+    int *const exponent = reinterpret_cast<int *>(lds + 3 * BUF);         // [BM + BN] of the rows' scales
+    int &outgrown = exponent[BM + BN];
     const int N = a.N, K = a.K;
     const int64_t M = a.M;
     // XCD b % 8 takes a contiguous range of the tiles, a tile of x against all matrices before the next
@@ -160,183 +175,222 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
     const int64_t m0 = int64_t(tile / ntn) * BM;
     const int nt = tile % ntn, set = nt / per_set, n0 = (nt % per_set) * BN;
     const float *const w = a.w[set];
-
-    // a thread's pieces of a step: eight numbers each of rows tid / 4 + RSTEP i, those of x before those of w
-    const int chunk = tid & 3, row0 = tid >> 2;
     const float *const xa = a.x + m0 * K, *const wb = w + int64_t(n0) * K;
     // (split or not, eight numbers are 32 bytes)
     const float *const xf = SPLIT ? reinterpret_cast<const float *>(a.split) + m0 * K : xa;
     const float *const wf = SPLIT ? reinterpret_cast<const float *>(a.split) + (M + int64_t(set) * N + n0) * K : wb;
-    uint32_t src[NC];
-    int dst[NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const int row = i < NP ? row0 + RSTEP * i : RSTEP * NP + (tid >> 3);
-        if (i == NP) {
-            src[i] = uint32_t(min(row - BM, N - 1 - n0)) * K + (tid & 7) * 4;
-            dst[i] = 2 * BM * 4 + (row - BM) * 4 + (((tid & 7) >> 1) ^ ((row >> 2) & 3));
-        } else if (RSTEP * i < BM) {
-            src[i] = uint32_t(min(int64_t(row), M - 1 - m0)) * K + chunk * 8;
-            dst[i] = row * 4 + (chunk ^ ((row >> 2) & 3));
-        } else {
-            src[i] = uint32_t(min(row - BM, N - 1 - n0)) * K + chunk * 8;
-            dst[i] = 2 * BM * 4 + (row - BM) * 4 + (chunk ^ ((row >> 2) & 3));
-        }
-    }
-    const int r = lane & 31, half = lane >> 5;
-    const int arow = wm * 32 * WM + r, brow = wn * 32 * WN + r;
-    int aoff[2], boff[2];
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-        aoff[kk] = arow * 4 + ((kk * 2 + half) ^ ((arow >> 2) & 3));
-        boff[kk] = 2 * BM * 4 + brow * 4 + ((kk * 2 + half) ^ ((brow >> 2) & 3));
-    }
-    float v[NC][8], scale[NC];
-    auto fetch = [&](int i, int k0) {
-        const int k = min(k0, K - BK);                  // (beyond the end: the last step again, never used)
-        const float *const p = (RSTEP * i < BM ? xf : wf) + k;
-        *reinterpret_cast<float4 *>(&v[i][0]) = *reinterpret_cast<const float4 *>(p + src[i]);
-        if (i < NP) *reinterpret_cast<float4 *>(&v[i][4]) = *reinterpret_cast<const float4 *>(p + src[i] + 4);
-    };
-    uint32_t h[4];
-    auto place = [&](uint4 *buf, int i, int p) {
-        const int plane = (RSTEP * i < BM ? BM : BN) * 4;
-        uint32_t o[4];
-        if (SPLIT) {                                    // it comes as it goes; of the half piece a thread has one term
-            const uint4 u = *reinterpret_cast<const uint4 *>(&v[i][i < NP ? 4 * p : 0]);
-            if (i < NP) buf[dst[i] + p * plane] = u;
-            else if (p == 0) buf[dst[i] + (tid & 1) * plane] = u;
-            return;
-        }
-#pragma unroll
-        for (int e = 0; e < (i < NP ? 4 : 2); ++e) {
-            if (p == 0) o[e] = h[e] = split_hi(v[i][2 * e], v[i][2 * e + 1], scale[i]);
-            else o[e] = split_lo(v[i][2 * e], v[i][2 * e + 1], scale[i], h[e]);
-        }
-        if (i < NP) buf[dst[i] + p * plane] = make_uint4(o[0], o[1], o[2], o[3]);
-        else reinterpret_cast<uint2 *>(buf + dst[i] + p * plane)[tid & 1] = make_uint2(o[0], o[1]);
-    };
-    uint4 fa[2][WM][2], fb[2][WN][2];                   // [half of the step][tile][hi, lo]
-    auto read = [&](const uint4 *buf, int kk, int n) {
-        if (n < 2 * WM) {
-            fa[kk][n % WM][n / WM] = buf[aoff[kk] + n / WM * BM * 4 + n % WM * 32 * 4];
-        } else {
-            n -= 2 * WM;
-            fb[kk][n % WN][n / WN] = buf[boff[kk] + n / WN * BN * 4 + n % WN * 32 * 4];
-        }
-    };
-    // steps 0 and 1 into their buffers, 2 on its way
-    f32x16_t acc[WM][WN] = {}, low[WM][WN] = {};
-#pragma unroll
-    for (int i = 0; i < NC; ++i) fetch(i, 0);
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        if constexpr (SPLIT) {
-            const int row = i < NP ? row0 + RSTEP * i : RSTEP * NP + (tid >> 3);
-            if ((i < NP ? chunk : tid & 7) == 0)
-                inverse[row] = a.split_inverse[RSTEP * i < BM ? min(m0 + row, M - 1) : M + int64_t(set) * N + min(n0 + row - BM, N - 1)];
-            place(lds, i, 0);
-            place(lds, i, 1);
-            fetch(i, BK);
-            continue;
-        }
-        float most = 0.f;
-#pragma unroll
-        for (int e = 0; e < (i < NP ? 8 : 4); ++e) most = fmaxf(most, fabsf(v[i][e]));
-        most = fmaxf(most, lane_xor<1>(most));
-        most = fmaxf(most, lane_xor<2>(most));
-        if (i == NP) most = fmaxf(most, lane_xor<4>(most));
-        const PowerOfTwo s = scale_to_one(most);
-        scale[i] = s.scale;
-        if (i < NP) {
-            if (chunk == 0) inverse[row0 + RSTEP * i] = s.inverse;
-        } else if ((tid & 7) == 0) {
-            inverse[RSTEP * NP + (tid >> 3)] = s.inverse;
-        }
-        place(lds, i, 0);
-        place(lds, i, 1);
-        fetch(i, BK);
-    }
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        place(lds + BUF, i, 0);
-        place(lds + BUF, i, 1);
-        fetch(i, 2 * BK);
-    }
-    lds_barrier();
-    uint4 *cur = lds, *nxt = lds + BUF, *put = lds + 2 * BUF;
-#pragma unroll
-    for (int n = 0; n < NR; ++n) read(cur, 0, n);
-#pragma unroll 1
-    for (int k0 = 0; k0 < K; k0 += BK) {
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-            for (int t = 0; t < 3; ++t) {
-                const int g = kk * 3 + t;
-#pragma unroll
-                for (int i = 0; i < WM; ++i)
-#pragma unroll
-                    for (int j = 0; j < WN; ++j) {
-                        if (t == 0) low[i][j] = mfma_f16(fa[kk][i][1], fb[kk][j][0], low[i][j]);
-                        if (t == 1) low[i][j] = mfma_f16(fa[kk][i][0], fb[kk][j][1], low[i][j]);
-                        if (t == 2) acc[i][j] = mfma_f16(fa[kk][i][0], fb[kk][j][0], acc[i][j]);
-                    }
-#pragma unroll
-                for (int n = t * NR / 3; n < (t + 1) * NR / 3; ++n) read(kk ? nxt : cur, kk ^ 1, n);
-                if (g < 2 * NC) {
-                    place(put, g / 2, g % 2);
-                    if (g % 2) fetch(g / 2, k0 + 3 * BK);
-                }
-#pragma unroll
-                for (int n = 0; n < WM * WN; ++n) {
-                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
-                    if (n == 0) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-                    else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x20, 2, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        lds_barrier();
-        uint4 *const o = cur;
-        cur = nxt;
-        nxt = put;
-        put = o;
-    }
-
-    // Results: the lane has 16 rows of one column of every 32 x 32 tile.
     const float *const bias = a.b[set];
     float *const out = a.out[set] + m0 * N + n0;
     const float *const residual = a.residual ? a.residual + m0 * N + n0 : nullptr;
     const int rows = (int)min(int64_t(BM), M - m0), cols = min(BN, N - n0);
-    bool bad = false;
+    bool bad;
+    // The rows' scales from a sample of them, 32 numbers from all parts of a row; where one has outgrown its sample (the results are
+    // infinite), the tile once more with the scales of the rows' largest numbers.
+#pragma unroll 1
+    for (int whole = 0;; ++whole) {
+        // (an opaque zero: what follows from the lane is formed anew in each pass, and none of it kept through the results)
+        int zero = 0;
+        asm volatile("" : "+v"(zero));
+        const int tid = threadIdx.x + zero, lane = tid & 63, wave = tid >> 6;
+        const int wm = wave % WAVES_M, wn = wave / WAVES_M;
+        // a thread's pieces of a step: eight numbers each of rows tid / 4 + RSTEP i, those of x before those of w
+        const int chunk = tid & 3, row0 = tid >> 2;
+        uint32_t src[NC];
+        int dst[NC];
 #pragma unroll
-    for (int j = 0; j < WN; ++j) {
-        const int n = wn * 32 * WN + j * 32 + r;
-        const float bv = bias ? bias[n0 + min(n, cols - 1)] : 0.f, sb = inverse[BM + n];
-#pragma unroll
-        for (int i = 0; i < WM; ++i) {
-            const int ml = wm * 32 * WM + i * 32;
-            float res[16];
-            if (residual) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    res[e] = residual[uint32_t(min(ml + mfma_row(e, half), rows - 1)) * N + min(n, cols - 1)];
+        for (int i = 0; i < NC; ++i) {
+            const int row = i < NP ? row0 + RSTEP * i : RSTEP * NP + (tid >> 3);
+            if (i == NP) {
+                src[i] = uint32_t(min(row - BM, N - 1 - n0)) * K + (tid & 7) * 4;
+                dst[i] = 2 * BM * 4 + (row - BM) * 4 + (((tid & 7) >> 1) ^ ((row >> 2) & 3));
+            } else if (RSTEP * i < BM) {
+                src[i] = uint32_t(min(int64_t(row), M - 1 - m0)) * K + chunk * 8;
+                dst[i] = row * 4 + (chunk ^ ((row >> 2) & 3));
+            } else {
+                src[i] = uint32_t(min(row - BM, N - 1 - n0)) * K + chunk * 8;
+                dst[i] = 2 * BM * 4 + (row - BM) * 4 + (chunk ^ ((row >> 2) & 3));
             }
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int m = ml + mfma_row(e, half);
-                float y = fmaf(low[i][j][e], 1 / SPLIT_LO, acc[i][j][e]) * inverse[m] * sb;
-                bad |= !is_finite(y);
-                y += bv;
-                if (residual) y += res[e];
-                if (m < rows && n < cols) out[uint32_t(m) * N + n] = y;
-            }
-            __builtin_amdgcn_sched_barrier(0);
         }
+        const int r = lane & 31, half = lane >> 5;
+        const int arow = wm * 32 * WM + r, brow = wn * 32 * WN + r;
+        int aoff[2], boff[2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            aoff[kk] = arow * 4 + ((kk * 2 + half) ^ ((arow >> 2) & 3));
+            boff[kk] = 2 * BM * 4 + brow * 4 + ((kk * 2 + half) ^ ((brow >> 2) & 3));
+        }
+        float v[NC][8], scale[NC];
+        auto fetch = [&](int i, int k0) {
+            const int k = min(k0, K - BK);                  // (beyond the end: the last step again, never used)
+            const float *const p = (RSTEP * i < BM ? xf : wf) + k;
+            *reinterpret_cast<float4 *>(&v[i][0]) = *reinterpret_cast<const float4 *>(p + src[i]);
+            if (i < NP) *reinterpret_cast<float4 *>(&v[i][4]) = *reinterpret_cast<const float4 *>(p + src[i] + 4);
+        };
+        uint32_t h[4];
+        auto place = [&](uint4 *buf, int i, int p) {
+            const int plane = (RSTEP * i < BM ? BM : BN) * 4;
+            uint32_t o[4];
+            if (SPLIT) {                                    // it comes as it goes; of the half piece a thread has one term
+                const uint4 u = *reinterpret_cast<const uint4 *>(&v[i][i < NP ? 4 * p : 0]);
+                if (i < NP) buf[dst[i] + p * plane] = u;
+                else if (p == 0) buf[dst[i] + (tid & 1) * plane] = u;
+                return;
+            }
+#pragma unroll
+            for (int e = 0; e < (i < NP ? 4 : 2); ++e) {
+                if (p == 0) o[e] = h[e] = split_hi(v[i][2 * e], v[i][2 * e + 1], scale[i]);
+                else o[e] = split_lo(v[i][2 * e], v[i][2 * e + 1], scale[i], h[e]);
+            }
+            if (i < NP) buf[dst[i] + p * plane] = make_uint4(o[0], o[1], o[2], o[3]);
+            else reinterpret_cast<uint2 *>(buf + dst[i] + p * plane)[tid & 1] = make_uint2(o[0], o[1]);
+        };
+        uint4 fa[2][WM][2], fb[2][WN][2];                   // [half of the step][tile][hi, lo]
+        auto read = [&](const uint4 *buf, int kk, int n) {
+            if (n < 2 * WM) {
+                fa[kk][n % WM][n / WM] = buf[aoff[kk] + n / WM * BM * 4 + n % WM * 32 * 4];
+            } else {
+                n -= 2 * WM;
+                fb[kk][n % WN][n / WN] = buf[boff[kk] + n / WN * BN * 4 + n % WN * 32 * 4];
+            }
+        };
+        // steps 0 and 1 into their buffers, 2 on its way
+        float most[NC] = {};
+        auto take = [&](int i, const float *p) {            // (beyond the end: the row's last numbers again)
+            const float4 f = *reinterpret_cast<const float4 *>(p);
+            most[i] = fmaxf(fmaxf(most[i], fmaxf(fabsf(f.x), fabsf(f.y))), fmaxf(fabsf(f.z), fabsf(f.w)));
+        };
+        if (!SPLIT) {
+            const int parts = whole ? K / BK : 1;
+#pragma unroll 4
+            for (int part = 0; part < parts; ++part)
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    // (a thread's share of the row's numbers: K / 4, of the half piece K / 8)
+                    const float *const row = (RSTEP * i < BM ? xf : wf) + src[i];
+                    if (i < NP) {
+                        const float *const p = row + chunk * (K / 4 - 8) + part * 8;
+                        take(i, p);
+                        take(i, p + 4);
+                    } else {
+                        take(i, row + (tid & 7) * (K / 8 - 4) + part * 4);
+                    }
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i) fetch(i, 0);
+        if (!SPLIT && tid == 0) outgrown = 0;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            if constexpr (SPLIT) {
+                const int row = i < NP ? row0 + RSTEP * i : RSTEP * NP + (tid >> 3);
+                if ((i < NP ? chunk : tid & 7) == 0)
+                    exponent[row] = a.split_exponent[RSTEP * i < BM ? min(m0 + row, M - 1) : M + int64_t(set) * N + min(n0 + row - BM, N - 1)];
+                place(lds, i, 0);
+                place(lds, i, 1);
+                fetch(i, BK);
+                continue;
+            }
+            float m = fmaxf(most[i], lane_xor<1>(most[i]));
+            m = fmaxf(m, lane_xor<2>(m));
+            if (i == NP) m = fmaxf(m, lane_xor<4>(m));
+            int back;
+            scale[i] = row_scale(m, whole ? TOP : TOP_OF_SAMPLE, back);
+            if (i < NP) {
+                if (chunk == 0) exponent[row0 + RSTEP * i] = back;
+            } else if ((tid & 7) == 0) {
+                exponent[RSTEP * NP + (tid >> 3)] = back;
+            }
+            place(lds, i, 0);
+            place(lds, i, 1);
+            fetch(i, BK);
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            place(lds + BUF, i, 0);
+            place(lds + BUF, i, 1);
+            fetch(i, 2 * BK);
+        }
+        lds_barrier();
+        f32x16_t acc[WM][WN] = {}, low[WM][WN] = {};
+        uint4 *cur = lds, *nxt = lds + BUF, *put = lds + 2 * BUF;
+#pragma unroll
+        for (int n = 0; n < NR; ++n) read(cur, 0, n);
+#pragma unroll 1
+        for (int k0 = 0; k0 < K; k0 += BK) {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {
+                    const int g = kk * 3 + t;
+#pragma unroll
+                    for (int i = 0; i < WM; ++i)
+#pragma unroll
+                        for (int j = 0; j < WN; ++j) {
+                            if (t == 0) low[i][j] = mfma_f16(fa[kk][i][1], fb[kk][j][0], low[i][j]);
+                            if (t == 1) low[i][j] = mfma_f16(fa[kk][i][0], fb[kk][j][1], low[i][j]);
+                            if (t == 2) acc[i][j] = mfma_f16(fa[kk][i][0], fb[kk][j][0], acc[i][j]);
+                        }
+#pragma unroll
+                    for (int n = t * NR / 3; n < (t + 1) * NR / 3; ++n) read(kk ? nxt : cur, kk ^ 1, n);
+                    if (g < 2 * NC) {
+                        place(put, g / 2, g % 2);
+                        if (g % 2) fetch(g / 2, k0 + 3 * BK);
+                    }
+#pragma unroll
+                    for (int n = 0; n < WM * WN; ++n) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+                        if (n == 0) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                        else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    }
+                    __builtin_amdgcn_sched_group_barrier(0x20, 2, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            lds_barrier();
+            uint4 *const o = cur;
+            cur = nxt;
+            nxt = put;
+            put = o;
+        }
+
+        // Results: the lane has 16 rows of one column of every 32 x 32 tile.
+        bad = false;
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            const int n = wn * 32 * WN + j * 32 + r;
+            const float bv = bias ? bias[n0 + min(n, cols - 1)] : 0.f;
+            const int back = exponent[BM + n];
+#pragma unroll
+            for (int i = 0; i < WM; ++i) {
+                const int ml = wm * 32 * WM + i * 32;
+                float res[16];
+                if (residual) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        res[e] = residual[uint32_t(min(ml + mfma_row(e, half), rows - 1)) * N + min(n, cols - 1)];
+                }
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int m = ml + mfma_row(e, half);
+                    float y = __builtin_amdgcn_ldexpf(fmaf(low[i][j][e], 1 / SPLIT_LO, acc[i][j][e]), exponent[m] + back);
+                    bad |= !is_finite(y);
+                    y += bv;
+                    if (residual) y += res[e];
+                    if (m < rows && n < cols) out[uint32_t(m) * N + n] = y;
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (SPLIT || whole) break;
+        if (__any(bad) && lane == 0) outgrown = 1;
+        __syncthreads();
+        const bool again = outgrown != 0;
+        __syncthreads();                                    // (read by all before it is cleared)
+        if (!again) return;
     }
     if (__any(bad)) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, half = lane >> 5;
+        const int wm = wave % WAVES_M, wn = wave / WAVES_M;
         // the split does not carry infinities: the wavefront's results once more, on the fp32 matrix cores
 #pragma unroll 1
         for (int t = 0; t < WM * WN; ++t) {
@@ -345,7 +399,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
             f32x16_t y = {};
 #pragma unroll 2
             for (int k = 0; k < K; k += 8) {
-                const float4 u = SPLIT ? joined(pa + k, inverse[ml + r]) : *reinterpret_cast<const float4 *>(pa + k), z = *reinterpret_cast<const float4 *>(pb + k);
+                const float4 u = SPLIT ? joined(pa + k, exponent[ml + r]) : *reinterpret_cast<const float4 *>(pa + k), z = *reinterpret_cast<const float4 *>(pb + k);
                 y = __builtin_amdgcn_mfma_f32_32x32x2f32(u.x, z.x, y, 0, 0, 0);
                 y = __builtin_amdgcn_mfma_f32_32x32x2f32(u.y, z.y, y, 0, 0, 0);
                 y = __builtin_amdgcn_mfma_f32_32x32x2f32(u.z, z.z, y, 0, 0, 0);
@@ -364,7 +418,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
 template <int WAVES_M, int WAVES_N, int WM, int WN, bool SPLIT>
 int launch(const LinearArgs &a, void *stream) {
     constexpr int BM = 32 * WM * WAVES_M, BN = 32 * WN * WAVES_N;
-    constexpr size_t lds = 3 * 2 * (BM + BN) * 64 + (BM + BN) * 4;
+    constexpr size_t lds = 3 * 2 * (BM + BN) * 64 + (BM + BN) * 4 + 4;
     static LdsGrant granted;
     if (lds > 65536 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(&linear_kernel<WAVES_M, WAVES_N, WM, WN, SPLIT>), lds, granted))
         return LFFN_ERR_LAUNCH;
@@ -444,7 +498,7 @@ extern "C" int lffn_linear_norm_f32(const float *x, const float *norm_weight, co
     a.split = p.split = static_cast<uint4 *>(workspace);
     a.M = p.M = M;
     p.rows = M + sets * N;
-    a.split_inverse = p.inverse = static_cast<float *>(workspace) + p.rows * K;
+    a.split_exponent = p.exponent = static_cast<int *>(workspace) + p.rows * K;
     a.N = p.N = (int)N;
     a.K = p.K = (int)K;
     a.sets = (int)sets;

@@ -63,6 +63,46 @@ def test_linear_keeps_scales_and_infinities(M):
     assert (((got[keep].double() - exact).abs() / exact.norm(dim=1, keepdim=True))[finite]).max() <= 1e-6
 
 
+# Both ways to the products (with LayerNorm's rows split beforehand only where there are rows enough to ask for it) against 64 bits where
+# some columns of x are far larger than others and meet weights of zero: what is left is as exact as if they were not there.  Rows that
+# are larger where their scale's sample does not see it, samples of zeros, and numbers near either end of fp32.
+@pytest.mark.parametrize("M,K", [(40, 64), (130, 768), (5000, 512)])
+@pytest.mark.parametrize("large", [1e4, 1e6, 1e9, 1e30])
+@pytest.mark.parametrize("where", ["first", "last", "unseen", "seen"])
+def test_linear_of_rows_of_many_sizes(M, K, large, where):
+    N = 200
+    x, w = _randn(M, K), _randn(N, K, seed=1) / K ** 0.5
+    seen = torch.zeros(K, dtype=torch.bool, device=DEV)             # (a fourth of the row begins with its share of the sample)
+    for c in range(4):
+        seen[c * K // 4:c * K // 4 + 8] = True
+    part = {"first": slice(0, 32), "last": slice(K - 32, K), "unseen": ~seen, "seen": seen}[where]
+    for rows in (x, w):                     # every third row; the others are what they were
+        big, other = rows.clone(), (w if rows is x else x).clone()
+        big[::3, part] *= large
+        other[:, part] = 0
+        # (unseen: the large numbers' products are zero and the sample's are left)
+        a, b = (big, other) if rows is x else (other, big)
+        got, want = ops.linear(a, [b], [None], None)[0], a.double().cpu() @ b.double().cpu().T
+        # 2^-44 of a row's largest number is lost of each at most: beyond 2^21 of the rest, that bound takes the products' place
+        share = LINEAR_REL + (0 if large <= 1e6 else 2.0 ** -44 * large * 2)
+        if share < 1:
+            assert _rel(got, want) <= share
+    norm, other = torch.ones(K, device=DEV), w.clone()
+    norm[part], other[:, part] = large, 0
+    got = ops.linear_norm(x, norm, None, 1e-5, [other], [None])[0]
+    want = torch.nn.functional.layer_norm(x.double().cpu(), (K,), norm.double().cpu(), None, 1e-5) @ other.double().cpu().T
+    assert share >= 1 or _rel(got, want) <= share + 2.0 ** -22
+    sample = x.clone()
+    sample[:, seen] = 0                     # nothing to be seen of the row
+    for size in (1.0, 1e-10, 1e-25, 1e12, 1e30):
+        got = ops.linear(sample * size, [w], [None], None)[0]
+        assert _rel(got, (sample * size).double().cpu() @ w.double().cpu().T) <= LINEAR_REL
+    for sx, sw in ((1e-37, 1e20), (1e37, 1e-20), (1e-30, 1e-5), (3e37, 1e-30)):
+        got = ops.linear(x * sx, [w * sw], [None], None)[0]
+        assert _rel(got, (x * sx).double().cpu() @ (w * sw).double().cpu().T) <= LINEAR_REL
+    assert torch.equal(ops.linear(torch.zeros_like(x), [w], [None], None)[0], torch.zeros(M, N, device=DEV))
+
+
 # tiles of 128 x 192: whole rounds and a remainder of rows, a last tile of 124 and of one column, one and three matrices, one step of k
 @pytest.mark.parametrize("M,N,K,sets", [(6145, 768, 768, 1), (6145, 700, 32, 1), (6700, 577, 96, 1), (2103, 768, 64, 3)])
 def test_linear_in_tiles_of_192_columns(M, N, K, sets):
