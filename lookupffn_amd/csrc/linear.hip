@@ -53,17 +53,8 @@ struct SplitArgs {
     float eps;
 };
 
-// A row's scale: its largest number, or that of a sample of it, to [2^top, 2^(top + 1)); the way back is added to the results'
-// exponents.  A number is then held to 22 bits down to 2^-(14 + top) of that largest one and a smaller one to 2^-(36 + top) of it.
-// A row of zeros, or of less than 2^-103, is scaled as one of 2^-103, so that a sample of zeros hides no small numbers behind it: they
-// outgrow it.
 constexpr int TOP = 13;             // the row's largest number: lo, times 2048, stays below 2^13
 constexpr int TOP_OF_SAMPLE = 8;    // a sample's, which the row may outgrow 128 times
-__device__ __forceinline__ float row_scale(float most, int top, int &exponent) {
-    const int bits = __float_as_uint(most) >> 23, e = bits == 255 ? 127 : max(bits, 24);     // (times 2048 still a number)
-    exponent = e - 127 - top;
-    return __uint_as_float((254 - e + top) << 23);
-}
 
 __device__ __forceinline__ float wave_max(float v) {
     v = fmaxf(v, lane_xor<1>(v));
@@ -125,7 +116,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(SplitArgs a) {
         for (int e = 0; e < 4; ++e)
             if (i * 64 + lane < quads && is_finite(v[i][e])) most = fmaxf(most, fabsf(v[i][e]));
     int exponent;
-    const float scale = row_scale(wave_max(most), TOP, exponent);
+    const float scale = scale_to(wave_max(most), TOP, exponent);
     uint4 *const to = a.split + row * quads;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -294,7 +285,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void linear_kernel(Linea
             m = fmaxf(m, lane_xor<2>(m));
             if (i == NP) m = fmaxf(m, lane_xor<4>(m));
             int back;
-            scale[i] = row_scale(m, whole ? TOP : TOP_OF_SAMPLE, back);
+            scale[i] = scale_to(m, whole ? TOP : TOP_OF_SAMPLE, back);
             if (i < NP) {
                 if (chunk == 0) exponent[row0 + RSTEP * i] = back;
             } else if ((tid & 7) == 0) {

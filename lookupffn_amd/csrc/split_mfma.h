@@ -65,5 +65,23 @@ __device__ __forceinline__ PowerOfTwo scale_to_one(float most) {
     return {__uint_as_float((254 - e) << 23), __uint_as_float(e << 23)};
 }
 
+// The power of two that takes numbers of largest magnitude `most`, or a sample's, to [2^top, 2^(top + 1)); `exponent` is that of the way
+// back.  A number is then held to 22 bits down to 2^-(14 + top) of that largest one and a smaller one to 2^-(36 + top) of it (lo without
+// its factor: 2^-(3 + top) and 2^-(25 + top)).  Nothing but zeros, or numbers below 2^-103, is scaled as 2^-103 would be, so that a sample
+// of zeros hides no small numbers behind it: they outgrow it.
+__device__ __forceinline__ float scale_to(float most, int top, int &exponent) {
+    const int bits = __float_as_uint(most) >> 23, e = bits == 255 ? 127 : max(bits, 24);     // (times 2048 still a number)
+    exponent = e - 127 - top;
+    return __uint_as_float((254 - e + top) << 23);
+}
+
+// Largest over the four rows of 16 lanes (row swaps on the vector ALU: an LDS permute would be waited for).
+__device__ __forceinline__ float rows_most(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // A barrier behind the LDS accesses issued so far; global loads stay in flight.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

@@ -206,6 +206,40 @@ def test_attention_masks_scales_and_infinities():
         assert _rel(got[b].nan_to_num(), want[b].nan_to_num()) <= 2e-6, b
 
 
+# Steps of 64 keys: values that grow from one to the next in all or some columns, columns and keys of many sizes, first keys that say
+# nothing of the others.
+@pytest.mark.parametrize("L", [70, 200, 512])
+@pytest.mark.parametrize("columns", [1, 3, 64])
+def test_attention_of_many_sizes(L, columns):
+    B, heads = 2, 3
+    q, k, v = (_randn(B, L, heads, 64, seed=s) for s in range(3))
+    mask = torch.ones(B, L, device=DEV)
+
+    def close(q, k, v, share=1e-6):                     # column for column
+        got, want = ops.attention(q, k, v, mask).double().cpu().flatten(0, 2), _exact_attention(q, k, v, mask).flatten(0, 2)
+        assert ((got - want).norm(dim=0) / want.norm(dim=0)).max() <= share
+
+    every = 64 // columns
+    for f in (1e2, 1e5, 1e12, 1e30):
+        grown = v.clone()
+        grown[:, 65::9, :, ::every] *= f                # (of one in nine keys behind the first step's)
+        grown[:, 65::30, :, ::every] *= f if f < 1e30 else 1e6
+        close(q, k, grown)
+        small = v.clone()
+        small[:, :65, :, ::every] /= f
+        close(q, k, small)
+    sizes = v * 10.0 ** (torch.arange(64, device=DEV) % 13 - 6)
+    close(q, k, sizes)
+    close(q, k * torch.where(torch.arange(L, device=DEV) % 3 == 1, 1e-7, 1.0)[:, None, None], sizes)
+    late = v * 1e-20
+    late[:, :64] = 0
+    close(q, k, late)
+    # a value a million times the others' that no query looks at: its column's others are held to 2^-39 of it (values beyond its step
+    # are, too): 2^-39 4e6 is 7e-6 at most of a value, a third of that on average of either sign, over at least 70 keys
+    k[:, 65], v[:, 65, :, ::every], mask[:, 65] = 0, 1e6, 0
+    close(q, k, v, 3e-6)
+
+
 def _config(hidden, heads):
     return Namespace(hidden_size=hidden, num_attention_heads=heads, attention_head_size=hidden // heads, attention_probs_dropout_prob=0.1,
                      hidden_dropout_prob=0.1, layer_norm_eps=1e-5, ffn_num_table=32, ffn_table_size=256, projection_type="bh4", block_size=1)
