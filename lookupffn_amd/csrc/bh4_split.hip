@@ -34,23 +34,23 @@ constexpr int BS = 64;          // block size this file is built for
 constexpr int PAD = 4;          // floats of padding per row of the fp32 tile
 constexpr float TOP = 16384.f;  // what the largest of a row is scaled to at least (and less than twice that)
 
+// Largest over the wavefront.
 __device__ __forceinline__ float wave_most(float v) {
     v = fmaxf(v, lane_xor<1>(v));
     v = fmaxf(v, lane_xor<2>(v));
     v = fmaxf(v, lane_xor<4>(v));
     v = fmaxf(v, lane_xor<8>(v));
-    v = fmaxf(v, lane_xor<16>(v));
-    return fmaxf(v, lane_xor<32>(v));
+    return rows_most(v);
 }
 
 // The 64-point transform of every block (bh4_block.hip: bh4_fold_kernel), split, ready for the product kernel.  One workgroup per stage, a wavefront per
-// block: the 16 output (forward; transposed: input) columns that a product wavefront has of every block are scaled together by a
-// power of two, their largest in the stage to [2^14, 2^15), so that lo needs no factor.  Per block and product wavefront four
-// fragments of 64 lanes x 8 numbers: hi of the first and the second eight columns of a lane's sixteen, then lo of them; behind all
-// blocks the inverse scales, [stage][4].
+// block: an output (transposed: input) column is scaled by a power of two, the same in every block (the butterflies add the blocks'
+// columns), its largest in the stage (transposed), or that of sixteen columns, to [2^14, 2^15), so that lo needs no factor.  Per block
+// and product wavefront four fragments of 64 lanes x 8 numbers: hi of the first and the second eight columns of a lane's sixteen, then lo
+// of them; behind all blocks the inverse scales, [stage][64].
 template <bool TRANSPOSED>
 __global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, uint32_t *out, float *inverse) {
-    __shared__ float most_s[16][4];
+    __shared__ float most_s[16][BS], scale_s[BS];
     const int num_block = blockDim.x / 64, wave = threadIdx.x >> 6;
     const int64_t blk = int64_t(blockIdx.x) * num_block + wave;
     const int i = threadIdx.x & 63;
@@ -70,34 +70,31 @@ __global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, ui
         }
     }
     if constexpr (!TRANSPOSED) {
+        // sixteen output columns by one scale: they are fp32 sums of the same 64 numbers, rounded to 2^-24 of the largest of those in any
+        // case (a scale for each, D = 1024: 9.2 -> 17.2 us a call)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             float most = 0.f;
 #pragma unroll
             for (int o = 16 * g; o < 16 * g + 16; ++o) most = fmaxf(most, fabsf(v[o]));
             most = wave_most(most);
-            if (i == 0) most_s[wave][g] = most;
+            if (i / 16 == g) most_s[wave][i] = most;
         }
     } else {
         float most = 0.f;
 #pragma unroll
         for (int o = 0; o < BS; ++o) most = fmaxf(most, fabsf(v[o]));
-        most = fmaxf(most, lane_xor<1>(most));
-        most = fmaxf(most, lane_xor<2>(most));
-        most = fmaxf(most, lane_xor<4>(most));
-        most = fmaxf(most, lane_xor<8>(most));
-        if (i % 16 == 0) most_s[wave][i / 16] = most;
+        most_s[wave][i] = most;
     }
     __syncthreads();
-    float scale[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    if (wave == 0) {
         float most = 0.f;
-        for (int n = 0; n < num_block; ++n) most = fmaxf(most, most_s[n][g]);
+        for (int n = 0; n < num_block; ++n) most = fmaxf(most, most_s[n][i]);
         const PowerOfTwo p = scale_to_one(most);
-        scale[g] = p.scale * TOP;
-        if (threadIdx.x == 0) inverse[blockIdx.x * 4 + g] = p.inverse * (1 / TOP);
+        scale_s[i] = p.scale * TOP;
+        inverse[blockIdx.x * BS + i] = p.inverse * (1 / TOP);
     }
+    __syncthreads();
     // eight consecutive k of a row of the A operand as hi and lo: fragment (row / 16, (k % 16) / 8), lane 16 (k / 16) + row % 16
     uint4 *const dst = reinterpret_cast<uint4 *>(out + blk * (BS * BS));
     auto store8 = [&](int row, int k, const float (&x)[8]) {
@@ -112,7 +109,7 @@ __global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, ui
         dst[at + 128] = make_uint4(l[0], l[1], l[2], l[3]);
     };
     if constexpr (TRANSPOSED) {
-        const float f = i < 32 ? (i < 16 ? scale[0] : scale[1]) : (i < 48 ? scale[2] : scale[3]);
+        const float f = scale_s[i];
 #pragma unroll
         for (int k = 0; k < BS; k += 8) {
             float x[8];
@@ -127,7 +124,7 @@ __global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, ui
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
 #pragma unroll
-            for (int o = 0; o < 16; ++o) t[o * 65 + i] = v[16 * g + o] * scale[g];
+            for (int o = 0; o < 16; ++o) t[o * 65 + i] = v[16 * g + o] * scale_s[16 * g + o];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
@@ -148,7 +145,7 @@ struct SplitArgs {
     const float *ln_b;     // [H]
     float ln_eps;
     const float *w;        // split weights
-    const float *wscale;   // their inverse scales [R*J][4]
+    const float *wscale;   // their inverse scales [R*J][64]
     const float *pbias;    // [T*8] or null
     int32_t *codes;        // [B, T]
     float *scores;         // [B, T]
@@ -232,7 +229,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     const int r = blockIdx.y;
     f32x4 acc[NBW];
 
-    // this wavefront's weights of a block: four fragments of 1 KB (WSPLIT: hi, hi, lo, lo; else 16 numbers a lane)
+    // this wavefront's weights of a block: four fragments of 1 KB (hi, hi, lo, lo)
     uint4 wq[AHEAD][4];
     auto load_w = [&](int s, int n) {
         if (n >= NBW) {                           // the next stage's first blocks (after the last stage: a harmless re-read)
@@ -260,12 +257,18 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         *reinterpret_cast<uint2 *>(p + TOK * LDP) = lo;
     };
 
-    // What the accumulators are to be multiplied with: the inverse scales of this wavefront's weights and of the lane's tokens.
-    float inv_w = 1.f, inv_x = 1.f;
+    // What the accumulators are to be multiplied with: the inverse scales of the lane's four columns of the weights and of its token.
+    f32x4 inv_w = {1.f, 1.f, 1.f, 1.f};
+    float inv_x = 1.f;
 
     // acc = (blocks of the stage's weights) x (the tile's tokens)
     auto product = [&](int s) {
-        inv_w = a.wscale[(r * J + s) * 4 + ow];
+        const float *const scales = a.wscale + (r * J + s) * BS + 16 * ow;         // uniform: scalar loads, chosen from by lane
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (BWD) inv_w[e] = kq < 2 ? (kq == 0 ? scales[e] : scales[4 + e]) : (kq == 2 ? scales[8 + e] : scales[12 + e]);
+            else inv_w[e] = scales[0];         // (the forward's sixteen columns have one)
+        }
         inv_x = unscale[c];
         uint4 xv[2][4];
         read_x(0, xv[0]);
@@ -344,23 +347,24 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             }
             __syncthreads();
         } else {
-            float most = 0.f;
+            f32x4 m4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int n = 0; n < NBW; ++n)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) most = fmaxf(most, fabsf(acc[n][e]));
-            most = rows_most(most) * inv_w;
+                for (int e = 0; e < 4; ++e) m4[e] = fmaxf(m4[e], fabsf(acc[n][e]));
+            m4 = m4 * inv_w;
+            const float most = rows_most(fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w)));
             if (kq == 0) most_s[c * 4 + ow] = most;
             __syncthreads();                      // every wavefront has read this stage's input and left its largest
             const float4 m = *reinterpret_cast<const float4 *>(most_s + c * 4);
             const PowerOfTwo s = scale_to_one(fmaxf(fmaxf(m.x, m.y), fmaxf(m.z, m.w)));
             if (kq == 0 && ow == 0) unscale[c] = inv_x * (s.inverse * (1 / TOP));
-            const float scale = inv_w * (s.scale * TOP);
+            const f32x4 scale = inv_w * (s.scale * TOP);
 #pragma unroll
             for (int n = 0; n < NBW; ++n) put(c, n * BS + 16 * ow + 4 * kq, acc[n] * scale);
             if (BWD && tok_base + c < B) {
                 float *o = save + size_t(c) * D + 16 * ow + 4 * kq;
-                const float f = inv_w * inv_x;
+                const f32x4 f = inv_w * inv_x;
 #pragma unroll
                 for (int n = 0; n < NBW; ++n) __builtin_nontemporal_store(acc[n] * f, reinterpret_cast<f32x4 *>(o + n * BS));
             }

@@ -241,7 +241,7 @@ lffn_block_front block_front(const Config &c, const Params &p, const Tensor &spl
 }
 
 // Floats of the split weights (lffn_bh4_fold_split_f32).
-int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 4); }
+int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 64); }
 
 // as_training: 64 x 64 blocks go through the training forward's kernel (block_weight: folded), so that a module in train() computes the
 // same codes with and without gradients (a checkpointed pass runs both); else through the faster one of inference (block_weight: split).

@@ -119,3 +119,17 @@ def test_scales_and_rows_of_their_own(B):
     got = front(y)
     assert torch.equal(got[rows + [7]], torch.cat([codes[rows], torch.zeros_like(codes[:1])]))
     assert not got[11].any() and not got[12].any()                  # NaN is not above zero
+
+
+# one stage of the backward, few and many workgroups: columns of the weights of very different sizes side by side, each by its own scale.
+# (The forward's columns are sums of 64 of them, rounded in fp32 to 2^-24 of the largest before they are split.)
+@pytest.mark.parametrize("B,D", [(40, 64), (33, 256), (9000, 256), (70, 512), (50, 1024)])
+def test_columns_of_many_sizes(B, D):
+    gen = torch.Generator(device=DEV).manual_seed(B + D)
+    sizes = 10.0 ** -(torch.arange(64, device=DEV) * 5 % 13)
+    g, w = _randn(gen, B, D), _randn(gen, 1, 1, D // 64, 64, 64) / 64 * sizes
+    some = list(range(min(B, 40)))
+    got = ops.bh4_block_bwd_split(g, ops.bh4_fold_split(w, True), 1, 1, D, D, 1.0, 0.0)[0][0][some].double().cpu()
+    want = _blocks(w[0, 0].double().cpu().transpose(-1, -2), g[some].double().cpu() @ _hadamard(D))
+    error, size = (t.view(len(some), D // 64, 64).norm(dim=(0, 1)) for t in (got - want, want))
+    assert (error / size).max() <= REL
