@@ -250,10 +250,11 @@ void infer(const Config &c, const Params &p, const Tensor &block_weight, bool as
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     // Rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half as many tokens
-    // more, and so are tables of which a token's rows are few.  One launch, two, us: fp32 768 tokens, 128 tables of 768 columns
-    // 45, 46, 128 of 512 32, 35, but 128 of 1024 60, 57 and 512 of 1024 218, 187; bfloat16 1152 tokens, 128 of 768 37, 56.
+    // more, and so are tables of which a token's rows are few.  One launch, two, us, tables not in the caches: fp32 768 tokens, 128
+    // tables of 768 columns 45.5, 48.8, of 832 48.7, 51.5, of 896 52.4, 53.3, but of 960 55.3, 53.7, of 1024 59.0, 57.0 and 512 of 1024
+    // 218, 187 (256 tables of 448 53.7, 63.7); bfloat16 1152 tokens, 128 of 768 37.8, 70, of 896 43.5, 45.2.
     if (c.fmt != 0) fused_max += fused_max / 2;
-    if (c.T * c.Do <= 128 * 768) fused_max += fused_max / 2;
+    if (c.T * c.Do <= 128 * 896) fused_max += fused_max / 2;
     if (c.one_launch && B <= fused_max) {
         const lffn_fused_layer layer{f32(p[0]), f32(p[1]), f32(p[2]), f32(p[3]), f32(p[4]), f32(p[5]), c.H, c.D, c.R, c.J, c.T,
                                      c.S, c.Do, (float)c.eps, (float)c.decay, (float)c.residual};

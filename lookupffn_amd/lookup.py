@@ -398,11 +398,11 @@ class LookupFFN(nn.Module):
         return (f"hidden_size={self.hidden_size}, num_table={self.num_table}, "
                 f"table_size={self.table_size}, output_size={self.output_size}")
 
-    # Up to this many tokens (half as many more for 16-bit rows, and again for at most 128 tables of 768 columns) the
+    # Up to this many tokens (half as many more for 16-bit rows, and again for at most 128 tables of 896 columns) the
     # one-launch form of the layer (a workgroup per token: LayerNorm, projection, hash and the token's gather-add) beats the
     # projection kernel followed by the table-major gather, which stages every table slice in LDS and needs many tokens to
-    # pay for it: 512 tokens, 128 tables of 768 fp32 columns 32 us against 38, 768 tokens 45 against 46, 1000 tokens 56
-    # against 53.
+    # pay for it: 512 tokens, 128 tables of 768 fp32 columns 33 us against 40, 768 tokens 45 against 49, 960 tokens 55.4
+    # against 54.9; 768 tokens, 896 columns 52 against 53, 960 columns 55 against 54.
     FUSED_LAYER_MAX_TOKENS = 512
 
     def _no_gradient_wanted(self, x):
@@ -415,7 +415,7 @@ class LookupFFN(nn.Module):
         most = self.FUSED_LAYER_MAX_TOKENS
         if self.tables.dtype != torch.float32:
             most += most // 2
-        if self.num_table * self.output_size <= 128 * 768:
+        if self.num_table * self.output_size <= 128 * 896:
             most += most // 2
         if not (x.shape[0] <= most and x.is_cuda and x.dtype == torch.float32
                 and self._no_gradient_wanted(x)):

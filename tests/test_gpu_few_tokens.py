@@ -1,10 +1,12 @@
 """A token's columns shared out over several workgroups (csrc/token_gather.h): as from one, bit for bit."""
 import ctypes
 import math
+from argparse import Namespace
 
 import pytest
 import torch
 
+import lookupffn_amd
 from lookupffn_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
@@ -77,3 +79,20 @@ def test_inner_product_by_token_and_not(T, Do, half):
         for t in range(0, T, 7):
             term = tables[rows[:B, t].long()].double() * g[:B].double()
             assert ((got[:, t].double() - term.sum(-1)).abs() <= (Do + 1) * 2.0 ** -24 * term.abs().sum(-1)).all()
+
+
+# either side of the line up to which a layer is one launch: tokens, tables times columns, rows of 16 bits
+@pytest.mark.parametrize("T,Do,dtype,most", [(128, 896, torch.float32, 768), (128, 960, torch.float32, 512), (64, 128, torch.float32, 768),
+                                             (128, 896, torch.bfloat16, 1152), (120, 1024, torch.float16, 768)])
+def test_layer_in_one_launch_and_not(T, Do, dtype, most):
+    cfg = Namespace(hidden_size=300, ffn_num_table=T, ffn_table_size=S, layer_norm_eps=1e-5, projection_type="bh4", block_size=1)
+    torch.manual_seed(Do)
+    layer = lookupffn_amd.LookupFFN(cfg, Do).to(DEV).eval()
+    layer.tables.data = layer.tables.data.to(dtype)
+    x, residual = torch.randn(most + 1, 300, device=DEV), torch.randn(most + 1, Do, device=DEV)
+    with torch.no_grad():
+        want = layer._forward_operators(x, residual)
+        for B in (most, most + 1):
+            assert layer.can_fuse_layer(x[:B]) == (B == most)
+            # the same products summed over the tables in another order: T 2^-24 of their magnitudes (some 0.02 T^0.5 and the residual)
+            assert (layer(x[:B], residual=residual[:B]) - want[:B]).abs().max() <= 1e-5
