@@ -544,10 +544,8 @@ def main():
         head = (x.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(), float(ln.eps))
         tail = (proj.bias.data_ptr(), records.data_ptr(), rec_plan[1], rec_plan[0])
         if block:
-            front = _lib.BlockFront(ln.weight.data_ptr(), ln.bias.data_ptr(), layer.hash.split_weight().data_ptr(), proj.bias.data_ptr(),
-                                    None, None, records.data_ptr(), rec_plan[1], *sizes[1:], rec_plan[0], float(ln.eps),
-                                    *coefs)
-            _lib.check(lib.lffn_bh4_block_front_split_f32(ctypes.byref(front), x.data_ptr(), B, stream), "lffn_bh4_block_front_split_f32")
+            _lib.check(lib.lffn_ln_bh4_block_hash_records_f32(*head, layer.hash.folded_weight().data_ptr(), *tail, *sizes, 64, *coefs, stream),
+                       "lffn_ln_bh4_block_hash_records_f32")
         else:
             _lib.check(lib.lffn_ln_project_hash_records_f32(*head, diag.data_ptr(), *tail, *sizes, *coefs, stream),
                        "lffn_ln_project_hash_records_f32")

@@ -767,10 +767,10 @@ int lffn_lookup_inner_f32(const int32_t *code, const float *g, const float *tabl
 /*
  * The kernels of lffn_ln_bh4_block_hash_f32 (inference) and lffn_bh4_block_bwd_f32 with every number as two
  * half-precision terms, which is faster and closer to 64 bits (csrc/bh4_split.hip).  They are rounded differently: a
- * code may differ where its z is within 1e-6 of the row's size of zero.  The layer runs this backward in every case
- * and this front end in eval() without gradients; in train() it runs lffn_ln_bh4_block_hash_f32 (or _records_f32)
- * without gradients, whose codes are those of lffn_ln_bh4_block_hash_train_f32 bit for bit.  lffn_bh4_block_bwd_f32
- * is the backward for callers that want fp32 products.
+ * code may differ where its z is within 1e-6 of the row's size of zero.  The layer runs this backward; its forward is
+ * lffn_ln_bh4_block_hash_f32 (or _records_f32) without gradients, whose codes are those of
+ * lffn_ln_bh4_block_hash_train_f32 bit for bit.  lffn_bh4_block_front_split_f32 is for callers that run no training
+ * forward beside it, lffn_bh4_block_bwd_f32 for those that want fp32 products.
  *
  * lffn_bh4_fold_split_f32: the 64-point transform of lffn_bh4_fold_mode_f32 (transposed == 0: mode 0, else
  * mode 1) of stages x num_block blocks, split.  w: [stages, num_block, 64, 64], num_block a power of two up to

@@ -18,9 +18,10 @@
 // 12.2.  Tried: 32 tokens a workgroup in 4 wavefronts (124-149 us from build to build) and 8 (151), 64 in 8 (145), four blocks' weights
 // ahead instead of two (134).  Error of the last stage against 64 bits 2.4e-7 (fp32 matrix cores 3.2e-7), input gradient 2.2e-7 (3.1e-7).
 //
-// A layer in train() stays on the fp32 matrix cores, with gradients and without (Hashing.forward_block, csrc/host.cpp): a projected
+// A layer's forward stays on the fp32 matrix cores, with gradients and without (Hashing.forward_block, csrc/host.cpp): a projected
 // value within rounding of zero takes either sign, with the sign the derivative of its score turns round, and neither should a
-// training step's gradients change with the kernel nor a checkpointed pass without gradients differ from its repetition with them.
+// training step's gradients change with the kernel nor a pass without gradients differ from one with them.  The layer takes the
+// backward from here; the hash form is an operator of its own (lffn_bh4_block_front_split_f32), for programs that run no training forward.
 #include "split_mfma.h"
 
 // the mix and the score keep the reference's operation order: no fused multiply-add

@@ -57,7 +57,6 @@ using torch::autograd::variable_list;
     X(lffn_ln_bh4_block_hash_train_f32)     \
     X(lffn_ln_bh4_block_hash_f32)           \
     X(lffn_ln_bh4_block_hash_records_f32)   \
-    X(lffn_bh4_block_front_split_f32)       \
     X(lffn_bh4_fold_split_f32)              \
     X(lffn_bh4_fold_mode_f32)               \
     X(lffn_lookup_scatter_workspace_bytes)  \
@@ -111,11 +110,10 @@ struct Parts {
     std::array<PyObject *, 6> params;
     double eps, decay;
     int64_t num_table, output_size;
-    bool training;                       // the hash's train() or eval()
 };
 
 PyObject *KEY_MODULES, *KEY_PARAMETERS, *KEY_LAYER_NORM, *KEY_HASH, *KEY_PROJECTION, *KEY_WEIGHT, *KEY_BIAS, *KEY_TABLES, *KEY_EPS,
-    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_FOLDED, *KEY_SPLIT, *KEY_TRAINING;      // interned
+    *KEY_DECAY, *KEY_NUM_TABLE, *KEY_OUTPUT_SIZE, *KEY_FOLDED;      // interned
 
 PyObject *dict_of(PyObject *o) {
     PyObject **d = o ? _PyObject_GetDictPtr(o) : nullptr;
@@ -157,9 +155,7 @@ bool find_parts(PyObject *layer, Parts &found) {
                     item(of_projection, KEY_BIAS), item(of_layer, KEY_TABLES), item(of_layer, KEY_BIAS)};
     for (PyObject *o : found.params)
         if (!o || !THPVariable_Check(o)) return false;
-    PyObject *mode = item(hash, KEY_TRAINING);
-    found.training = mode == Py_True;
-    return (found.training || mode == Py_False) && number(item(norm, KEY_EPS), found.eps) && number(item(projection, KEY_DECAY), found.decay) &&
+    return number(item(norm, KEY_EPS), found.eps) && number(item(projection, KEY_DECAY), found.decay) &&
            whole(item(own, KEY_NUM_TABLE), found.num_table) && whole(item(own, KEY_OUTPUT_SIZE), found.output_size);
 }
 
@@ -222,31 +218,14 @@ void gather(const Config &c, const Tensor &codes, const Tensor &scores, const Te
 // The layer's parameters: LayerNorm's, the projection's, tables and output bias.
 using Params = std::array<Tensor, 6>;
 
-// The 64 x 64 blocks' kernel with the layer's parameters, its outputs open.
-lffn_block_front block_front(const Config &c, const Params &p, const Tensor &split) {
-    lffn_block_front f{};
-    f.ln_weight = f32(p[0]);
-    f.ln_bias = f32(p[1]);
-    f.w_split = f32(split);
-    f.proj_bias = f32(p[3]);
-    f.H = c.H;
-    f.D = c.D;
-    f.R = c.R;
-    f.J = c.J;
-    f.T = c.T;
-    f.ln_eps = (float)c.eps;
-    f.decay = (float)c.decay;
-    f.residual = (float)c.residual;
-    return f;
-}
-
 // Floats of the split weights (lffn_bh4_fold_split_f32).
 int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 64); }
 
-// as_training: 64 x 64 blocks go through the training forward's kernel (block_weight: folded), so that a module in train() computes the
-// same codes with and without gradients (a checkpointed pass runs both); else through the faster one of inference (block_weight: split).
-void infer(const Config &c, const Params &p, const Tensor &block_weight, bool as_training, const Tensor &x, const float *residual,
-           Tensor &out, int64_t B, int64_t fused_max) {
+// folded: the 64 x 64 blocks' weights.  Their kernel is the training forward's: with the split products of the backward (csrc/bh4_split.hip,
+// 252 us a call instead of 333 at 32768 x 512, 128 tables of 512 columns) a value within rounding of zero took the other sign and its token other table rows,
+// two in four million, so that a layer computed one thing with gradients recorded and another without (a checkpointed pass runs both).
+void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor &x, const float *residual, Tensor &out, int64_t B,
+           int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
     // Rows of 16 bits are half the traffic of a form that reads every token's rows from memory, and so good for half as many tokens
@@ -270,16 +249,9 @@ void infer(const Config &c, const Params &p, const Tensor &block_weight, bool as
         if (c.form == DIAG)
             CALL(lffn_ln_project_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, decay, res, st);
-        else if (as_training)
-            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(block_weight), f32(p[3]), rp, plan.stride,
+        else
+            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
-        else {
-            lffn_block_front front = block_front(c, p, block_weight);
-            front.records = rp;
-            front.record_stride = plan.stride;
-            front.tokens_per_workgroup = plan.tokens;
-            CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
-        }
         if (plan.parts.parts)
             CALL(lffn_lookup_gather_parts_rows, &plan.parts, nullptr, nullptr, p[4].data_ptr(), f32(p[5]), residual, f32(out), rp, plan.bytes,
                  B, c.T, c.S, c.Do, (int32_t)c.fmt, st);
@@ -293,15 +265,9 @@ void infer(const Config &c, const Params &p, const Tensor &block_weight, bool as
     if (c.form == DIAG)
         CALL(lffn_ln_project_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), nullptr, cp, f32(scores), B, c.H,
              c.D, c.R, c.J, c.T, decay, res, st);
-    else if (as_training)
-        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(block_weight), f32(p[3]), cp, f32(scores), B, c.H, c.D,
+    else
+        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), B, c.H, c.D,
              c.R, c.J, c.T, 64, decay, res, st);
-    else {
-        lffn_block_front front = block_front(c, p, block_weight);
-        front.codes = cp;
-        front.scores = f32(scores);
-        CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
-    }
     gather(c, codes, scores, p[4], p[5], residual, out, B, plan, st);
 }
 
@@ -567,19 +533,19 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._folded or hash._split = ((version, address, device), folded or split weights, what they were made from), as
-// Hashing.block_weight keeps them: those weights if they are w's.
-Tensor weight_of(PyObject *hash, PyObject *name, const Tensor &w, int64_t words) {
-    PyObject *kept = item(dict_of(hash), name);
+// hash._folded = ((version, address, device), folded weights, what they were folded from), as Hashing.folded_weight keeps them: the
+// folded weights if they are w's.
+Tensor folded_of(PyObject *hash, const Tensor &w) {
+    PyObject *kept = item(dict_of(hash), KEY_FOLDED);
     if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3) return {};
-    PyObject *key = PyTuple_GET_ITEM(kept, 0), *made = PyTuple_GET_ITEM(kept, 1);
+    PyObject *key = PyTuple_GET_ITEM(kept, 0), *folded = PyTuple_GET_ITEM(kept, 1);
     int64_t version = 0, address = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
-        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(made))
+        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(folded))
         return {};
-    const Tensor &f = THPVariable_Unpack(made);
+    const Tensor &f = THPVariable_Unpack(folded);
     const bool same = w._version() == (uint32_t)version && w.data_ptr() == reinterpret_cast<void *>(address) && f.device() == w.device() &&
-                      f.numel() == words;
+                      f.numel() == w.numel();
     return same ? f : Tensor();
 }
 
@@ -590,7 +556,7 @@ struct WithoutInterpreter {
 };
 
 // forward(layer, x, residual or None, tokens up to which the one-launch form is taken) -> a tensor; None: not for this path;
-// False: the blocks' weights (Hashing.block_weight) are not up to date
+// False: the folded weights (Hashing.folded_weight) are not up to date
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 4, "forward: 4 arguments");
@@ -626,17 +592,13 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         for (const Tensor &t : params) grads = grads || t.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;
-    Tensor block_weight;
-    if (!grads && c.form == BLOCK) {
-        block_weight = parts.training ? weight_of(parts.hash, KEY_FOLDED, params[2], params[2].numel())
-                                      : weight_of(parts.hash, KEY_SPLIT, params[2], split_words(c));
-        if (!block_weight.defined()) Py_RETURN_FALSE;
-    }
+    Tensor folded;
+    if (!grads && c.form == BLOCK && !(folded = folded_of(parts.hash, params[2])).defined()) Py_RETURN_FALSE;
     const int64_t fused_max = PyLong_AsLongLong(args[3]);
     if (fused_max == -1 && PyErr_Occurred()) return nullptr;
     Tensor out;
     {
-        // (from here on only what is owned here is used: x, the residual, the parameters and the blocks' weights)
+        // (from here on only what is owned here is used: x, the residual, the parameters and the folded weights)
         const WithoutInterpreter unlocked;
         // any layout of x and any shape and type of the residual, as the Python path makes them
         x = x.contiguous();
@@ -646,7 +608,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
             (!residual.defined() || reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0)) {
             out = empty_f32(sizes, dev);
             if (grads) train(c, params, x, residual, out, B);
-            else infer(c, params, block_weight, parts.training, x, f32(residual), out, B, fused_max);
+            else infer(c, params, folded, x, f32(residual), out, B, fused_max);
         }
     }
     if (!out.defined()) Py_RETURN_NONE;
@@ -669,7 +631,7 @@ PyMODINIT_FUNC PyInit__host() {
         {&KEY_MODULES, "_modules"}, {&KEY_PARAMETERS, "_parameters"}, {&KEY_LAYER_NORM, "LayerNorm"}, {&KEY_HASH, "hash"},
         {&KEY_PROJECTION, "projection"}, {&KEY_WEIGHT, "weight"}, {&KEY_BIAS, "bias"}, {&KEY_TABLES, "tables"},
         {&KEY_EPS, "eps"}, {&KEY_DECAY, "decay_coeff"}, {&KEY_NUM_TABLE, "num_table"},
-        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_FOLDED, "_folded"}, {&KEY_SPLIT, "_split"}, {&KEY_TRAINING, "training"},
+        {&KEY_OUTPUT_SIZE, "output_size"}, {&KEY_FOLDED, "_folded"},
     };
     for (const auto &[key, name] : keys)
         if (!(*key = PyUnicode_InternFromString(name))) return nullptr;

@@ -190,35 +190,23 @@ class Hashing(nn.Module):
         ``invalidate_folded_weight()``; switching the module between train() and eval() drops
         the cached copy as well.  The weights it was folded from stay allocated with it, so that no
         other weight takes their address."""
-        return self._kept("_folded", ops.bh4_fold)
-
-    def split_weight(self):
-        """folded_weight() as the inference kernel multiplies it (ops.bh4_fold_split), kept in the same way."""
-        return self._kept("_split", lambda w: ops.bh4_fold_split(w, False))
-
-    def block_weight(self):
-        """What forward_block's kernel for 8-bit codes takes in this mode."""
-        return self.folded_weight() if self.training else self.split_weight()
-
-    def _kept(self, name, make):
         w = self.projection.weight
         key = (w._version, w.data_ptr(), w.device)
-        cached = getattr(self, name, None)
+        cached = getattr(self, "_folded", None)
         if cached is None or cached[0] != key:
             alias = w.detach()
-            cached = (key, make(alias.contiguous()), alias)
-            setattr(self, name, cached)
+            cached = (key, ops.bh4_fold(alias.contiguous()), alias)
+            self._folded = cached
         return cached[1]
 
     def __getstate__(self):
         state = self.__dict__.copy()
-        for name in ("_folded", "_split"):
-            state.pop(name, None)         # derived from the weight, and names its address
+        state.pop("_folded", None)        # derived from the weight, and names its address
         return state
 
     def invalidate_folded_weight(self):
-        """Forget the folded copies of the BH4 weights: the next block-64 inference call folds again."""
-        self._folded = self._split = None
+        """Forget the folded copy of the BH4 weights: the next block-64 inference call folds again."""
+        self._folded = None
 
     def train(self, mode=True):
         if mode != self.training:
@@ -227,22 +215,17 @@ class Hashing(nn.Module):
 
     def forward_block(self, x, layer_norm=None):
         """8-bit codes: one kernel, (LayerNorm ->) BH4 on the matrix cores -> mix -> bias ->
-        code + score.  In eval() on the fp16 matrix cores; in train() the kernel of the training
-        forward, whose codes are the same bit for bit: a value within rounding of zero takes either
-        sign, and what a module in train() computes must not depend on whether gradients are recorded
-        (a checkpointed pass runs once without and once with them).  Other code lengths: the BH4
-        kernel, then mix + hash in a second one."""
+        code + score: that of the training forward, whose codes are the same bit for bit (a value within
+        rounding of zero takes either sign, and what a module computes must not depend on whether gradients
+        are recorded).  Other code lengths: the BH4 kernel, then mix + hash in a second one."""
         p = self.projection
         x = x.contiguous()
         if self.code_length == 8:
             lw = None if layer_norm is None else layer_norm.weight
             lb = None if layer_norm is None else layer_norm.bias
             eps = 0.0 if layer_norm is None else float(layer_norm.eps)
-            if self.training:
-                return ops.ln_bh4_block_hash(x, lw, lb, eps, self.folded_weight(), p.bias, self.num_table,
-                                             float(p.decay_coeff), float(1 - p.decay_coeff))
-            return ops.bh4_block_front(x, lw, lb, eps, self.split_weight(), p.num_repeat, p.weight.shape[1], p.padded_in_dim, p.bias,
-                                       self.num_table, float(p.decay_coeff), float(1 - p.decay_coeff))
+            return ops.ln_bh4_block_hash(x, lw, lb, eps, self.folded_weight(), p.bias, self.num_table,
+                                         float(p.decay_coeff), float(1 - p.decay_coeff))
         if layer_norm is not None:
             x = layer_norm(x)
         y = ops.bh4_block(x, self.folded_weight())
@@ -436,7 +419,7 @@ class LookupFFN(nn.Module):
             return None
         out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         if out is False:                  # the 64 x 64 blocks have changed since they were folded
-            self.hash.block_weight()
+            self.hash.folded_weight()
             out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         return None if out is False else out
 

@@ -1,4 +1,4 @@
-"""A module in train() computes the same whether gradients are recorded or not."""
+"""A module computes the same whether gradients are recorded or not."""
 import math
 from argparse import Namespace
 
@@ -32,8 +32,9 @@ def _same_rows(a, b):
 # size has 17 million projected values, a few of them within rounding of zero.
 @pytest.mark.parametrize("tokens,hidden,tables,block", [(17, 256, 128, 64), (300, 512, 64, 64), (2103, 500, 128, 64), (3000, 1024, 32, 64),
                                                         (65, 64, 32, 64), (40, 256, 32, 1), (1500, 768, 128, 1), (16384, 512, 128, 64)])
-def test_a_layer_in_train_with_and_without_gradients(tokens, hidden, tables, block):
-    layer = _layer(hidden, tables, block, 64)
+@pytest.mark.parametrize("training", [True, False])
+def test_a_layer_with_and_without_gradients(tokens, hidden, tables, block, training):
+    layer = _layer(hidden, tables, block, 64, training)
     x = torch.randn(tokens, hidden, device=DEV)
     code, score = layer.hash(x)
     out = layer(x)
@@ -48,15 +49,15 @@ def test_a_layer_in_train_with_and_without_gradients(tokens, hidden, tables, blo
 
 
 @pytest.mark.parametrize("training", [True, False])
-def test_the_blocks_weights_are_those_of_the_mode(training):
+def test_the_folded_blocks_follow_the_weights(training):
     layer = _layer(256, 32, 64, 64, training)
     x = torch.randn(50, 256, device=DEV)
     with torch.no_grad():
         for change in (lambda: None, lambda: layer.hash.projection.weight.mul_(1.5), lambda: layer.train(not training).train(training)):
             change()
             assert _same_rows(layer(x), layer._forward_operators(x, None))
-            kept = layer.hash.__dict__.get("_folded" if training else "_split")
-            assert kept is not None and kept[1] is layer.hash.block_weight()
+            kept = layer.hash.__dict__.get("_folded")
+            assert kept is not None and kept[1] is layer.hash.folded_weight()
 
 
 def test_an_encoder_layer_in_train_with_and_without_gradients():
