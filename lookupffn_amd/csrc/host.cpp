@@ -533,15 +533,20 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._folded = ((version, address, device), folded weights, what they were folded from), as Hashing.folded_weight keeps them: the
-// folded weights if they are w's.
+// hash._folded = ((version, address, device), folded weights, what they were folded from, stream, event), as Hashing.folded_weight keeps
+// them: the folded weights if they are w's and of this stream, on which they come before whatever is launched now.
 Tensor folded_of(PyObject *hash, const Tensor &w) {
     PyObject *kept = item(dict_of(hash), KEY_FOLDED);
-    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 3) return {};
+    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 5) return {};
     PyObject *key = PyTuple_GET_ITEM(kept, 0), *folded = PyTuple_GET_ITEM(kept, 1);
-    int64_t version = 0, address = 0;
+    int64_t version = 0, address = 0, made_on = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
-        !whole(PyTuple_GET_ITEM(key, 1), address) || !THPVariable_Check(folded))
+        !whole(PyTuple_GET_ITEM(key, 1), address) || !whole(PyTuple_GET_ITEM(kept, 3), made_on) || !THPVariable_Check(folded))
+        return {};
+    const hipStream_t stream = stream_on(w.device());
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (reinterpret_cast<hipStream_t>(made_on) != stream || hipStreamIsCapturing(stream, &capture) != hipSuccess ||
+        capture != hipStreamCaptureStatusNone)
         return {};
     const Tensor &f = THPVariable_Unpack(folded);
     const bool same = w._version() == (uint32_t)version && w.data_ptr() == reinterpret_cast<void *>(address) && f.device() == w.device() &&
@@ -555,11 +560,11 @@ struct WithoutInterpreter {
     ~WithoutInterpreter() { PyEval_RestoreThread(state); }
 };
 
-// forward(layer, x, residual or None, tokens up to which the one-launch form is taken) -> a tensor; None: not for this path;
-// False: the folded weights (Hashing.folded_weight) are not up to date
+// forward(layer, x, residual or None, tokens up to which the one-launch form is taken[, folded weights]) -> a tensor; None: not for
+// this path; False: the folded weights (Hashing.folded_weight) are wanted
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(n == 4, "forward: 4 arguments");
+    TORCH_CHECK(n == 4 || n == 5, "forward: 4 or 5 arguments");
     if (watched_over() || !plain(args[1])) Py_RETURN_NONE;
     Tensor x = THPVariable_Unpack(args[1]);
     const at::Device dev = x.device();
@@ -593,7 +598,17 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     if (grads && !c.trainable) Py_RETURN_NONE;
     Tensor folded;
-    if (!grads && c.form == BLOCK && !(folded = folded_of(parts.hash, params[2])).defined()) Py_RETURN_FALSE;
+    if (!grads && c.form == BLOCK) {
+        if (n == 4) {
+            folded = folded_of(parts.hash, params[2]);
+            if (!folded.defined()) Py_RETURN_FALSE;
+        } else {
+            if (!plain(args[4])) Py_RETURN_NONE;
+            folded = THPVariable_Unpack(args[4]);
+            if (folded.device() != dev || folded.scalar_type() != at::kFloat || folded.numel() != params[2].numel() || !folded.is_contiguous())
+                Py_RETURN_NONE;
+        }
+    }
     const int64_t fused_max = PyLong_AsLongLong(args[3]);
     if (fused_max == -1 && PyErr_Occurred()) return nullptr;
     Tensor out;

@@ -189,14 +189,28 @@ class Hashing(nn.Module):
         hand-written optimizers) do not advance: after such a write call
         ``invalidate_folded_weight()``; switching the module between train() and eval() drops
         the cached copy as well.  The weights it was folded from stay allocated with it, so that no
-        other weight takes their address."""
+        other weight takes their address.
+
+        The copy belongs to the stream it was made on: a call on another one waits for it and tells the
+        allocator.  What a stream capture runs is folded inside it, anew and for it alone: a copy made there
+        is not written before the first replay, and a copy made before may be dropped while the graph lives."""
         w = self.projection.weight
         key = (w._version, w.data_ptr(), w.device)
-        cached = getattr(self, "_folded", None)
-        if cached is None or cached[0] != key:
-            alias = w.detach()
-            cached = (key, ops.bh4_fold(alias.contiguous()), alias)
-            self._folded = cached
+        if not w.is_cuda:
+            return ops.bh4_fold(w.detach().contiguous())          # (an error)
+        with torch.cuda.device(w.device):
+            if torch.cuda.is_current_stream_capturing():
+                return ops.bh4_fold(w.detach().contiguous())
+            stream = torch.cuda.current_stream()
+            cached = getattr(self, "_folded", None)
+            if cached is None or cached[0] != key:
+                alias = w.detach()
+                folded = ops.bh4_fold(alias.contiguous())
+                cached = (key, folded, alias, stream.cuda_stream, stream.record_event())
+                self._folded = cached
+            elif cached[3] != stream.cuda_stream:
+                stream.wait_event(cached[4])
+                cached[1].record_stream(stream)
         return cached[1]
 
     def __getstate__(self):
@@ -418,9 +432,8 @@ class LookupFFN(nn.Module):
         if not host:
             return None
         out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
-        if out is False:                  # the 64 x 64 blocks have changed since they were folded
-            self.hash.folded_weight()
-            out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
+        if out is False:                  # no folded copy of the 64 x 64 blocks as they are, or one of another stream
+            out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS, self.hash.folded_weight())
         return None if out is False else out
 
     def _forward(self, hidden_states, residual=None):
@@ -480,8 +493,8 @@ class LookupFFN(nn.Module):
             if host is None:
                 host = _lib.host()
             out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS) if host else None
-            if out is False:
-                out = self._forward_host(hidden_states, residual)
+            if out is False:              # (as in _forward_host)
+                out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS, self.hash.folded_weight())
             if out is not None:
                 return out
         shape = hidden_states.shape[:-1]

@@ -378,6 +378,59 @@ def test_folded_blocks_are_those_of_the_weight_the_layer_has():
         assert torch.equal(twin(x), layer(x))
 
 
+@pytest.fixture(params=[True, False], ids=["host", "operators"])
+def either_path(request, monkeypatch):
+    if not request.param:
+        monkeypatch.setattr(_lib, "loaded_host", False)
+
+
+def test_folded_blocks_of_a_capture(either_path):
+    """What a capture folds is not there before a replay, and its replays take the weights as they are then."""
+    x = torch.randn(300, 256, device=DEV)
+    with torch.no_grad():
+        want = _layer(64).eval()(x)                           # (a layer of the same weights)
+        layer = _layer(64).eval()
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            static = layer(x)
+        assert torch.equal(layer(x), want)
+        for _ in range(4):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(static, layer(x))
+            layer.hash.projection.weight.mul_(0.75)
+            layer.hash.invalidate_folded_weight()
+            junk = [torch.full_like(layer.hash.projection.weight, float("nan")) for _ in range(8)]
+    assert len(junk) == 8
+
+
+def test_folded_blocks_made_on_another_stream(either_path):
+    """A call on another stream waits for them, and they stay until it has read them."""
+    x = torch.randn(300, 256, device=DEV)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.no_grad():
+        want = _layer(64).eval()(x)
+        layer = _layer(64).eval()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(20_000_000)                     # some 10 to 200 ms
+            layer(x)
+        with torch.cuda.stream(second):
+            got = layer(x)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        with torch.cuda.stream(second):
+            torch.cuda._sleep(20_000_000)
+            got = layer(x)
+        with torch.cuda.stream(first):
+            layer.hash.invalidate_folded_weight()
+            junk = [torch.full_like(layer.hash.projection.weight, float("nan")) for _ in range(8)]
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and len(junk) == 8
+
+
 # The backward exists twice, as one node in C++ and as the operators' autograd functions: at sizes where the forms of a kernel change
 # (few tokens' gradients to 384, one-launch column sums to 1024 rows, lists to 2048, the sorted scatter and its chunks), for every
 # gradient and for each one alone
