@@ -112,21 +112,28 @@ def row_format(wl):
     return 1 if wl["bf16"] else (2 if wl.get("f16") else 0)
 
 
+def records_plan(B, T, S, Do, fmt):
+    """The gather from the projection's record stream that the layer runs for a shape and row format (csrc/host.cpp, plan_for), parts 0
+    where one workgroup has all tables of a tile; None where it runs from codes and scores (host-side queries only)."""
+    from lookupffn_amd import _lib, ops
+    if T % 2:
+        return None
+    plan = _lib.GatherParts()
+    _lib.check(_lib.load().lffn_lookup_gather_parts_plan(B, T, S, Do, fmt, 1, ctypes.byref(plan)), "parts plan")
+    if plan.parts:
+        return plan
+    whole = ops.lookup_gather_records_plan(B, T, S, Do, fmt)
+    return whole and _lib.GatherParts(tokens_per_workgroup=whole[0], parts=0, record_stride=whole[1], bytes=whole[2])
+
+
 def gather_form(B, T, S, Do, fmt):
     """Which gather kernel the layer runs for a shape and row format, as a short string (host-side queries only)."""
-    import ctypes
-
     from lookupffn_amd import _lib
     lib = _lib.load()
-    plan = _lib.GatherParts()
-    _lib.check(lib.lffn_lookup_gather_parts_plan(B, T, S, Do, fmt, 1, ctypes.byref(plan)), "parts plan")
-    if plan.parts:
-        return f"record stream (four lanes per token), {plan.tokens_per_workgroup} tokens and 1/{plan.parts} of the tables per workgroup"
-    tok, stride, nbytes = ctypes.c_int32(0), ctypes.c_int64(0), ctypes.c_int64(0)
-    _lib.check(lib.lffn_lookup_gather_records_plan_rows(B, T, S, Do, fmt, ctypes.byref(tok), ctypes.byref(stride),
-                                                        ctypes.byref(nbytes)), "records plan")
-    if nbytes.value > 0:
-        return f"record stream (four lanes per token), {tok.value} tokens per workgroup"
+    plan = records_plan(B, T, S, Do, fmt)
+    if plan is not None:
+        share = f" and 1/{plan.parts} of the tables" if plan.parts else ""
+        return f"record stream (four lanes per token), {plan.tokens_per_workgroup} tokens{share} per workgroup"
     ws = ctypes.c_int64(0)
     _lib.check(lib.lffn_lookup_gather_workspace_bytes(B, T, S, Do, fmt, ctypes.byref(ws)), "workspace query")
     form = ctypes.c_int32(-1)
@@ -530,19 +537,19 @@ def main():
     with torch.no_grad():
         diag = None if block else proj.weight.reshape(proj.num_repeat, proj.weight.shape[1], proj.padded_in_dim)
     coefs = float(proj.decay_coeff), float(1 - proj.decay_coeff)
-    rec_plan = None
-    if not fused_layer and T % 2 == 0:
-        rec_plan = ops.lookup_gather_records_plan(B, T, S, Do, fmt)
+    rec_plan = None if fused_layer else records_plan(B, T, S, Do, fmt)
+    gather_step = ("two kernels: gather-add of parts of the tables, their sum + bias" if rec_plan and rec_plan.parts else
+                   "one kernel: gather-add + bias")
 
     # The stages on their own, by the entry points of the C ABI that LookupFFN.forward goes through
     lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
-    records = torch.empty(rec_plan[2] // 4, dtype=torch.int32, device=dev) if rec_plan is not None else None
+    records = torch.empty(rec_plan.bytes // 4, dtype=torch.int32, device=dev) if rec_plan is not None else None
     staged_out = torch.empty(B, Do, dtype=torch.float32, device=dev)
 
     def records_front():
         sizes = (B, H, proj.padded_in_dim, proj.num_repeat, proj.weight.shape[1], T)
         head = (x.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(), float(ln.eps))
-        tail = (proj.bias.data_ptr(), records.data_ptr(), rec_plan[1], rec_plan[0])
+        tail = (proj.bias.data_ptr(), records.data_ptr(), rec_plan.record_stride, rec_plan.tokens_per_workgroup)
         if block:
             _lib.check(lib.lffn_ln_bh4_block_hash_records_f32(*head, layer.hash.folded_weight().data_ptr(), *tail, *sizes, 64, *coefs, stream),
                        "lffn_ln_bh4_block_hash_records_f32")
@@ -551,9 +558,14 @@ def main():
                        "lffn_ln_project_hash_records_f32")
 
     def records_gather():
-        _lib.check(lib.lffn_lookup_gather_records_rows(records.data_ptr(), rec_plan[1], layer.tables.data_ptr(), layer.bias.data_ptr(), None,
-                                                       staged_out.data_ptr(), B, T, S, Do, fmt, rec_plan[0], stream),
-                   "lffn_lookup_gather_records_rows")
+        if rec_plan.parts:
+            _lib.check(lib.lffn_lookup_gather_parts_rows(ctypes.byref(rec_plan), None, None, layer.tables.data_ptr(), layer.bias.data_ptr(),
+                                                         None, staged_out.data_ptr(), records.data_ptr(), rec_plan.bytes, B, T, S, Do, fmt,
+                                                         stream), "lffn_lookup_gather_parts_rows")
+        else:
+            _lib.check(lib.lffn_lookup_gather_records_rows(records.data_ptr(), rec_plan.record_stride, layer.tables.data_ptr(),
+                                                           layer.bias.data_ptr(), None, staged_out.data_ptr(), B, T, S, Do, fmt,
+                                                           rec_plan.tokens_per_workgroup, stream), "lffn_lookup_gather_records_rows")
         return staged_out
 
     def step():
@@ -688,12 +700,12 @@ def main():
                  "synthetic (seeded N(0,1) tokens, seeded +-1/sqrt(D) sign diagonals, N(0,0.02) tables)"),
         "config": {"workload": wl["desc"], "tokens": B, "d_model": H, "fht_dim": layer.hash.projection.padded_in_dim,
                    "tables": T, "table_size": S, "d_out": Do,
-                   "step": ("one kernel: LayerNorm + BH4(block 64)x4 on fp16 MFMA, two terms a number, + mix + hash (weights folded once, "
+                   "step": ("one kernel: LayerNorm + BH4(block 64)x4 on fp32 MFMA + mix + hash (weights folded once, "
                             "outside the step)" + (", written as the gather's record stream" if rec_plan is not None else "") +
-                            "; one kernel: gather-add + bias") if block else
+                            "; " + gather_step) if block else
                            ("one kernel: LayerNorm + BH4(block 1)x4 + mix + hash + gather-add + bias" if fused_layer else
-                            ("one kernel: LayerNorm + BH4(block 1)x4 + mix + hash, written as the gather's record stream; "
-                             "one kernel: gather-add + bias") if rec_plan is not None else
+                            "one kernel: LayerNorm + BH4(block 1)x4 + mix + hash, written as the gather's record stream; " + gather_step
+                            if rec_plan is not None else
                             "one kernel: LayerNorm + BH4(block 1)x4 + mix + hash; one kernel: gather-add + bias")},
         "roofline": roofline,
         "stages_ms": ({"whole_layer": gather_ms} if fused_layer else

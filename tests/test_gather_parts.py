@@ -1,5 +1,6 @@
 """The gather whose table pairs are shared out over several workgroups (csrc/lookup_gather_quad.hip, lookup_gather.hip)."""
 import ctypes
+import sys
 
 import pytest
 import torch
@@ -120,3 +121,15 @@ def test_operators_take_it(B, T, Do, fmt):
     rows[1], weights = rows[1, order], score.clone()                                                # one token out of table form
     weights[1] = score[1, order]
     _check(ops.gather_add(rows, flat, weights), tables, code, score)
+
+
+# the benchmark times the layer's stages apart and asks for the layer's result bit for bit
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,bs", [(6144, 1), (2103, 1), (4096, 64)])
+def test_the_benchmarks_stages_are_the_layers(B, bs, monkeypatch, capsys):
+    import bench
+    assert _plan(B, 128, 768, 0, 1).parts
+    monkeypatch.setitem(bench.WORKLOADS, "parts", dict(B=B, H=768, T=128, S=S, Do=768, bf16=False, bs=bs, desc=""))
+    monkeypatch.setattr(sys, "argv", "bench.py --workload parts --steps 2 --warmup 1 --no-settle --no-cpu-baseline".split())
+    bench.main()
+    assert "of the tables per workgroup" in capsys.readouterr().out
