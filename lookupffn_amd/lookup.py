@@ -193,11 +193,12 @@ class Hashing(nn.Module):
 
         The copy belongs to the stream it was made on: a call on another one waits for it and tells the
         allocator.  What a stream capture runs is folded inside it, anew and for it alone: a copy made there
-        is not written before the first replay, and a copy made before may be dropped while the graph lives."""
+        is not written before the first replay, and a copy made before may be dropped while the graph lives.
+        A compiled call folds as well: a graph of operators knows no version and no stream."""
         w = self.projection.weight
+        if is_compiling() or not w.is_cuda:                       # (not on the GPU: an error)
+            return ops.bh4_fold(w.detach().contiguous())
         key = (w._version, w.data_ptr(), w.device)
-        if not w.is_cuda:
-            return ops.bh4_fold(w.detach().contiguous())          # (an error)
         with torch.cuda.device(w.device):
             if torch.cuda.is_current_stream_capturing():
                 return ops.bh4_fold(w.detach().contiguous())

@@ -406,6 +406,17 @@ def test_folded_blocks_of_a_capture(either_path):
     assert len(junk) == 8
 
 
+@pytest.mark.parametrize("block", [1, 64])
+def test_a_compiled_layer(block):
+    x = torch.randn(300, 256, device=DEV)
+    layer = _layer(block).eval()
+    compiled = torch.compile(layer, backend="eager")
+    with torch.no_grad():
+        for _ in range(2):                                    # (one launch and two may differ in the order of their sums)
+            assert torch.allclose(compiled(x), layer(x), rtol=1e-5, atol=1e-6)
+            layer.hash.projection.weight.mul_(0.75)
+
+
 def test_folded_blocks_made_on_another_stream(either_path):
     """A call on another stream waits for them, and they stay until it has read them."""
     x = torch.randn(300, 256, device=DEV)
