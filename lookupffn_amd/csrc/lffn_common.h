@@ -316,7 +316,6 @@ constexpr int TOUCH_SINK_BYTES = 256;
 // s_waitcnt immediates (vmcnt in bits 3:0, the other counters left alone)
 constexpr int WAIT_VMCNT_0 = 0x0F70;
 constexpr int WAIT_VMCNT_1 = 0x0F71;
-constexpr int WAIT_VMCNT_2 = 0x0F72;
 __device__ __forceinline__ void l2_touch(const char *base, uint32_t lane_offset, uint32_t lds_byte_addr) {
     // M0 is put back: the compiler reserves it for its own use and does not honour a clobber
     // declaration of it, so the statement must leave it as it found it
