@@ -469,7 +469,7 @@ def main_encoder(args):
         "vs_baseline": None, "dtype": "f32", "data": "synthetic (random token ids, random-init weights, seeded sign diagonals)",
         "config": {"workload": wl["desc"], "tokens": batch * seq, "layers": 12, "hidden": 768, "heads": 12,
                    "seq_len": seq, "batch": batch, "tables": wl["T"], "table_size": wl["S"],
-                   "attention": "torch scaled_dot_product_attention, fp32"},
+                   "attention": "this package's kernels, fp32 in and out, two half-precision terms a number"},
         "roofline": None, "cpu_baseline": None,
         "lookupffn_ms_per_forward": ffn_ms, "forward_ms_with_events": total_ms,
         "lookupffn_share": ffn_ms / total_ms,

@@ -809,8 +809,11 @@ int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float
  * the encoder's attention (PL/layer.py:23-26, 28), query, key and value together.  x: [M, K]; w[s]: [N, K];
  * bias[s]: [N] or NULL; residual: [M, N] or NULL; out[s]: [M, N], fp32.  w, bias and out are HOST arrays of
  * `sets` device pointers, read before the call returns.  1 <= sets <= 3; K a multiple of 32; K, N <= 2^20;
- * x and w[s] 16-byte aligned.  fp32 accuracy (2e-7 of the result's norm against 64 bits); infinities and
- * NaN as in an fp32 sum of products.  No output may overlap an input.
+ * x and w[s] 16-byte aligned.  fp32 accuracy (2e-7 of the result's norm against 64 bits; 5e-7 on the fp32
+ * matrix cores).  A number of x or w is held to 2^-22 of itself, or to 2^-44 of the largest of its row where
+ * that is more: one 2^22 times smaller than the largest of its row loses bits that fp32 keeps, which shows
+ * where everything near that largest meets zeros.  Infinities and NaN as in an fp32 sum of products.  No output
+ * may overlap an input.
  */
 int lffn_linear_f32(const float *x, const float *const *w, const float *const *bias, const float *residual,
                     float *const *out, int64_t sets, int64_t M, int64_t N, int64_t K, void *stream);
@@ -831,7 +834,10 @@ int lffn_linear_norm_f32(const float *x, const float *norm_weight, const float *
  * out[b, i, h, :] = sum_j p_j v[b, j, h, :],  p = softmax_j(q[b, i, h, :] . k[b, j, h, :] / 8 - 1000 (1 - mask[b, j]))
  * for heads of 64 columns, the encoder's attention (PL/layer.py:33-47), fp32.  q, k, v, out:
  * [B, L, heads, 64], 16-byte aligned; mask: [B, L], any numbers.  L <= LFFN_ATTENTION_MAX_KEYS.  A query
- * whose keys are all masked by an infinity gets zeros.
+ * whose keys are all masked by an infinity gets zeros.  fp32 accuracy (3.4e-7 against 64 bits; fp32 matrix
+ * cores 4.6e-7); a number is held to 2^-22 of itself, or to 2^-39 of the largest of its query, of eight
+ * neighbouring keys, of its column of the values or of the query's weights where that is more.  Infinities and
+ * NaN as in an fp32 sum of products.  out may not overlap an input.
  */
 #define LFFN_ATTENTION_MAX_KEYS 2048
 int lffn_attention_f32(const float *q, const float *k, const float *v, const float *mask, float *out, int64_t B,

@@ -15,7 +15,8 @@
 // but padding comes out 100 times closer to 64 bits than with -1000 in fp32.  Infinities and NaN are not carried by the split: a
 // wavefront with such results does its queries again in fp32, key by key (2.1 ms where every wavefront has to).
 //
-// 32 x 512 tokens, 12 heads: 110 us, 235 TFLOP/s of fp32 product (library, fp32 matrix cores: 490 and 35 for a copy); 113 with a scale
+// 32 x 512 tokens, 12 heads: 110 us, 235 TFLOP/s of fp32 product, of the same tensors again and again, 126 of three sets in turn (library,
+// fp32 matrix cores: 490 and 35 for a copy); 113 with a scale
 // for every key, 103 with one for all keys and one for all values taken from the first 64 (which lost numbers far smaller and sent
 // numbers 500 times larger through the fp32 loop).  The three products' matrix instructions are 67 us of that at the rate a large
 // half-precision product reaches, the vector work on a score (two multiply-adds, exp2, maximum, sum, split) as much again, partly

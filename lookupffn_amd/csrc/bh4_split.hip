@@ -1,4 +1,4 @@
-// BH4 with 64 x 64 blocks (PL/bh4/kernel.py:23-36) for inference and for the backward, on the fp16 matrix cores: the stages of
+// BH4 with 64 x 64 blocks (PL/bh4/kernel.py:23-36), hash and backward, on the fp16 matrix cores: the stages of
 // bh4_block.hip, (H_NB (x) I_64) * blockdiag(H_64 W[r,s,n]) each, with the weights and the tokens' rows as two half-precision terms
 // a number (split_mfma.h).
 //
@@ -9,14 +9,18 @@
 // Between two stages a token's row is scaled by a power of two, its largest to [2^14, 2^15), split, and written to the tile (hi and
 // lo, 4 bytes a number, as much as it was in fp32); both terms are then normal half-precision numbers or smaller than 2^-38 of the
 // row's largest, so neither needs a factor, the six instructions of a block add into one accumulator, and nothing overflows however a
-// stage amplifies.  A row's scale depends on that row alone: its results do not depend on its neighbours.
+// stage amplifies.  A row's scale depends on that row alone: its results do not depend on its neighbours.  A row with an infinity or
+// NaN comes out as NaN.
 //
-// What bounds it: the forward the weights' way from the L2 (2.1 GB in 128 us at 32768 tokens, D = 512, two repeats; 16 tokens a
-// workgroup) and the vector work (LayerNorm 18, a stage 9, hash 18 instructions a number), the backward the gradients it writes to
-// memory (0.8 GB in 205 us).  Products on the fp32 matrix cores (bh4_block.hip) take 16/3 of the time of these.  32768 tokens, D = 512,
-// two repeats: forward 235 -> 128-144 us, backward 280 -> 205; 16384, D = 1024 125 -> 75, 128 -> 103; 385, D = 512 18.5 -> 12.3, 18.7 ->
-// 12.2.  Tried: 32 tokens a workgroup in 4 wavefronts (124-149 us from build to build) and 8 (151), 64 in 8 (145), four blocks' weights
-// ahead instead of two (134).  Error of the last stage against 64 bits 2.4e-7 (fp32 matrix cores 3.2e-7), input gradient 2.2e-7 (3.1e-7).
+// What bounds it: the hash form the weights' way from the L2 (2.1 GB in 121 us at 32768 tokens, D = 512, two repeats; 16 tokens a
+// workgroup) and the vector work (LayerNorm 18, a stage 9, hash 18 instructions a number), the backward the 0.67 GB of gradients it
+// writes, together with what the kernels around it leave to be written.  Products on the fp32 matrix cores (bh4_block.hip) take 16/3 of
+// the time of these.  us, fp32 kernel -> this one, inputs in turn: hash 32768 tokens, D = 512, two repeats 202 -> 121; 16384, D = 1024
+// 113 -> 73; 385, D = 512 18.6 -> 12.3.  Backward in a training step, between the kernels that write its input and read its output:
+// 256 -> 256, 126 -> 130; alone, again and again, 232 -> 199, 118 -> 110; few tokens 18.7 -> 12.2 and 2103, D = 1024 35.6 -> 23.0.
+// Tried for the hash form: 32 tokens a workgroup in 4 wavefronts (124-149 us from build to build) and 8 (151), 64 in 8 (145), four
+// blocks' weights ahead instead of two (134).  Error of the last stage against 64 bits 2.4e-7 (fp32 matrix cores 3.2e-7), input gradient
+// 2.2e-7 (3.1e-7).
 //
 // A layer's forward stays on the fp32 matrix cores, with gradients and without (Hashing.forward_block, csrc/host.cpp): a projected
 // value within rounding of zero takes either sign, with the sign the derivative of its score turns round, and neither should a

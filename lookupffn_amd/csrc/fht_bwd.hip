@@ -19,7 +19,8 @@
 // Bound by instruction issue: some 120 vector instructions a number at two wavefronts per SIMD, 60 of them in the 7 transforms (a
 // transform's ten butterflies took 17 a number), the rest the diagonals, their gradients, the score's gradient and LayerNorm; a
 // transform's 8 matrix instructions of 32 clocks lie under the other wavefront's.  16384 rows of 768, 1024 points: 131 -> 89 us.  One
-// row's result is off by 2.0e-7 (butterflies 2.2e-7), a diagonal's gradient over 16384 rows by 2.6e-7 (2.8e-7).
+// row's result is off by 2.0e-7 (butterflies 2.2e-7), a diagonal's gradient over 16384 rows by 2.6e-7 (2.8e-7).  A row with an infinity
+// or NaN comes out as NaN, by itself.
 #include "split_mfma.h"
 
 #include "fht_bwd.h"

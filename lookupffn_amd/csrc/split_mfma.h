@@ -1,7 +1,8 @@
 // fp32 products on the fp16 matrix cores.
 //
 // A number x is taken as hi + lo / 2048: hi is x rounded to half precision, lo the rest times 2048 rounded to half precision (the
-// factor keeps it among half's normal numbers), together 22 bits and a sign.  Of a product of two such numbers
+// factor keeps it among half's normal numbers), together 22 bits and a sign (the split of Ootomo and Yokota, "Recovering single
+// precision accuracy from Tensor Cores while surpassing the FP32 theoretical peak performance", 2022).  Of a product of two such numbers
 //     hi hi  +  (hi lo + lo hi) / 2048
 // is formed, each partial product exact in the matrix core; what is left out (lo lo) and what the rounding of lo takes are at most
 // 2^-22 of the product, of either sign, and smaller still against a sum of many.  The two parts have an accumulator each: one
@@ -12,7 +13,8 @@
 //
 // Half precision's range: hi is off by less than 2^-12 of x from 6e-5 to 65504 and both together by less than 2^-36 below.  So what
 // goes in is scaled by powers of two (exact) to a size around 1, and what does not fit all the same comes out as an infinity or NaN:
-// kernels that use this look at their results and form the ones that are not finite again in plain fp32.
+// linear.hip and attention.hip look at their results and form the ones that are not finite again in plain fp32.  bh4_split.hip and
+// fht_bwd.hip scale by a row's largest number, so that a finite row fits; one with an infinity or NaN comes out as NaN, by itself.
 #pragma once
 
 #include "lffn_common.h"

@@ -109,7 +109,7 @@ class Attention(nn.Module):
         gradients, heads of 64 columns, and every part of the module the one it was built with.  A module in train() keeps the
         library's with and without gradients: a checkpointed pass runs both, and the LookupFFN behind turns a rounding into another
         table row.  Against the library's fp32
-        products and attention the encoder layer takes, 32 x 512 tokens of 768, 619 us instead of 1279, 4 x 128 tokens 86 instead of
+        products and attention the encoder layer takes, 32 x 512 tokens of 768, 624 us instead of 1279, 4 x 128 tokens 86 instead of
         164, 16 tokens 86 instead of 166, and its attention half is half as far from 64 bits (5e-7 against 9e-7)."""
         linears = (self.query, self.key, self.value, self.dense)
         if not (x.is_cuda and x.dim() == 3 and x.dtype == torch.float32 and x.numel() > 0 and type(x) in (torch.Tensor, nn.Parameter)
