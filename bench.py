@@ -551,8 +551,9 @@ def main():
         head = (x.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(), float(ln.eps))
         tail = (proj.bias.data_ptr(), records.data_ptr(), rec_plan.record_stride, rec_plan.tokens_per_workgroup)
         if block:
-            _lib.check(lib.lffn_ln_bh4_block_hash_records_f32(*head, layer.hash.folded_weight().data_ptr(), *tail, *sizes, 64, *coefs, stream),
-                       "lffn_ln_bh4_block_hash_records_f32")
+            block_front = _lib.BlockFront(*head[1:3], layer.hash.split_weight().data_ptr(), tail[0], None, None, *tail[1:3], *sizes[1:],
+                                          tail[3], head[3], *coefs)
+            _lib.check(lib.lffn_bh4_block_front_split_f32(ctypes.byref(block_front), x.data_ptr(), B, stream), "lffn_bh4_block_front_split_f32")
         else:
             _lib.check(lib.lffn_ln_project_hash_records_f32(*head, diag.data_ptr(), *tail, *sizes, *coefs, stream),
                        "lffn_ln_project_hash_records_f32")

@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 12
+#define LFFN_ABI_VERSION 13
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -762,15 +762,14 @@ int lffn_lookup_backward_f32(const int32_t *code, const float *score, const floa
 int lffn_lookup_inner_f32(const int32_t *code, const float *g, const float *tables, float *grad_score,
                           int64_t B, int64_t T, int64_t S, int64_t Do, void *stream);
 
-/* ------------------------- 64 x 64 blocks on the fp16 matrix cores: inference and backward */
+/* ------------------------- 64 x 64 blocks on the fp16 matrix cores: forward and backward */
 
 /*
- * The kernels of lffn_ln_bh4_block_hash_f32 (inference) and lffn_bh4_block_bwd_f32 with every number as two
- * half-precision terms, which is faster and closer to 64 bits (csrc/bh4_split.hip).  They are rounded differently: a
- * code may differ where its z is within 1e-6 of the row's size of zero.  The layer runs this backward; its forward is
- * lffn_ln_bh4_block_hash_f32 (or _records_f32) without gradients, whose codes are those of
- * lffn_ln_bh4_block_hash_train_f32 bit for bit.  lffn_bh4_block_front_split_f32 is for callers that run no training
- * forward beside it, lffn_bh4_block_bwd_f32 for those that want fp32 products.
+ * The kernels of lffn_ln_bh4_block_hash_f32, lffn_ln_bh4_block_hash_train_f32 and lffn_bh4_block_bwd_f32 with every
+ * number as two half-precision terms, which is faster and closer to 64 bits (csrc/bh4_split.hip).  They are rounded
+ * differently: a code may differ where its z is within 1e-6 of the row's size of zero.  The layer runs these,
+ * forward with gradients and without (lffn_bh4_block_front_train_split_f32 and lffn_bh4_block_front_split_f32, whose codes
+ * and scores are the same bit for bit); those with fp32 products are for callers that want them.
  *
  * lffn_bh4_fold_split_f32: the 64-point transform of lffn_bh4_fold_mode_f32 (transposed == 0: mode 0, else
  * mode 1) of stages x num_block blocks, split.  w: [stages, num_block, 64, 64], num_block a power of two up to
@@ -796,6 +795,13 @@ typedef struct lffn_block_front {
     float ln_eps, decay, residual;
 } lffn_block_front;
 int lffn_bh4_block_front_split_f32(const lffn_block_front *front, const float *x, int64_t B, void *stream);
+
+/*
+ * The same with what the backward needs (lffn_ln_bh4_block_hash_train_f32): codes and scores, no records; z [B, T*8];
+ * stage_inputs [R, J-1, B, D], NULL if J == 1; row_stats [B, 2], every row's mean and 1/sigma, NULL without LayerNorm.
+ */
+int lffn_bh4_block_front_train_split_f32(const lffn_block_front *front, const float *x, float *z, float *stage_inputs,
+                                         float *row_stats, int64_t B, void *stream);
 
 /* lffn_bh4_block_bwd_f32 with weights of lffn_bh4_fold_split_f32, transposed != 0. */
 int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float *g_x, float *stage_grads, int64_t B,

@@ -16,7 +16,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # LOOKUPFFN_HIP_LIB points at another build of the same ABI (e.g. a tuning build)
 LIB_PATH = os.environ.get("LOOKUPFFN_HIP_LIB") or os.path.join(_PKG_DIR, "liblookupffn_hip.so")
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 LFFN_OK = 0
 LFFN_ERR_BAD_ARG = -1
@@ -138,6 +138,7 @@ class BlockFront(ctypes.Structure):
 
 
 SIGNATURES["lffn_bh4_block_front_split_f32"] = [ctypes.POINTER(BlockFront), _vp, _i64, _vp]
+SIGNATURES["lffn_bh4_block_front_train_split_f32"] = [ctypes.POINTER(BlockFront), _vp, _vp, _vp, _vp, _i64, _vp]
 SIGNATURES["lffn_lookup_ffn_fused_layer_f32"] = [ctypes.POINTER(FusedLayer), _vp, _vp, _vp, _i64, _vp]
 SIGNATURES["lffn_lookup_ffn_fused_layer_rows"] = [ctypes.POINTER(FusedLayer), ctypes.c_int32, _vp, _vp, _vp, _i64, _vp]
 

@@ -30,7 +30,7 @@
 // on the accumulators (x is read again and normalised with the kept statistics) and
 // the code and score of every 8 columns: a group is split over the lane pair
 // (l, l+16), whose second lane continues the first lane's running sum and product so
-// that the operations run in column order.
+// that the operations run in column order.  The layer itself takes bh4_split.hip's forms.
 #include "lffn_common.h"
 
 // the mix and the score keep the reference's operation order: no fused multiply-add

@@ -1,4 +1,4 @@
-// BH4 with 64 x 64 blocks (PL/bh4/kernel.py:23-36), hash and backward, on the fp16 matrix cores: the stages of
+// BH4 with 64 x 64 blocks (PL/bh4/kernel.py:23-36), forward and backward, on the fp16 matrix cores: the stages of
 // bh4_block.hip, (H_NB (x) I_64) * blockdiag(H_64 W[r,s,n]) each, with the weights and the tokens' rows as two half-precision terms
 // a number (split_mfma.h).
 //
@@ -16,16 +16,18 @@
 // workgroup) and the vector work (LayerNorm 18, a stage 9, hash 18 instructions a number), the backward the 0.67 GB of gradients it
 // writes, together with what the kernels around it leave to be written.  Products on the fp32 matrix cores (bh4_block.hip) take 16/3 of
 // the time of these.  us, fp32 kernel -> this one, inputs in turn: hash 32768 tokens, D = 512, two repeats 202 -> 121; 16384, D = 1024
-// 113 -> 73; 385, D = 512 18.6 -> 12.3.  Backward in a training step, between the kernels that write its input and read its output:
+// 113 -> 73; 385, D = 512 18.6 -> 12.3.  Training form, which writes z and the stages' inputs (0.54 GB at
+// 32768, D = 512, two repeats): 278 -> 209; 385, D = 512 24.9 -> 15.5.  Backward in a training step, between the kernels that write its input and read its output:
 // 256 -> 256, 126 -> 130; alone, again and again, 232 -> 199, 118 -> 110; few tokens 18.7 -> 12.2 and 2103, D = 1024 35.6 -> 23.0.
 // Tried for the hash form: 32 tokens a workgroup in 4 wavefronts (124-149 us from build to build) and 8 (151), 64 in 8 (145), four
 // blocks' weights ahead instead of two (134).  Error of the last stage against 64 bits 2.4e-7 (fp32 matrix cores 3.2e-7), input gradient
 // 2.2e-7 (3.1e-7).
 //
-// A layer's forward stays on the fp32 matrix cores, with gradients and without (Hashing.forward_block, csrc/host.cpp): a projected
-// value within rounding of zero takes either sign, with the sign the derivative of its score turns round, and neither should a
-// training step's gradients change with the kernel nor a pass without gradients differ from one with them.  The layer takes the
-// backward from here; the hash form is an operator of its own (lffn_bh4_block_front_split_f32), for programs that run no training forward.
+// A layer runs this forward with gradients and without, in train() and eval() (Hashing.forward_block, csrc/host.cpp): a projected
+// value within rounding of zero takes either sign, with the sign the derivative of its score turns round, and a pass without
+// gradients must not differ from one with them.  The training form is the hash form with stores: its codes and scores are the same
+// bit for bit.  Against 64 bits, LayerNorm included, 200 rows of D = 512, fp32 kernel -> this one: z 3.1e-7 -> 2.4e-7, stage inputs
+// 2.4e-7 -> 1.8e-7, scores 4.5e-7 -> 3.4e-7 (rows spread over e^1.5 in size: 3.2e-7, 2.4e-7, 4.6e-7 -> 2.4e-7, 1.9e-7, 3.9e-7).
 #include "split_mfma.h"
 
 // the mix and the score keep the reference's operation order: no fused multiply-add
@@ -157,9 +159,12 @@ struct SplitArgs {
     uint32_t *records;     // instead of codes and scores: the record stream of the four-lanes-per-token gather,
     int64_t rec_stride;    // [T/2][rec_stride][3] (lffn_quad_record_slot)
     int rec_tile;          // tokens per workgroup of the gather the records are written for
+    float *z;              // training: [B, T*8] z, kept for the backward
+    float *row_stats;      // training, with LayerNorm: [B, 2] every row's mean and 1/sigma
     const float *gz;       // backward: [B, T*8] gradient of z
     float *g_x;            // backward: [R, B, H]
-    float *stage_grads;    // backward: [R, J, B, D] gradient before the product of each stage
+    float *stage_save;     // training: [R, J-1, B, D] inputs of stages 1 .. J-1;
+                           // backward: [R, J, B, D] gradient before the product of each stage
     int64_t B;
     int H, R, J, T;
     float decay, residual;
@@ -186,8 +191,12 @@ __device__ __forceinline__ void split4(f32x4 v, uint2 &hi, uint2 &lo) {
 // gradient P_s = (H_NB (x) I) G_{s+1} is also written to memory: the gradient w.r.t. the folded weights is the per-block product
 // P_s^T U_s over all tokens (U_s = the stage's input, which the forward saved), formed by the caller.  First gradient: decay * grad z;
 // result: grad x of this repeat = G_0[:, :H] + residual * grad z[:, :H].
-template <int NB, bool BWD, int BG>
+enum Form { HASH, TRAIN, BACKWARD };       // TRAIN: the hash form that also keeps what the backward needs
+
+template <int NB, Form FORM, int BG>
 __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split_kernel(SplitArgs a) {
+    constexpr bool BWD = FORM == BACKWARD;
+    constexpr bool SAVE = FORM != HASH;           // the numbers between the stages go to memory
     static_assert(BG == 1 || (BG == 4 && NB >= 4), "the wide form: four groups of blocks");
     constexpr int TOK = 16;                       // tokens per workgroup
     constexpr int NWAVE = 4 * BG;
@@ -343,7 +352,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 if constexpr (NBW > 2) most = fmaxf(most, lane_xor<32>(most));
                 const PowerOfTwo s = scale_to_one(most);
                 if (tid % (16 * NBW) == 0) unscale[row] = inv * (s.inverse * (1 / TOP));
-                const bool live = BWD && tok_base + row < B;
+                const bool live = SAVE && tok_base + row < B;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     put(row, (n * BG + k) * BS + c4, v[k] * (s.scale * TOP));
@@ -367,7 +376,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             const f32x4 scale = inv_w * (s.scale * TOP);
 #pragma unroll
             for (int n = 0; n < NBW; ++n) put(c, n * BS + 16 * ow + 4 * kq, acc[n] * scale);
-            if (BWD && tok_base + c < B) {
+            if (SAVE && tok_base + c < B) {
                 float *o = save + size_t(c) * D + 16 * ow + 4 * kq;
                 const f32x4 f = inv_w * inv_x;
 #pragma unroll
@@ -418,7 +427,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
 #pragma unroll 1
         for (int s = J - 1; s >= 0; --s) {
             butterflies();
-            hand_over(a.stage_grads + ((size_t(r) * J + s) * B + tok_base) * D);
+            hand_over(a.stage_save + ((size_t(r) * J + s) * B + tok_base) * D);
             product(s);
         }
     } else {
@@ -480,6 +489,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 if (tid % LANES == 0) {
                     stats[2 * row] = mean;
                     stats[2 * row + 1] = rstd;
+                    if (SAVE && r == 0 && tok < B) *reinterpret_cast<float2 *>(a.row_stats + 2 * tok) = make_float2(mean, rstd);
                 }
             }
             float most = 0.f;
@@ -505,7 +515,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         for (int s = 0; s < J; ++s) {
             product(s);
             butterflies();
-            if (s + 1 < J) hand_over(nullptr);
+            if (s + 1 < J) hand_over(SAVE ? a.stage_save + ((size_t(r) * (J - 1) + s) * B + tok_base) * D : nullptr);
         }
         last_strides();
     }
@@ -550,6 +560,8 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                              *reinterpret_cast<const f32x4 *>(lnb_s + xc);
             const f32x4 z = a.decay * (inv_w * inv_x) * acc[n] + a.residual * xv +      // (decay times a power of two: as decay * y)
                             *reinterpret_cast<const f32x4 *>(pbias_s + xc);
+            if (SAVE && token < B && r * D + xc < ncols)
+                __builtin_nontemporal_store(z, reinterpret_cast<f32x4 *>(a.z + token * ncols + r * D + xc));
             return z;
         };
         // Columns 8 g .. 8 g + 3 sit in the lane with even kq, 8 g + 4 .. 8 g + 7 in lane + 16.  Two groups of four are taken at a
@@ -627,12 +639,12 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     }
 }
 
-template <int NB, bool BWD, int BG>
+template <int NB, Form FORM, int BG>
 int launch_form(const SplitArgs &a, hipStream_t st) {
     constexpr int TOK = 16, D = BS * NB;
-    constexpr size_t lds_bytes = 2 * TOK * (2 * D + 16) + (BG > 1 ? TOK * (D + PAD) * 4 : 0) + 7 * TOK * 4 + (BWD ? 0 : 3 * D * 4);
+    constexpr size_t lds_bytes = 2 * TOK * (2 * D + 16) + (BG > 1 ? TOK * (D + PAD) * 4 : 0) + 7 * TOK * 4 + (FORM == BACKWARD ? 0 : 3 * D * 4);
     static_assert(lds_bytes <= 160 * 1024);
-    auto kern = bh4_split_kernel<NB, BWD, BG>;
+    auto kern = bh4_split_kernel<NB, FORM, BG>;
     static LdsGrant granted;      // one record per kernel instantiation
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(kern), lds_bytes, granted)) return LFFN_ERR_LAUNCH;
     const dim3 grid((unsigned)((a.B + TOK - 1) / TOK), (unsigned)a.R);
@@ -645,21 +657,21 @@ int launch_form(const SplitArgs &a, hipStream_t st) {
 // 12.2; 600, D = 256, four repeats 9.6 -> 9.7 / 10.4 -> 9.4.  Two rounds of it: 4096, D = 512, two repeats 19.1 -> 26.8 / 30.7 -> 29.7.
 constexpr int64_t WIDE_WORKGROUPS = 256;
 
-template <int NB, bool BWD>
+template <int NB, Form FORM>
 int launch_block(const SplitArgs &a, hipStream_t st) {
     if constexpr (NB >= 4)
-        if ((a.B + 15) / 16 * a.R <= WIDE_WORKGROUPS) return launch_form<NB, BWD, 4>(a, st);
-    return launch_form<NB, BWD, 1>(a, st);
+        if ((a.B + 15) / 16 * a.R <= WIDE_WORKGROUPS) return launch_form<NB, FORM, 4>(a, st);
+    return launch_form<NB, FORM, 1>(a, st);
 }
 
-template <bool BWD>
+template <Form FORM>
 int dispatch_block(const SplitArgs &a, int64_t D, hipStream_t st) {
     switch (D / BS) {
-        case 1: return launch_block<1, BWD>(a, st);
-        case 2: return launch_block<2, BWD>(a, st);
-        case 4: return launch_block<4, BWD>(a, st);
-        case 8: return launch_block<8, BWD>(a, st);
-        default: return launch_block<16, BWD>(a, st);
+        case 1: return launch_block<1, FORM>(a, st);
+        case 2: return launch_block<2, FORM>(a, st);
+        case 4: return launch_block<4, FORM>(a, st);
+        case 8: return launch_block<8, FORM>(a, st);
+        default: return launch_block<16, FORM>(a, st);
     }
 }
 
@@ -681,27 +693,48 @@ extern "C" int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t s
     return lffn_launch_status();
 }
 
-extern "C" int lffn_bh4_block_front_split_f32(const lffn_block_front *f, const float *x, int64_t B, void *stream) {
+namespace {
+
+// the hash forms' arguments, checked
+int front_args(const lffn_block_front *f, const float *x, int64_t B, SplitArgs &a) {
     LFFN_REQUIRE(f, LFFN_ERR_BAD_ARG);
     const int64_t H = f->H, D = f->D, R = f->R, J = f->J, T = f->T;
-    LFFN_REQUIRE(B >= 0 && R >= 1 && J >= 1 && D >= 1 && H >= 1 && H <= D && T >= 1, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(B >= 0 && R >= 1 && J >= 1 && D >= 1 && H >= 1 && H <= D && T >= 0, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(H % 4 == 0 && J <= 64, LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(lffn_is_pow2(D) && D >= BS && D <= 1024, LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(R <= 4096 && B <= (int64_t(1) << 31) - 1 && T <= (1 << 24), LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(T * 8 <= R * D, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(!f->ln_weight || (f->ln_bias && f->ln_eps >= 0.f), LFFN_ERR_BAD_ARG);
-    if (B == 0) return LFFN_OK;
+    if (B == 0 || T == 0) return LFFN_OK;
     LFFN_REQUIRE(x && f->w_split && (f->records || (f->codes && f->scores)), LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(!f->records || (T % 2 == 0 && lffn_record_layout_ok(B, f->record_stride, f->tokens_per_workgroup) &&
                                  (uintptr_t)f->records % 4 == 0), LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(lffn_aligned16(x) && lffn_aligned16(f->w_split) && lffn_aligned16(f->proj_bias) && lffn_aligned16(f->ln_weight) &&
                      lffn_aligned16(f->ln_bias), LFFN_ERR_BAD_ARG);
-    SplitArgs a{};
     a.x = x; a.ln_w = f->ln_weight; a.ln_b = f->ln_bias; a.ln_eps = f->ln_eps; a.w = f->w_split;
     a.wscale = f->w_split + R * J * D * BS; a.pbias = f->proj_bias; a.codes = f->codes; a.scores = f->scores;
     a.records = f->records; a.rec_stride = f->record_stride; a.rec_tile = f->tokens_per_workgroup;
     a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = f->decay; a.residual = f->residual;
-    return dispatch_block<false>(a, D, static_cast<hipStream_t>(stream));
+    return LFFN_OK;
+}
+
+}  // namespace
+
+extern "C" int lffn_bh4_block_front_split_f32(const lffn_block_front *f, const float *x, int64_t B, void *stream) {
+    SplitArgs a{};
+    const int rc = front_args(f, x, B, a);
+    return rc != LFFN_OK || B == 0 || f->T == 0 ? rc : dispatch_block<HASH>(a, f->D, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int lffn_bh4_block_front_train_split_f32(const lffn_block_front *f, const float *x, float *z, float *stage_inputs,
+                                                     float *row_stats, int64_t B, void *stream) {
+    SplitArgs a{};
+    const int rc = front_args(f, x, B, a);
+    if (rc != LFFN_OK || B == 0 || f->T == 0) return rc;
+    LFFN_REQUIRE(f->codes && f->scores && !f->records && z && (stage_inputs || f->J == 1) && (row_stats || !f->ln_weight), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(z) && lffn_aligned16(stage_inputs) && (uintptr_t)row_stats % 8 == 0, LFFN_ERR_BAD_ARG);
+    a.z = z; a.stage_save = stage_inputs; a.row_stats = row_stats;
+    return dispatch_block<TRAIN>(a, f->D, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float *g_x, float *stage_grads, int64_t B,
@@ -716,7 +749,7 @@ extern "C" int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_spl
     LFFN_REQUIRE(g_z && w_split_t && g_x && stage_grads, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(lffn_aligned16(g_z) && lffn_aligned16(w_split_t) && lffn_aligned16(g_x) && lffn_aligned16(stage_grads), LFFN_ERR_BAD_ARG);
     SplitArgs a{};
-    a.gz = g_z; a.w = w_split_t; a.wscale = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_grads = stage_grads;
+    a.gz = g_z; a.w = w_split_t; a.wscale = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_save = stage_grads;
     a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = decay; a.residual = residual;
-    return dispatch_block<true>(a, D, static_cast<hipStream_t>(stream));
+    return dispatch_block<BACKWARD>(a, D, static_cast<hipStream_t>(stream));
 }

@@ -54,9 +54,8 @@ using torch::autograd::variable_list;
     X(lffn_lookup_gather_ws_f32)            \
     X(lffn_lookup_gather_ws_bf16)           \
     X(lffn_lookup_gather_ws_f16)            \
-    X(lffn_ln_bh4_block_hash_train_f32)     \
-    X(lffn_ln_bh4_block_hash_f32)           \
-    X(lffn_ln_bh4_block_hash_records_f32)   \
+    X(lffn_bh4_block_front_split_f32)       \
+    X(lffn_bh4_block_front_train_split_f32) \
     X(lffn_bh4_fold_split_f32)              \
     X(lffn_bh4_fold_mode_f32)               \
     X(lffn_lookup_scatter_workspace_bytes)  \
@@ -221,10 +220,17 @@ using Params = std::array<Tensor, 6>;
 // Floats of the split weights (lffn_bh4_fold_split_f32).
 int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 64); }
 
-// folded: the 64 x 64 blocks' weights.  Their kernel is the training forward's: with the split products of the backward (csrc/bh4_split.hip,
-// 252 us a call instead of 333 at 32768 x 512, 128 tables of 512 columns) a value within rounding of zero took the other sign and its token other table rows,
-// two in four million, so that a layer computed one thing with gradients recorded and another without (a checkpointed pass runs both).
-void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor &x, const float *residual, Tensor &out, int64_t B,
+// The front end of 64 x 64 blocks; split: their weights (lffn_bh4_fold_split_f32).  The kernel is the training forward's, so that a layer
+// computes the same codes with gradients recorded and without (a checkpointed pass runs both).
+lffn_block_front block_front(const Config &c, const Params &p, const Tensor &split) {
+    lffn_block_front f{};
+    f.ln_weight = f32(p[0]); f.ln_bias = f32(p[1]); f.w_split = f32(split); f.proj_bias = f32(p[3]);
+    f.H = c.H; f.D = c.D; f.R = c.R; f.J = c.J; f.T = c.T;
+    f.ln_eps = (float)c.eps; f.decay = (float)c.decay; f.residual = (float)c.residual;
+    return f;
+}
+
+void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &x, const float *residual, Tensor &out, int64_t B,
            int64_t fused_max) {
     const at::Device dev = x.device();
     void *st = stream_on(dev);
@@ -249,9 +255,13 @@ void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor 
         if (c.form == DIAG)
             CALL(lffn_ln_project_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), rp, plan.stride,
                  plan.tokens, B, c.H, c.D, c.R, c.J, c.T, decay, res, st);
-        else
-            CALL(lffn_ln_bh4_block_hash_records_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), rp, plan.stride,
-                 plan.tokens, B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
+        else {
+            lffn_block_front front = block_front(c, p, split);
+            front.records = rp;
+            front.record_stride = plan.stride;
+            front.tokens_per_workgroup = plan.tokens;
+            CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
+        }
         if (plan.parts.parts)
             CALL(lffn_lookup_gather_parts_rows, &plan.parts, nullptr, nullptr, p[4].data_ptr(), f32(p[5]), residual, f32(out), rp, plan.bytes,
                  B, c.T, c.S, c.Do, (int32_t)c.fmt, st);
@@ -265,9 +275,12 @@ void infer(const Config &c, const Params &p, const Tensor &folded, const Tensor 
     if (c.form == DIAG)
         CALL(lffn_ln_project_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(p[2]), f32(p[3]), nullptr, cp, f32(scores), B, c.H,
              c.D, c.R, c.J, c.T, decay, res, st);
-    else
-        CALL(lffn_ln_bh4_block_hash_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), B, c.H, c.D,
-             c.R, c.J, c.T, 64, decay, res, st);
+    else {
+        lffn_block_front front = block_front(c, p, split);
+        front.codes = cp;
+        front.scores = f32(scores);
+        CALL(lffn_bh4_block_front_split_f32, &front, f32(x), B, st);
+    }
     gather(c, codes, scores, p[4], p[5], residual, out, B, plan, st);
 }
 
@@ -429,10 +442,12 @@ void train(const Config &c, const Params &p, const Tensor &x, const Tensor &resi
     } else {
         stage = empty_f32({c.R, c.J - 1, B, c.D}, dev);
         stats = empty_f32({B, 2}, dev);
-        Tensor folded = at::empty_like(p[2]);
-        CALL(lffn_bh4_fold_mode_f32, f32(p[2]), f32(folded), c.R * c.J * (c.D / 64), 64, 0, st);
-        CALL(lffn_ln_bh4_block_hash_train_f32, f32(x), f32(p[0]), f32(p[1]), eps, f32(folded), f32(p[3]), cp, f32(scores), f32(z),
-             c.J > 1 ? f32(stage) : nullptr, f32(stats), B, c.H, c.D, c.R, c.J, c.T, 64, decay, res, st);
+        Tensor split = empty_f32({split_words(c)}, dev);
+        CALL(lffn_bh4_fold_split_f32, f32(p[2]), f32(split), c.R * c.J, c.D / 64, 64, 0, st);
+        lffn_block_front front = block_front(c, p, split);
+        front.codes = cp;
+        front.scores = f32(scores);
+        CALL(lffn_bh4_block_front_train_split_f32, &front, f32(x), f32(z), c.J > 1 ? f32(stage) : nullptr, f32(stats), B, st);
     }
     gather(c, codes, scores, p[4], p[5], f32(residual), out, B, plan_for(c, B, false), st);
 
@@ -533,24 +548,24 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._folded = ((version, address, device), folded weights, what they were folded from, stream, event), as Hashing.folded_weight keeps
-// them: the folded weights if they are w's and of this stream, on which they come before whatever is launched now.
-Tensor folded_of(PyObject *hash, const Tensor &w) {
+// hash._folded = ((version, address, device), folded weights, what they were folded from, stream, event, split weights), as Hashing keeps
+// them: the split weights if they are w's and of this stream, on which they come before whatever is launched now.
+Tensor split_of(PyObject *hash, const Tensor &w, int64_t words) {
     PyObject *kept = item(dict_of(hash), KEY_FOLDED);
-    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 5) return {};
-    PyObject *key = PyTuple_GET_ITEM(kept, 0), *folded = PyTuple_GET_ITEM(kept, 1);
+    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 6) return {};
+    PyObject *key = PyTuple_GET_ITEM(kept, 0), *split = PyTuple_GET_ITEM(kept, 5);
     int64_t version = 0, address = 0, made_on = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
-        !whole(PyTuple_GET_ITEM(key, 1), address) || !whole(PyTuple_GET_ITEM(kept, 3), made_on) || !THPVariable_Check(folded))
+        !whole(PyTuple_GET_ITEM(key, 1), address) || !whole(PyTuple_GET_ITEM(kept, 3), made_on) || !THPVariable_Check(split))
         return {};
     const hipStream_t stream = stream_on(w.device());
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (reinterpret_cast<hipStream_t>(made_on) != stream || hipStreamIsCapturing(stream, &capture) != hipSuccess ||
         capture != hipStreamCaptureStatusNone)
         return {};
-    const Tensor &f = THPVariable_Unpack(folded);
+    const Tensor &f = THPVariable_Unpack(split);
     const bool same = w._version() == (uint32_t)version && w.data_ptr() == reinterpret_cast<void *>(address) && f.device() == w.device() &&
-                      f.numel() == w.numel();
+                      f.numel() == words;
     return same ? f : Tensor();
 }
 
@@ -560,8 +575,8 @@ struct WithoutInterpreter {
     ~WithoutInterpreter() { PyEval_RestoreThread(state); }
 };
 
-// forward(layer, x, residual or None, tokens up to which the one-launch form is taken[, folded weights]) -> a tensor; None: not for
-// this path; False: the folded weights (Hashing.folded_weight) are wanted
+// forward(layer, x, residual or None, tokens up to which the one-launch form is taken[, split weights]) -> a tensor; None: not for
+// this path; False: the split weights (Hashing.split_weight) are wanted
 PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     TORCH_CHECK(n == 4 || n == 5, "forward: 4 or 5 arguments");
@@ -597,15 +612,15 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
         for (const Tensor &t : params) grads = grads || t.requires_grad();
     }
     if (grads && !c.trainable) Py_RETURN_NONE;
-    Tensor folded;
+    Tensor split;
     if (!grads && c.form == BLOCK) {
         if (n == 4) {
-            folded = folded_of(parts.hash, params[2]);
-            if (!folded.defined()) Py_RETURN_FALSE;
+            split = split_of(parts.hash, params[2], split_words(c));
+            if (!split.defined()) Py_RETURN_FALSE;
         } else {
             if (!plain(args[4])) Py_RETURN_NONE;
-            folded = THPVariable_Unpack(args[4]);
-            if (folded.device() != dev || folded.scalar_type() != at::kFloat || folded.numel() != params[2].numel() || !folded.is_contiguous())
+            split = THPVariable_Unpack(args[4]);
+            if (split.device() != dev || split.scalar_type() != at::kFloat || split.numel() != split_words(c) || !split.is_contiguous())
                 Py_RETURN_NONE;
         }
     }
@@ -613,7 +628,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (fused_max == -1 && PyErr_Occurred()) return nullptr;
     Tensor out;
     {
-        // (from here on only what is owned here is used: x, the residual, the parameters and the folded weights)
+        // (from here on only what is owned here is used: x, the residual, the parameters and the split weights)
         const WithoutInterpreter unlocked;
         // any layout of x and any shape and type of the residual, as the Python path makes them
         x = x.contiguous();
@@ -623,7 +638,7 @@ PyObject *forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
             (!residual.defined() || reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 == 0)) {
             out = empty_f32(sizes, dev);
             if (grads) train(c, params, x, residual, out, B);
-            else infer(c, params, folded, x, f32(residual), out, B, fused_max);
+            else infer(c, params, split, x, f32(residual), out, B, fused_max);
         }
     }
     if (!out.defined()) Py_RETURN_NONE;

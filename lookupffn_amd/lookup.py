@@ -106,8 +106,9 @@ class BlockProjectHash(torch.autograd.Function):
     def forward(ctx, x, weight, bias, T, decay):
         x = x.contiguous()
         w = weight.contiguous()
-        folded = ops.bh4_fold_mode(w, 0)
-        code, score, z, stage_in = ops.bh4_block_hash_train(x, folded, bias, T, float(decay), float(1 - decay))
+        R, J, NB, bs, _ = w.shape
+        code, score, z, stage_in, _ = ops.bh4_block_front_train(x, None, None, 0.0, ops.bh4_fold_split(w, False), R, J, NB * bs, bias, T,
+                                                                float(decay), float(1 - decay))
         ctx.save_for_backward(x, w, z, stage_in)
         ctx.has_bias = bias is not None
         ctx.decay = float(decay)
@@ -195,24 +196,39 @@ class Hashing(nn.Module):
         allocator.  What a stream capture runs is folded inside it, anew and for it alone: a copy made there
         is not written before the first replay, and a copy made before may be dropped while the graph lives.
         A compiled call folds as well: a graph of operators knows no version and no stream."""
+        kept = self._kept_folds()
+        return ops.bh4_fold(self.projection.weight.detach().contiguous()) if kept is None else kept[1]
+
+    def split_weight(self):
+        """The same for 8-bit codes' kernel (ops.bh4_fold_split), kept in the same way."""
+        kept = self._kept_folds()
+        return ops.bh4_fold_split(self.projection.weight.detach().contiguous(), False) if kept is None else kept[5]
+
+    def _kept_folds(self):
+        """((version, address, device), folded, what it was folded from, stream, event, split), split for 8-bit codes;
+        None where nothing is kept."""
         w = self.projection.weight
         if is_compiling() or not w.is_cuda:                       # (not on the GPU: an error)
-            return ops.bh4_fold(w.detach().contiguous())
+            return None
         key = (w._version, w.data_ptr(), w.device)
         with torch.cuda.device(w.device):
             if torch.cuda.is_current_stream_capturing():
-                return ops.bh4_fold(w.detach().contiguous())
+                return None
             stream = torch.cuda.current_stream()
             cached = getattr(self, "_folded", None)
             if cached is None or cached[0] != key:
                 alias = w.detach()
-                folded = ops.bh4_fold(alias.contiguous())
-                cached = (key, folded, alias, stream.cuda_stream, stream.record_event())
+                source = alias.contiguous()
+                folded = ops.bh4_fold(source)
+                split = ops.bh4_fold_split(source, False) if self.code_length == 8 else None
+                cached = (key, folded, alias, stream.cuda_stream, stream.record_event(), split)
                 self._folded = cached
             elif cached[3] != stream.cuda_stream:
                 stream.wait_event(cached[4])
-                cached[1].record_stream(stream)
-        return cached[1]
+                for t in cached[1], cached[5]:
+                    if t is not None:
+                        t.record_stream(stream)
+        return cached
 
     def __getstate__(self):
         state = self.__dict__.copy()
@@ -230,7 +246,7 @@ class Hashing(nn.Module):
 
     def forward_block(self, x, layer_norm=None):
         """8-bit codes: one kernel, (LayerNorm ->) BH4 on the matrix cores -> mix -> bias ->
-        code + score: that of the training forward, whose codes are the same bit for bit (a value within
+        code + score: the training forward's without its stores, the same codes bit for bit (a value within
         rounding of zero takes either sign, and what a module computes must not depend on whether gradients
         are recorded).  Other code lengths: the BH4 kernel, then mix + hash in a second one."""
         p = self.projection
@@ -239,8 +255,8 @@ class Hashing(nn.Module):
             lw = None if layer_norm is None else layer_norm.weight
             lb = None if layer_norm is None else layer_norm.bias
             eps = 0.0 if layer_norm is None else float(layer_norm.eps)
-            return ops.ln_bh4_block_hash(x, lw, lb, eps, self.folded_weight(), p.bias, self.num_table,
-                                         float(p.decay_coeff), float(1 - p.decay_coeff))
+            return ops.bh4_block_front(x, lw, lb, eps, self.split_weight(), p.num_repeat, p.weight.shape[1], p.padded_in_dim, p.bias,
+                                       self.num_table, float(p.decay_coeff), float(1 - p.decay_coeff))
         if layer_norm is not None:
             x = layer_norm(x)
         y = ops.bh4_block(x, self.folded_weight())
@@ -344,9 +360,9 @@ class LnBlockProjectHash(torch.autograd.Function):
     def forward(ctx, x, ln_weight, ln_bias, eps, weight, bias, T, decay):
         x = x.contiguous()
         w = weight.contiguous()
-        folded = ops.bh4_fold_mode(w, 0)
-        code, score, z, stage_in, stats = ops.ln_bh4_block_hash_train(x, ln_weight, ln_bias, float(eps), folded, bias, T,
-                                                                      float(decay), float(1 - decay))
+        R, J, NB, bs, _ = w.shape
+        code, score, z, stage_in, stats = ops.bh4_block_front_train(x, ln_weight, ln_bias, float(eps), ops.bh4_fold_split(w, False), R, J,
+                                                                    NB * bs, bias, T, float(decay), float(1 - decay))
         ctx.save_for_backward(x, ln_weight, ln_bias, w, z, stage_in, stats)
         ctx.eps = float(eps)
         ctx.has_bias = bias is not None
@@ -434,7 +450,7 @@ class LookupFFN(nn.Module):
             return None
         out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS)
         if out is False:                  # no folded copy of the 64 x 64 blocks as they are, or one of another stream
-            out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS, self.hash.folded_weight())
+            out = host.forward(self, x, residual, self.FUSED_LAYER_MAX_TOKENS, self.hash.split_weight())
         return None if out is False else out
 
     def _forward(self, hidden_states, residual=None):
@@ -495,7 +511,7 @@ class LookupFFN(nn.Module):
                 host = _lib.host()
             out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS) if host else None
             if out is False:              # (as in _forward_host)
-                out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS, self.hash.folded_weight())
+                out = host.forward(self, hidden_states, residual, self.FUSED_LAYER_MAX_TOKENS, self.hash.split_weight())
             if out is not None:
                 return out
         shape = hidden_states.shape[:-1]

@@ -434,8 +434,8 @@ _L.define("bh4_block_front(Tensor x, Tensor? ln_w, Tensor? ln_b, float eps, Tens
           "float decay, float residual) -> (Tensor, Tensor)")
 
 
-def _bh4_block_front_impl(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
-    """(LayerNorm ->) 64 x 64 blocks -> mix -> hash -> (codes [B,T], scores [B,T])."""
+def _block_front(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
+    """The arguments of the split front ends, with new codes and scores."""
     _lib.require_gpu(x, ln_w, ln_b, w_split, bias)
     for t in (x, ln_w, ln_b, w_split, bias):
         assert t is None or (t.dtype == torch.float32 and t.is_contiguous())
@@ -447,6 +447,13 @@ def _bh4_block_front_impl(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, 
     scores = torch.empty(B, T, dtype=torch.float32, device=x.device)
     front = _lib.BlockFront(_lib.ptr(ln_w), _lib.ptr(ln_b), _lib.ptr(w_split), _lib.ptr(bias), codes.data_ptr(), scores.data_ptr(), None,
                             0, H, D, R, J, T, 0, eps, decay, residual)
+    return front, codes, scores
+
+
+def _bh4_block_front_impl(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
+    """(LayerNorm ->) 64 x 64 blocks -> mix -> hash -> (codes [B,T], scores [B,T])."""
+    front, codes, scores = _block_front(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual)
+    B, H = x.shape
     with _dev_guard(x):
         rc = _lib.load().lffn_bh4_block_front_split_f32(ctypes.byref(front), _lib.ptr(x), B, _lib.stream_of(x))
     _lib.check(rc, f"lffn_bh4_block_front_split_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
@@ -459,6 +466,36 @@ _L.impl("bh4_block_front", _bh4_block_front_impl, "CUDA")
 @torch.library.register_fake("lookupffn::bh4_block_front")
 def _(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
     return torch.empty(x.shape[0], T, dtype=torch.int32, device=x.device), x.new_empty(x.shape[0], T)
+
+
+_L.define("bh4_block_front_train(Tensor x, Tensor? ln_w, Tensor? ln_b, float eps, Tensor w_split, int R, int J, int D, Tensor? bias, "
+          "int T, float decay, float residual) -> (Tensor, Tensor, Tensor, Tensor, Tensor)")
+
+
+def _bh4_block_front_train_impl(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
+    """bh4_block_front with what the backward needs -> (codes [B,T], scores [B,T], z [B,T*8], stage_inputs [R,J-1,B,D],
+    row_stats [B,2] = every row's mean and 1/sigma, empty without LayerNorm)."""
+    front, codes, scores = _block_front(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual)
+    B, H = x.shape
+    z = x.new_empty(B, T * 8)
+    stage_in = x.new_empty(R, max(J - 1, 0), B, D)
+    stats = x.new_empty(B if ln_w is not None else 0, 2)
+    with _dev_guard(x):
+        rc = _lib.load().lffn_bh4_block_front_train_split_f32(
+            ctypes.byref(front), _lib.ptr(x), _lib.ptr(z), _lib.ptr(stage_in) if J > 1 else None,
+            _lib.ptr(stats) if ln_w is not None else None, B, _lib.stream_of(x))
+    _lib.check(rc, f"lffn_bh4_block_front_train_split_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
+    return codes, scores, z, stage_in, stats
+
+
+_L.impl("bh4_block_front_train", _bh4_block_front_train_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::bh4_block_front_train")
+def _(x, ln_w, ln_b, eps, w_split, R, J, D, bias, T, decay, residual):
+    B = x.shape[0]
+    return (torch.empty(B, T, dtype=torch.int32, device=x.device), x.new_empty(B, T), x.new_empty(B, T * 8),
+            x.new_empty(R, max(J - 1, 0), B, D), x.new_empty(B if ln_w is not None else 0, 2))
 
 
 _L.define("bh4_block_bwd_split(Tensor g_z, Tensor w_split_t, int R, int J, int D, int H, float decay, float residual) -> (Tensor, Tensor)")
@@ -1258,6 +1295,7 @@ bh4_block = torch.ops.lookupffn.bh4_block
 mix_code_score = torch.ops.lookupffn.mix_code_score
 bh4_fold_split = torch.ops.lookupffn.bh4_fold_split
 bh4_block_front = torch.ops.lookupffn.bh4_block_front
+bh4_block_front_train = torch.ops.lookupffn.bh4_block_front_train
 bh4_block_bwd_split = torch.ops.lookupffn.bh4_block_bwd_split
 bh4_fold_mode = torch.ops.lookupffn.bh4_fold_mode
 bh4_block_hash_train = torch.ops.lookupffn.bh4_block_hash_train

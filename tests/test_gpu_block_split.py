@@ -88,6 +88,43 @@ def test_against_64_bits(B, H, D, R, T, with_ln):
         assert _rel(g_x[r][some], (G + 0.3 * g)[:, :H]) <= REL
 
 
+# both forms of the kernel (few and many workgroups), rows around the 16 of a tile, columns short of D, codes short of them
+@pytest.mark.parametrize("B,H,D,R,T", [(1, 64, 64, 2, 16), (33, 100, 128, 2, 30), (70, 256, 256, 1, 32), (4200, 200, 256, 1, 32),
+                                       (31, 512, 512, 2, 100), (2300, 500, 512, 2, 128), (17, 768, 1024, 1, 128), (4100, 1024, 1024, 1, 128)])
+@pytest.mark.parametrize("with_ln", [True, False])
+def test_what_the_training_form_keeps(B, H, D, R, T, with_ln):
+    """Codes and scores of the form without gradients, bit for bit; z, the stages' inputs and the rows' statistics against 64 bits."""
+    gen = torch.Generator(device=DEV).manual_seed(B + D + 1)
+    J, NB = 4, D // 64
+    x, w = 1.5 * _randn(gen, B, H) + 0.3, _randn(gen, R, J, NB, 64, 64) / math.sqrt(64 * D)
+    lw, lb = (1 + 0.1 * _randn(gen, H), 0.1 * _randn(gen, H)) if with_ln else (None, None)
+    bias = 0.05 * _randn(gen, T * 8) if with_ln else None
+    split = ops.bh4_fold_split(w, False)
+    codes, scores = ops.bh4_block_front(x, lw, lb, 1e-5, split, R, J, D, bias, T, 0.7, 0.3)
+    got = ops.bh4_block_front_train(x, lw, lb, 1e-5, split, R, J, D, bias, T, 0.7, 0.3)
+    assert torch.equal(got[0], codes) and torch.equal(got[1], scores)
+    _, _, z, stages, stats = got
+    few = min(B, 20)
+    part = ops.bh4_block_front_train(x[:few], lw, lb, 1e-5, split, R, J, D, bias, T, 0.7, 0.3)
+    assert torch.equal(part[2], z[:few]) and torch.equal(part[3], stages[:, :, :few])
+    some = list(range(min(B, 40))) + [B - 1]
+    h = x[some].double().cpu()
+    if with_ln:
+        assert _rel(stats[some, 0], h.mean(1)) <= REL and _rel(stats[some, 1], (h.var(1, unbiased=False) + 1e-5).rsqrt()) <= REL
+        h = torch.nn.functional.layer_norm(h, (H,), lw.double().cpu(), lb.double().cpu(), 1e-5)
+    h = torch.cat([h, torch.zeros(len(some), D - H, dtype=torch.float64)], 1)
+    w64, HD, want = w.double().cpu(), _hadamard(D), []
+    for r in range(R):
+        u = h
+        for j in range(J):
+            if j > 0:
+                assert _rel(stages[r, j - 1][some], u) <= 2 * REL          # (LayerNorm's rounding as large again)
+            u = _blocks(w64[r, j], u) @ HD
+        want.append(0.7 * u + 0.3 * h)
+    assert _rel(z[some], torch.cat(want, 1)[:, :T * 8] + (bias.double().cpu() if with_ln else 0)) <= 2 * REL
+    assert torch.equal((z.view(B, T, 8) > 0).mul(2 ** torch.arange(7, -1, -1, device=DEV)).sum(-1).int(), codes)
+
+
 @pytest.mark.parametrize("B", [40, 9000])
 def test_scales_and_rows_of_their_own(B):
     """Any size of gradients and weights, rows of very different sizes side by side, and a row that is not finite stays alone."""
