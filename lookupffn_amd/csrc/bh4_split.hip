@@ -12,13 +12,16 @@
 // stage amplifies.  A row's scale depends on that row alone: its results do not depend on its neighbours.  A row with an infinity or
 // NaN comes out as NaN.
 //
-// What bounds it: the hash form the weights' way from the L2 (2.1 GB in 121 us at 32768 tokens, D = 512, two repeats; 16 tokens a
-// workgroup) and the vector work (LayerNorm 18, a stage 9, hash 18 instructions a number), the backward the 0.67 GB of gradients it
-// writes, together with what the kernels around it leave to be written.  Products on the fp32 matrix cores (bh4_block.hip) take 16/3 of
-// the time of these.  us, fp32 kernel -> this one, inputs in turn: hash 32768 tokens, D = 512, two repeats 202 -> 121; 16384, D = 1024
-// 113 -> 73; 385, D = 512 18.6 -> 12.3.  Training form, which writes z and the stages' inputs (0.54 GB at
-// 32768, D = 512, two repeats): 278 -> 209; 385, D = 512 24.9 -> 15.5.  Backward in a training step, between the kernels that write its input and read its output:
-// 256 -> 256, 126 -> 130; alone, again and again, 232 -> 199, 118 -> 110; few tokens 18.7 -> 12.2 and 2103, D = 1024 35.6 -> 23.0.
+// What bounds it: vector work (LayerNorm 18, a stage 9, hash 18 instructions a number) and the latencies between it and the products;
+// with all weights from the L1 the hash form at 32768 tokens, D = 512, two repeats takes 113 us instead of 121, so the weights' way from
+// the L2 (2.1 GB) is no more than a part.  The training form and the backward write 0.54 and 0.67 GB at that size, which go out at the
+// memory's rate and hide little behind the products (137 and 128 us without them).  They go out as whole rows, turned round through LDS
+// in fp32, where a wavefront stored 64 bytes of sixteen rows straight from its accumulators: 196 -> 166 and 200 -> 173 us, 209 -> 168 and
+// 250 -> 195 in a training step; 16384, D = 1024 115 -> 99 and 106 -> 98; 32768, D = 256, four repeats 184 -> 175 and 185 -> 162.  Stores held
+// back until the next product: 193 and 217, from spills.
+// Products on the fp32 matrix cores (bh4_block.hip) take 16/3 of the time of these.  us, fp32 kernel -> this one, inputs in turn: hash
+// 32768 tokens, D = 512, two repeats 202 -> 121; 16384, D = 1024 113 -> 73; 385, D = 512 18.6 -> 12.3.  Training form 278 -> 168; 385,
+// D = 512 24.9 -> 15.5.  Backward in a training step 256 -> 195; few tokens 18.7 -> 12.2 and 2103, D = 1024 35.6 -> 23.0.
 // Tried for the hash form: 32 tokens a workgroup in 4 wavefronts (124-149 us from build to build) and 8 (151), 64 in 8 (145), four
 // blocks' weights ahead instead of two (134).  Error of the last stage against 64 bits 2.4e-7 (fp32 matrix cores 3.2e-7), input gradient
 // 2.2e-7 (3.1e-7).
@@ -203,15 +206,16 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     constexpr int NBW = NB / BG;                  // blocks of a wavefront: bg + BG * n, n < NBW
     const float *__restrict__ x = a.x;
     const int64_t B = a.B;
-    const int H = a.H, R = a.R, J = a.J;
+    const int H = a.H, J = a.J;
     constexpr int D = BS * NB;
-    constexpr int LDP = 2 * D + 16;               // bytes of a tile row: 16 rows' reads of a fragment fall on different banks
-    constexpr int LDR = D + PAD;
+    constexpr int LDR = D + PAD;                  // floats of a row in fp32
+    constexpr int LDP = 4 * LDR;                  // bytes of a tile row, hi and lo: 16 rows' reads of a fragment fall on different banks
     constexpr int AHEAD = NBW < 2 ? NBW : 2;     // blocks whose weights are on their way
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    char *const tile = lds;                       // [2][TOK] rows of LDP bytes: hi, lo
-    float *const wide_tile = reinterpret_cast<float *>(lds + 2 * TOK * LDP);          // wide form: [TOK][LDR] in fp32
-    float *const stats = wide_tile + (BG > 1 ? TOK * LDR : 0);                        // [TOK][2]: LayerNorm's mean and 1/sigma
+    char *const tile = lds;                       // [TOK] rows of LDP bytes: hi, then lo
+    // [TOK][LDR] in fp32: the narrow form's in the tile's place, where a row's two terms lie within its own numbers
+    float *const rows32 = reinterpret_cast<float *>(lds + (BG > 1 ? TOK * LDP : 0));
+    float *const stats = rows32 + TOK * LDR;      // [TOK][2]: LayerNorm's mean and 1/sigma
     float *const unscale = stats + 2 * TOK;       // [TOK] 1 / scale of a token's row
     float *const most_s = unscale + TOK;          // [TOK][4] largest of a token's row in a wavefront's columns
     float *const lnw_s = most_s + 4 * TOK;        // hash form: [D] each LayerNorm's weight and bias, the projection's bias
@@ -259,8 +263,8 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         const char *p = tile + c * LDP + (n * BG + bg) * 128 + kq * 32;
         f[0] = *reinterpret_cast<const uint4 *>(p);
         f[1] = *reinterpret_cast<const uint4 *>(p + 16);
-        f[2] = *reinterpret_cast<const uint4 *>(p + TOK * LDP);
-        f[3] = *reinterpret_cast<const uint4 *>(p + TOK * LDP + 16);
+        f[2] = *reinterpret_cast<const uint4 *>(p + 2 * D);
+        f[3] = *reinterpret_cast<const uint4 *>(p + 2 * D + 16);
     };
     // four numbers of a token's row into the tile
     auto put = [&](int row, int col, f32x4 v) {
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         split4(v, hi, lo);
         char *p = tile + row * LDP + col * 2;
         *reinterpret_cast<uint2 *>(p) = hi;
-        *reinterpret_cast<uint2 *>(p + TOK * LDP) = lo;
+        *reinterpret_cast<uint2 *>(p + 2 * D) = lo;
     };
 
     // What the accumulators are to be multiplied with: the inverse scales of the lane's four columns of the weights and of its token.
@@ -319,20 +323,33 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         }
     };
 
+    // The accumulators times f as rows of fp32 in LDS, and the four rows of a wavefront from there, NB vectors a lane: vector i of
+    // lane l is row row_of(i), columns col_of(i) .. + 3.
+    constexpr int ROW_LANES = D < 256 ? D / 4 : 64, ROW_VALUES = D < 256 ? 1 : D / 256;
+    auto row_of = [&](int i) { return 4 * wave + (D < 256 ? i * (64 / ROW_LANES) + lane / ROW_LANES : i / ROW_VALUES); };
+    auto col_of = [&](int i) { return 4 * (lane % ROW_LANES) + (D < 256 ? 0 : 256 * (i % ROW_VALUES)); };
+    auto to_rows = [&](f32x4 f) {
+#pragma unroll
+        for (int n = 0; n < NBW; ++n)
+            *reinterpret_cast<f32x4 *>(rows32 + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n] * f;
+    };
+    auto from_rows = [&](f32x4 (&v)[NB]) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) v[i] = *reinterpret_cast<const f32x4 *>(rows32 + row_of(i) * LDR + col_of(i));
+    };
+
     // The accumulators (after butterflies()) become the next product's tile, and the rows of D floats at `save` where they are kept:
     // a token's row is scaled by the power of two that takes its largest to [2^14, 2^15).
     auto hand_over = [&](float *save) {
         if constexpr (BG > 1) {
             // strides 2 and 1, which take four wavefronts' accumulators: a pass over the tile in fp32, 16 bytes of blocks
             // 4 n .. 4 n + 3 per thread; the 16 NBW threads of a row are neighbours in a wavefront
-#pragma unroll
-            for (int n = 0; n < NBW; ++n)
-                *reinterpret_cast<f32x4 *>(wide_tile + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n] * inv_w;
+            to_rows(inv_w);
             if (bg == 0 && ow == 0 && kq == 0) unscale[c] = inv_x;
             __syncthreads();
             if (tid < TOK * 16 * NBW) {
                 const int row = tid / (16 * NBW), n = (tid / 16) % NBW, c4 = (tid % 16) * 4;
-                const float *p = wide_tile + row * LDR + n * BG * BS + c4;
+                const float *p = rows32 + row * LDR + n * BG * BS + c4;
                 const float inv = unscale[row];
                 f32x4 v[4];
 #pragma unroll
@@ -360,6 +377,39 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 }
             }
             __syncthreads();
+        } else if constexpr (SAVE) {
+            // the rows go out as whole lines: through LDS in fp32, and a wavefront has four rows from there
+            __syncthreads();                      // every wavefront has read this stage's input
+            to_rows(inv_w);
+            if (ow == 0 && kq == 0) unscale[c] = inv_x;
+            __syncthreads();
+            f32x4 v[NB];
+            from_rows(v);
+#pragma unroll
+            for (int i = 0; i < NB; i += ROW_VALUES) {
+                const int row = row_of(i);
+                float most = 0.f;
+#pragma unroll
+                for (int k = i; k < i + ROW_VALUES; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) most = fmaxf(most, fabsf(v[k][e]));
+                most = fmaxf(most, lane_xor<1>(most));
+                most = fmaxf(most, lane_xor<2>(most));
+                most = fmaxf(most, lane_xor<4>(most));
+                most = fmaxf(most, lane_xor<8>(most));
+                if constexpr (ROW_LANES == 32) most = fmaxf(most, lane_xor<16>(most));
+                if constexpr (ROW_LANES == 64) most = rows_most(most);
+                const PowerOfTwo s = scale_to_one(most);
+                const float inv = unscale[row];
+                const bool live = tok_base + row < B;
+#pragma unroll
+                for (int k = i; k < i + ROW_VALUES; ++k) {
+                    if (live) __builtin_nontemporal_store(v[k] * inv, reinterpret_cast<f32x4 *>(save + size_t(row) * D + col_of(k)));
+                    put(row, col_of(k), v[k] * (s.scale * TOP));
+                }
+                if (lane % ROW_LANES == 0) unscale[row] = inv * (s.inverse * (1 / TOP));
+            }
+            __syncthreads();
         } else {
             f32x4 m4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -376,12 +426,6 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             const f32x4 scale = inv_w * (s.scale * TOP);
 #pragma unroll
             for (int n = 0; n < NBW; ++n) put(c, n * BS + 16 * ow + 4 * kq, acc[n] * scale);
-            if (SAVE && tok_base + c < B) {
-                float *o = save + size_t(c) * D + 16 * ow + 4 * kq;
-                const f32x4 f = inv_w * inv_x;
-#pragma unroll
-                for (int n = 0; n < NBW; ++n) __builtin_nontemporal_store(acc[n] * f, reinterpret_cast<f32x4 *>(o + n * BS));
-            }
             __syncthreads();
         }
     };
@@ -390,11 +434,11 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         if constexpr (BG > 1) {
 #pragma unroll
             for (int n = 0; n < NBW; ++n)
-                *reinterpret_cast<f32x4 *>(wide_tile + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n];
+                *reinterpret_cast<f32x4 *>(rows32 + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n];
             __syncthreads();
             if (tid < TOK * 16 * NBW) {
                 const int row = tid / (16 * NBW), n = (tid / 16) % NBW, c4 = (tid % 16) * 4;
-                float *p = wide_tile + row * LDR + n * BG * BS + c4;
+                float *p = rows32 + row * LDR + n * BG * BS + c4;
                 f32x4 v[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4 *>(p + k * BS);
@@ -406,7 +450,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             __syncthreads();
 #pragma unroll
             for (int n = 0; n < NBW; ++n)
-                acc[n] = *reinterpret_cast<const f32x4 *>(wide_tile + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq);
+                acc[n] = *reinterpret_cast<const f32x4 *>(rows32 + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq);
         }
     };
 
@@ -523,7 +567,22 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     if constexpr (BWD) {
         // grad x of this repeat: the first H columns, plus the residual path of the mix
         const int ncols = a.T * 8;
-        if (token < B) {
+        if constexpr (BG == 1) {                  // whole rows again
+            __syncthreads();
+            to_rows(inv_w * inv_x);
+            __syncthreads();
+            f32x4 v[NB];
+            from_rows(v);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int64_t tok = tok_base + row_of(i);
+                const int xc = col_of(i);
+                if (tok < B && xc < H) {
+                    if (r * D + xc < ncols) v[i] = v[i] + a.residual * *reinterpret_cast<const f32x4 *>(a.gz + tok * ncols + r * D + xc);
+                    *reinterpret_cast<f32x4 *>(a.g_x + (size_t(r) * B + tok) * H + xc) = v[i];
+                }
+            }
+        } else if (token < B) {
 #pragma unroll
             for (int n = 0; n < NBW; ++n) {
                 const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq;
@@ -560,9 +619,28 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                              *reinterpret_cast<const f32x4 *>(lnb_s + xc);
             const f32x4 z = a.decay * (inv_w * inv_x) * acc[n] + a.residual * xv +      // (decay times a power of two: as decay * y)
                             *reinterpret_cast<const f32x4 *>(pbias_s + xc);
-            if (SAVE && token < B && r * D + xc < ncols)
+            if (SAVE && BG > 1 && token < B && r * D + xc < ncols)
                 __builtin_nontemporal_store(z, reinterpret_cast<f32x4 *>(a.z + token * ncols + r * D + xc));
             return z;
+        };
+        if constexpr (SAVE && BG == 1) {          // z as whole rows
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) acc[n] = form_z(n);
+            to_rows((f32x4){1.f, 1.f, 1.f, 1.f});
+            __syncthreads();
+            f32x4 v[NB];
+            from_rows(v);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int64_t tok = tok_base + row_of(i);
+                const int col = r * D + col_of(i);
+                if (tok < B && col < ncols) __builtin_nontemporal_store(v[i], reinterpret_cast<f32x4 *>(a.z + tok * ncols + col));
+            }
+            __syncthreads();
+        }
+        auto z_of = [&](int n) {
+            if constexpr (SAVE && BG == 1) return acc[n];
+            else return form_z(n);
         };
         // Columns 8 g .. 8 g + 3 sit in the lane with even kq, 8 g + 4 .. 8 g + 7 in lane + 16.  Two groups of four are taken at a
         // time and exchanged between the lanes' rows, so that an even row has all eight columns of the first and an odd row of the
@@ -571,7 +649,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
 #pragma unroll
         for (int i = 0; i < ITEMS; i += 2) {
             const int i1 = i + 1 < ITEMS ? i + 1 : i;              // (a single one: with itself, the odd rows' copy is not used)
-            const f32x4 za = form_z(i), zb = form_z(i1);
+            const f32x4 za = z_of(i), zb = z_of(i1);
             float z[8];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -642,7 +720,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
 template <int NB, Form FORM, int BG>
 int launch_form(const SplitArgs &a, hipStream_t st) {
     constexpr int TOK = 16, D = BS * NB;
-    constexpr size_t lds_bytes = 2 * TOK * (2 * D + 16) + (BG > 1 ? TOK * (D + PAD) * 4 : 0) + 7 * TOK * 4 + (FORM == BACKWARD ? 0 : 3 * D * 4);
+    constexpr size_t lds_bytes = (BG > 1 ? 2 : 1) * TOK * (D + PAD) * 4 + 7 * TOK * 4 + (FORM == BACKWARD ? 0 : 3 * D * 4);
     static_assert(lds_bytes <= 160 * 1024);
     auto kern = bh4_split_kernel<NB, FORM, BG>;
     static LdsGrant granted;      // one record per kernel instantiation
