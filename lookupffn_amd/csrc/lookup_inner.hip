@@ -251,10 +251,22 @@ int launch_inner(const InnerArgs &a, hipStream_t stream) {
 
 }  // namespace
 
+// Table pairs per workgroup of the four-lanes-per-token kernel (lookup_inner_quad.hip), 0: another kernel.  A workgroup of 1024 tokens
+// fetches its g once per slice for its pairs, so as many of them as still give the chip most of a round; one pair where that is one
+// round.  us at 4 | 2 | 1 pairs a workgroup | the other kernels, workgroups of one pair in brackets:
+//   4096 x 128 x 512 (256)  99 |  62 |  45       4096 x 128 x 768 (256) 135 |  86 |  63        1500 x 256 x 512 (256) 107 |  63 |  49
+//   3000 x 128 x 768 (192) 139 |  87 |  61      16384 x 32 x 256 (256)   48 |  31 |  23        5120 x 128 x 768 (320) 133 |  86 | 127
+//   2048 x 128 x 512 (128) 110 |  65 |  43 | 49  4096 x 64 x 768 (128)  141 |  89 |  62 | 73    1024 x 256 x 768 (128) 176 | 108 | 77 | 89
+//   8192 x 32 x 512 (128)   87 |  56 |  40 | 37  1024 x 128 x 768 (64)  179 | 107 |  69 | 46
+static int quad_chunk(int64_t B, int64_t T) {
+    const int64_t tiles = (B + 1023) / 1024, pairs = T / 2;
+    if (tiles * ((pairs + 3) / 4) >= 200) return 4;
+    if (tiles * pairs <= 256 && tiles * pairs >= (pairs >= 32 ? 128 : 192)) return 1;
+    return tiles * ((pairs + 1) / 2) >= 96 ? 2 : 0;
+}
+
 // The four-lanes-per-token kernel (lookup_inner_quad.hip) where the shape qualifies: S = 256, T even, tiles of
-// 1024 tokens x chunks of 4 or 2 table pairs; 4 when that still gives the chip a round of workgroups (the g
-// values are fetched once per chunk and slice), 2 otherwise, and not at all when even 2 leaves most of the chip
-// idle.  g: token b's 32 columns of slice s at g + b * g_token_stride + s * g_slice_stride floats.  Returns
+// 1024 tokens x chunks of quad_chunk table pairs.  g: token b's 32 columns of slice s at g + b * g_token_stride + s * g_slice_stride floats.  Returns
 // false when the shape does not qualify (nothing launched), true with the launch status in *rc otherwise.
 bool lffn_internal_lookup_inner_quad_try(const int32_t *code, const float *g, int64_t g_token_stride,
                                          int64_t g_slice_stride, const void *tables, float *grad_score, int64_t B,
@@ -262,9 +274,8 @@ bool lffn_internal_lookup_inner_quad_try(const int32_t *code, const float *g, in
     if (!(S == MAX_S && T % 2 == 0 && Do % 32 == 0 && B >= 1 && reinterpret_cast<uintptr_t>(code) % 8 == 0 &&
           2 * S * Do * 4 < (int64_t(1) << 32)))
         return false;
-    const int64_t tiles = (B + 1023) / 1024, pairs = T / 2;
-    const int c = tiles * ((pairs + 3) / 4) >= 200 ? 4 : (tiles * ((pairs + 1) / 2) >= 96 ? 2 : 0);
-    if (!c || tiles * ((pairs + c - 1) / c) > (int64_t(1) << 30)) return false;
+    const int c = quad_chunk(B, T);
+    if (!c || (B + 1023) / 1024 * ((T / 2 + c - 1) / c) > (int64_t(1) << 30)) return false;
     *rc = lffn_internal_lookup_inner_quad(code, g, g_token_stride, g_slice_stride, tables, grad_score, B, T, S, Do, 4, c, stream);
     return true;
 }
@@ -280,9 +291,8 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
     if (B * T == 0) return LFFN_OK;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t nslices = Do / 64;
-    // Four lanes per token, one owner per (token, table) (lookup_inner_quad.hip): tiles of 1024 tokens x
-    // chunks of 4 or 2 table pairs; 4 when that still gives the chip a round of workgroups (the g values are
-    // fetched once per chunk and slice), and the form below when even 2 leaves most of it idle.
+    // few tokens a workgroup each; then four lanes per token, one owner per (token, table), and the form below where that leaves most of
+    // the chip idle
     {
         int rc = LFFN_OK;
         if (lffn_internal_lookup_inner_tokens_try(code, g, tables, grad_score, B, T, S, Do, stream, &rc)) return rc;
@@ -326,17 +336,16 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
 namespace {
 
 // The four-lanes-per-token form for row numbers in table form (256-row tables): its steps (table pair x slice, about
-// 1.3 us each, rounds of 256 workgroups) against the token-major kernel's 9.4 TB/s, with 6 us for the flags and the
+// 1.3 us each, twice that where a step is a slice; rounds of 256 workgroups) against the token-major kernel's 9.4 TB/s, with 6 us for the flags and the
 // launch that ends at once and a margin for the prediction.
 bool inner_try_tables(int64_t B, int64_t I, int64_t source_size, int64_t Dv) {
     if (B < 1 || I < 2 || I % 2 != 0 || source_size != I * MAX_S || Dv < 64 || Dv % 64 != 0 || Dv > (1 << 20) ||
         B * I >= (int64_t(1) << 31) || 2 * MAX_S * Dv * 4 >= (int64_t(1) << 32))
         return false;
-    const int64_t tiles = (B + 1023) / 1024, pairs = I / 2;
-    const int c = tiles * ((pairs + 3) / 4) >= 200 ? 4 : (tiles * ((pairs + 1) / 2) >= 96 ? 2 : 0);
+    const int c = quad_chunk(B, I);
     if (!c) return false;
-    const int64_t rounds = (tiles * ((pairs + c - 1) / c) + 255) / 256;
-    const double us = double(rounds) * double(Dv / 32) * c * 1.3 + 6.0;
+    const int64_t rounds = ((B + 1023) / 1024 * ((I / 2 + c - 1) / c) + 255) / 256;
+    const double us = double(rounds) * double(Dv / 32) * (c > 1 ? c : 2) * 1.3 + 6.0;
     return us + 6.0 < 0.8 * (double(B) * double(I) * double(Dv) * 4 / 9.4e6);
 }
 

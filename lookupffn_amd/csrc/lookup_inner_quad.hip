@@ -410,6 +410,7 @@ int lffn_internal_lookup_inner_quad(const int32_t *code, const float *g, int64_t
     switch (np * 10 + c) {
         case 44: return launch_inner_quad<4, 4>(a, st);
         case 42: return launch_inner_quad<4, 2>(a, st);
+        case 41: return launch_inner_quad<4, 1>(a, st);
         default: return LFFN_ERR_BAD_ARG;
     }
 }
