@@ -94,6 +94,40 @@ __device__ __forceinline__ void lane_stage(float (&v)[NJ][4], int lr) {
     }
 }
 
+// Butterflies across lanes 1, 2 or 8 apart in one instruction a value instead of two: every lane gets own + partner * sgn (`sgn` as in
+// butterfly_xor), so the lane whose M bit is set gets own - partner, the result with its sign turned round (exact: a - b and b - a
+// round alike).  What follows is linear and takes the sign along; in the next transform the partners of this butterfly have opposite
+// signs, and with -sgn both come out upright again.  So `sgn` alternates from transform to transform, and after an even number of
+// them nothing is left of it.  (As fmaf(lane_xor(v), sgn, v) the compiler does not fold the move into the multiply-add.  A value that a
+// vector instruction has just written is ready for DPP two instructions later: hence the s_nop.)
+template <int M>
+__device__ __forceinline__ void turning_butterflies(float (&a)[4], float (&b)[4], float sgn) {
+    static_assert(M == 1 || M == 2 || M == 8, "one DPP move");
+#define LFFN_TURN8(ctrl)                                                                                                              \
+    asm("s_nop 1\n\t"                                                                                                                 \
+        "v_fmac_f32_dpp %0, %0, %8 " ctrl "\n\tv_fmac_f32_dpp %1, %1, %8 " ctrl "\n\tv_fmac_f32_dpp %2, %2, %8 " ctrl "\n\t"          \
+        "v_fmac_f32_dpp %3, %3, %8 " ctrl "\n\tv_fmac_f32_dpp %4, %4, %8 " ctrl "\n\tv_fmac_f32_dpp %5, %5, %8 " ctrl "\n\t"          \
+        "v_fmac_f32_dpp %6, %6, %8 " ctrl "\n\tv_fmac_f32_dpp %7, %7, %8 " ctrl                                                       \
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3])                                \
+        : "v"(sgn))
+    if constexpr (M == 1) LFFN_TURN8("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf");
+    else if constexpr (M == 2) LFFN_TURN8("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf");
+    else LFFN_TURN8("row_ror:8 row_mask:0xf bank_mask:0xf");
+#undef LFFN_TURN8
+}
+
+// TURN: the lane stages of distance M that turn signs (turning_butterflies), with turn = +1 or -1 from transform to transform
+template <int M, int NJ, bool TURN>
+__device__ __forceinline__ void last_lane_stage(float (&v)[NJ][4], int lr, float turn) {
+    if constexpr (TURN && NJ % 2 == 0) {
+        const float sgn = (lr & M) ? -turn : turn;
+#pragma unroll
+        for (int j = 0; j < NJ; j += 2) turning_butterflies<M>(v[j], v[j + 1], sgn);
+    } else {
+        lane_stage<M, 64, NJ, false>(v, lr);
+    }
+}
+
 template <int LOGD, bool SWAP = false>
 __device__ __forceinline__ void fht_rows(float (&v)[FhtCfg<LOGD>::NJ][4], int lr) {
     using C = FhtCfg<LOGD>;
@@ -167,8 +201,8 @@ __device__ __forceinline__ void wave_lds_handover() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int LOGD>
-__device__ __forceinline__ void fht_rows_xl(float (&v)[FhtCfg<LOGD>::NJ][4], int lr, float *wl) {
+template <int LOGD, bool TURN>
+__device__ __forceinline__ void fht_rows_xl(float (&v)[FhtCfg<LOGD>::NJ][4], int lr, float *wl, float turn) {
     using X = XlCfg<LOGD>;
     constexpr int NJ = X::NJ, NV = X::NV, STEP = X::STEP, BLOCK = X::BLOCK;
     if constexpr (NJ == 4) {
@@ -217,8 +251,8 @@ __device__ __forceinline__ void fht_rows_xl(float (&v)[FhtCfg<LOGD>::NJ][4], int
     }
     // lane strides STEP/8 .. 1 (element strides STEP/2 .. 4)
     if constexpr (STEP / 8 >= 4) lane_stage<4, 64, NJ, false>(v, lr);
-    lane_stage<2, 64, NJ, false>(v, lr);
-    lane_stage<1, 64, NJ, false>(v, lr);
+    last_lane_stage<2, NJ, TURN>(v, lr, turn);
+    last_lane_stage<1, NJ, TURN>(v, lr, turn);
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         float a0 = v[j][0], a1 = v[j][1], a2 = v[j][2], a3 = v[j][3];
@@ -275,6 +309,7 @@ template <int LOGD, bool HASH>
 __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
     using C = FhtCfg<LOGD>;
     constexpr int D = C::D, NJ = C::NJ, LPR = C::LPR, RPW = C::RPW;
+    constexpr bool TURN = HASH && LOGD >= 9;      // (a transform by itself keeps the signs of its zeros)
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int lr = lane % LPR;
@@ -359,6 +394,7 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) v[j][c] = orig[j][c];
 
+        float turn = 1.f;
         for (int s = 0; s < a.J; ++s) {
             if (a.diag) {
                 const float *dg = a.diag + (int64_t(r) * a.J + s) * D;
@@ -373,9 +409,19 @@ __global__ __launch_bounds__(256) void project_kernel(ProjectArgs a) {
             }
             if constexpr (LOGD == 10 || LOGD == 9) {
                 __shared__ float xl[4 * XlCfg<LOGD>::ROW];
-                fht_rows_xl<LOGD>(v, lr, xl + wave * XlCfg<LOGD>::ROW);
+                fht_rows_xl<LOGD, TURN>(v, lr, xl + wave * XlCfg<LOGD>::ROW, turn);
+                turn = -turn;
             } else {
                 fht_rows<LOGD>(v, lr);
+            }
+        }
+        if constexpr (TURN) {
+            if (a.J & 1) {                         // uniform: an odd number of transforms leaves signs turned
+                const float sgn = __popc(lr & 3) & 1 ? -1.f : 1.f;
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[j][c] = v[j][c] * sgn;
             }
         }
 
@@ -1021,7 +1067,7 @@ __global__ __launch_bounds__(256) void fht16_kernel(const uint16_t *__restrict__
     }
     if constexpr (LOGD == 10 || LOGD == 9) {
         __shared__ float xl[4 * XlCfg<LOGD>::ROW];
-        fht_rows_xl<LOGD>(v, lr, xl + wave * XlCfg<LOGD>::ROW);
+        fht_rows_xl<LOGD, false>(v, lr, xl + wave * XlCfg<LOGD>::ROW, 1.f);
     } else {
         fht_rows<LOGD>(v, lr);
     }
