@@ -196,6 +196,19 @@ def test_block_weight_gradient_over_chunks(B):
     assert (np.abs(got - want) <= (B + 4) * 2.0 ** -24 * scale).all()
 
 
+@pytest.mark.parametrize("B", [7200, 14337])
+def test_block_weight_gradient_over_long_chunks(B):
+    """Chunks of 1024 and 2048 tokens, the last one short; bound as above."""
+    torch.manual_seed(B)
+    R, J, D = 8, 4, 128
+    sg, x, si = (torch.randn(*s, device="cuda") for s in ((R * J, B, D), (B, D), (R, J - 1, B, D)))
+    got = lookupffn_amd.ops.bh4_block_wgrad(sg, x, si, R, J)
+    for s in range(R * J):
+        u = (x if s % J == 0 else si[s // J, s % J - 1]).double().view(B, D // 64, 64).permute(1, 0, 2).contiguous()
+        p = sg[s].double().view(B, D // 64, 64).permute(1, 2, 0).contiguous()
+        assert ((got[s] - torch.bmm(p, u)).abs() <= (B + 4) * 2.0 ** -24 * torch.bmm(p.abs(), u.abs())).all(), s
+
+
 # Both gradients of the layer's gather for few tokens and just past it: row groups of 32 and smaller tables, column passes, every token
 # on one row, adding to what is there
 @pytest.mark.parametrize("B,T,S,Do", [(1, 1, 256, 64), (5, 9, 16, 320), (64, 3, 32, 1088), (384, 65, 256, 768), (385, 8, 128, 256),
