@@ -808,6 +808,15 @@ int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float
                                  int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t block_size, float decay,
                                  float residual, void *stream);
 
+/*
+ * lffn_bh4_block_bwd_split_f32 behind the gradient of the 8-bit scores: from z [B, T*8] (16-byte aligned) and g_score [B, T], with the
+ * gradient of z that lffn_code_score_bwd_f32 computes formed inside.  bias_parts: [ceil(B / 16), T*8] or NULL, every sixteen tokens'
+ * sum of it (the projection bias's gradient is the sum of these rows).
+ */
+int lffn_bh4_block_score_bwd_split_f32(const float *z, const float *g_score, const float *w_split_t, float *g_x,
+                                       float *stage_grads, float *bias_parts, int64_t B, int64_t H, int64_t D, int64_t R,
+                                       int64_t J, int64_t T, int64_t block_size, float decay, float residual, void *stream);
+
 /* ------------------------------------------------- the encoder around the layer */
 
 /*

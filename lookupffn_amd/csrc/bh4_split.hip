@@ -162,7 +162,9 @@ struct SplitArgs {
     uint32_t *records;     // instead of codes and scores: the record stream of the four-lanes-per-token gather,
     int64_t rec_stride;    // [T/2][rec_stride][3] (lffn_quad_record_slot)
     int rec_tile;          // tokens per workgroup of the gather the records are written for
-    float *z;              // training: [B, T*8] z, kept for the backward
+    float *z;              // training: [B, T*8] z, kept for the backward (backward from scores: read)
+    const float *g_score;  // backward from scores: [B, T] gradient of the scores
+    float *bias_parts;     // backward from scores: [ceil(B/16), T*8] column sums of the gradient of z, or null
     float *row_stats;      // training, with LayerNorm: [B, 2] every row's mean and 1/sigma
     const float *gz;       // backward: [B, T*8] gradient of z
     float *g_x;            // backward: [R, B, H]
@@ -194,11 +196,16 @@ __device__ __forceinline__ void split4(f32x4 v, uint2 &hi, uint2 &lo) {
 // gradient P_s = (H_NB (x) I) G_{s+1} is also written to memory: the gradient w.r.t. the folded weights is the per-block product
 // P_s^T U_s over all tokens (U_s = the stage's input, which the forward saved), formed by the caller.  First gradient: decay * grad z;
 // result: grad x of this repeat = G_0[:, :H] + residual * grad z[:, :H].
-enum Form { HASH, TRAIN, BACKWARD };       // TRAIN: the hash form that also keeps what the backward needs
+//
+// SCORES_BACKWARD: the same from z and the scores' gradient.  The gradient of z is formed where it is used, at the start and for the
+// residual (a sixteen tokens' rows wait nowhere that is not needed), and its columns' sums, the projection bias's gradient, go out
+// with it: TIMES
+enum Form { HASH, TRAIN, BACKWARD, SCORES_BACKWARD };       // TRAIN: the hash form that also keeps what the backward needs
 
 template <int NB, Form FORM, int BG>
 __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split_kernel(SplitArgs a) {
-    constexpr bool BWD = FORM == BACKWARD;
+    constexpr bool BWD = FORM >= BACKWARD;
+    constexpr bool SCORES = FORM == SCORES_BACKWARD;
     constexpr bool SAVE = FORM != HASH;           // the numbers between the stages go to memory
     static_assert(BG == 1 || (BG == 4 && NB >= 4), "the wide form: four groups of blocks");
     constexpr int TOK = 16;                       // tokens per workgroup
@@ -456,17 +463,71 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
 
 #pragma unroll
     for (int n = 0; n < AHEAD; ++n) load_w(BWD ? J - 1 : 0, n);
+    // Backward from scores: the workgroup's tokens' rows as NBW vectors of four columns a thread, a few
+    // at a time; two neighbouring lanes have the eight columns of a score.
+    auto z_gradient = [&](f32x4 z, float g) {
+        const bool odd = lane & 1;                // the second four of the eight
+        float v[8], away[8], out[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float own = expf(-2.0f * fabsf(z[e])), z_other = lane_xor<1>(z[e]), other = lane_xor<1>(own);
+            v[e] = odd ? z_other : z[e];
+            v[e + 4] = odd ? z[e] : z_other;
+            away[e] = odd ? other : own;
+            away[e + 4] = odd ? own : other;
+        }
+        score_gradient<8>(v, away, g, out);
+        return odd ? (f32x4){out[4], out[5], out[6], out[7]} : (f32x4){out[0], out[1], out[2], out[3]};
+    };
+    auto z_gradients = [&](auto take) {
+        constexpr int FEW = NBW < 4 ? NBW : 4;
+#pragma unroll 1
+        for (int i0 = 0; i0 < NBW; i0 += FEW) {
+            f32x4 z[FEW];
+            float g[FEW];
+            int at[FEW];
+#pragma unroll
+            for (int i = 0; i < FEW; ++i) {
+                at[i] = tid + (i0 + i) * 256 * BG;
+                const int64_t tok = min(tok_base + at[i] / (D / 4), B - 1);
+                const int col = r * D + 4 * (at[i] % (D / 4));
+                const bool in = col < a.T * 8;
+                z[i] = *reinterpret_cast<const f32x4 *>(a.z + tok * (a.T * 8) + (in ? col : 0));
+                g[i] = a.g_score[tok * a.T + (in ? col / 8 : 0)];
+                if (!in || tok_base + at[i] / (D / 4) >= B) g[i] = 0.f, z[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int i = 0; i < FEW; ++i) take(at[i] / (D / 4), 4 * (at[i] % (D / 4)), z_gradient(z[i], g[i]));
+        }
+    };
     if constexpr (BWD) {
         const int ncols = a.T * 8;
         // The matrix cores' sums are off to one side by a little, a twentieth of what a result is off in any direction; the gradient
         // of the weights, a sum over the tokens, would keep that, so every other token's row has its sign turned on the way.
         inv_x = c & 1 ? -1.f : 1.f;
+        if constexpr (SCORES) {
+            z_gradients([&](int row, int col, f32x4 g) { *reinterpret_cast<f32x4 *>(rows32 + row * LDR + col) = g; });
+            __syncthreads();
+            if (a.bias_parts) {
+                for (int e = tid; e < D && r * D + e < ncols; e += 256 * BG) {
+                    float sum = 0.f;
 #pragma unroll
-        for (int n = 0; n < NBW; ++n) {
-            const int gcol = r * D + (n * BG + bg) * BS + 16 * ow + 4 * kq;
-            f32x4 g = {0.f, 0.f, 0.f, 0.f};
-            if (tok_base + c < B && gcol < ncols) g = *reinterpret_cast<const f32x4 *>(a.gz + (tok_base + c) * ncols + gcol);
-            acc[n] = (a.decay * inv_x) * g;
+                    for (int t = 0; t < TOK; ++t) sum += rows32[t * LDR + e];
+                    a.bias_parts[size_t(blockIdx.x) * ncols + r * D + e] = sum;
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < NBW; ++n)
+                acc[n] = (a.decay * inv_x) * *reinterpret_cast<const f32x4 *>(rows32 + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq);
+            if constexpr (BG > 1) __syncthreads();             // (the narrow form's hand_over begins with one)
+        } else {
+#pragma unroll
+            for (int n = 0; n < NBW; ++n) {
+                const int gcol = r * D + (n * BG + bg) * BS + 16 * ow + 4 * kq;
+                f32x4 g = {0.f, 0.f, 0.f, 0.f};
+                if (tok_base + c < B && gcol < ncols) g = *reinterpret_cast<const f32x4 *>(a.gz + (tok_base + c) * ncols + gcol);
+                acc[n] = (a.decay * inv_x) * g;
+            }
         }
 #pragma unroll 1
         for (int s = J - 1; s >= 0; --s) {
@@ -567,7 +628,16 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     if constexpr (BWD) {
         // grad x of this repeat: the first H columns, plus the residual path of the mix
         const int ncols = a.T * 8;
-        if constexpr (BG == 1) {                  // whole rows again
+        if constexpr (SCORES) {                   // whole rows again
+            __syncthreads();
+            to_rows(inv_w * inv_x);
+            __syncthreads();
+            z_gradients([&](int row, int col, f32x4 g) {
+                f32x4 v = *reinterpret_cast<const f32x4 *>(rows32 + row * LDR + col);
+                v = v + a.residual * g;           // (beyond T*8 columns: 0)
+                if (tok_base + row < B && col < H) *reinterpret_cast<f32x4 *>(a.g_x + (size_t(r) * B + tok_base + row) * H + col) = v;
+            });
+        } else if constexpr (BG == 1) {
             __syncthreads();
             to_rows(inv_w * inv_x);
             __syncthreads();
@@ -720,7 +790,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
 template <int NB, Form FORM, int BG>
 int launch_form(const SplitArgs &a, hipStream_t st) {
     constexpr int TOK = 16, D = BS * NB;
-    constexpr size_t lds_bytes = (BG > 1 ? 2 : 1) * TOK * (D + PAD) * 4 + 7 * TOK * 4 + (FORM == BACKWARD ? 0 : 3 * D * 4);
+    constexpr size_t lds_bytes = (BG > 1 ? 2 : 1) * TOK * (D + PAD) * 4 + 7 * TOK * 4 + (FORM >= BACKWARD ? 0 : 3 * D * 4);
     static_assert(lds_bytes <= 160 * 1024);
     auto kern = bh4_split_kernel<NB, FORM, BG>;
     static LdsGrant granted;      // one record per kernel instantiation
@@ -815,19 +885,44 @@ extern "C" int lffn_bh4_block_front_train_split_f32(const lffn_block_front *f, c
     return dispatch_block<TRAIN>(a, f->D, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float *g_x, float *stage_grads, int64_t B,
-                                            int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t block_size, float decay,
-                                            float residual, void *stream) {
+namespace {
+
+// the backwards' arguments, checked
+int back_args(const float *w_split_t, float *g_x, float *stage_grads, int64_t B, int64_t H, int64_t D, int64_t R, int64_t J, int64_t T,
+              int64_t block_size, float decay, float residual, SplitArgs &a) {
     LFFN_REQUIRE(B >= 0 && R >= 1 && J >= 1 && D >= 1 && H >= 1 && H <= D && T >= 1, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(H % 4 == 0 && J <= 64, LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(block_size == BS && lffn_is_pow2(D) && D >= BS && D <= 1024, LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(R <= 4096 && B <= (int64_t(1) << 31) - 1 && T <= (1 << 24), LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(T * 8 <= R * D, LFFN_ERR_BAD_ARG);
     if (B == 0) return LFFN_OK;
-    LFFN_REQUIRE(g_z && w_split_t && g_x && stage_grads, LFFN_ERR_BAD_ARG);
-    LFFN_REQUIRE(lffn_aligned16(g_z) && lffn_aligned16(w_split_t) && lffn_aligned16(g_x) && lffn_aligned16(stage_grads), LFFN_ERR_BAD_ARG);
-    SplitArgs a{};
-    a.gz = g_z; a.w = w_split_t; a.wscale = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_save = stage_grads;
+    LFFN_REQUIRE(w_split_t && g_x && stage_grads, LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(lffn_aligned16(w_split_t) && lffn_aligned16(g_x) && lffn_aligned16(stage_grads), LFFN_ERR_BAD_ARG);
+    a.w = w_split_t; a.wscale = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_save = stage_grads;
     a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = decay; a.residual = residual;
+    return LFFN_OK;
+}
+
+}  // namespace
+
+extern "C" int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float *g_x, float *stage_grads, int64_t B,
+                                            int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t block_size, float decay,
+                                            float residual, void *stream) {
+    SplitArgs a{};
+    const int rc = back_args(w_split_t, g_x, stage_grads, B, H, D, R, J, T, block_size, decay, residual, a);
+    if (rc != LFFN_OK || B == 0) return rc;
+    LFFN_REQUIRE(g_z && lffn_aligned16(g_z), LFFN_ERR_BAD_ARG);
+    a.gz = g_z;
     return dispatch_block<BACKWARD>(a, D, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int lffn_bh4_block_score_bwd_split_f32(const float *z, const float *g_score, const float *w_split_t, float *g_x,
+                                                  float *stage_grads, float *bias_parts, int64_t B, int64_t H, int64_t D, int64_t R,
+                                                  int64_t J, int64_t T, int64_t block_size, float decay, float residual, void *stream) {
+    SplitArgs a{};
+    const int rc = back_args(w_split_t, g_x, stage_grads, B, H, D, R, J, T, block_size, decay, residual, a);
+    if (rc != LFFN_OK || B == 0) return rc;
+    LFFN_REQUIRE(z && g_score && lffn_aligned16(z), LFFN_ERR_BAD_ARG);
+    a.z = const_cast<float *>(z); a.g_score = g_score; a.bias_parts = bias_parts;
+    return dispatch_block<SCORES_BACKWARD>(a, D, static_cast<hipStream_t>(stream));
 }

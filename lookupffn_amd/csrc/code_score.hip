@@ -112,21 +112,10 @@ __global__ __launch_bounds__(256) void code_score_bwd_kernel(const float *__rest
             const float4 t = reinterpret_cast<const float4 *>(z + n * K)[q];
             v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
         }
-        float S = 0.f, P = 1.f;
 #pragma unroll
-        for (int d = 0; d < K; ++d) {
-            const float a = fabsf(v[d]);
-            e[d] = expf(-2.0f * a);
-            S = S + a;
-            P = P * (1.0f + e[d]);
-        }
-        const float gp = g_score[n] / P;
+        for (int d = 0; d < K; ++d) e[d] = expf(-2.0f * fabsf(v[d]));
         float o[K];
-#pragma unroll
-        for (int d = 0; d < K; ++d) {
-            const float sg = v[d] > 0.f ? gp : (v[d] < 0.f ? -gp : 0.f);
-            o[d] = sg * (1.0f + S * 2.0f * (e[d] * __builtin_amdgcn_rcpf(1.0f + e[d])));   // hardware reciprocal, 1 ulp
-        }
+        score_gradient<K>(v, e, g_score[n], o);
 #pragma unroll
         for (int q = 0; q < K / 4; ++q)
             reinterpret_cast<float4 *>(g_z + n * K)[q] = make_float4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);

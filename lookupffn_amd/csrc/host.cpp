@@ -64,8 +64,7 @@ using torch::autograd::variable_list;
     X(lffn_lookup_scatter_f32)              \
     X(lffn_lookup_scatter_sorted_f32)       \
     X(lffn_ln_project_hash_bwd_f32)         \
-    X(lffn_code_score_bwd_f32)              \
-    X(lffn_bh4_block_bwd_split_f32)         \
+        X(lffn_bh4_block_score_bwd_split_f32)   \
     X(lffn_ln_bh4_block_wgrad_f32)          \
     X(lffn_layer_norm_bwd_f32)              \
     X(lffn_sum_partials_f32)
@@ -398,11 +397,13 @@ struct LookupFFNBackward : public torch::autograd::Node {
             }
         } else {
             const Tensor stage = stage_in.unpack(self), st_ = stats.unpack(self);
-            Tensor g_z = empty_f32({B, T * 8}, dev), stage_g = empty_f32({R * J, B, D}, dev), split = empty_f32({split_words(c)}, dev);
-            CALL(lffn_code_score_bwd_f32, f32(z_), f32(g_score), f32(g_z), B * T, 8, st);
+            const int64_t parts = (B + 15) / 16;               // of the projection bias's gradient
+            Tensor g_b = need[PBIAS] ? empty_f32({parts * T * 8}, dev) : Tensor();
+            Tensor stage_g = empty_f32({R * J, B, D}, dev), split = empty_f32({split_words(c)}, dev);
             const int64_t blocks = R * J * (D / 64);
             CALL(lffn_bh4_fold_split_f32, f32(w), f32(split), R * J, D / 64, 64, 1, st);
-            CALL(lffn_bh4_block_bwd_split_f32, f32(g_z), f32(split), f32(g_h), f32(stage_g), B, H, D, R, J, T, 64, decay, res, st);
+            CALL(lffn_bh4_block_score_bwd_split_f32, f32(z_), f32(g_score), f32(split), f32(g_h), f32(stage_g), need[PBIAS] ? f32(g_b) : nullptr,
+                 B, H, D, R, J, T, 64, decay, res, st);
             if (need[WEIGHT]) {
                 Tensor g_folded = at::zeros({R * J, D / 64, 64, 64}, at::TensorOptions().dtype(at::kFloat).device(dev));
                 CALL(lffn_ln_bh4_block_wgrad_f32, f32(stage_g), f32(x_), f32(lw), f32(lb), f32(st_), J > 1 ? f32(stage) : nullptr, f32(g_folded),
@@ -412,7 +413,7 @@ struct LookupFFNBackward : public torch::autograd::Node {
             }
             if (need[PBIAS]) {
                 out[PBIAS] = empty_f32({T * 8}, dev);
-                column_sums(f32(g_z), f32(out[PBIAS]), T * 8, nullptr, nullptr, 0, B, dev, st);
+                column_sums(f32(g_b), f32(out[PBIAS]), T * 8, nullptr, nullptr, 0, parts, dev, st);
             }
         }
         if (need_ln) {

@@ -351,5 +351,24 @@ constexpr int TOUCH_AHEAD = 2;
 // the scores agree with the float64 oracle as before (2e-6).
 __device__ __forceinline__ float exp_minus_2a(float a) { return __builtin_amdgcn_exp2f(-2.885390081777927f * a); }
 
+// Gradient of a score, sum |v| / prod (1 + exp(-2 |v|)) over K values, with respect to them, times g; away[d] is
+// exp(-2 |v[d]|).  Sum and product in the forward's order (code_score.hip), no fused multiply-add.
+template <int K>
+__device__ __forceinline__ void score_gradient(const float (&v)[K], const float (&away)[K], float g, float (&out)[K]) {
+#pragma clang fp contract(off)
+    float S = 0.f, P = 1.f;
+#pragma unroll
+    for (int d = 0; d < K; ++d) {
+        S = S + fabsf(v[d]);
+        P = P * (1.0f + away[d]);
+    }
+    const float gp = g / P;
+#pragma unroll
+    for (int d = 0; d < K; ++d) {
+        const float sg = v[d] > 0.f ? gp : (v[d] < 0.f ? -gp : 0.f);
+        out[d] = sg * (1.0f + S * 2.0f * (away[d] * __builtin_amdgcn_rcpf(1.0f + away[d])));   // hardware reciprocal, 1 ulp
+    }
+}
+
 __device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_float(packed & 0xFFFF0000u); }

@@ -96,7 +96,7 @@ class ProjectHash(torch.autograd.Function):
 class BlockProjectHash(torch.autograd.Function):
     """BH4 with 64 x 64 blocks -> mix -> bias -> 8-bit code + score as one differentiable
     operator.  Forward: one matrix-core kernel that also keeps z and the input of every stage.
-    Backward: the score derivative, one matrix-core kernel walking the stages down (grad x and
+    Backward: one matrix-core kernel from the scores' derivative down the stages (grad x, the bias's gradient and
     the gradient in front of every block product), then the weight gradient: a matrix-core
     kernel summing, per block, those gradients against the saved stage inputs over the tokens,
     taken back through the 64-point transform.  Same mathematics as bh4_cuda + BH4._forward + compute_code_score under
@@ -121,16 +121,15 @@ class BlockProjectHash(torch.autograd.Function):
         R, J, NB, bs, _ = w.shape
         B, H = x.shape
         T = g_score.shape[1]
-        g_z = ops.code_score_bwd(z.reshape(B, T, 8), g_score.contiguous()).reshape(B, T * 8)
-        g_x, stage_g = ops.bh4_block_bwd_split(g_z, ops.bh4_fold_split(w, True), R, J, NB * bs, H, ctx.decay, 1 - ctx.decay)
+        g_x, stage_g, g_bias = ops.bh4_block_score_bwd_split(z, g_score.contiguous(), ops.bh4_fold_split(w, True), R, J, NB * bs, H,
+                                                             ctx.decay, 1 - ctx.decay, ctx.has_bias and ctx.needs_input_grad[2])
         g_w = None
         if ctx.needs_input_grad[1]:
             # stage 0 reads x (zero beyond its H columns), stage j the saved input of that stage
             g_folded = ops.bh4_block_wgrad(stage_g.reshape(R * J, B, NB * bs), x, stage_in, R, J).view_as(w)
             g_w = ops.bh4_fold_mode(g_folded, 2)
         g_x = g_x[0] if R == 1 else g_x.sum(0)
-        g_bias = ops.column_sums(g_z) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
-        return (g_x if ctx.needs_input_grad[0] else None, g_w, g_bias, None, None)
+        return (g_x if ctx.needs_input_grad[0] else None, g_w, g_bias if (ctx.has_bias and ctx.needs_input_grad[2]) else None, None, None)
 
 
 class Hashing(nn.Module):
@@ -377,8 +376,8 @@ class LnBlockProjectHash(torch.autograd.Function):
         B, H = x.shape
         T = g_score.shape[1]
         need = ctx.needs_input_grad
-        g_z = ops.code_score_bwd(z.reshape(B, T, 8), g_score.contiguous()).reshape(B, T * 8)
-        g_h, stage_g = ops.bh4_block_bwd_split(g_z, ops.bh4_fold_split(w, True), R, J, NB * bs, H, ctx.decay, 1 - ctx.decay)
+        g_h, stage_g, g_bias = ops.bh4_block_score_bwd_split(z, g_score.contiguous(), ops.bh4_fold_split(w, True), R, J, NB * bs, H,
+                                                             ctx.decay, 1 - ctx.decay, ctx.has_bias and need[5])
         g_w = None
         if need[4]:
             g_folded = ops.ln_bh4_block_wgrad(stage_g.reshape(R * J, B, NB * bs), x, ln_weight, ln_bias, stats, stage_in,
@@ -387,9 +386,8 @@ class LnBlockProjectHash(torch.autograd.Function):
         g_x = g_lw = g_lb = None
         if need[0] or need[1] or need[2]:
             g_x, g_lw, g_lb = ops.layer_norm_bwd(x, ln_weight, ctx.eps, g_h)      # adds the R repeats' gradients
-        g_bias = ops.column_sums(g_z) if (ctx.has_bias and need[5]) else None
-        return (g_x if need[0] else None, g_lw if need[1] else None, g_lb if need[2] else None, None, g_w, g_bias,
-                None, None)
+        return (g_x if need[0] else None, g_lw if need[1] else None, g_lb if need[2] else None, None, g_w,
+                g_bias if (ctx.has_bias and need[5]) else None, None, None)
 
 
 class LookupFFN(nn.Module):

@@ -523,6 +523,38 @@ def _(g_z, w_split_t, R, J, D, H, decay, residual):
     return g_z.new_empty(R, g_z.shape[0], H), g_z.new_empty(R, J, g_z.shape[0], D)
 
 
+_L.define("bh4_block_score_bwd_split(Tensor z, Tensor g_score, Tensor w_split_t, int R, int J, int D, int H, float decay, float residual, "
+          "bool bias) -> (Tensor, Tensor, Tensor)")
+
+
+def _bh4_block_score_bwd_split_impl(z, g_score, w_split_t, R, J, D, H, decay, residual, bias):
+    """bh4_block_bwd_split behind code_score_bwd -> (g_x [R,B,H], stage_grads [R,J,B,D], the projection bias's gradient [T*8], or
+    empty without `bias`)."""
+    _lib.require_gpu(z, g_score, w_split_t)
+    assert z.dim() == 2 and z.dtype == torch.float32 and z.is_contiguous() and z.shape[1] % 8 == 0
+    B, T = z.shape[0], z.shape[1] // 8
+    assert g_score.dtype == torch.float32 and g_score.is_contiguous() and tuple(g_score.shape) == (B, T)
+    assert w_split_t.dtype == torch.float32 and w_split_t.is_contiguous() and w_split_t.numel() == split_words((R, J, D // 64, 64, 64))
+    g_x, stage_g = z.new_empty(R, B, H), z.new_empty(R, J, B, D)
+    if B == 0:
+        return g_x, stage_g, z.new_zeros(T * 8 if bias else 0)
+    parts = z.new_empty((B + 15) // 16, T * 8) if bias else None
+    with _dev_guard(z):
+        rc = _lib.load().lffn_bh4_block_score_bwd_split_f32(_lib.ptr(z), _lib.ptr(g_score), _lib.ptr(w_split_t), _lib.ptr(g_x),
+                                                            _lib.ptr(stage_g), _lib.ptr(parts), B, H, D, R, J, T, 64, decay, residual,
+                                                            _lib.stream_of(z))
+    _lib.check(rc, f"lffn_bh4_block_score_bwd_split_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
+    return g_x, stage_g, _sum_partials(parts)[0] if bias else z.new_empty(0)
+
+
+_L.impl("bh4_block_score_bwd_split", _bh4_block_score_bwd_split_impl, "CUDA")
+
+
+@torch.library.register_fake("lookupffn::bh4_block_score_bwd_split")
+def _(z, g_score, w_split_t, R, J, D, H, decay, residual, bias):
+    return z.new_empty(R, z.shape[0], H), z.new_empty(R, J, z.shape[0], D), z.new_empty(z.shape[1] if bias else 0)
+
+
 _L.define("bh4_block_wgrad(Tensor stage_grads, Tensor x, Tensor stage_inputs, int R, int J) -> Tensor")
 
 
@@ -1297,6 +1329,7 @@ bh4_fold_split = torch.ops.lookupffn.bh4_fold_split
 bh4_block_front = torch.ops.lookupffn.bh4_block_front
 bh4_block_front_train = torch.ops.lookupffn.bh4_block_front_train
 bh4_block_bwd_split = torch.ops.lookupffn.bh4_block_bwd_split
+bh4_block_score_bwd_split = torch.ops.lookupffn.bh4_block_score_bwd_split
 bh4_fold_mode = torch.ops.lookupffn.bh4_fold_mode
 bh4_block_hash_train = torch.ops.lookupffn.bh4_block_hash_train
 bh4_block_bwd = torch.ops.lookupffn.bh4_block_bwd

@@ -88,6 +88,25 @@ def test_against_64_bits(B, H, D, R, T, with_ln):
         assert _rel(g_x[r][some], (G + 0.3 * g)[:, :H]) <= REL
 
 
+@pytest.mark.parametrize("B,H,D,R,T", [(1, 64, 64, 2, 16), (33, 100, 128, 2, 29), (70, 256, 256, 1, 32), (4200, 200, 256, 1, 31),
+                                       (31, 512, 512, 2, 100), (2300, 500, 512, 2, 128), (17, 768, 1024, 1, 127), (4100, 1024, 1024, 1, 128)])
+def test_backward_from_scores(B, H, D, R, T):
+    """The scores' derivative inside the kernel: what code_score_bwd and the backward from its result give, bit for bit; the bias's
+    gradient, sums of sixteen and then of at most 256 numbers and chunks, within that many roundings of their magnitudes."""
+    gen = torch.Generator(device=DEV).manual_seed(B + T)
+    J = 4
+    split_t = ops.bh4_fold_split(_randn(gen, R, J, D // 64, 64, 64) / math.sqrt(64 * D), True)
+    z, g_score = 2 * _randn(gen, B, T * 8), _randn(gen, B, T)
+    z[0, :8] = 0
+    z[-1, ::3] *= 1e-8
+    g_z = ops.code_score_bwd(z.view(B, T, 8), g_score).view(B, T * 8)
+    g_x, stage_g, g_bias = ops.bh4_block_score_bwd_split(z, g_score, split_t, R, J, D, H, 0.7, 0.3, True)
+    want_x, want_stage = ops.bh4_block_bwd_split(g_z, split_t, R, J, D, H, 0.7, 0.3)
+    assert torch.equal(g_x, want_x) and torch.equal(stage_g, want_stage)
+    assert ((g_bias - g_z.double().sum(0)).abs() <= 64 * 2.0 ** -24 * g_z.double().abs().sum(0)).all()
+    assert ops.bh4_block_score_bwd_split(z, g_score, split_t, R, J, D, H, 0.7, 0.3, False)[2].numel() == 0
+
+
 # both forms of the kernel (few and many workgroups), rows around the 16 of a tile, columns short of D, codes short of them
 @pytest.mark.parametrize("B,H,D,R,T", [(1, 64, 64, 2, 16), (33, 100, 128, 2, 30), (70, 256, 256, 1, 32), (4200, 200, 256, 1, 32),
                                        (31, 512, 512, 2, 100), (2300, 500, 512, 2, 128), (17, 768, 1024, 1, 128), (4100, 1024, 1024, 1, 128)])
