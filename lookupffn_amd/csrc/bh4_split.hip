@@ -466,18 +466,13 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     // Backward from scores: the workgroup's tokens' rows as NBW vectors of four columns a thread, a few
     // at a time; two neighbouring lanes have the eight columns of a score.
     auto z_gradient = [&](f32x4 z, float g) {
-        const bool odd = lane & 1;                // the second four of the eight
-        float v[8], away[8], out[8];
+        const float zq[4] = {z.x, z.y, z.z, z.w};
+        const ScorePart own = score_part(zq);
+        const float twice = 2.0f * (own.sum + lane_xor<1>(own.sum)), g_over_p = g / (own.product * lane_xor<1>(own.product));
+        f32x4 out;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float own = expf(-2.0f * fabsf(z[e])), z_other = lane_xor<1>(z[e]), other = lane_xor<1>(own);
-            v[e] = odd ? z_other : z[e];
-            v[e + 4] = odd ? z[e] : z_other;
-            away[e] = odd ? other : own;
-            away[e + 4] = odd ? own : other;
-        }
-        score_gradient<8>(v, away, g, out);
-        return odd ? (f32x4){out[4], out[5], out[6], out[7]} : (f32x4){out[0], out[1], out[2], out[3]};
+        for (int e = 0; e < 4; ++e) out[e] = score_derivative(zq[e], own.away[e], twice, g_over_p);
+        return out;
     };
     auto z_gradients = [&](auto take) {
         constexpr int FEW = NBW < 4 ? NBW : 4;

@@ -106,19 +106,24 @@ __global__ __launch_bounds__(256) void code_score_bwd_kernel(const float *__rest
     const int64_t n = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (n >= N) return;
     if constexpr (K > 0) {
-        float v[K], e[K];
+        ScorePart part[K / 4];
+        float v[K / 4][4], sum = 0.f, product = 1.f;
 #pragma unroll
         for (int q = 0; q < K / 4; ++q) {
             const float4 t = reinterpret_cast<const float4 *>(z + n * K)[q];
-            v[4 * q] = t.x, v[4 * q + 1] = t.y, v[4 * q + 2] = t.z, v[4 * q + 3] = t.w;
+            v[q][0] = t.x, v[q][1] = t.y, v[q][2] = t.z, v[q][3] = t.w;
+            part[q] = score_part(v[q]);
+            sum += part[q].sum;
+            product *= part[q].product;
         }
+        const float twice = 2.0f * sum, g_over_p = g_score[n] / product;
 #pragma unroll
-        for (int d = 0; d < K; ++d) e[d] = expf(-2.0f * fabsf(v[d]));
-        float o[K];
-        score_gradient<K>(v, e, g_score[n], o);
+        for (int q = 0; q < K / 4; ++q) {
+            float o[4];
 #pragma unroll
-        for (int q = 0; q < K / 4; ++q)
-            reinterpret_cast<float4 *>(g_z + n * K)[q] = make_float4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
+            for (int c = 0; c < 4; ++c) o[c] = score_derivative(v[q][c], part[q].away[c], twice, g_over_p);
+            reinterpret_cast<float4 *>(g_z + n * K)[q] = make_float4(o[0], o[1], o[2], o[3]);
+        }
     } else {
         const float *p = z + n * k;
         float S = 0.f, P = 1.f;

@@ -37,16 +37,6 @@ struct Tile {
     static_assert(LOGD >= 8 && LOGD <= 10, "256, 512 and 1024 points");
 };
 
-// exp(-2 a), a >= 0: the instruction's 2^t with what rounding takes from t = -2 a log2 e put back to first order (t grows with a, and a
-// rounded t alone is off by 9e-7 of the result at a = 8).  Beyond 128 the result is 0; there a is held, so that no infinity meets it.
-// (84 -> 86 us of the kernel; expf 89.  Gradients of z of 0.5 to 3: rms error 1.45e-7 -> 1.39e-7.)
-__device__ __forceinline__ float exp_minus_twice(float a) {
-    constexpr float C = -2.885390081777927f, C_REST = float(-2.8853900817779268 - double(C)), LN2 = 0.6931471805599453f;
-    a = fminf(a, 128.f);
-    const float t = a * C, rest = fmaf(a, C_REST, fmaf(a, C, -t)), e = __builtin_amdgcn_exp2f(t);
-    return fmaf(e * LN2, rest, e);
-}
-
 __device__ __forceinline__ uint32_t max_u32(uint32_t a, uint32_t b) { return a > b ? a : b; }
 __device__ __forceinline__ uint32_t magnitude(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
 
@@ -307,30 +297,18 @@ __global__ __launch_bounds__(256, 2) void project_hash_bwd_mfma_kernel(ProjectBw
         transform<LOGD, true>(t, fa, fb, turned, lane);
         keep(3);
 
-        // The gradient of z from the closed form of the score (PL/compute_code_score/kernel.py:51-53 differentiated).  A group of
-        // eight columns sits in four registers of the two halves of the wavefront.
+        // The gradient of z.  A group of eight columns sits in four registers of the two halves of the wavefront.
         float gz[16];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            float ez[4], sum = 0.f, product = 1.f;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const float az = fabsf(z[4 * q + c]);
-                ez[c] = exp_minus_twice(az);
-                sum += az;
-                product *= 1.0f + ez[c];
-            }
-            const auto ss = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
-            const auto pp = __builtin_amdgcn_permlane32_swap(__float_as_uint(product), __float_as_uint(product), false, false);
+            const float zq[4] = {z[4 * q], z[4 * q + 1], z[4 * q + 2], z[4 * q + 3]};
+            const ScorePart own = score_part(zq);
+            const auto ss = __builtin_amdgcn_permlane32_swap(__float_as_uint(own.sum), __float_as_uint(own.sum), false, false);
+            const auto pp = __builtin_amdgcn_permlane32_swap(__float_as_uint(own.product), __float_as_uint(own.product), false, false);
             const float twice = 2.0f * (__uint_as_float(ss[0]) + __uint_as_float(ss[1]));
             const float g_over_p = g[q] / (__uint_as_float(pp[0]) * __uint_as_float(pp[1]));
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const float zz = z[4 * q + c], w = ez[c] * __builtin_amdgcn_rcpf(1.0f + ez[c]);          // (1 ulp)
-                // times the sign of z; 0 where z is
-                const float v = __uint_as_float(__float_as_uint((1.0f + twice * w) * g_over_p) ^ (__float_as_uint(zz) & 0x80000000u));
-                gz[4 * q + c] = zz != 0.f ? v : 0.f;
-            }
+            for (int c = 0; c < 4; ++c) gz[4 * q + c] = score_derivative(zq[c], own.away[c], twice, g_over_p);
             float4 sb = sum_b[wave][q][lane];
             sb.x += gz[4 * q]; sb.y += gz[4 * q + 1]; sb.z += gz[4 * q + 2]; sb.w += gz[4 * q + 3];
             sum_b[wave][q][lane] = sb;

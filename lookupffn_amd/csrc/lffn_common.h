@@ -351,23 +351,38 @@ constexpr int TOUCH_AHEAD = 2;
 // the scores agree with the float64 oracle as before (2e-6).
 __device__ __forceinline__ float exp_minus_2a(float a) { return __builtin_amdgcn_exp2f(-2.885390081777927f * a); }
 
-// Gradient of a score, sum |v| / prod (1 + exp(-2 |v|)) over K values, with respect to them, times g; away[d] is
-// exp(-2 |v[d]|).  Sum and product in the forward's order (code_score.hip), no fused multiply-add.
-template <int K>
-__device__ __forceinline__ void score_gradient(const float (&v)[K], const float (&away)[K], float g, float (&out)[K]) {
-#pragma clang fp contract(off)
-    float S = 0.f, P = 1.f;
+// exp(-2 a), a >= 0: the instruction's 2^t with what rounding takes from t = -2 a log2 e put back to first order (t grows with a, and a
+// rounded t alone is off by 9e-7 of the result at a = 8).  Beyond 128 the result is 0; there a is held, so that no infinity meets it.
+// (Projection backward at 16384 x 1024 84 -> 86 us, with expf 89.  Gradients of z of 0.5 to 3: rms error 1.45e-7 -> 1.39e-7.)
+__device__ __forceinline__ float exp_minus_twice(float a) {
+    constexpr float C = -2.885390081777927f, C_REST = float(-2.8853900817779268 - double(C)), LN2 = 0.6931471805599453f;
+    a = fminf(a, 128.f);
+    const float t = a * C, rest = fmaf(a, C_REST, fmaf(a, C, -t)), e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e * LN2, rest, e);
+}
+
+// Gradient of a score, s = sum |z| / prod (1 + exp(-2 |z|)), with respect to its z (the closed form of
+// PL/compute_code_score/kernel.py:51-53 differentiated), four columns at a time: away = exp(-2 |z|), and the four's part of
+// sum and product, which the caller combines over the score's fours.
+struct ScorePart {
+    float away[4], sum, product;
+};
+__device__ __forceinline__ ScorePart score_part(const float (&z)[4]) {
+    ScorePart p{{}, 0.f, 1.f};
 #pragma unroll
-    for (int d = 0; d < K; ++d) {
-        S = S + fabsf(v[d]);
-        P = P * (1.0f + away[d]);
+    for (int c = 0; c < 4; ++c) {
+        const float a = fabsf(z[c]);
+        p.away[c] = exp_minus_twice(a);
+        p.sum += a;
+        p.product *= 1.0f + p.away[c];
     }
-    const float gp = g / P;
-#pragma unroll
-    for (int d = 0; d < K; ++d) {
-        const float sg = v[d] > 0.f ? gp : (v[d] < 0.f ? -gp : 0.f);
-        out[d] = sg * (1.0f + S * 2.0f * (away[d] * __builtin_amdgcn_rcpf(1.0f + away[d])));   // hardware reciprocal, 1 ulp
-    }
+    return p;
+}
+__device__ __forceinline__ float score_derivative(float z, float away, float twice_sum, float g_over_product) {
+    const float w = away * __builtin_amdgcn_rcpf(1.0f + away);          // (1 ulp)
+    // times the sign of z; 0 where z is
+    const float v = __uint_as_float(__float_as_uint(fmaf(twice_sum, w, 1.0f) * g_over_product) ^ (__float_as_uint(z) & 0x80000000u));
+    return z != 0.f ? v : 0.f;
 }
 
 __device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
