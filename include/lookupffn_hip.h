@@ -209,6 +209,15 @@ int lffn_bh4_block_bwd_f32(const float *g_z, const float *w_folded_t, float *g_x
 int lffn_sum_partials_f32(const float *parts_a, float *out_a, int64_t n_a, const float *parts_b, float *out_b,
                           int64_t n_b, int64_t num_partials, int64_t chunks, void *stream);
 
+/* Column sums of up to eight arrays in one launch: sums[i].out[c] = sum_p sums[i].parts[p][c], c < n (a multiple of 4), p <
+ * num_partials, in a fixed order.  `sums` is a host array, read before the call returns. */
+typedef struct lffn_sum {
+    const float *parts;
+    float *out;
+    int64_t n, num_partials;
+} lffn_sum;
+int lffn_sum_many_f32(const lffn_sum *sums, int32_t count, void *stream);
+
 /*
  * Backward of the layer's LayerNorm (torch.nn.LayerNorm over the last dimension, PL/lookup.py:84,99)
  * in one kernel; mean and 1/sigma are recomputed from x.
@@ -744,6 +753,13 @@ int lffn_lookup_scatter_sorted_f32(const int32_t *code, const float *score, cons
 int lffn_lookup_backward_f32(const int32_t *code, const float *score, const float *g, const float *tables,
                              float *grad_score, float *grad_tables, void *workspace, int64_t workspace_bytes,
                              int64_t B, int64_t T, int64_t S, int64_t Do, int32_t accumulate, void *stream);
+
+/* The same with partial column sums of g, [rows, Do] with rows of lffn_lookup_backward_sums_rows: the output bias's gradient
+ * (PL/lookup.py:108) is the sum of these rows. */
+int lffn_lookup_backward_sums_f32(const int32_t *code, const float *score, const float *g, const float *tables,
+                                  float *grad_score, float *grad_tables, float *sums, void *workspace, int64_t workspace_bytes,
+                                  int64_t B, int64_t T, int64_t S, int64_t Do, int32_t accumulate, void *stream);
+int lffn_lookup_backward_sums_rows(int64_t B, int64_t *rows);
 
 /*
  * The indexed inner product as the layer's backward issues it: table-local codes,

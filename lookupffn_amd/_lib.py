@@ -138,6 +138,14 @@ class BlockFront(ctypes.Structure):
                 ("ln_eps", _f32), ("decay", _f32), ("residual", _f32)]
 
 
+class Sum(ctypes.Structure):
+    """struct lffn_sum of include/lookupffn_hip.h."""
+    _fields_ = [("parts", _vp), ("out", _vp), ("n", _i64), ("num_partials", _i64)]
+
+
+SIGNATURES["lffn_sum_many_f32"] = [ctypes.POINTER(Sum), _i32, _vp]
+SIGNATURES["lffn_lookup_backward_sums_f32"] = [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _vp]
+SIGNATURES["lffn_lookup_backward_sums_rows"] = [_i64, ctypes.POINTER(_i64)]
 SIGNATURES["lffn_bh4_block_front_split_f32"] = [ctypes.POINTER(BlockFront), _vp, _i64, _vp]
 SIGNATURES["lffn_bh4_block_front_train_split_f32"] = [ctypes.POINTER(BlockFront), _vp, _vp, _vp, _vp, _i64, _vp]
 SIGNATURES["lffn_lookup_ffn_fused_layer_f32"] = [ctypes.POINTER(FusedLayer), _vp, _vp, _vp, _i64, _vp]

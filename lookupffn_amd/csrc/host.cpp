@@ -31,6 +31,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/lookupffn_hip.h"
 
@@ -59,15 +60,17 @@ using torch::autograd::variable_list;
     X(lffn_bh4_fold_split_f32)              \
     X(lffn_bh4_fold_mode_f32)               \
     X(lffn_lookup_scatter_workspace_bytes)  \
-    X(lffn_lookup_backward_f32)             \
+    X(lffn_lookup_backward_sums_f32)        \
+    X(lffn_lookup_backward_sums_rows)       \
     X(lffn_lookup_inner_f32)                \
     X(lffn_lookup_scatter_f32)              \
     X(lffn_lookup_scatter_sorted_f32)       \
     X(lffn_ln_project_hash_bwd_f32)         \
-        X(lffn_bh4_block_score_bwd_split_f32)   \
+    X(lffn_bh4_block_score_bwd_split_f32)   \
     X(lffn_ln_bh4_block_wgrad_f32)          \
     X(lffn_layer_norm_bwd_f32)              \
-    X(lffn_sum_partials_f32)
+    X(lffn_sum_partials_f32)                \
+    X(lffn_sum_many_f32)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -283,22 +286,32 @@ void infer(const Config &c, const Params &p, const Tensor &split, const Tensor &
     gather(c, codes, scores, p[4], p[5], residual, out, B, plan, st);
 }
 
-// Column sums of one or two [P, n] arrays of partial sums, fixed order of additions; many rows go through a first
-// pass over chunks of rows on many workgroups.
-void column_sums(const float *a, float *out_a, int64_t na, const float *b, float *out_b, int64_t nb, int64_t P,
-                 const at::Device &dev, void *st) {
-    Tensor mid;
-    if (P > 4 * limits.sum_chunk_rows) {
-        int64_t chunks = (P + limits.sum_chunk_rows - 1) / limits.sum_chunk_rows;
-        const int64_t each = (P + chunks - 1) / chunks;
-        chunks = (P + each - 1) / each;                    // no empty chunk
-        mid = empty_f32({chunks * (na + nb)}, dev);
-        float *ma = f32(mid), *mb = nb ? ma + chunks * na : nullptr;
-        CALL(lffn_sum_partials_f32, a, ma, na, b, mb, nb, P, chunks, st);
-        a = ma; b = mb; P = chunks;
+// Column sums of [P, n] arrays of partial sums, all in one launch at the end, fixed order of additions.  Very many rows go through a
+// first pass over chunks of rows on many workgroups.
+struct ColumnSums {
+    std::array<lffn_sum, 8> sums{};
+    int32_t count = 0;
+    std::vector<Tensor> held;               // until finish(): what they are formed from, and results that nobody else may hold
+
+    void add(const Tensor &parts, const float *a, const Tensor &out, int64_t n, int64_t P, const at::Device &dev, void *st) {
+        held.push_back(parts);
+        held.push_back(out);
+        if (P > MANY_ROWS) {
+            int64_t chunks = (P + limits.sum_chunk_rows - 1) / limits.sum_chunk_rows;
+            const int64_t each = (P + chunks - 1) / chunks;
+            chunks = (P + each - 1) / each;                    // no empty chunk
+            held.push_back(empty_f32({chunks * n}, dev));
+            float *mid = f32(held.back());
+            CALL(lffn_sum_partials_f32, a, mid, n, nullptr, nullptr, 0, P, chunks, st);
+            a = mid; P = chunks;
+        }
+        sums.at(count++) = {a, f32(out), n, P};
     }
-    CALL(lffn_sum_partials_f32, a, out_a, na, b, out_b, nb, P, 1, st);
-}
+    void finish(void *st) {
+        if (count) CALL(lffn_sum_many_f32, sums.data(), count, st);
+    }
+    static constexpr int64_t MANY_ROWS = 4096;
+};
 
 // Inputs of the node, in the order of its gradients.
 enum Input { X, LN_W, LN_B, WEIGHT, PBIAS, TABLES, OBIAS, RESIDUAL, INPUTS };
@@ -353,10 +366,9 @@ struct LookupFFNBackward : public torch::autograd::Node {
         bool need[INPUTS];
         for (int i = 0; i < INPUTS; ++i) need[i] = task_should_compute_output(i);
         if (need[RESIDUAL]) out[RESIDUAL] = grads[0];
-        if (need[OBIAS]) {
-            out[OBIAS] = empty_f32({Do}, dev);
-            column_sums(f32(g), f32(out[OBIAS]), Do, nullptr, nullptr, 0, B, dev, st);
-        }
+        ColumnSums column_sums;
+        if (need[OBIAS]) out[OBIAS] = empty_f32({Do}, dev);
+        bool bias_summed = !need[OBIAS];                        // in the scatter's copy of g
         const bool need_ln = need[X] || need[LN_W] || need[LN_B];
         const bool need_score = need_ln || need[WEIGHT] || need[PBIAS];
         // both gradients of the gather: one call with one workspace where the sorted scatter is the one to use
@@ -369,17 +381,26 @@ struct LookupFFNBackward : public torch::autograd::Node {
             if (B <= LFFN_SCATTER_LIST_TOKENS || B * T * Do < limits.sorted_min_work) ws_bytes = 0;
             if (need[TABLES] && ws_bytes > 0) {
                 Tensor ws = empty_bytes(ws_bytes, dev);
-                if (need_score)
-                    CALL(lffn_lookup_backward_f32, cp, f32(score), f32(g), f32(tab), f32(g_score), f32(out[TABLES]), ws.data_ptr(), ws_bytes, B,
-                         T, S, Do, 0, st);
-                else
+                if (need_score) {
+                    int64_t rows = 0;
+                    CALL(lffn_lookup_backward_sums_rows, B, &rows);
+                    Tensor parts = bias_summed ? Tensor() : empty_f32({rows * Do}, dev);
+                    CALL(lffn_lookup_backward_sums_f32, cp, f32(score), f32(g), f32(tab), f32(g_score), f32(out[TABLES]),
+                         bias_summed ? nullptr : f32(parts), ws.data_ptr(), ws_bytes, B, T, S, Do, 0, st);
+                    if (!bias_summed) column_sums.add(parts, f32(parts), out[OBIAS], Do, rows, dev, st);
+                    bias_summed = true;
+                } else
                     CALL(lffn_lookup_scatter_sorted_f32, cp, f32(score), f32(g), f32(out[TABLES]), ws.data_ptr(), ws_bytes, B, T, S, Do, 0, st);
             } else {
                 if (need_score) CALL(lffn_lookup_inner_f32, cp, f32(g), f32(tab), f32(g_score), B, T, S, Do, st);
                 if (need[TABLES]) CALL(lffn_lookup_scatter_f32, cp, f32(score), f32(g), f32(out[TABLES]), B, T, S, Do, 0, st);
             }
         }
-        if (!need_score) return out;
+        if (!bias_summed) column_sums.add(g, f32(g), out[OBIAS], Do, B, dev, st);
+        if (!need_score) {
+            column_sums.finish(st);
+            return out;
+        }
 
         const float decay = (float)c.decay, res = (float)c.residual, eps = (float)c.eps;
         Tensor g_h = empty_f32({R, B, H}, dev);            // gradient of the LayerNorm output, one slab per repeat
@@ -391,7 +412,8 @@ struct LookupFFNBackward : public torch::autograd::Node {
                  T, n, decay, res, st);
             if (need[WEIGHT] || need[PBIAS]) {
                 Tensor g_w = at::empty_like(w), g_b = empty_f32({R * D}, dev);
-                column_sums(pd, f32(g_w), R * J * D, pb, f32(g_b), R * D, n, dev, st);
+                column_sums.add(parts, pd, g_w, R * J * D, n, dev, st);
+                column_sums.add(parts, pb, g_b, R * D, n, dev, st);
                 if (need[WEIGHT]) out[WEIGHT] = g_w;
                 if (need[PBIAS]) out[PBIAS] = g_b.narrow(0, 0, T * 8);
             }
@@ -413,18 +435,20 @@ struct LookupFFNBackward : public torch::autograd::Node {
             }
             if (need[PBIAS]) {
                 out[PBIAS] = empty_f32({T * 8}, dev);
-                column_sums(f32(g_b), f32(out[PBIAS]), T * 8, nullptr, nullptr, 0, parts, dev, st);
+                column_sums.add(g_b, f32(g_b), out[PBIAS], T * 8, parts, dev, st);
             }
         }
         if (need_ln) {
             const int64_t n = std::max<int64_t>(1, std::min(limits.ln_partials, (B + 3) / 4));
             Tensor parts = empty_f32({2 * n * H}, dev), g_x = at::empty_like(x_), g_lw = empty_f32({H}, dev), g_lb = empty_f32({H}, dev);
             CALL(lffn_layer_norm_bwd_f32, f32(x_), f32(lw), eps, f32(g_h), f32(g_x), f32(parts), f32(parts) + n * H, B, H, R, n, st);
-            column_sums(f32(parts), f32(g_lw), H, f32(parts) + n * H, f32(g_lb), H, n, dev, st);
+            column_sums.add(parts, f32(parts), g_lw, H, n, dev, st);
+            column_sums.add(parts, f32(parts) + n * H, g_lb, H, n, dev, st);
             if (need[X]) out[X] = g_x;
             if (need[LN_W]) out[LN_W] = g_lw;
             if (need[LN_B]) out[LN_B] = g_lb;
         }
+        column_sums.finish(st);
         return out;
     }
 };

@@ -162,6 +162,60 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(SumPartialsArgs a) {
     }
 }
 
+// Column sums of several arrays in one launch: what a layer's backward leaves for its end.  A workgroup owns 32 columns of one
+// array; eight lanes side by side read 128 contiguous bytes of a row, the 128 lane groups take rows 128 apart, four loads in flight
+// each.  Fixed order: a lane's rows ascending, the eight groups of a wavefront by halves, the wavefronts ascending.
+// One launch in the place of three to six of 3 to 6 us that are nothing but round trips: TIMES
+constexpr int MANY = 8, MANY_WG = 1024, MANY_COLS = 32, MANY_GROUPS = MANY_WG / (MANY_COLS / 4);
+struct SumManyArgs {
+    const float *parts[MANY];
+    float *out[MANY];
+    int64_t n[MANY], P[MANY];
+    int first[MANY + 1];   // workgroup number of an array's first
+};
+
+__global__ __launch_bounds__(MANY_WG) void sum_many_kernel(SumManyArgs a) {
+    __shared__ float4 red[MANY_WG / 64][MANY_COLS / 4];
+    int i = 0;
+    while ((int)blockIdx.x >= a.first[i + 1]) ++i;            // uniform
+    const int64_t n = a.n[i], P = a.P[i];
+    const float *parts = a.parts[i];
+    const int c4 = threadIdx.x % (MANY_COLS / 4), wave = threadIdx.x >> 6;
+    const int64_t col = int64_t(blockIdx.x - a.first[i]) * MANY_COLS + c4 * 4;
+    const bool on = col < n;                                  // n % 4 == 0: all four columns or none
+    const int64_t colc = on ? col : 0;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    constexpr int DEPTH = 4;
+    for (int64_t p0 = threadIdx.x / (MANY_COLS / 4); p0 < P; p0 += MANY_GROUPS * DEPTH) {
+        float4 v[DEPTH];
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u)                       // unconditional loads at clamped rows
+            v[u] = *reinterpret_cast<const float4 *>(parts + min<int64_t>(p0 + MANY_GROUPS * u, P - 1) * n + colc);
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) {
+            if (p0 + MANY_GROUPS * u < P) { acc.x += v[u].x; acc.y += v[u].y; acc.z += v[u].z; acc.w += v[u].w; }
+        }
+    }
+    auto over_groups = [](float v) {
+        v += lane_xor<8>(v);
+        v += lane_xor<16>(v);
+        v += lane_xor<32>(v);
+        return v;
+    };
+    acc.x = over_groups(acc.x); acc.y = over_groups(acc.y); acc.z = over_groups(acc.z); acc.w = over_groups(acc.w);
+    if ((threadIdx.x & 63) < MANY_COLS / 4) red[wave][c4] = acc;
+    __syncthreads();
+    if (threadIdx.x < MANY_COLS / 4 && on) {
+        float4 s = red[0][c4];
+#pragma unroll
+        for (int w = 1; w < MANY_WG / 64; ++w) {
+            const float4 q = red[w][c4];
+            s.x += q.x; s.y += q.y; s.z += q.z; s.w += q.w;
+        }
+        *reinterpret_cast<float4 *>(a.out[i] + col) = s;
+    }
+}
+
 }  // namespace
 
 // Scratch of lffn_layer_norm_bwd_noalloc_f32: the per-workgroup partial sums of the weight and bias
@@ -213,6 +267,28 @@ extern "C" int lffn_sum_partials_f32(const float *parts_a, float *out_a, int64_t
     LFFN_REQUIRE((chunks - 1) * (int64_t)a.rows_per_chunk < num_partials, LFFN_ERR_BAD_ARG);
     hipLaunchKernelGGL(sum_partials_kernel, dim3((unsigned)blocks, (unsigned)chunks), dim3(256), 0,
                        static_cast<hipStream_t>(stream), a);
+    return lffn_launch_status();
+}
+
+extern "C" int lffn_sum_many_f32(const lffn_sum *sums, int32_t count, void *stream) {
+    LFFN_REQUIRE(count >= 0 && count <= MANY && (sums || count == 0), LFFN_ERR_BAD_ARG);
+    SumManyArgs a{};
+    int64_t blocks = 0;
+    int used = 0;
+    for (int i = 0; i < count; ++i) {
+        const lffn_sum &s = sums[i];
+        LFFN_REQUIRE(s.n >= 0 && s.num_partials >= 1 && s.num_partials <= (int64_t(1) << 30), LFFN_ERR_BAD_ARG);
+        LFFN_REQUIRE(s.n % 4 == 0 && s.n <= (int64_t(1) << 30), LFFN_ERR_UNSUPPORTED);
+        if (s.n == 0) continue;
+        LFFN_REQUIRE(s.parts && s.out && lffn_aligned16(s.parts) && lffn_aligned16(s.out), LFFN_ERR_BAD_ARG);
+        a.parts[used] = s.parts; a.out[used] = s.out; a.n[used] = s.n; a.P[used] = s.num_partials;
+        a.first[used++] = (int)blocks;
+        blocks += (s.n + MANY_COLS - 1) / MANY_COLS;
+        LFFN_REQUIRE(blocks <= 0x7fffffff, LFFN_ERR_UNSUPPORTED);
+    }
+    if (used == 0) return LFFN_OK;
+    for (int i = used; i <= MANY; ++i) a.first[i] = (int)blocks;
+    hipLaunchKernelGGL(sum_many_kernel, dim3((unsigned)blocks), dim3(MANY_WG), 0, static_cast<hipStream_t>(stream), a);
     return lffn_launch_status();
 }
 

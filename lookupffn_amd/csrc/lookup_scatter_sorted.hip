@@ -59,6 +59,7 @@ struct PrepArgs {
     uint16_t *code_t;      // [T, Bp]
     float *score_t;        // [T, Bp]
     float *g_packed;       // [Do / SC][B + 1][SC], the last row zero
+    float *sums;           // [ceil((B + 1) / PACK_TOKENS), Do] or null: column sums of the rows of g that a workgroup copies
     int64_t B, Bp;
     int T, S, Do, tiles_t;
 };
@@ -101,29 +102,45 @@ __global__ __launch_bounds__(256) void lookup_prep_kernel(PrepArgs a) {
 
 constexpr int PACK_TOKENS = 32;      // rows of g per workgroup of the slice-major copy
 
-// PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy); row B is the padding's
+// PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy); row B is the padding's.  A thread has four
+// columns of every G-th row, so that their sum (the output bias's gradient) is a few additions and a pass over LDS: TIMES
 __device__ __forceinline__ void pack_rows(const PrepArgs &a, int64_t blk) {
+    extern __shared__ int sm[];
+    float4 *const part = reinterpret_cast<float4 *>(sm);     // [SORT_WG]
     const int64_t b0 = blk * PACK_TOKENS;
-    const int q = a.Do / 4;
-    // eight loads per thread in flight before the first store (a store must not overtake a load the compiler
-    // cannot prove independent of it, so load-store pairs one after the other would each wait out a round trip)
-    constexpr int DEPTH = 8;
-    for (int e0 = threadIdx.x; e0 < PACK_TOKENS * q; e0 += SORT_WG * DEPTH) {
-        float4 v[DEPTH];
+    for (int q0 = 0; q0 < a.Do / 4; q0 += SORT_WG) {
+        const int q = min(a.Do / 4 - q0, SORT_WG), G = SORT_WG / q;
+        const int grp = threadIdx.x / q, col = (q0 + (int)threadIdx.x % q) * 4;
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        // eight loads per thread in flight before the first store (a store must not overtake a load the compiler
+        // cannot prove independent of it, so load-store pairs one after the other would each wait out a round trip)
+        constexpr int DEPTH = 8;
+        for (int r0 = grp < G ? grp : PACK_TOKENS; r0 < PACK_TOKENS; r0 += G * DEPTH) {
+            float4 v[DEPTH];
 #pragma unroll
-        for (int i = 0; i < DEPTH; ++i) {
-            const int e = e0 + i * SORT_WG;
-            const int64_t b = b0 + e / q;
-            v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (e < PACK_TOKENS * q && b < a.B) v[i] = *reinterpret_cast<const float4 *>(a.g + (size_t)b * a.Do + (e % q) * 4);
+            for (int i = 0; i < DEPTH; ++i) {
+                const int64_t b = b0 + r0 + i * G;
+                v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (r0 + i * G < PACK_TOKENS && b < a.B) v[i] = *reinterpret_cast<const float4 *>(a.g + (size_t)b * a.Do + col);
+            }
+#pragma unroll
+            for (int i = 0; i < DEPTH; ++i) {
+                const int64_t b = b0 + r0 + i * G;
+                sum.x += v[i].x; sum.y += v[i].y; sum.z += v[i].z; sum.w += v[i].w;
+                if (r0 + i * G < PACK_TOKENS && b <= a.B)
+                    *reinterpret_cast<float4 *>(a.g_packed + ((size_t)(col / SC) * (a.B + 1) + b) * SC + col % SC) = v[i];
+            }
         }
-#pragma unroll
-        for (int i = 0; i < DEPTH; ++i) {
-            const int e = e0 + i * SORT_WG;
-            const int64_t b = b0 + e / q;
-            const int col = (e % q) * 4;
-            if (e < PACK_TOKENS * q && b <= a.B)
-                *reinterpret_cast<float4 *>(a.g_packed + ((size_t)(col / SC) * (a.B + 1) + b) * SC + col % SC) = v[i];
+        if (!a.sums) continue;                                // uniform
+        __syncthreads();                                      // (the columns before have been read)
+        part[threadIdx.x] = sum;
+        __syncthreads();
+        if (grp == 0) {
+            for (int k = 1; k < G; ++k) {
+                const float4 t = part[threadIdx.x + k * q];
+                sum.x += t.x; sum.y += t.y; sum.z += t.z; sum.w += t.w;
+            }
+            *reinterpret_cast<float4 *>(a.sums + blk * a.Do + col) = sum;
         }
     }
 }
@@ -470,6 +487,7 @@ inline bool sorted_supported(int64_t B, int64_t T, int64_t S, int64_t Do) {
            B <= (int64_t(1) << 31) - 1 && T <= (1 << 20) && T * ((Do / SC + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff;
 }
 
+inline int64_t pack_workgroups(int64_t Bc) { return (Bc + 1 + PACK_TOKENS - 1) / PACK_TOKENS; }
 inline int64_t round16(int64_t v) { return (v + 15) & ~int64_t(15); }
 inline int64_t padded_tokens(int64_t B) { return (B + 63) & ~int64_t(63); }
 
@@ -508,7 +526,7 @@ namespace {
 // chunk from the same slice-major copy of g the scatter reads (lookup_prep_kernel writes it once per chunk).
 // grad_tables may be null (score gradient only).
 int sorted_backward(const int32_t *code, const float *score, const float *g, const float *tables, float *grad_score,
-                    float *grad_tables, void *workspace, int64_t workspace_bytes, int64_t B, int64_t T, int64_t S,
+                    float *grad_tables, float *sums, void *workspace, int64_t workspace_bytes, int64_t B, int64_t T, int64_t S,
                     int64_t Do, int32_t accumulate, void *stream) {
     const Workspace w = workspace_layout(B, T, S, Do);
     LFFN_REQUIRE(workspace_bytes >= w.total, LFFN_ERR_BAD_ARG);
@@ -527,10 +545,12 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         pa.score_t = reinterpret_cast<float *>(base + w.score_t);
         pa.g_packed = reinterpret_cast<float *>(base + w.g_packed);
         pa.B = Bc; pa.Bp = Bp; pa.T = (int)T; pa.S = (int)S; pa.Do = (int)Do;
+        pa.sums = sums;
         pa.tiles_t = (int)((T + 63) / 64);
         // (score gradient only: the codes and scores need no transposing or sorting, only g its slice-major copy)
         const int64_t transpose_blocks = grad_tables ? (Bp / 64) * pa.tiles_t : 0;
-        const int64_t pack_blocks = (Bc + 1 + PACK_TOKENS - 1) / PACK_TOKENS;
+        const int64_t pack_blocks = pack_workgroups(Bc);
+        if (sums) sums += pack_blocks * Do;
         const int64_t nsort = grad_tables ? T : 0;
         LFFN_REQUIRE(transpose_blocks <= 0x7fffffff && nsort + pack_blocks <= 0x7fffffff, LFFN_ERR_UNSUPPORTED);
         int rc = LFFN_OK;
@@ -548,7 +568,8 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         const size_t tables_lds = (size_t(SORT_WAVES) * S + 2 * S + 4 + 4) * sizeof(int);
         const size_t staged_lds = tables_lds + size_t(stride) * 6 + 16;
         sa.stage = staged_lds <= 160 * 1024 ? 1 : 0;            // 512-row tables: the list goes straight to memory
-        const size_t sort_lds = nsort ? (sa.stage ? staged_lds : tables_lds) : 0;
+        size_t sort_lds = nsort ? (sa.stage ? staged_lds : tables_lds) : 0;
+        if (pa.sums && sort_lds < SORT_WG * sizeof(float4)) sort_lds = SORT_WG * sizeof(float4);
         static LdsGrant granted;
         if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_sort_pack_kernel), sort_lds, granted))
             return LFFN_ERR_LAUNCH;
@@ -587,7 +608,7 @@ extern "C" int lffn_lookup_scatter_sorted_f32(const int32_t *code, const float *
     LFFN_REQUIRE(sorted_supported(B, T, S, Do), LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(code && score && g && grad_tables && workspace, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(lffn_aligned16(grad_tables) && lffn_aligned16(g) && lffn_aligned16(workspace), LFFN_ERR_BAD_ARG);
-    return sorted_backward(code, score, g, nullptr, nullptr, grad_tables, workspace, workspace_bytes, B, T, S, Do, accumulate,
+    return sorted_backward(code, score, g, nullptr, nullptr, grad_tables, nullptr, workspace, workspace_bytes, B, T, S, Do, accumulate,
                            stream);
 }
 
@@ -596,18 +617,31 @@ extern "C" int lffn_lookup_scatter_sorted_f32(const int32_t *code, const float *
 //   grad_tables[t,s] = sum over b with code[b,t] = s of score[b,t] * g[b,:]   (overwritten, or added to)
 // Per chunk of 16384 tokens: one kernel transposes code and score and copies g slice-major, the score-gradient
 // kernel and the sorted scatter both read that copy.
-extern "C" int lffn_lookup_backward_f32(const int32_t *code, const float *score, const float *g, const float *tables,
-                                        float *grad_score, float *grad_tables, void *workspace,
-                                        int64_t workspace_bytes, int64_t B, int64_t T, int64_t S, int64_t Do,
-                                        int32_t accumulate, void *stream) {
+extern "C" int lffn_lookup_backward_sums_f32(const int32_t *code, const float *score, const float *g, const float *tables,
+                                             float *grad_score, float *grad_tables, float *sums, void *workspace,
+                                             int64_t workspace_bytes, int64_t B, int64_t T, int64_t S, int64_t Do,
+                                             int32_t accumulate, void *stream) {
     LFFN_REQUIRE(B >= 0 && T >= 0 && S >= 1 && Do >= 1, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(sorted_supported(B, T, S, Do) && Do % 64 == 0, LFFN_ERR_UNSUPPORTED);
     LFFN_REQUIRE(code && g && workspace && (grad_score || grad_tables), LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE((!grad_score || tables) && (!grad_tables || score), LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(lffn_aligned16(g) && lffn_aligned16(workspace) && (!grad_tables || lffn_aligned16(grad_tables)) &&
-                     (!tables || lffn_aligned16(tables)), LFFN_ERR_BAD_ARG);
-    return sorted_backward(code, score, g, tables, grad_score, grad_tables, workspace, workspace_bytes, B, T, S, Do,
+                     (!tables || lffn_aligned16(tables)) && lffn_aligned16(sums), LFFN_ERR_BAD_ARG);
+    return sorted_backward(code, score, g, tables, grad_score, grad_tables, sums, workspace, workspace_bytes, B, T, S, Do,
                            accumulate, stream);
+}
+
+extern "C" int lffn_lookup_backward_f32(const int32_t *code, const float *score, const float *g, const float *tables,
+                                        float *grad_score, float *grad_tables, void *workspace, int64_t workspace_bytes,
+                                        int64_t B, int64_t T, int64_t S, int64_t Do, int32_t accumulate, void *stream) {
+    return lffn_lookup_backward_sums_f32(code, score, g, tables, grad_score, grad_tables, nullptr, workspace, workspace_bytes, B, T, S,
+                                         Do, accumulate, stream);
+}
+
+extern "C" int lffn_lookup_backward_sums_rows(int64_t B, int64_t *rows) {
+    LFFN_REQUIRE(rows && B >= 0, LFFN_ERR_BAD_ARG);
+    *rows = B / CHUNK * pack_workgroups(CHUNK) + (B % CHUNK ? pack_workgroups(B % CHUNK) : 0);
+    return LFFN_OK;
 }
 
 // ---------------------------------------------------------------------------

@@ -209,6 +209,41 @@ def test_block_weight_gradient_over_long_chunks(B):
         assert ((got[s] - torch.bmm(p, u)).abs() <= (B + 4) * 2.0 ** -24 * torch.bmm(p.abs(), u.abs())).all(), s
 
 
+@pytest.mark.parametrize("shapes", [[(1, 4)], [(513, 768), (2, 36), (127, 32)], [(2049, 64), (128, 1024), (129, 4), (512, 4096), (3, 8)] + 3 * [(40, 0)]])
+def test_sums_of_many_arrays(shapes):
+    """At most 17 numbers to a lane, then 3 + 15 additions: 36 roundings of the magnitudes' sum."""
+    gen = torch.Generator(device="cuda").manual_seed(len(shapes))
+    parts = [torch.randn(s, generator=gen, device="cuda") for s in shapes]
+    outs = [torch.full((n,), float("nan"), device="cuda") for _, n in shapes]
+    sums = (_lib.Sum * len(shapes))(*[_lib.Sum(p.data_ptr(), o.data_ptr(), n, P) for p, o, (P, n) in zip(parts, outs, shapes)])
+    assert _lib.load().lffn_sum_many_f32(sums, len(shapes), _lib.stream_of(parts[0])) == 0
+    for p, o in zip(parts, outs):
+        assert ((o - p.double().sum(0)).abs() <= 36 * 2.0 ** -24 * p.double().abs().sum(0)).all()
+
+
+# rows around the copy's 32 and its chunks of 16384; columns that leave threads idle, and more than one workgroup has threads for
+@pytest.mark.parametrize("B,Do", [(1, 64), (31, 192), (32, 512), (1000, 1088), (70, 8192), (16384, 64), (16385, 128)])
+def test_column_sums_of_the_backwards_copy(B, Do):
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    T, S, L = 8, 16, _lib.load()
+    code = torch.randint(0, S, (B, T), generator=gen, device="cuda", dtype=torch.int32)
+    score, g = torch.rand(B, T, generator=gen, device="cuda"), torch.randn(B, Do, generator=gen, device="cuda")
+    tables = torch.randn(T, S, Do, generator=gen, device="cuda")
+    size = ctypes.c_int64()
+    assert L.lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(size)) == 0
+    ws, results = torch.empty(size.value, dtype=torch.uint8, device="cuda"), []
+    assert L.lffn_lookup_backward_sums_rows(B, ctypes.byref(size)) == 0
+    sums = torch.full((size.value, Do), float("nan"), device="cuda")
+    for to in (sums, None):
+        gs, gt = torch.empty(B, T, device="cuda"), torch.empty_like(tables)
+        assert L.lffn_lookup_backward_sums_f32(code.data_ptr(), score.data_ptr(), g.data_ptr(), tables.data_ptr(), gs.data_ptr(), gt.data_ptr(),
+                                               _lib.ptr(to), ws.data_ptr(), ws.numel(), B, T, S, Do, 0, _lib.stream_of(g)) == 0
+        results.append((gs, gt))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+    got = sums.double().sum(0)                              # each row of it the sum of at most 32 numbers
+    assert ((got - g.double().sum(0)).abs() <= 32 * 2.0 ** -24 * g.double().abs().sum(0)).all()
+
+
 # Both gradients of the layer's gather for few tokens and just past it: row groups of 32 and smaller tables, column passes, every token
 # on one row, adding to what is there
 @pytest.mark.parametrize("B,T,S,Do", [(1, 1, 256, 64), (5, 9, 16, 320), (64, 3, 32, 1088), (384, 65, 256, 768), (385, 8, 128, 256),
