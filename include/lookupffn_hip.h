@@ -793,6 +793,9 @@ int lffn_lookup_inner_f32(const int32_t *code, const float *g, const float *tabl
  */
 int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t stages, int64_t num_block, int64_t block_size,
                             int32_t transposed, void *stream);
+/* Both forms, transposed and not, in one launch: what a training step takes. */
+int lffn_bh4_fold_split_both_f32(const float *w, float *w_split, float *w_split_t, int64_t stages, int64_t num_block,
+                                 int64_t block_size, void *stream);
 
 /*
  * The hashing front end: lffn_ln_bh4_block_hash_f32 (codes and scores) or, with records set,
@@ -827,10 +830,11 @@ int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float
 /*
  * lffn_bh4_block_bwd_split_f32 behind the gradient of the 8-bit scores: from z [B, T*8] (16-byte aligned) and g_score [B, T], with the
  * gradient of z that lffn_code_score_bwd_f32 computes formed inside.  bias_parts: [ceil(B / 16), T*8] or NULL, every sixteen tokens'
- * sum of it (the projection bias's gradient is the sum of these rows).
+ * sum of it (the projection bias's gradient is the sum of these rows).  clear: an array of clear_n floats (a multiple of 4; 16-byte aligned)
+ * that is set to zero on the way, such as what the weight gradient is added to, or NULL.
  */
 int lffn_bh4_block_score_bwd_split_f32(const float *z, const float *g_score, const float *w_split_t, float *g_x,
-                                       float *stage_grads, float *bias_parts, int64_t B, int64_t H, int64_t D, int64_t R,
+                                       float *stage_grads, float *bias_parts, float *clear, int64_t clear_n, int64_t B, int64_t H, int64_t D, int64_t R,
                                        int64_t J, int64_t T, int64_t block_size, float decay, float residual, void *stream);
 
 /* ------------------------------------------------- the encoder around the layer */

@@ -108,7 +108,8 @@ SIGNATURES = {
     "lffn_scatter_rows_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)],
     "lffn_scatter_rows": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i32, _i32, _vp],
     "lffn_bh4_fold_split_f32": [_vp, _vp, _i64, _i64, _i64, _i32, _vp],
-    "lffn_bh4_block_score_bwd_split_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp],
+    "lffn_bh4_fold_split_both_f32": [_vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "lffn_bh4_block_score_bwd_split_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp],
     "lffn_bh4_block_bwd_split_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp],
     "lffn_linear_f32": [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _vp, ctypes.POINTER(_vp), _i64, _i64, _i64, _i64, _vp],
     "lffn_linear_norm_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(_i64)],

@@ -59,7 +59,7 @@ __device__ __forceinline__ float wave_most(float v) {
 // and product wavefront four fragments of 64 lanes x 8 numbers: hi of the first and the second eight columns of a lane's sixteen, then lo
 // of them; behind all blocks the inverse scales, [stage][64].
 template <bool TRANSPOSED>
-__global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, uint32_t *out, float *inverse) {
+__device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float *inverse) {
     __shared__ float most_s[16][BS], scale_s[BS];
     const int num_block = blockDim.x / 64, wave = threadIdx.x >> 6;
     const int64_t blk = int64_t(blockIdx.x) * num_block + wave;
@@ -149,6 +149,12 @@ __global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, ui
     }
 }
 
+// One of the two forms, or both (gridDim.y 2: a training step's, in one launch)
+__global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, float *out, float *out_t, int64_t numbers) {
+    if (blockIdx.y == 0 && out) fold_split<false>(w, reinterpret_cast<uint32_t *>(out), out + numbers);
+    else fold_split<true>(w, reinterpret_cast<uint32_t *>(out_t), out_t + numbers);
+}
+
 struct SplitArgs {
     const float *x;        // [B, H]
     const float *ln_w;     // [H] LayerNorm weight, or null: no LayerNorm
@@ -164,6 +170,8 @@ struct SplitArgs {
     int rec_tile;          // tokens per workgroup of the gather the records are written for
     float *z;              // training: [B, T*8] z, kept for the backward (backward from scores: read)
     const float *g_score;  // backward from scores: [B, T] gradient of the scores
+    float4 *clear;         // backward from scores: an array to clear on the way (the sum of the weights' gradient), or null
+    int64_t clear_n;
     float *bias_parts;     // backward from scores: [ceil(B/16), T*8] column sums of the gradient of z, or null
     float *row_stats;      // training, with LayerNorm: [B, 2] every row's mean and 1/sigma
     const float *gz;       // backward: [B, T*8] gradient of z
@@ -501,6 +509,10 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         // of the weights, a sum over the tokens, would keep that, so every other token's row has its sign turned on the way.
         inv_x = c & 1 ? -1.f : 1.f;
         if constexpr (SCORES) {
+            if (a.clear)
+                for (int64_t i = (int64_t(blockIdx.y) * gridDim.x + blockIdx.x) * (256 * BG) + tid; i < a.clear_n;
+                     i += int64_t(gridDim.x) * gridDim.y * (256 * BG))
+                    a.clear[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             z_gradients([&](int row, int col, f32x4 g) { *reinterpret_cast<f32x4 *>(rows32 + row * LDR + col) = g; });
             __syncthreads();
             if (a.bias_parts) {
@@ -820,20 +832,32 @@ int dispatch_block(const SplitArgs &a, int64_t D, hipStream_t st) {
 
 }  // namespace
 
-extern "C" int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t stages, int64_t num_block, int64_t block_size,
-                                       int32_t transposed, void *stream) {
+namespace {
+
+int fold_split_entry(const float *w, float *out, float *out_t, int64_t stages, int64_t num_block, int64_t block_size, void *stream) {
     LFFN_REQUIRE(stages >= 0 && stages <= (1 << 20) && num_block >= 1, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(block_size == BS && lffn_is_pow2(num_block) && num_block <= 16, LFFN_ERR_UNSUPPORTED);
     if (stages == 0) return LFFN_OK;
-    LFFN_REQUIRE(w && w_split && w != w_split && lffn_aligned16(w_split), LFFN_ERR_BAD_ARG);
-    float *inverse = w_split + stages * num_block * (BS * BS);
-    auto kern = transposed ? bh4_fold_split_kernel<true> : bh4_fold_split_kernel<false>;
-    const size_t lds = transposed ? 0 : num_block * 16 * 65 * sizeof(float);
+    LFFN_REQUIRE(w && (out || out_t) && w != out && w != out_t && lffn_aligned16(out) && lffn_aligned16(out_t), LFFN_ERR_BAD_ARG);
+    const size_t lds = out ? num_block * 16 * 65 * sizeof(float) : 0;
     static LdsGrant granted;
-    if (lds > 65000 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(kern), lds, granted)) return LFFN_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)stages), dim3((unsigned)(BS * num_block)), lds, static_cast<hipStream_t>(stream), w,
-                       reinterpret_cast<uint32_t *>(w_split), inverse);
+    if (lds > 50000 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(bh4_fold_split_kernel), lds, granted)) return LFFN_ERR_LAUNCH;
+    hipLaunchKernelGGL(bh4_fold_split_kernel, dim3((unsigned)stages, out && out_t ? 2 : 1), dim3((unsigned)(BS * num_block)), lds,
+                       static_cast<hipStream_t>(stream), w, out, out_t, stages * num_block * (BS * BS));
     return lffn_launch_status();
+}
+
+}  // namespace
+
+extern "C" int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t stages, int64_t num_block, int64_t block_size,
+                                       int32_t transposed, void *stream) {
+    return fold_split_entry(w, transposed ? nullptr : w_split, transposed ? w_split : nullptr, stages, num_block, block_size, stream);
+}
+
+extern "C" int lffn_bh4_fold_split_both_f32(const float *w, float *w_split, float *w_split_t, int64_t stages, int64_t num_block,
+                                            int64_t block_size, void *stream) {
+    LFFN_REQUIRE(stages == 0 || (w_split && w_split_t && w_split != w_split_t), LFFN_ERR_BAD_ARG);
+    return fold_split_entry(w, w_split, w_split_t, stages, num_block, block_size, stream);
 }
 
 namespace {
@@ -912,12 +936,15 @@ extern "C" int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_spl
 }
 
 extern "C" int lffn_bh4_block_score_bwd_split_f32(const float *z, const float *g_score, const float *w_split_t, float *g_x,
-                                                  float *stage_grads, float *bias_parts, int64_t B, int64_t H, int64_t D, int64_t R,
-                                                  int64_t J, int64_t T, int64_t block_size, float decay, float residual, void *stream) {
+                                                  float *stage_grads, float *bias_parts, float *clear, int64_t clear_n, int64_t B,
+                                                  int64_t H, int64_t D, int64_t R, int64_t J, int64_t T, int64_t block_size, float decay,
+                                                  float residual, void *stream) {
     SplitArgs a{};
     const int rc = back_args(w_split_t, g_x, stage_grads, B, H, D, R, J, T, block_size, decay, residual, a);
     if (rc != LFFN_OK || B == 0) return rc;
-    LFFN_REQUIRE(z && g_score && lffn_aligned16(z), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(z && g_score && lffn_aligned16(z) && lffn_aligned16(clear), LFFN_ERR_BAD_ARG);
+    LFFN_REQUIRE(!clear || (clear_n >= 0 && clear_n % 4 == 0), LFFN_ERR_BAD_ARG);
+    a.clear = reinterpret_cast<float4 *>(clear); a.clear_n = clear ? clear_n / 4 : 0;
     a.z = const_cast<float *>(z); a.g_score = g_score; a.bias_parts = bias_parts;
     return dispatch_block<SCORES_BACKWARD>(a, D, static_cast<hipStream_t>(stream));
 }

@@ -57,7 +57,7 @@ using torch::autograd::variable_list;
     X(lffn_lookup_gather_ws_f16)            \
     X(lffn_bh4_block_front_split_f32)       \
     X(lffn_bh4_block_front_train_split_f32) \
-    X(lffn_bh4_fold_split_f32)              \
+    X(lffn_bh4_fold_split_both_f32)         \
     X(lffn_bh4_fold_mode_f32)               \
     X(lffn_lookup_scatter_workspace_bytes)  \
     X(lffn_lookup_backward_sums_f32)        \
@@ -328,12 +328,12 @@ struct NoSecondDerivative : public torch::autograd::Node {
 struct LookupFFNBackward : public torch::autograd::Node {
     Config c{};
     int64_t B = 0;
-    SavedVariable x, ln_w, ln_b, weight, tables, codes, scores, z, stage_in, stats;
+    SavedVariable x, ln_w, ln_b, weight, tables, codes, scores, z, stage_in, stats, split_t;
 
     std::string name() const override { return "LookupFFNBackward"; }
 
     void release_variables() override {
-        for (SavedVariable *v : {&x, &ln_w, &ln_b, &weight, &tables, &codes, &scores, &z, &stage_in, &stats}) v->reset_data();
+        for (SavedVariable *v : {&x, &ln_w, &ln_b, &weight, &tables, &codes, &scores, &z, &stage_in, &stats, &split_t}) v->reset_data();
     }
 
     variable_list apply(variable_list &&grads) override {
@@ -418,16 +418,14 @@ struct LookupFFNBackward : public torch::autograd::Node {
                 if (need[PBIAS]) out[PBIAS] = g_b.narrow(0, 0, T * 8);
             }
         } else {
-            const Tensor stage = stage_in.unpack(self), st_ = stats.unpack(self);
+            const Tensor stage = stage_in.unpack(self), st_ = stats.unpack(self), split = split_t.unpack(self);
             const int64_t parts = (B + 15) / 16;               // of the projection bias's gradient
             Tensor g_b = need[PBIAS] ? empty_f32({parts * T * 8}, dev) : Tensor();
-            Tensor stage_g = empty_f32({R * J, B, D}, dev), split = empty_f32({split_words(c)}, dev);
+            Tensor stage_g = empty_f32({R * J, B, D}, dev), g_folded = need[WEIGHT] ? empty_f32({R * J * D * 64}, dev) : Tensor();
             const int64_t blocks = R * J * (D / 64);
-            CALL(lffn_bh4_fold_split_f32, f32(w), f32(split), R * J, D / 64, 64, 1, st);
             CALL(lffn_bh4_block_score_bwd_split_f32, f32(z_), f32(g_score), f32(split), f32(g_h), f32(stage_g), need[PBIAS] ? f32(g_b) : nullptr,
-                 B, H, D, R, J, T, 64, decay, res, st);
+                 need[WEIGHT] ? f32(g_folded) : nullptr, need[WEIGHT] ? R * J * D * 64 : 0, B, H, D, R, J, T, 64, decay, res, st);
             if (need[WEIGHT]) {
-                Tensor g_folded = at::zeros({R * J, D / 64, 64, 64}, at::TensorOptions().dtype(at::kFloat).device(dev));
                 CALL(lffn_ln_bh4_block_wgrad_f32, f32(stage_g), f32(x_), f32(lw), f32(lb), f32(st_), J > 1 ? f32(stage) : nullptr, f32(g_folded),
                      B, H, D, R, J, 64, st);
                 out[WEIGHT] = at::empty_like(w);
@@ -458,7 +456,7 @@ void train(const Config &c, const Params &p, const Tensor &x, const Tensor &resi
     void *st = stream_on(dev);
     auto node = std::shared_ptr<LookupFFNBackward>(new LookupFFNBackward(), torch::autograd::deleteNode);
     const auto int32 = at::TensorOptions().dtype(at::kInt).device(dev);
-    Tensor codes = at::empty({B, c.T}, int32), scores = empty_f32({B, c.T}, dev), z = empty_f32({B, c.T * 8}, dev), stage, stats;
+    Tensor codes = at::empty({B, c.T}, int32), scores = empty_f32({B, c.T}, dev), z = empty_f32({B, c.T * 8}, dev), stage, stats, split_t;
     int32_t *cp = static_cast<int32_t *>(codes.data_ptr());
     const float eps = (float)c.eps, decay = (float)c.decay, res = (float)c.residual;
     if (c.form == DIAG) {
@@ -468,7 +466,8 @@ void train(const Config &c, const Params &p, const Tensor &x, const Tensor &resi
         stage = empty_f32({c.R, c.J - 1, B, c.D}, dev);
         stats = empty_f32({B, 2}, dev);
         Tensor split = empty_f32({split_words(c)}, dev);
-        CALL(lffn_bh4_fold_split_f32, f32(p[2]), f32(split), c.R * c.J, c.D / 64, 64, 0, st);
+        split_t = empty_f32({split_words(c)}, dev);             // the backward's
+        CALL(lffn_bh4_fold_split_both_f32, f32(p[2]), f32(split), f32(split_t), c.R * c.J, c.D / 64, 64, st);
         lffn_block_front front = block_front(c, p, split);
         front.codes = cp;
         front.scores = f32(scores);
@@ -489,6 +488,7 @@ void train(const Config &c, const Params &p, const Tensor &x, const Tensor &resi
     node->z = SavedVariable(z, false);
     node->stage_in = SavedVariable(stage, false);
     node->stats = SavedVariable(stats, false);
+    node->split_t = SavedVariable(split_t, false);
     torch::autograd::set_history(out, node);
 }
 

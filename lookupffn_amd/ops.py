@@ -541,7 +541,7 @@ def _bh4_block_score_bwd_split_impl(z, g_score, w_split_t, R, J, D, H, decay, re
     parts = z.new_empty((B + 15) // 16, T * 8) if bias else None
     with _dev_guard(z):
         rc = _lib.load().lffn_bh4_block_score_bwd_split_f32(_lib.ptr(z), _lib.ptr(g_score), _lib.ptr(w_split_t), _lib.ptr(g_x),
-                                                            _lib.ptr(stage_g), _lib.ptr(parts), B, H, D, R, J, T, 64, decay, residual,
+                                                            _lib.ptr(stage_g), _lib.ptr(parts), None, 0, B, H, D, R, J, T, 64, decay, residual,
                                                             _lib.stream_of(z))
     _lib.check(rc, f"lffn_bh4_block_score_bwd_split_f32(B={B}, H={H}, D={D}, R={R}, J={J}, T={T})")
     return g_x, stage_g, _sum_partials(parts)[0] if bias else z.new_empty(0)

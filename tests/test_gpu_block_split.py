@@ -4,7 +4,7 @@ import math
 import pytest
 import torch
 
-from lookupffn_amd import ops
+from lookupffn_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -105,6 +105,20 @@ def test_backward_from_scores(B, H, D, R, T):
     assert torch.equal(g_x, want_x) and torch.equal(stage_g, want_stage)
     assert ((g_bias - g_z.double().sum(0)).abs() <= 64 * 2.0 ** -24 * g_z.double().abs().sum(0)).all()
     assert ops.bh4_block_score_bwd_split(z, g_score, split_t, R, J, D, H, 0.7, 0.3, False)[2].numel() == 0
+    for n in (4, 100004, 3 << 20):                    # and the array that it clears, to its last number and no further
+        clear = torch.ones(n + 4, device=DEV)
+        rc = _lib.load().lffn_bh4_block_score_bwd_split_f32(z.data_ptr(), g_score.data_ptr(), split_t.data_ptr(), g_x.data_ptr(), stage_g.data_ptr(),
+                                                            None, clear.data_ptr(), n, B, H, D, R, J, T, 64, 0.7, 0.3, _lib.stream_of(z))
+        assert rc == 0 and not clear[:n].any() and clear[n:].all()
+
+
+@pytest.mark.parametrize("stages,NB", [(1, 1), (3, 2), (8, 8), (4, 16)])
+def test_both_foldings_in_one_launch(stages, NB):
+    w = torch.randn(stages, 1, NB, 64, 64, device=DEV)
+    want = [ops.bh4_fold_split(w, t) for t in (False, True)]
+    got = [torch.full_like(s, float("nan")) for s in want]
+    assert _lib.load().lffn_bh4_fold_split_both_f32(w.data_ptr(), got[0].data_ptr(), got[1].data_ptr(), stages, NB, 64, _lib.stream_of(w)) == 0
+    assert all(torch.equal(a.view(torch.int32), b.view(torch.int32)) for a, b in zip(got, want))
 
 
 # both forms of the kernel (few and many workgroups), rows around the 16 of a tile, columns short of D, codes short of them
