@@ -651,13 +651,14 @@ extern "C" int lffn_lookup_backward_sums_rows(int64_t B, int64_t *rows) {
 //
 // Fp32 atomics on the output rows run at 79 G/s on this part, one per product: 3.4 ms at 4096 x 128 x 512.  The
 // accumulation above needs the (token, weight) pairs listed row by row instead, which takes one integer atomic per pair:
-//   rows_rank_kernel    a pair's place among the pairs of its row: the value its atomic add on the row's counter returns
+//   rows_rank_kernel    a pair's place among the pairs of its row: the value its atomic add on the row's counter returns, or a
+//                       workgroup's one such add for all its pairs of the row
 //   rows_claim_kernel   one workgroup per 256 rows (a "table" of the accumulation) scans their padded counts and takes that
 //                       much of the list; which table's part comes first does not matter
 //   rows_place_kernel   pairs into the list (and a row's padding, which names the zero row, by its first pair); other workgroups copy
 //                       g slice-major
 // The order inside a row is the order of arrival: sums differ from run to run in their last bit, as they did with
-// atomics.  Measured at 4096 x 128 x 512, 32768 rows: see launch_rows.
+// atomics.
 namespace {
 
 constexpr int VT = 256;                 // rows per "table"
@@ -669,6 +670,7 @@ struct RowsArgs {
     int32_t *count;        // [tables * VT] pairs per row, then (one word) the list's end in units of eight entries
     int32_t *rank;         // [B * I]
     int32_t *off8;         // [tables, VT + 1]
+    int32_t *flags;        // [TABLE_FLAGS] not zero where a row number lies outside its column's table, or null: not looked for
     uint2 *pairs;
     float *g_packed;       // [Dv / SC][B + 1][SC], the last row zero
     int64_t B, n, rows;
@@ -680,13 +682,80 @@ __device__ __forceinline__ int row_of(const RowsArgs &a, int64_t e) {
     return (int)(raw < 0 ? 0 : (raw > hi ? hi : raw));
 }
 
-__global__ __launch_bounds__(256) void rows_zero_kernel(int4 *p, int64_t n4) {
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n4; i += int64_t(gridDim.x) * 256) p[i] = make_int4(0, 0, 0, 0);
+// The counters to zero; with flags, what table_form_kernel (gather.hip) leaves there for these row numbers.
+__global__ __launch_bounds__(1024) void rows_zero_kernel(RowsArgs a, int64_t n4) {
+    __shared__ int s_bad[16];
+    const int64_t first = int64_t(blockIdx.x) * 1024 + threadIdx.x, stride = int64_t(gridDim.x) * 1024;
+    for (int64_t i = first; i < n4; i += stride) reinterpret_cast<int4 *>(a.count)[i] = make_int4(0, 0, 0, 0);
+    if (!a.flags) return;                         // uniform
+    int bad = 0, i = (int)(first % a.I);
+    const int step = (int)(stride % a.I);
+    for (int64_t e = first; e < a.n; e += stride) {
+        bad |= (a.idx[e] >> 8) ^ i;
+        i += step;
+        if (i >= a.I) i -= a.I;
+    }
+    const unsigned long long m = __ballot(bad != 0);
+    if ((threadIdx.x & 63) == 0) s_bad[threadIdx.x >> 6] = m != 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) any |= s_bad[w];
+        a.flags[blockIdx.x] = any;
+    }
 }
 
 __global__ __launch_bounds__(256) void rows_rank_kernel(RowsArgs a) {
     const int64_t stride = int64_t(gridDim.x) * 256;
     for (int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) a.rank[e] = atomicAdd(a.count + row_of(a, e), 1);
+}
+
+// The same for many tokens.  Row numbers as the layer forms them lie in table i in column i: then a workgroup has RANK_TOKENS tokens of
+// RANK_COLS columns, counts them in LDS and takes their places from one add per row.  What bounds it is the adds that return something,
+// 24 G/s: 4096 x 128 pairs, 32768 rows, 22 -> 7 us, 16000 x 64 41 -> 9.5, 2500 x 256 27 -> 8.  For other row numbers an add for every pair, in
+// their order (in the order of the tables' form, sixteen bytes of a token's at a time, 22 -> 25 us, 45 -> 54).  From RANK_TABLES_TOKENS
+// on: at 1024 tokens a row has four pairs in a table, and there is nothing to win.
+constexpr int64_t RANK_TABLES_TOKENS = 2048;
+constexpr int RANK_TOKENS = 1024, RANK_COLS = 4, RANK_WG = 1024;
+__global__ __launch_bounds__(RANK_WG) void rows_rank_tables_kernel(RowsArgs a, int col_groups) {
+    __shared__ int place[RANK_COLS * VT];
+    constexpr int EACH = RANK_TOKENS * RANK_COLS / RANK_WG;
+    if (table_guard_ends(TableGuard{a.flags, 1})) {           // uniform: not in table form
+        const int64_t stride = int64_t(gridDim.x) * RANK_WG;
+        for (int64_t e0 = int64_t(blockIdx.x) * RANK_WG + threadIdx.x; e0 < a.n; e0 += stride * EACH) {
+            int rank[EACH];
+#pragma unroll
+            for (int k = 0; k < EACH; ++k) rank[k] = e0 + k * stride < a.n ? atomicAdd(a.count + row_of(a, e0 + k * stride), 1) : 0;
+#pragma unroll
+            for (int k = 0; k < EACH; ++k)
+                if (e0 + k * stride < a.n) a.rank[e0 + k * stride] = rank[k];
+        }
+        return;
+    }
+    const int c = threadIdx.x % RANK_COLS, col0 = int(blockIdx.x % col_groups) * RANK_COLS, col = col0 + c;
+    const int64_t b0 = int64_t(blockIdx.x / col_groups) * RANK_TOKENS + threadIdx.x / RANK_COLS;
+    int row[EACH], rank[EACH];
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) {
+        const int64_t b = b0 + k * (RANK_WG / RANK_COLS);
+        row[k] = b < a.B && col < a.I ? row_of(a, b * a.I + col) : -1;
+    }
+    static_assert(RANK_COLS * VT == RANK_WG, "a counter per thread");
+    place[threadIdx.x] = 0;
+    __syncthreads();
+    auto in_table = [&](int k) { return row[k] / VT == col; };            // (-1 / VT == 0, but such a thread writes nothing)
+#pragma unroll
+    for (int k = 0; k < EACH; ++k)
+        if (row[k] >= 0) rank[k] = in_table(k) ? atomicAdd(&place[c * VT + row[k] % VT], 1) : atomicAdd(a.count + row[k], 1);
+    __syncthreads();
+    const int n = place[threadIdx.x];             // row threadIdx.x % VT of table col0 + threadIdx.x / VT
+    if (n > 0) place[threadIdx.x] = atomicAdd(a.count + (size_t)col0 * VT + threadIdx.x, n);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < EACH; ++k)
+        if (row[k] >= 0)
+            a.rank[(b0 + k * (RANK_WG / RANK_COLS)) * a.I + col] = rank[k] + (in_table(k) ? place[c * VT + row[k] % VT] : 0);
 }
 
 __global__ __launch_bounds__(VT) void rows_claim_kernel(RowsArgs a) {
@@ -868,7 +937,7 @@ int launch_rows_sum(const RowsArgs &a, float *out, int accumulate, hipStream_t s
 }
 
 struct RowsWorkspace {
-    int64_t count, rank, off8, pairs, g_packed, total;
+    int64_t count, rank, off8, pairs, g_packed, flags, total;
 };
 
 // Worth it from 3e6 products on (five launches, about 30 us of them whatever the size, against 79 G atomics/s; forward and backward at 512
@@ -891,7 +960,8 @@ RowsWorkspace rows_layout(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
     w.pairs = w.off8 + round16(tables * (VT + 1) * 4);
     w.g_packed = w.pairs + (n + 7 * (n < rows ? n : rows)) * 8 + 8;
     w.g_packed = round16(w.g_packed);
-    w.total = w.g_packed + (Bc + 1) * Dv * 4;
+    w.flags = w.g_packed + (Bc + 1) * Dv * 4;               // (a multiple of 128)
+    w.total = w.flags + TABLE_FLAGS * 4;
     return w;
 }
 
@@ -931,9 +1001,17 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         const bool sparse = a.n <= SPARSE_PAIRS * out_size;      // (no slice-major copy of g)
         const int64_t pack_blocks = sparse ? 0 : ((a.B + 1) * (Dv / 4) + 1023) / 1024;
         const int64_t zero4 = l.rank / 16;                      // the counters and the list's end
-        hipLaunchKernelGGL(rows_zero_kernel, dim3((unsigned)((zero4 + 255) / 256 < 1024 ? (zero4 + 255) / 256 : 1024)), dim3(256), 0, st,
-                           reinterpret_cast<int4 *>(base), zero4);
-        hipLaunchKernelGGL(rows_rank_kernel, dim3((unsigned)a.place_blocks), dim3(256), 0, st, a);
+        a.flags = a.B >= RANK_TABLES_TOKENS ? reinterpret_cast<int32_t *>(base + l.flags) : nullptr;
+        const int64_t zero_blocks = (zero4 + 1023) / 1024;
+        hipLaunchKernelGGL(rows_zero_kernel, dim3((unsigned)(a.flags || zero_blocks > TABLE_FLAGS ? TABLE_FLAGS : zero_blocks)), dim3(1024), 0, st, a,
+                           zero4);
+        if (a.flags) {
+            const int col_groups = (int)((I + RANK_COLS - 1) / RANK_COLS);      // (workgroups: fewer than pairs)
+            hipLaunchKernelGGL(rows_rank_tables_kernel, dim3((unsigned)((a.B + RANK_TOKENS - 1) / RANK_TOKENS * col_groups)), dim3(RANK_WG), 0,
+                               st, a, col_groups);
+        } else {
+            hipLaunchKernelGGL(rows_rank_kernel, dim3((unsigned)a.place_blocks), dim3(256), 0, st, a);
+        }
         hipLaunchKernelGGL(rows_claim_kernel, dim3((unsigned)a.tables), dim3(VT), 0, st, a);
         const dim3 grid((unsigned)(a.place_blocks + pack_blocks));
         if (g_format == LFFN_ROWS_F16) hipLaunchKernelGGL(rows_place_kernel<_Float16>, grid, dim3(256), 0, st, a);

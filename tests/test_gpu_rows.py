@@ -209,6 +209,30 @@ def test_block_weight_gradient_over_long_chunks(B):
         assert ((got[s] - torch.bmm(p, u)).abs() <= (B + 4) * 2.0 ** -24 * torch.bmm(p.abs(), u.abs())).all(), s
 
 
+# pairs counted in LDS (row numbers of column i in table i) beside pairs that are not, tokens and columns short of a workgroup's 1024 x 4
+@pytest.mark.parametrize("B,I,in_tables", [(2047, 9, 1.0), (2048, 13, 1.0), (3000, 12, 0.0), (2049, 33, 0.5), (3073, 70, 0.97)])
+def test_row_sums_of_mixed_row_numbers(B, I, in_tables):
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    rows, Dv = I * 256 - 100, 320
+    idx = torch.randint(0, 256, (B, I), generator=gen, device="cuda") + 256 * torch.arange(I, device="cuda")
+    other = torch.randint(-300, rows + 300, (B, I), generator=gen, device="cuda")          # (row numbers are held to the range)
+    idx = torch.where(torch.rand(B, I, generator=gen, device="cuda") < in_tables, idx, other).int()
+    idx[:, 1] = torch.where(torch.arange(B, device="cuda") % 3 == 0, 300, idx[:, 1])      # a row of many pairs
+    w, g = torch.randn(B, I, generator=gen, device="cuda"), torch.randn(B, Dv, generator=gen, device="cuda")
+    size = ctypes.c_int64()
+    assert _lib.load().lffn_scatter_rows_workspace_bytes(B, I, rows, Dv, ctypes.byref(size)) == 0 and size.value > 0
+    ws, out = torch.empty(size.value, dtype=torch.uint8, device="cuda"), torch.full((rows, Dv), float("nan"), device="cuda")
+    assert _lib.load().lffn_scatter_rows(idx.data_ptr(), g.data_ptr(), w.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), B, I, rows, Dv,
+                                         0, 0, _lib.stream_of(g)) == 0
+    at, want, scale = idx.long().clamp(0, rows - 1), torch.zeros(rows, Dv, device="cuda").double(), torch.zeros(rows, Dv, device="cuda").double()
+    for i in range(I):
+        part = w[:, i:i + 1].double() * g.double()
+        want.index_add_(0, at[:, i], part)
+        scale.index_add_(0, at[:, i], part.abs())
+    most = torch.bincount(at.flatten(), minlength=rows)[:, None]
+    assert ((out - want).abs() <= (most + 4) * 2.0 ** -24 * scale).all()
+
+
 @pytest.mark.parametrize("shapes", [[(1, 4)], [(513, 768), (2, 36), (127, 32)], [(2049, 64), (128, 1024), (129, 4), (512, 4096), (3, 8)] + 3 * [(40, 0)]])
 def test_sums_of_many_arrays(shapes):
     """At most 17 numbers to a lane, then 3 + 15 additions: 36 roundings of the magnitudes' sum."""
