@@ -45,23 +45,40 @@ __global__ __launch_bounds__(256) void layer_norm_bwd_kernel(LnBwdArgs a) {
         ab[j] = aw[j];
     }
 
-    for (int64_t row = int64_t(blockIdx.x) * 4 + wave; row < a.B; row += int64_t(gridDim.x) * 4) {
+    // A row's numbers are requested while the row before is reduced (four sums over the wavefront, one after the other), at clamped rows
+    // and columns so that no branch stands in front of them: of the repeats' gradients the first two, the others where they are added.
+    // 32768 x 512, two repeats 65 -> 51 us with the sums' launch, 16384 x 768 36 -> 33, x 1024 44 -> 40 (twice the workgroups: 58, 38, 47).
+    float4 xn[NJ], g0[NJ], g1[NJ];
+    auto fetch = [&](int64_t row) {
+        row = min(row, a.B - 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int64_t at = row * a.H + min(256 * j + 4 * lane, a.H - 4);
+            xn[j] = *reinterpret_cast<const float4 *>(a.x + at);
+            g0[j] = *reinterpret_cast<const float4 *>(a.gy + at);
+            if (a.R > 1) g1[j] = *reinterpret_cast<const float4 *>(a.gy + a.B * a.H + at);      // uniform
+        }
+    };
+    const int64_t stride = int64_t(gridDim.x) * 4;
+    int64_t row = int64_t(blockIdx.x) * 4 + wave;
+    if (row < a.B) fetch(row);
+    for (; row < a.B; row += stride) {
         float4 xv[NJ], g[NJ];
         float s = 0.f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int e = 256 * j + 4 * lane;
-            xv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-            g[j] = xv[j];
-            if (e < a.H) {
-                xv[j] = *reinterpret_cast<const float4 *>(a.x + row * a.H + e);
-                for (int r = 0; r < a.R; ++r) {
-                    const float4 t = *reinterpret_cast<const float4 *>(a.gy + (int64_t(r) * a.B + row) * a.H + e);
-                    g[j].x += t.x; g[j].y += t.y; g[j].z += t.z; g[j].w += t.w;
-                }
+            xv[j] = xn[j];
+            g[j] = g0[j];
+            if (a.R > 1) { g[j].x += g1[j].x; g[j].y += g1[j].y; g[j].z += g1[j].z; g[j].w += g1[j].w; }
+            for (int r = 2; r < a.R; ++r) {
+                const float4 t = *reinterpret_cast<const float4 *>(a.gy + (int64_t(r) * a.B + row) * a.H + min(e, a.H - 4));
+                g[j].x += t.x; g[j].y += t.y; g[j].z += t.z; g[j].w += t.w;
             }
+            if (e >= a.H) xv[j] = g[j] = make_float4(0.f, 0.f, 0.f, 0.f);
             s += (xv[j].x + xv[j].y) + (xv[j].z + xv[j].w);
         }
+        fetch(row + stride);
         const float mean = wave_sum(s) * inv_h;
         float v = 0.f;
 #pragma unroll
@@ -165,7 +182,8 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(SumPartialsArgs a) {
 // Column sums of several arrays in one launch: what a layer's backward leaves for its end.  A workgroup owns 32 columns of one
 // array; eight lanes side by side read 128 contiguous bytes of a row, the 128 lane groups take rows 128 apart, four loads in flight
 // each.  Fixed order: a lane's rows ascending, the eight groups of a wavefront by halves, the wavefronts ascending.
-// One launch in the place of three to six of 3 to 6 us that are nothing but round trips: TIMES
+// One launch in the place of three to six of 3 to 6 us that are nothing but round trips: 6.6 us for the 4096 + 1024 + 3 x 768 columns of a
+// diagonal layer at 16384 tokens, 3.4 for the 512-column layer at 385.
 constexpr int MANY = 8, MANY_WG = 1024, MANY_COLS = 32, MANY_GROUPS = MANY_WG / (MANY_COLS / 4);
 struct SumManyArgs {
     const float *parts[MANY];

@@ -103,7 +103,8 @@ __global__ __launch_bounds__(256) void lookup_prep_kernel(PrepArgs a) {
 constexpr int PACK_TOKENS = 32;      // rows of g per workgroup of the slice-major copy
 
 // PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy); row B is the padding's.  A thread has four
-// columns of every G-th row, so that their sum (the output bias's gradient) is a few additions and a pass over LDS: TIMES
+// columns of every G-th row, so that their sum (the output bias's gradient) is a few additions and a pass over LDS (a
+// launch of its own for them took 14 us at 16384 x 768, this one is no longer for it).
 __device__ __forceinline__ void pack_rows(const PrepArgs &a, int64_t blk) {
     extern __shared__ int sm[];
     float4 *const part = reinterpret_cast<float4 *>(sm);     // [SORT_WG]
