@@ -206,8 +206,9 @@ __device__ __forceinline__ void split4(f32x4 v, uint2 &hi, uint2 &lo) {
 // result: grad x of this repeat = G_0[:, :H] + residual * grad z[:, :H].
 //
 // SCORES_BACKWARD: the same from z and the scores' gradient.  The gradient of z is formed where it is used, at the start and for the
-// residual (a sixteen tokens' rows wait nowhere that is not needed), and its columns' sums, the projection bias's gradient, go out
-// with it: TIMES
+// residual, and its columns' sums, the projection bias's gradient, go out with it.  32768 x 512, two repeats: 263 us where a kernel that
+// formed it took 48, this one 200 and the sums 24.  Written to g_x at the start and read back at the end instead: 288; the scores'
+// derivatives kept by the training form instead of z: 260 to 273, and the forward longer.
 enum Form { HASH, TRAIN, BACKWARD, SCORES_BACKWARD };       // TRAIN: the hash form that also keeps what the backward needs
 
 template <int NB, Form FORM, int BG>
@@ -484,6 +485,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     };
     auto z_gradients = [&](auto take) {
         constexpr int FEW = NBW < 4 ? NBW : 4;
+        // (nontemporal, both times: kept, z would push out what the stages write, 32768 x 512 10 us of the step)
 #pragma unroll 1
         for (int i0 = 0; i0 < NBW; i0 += FEW) {
             f32x4 z[FEW];
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 const int64_t tok = min(tok_base + at[i] / (D / 4), B - 1);
                 const int col = r * D + 4 * (at[i] % (D / 4));
                 const bool in = col < a.T * 8;
-                z[i] = *reinterpret_cast<const f32x4 *>(a.z + tok * (a.T * 8) + (in ? col : 0));
+                z[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(a.z + tok * (a.T * 8) + (in ? col : 0)));
                 g[i] = a.g_score[tok * a.T + (in ? col / 8 : 0)];
                 if (!in || tok_base + at[i] / (D / 4) >= B) g[i] = 0.f, z[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
