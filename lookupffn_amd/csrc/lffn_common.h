@@ -363,7 +363,8 @@ __device__ __forceinline__ float exp_minus_twice(float a) {
 
 // Gradient of a score, s = sum |z| / prod (1 + exp(-2 |z|)), with respect to its z (the closed form of
 // PL/compute_code_score/kernel.py:51-53 differentiated), four columns at a time: away = exp(-2 |z|), and the four's part of
-// sum and product, which the caller combines over the score's fours.
+// sum and product, which the caller combines over the score's fours.  (With expf and sum and product in one chain, as it was in
+// code_score.hip, z of 1: error against 64 bits 1.34e-7; so 1.32e-7.)
 struct ScorePart {
     float away[4], sum, product;
 };
