@@ -897,7 +897,8 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, i
             const float4 old = *dst;
             v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
         }
-        *dst = v;
+        // (rows of no further use here: 64 tokens of 512 tables of 1024 columns, the operator's pass 197 -> 184 us, 500 of 256 244 -> 223)
+        __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(dst));
     };
     for (int col0 = 4 * lane; col0 - 4 * lane < a.Dv; col0 += 256 * NC) {
         for (int r = wave; r < nrows; r += 4) {
