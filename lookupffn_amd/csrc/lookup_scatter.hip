@@ -30,6 +30,8 @@
 
 namespace {
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int WG = 1024;
 constexpr int WAVES = WG / 64;
 constexpr int COLS = 64;           // columns per slice = lanes per token
@@ -244,7 +246,9 @@ __global__ __launch_bounds__(256) void lookup_scatter_list_kernel(ScatterArgs a,
                     const float4 old = *reinterpret_cast<const float4 *>(dst + col[c]);
                     v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
                 }
-                *reinterpret_cast<float4 *>(dst + col[c]) = v;
+                // (of no further use here, and in the caches they take the place of g and of what the rest of the backward reads: training
+                // steps of 500 tokens of 512 tables of 1024 columns 519 -> 474 us, 128 270 -> 248, 1500 of 128 x 768 249 -> 237)
+                __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(dst + col[c]));
             }
         }
     }
