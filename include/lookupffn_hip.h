@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 13
+#define LFFN_ABI_VERSION 14
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -789,7 +789,7 @@ int lffn_lookup_inner_f32(const int32_t *code, const float *g, const float *tabl
  *
  * lffn_bh4_fold_split_f32: the 64-point transform of lffn_bh4_fold_mode_f32 (transposed == 0: mode 0, else
  * mode 1) of stages x num_block blocks, split.  w: [stages, num_block, 64, 64], num_block a power of two up to
- * 16, stages = R * J; w_split: stages * (num_block * 4096 + 64) floats, 16-byte aligned.
+ * 16, stages = R * J; w_split: stages * (num_block * 4160 + 1) floats, 16-byte aligned.
  */
 int lffn_bh4_fold_split_f32(const float *w, float *w_split, int64_t stages, int64_t num_block, int64_t block_size,
                             int32_t transposed, void *stream);

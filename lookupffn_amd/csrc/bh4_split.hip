@@ -44,23 +44,37 @@ constexpr int BS = 64;          // block size this file is built for
 constexpr int PAD = 4;          // floats of padding per row of the fp32 tile
 constexpr float TOP = 16384.f;  // what the largest of a row is scaled to at least (and less than twice that)
 
-// Largest over the wavefront.
-__device__ __forceinline__ float wave_most(float v) {
-    v = fmaxf(v, lane_xor<1>(v));
-    v = fmaxf(v, lane_xor<2>(v));
-    v = fmaxf(v, lane_xor<4>(v));
-    v = fmaxf(v, lane_xor<8>(v));
-    return rows_most(v);
+// Largest and smallest over the wavefront.
+__device__ __forceinline__ void wave_range(float v, float &most, float &least) {
+    most = least = v;
+    auto step = [&](float m, float l) { most = fmaxf(most, m), least = fminf(least, l); };
+    step(lane_xor<1>(most), lane_xor<1>(least));
+    step(lane_xor<2>(most), lane_xor<2>(least));
+    step(lane_xor<4>(most), lane_xor<4>(least));
+    step(lane_xor<8>(most), lane_xor<8>(least));
+    step(lane_xor<16>(most), lane_xor<16>(least));
+    step(lane_xor<32>(most), lane_xor<32>(least));
 }
 
-// The 64-point transform of every block (bh4_block.hip: bh4_fold_kernel), split, ready for the product kernel.  One workgroup per stage, a wavefront per
-// block: an output (transposed: input) column is scaled by a power of two, the same in every block (the butterflies add the blocks'
-// columns), its largest in the stage (transposed), or that of sixteen columns, to [2^14, 2^15), so that lo needs no factor.  Per block
-// and product wavefront four fragments of 64 lanes x 8 numbers: hi of the first and the second eight columns of a lane's sixteen, then lo
-// of them; behind all blocks the inverse scales, [stage][64].
+// The 64-point transform of every block (bh4_block.hip: bh4_fold_kernel), split, ready for the product kernel.  One workgroup per
+// stage, a wavefront per block.  The weights are scaled by a power of two, so that lo needs no factor.  The 64 numbers of an input
+// column of a block are fp32 sums of the same 64, so what the split leaves of a small one of them is as good as it was; but a
+// column's size is that of the weights, and a small column meets a large input (forward) or gives a small gradient (backward).  So:
+//   columns that all lie within SPAN of the stage's largest number are scaled together, that number to [2^14, 2^15); a column still has
+//     22 bits down to 2^-9 of its own largest, and is held to 2^-31 of that below;
+//   else every column of every block by itself, its largest to [2^14, 2^15), and the product kernel multiplies by the way back: the
+//     forward its rows, before it takes their largest, the backward what it has formed.
+// At 32768 tokens, D = 512, two repeats the second costs 8, 13 and 5 us of hash, training form and backward, the choice between them 0, 5
+// and 0.  With one scale for a stage's column (sixteen of the forward's) in all blocks, as it was, the relative error was 4e-5 where columns
+// are spread over 1e8 and their inputs the other way round, and 4e-4 in the gradient of a small block; so it is 1.2e-7 and 1.9e-7, as it is
+// for numbers of one size (fp32 kernel 1.7e-7 and 2.8e-7).
+// Per block and product wavefront four fragments of 64 lanes x 8 numbers: hi of the first and the second eight columns of a lane's
+// sixteen, then lo of them; behind all blocks the way back of every column over 2^14, [stage][64 * num_block], 0 for a column of zeros
+// (its input must not set its row's scale), and [stage] the one of the stage's scale or 0.
+constexpr float SPAN = 1.f / 256;
 template <bool TRANSPOSED>
-__device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float *inverse) {
-    __shared__ float most_s[16][BS], scale_s[BS];
+__device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float *back, float *together) {
+    __shared__ float range_s[2][16];
     const int num_block = blockDim.x / 64, wave = threadIdx.x >> 6;
     const int64_t blk = int64_t(blockIdx.x) * num_block + wave;
     const int i = threadIdx.x & 63;
@@ -79,32 +93,19 @@ __device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float 
             }
         }
     }
-    if constexpr (!TRANSPOSED) {
-        // sixteen output columns by one scale: they are fp32 sums of the same 64 numbers, rounded to 2^-24 of the largest of those in any
-        // case (a scale for each, D = 1024: 9.2 -> 17.2 us a call)
+    float most = 0.f;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            float most = 0.f;
-#pragma unroll
-            for (int o = 16 * g; o < 16 * g + 16; ++o) most = fmaxf(most, fabsf(v[o]));
-            most = wave_most(most);
-            if (i / 16 == g) most_s[wave][i] = most;
-        }
-    } else {
-        float most = 0.f;
-#pragma unroll
-        for (int o = 0; o < BS; ++o) most = fmaxf(most, fabsf(v[o]));
-        most_s[wave][i] = most;
-    }
+    for (int o = 0; o < BS; ++o) most = fmaxf(most, fabsf(v[o]));
+    float largest, least;
+    wave_range(most, largest, least);
+    range_s[0][wave] = largest, range_s[1][wave] = least;
     __syncthreads();
-    if (wave == 0) {
-        float most = 0.f;
-        for (int n = 0; n < num_block; ++n) most = fmaxf(most, most_s[n][i]);
-        const PowerOfTwo p = scale_to_one(most);
-        scale_s[i] = p.scale * TOP;
-        inverse[blockIdx.x * BS + i] = p.inverse * (1 / TOP);
-    }
-    __syncthreads();
+    for (int n = 0; n < num_block; ++n) largest = fmaxf(largest, range_s[0][n]), least = fminf(least, range_s[1][n]);
+    const bool one = least >= largest * SPAN;                 // uniform
+    const PowerOfTwo p = scale_to_one(one ? largest : most);
+    const float f = p.scale * TOP;
+    back[blk * BS + i] = most > 0.f ? p.inverse * (1 / TOP) : 0.f;
+    if (threadIdx.x == 0) together[blockIdx.x] = one ? p.inverse * (1 / TOP) : 0.f;
     // eight consecutive k of a row of the A operand as hi and lo: fragment (row / 16, (k % 16) / 8), lane 16 (k / 16) + row % 16
     uint4 *const dst = reinterpret_cast<uint4 *>(out + blk * (BS * BS));
     auto store8 = [&](int row, int k, const float (&x)[8]) {
@@ -119,7 +120,6 @@ __device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float 
         dst[at + 128] = make_uint4(l[0], l[1], l[2], l[3]);
     };
     if constexpr (TRANSPOSED) {
-        const float f = scale_s[i];
 #pragma unroll
         for (int k = 0; k < BS; k += 8) {
             float x[8];
@@ -134,7 +134,7 @@ __device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float 
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
 #pragma unroll
-            for (int o = 0; o < 16; ++o) t[o * 65 + i] = v[16 * g + o] * scale_s[16 * g + o];
+            for (int o = 0; o < 16; ++o) t[o * 65 + i] = v[16 * g + o] * f;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
@@ -151,8 +151,8 @@ __device__ __forceinline__ void fold_split(const float *w, uint32_t *out, float 
 
 // One of the two forms, or both (gridDim.y 2: a training step's, in one launch)
 __global__ __launch_bounds__(1024) void bh4_fold_split_kernel(const float *w, float *out, float *out_t, int64_t numbers) {
-    if (blockIdx.y == 0 && out) fold_split<false>(w, reinterpret_cast<uint32_t *>(out), out + numbers);
-    else fold_split<true>(w, reinterpret_cast<uint32_t *>(out_t), out_t + numbers);
+    if (blockIdx.y == 0 && out) fold_split<false>(w, reinterpret_cast<uint32_t *>(out), out + numbers, out + numbers + numbers / BS);
+    else fold_split<true>(w, reinterpret_cast<uint32_t *>(out_t), out_t + numbers, out_t + numbers + numbers / BS);
 }
 
 struct SplitArgs {
@@ -161,7 +161,7 @@ struct SplitArgs {
     const float *ln_b;     // [H]
     float ln_eps;
     const float *w;        // split weights
-    const float *wscale;   // their inverse scales [R*J][64]
+    const float *wback;    // [R*J][D] the way back of their columns, [R*J] of a stage's together
     const float *pbias;    // [T*8] or null
     int32_t *codes;        // [B, T]
     float *scores;         // [B, T]
@@ -291,19 +291,31 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         *reinterpret_cast<uint2 *>(p + 2 * D) = lo;
     };
 
-    // What the accumulators are to be multiplied with: the inverse scales of the lane's four columns of the weights and of its token.
-    f32x4 inv_w = {1.f, 1.f, 1.f, 1.f};
+    // What the accumulators are to be multiplied with: the weights' part, and the way back of the lane's token.
+    constexpr float INV_W = BWD ? 1.f : 1 / TOP;
     float inv_x = 1.f;
+    // the way back of a stage's weights, over 2^14: of all together, or 0 and of columns col .. + 3
+    // (no store of this kernel meets the weights: a scalar load)
+    const auto *const each = (const __attribute__((address_space(4))) float *)(uintptr_t)(a.wback + size_t(a.R) * J * D + r * J);
+    auto together_of = [&](int s) { return each[s]; };
+    float together = together_of(BWD ? J - 1 : 0);            // of the stage whose product is next
+    auto back_of = [&](int s, int col) { return *reinterpret_cast<const f32x4 *>(a.wback + size_t(r * J + s) * D + col); };
+    // v[i] times the way back of four columns (a few at a time: registers), over 2^14 times f
+    auto go_back = [&](int s, auto &v, auto col, float f) {
+        constexpr int N = sizeof(v) / sizeof(v[0]);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            v[i] = v[i] * (back_of(s, col(i)) * f);
+            if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto own_col = [&](int n) { return (n * BG + bg) * BS + 16 * ow + 4 * kq; };       // of the lane's accumulator n
 
     // acc = (blocks of the stage's weights) x (the tile's tokens)
     auto product = [&](int s) {
-        const float *const scales = a.wscale + (r * J + s) * BS + 16 * ow;         // uniform: scalar loads, chosen from by lane
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if constexpr (BWD) inv_w[e] = kq < 2 ? (kq == 0 ? scales[e] : scales[4 + e]) : (kq == 2 ? scales[8 + e] : scales[12 + e]);
-            else inv_w[e] = scales[0];         // (the forward's sixteen columns have one)
-        }
-        inv_x = unscale[c];
+        const float own = together;
+        inv_x = own != 0.f ? unscale[c] * (own * (BWD ? 1.f : TOP)) : unscale[c];
+        together = together_of(BWD ? max(s - 1, 0) : min(s + 1, J - 1));
         uint4 xv[2][4];
         read_x(0, xv[0]);
         static_for<NBW>([&](auto n_c) {
@@ -322,6 +334,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             __builtin_amdgcn_sched_barrier(0);
         });
         load_w(s, NBW - 1 + AHEAD);
+        if (BWD && own == 0.f) go_back(s, acc, own_col, 1.f);                   // uniform
     };
 
     // H_NB across the blocks of the accumulators, from stride NB / 2 down (wide form: down to BG)
@@ -344,23 +357,24 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     constexpr int ROW_LANES = D < 256 ? D / 4 : 64, ROW_VALUES = D < 256 ? 1 : D / 256;
     auto row_of = [&](int i) { return 4 * wave + (D < 256 ? i * (64 / ROW_LANES) + lane / ROW_LANES : i / ROW_VALUES); };
     auto col_of = [&](int i) { return 4 * (lane % ROW_LANES) + (D < 256 ? 0 : 256 * (i % ROW_VALUES)); };
-    auto to_rows = [&](f32x4 f) {
+    auto to_rows = [&](float f) {
 #pragma unroll
         for (int n = 0; n < NBW; ++n)
-            *reinterpret_cast<f32x4 *>(rows32 + c * LDR + (n * BG + bg) * BS + 16 * ow + 4 * kq) = acc[n] * f;
+            *reinterpret_cast<f32x4 *>(rows32 + c * LDR + own_col(n)) = acc[n] * f;
     };
     auto from_rows = [&](f32x4 (&v)[NB]) {
 #pragma unroll
         for (int i = 0; i < NB; ++i) v[i] = *reinterpret_cast<const f32x4 *>(rows32 + row_of(i) * LDR + col_of(i));
     };
 
-    // The accumulators (after butterflies()) become the next product's tile, and the rows of D floats at `save` where they are kept:
-    // a token's row is scaled by the power of two that takes its largest to [2^14, 2^15).
-    auto hand_over = [&](float *save) {
+    // The accumulators (after butterflies()) become the tile of the product of stage s, and the rows of D floats at `save` where they are
+    // kept: a token's row, forward times the way back of the columns that it meets where those are not scaled together, is scaled by the power of two that takes its largest
+    // to [2^14, 2^15).
+    auto hand_over = [&](int s, float *save) {
         if constexpr (BG > 1) {
             // strides 2 and 1, which take four wavefronts' accumulators: a pass over the tile in fp32, 16 bytes of blocks
             // 4 n .. 4 n + 3 per thread; the 16 NBW threads of a row are neighbours in a wavefront
-            to_rows(inv_w);
+            to_rows(INV_W);
             if (bg == 0 && ow == 0 && kq == 0) unscale[c] = inv_x;
             __syncthreads();
             if (tid < TOK * 16 * NBW) {
@@ -372,6 +386,13 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const f32x4 *>(p + k * BS);
                 const f32x4 s0 = v[0] + v[2], s1 = v[1] + v[3], d0 = v[0] - v[2], d1 = v[1] - v[3];
                 v[0] = s0 + s1; v[1] = s0 - s1; v[2] = d0 + d1; v[3] = d0 - d1;
+                const bool live = SAVE && tok_base + row < B;
+                if (live) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        __builtin_nontemporal_store(v[k] * inv, reinterpret_cast<f32x4 *>(save + size_t(row) * D + (n * BG + k) * BS + c4));
+                }
+                if (!BWD && together == 0.f) go_back(s, v, [&](int k) { return (n * BG + k) * BS + c4; }, TOP);
                 float most = 0.f;
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
@@ -383,27 +404,30 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 most = fmaxf(most, lane_xor<8>(most));
                 if constexpr (NBW > 1) most = fmaxf(most, lane_xor<16>(most));
                 if constexpr (NBW > 2) most = fmaxf(most, lane_xor<32>(most));
-                const PowerOfTwo s = scale_to_one(most);
-                if (tid % (16 * NBW) == 0) unscale[row] = inv * (s.inverse * (1 / TOP));
-                const bool live = SAVE && tok_base + row < B;
+                const PowerOfTwo p2 = scale_to_one(most);
+                if (tid % (16 * NBW) == 0) unscale[row] = inv * (p2.inverse * (1 / TOP));
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    put(row, (n * BG + k) * BS + c4, v[k] * (s.scale * TOP));
-                    if (live) __builtin_nontemporal_store(v[k] * inv, reinterpret_cast<f32x4 *>(save + size_t(row) * D + (n * BG + k) * BS + c4));
-                }
+                for (int k = 0; k < 4; ++k) put(row, (n * BG + k) * BS + c4, v[k] * (p2.scale * TOP));
             }
             __syncthreads();
         } else if constexpr (SAVE) {
             // the rows go out as whole lines: through LDS in fp32, and a wavefront has four rows from there
             __syncthreads();                      // every wavefront has read this stage's input
-            to_rows(inv_w);
+            to_rows(INV_W);
             if (ow == 0 && kq == 0) unscale[c] = inv_x;
             __syncthreads();
             f32x4 v[NB];
             from_rows(v);
 #pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const int row = row_of(i);
+                if (tok_base + row < B) __builtin_nontemporal_store(v[i] * unscale[row], reinterpret_cast<f32x4 *>(save + size_t(row) * D + col_of(i)));
+            }
+            if (!BWD && together == 0.f) go_back(s, v, col_of, TOP);
+#pragma unroll
             for (int i = 0; i < NB; i += ROW_VALUES) {
                 const int row = row_of(i);
+                const float inv = unscale[row];
                 float most = 0.f;
 #pragma unroll
                 for (int k = i; k < i + ROW_VALUES; ++k)
@@ -415,33 +439,28 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                 most = fmaxf(most, lane_xor<8>(most));
                 if constexpr (ROW_LANES == 32) most = fmaxf(most, lane_xor<16>(most));
                 if constexpr (ROW_LANES == 64) most = rows_most(most);
-                const PowerOfTwo s = scale_to_one(most);
-                const float inv = unscale[row];
-                const bool live = tok_base + row < B;
+                const PowerOfTwo p2 = scale_to_one(most);
 #pragma unroll
-                for (int k = i; k < i + ROW_VALUES; ++k) {
-                    if (live) __builtin_nontemporal_store(v[k] * inv, reinterpret_cast<f32x4 *>(save + size_t(row) * D + col_of(k)));
-                    put(row, col_of(k), v[k] * (s.scale * TOP));
-                }
-                if (lane % ROW_LANES == 0) unscale[row] = inv * (s.inverse * (1 / TOP));
+                for (int k = i; k < i + ROW_VALUES; ++k) put(row, col_of(k), v[k] * (p2.scale * TOP));
+                if (lane % ROW_LANES == 0) unscale[row] = inv * (p2.inverse * (1 / TOP));
             }
             __syncthreads();
         } else {
+            if (together == 0.f) go_back(s, acc, own_col, TOP);
             f32x4 m4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int n = 0; n < NBW; ++n)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) m4[e] = fmaxf(m4[e], fabsf(acc[n][e]));
-            m4 = m4 * inv_w;
+            m4 = m4 * INV_W;
             const float most = rows_most(fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w)));
             if (kq == 0) most_s[c * 4 + ow] = most;
             __syncthreads();                      // every wavefront has read this stage's input and left its largest
             const float4 m = *reinterpret_cast<const float4 *>(most_s + c * 4);
-            const PowerOfTwo s = scale_to_one(fmaxf(fmaxf(m.x, m.y), fmaxf(m.z, m.w)));
-            if (kq == 0 && ow == 0) unscale[c] = inv_x * (s.inverse * (1 / TOP));
-            const f32x4 scale = inv_w * (s.scale * TOP);
+            const PowerOfTwo p2 = scale_to_one(fmaxf(fmaxf(m.x, m.y), fmaxf(m.z, m.w)));
+            if (kq == 0 && ow == 0) unscale[c] = inv_x * (p2.inverse * (1 / TOP));
 #pragma unroll
-            for (int n = 0; n < NBW; ++n) put(c, n * BS + 16 * ow + 4 * kq, acc[n] * scale);
+            for (int n = 0; n < NBW; ++n) put(c, own_col(n), acc[n] * (INV_W * TOP * p2.scale));
             __syncthreads();
         }
     };
@@ -541,7 +560,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
 #pragma unroll 1
         for (int s = J - 1; s >= 0; --s) {
             butterflies();
-            hand_over(a.stage_save + ((size_t(r) * J + s) * B + tok_base) * D);
+            hand_over(s, a.stage_save + ((size_t(r) * J + s) * B + tok_base) * D);
             product(s);
         }
     } else {
@@ -606,6 +625,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                     if (SAVE && r == 0 && tok < B) *reinterpret_cast<float2 *>(a.row_stats + 2 * tok) = make_float2(mean, rstd);
                 }
             }
+            if (together == 0.f) go_back(0, v, column, TOP);
             float most = 0.f;
 #pragma unroll
             for (int i = 0; i < NQ; ++i)
@@ -629,7 +649,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         for (int s = 0; s < J; ++s) {
             product(s);
             butterflies();
-            if (s + 1 < J) hand_over(SAVE ? a.stage_save + ((size_t(r) * (J - 1) + s) * B + tok_base) * D : nullptr);
+            if (s + 1 < J) hand_over(s + 1, SAVE ? a.stage_save + ((size_t(r) * (J - 1) + s) * B + tok_base) * D : nullptr);
         }
         last_strides();
     }
@@ -639,7 +659,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         const int ncols = a.T * 8;
         if constexpr (SCORES) {                   // whole rows again
             __syncthreads();
-            to_rows(inv_w * inv_x);
+            to_rows(inv_x);
             __syncthreads();
             z_gradients([&](int row, int col, f32x4 g) {
                 f32x4 v = *reinterpret_cast<const f32x4 *>(rows32 + row * LDR + col);
@@ -648,7 +668,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             });
         } else if constexpr (BG == 1) {
             __syncthreads();
-            to_rows(inv_w * inv_x);
+            to_rows(inv_x);
             __syncthreads();
             f32x4 v[NB];
             from_rows(v);
@@ -666,7 +686,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             for (int n = 0; n < NBW; ++n) {
                 const int xc = (n * BG + bg) * BS + 16 * ow + 4 * kq;
                 if (xc < H) {
-                    f32x4 o = acc[n] * (inv_w * inv_x);
+                    f32x4 o = acc[n] * inv_x;
                     if (r * D + xc < ncols) o = o + a.residual * *reinterpret_cast<const f32x4 *>(a.gz + token * ncols + r * D + xc);
                     *reinterpret_cast<f32x4 *>(a.g_x + (size_t(r) * B + token) * H + xc) = o;
                 }
@@ -696,7 +716,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             // (without LayerNorm or bias: 0, 1, 1, 0 and 0; the weight is zero beyond column H)
             const f32x4 xv = (xin[n] - mean) * rstd * *reinterpret_cast<const f32x4 *>(lnw_s + xc) +
                              *reinterpret_cast<const f32x4 *>(lnb_s + xc);
-            const f32x4 z = a.decay * (inv_w * inv_x) * acc[n] + a.residual * xv +      // (decay times a power of two: as decay * y)
+            const f32x4 z = a.decay * (INV_W * inv_x) * acc[n] + a.residual * xv +      // (decay times a power of two: as decay * y)
                             *reinterpret_cast<const f32x4 *>(pbias_s + xc);
             if (SAVE && BG > 1 && token < B && r * D + xc < ncols)
                 __builtin_nontemporal_store(z, reinterpret_cast<f32x4 *>(a.z + token * ncols + r * D + xc));
@@ -705,7 +725,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
         if constexpr (SAVE && BG == 1) {          // z as whole rows
 #pragma unroll
             for (int n = 0; n < NBW; ++n) acc[n] = form_z(n);
-            to_rows((f32x4){1.f, 1.f, 1.f, 1.f});
+            to_rows(1.f);
             __syncthreads();
             f32x4 v[NB];
             from_rows(v);
@@ -881,7 +901,7 @@ int front_args(const lffn_block_front *f, const float *x, int64_t B, SplitArgs &
     LFFN_REQUIRE(lffn_aligned16(x) && lffn_aligned16(f->w_split) && lffn_aligned16(f->proj_bias) && lffn_aligned16(f->ln_weight) &&
                      lffn_aligned16(f->ln_bias), LFFN_ERR_BAD_ARG);
     a.x = x; a.ln_w = f->ln_weight; a.ln_b = f->ln_bias; a.ln_eps = f->ln_eps; a.w = f->w_split;
-    a.wscale = f->w_split + R * J * D * BS; a.pbias = f->proj_bias; a.codes = f->codes; a.scores = f->scores;
+    a.wback = f->w_split + R * J * D * BS; a.pbias = f->proj_bias; a.codes = f->codes; a.scores = f->scores;
     a.records = f->records; a.rec_stride = f->record_stride; a.rec_tile = f->tokens_per_workgroup;
     a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = f->decay; a.residual = f->residual;
     return LFFN_OK;
@@ -919,7 +939,7 @@ int back_args(const float *w_split_t, float *g_x, float *stage_grads, int64_t B,
     if (B == 0) return LFFN_OK;
     LFFN_REQUIRE(w_split_t && g_x && stage_grads, LFFN_ERR_BAD_ARG);
     LFFN_REQUIRE(lffn_aligned16(w_split_t) && lffn_aligned16(g_x) && lffn_aligned16(stage_grads), LFFN_ERR_BAD_ARG);
-    a.w = w_split_t; a.wscale = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_save = stage_grads;
+    a.w = w_split_t; a.wback = w_split_t + R * J * D * BS; a.g_x = g_x; a.stage_save = stage_grads;
     a.B = B; a.H = (int)H; a.R = (int)R; a.J = (int)J; a.T = (int)T; a.decay = decay; a.residual = residual;
     return LFFN_OK;
 }

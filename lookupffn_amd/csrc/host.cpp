@@ -220,7 +220,7 @@ void gather(const Config &c, const Tensor &codes, const Tensor &scores, const Te
 using Params = std::array<Tensor, 6>;
 
 // Floats of the split weights (lffn_bh4_fold_split_f32).
-int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 64 + 64); }
+int64_t split_words(const Config &c) { return c.R * c.J * (c.D * 65 + 1); }
 
 // The front end of 64 x 64 blocks; split: their weights (lffn_bh4_fold_split_f32).  The kernel is the training forward's, so that a layer
 // computes the same codes with gradients recorded and without (a checkpointed pass runs both).

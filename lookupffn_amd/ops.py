@@ -406,7 +406,7 @@ _L.define("bh4_fold_split(Tensor w, bool transposed) -> Tensor")
 def split_words(w_shape):
     """Words of the split form of weights [R, J, D/64, 64, 64]."""
     R, J, NB, _, _ = w_shape
-    return R * J * (NB * 4096 + 64)
+    return R * J * (NB * (4096 + 64) + 1)
 
 
 def _bh4_fold_split_impl(w: torch.Tensor, transposed: bool) -> torch.Tensor:

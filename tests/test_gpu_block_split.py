@@ -191,8 +191,7 @@ def test_scales_and_rows_of_their_own(B):
     assert not got[11].any() and not got[12].any()                  # NaN is not above zero
 
 
-# one stage of the backward, few and many workgroups: columns of the weights of very different sizes side by side, each by its own scale.
-# (The forward's columns are sums of 64 of them, rounded in fp32 to 2^-24 of the largest before they are split.)
+# one stage of the backward, few and many workgroups: columns of the weights of very different sizes side by side, each by its own scale
 @pytest.mark.parametrize("B,D", [(40, 64), (33, 256), (9000, 256), (70, 512), (50, 1024)])
 def test_columns_of_many_sizes(B, D):
     gen = torch.Generator(device=DEV).manual_seed(B + D)
@@ -203,3 +202,59 @@ def test_columns_of_many_sizes(B, D):
     want = _blocks(w[0, 0].double().cpu().transpose(-1, -2), g[some].double().cpu() @ _hadamard(D))
     error, size = (t.view(len(some), D // 64, 64).norm(dim=(0, 1)) for t in (got - want, want))
     assert (error / size).max() <= REL
+
+
+# the same with blocks of different sizes, whose columns have nothing to do with each other
+@pytest.mark.parametrize("B,D", [(33, 128), (33, 256), (9000, 256), (70, 512), (50, 1024), (4100, 1024)])
+def test_blocks_of_many_sizes(B, D):
+    gen = torch.Generator(device=DEV).manual_seed(B + D)
+    sizes = (10.0 ** -(torch.arange(64, device=DEV) * 5 % 13)).view(1, 1, 64) * (10.0 ** -(torch.arange(D // 64, device=DEV) * 5 % 9)).view(-1, 1, 1)
+    g, w = _randn(gen, B, D), _randn(gen, 1, 1, D // 64, 64, 64) / 64 * sizes
+    some = list(range(min(B, 40)))
+    got = ops.bh4_block_bwd_split(g, ops.bh4_fold_split(w, True), 1, 1, D, D, 1.0, 0.0)[0][0][some].double().cpu()
+    want = _blocks(w[0, 0].double().cpu().transpose(-1, -2), g[some].double().cpu() @ _hadamard(D))
+    assert ((got - want).norm(dim=0) / want.norm(dim=0)).max() <= REL
+
+
+# Two stages of the forward, few and many workgroups, where the size of a result comes from a small column of the weights and a large
+# input as much as from a large column and a small input ("few": within what is scaled together); nor do inputs count that nothing is
+# multiplied with.  The error is what it is on numbers of one size, and no larger than that of the kernel with fp32 products (beside
+# "zeros", where a third of that one's additions are of zeros and round nothing, while a product is split as ever).
+@pytest.mark.parametrize("B,D", [(40, 64), (33, 128), (33, 256), (9000, 256), (70, 512), (2300, 512), (50, 1024), (4100, 1024)])
+@pytest.mark.parametrize("kind", ["few", "columns", "blocks", "norm", "zeros"])
+def test_columns_against_their_inputs(B, D, kind):
+    gen = torch.Generator(device=DEV).manual_seed(B + D)
+    J, NB, T = 2, D // 64, D // 8
+    x, w = _randn(gen, B, D), _randn(gen, 1, J, NB, 64, 64) / math.sqrt(64 * D)
+    lw = lb = None
+    decades = 1.5 if kind == "few" else 12
+    spread = lambda *shape: 10.0 ** (decades * torch.rand(*shape, generator=gen, device=DEV) - decades / 2)
+    w[0, 1] *= spread(NB, 1, 64)                                    # (the second stage's meet numbers of one size)
+    if kind == "zeros":
+        w[0, 0, :, :, ::3] = 0
+        x[:, ::3] *= 1e12
+    else:
+        e = spread(NB, 1, 1 if kind == "blocks" else 64).expand(NB, 1, 64)
+        w[0, 0] *= e
+        if kind == "norm":
+            lw, lb = (1 + 0.1 * _randn(gen, D)) / e.reshape(D), 0.1 * _randn(gen, D) / e.reshape(D)
+        else:
+            x /= e.reshape(D)
+    some = list(range(min(B, 40))) + [B - 1]
+    u = x[some].double().cpu()
+    if lw is not None:
+        u = torch.nn.functional.layer_norm(u, (D,), lw.double().cpu(), lb.double().cpu(), 1e-5)
+    first = _blocks(w[0, 0].double().cpu(), u) @ _hadamard(D)
+    want = _blocks(w[0, 1].double().cpu(), first) @ _hadamard(D)
+    _, _, z, stages, _ = ops.bh4_block_front_train(x, lw, lb, 1e-5, ops.bh4_fold_split(w, False), 1, J, D, None, T, 1.0, 0.0)
+    folded = ops.bh4_fold_mode(w, 0)
+    plain = (ops.bh4_block_hash_train(x, folded, None, T, 1.0, 0.0) if lw is None else
+             ops.ln_bh4_block_hash_train(x, lw, lb, 1e-5, folded, None, T, 1.0, 0.0))
+    limit = lambda t, want: REL if kind == "zeros" else min(REL, _rel(t, want))
+    assert _rel(stages[0, 0][some], first) <= limit(plain[3][0, 0][some], first)
+    assert _rel(z[some], want) <= limit(plain[2][some], want)
+    # without gradients the same codes, whichever form of the kernel and whatever the neighbours
+    few = min(B, 20)
+    codes, scores = ops.bh4_block_front(x[:few], lw, lb, 1e-5, ops.bh4_fold_split(w, False), 1, J, D, None, T, 1.0, 0.0)
+    got = ops.bh4_block_front_train(x, lw, lb, 1e-5, ops.bh4_fold_split(w, False), 1, J, D, None, T, 1.0, 0.0)
+    assert torch.equal(codes, got[0][:few]) and torch.equal(scores, got[1][:few])
