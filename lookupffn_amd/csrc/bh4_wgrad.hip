@@ -49,9 +49,17 @@ constexpr int DEPTH = 4;          // token quads a step: their loads are in flig
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
+// Tokens that a wavefront adds up from zero: a sum's rounding grows with its length.  Relative error against 64 bits and us, a chunk's sum
+// in one | in runs of 64 tokens:
+//   32768 tokens, D = 512, two repeats (chunks of 2048) 4.15e-7 | 1.77e-7, 214 | 224; 16384, D = 1024 (2048) 4.1e-7 | 1.7e-7, 103 | 104
+//   16384, D = 512 (1024) 3.0e-7 | 1.7e-7, 54 | 54; 4096, D = 512 (512) 2.14e-7 | 1.62e-7, 17.8 | 18.2
+// The first step of a run begun from zero in the instruction, four steps a turn: 42 spilled registers, 256 us.
+constexpr int RUN = 64;
+static_assert(RUN % (8 * DEPTH) == 0);
+
 constexpr int ONCE = 2;           // a load's cache policy: nontemporal, read once
 
-// What bounds it: memory (32768 tokens, D = 512, two repeats: 1.07 GB in 199 us, 5.4 TB/s; the products are 112 of it by themselves).  Loads
+// What bounds it: memory (32768 tokens, D = 512, two repeats: 1.07 GB in 208 us, 5.1 TB/s; the products are 112 of it by themselves).  Loads
 // that were branched around for a chunk's end waited for each other, four round trips a step: 277 us and 131 at 16384, D = 1024 instead
 // of 199 and 91, 23 -> 16 at 4096, 10 -> 8.4 at 1000.  The nontemporal loads matter most behind the backward, whose stores they would push
 // out of the memory-side cache line by line: both kernels in turn 473 -> 390 and 230 -> 186 us.
@@ -89,11 +97,20 @@ __global__ __launch_bounds__(256, 2) void bh4_wgrad_kernel(const float *stage_gr
     const auto sr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(ln ? row_stats + 2 * first : p), 0, ln ? live * 8 : 0, 0x00020000);
     const int p_at = (kq * D + 4 * c) * 4, u_at = u_live ? (kq * Hu + 4 * c) * 4 : 0x40000000;
 
-    f32x4 acc[4][4];                               // [o tile][i tile]
+    f32x4 acc[4][4], total[4][4];                  // [o tile][i tile]
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < 4; ++b) acc[a][b] = total[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto end_run = [&]() {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                total[a][b] += acc[a][b];
+                acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
+    };
 
     struct Step {
         u32x4 p[DEPTH], u[DEPTH];
@@ -148,7 +165,9 @@ __global__ __launch_bounds__(256, 2) void bh4_wgrad_kernel(const float *stage_gr
         for (int t = 0; t < live; t += 8 * DEPTH) {
             step(t, v0, v1);
             if (t + 4 * DEPTH < live) step(t + 4 * DEPTH, v1, v0);
+            if (t % RUN == RUN - 8 * DEPTH) end_run();
         }
+        end_run();
     };
     if (ln) run(std::true_type{});
     else run(std::false_type{});
@@ -164,7 +183,7 @@ __global__ __launch_bounds__(256, 2) void bh4_wgrad_kernel(const float *stage_gr
         for (int b = 0; b < 4; ++b)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                red[wave][((4 * kq + r) * 16 + c) * 4 + b] = acc[a][b][r];       // [o' = 4kq+r][c][b]
+                red[wave][((4 * kq + r) * 16 + c) * 4 + b] = total[a][b][r];       // [o' = 4kq+r][c][b]
         __syncthreads();
         // 16 rows o' x 64 columns of this quarter: thread t adds element t, t+256, ...
         for (int e = threadIdx.x; e < BS * BS / 4; e += 256) {
