@@ -573,12 +573,12 @@ bool configure(const Parts &parts, const Params &p, const at::Device &dev, Confi
     return true;
 }
 
-// hash._folded = ((version, address, device), folded weights, what they were folded from, stream, event, split weights), as Hashing keeps
-// them: the split weights if they are w's and of this stream, on which they come before whatever is launched now.
+// hash._folded = ((version, address, device), split weights, what they were folded from, stream, event), as Hashing keeps them for 8-bit
+// codes: the split weights if they are w's and of this stream, on which they come before whatever is launched now.
 Tensor split_of(PyObject *hash, const Tensor &w, int64_t words) {
     PyObject *kept = item(dict_of(hash), KEY_FOLDED);
-    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 6) return {};
-    PyObject *key = PyTuple_GET_ITEM(kept, 0), *split = PyTuple_GET_ITEM(kept, 5);
+    if (!kept || !PyTuple_Check(kept) || PyTuple_GET_SIZE(kept) != 5) return {};
+    PyObject *key = PyTuple_GET_ITEM(kept, 0), *split = PyTuple_GET_ITEM(kept, 1);
     int64_t version = 0, address = 0, made_on = 0;
     if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 3 || !whole(PyTuple_GET_ITEM(key, 0), version) ||
         !whole(PyTuple_GET_ITEM(key, 1), address) || !whole(PyTuple_GET_ITEM(kept, 3), made_on) || !THPVariable_Check(split))

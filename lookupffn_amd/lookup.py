@@ -195,48 +195,44 @@ class Hashing(nn.Module):
         allocator.  What a stream capture runs is folded inside it, anew and for it alone: a copy made there
         is not written before the first replay, and a copy made before may be dropped while the graph lives.
         A compiled call folds as well: a graph of operators knows no version and no stream."""
-        kept = self._kept_folds()
-        return ops.bh4_fold(self.projection.weight.detach().contiguous()) if kept is None else kept[1]
+        return self._kept_fold(False)
 
     def split_weight(self):
         """The same for 8-bit codes' kernel (ops.bh4_fold_split), kept in the same way."""
-        kept = self._kept_folds()
-        return ops.bh4_fold_split(self.projection.weight.detach().contiguous(), False) if kept is None else kept[5]
+        return self._kept_fold(True)
 
-    def _kept_folds(self):
-        """((version, address, device), folded, what it was folded from, stream, event, split), split for 8-bit codes;
-        None where nothing is kept."""
+    def _kept_fold(self, split):
+        """The copy asked for, made when it first is: the one that the layer's own kernel takes in _folded = ((version, address, device),
+        copy, what it was folded from, stream, event), one for other callers beside it."""
+        fold = (lambda w: ops.bh4_fold_split(w, False)) if split else ops.bh4_fold
         w = self.projection.weight
         if is_compiling() or not w.is_cuda:                       # (not on the GPU: an error)
-            return None
+            return fold(w.detach().contiguous())
+        name = "_folded" if split == (self.code_length == 8) else "_folded_other"
         key = (w._version, w.data_ptr(), w.device)
         with torch.cuda.device(w.device):
             if torch.cuda.is_current_stream_capturing():
-                return None
+                return fold(w.detach().contiguous())
             stream = torch.cuda.current_stream()
-            cached = getattr(self, "_folded", None)
+            cached = getattr(self, name, None)
             if cached is None or cached[0] != key:
                 alias = w.detach()
-                source = alias.contiguous()
-                folded = ops.bh4_fold(source)
-                split = ops.bh4_fold_split(source, False) if self.code_length == 8 else None
-                cached = (key, folded, alias, stream.cuda_stream, stream.record_event(), split)
-                self._folded = cached
+                cached = (key, fold(alias.contiguous()), alias, stream.cuda_stream, stream.record_event())
+                setattr(self, name, cached)
             elif cached[3] != stream.cuda_stream:
                 stream.wait_event(cached[4])
-                for t in cached[1], cached[5]:
-                    if t is not None:
-                        t.record_stream(stream)
-        return cached
+                cached[1].record_stream(stream)
+        return cached[1]
 
     def __getstate__(self):
         state = self.__dict__.copy()
-        state.pop("_folded", None)        # derived from the weight, and names its address
+        for name in ("_folded", "_folded_other"):        # derived from the weight, and names its address
+            state.pop(name, None)
         return state
 
     def invalidate_folded_weight(self):
-        """Forget the folded copy of the BH4 weights: the next block-64 inference call folds again."""
-        self._folded = None
+        """Forget the folded copies of the BH4 weights: the next block-64 inference call folds again."""
+        self._folded = self._folded_other = None
 
     def train(self, mode=True):
         if mode != self.training:

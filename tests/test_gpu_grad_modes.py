@@ -57,7 +57,32 @@ def test_the_folded_blocks_follow_the_weights(training):
             change()
             assert _same_rows(layer(x), layer._forward_operators(x, None))
             kept = layer.hash.__dict__.get("_folded")
-            assert kept is not None and kept[1] is layer.hash.folded_weight()
+            assert kept is not None and kept[1] is layer.hash.split_weight()
+
+
+def test_only_the_copy_asked_for_is_folded(monkeypatch):
+    """One launch after a change of the weights, whoever asks; another caller's copy beside it, and both follow the weights."""
+    layer, made = _layer(256, 32, 64, 64, False), []
+    for name in ("bh4_fold", "bh4_fold_split"):
+        monkeypatch.setattr(lookupffn_amd.ops, name, lambda *a, name=name, fold=getattr(lookupffn_amd.ops, name): made.append(name) or fold(*a))
+    x = torch.randn(50, 256, device=DEV)
+    with torch.no_grad():
+        for _ in range(2):
+            layer(x), layer(x), layer._forward_operators(x, None)
+            assert made == ["bh4_fold_split"]
+            w = layer.hash.folded_weight()
+            assert layer.hash.folded_weight() is w and made == ["bh4_fold_split", "bh4_fold"]
+            assert torch.equal(w, lookupffn_amd.ops.bh4_fold_mode(layer.hash.projection.weight, 0).view_as(w))
+            assert layer.hash.split_weight().numel() == lookupffn_amd.ops.split_words(layer.hash.projection.weight.shape)
+            layer(x)
+            assert len(made) == 2
+            layer.hash.projection.weight.mul_(1.5)
+            del made[:]
+        state = layer.hash.__getstate__()
+        assert not any(name.startswith("_folded") for name in state)
+        layer.hash.invalidate_folded_weight()
+        layer(x), layer.hash.folded_weight()
+        assert made == ["bh4_fold_split", "bh4_fold"]
 
 
 def test_an_encoder_layer_in_train_with_and_without_gradients():
