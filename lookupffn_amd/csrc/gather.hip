@@ -714,6 +714,9 @@ bool lffn_internal_lookup_inner_tokens_try(const int32_t *code, const float *g, 
     return true;
 }
 
+// Passes of the token-major inner product over a token's rows of Do columns.
+int lffn_internal_row_passes(int64_t Do) { return pick_tiling((int)(Do / Row<LFFN_ROWS_F32>::EPV)).chunks; }
+
 // Token-major inner product on table-local codes: the fallback of lookup_inner.hip.
 int lffn_internal_lookup_inner_token_major(const int32_t *code, const float *g, const float *tables,
                                            float *out, int64_t B, int64_t T, int64_t S, int64_t Do,

@@ -71,6 +71,10 @@ int lffn_internal_lookup_inner_token_major(const int32_t *code, const float *g, 
                                            float *out, int64_t B, int64_t T, int64_t S, int64_t Do,
                                            void *stream);
 
+// gather.hip: passes of that kernel over a token's rows (not exported)
+__attribute__((visibility("hidden")))
+int lffn_internal_row_passes(int64_t Do);
+
 // lookup_gather_pair.hip: the two-tables-per-buffer LDS gather (not exported)
 __attribute__((visibility("hidden")))
 int lffn_internal_lookup_gather_pair(const int32_t *code, const float *score, const void *tables,

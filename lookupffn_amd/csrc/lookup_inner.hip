@@ -28,6 +28,8 @@
 // time unchanged: with 832 tokens a tile the table time is the slice copy
 // (about 1.1 us for 64 KB per compute unit) plus the part of the arithmetic that
 // does not overlap with it.
+#include <algorithm>
+
 #include "lffn_common.h"
 
 #include <hip/amd_detail/amd_hip_unsafe_atomics.h>
@@ -251,6 +253,11 @@ int launch_inner(const InnerArgs &a, hipStream_t stream) {
 
 }  // namespace
 
+// LDS form (tables that fit its buffers): enough (token tile, slice) units to fill most CUs
+static bool lds_form(int64_t B, int64_t T, int64_t Do) {
+    return T >= 4 && B * T < (int64_t(1) << 30) && ((B + 255) / 256) * (Do / 64) >= 192 && B * (Do / 64) <= (int64_t(1) << 30);
+}
+
 // Table pairs per workgroup of the four-lanes-per-token kernel (lookup_inner_quad.hip), 0: another kernel.  A workgroup of 1024 tokens
 // fetches its g once per slice for its pairs, so as many of them as still give the chip most of a round; one pair where that is one
 // round.  us at 4 | 2 | 1 pairs a workgroup | the other kernels, workgroups of one pair in brackets:
@@ -258,10 +265,25 @@ int launch_inner(const InnerArgs &a, hipStream_t stream) {
 //   3000 x 128 x 768 (192) 139 |  87 |  61      16384 x 32 x 256 (256)   48 |  31 |  23        5120 x 128 x 768 (320) 133 |  86 | 127
 //   2048 x 128 x 512 (128) 110 |  65 |  43 | 49  4096 x 64 x 768 (128)  141 |  89 |  62 | 73    1024 x 256 x 768 (128) 176 | 108 | 77 | 89
 //   8192 x 32 x 512 (128)   87 |  56 |  40 | 37  1024 x 128 x 768 (64)  179 | 107 |  69 | 46
-static int quad_chunk(int64_t B, int64_t T) {
+// Below 192 workgroups two pairs are no choice, and whether one pair is depends on how full the tiles are: its time is that of full
+// ones.  There both sides are estimated, us: a step of 32 columns 2.25, or the tables from memory; against it the LDS form by its tables,
+// or the token-major kernel by the rows it reads, but no less than its chain of a token's rows.  Others -> one pair:
+//   1030 x 128 x 512 34 -> 40, 1300 40 -> 40, 2048 49 -> 41; x 768 55 -> 65, 1300 64 -> 64, 2048 78 -> 63; x 1024 72 -> 76, 1300 90 -> 74
+//   400 x 256 x 1024 68 -> 96, 700 86 -> 107, 1024 119 -> 116; x 768 520 63 -> 69, 900 80 -> 76; 900 x 256 x 512 60 -> 48
+//   4096 x 64 x 256 20 -> 22, x 384 27 -> 33, x 512 56 -> 40, x 1024 65 -> 74 (the LDS form); 5000 x 64 x 384 40 -> 33
+//   1600 x 128 x 64 27 -> 7, x 640 (five passes over a token's rows) 110 -> 56; 520 x 256 x 896 (seven) 302 -> 77
+static bool one_pair_pays(int64_t B, int64_t T, int64_t Do) {
+    const double tables = double(T) * MAX_S * double(Do) * 4e-6, rows = double(B * T) * double(Do) * 4e-6;          // MB
+    const double one_pair = std::max(2.25 * double(Do / 32) + 4.0, tables / (tables <= 256.0 ? 2.8 : 2.4));
+    if (lds_form(B, T, Do)) return one_pair < 1.05 * double(T);
+    const int passes = lffn_internal_row_passes(Do);
+    const double chain = double(T) * (passes > 1 ? 0.17 * passes : 0.21);
+    return one_pair < std::max(chain, tables <= 26.0 ? rows / 15.5 : 0.033 * double(Do) + rows / 13.0);
+}
+static int quad_chunk(int64_t B, int64_t T, int64_t Do) {
     const int64_t tiles = (B + 1023) / 1024, pairs = T / 2;
     if (tiles * ((pairs + 3) / 4) >= 200) return 4;
-    if (tiles * pairs <= 256 && tiles * pairs >= (pairs >= 32 ? 128 : 192)) return 1;
+    if (tiles * pairs <= 256 && (tiles * pairs >= 192 || (pairs >= 32 && tiles * pairs >= 128 && one_pair_pays(B, T, Do)))) return 1;
     return tiles * ((pairs + 1) / 2) >= 96 ? 2 : 0;
 }
 
@@ -274,7 +296,7 @@ bool lffn_internal_lookup_inner_quad_try(const int32_t *code, const float *g, in
     if (!(S == MAX_S && T % 2 == 0 && Do % 32 == 0 && B >= 1 && reinterpret_cast<uintptr_t>(code) % 8 == 0 &&
           2 * S * Do * 4 < (int64_t(1) << 32)))
         return false;
-    const int c = quad_chunk(B, T);
+    const int c = quad_chunk(B, T, Do);
     if (!c || (B + 1023) / 1024 * ((T / 2 + c - 1) / c) > (int64_t(1) << 30)) return false;
     *rc = lffn_internal_lookup_inner_quad(code, g, g_token_stride, g_slice_stride, tables, grad_score, B, T, S, Do, 4, c, stream);
     return true;
@@ -299,10 +321,7 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
         if (lffn_internal_lookup_inner_quad_try(code, g, Do, 32, tables, grad_score, B, T, S, Do, stream, &rc)) return rc;
     }
 
-    // LDS form: table fits the buffers, and enough (token tile, slice) units to fill most CUs
-    const bool lds_ok = S <= MAX_S && T >= 4 && B * T < (int64_t(1) << 30) &&
-                        ((B + 255) / 256) * nslices >= 192 && B * nslices <= (int64_t(1) << 30);
-    if (!lds_ok) return lffn_internal_lookup_inner_token_major(code, g, tables, grad_score, B, T, S, Do, stream);
+    if (S > MAX_S || !lds_form(B, T, Do)) return lffn_internal_lookup_inner_token_major(code, g, tables, grad_score, B, T, S, Do, stream);
 
     const int64_t n = B * T;
     const int64_t blocks = (n + 255) / 256;
@@ -342,7 +361,7 @@ bool inner_try_tables(int64_t B, int64_t I, int64_t source_size, int64_t Dv) {
     if (B < 1 || I < 2 || I % 2 != 0 || source_size != I * MAX_S || Dv < 64 || Dv % 64 != 0 || Dv > (1 << 20) ||
         B * I >= (int64_t(1) << 31) || 2 * MAX_S * Dv * 4 >= (int64_t(1) << 32))
         return false;
-    const int c = quad_chunk(B, I);
+    const int c = quad_chunk(B, I, Dv);
     if (!c) return false;
     const int64_t rounds = ((B + 1023) / 1024 * ((I / 2 + c - 1) / c) + 255) / 256;
     const double us = double(rounds) * double(Dv / 32) * (c > 1 ? c : 2) * 1.3 + 6.0;

@@ -23,3 +23,19 @@ def test_inner_of_one_table_pair_a_workgroup(B, T, Do):
         want, bound = (rows * g).sum(1), (np.abs(rows) * np.abs(g)).sum(1) * Do * 2.0 ** -24
         assert (np.abs(got[:, t] - want) <= bound).all()
     assert np.array_equal(got, cabi.lookup_inner(code, g, tables))      # one owner a sum
+
+
+# 128 to 191 workgroups of one pair, where tiles that are hardly filled, small tables and wide rows go to the other kernels and the rest
+# does not: either side of each line, and either side of 192 workgroups
+@pytest.mark.parametrize("B,T,Do", [(1026, 128, 512), (2047, 128, 512), (1700, 128, 64), (1537, 128, 320), (520, 256, 896), (520, 256, 832),
+                                    (3073, 64, 256), (3073, 64, 384), (5100, 64, 384), (3073, 64, 960), (3073, 64, 1024), (3072, 96, 1024),
+                                    (3072, 126, 384), (3073, 96, 256)])
+def test_inner_where_one_table_pair_a_workgroup_may_pay(B, T, Do):
+    rng = np.random.RandomState(B + T)
+    tables, g = rng.randn(T, 256, Do).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    code = rng.randint(0, 256, size=(B, T)).astype(np.int32)
+    got = cabi.lookup_inner(code, g, tables)
+    for t in range(T):
+        rows = tables[t, code[:, t]].astype(np.float64)
+        want, bound = (rows * g).sum(1), (np.abs(rows) * np.abs(g)).sum(1) * Do * 2.0 ** -24
+        assert (np.abs(got[:, t] - want) <= bound).all()
