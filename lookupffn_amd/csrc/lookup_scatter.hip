@@ -48,6 +48,7 @@ struct ScatterArgs {
     int T, S, Do;
     int nslices, per_xcd;
     int accumulate;
+    int past_caches;       // lffn_rows_written_past_caches
 };
 
 __global__ __launch_bounds__(WG) void lookup_scatter_lds_kernel(ScatterArgs a) {
@@ -246,9 +247,8 @@ __global__ __launch_bounds__(256) void lookup_scatter_list_kernel(ScatterArgs a,
                     const float4 old = *reinterpret_cast<const float4 *>(dst + col[c]);
                     v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
                 }
-                // (of no further use here, and in the caches they take the place of g and of what the rest of the backward reads: training
-                // steps of 500 tokens of 512 tables of 1024 columns 519 -> 474 us, 128 270 -> 248, 1500 of 128 x 768 249 -> 237)
-                __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(dst + col[c]));
+                if (a.past_caches) __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(dst + col[c]));
+                else *reinterpret_cast<float4 *>(dst + col[c]) = v;
             }
         }
     }
@@ -301,6 +301,7 @@ __global__ __launch_bounds__(256) void lookup_scatter_list_kernel(ScatterArgs a,
 int launch_list(const ScatterArgs &args, hipStream_t st) {
     ScatterArgs a = args;
     const int groups = a.S > ROWS_PER_WG ? a.S / ROWS_PER_WG : 1;
+    a.past_caches = lffn_rows_written_past_caches(int64_t(a.T) * a.S, a.Do);
     a.per_xcd = (a.T * groups + XCDS - 1) / XCDS;
     const dim3 grid((unsigned)(a.per_xcd * XCDS));
     const size_t lds_bytes = (size_t)a.B * sizeof(uint2);

@@ -305,7 +305,7 @@ struct SortedArgs {
     int64_t stride, rows;
     unsigned last_token;   // B: the padding's
     int T, S, Do, nslices, accumulate;
-    int more;              // a later launch adds to these rows
+    int past_caches;       // lffn_rows_written_past_caches, and no later launch adds to these rows
 };
 
 __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
@@ -358,11 +358,9 @@ __global__ __launch_bounds__(MWG) void lookup_scatter_sorted_kernel(SortedArgs a
     __syncthreads();
 
     float *orow = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC + j * 4;     // + code * Do
-    // Rows that nothing adds to any more go out nontemporally: in the caches they would take the place of g (the operator's pass at 4096 x
-    // 128 x 512 233 -> 226 us); where they are read again next, 32768 x 512, that costs 7 of 1490.
     auto store_row = [&](float *p, float4 v) {
-        if (a.more) *reinterpret_cast<float4 *>(p) = v;                            // uniform
-        else __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(p));
+        if (a.past_caches) __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(p));      // uniform
+        else *reinterpret_cast<float4 *>(p) = v;
     };
     if (!ADD)                                                 // rows no token points at
         for (int q = tid; q < S * 8; q += MWG) {
@@ -605,7 +603,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         ma.last_token = (unsigned)Bc;
         ma.T = (int)T; ma.S = (int)S; ma.Do = (int)Do; ma.nslices = (int)(Do / SC);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
-        ma.more = c0 + CHUNK < B ? 1 : 0;
+        ma.past_caches = c0 + CHUNK >= B && lffn_rows_written_past_caches(T * S, Do);
         rc = launch_sorted(ma, st);
         if (rc != LFFN_OK) return rc;
     }
@@ -880,7 +878,7 @@ __device__ __forceinline__ void add_pairs(float4 (&acc)[NC], const G *g, const u
 }
 
 template <typename G, int NC>
-__global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, int accumulate) {
+__global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, int accumulate, int past_caches) {
     __shared__ float4 part[4][NC][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -897,8 +895,8 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, i
             const float4 old = *dst;
             v.x += old.x; v.y += old.y; v.z += old.z; v.w += old.w;
         }
-        // (rows of no further use here: 64 tokens of 512 tables of 1024 columns, the operator's pass 197 -> 184 us, 500 of 256 244 -> 223)
-        __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(dst));
+        if (past_caches) __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(dst));      // uniform
+        else *dst = v;
     };
     for (int col0 = 4 * lane; col0 - 4 * lane < a.Dv; col0 += 256 * NC) {
         for (int r = wave; r < nrows; r += 4) {
@@ -942,11 +940,12 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, i
 template <typename G>
 int launch_rows_sum(const RowsArgs &a, float *out, int accumulate, hipStream_t st) {
     const dim3 grid((unsigned)((a.rows + ROW_GROUP - 1) / ROW_GROUP));
+    const int past_caches = lffn_rows_written_past_caches(a.rows, a.Dv);
     switch ((a.Dv + 255) / 256) {
-        case 1: hipLaunchKernelGGL((rows_sum_kernel<G, 1>), grid, dim3(256), 0, st, a, out, accumulate); break;
-        case 2: hipLaunchKernelGGL((rows_sum_kernel<G, 2>), grid, dim3(256), 0, st, a, out, accumulate); break;
-        case 3: hipLaunchKernelGGL((rows_sum_kernel<G, 3>), grid, dim3(256), 0, st, a, out, accumulate); break;
-        default: hipLaunchKernelGGL((rows_sum_kernel<G, 4>), grid, dim3(256), 0, st, a, out, accumulate); break;
+        case 1: hipLaunchKernelGGL((rows_sum_kernel<G, 1>), grid, dim3(256), 0, st, a, out, accumulate, past_caches); break;
+        case 2: hipLaunchKernelGGL((rows_sum_kernel<G, 2>), grid, dim3(256), 0, st, a, out, accumulate, past_caches); break;
+        case 3: hipLaunchKernelGGL((rows_sum_kernel<G, 3>), grid, dim3(256), 0, st, a, out, accumulate, past_caches); break;
+        default: hipLaunchKernelGGL((rows_sum_kernel<G, 4>), grid, dim3(256), 0, st, a, out, accumulate, past_caches); break;
     }
     return lffn_launch_status();
 }
@@ -1044,7 +1043,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         ma.last_token = (unsigned)a.B;
         ma.T = a.tables; ma.S = VT; ma.Do = (int)Dv; ma.nslices = (int)(Dv / SC);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
-        ma.more = c0 + CHUNK < B ? 1 : 0;
+        ma.past_caches = c0 + CHUNK >= B && lffn_rows_written_past_caches(out_size, Dv);
         rc = launch_sorted(ma, st);
         if (rc != LFFN_OK) return rc;
     }
