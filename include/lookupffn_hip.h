@@ -831,7 +831,7 @@ int lffn_bh4_block_bwd_split_f32(const float *g_z, const float *w_split_t, float
  * lffn_bh4_block_bwd_split_f32 behind the gradient of the 8-bit scores: from z [B, T*8] (16-byte aligned) and g_score [B, T], with the
  * gradient of z that lffn_code_score_bwd_f32 computes formed inside.  bias_parts: [ceil(B / 16), T*8] or NULL, every sixteen tokens'
  * sum of it (the projection bias's gradient is the sum of these rows).  clear: an array of clear_n floats (a multiple of 4; 16-byte aligned)
- * that is set to zero on the way, such as what the weight gradient is added to, or NULL.
+ * that is set to zero on the way (B = 0 included), such as what the weight gradient is added to, or NULL.
  */
 int lffn_bh4_block_score_bwd_split_f32(const float *z, const float *g_score, const float *w_split_t, float *g_x,
                                        float *stage_grads, float *bias_parts, float *clear, int64_t clear_n, int64_t B, int64_t H, int64_t D, int64_t R,

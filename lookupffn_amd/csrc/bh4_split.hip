@@ -31,6 +31,8 @@
 // gradients must not differ from one with them.  The training form is the hash form with stores: its codes and scores are the same
 // bit for bit.  Against 64 bits, LayerNorm included, 200 rows of D = 512, fp32 kernel -> this one: z 3.1e-7 -> 2.4e-7, stage inputs
 // 2.4e-7 -> 1.8e-7, scores 4.5e-7 -> 3.4e-7 (rows spread over e^1.5 in size: 3.2e-7, 2.4e-7, 4.6e-7 -> 2.4e-7, 1.9e-7, 3.9e-7).
+#include <algorithm>
+
 #include "split_mfma.h"
 
 // the mix and the score keep the reference's operation order: no fused multiply-add
@@ -928,6 +930,10 @@ extern "C" int lffn_bh4_block_front_train_split_f32(const lffn_block_front *f, c
 
 namespace {
 
+__global__ __launch_bounds__(256) void clear_kernel(float4 *p, int64_t n) {
+    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x) * 256) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
 // the backwards' arguments, checked
 int back_args(const float *w_split_t, float *g_x, float *stage_grads, int64_t B, int64_t H, int64_t D, int64_t R, int64_t J, int64_t T,
               int64_t block_size, float decay, float residual, SplitArgs &a) {
@@ -963,9 +969,15 @@ extern "C" int lffn_bh4_block_score_bwd_split_f32(const float *z, const float *g
                                                   float residual, void *stream) {
     SplitArgs a{};
     const int rc = back_args(w_split_t, g_x, stage_grads, B, H, D, R, J, T, block_size, decay, residual, a);
-    if (rc != LFFN_OK || B == 0) return rc;
-    LFFN_REQUIRE(z && g_score && lffn_aligned16(z) && lffn_aligned16(clear), LFFN_ERR_BAD_ARG);
-    LFFN_REQUIRE(!clear || (clear_n >= 0 && clear_n % 4 == 0), LFFN_ERR_BAD_ARG);
+    if (rc != LFFN_OK) return rc;
+    LFFN_REQUIRE(!clear || (clear_n >= 0 && clear_n % 4 == 0 && lffn_aligned16(clear)), LFFN_ERR_BAD_ARG);
+    if (B == 0) {                                 // nothing but that
+        if (!clear || clear_n == 0) return LFFN_OK;
+        hipLaunchKernelGGL(clear_kernel, dim3((unsigned)std::min<int64_t>((clear_n / 4 + 255) / 256, 4096)), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), reinterpret_cast<float4 *>(clear), clear_n / 4);
+        return lffn_launch_status();
+    }
+    LFFN_REQUIRE(z && g_score && lffn_aligned16(z), LFFN_ERR_BAD_ARG);
     a.clear = reinterpret_cast<float4 *>(clear); a.clear_n = clear ? clear_n / 4 : 0;
     a.z = const_cast<float *>(z); a.g_score = g_score; a.bias_parts = bias_parts;
     return dispatch_block<SCORES_BACKWARD>(a, D, static_cast<hipStream_t>(stream));

@@ -112,6 +112,15 @@ def test_backward_from_scores(B, H, D, R, T):
         assert rc == 0 and not clear[:n].any() and clear[n:].all()
 
 
+@pytest.mark.parametrize("n", [0, 4, 1000, 3 << 20])
+def test_backward_of_no_tokens_clears(n):
+    clear = torch.ones(n + 4, device=DEV)
+    args = (0, 256, 256, 1, 4, 32, 64, 0.7, 0.3, _lib.stream_of(clear))
+    entry = _lib.load().lffn_bh4_block_score_bwd_split_f32
+    assert entry(None, None, None, None, None, None, None, 0, *args) == 0
+    assert entry(None, None, None, None, None, None, clear.data_ptr(), n, *args) == 0 and not clear[:n].any() and clear[n:].all()
+
+
 @pytest.mark.parametrize("stages,NB", [(1, 1), (3, 2), (8, 8), (4, 16)])
 def test_both_foldings_in_one_launch(stages, NB):
     w = torch.randn(stages, 1, NB, 64, 64, device=DEV)
