@@ -94,7 +94,7 @@ __device__ __forceinline__ void lane_stage(float (&v)[NJ][4], int lr) {
     }
 }
 
-// Butterflies across lanes 1, 2 or 8 apart in one instruction a value instead of two: every lane gets own + partner * sgn (`sgn` as in
+// Butterflies across lanes 1 or 2 apart in one instruction a value instead of two: every lane gets own + partner * sgn (`sgn` as in
 // butterfly_xor), so the lane whose M bit is set gets own - partner, the result with its sign turned round (exact: a - b and b - a
 // round alike).  What follows is linear and takes the sign along; in the next transform the partners of this butterfly have opposite
 // signs, and with -sgn both come out upright again.  So `sgn` alternates from transform to transform, and after an even number of
@@ -102,7 +102,7 @@ __device__ __forceinline__ void lane_stage(float (&v)[NJ][4], int lr) {
 // vector instruction has just written is ready for DPP two instructions later: hence the s_nop.)
 template <int M>
 __device__ __forceinline__ void turning_butterflies(float (&a)[4], float (&b)[4], float sgn) {
-    static_assert(M == 1 || M == 2 || M == 8, "one DPP move");
+    static_assert(M == 1 || M == 2, "one DPP move");
 #define LFFN_TURN8(ctrl)                                                                                                              \
     asm("s_nop 1\n\t"                                                                                                                 \
         "v_fmac_f32_dpp %0, %0, %8 " ctrl "\n\tv_fmac_f32_dpp %1, %1, %8 " ctrl "\n\tv_fmac_f32_dpp %2, %2, %8 " ctrl "\n\t"          \
@@ -111,8 +111,7 @@ __device__ __forceinline__ void turning_butterflies(float (&a)[4], float (&b)[4]
         : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3])                                \
         : "v"(sgn))
     if constexpr (M == 1) LFFN_TURN8("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf");
-    else if constexpr (M == 2) LFFN_TURN8("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf");
-    else LFFN_TURN8("row_ror:8 row_mask:0xf bank_mask:0xf");
+    else LFFN_TURN8("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf");
 #undef LFFN_TURN8
 }
 
