@@ -701,7 +701,7 @@ def main():
                  "synthetic (seeded N(0,1) tokens, seeded +-1/sqrt(D) sign diagonals, N(0,0.02) tables)"),
         "config": {"workload": wl["desc"], "tokens": B, "d_model": H, "fht_dim": layer.hash.projection.padded_in_dim,
                    "tables": T, "table_size": S, "d_out": Do,
-                   "step": ("one kernel: LayerNorm + BH4(block 64)x4 on fp32 MFMA + mix + hash (weights folded once, "
+                   "step": ("one kernel: LayerNorm + BH4(block 64)x4 on fp16 MFMA, two terms a number, + mix + hash (weights folded once, "
                             "outside the step)" + (", written as the gather's record stream" if rec_plan is not None else "") +
                             "; " + gather_step) if block else
                            ("one kernel: LayerNorm + BH4(block 1)x4 + mix + hash + gather-add + bias" if fused_layer else
