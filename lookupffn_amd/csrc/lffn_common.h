@@ -390,7 +390,7 @@ __device__ __forceinline__ float score_derivative(float z, float away, float twi
     return z != 0.f ? v : 0.f;
 }
 
-// Are the table gradients of so many rows written nontemporally?  A training program reads them next, with the tables: up to half of
+// Are the table gradients of so many rows, of few tokens, written nontemporally?  A training program reads them next, with the tables: up to half of
 // the 256 MB memory-side cache both may still be there, beyond it the rows only take the place of g and of what the rest of the backward
 // reads.  us of a training step, and of one with an SGD step, clipping and SGD, Adam behind it, written plainly -> nontemporally:
 //   1500 tokens of 128 tables x 768 (101 MB)  208 -> 199, 274 -> 268, 353 -> 374, 432 -> 426    500 of 128 x 768  117 -> 118, 135 -> 154, 216 -> 232
@@ -398,7 +398,6 @@ __device__ __forceinline__ float score_derivative(float z, float away, float twi
 //   500 of 256 x 768 (201 MB)  223 -> 192, 334 -> 307, 474 -> 484, 551 -> 534      500 of 512 x 1024  512 -> 465, 881 -> 834, 1317 -> 1293, 1486 -> 1447
 // and of the operator's pass, alone and with an SGD step:
 //   1000 of 128 x 768  138 -> 137, 188 -> 201    300 of 384 x 768 (302 MB)  229 -> 195, 431 -> 390    64 of 512 x 1024  195 -> 171, 555 -> 531
-//   8192 of 256 x 512 (134 MB)  601 -> 586, 671 -> 662 (the sorted accumulation; training steps of 2500 tokens and more: within 1% either way)
 inline bool lffn_rows_written_past_caches(int64_t rows, int64_t columns) { return rows * columns * 4 >= int64_t(1) << 27; }
 
 __device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }

@@ -305,7 +305,7 @@ struct SortedArgs {
     int64_t stride, rows;
     unsigned last_token;   // B: the padding's
     int T, S, Do, nslices, accumulate;
-    int past_caches;       // lffn_rows_written_past_caches, and no later launch adds to these rows
+    int more;              // a later launch adds to these rows
 };
 
 __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
@@ -358,9 +358,15 @@ __global__ __launch_bounds__(MWG) void lookup_scatter_sorted_kernel(SortedArgs a
     __syncthreads();
 
     float *orow = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC + j * 4;     // + code * Do
+    // Rows that nothing adds to any more go out nontemporally: in the caches they would take the place of g.  Read again next, 32768 x 512,
+    // that costs 7 us of 1490.  With a reader behind the pass, unlike the lists and the sums of few pairs (lffn_rows_written_past_caches), it
+    // costs no more than it gives: a training step of 2500 tokens and more of 128 to 512 tables takes the same alone and with SGD, clipping
+    // or Adam behind it; the operator's pass, plainly -> nontemporally, alone, with SGD, with Adam:
+    //   4096 x 128 x 512  231 -> 226 (219 for 229 where the passes' results stay), 270 -> 264, 317 -> 318    3000 x 128 x 512  206 -> 204, 245 -> 239, 295 -> 298
+    //   8192 x 64 x 512  217 -> 202, 232 -> 240, 283 -> 284    2500 x 128 x 768  266 -> 265, 332 -> 337, 462 -> 462    8192 x 256 x 512  601 -> 586, 671 -> 662
     auto store_row = [&](float *p, float4 v) {
-        if (a.past_caches) __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(p));      // uniform
-        else *reinterpret_cast<float4 *>(p) = v;
+        if (a.more) *reinterpret_cast<float4 *>(p) = v;                            // uniform
+        else __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(p));
     };
     if (!ADD)                                                 // rows no token points at
         for (int q = tid; q < S * 8; q += MWG) {
@@ -603,7 +609,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         ma.last_token = (unsigned)Bc;
         ma.T = (int)T; ma.S = (int)S; ma.Do = (int)Do; ma.nslices = (int)(Do / SC);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
-        ma.past_caches = c0 + CHUNK >= B && lffn_rows_written_past_caches(T * S, Do);
+        ma.more = c0 + CHUNK < B ? 1 : 0;
         rc = launch_sorted(ma, st);
         if (rc != LFFN_OK) return rc;
     }
@@ -1043,7 +1049,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         ma.last_token = (unsigned)a.B;
         ma.T = a.tables; ma.S = VT; ma.Do = (int)Dv; ma.nslices = (int)(Dv / SC);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
-        ma.past_caches = c0 + CHUNK >= B && lffn_rows_written_past_caches(out_size, Dv);
+        ma.more = c0 + CHUNK < B ? 1 : 0;
         rc = launch_sorted(ma, st);
         if (rc != LFFN_OK) return rc;
     }
