@@ -398,7 +398,11 @@ __device__ __forceinline__ float score_derivative(float z, float away, float twi
 //   500 of 256 x 768 (201 MB)  223 -> 192, 334 -> 307, 474 -> 484, 551 -> 534      500 of 512 x 1024  512 -> 465, 881 -> 834, 1317 -> 1293, 1486 -> 1447
 // and of the operator's pass, alone and with an SGD step:
 //   1000 of 128 x 768  138 -> 137, 188 -> 201    300 of 384 x 768 (302 MB)  229 -> 195, 431 -> 390    64 of 512 x 1024  195 -> 171, 555 -> 531
-inline bool lffn_rows_written_past_caches(int64_t rows, int64_t columns) { return rows * columns * 4 >= int64_t(1) << 27; }
+// Of an all-half call (`alone`) the rows are read by themselves, at once, to be rounded, and all of the cache is theirs:
+//   300 of 256 x 512 (134 MB)  122 -> 133, 500 of 256 x 768 (201 MB)  179 -> 189, 200 of 256 x 1024 (268 MB)  198 -> 194, 64 of 512 x 1024  333 -> 318
+inline bool lffn_rows_written_past_caches(int64_t rows, int64_t columns, bool alone = false) {
+    return rows * columns * 4 >= int64_t(1) << (alone ? 28 : 27);
+}
 
 __device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_float(packed & 0xFFFF0000u); }

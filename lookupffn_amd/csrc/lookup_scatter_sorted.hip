@@ -946,7 +946,7 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, i
 template <typename G>
 int launch_rows_sum(const RowsArgs &a, float *out, int accumulate, hipStream_t st) {
     const dim3 grid((unsigned)((a.rows + ROW_GROUP - 1) / ROW_GROUP));
-    const int past_caches = lffn_rows_written_past_caches(a.rows, a.Dv);
+    const int past_caches = lffn_rows_written_past_caches(a.rows, a.Dv, sizeof(G) == 2);
     switch ((a.Dv + 255) / 256) {
         case 1: hipLaunchKernelGGL((rows_sum_kernel<G, 1>), grid, dim3(256), 0, st, a, out, accumulate, past_caches); break;
         case 2: hipLaunchKernelGGL((rows_sum_kernel<G, 2>), grid, dim3(256), 0, st, a, out, accumulate, past_caches); break;
