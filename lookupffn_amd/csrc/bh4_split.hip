@@ -66,7 +66,7 @@ __device__ __forceinline__ void wave_range(float v, float &most, float &least) {
 //     22 bits down to 2^-9 of its own largest, and is held to 2^-31 of that below;
 //   else every column of every block by itself, its largest to [2^14, 2^15), and the product kernel multiplies by the way back: the
 //     forward its rows, before it takes their largest, the backward what it has formed.
-// At 32768 tokens, D = 512, two repeats the second costs 8, 13 and 5 us of hash, training form and backward, the choice between them 0, 5
+// At 32768 tokens, D = 512, two repeats the second costs 8, 13 and 5 us of hash, training form and backward, the choice between them 0, 4
 // and 0.  With one scale for a stage's column (sixteen of the forward's) in all blocks, as it was, the relative error was 4e-5 where columns
 // are spread over 1e8 and their inputs the other way round, and 4e-4 in the gradient of a small block; so it is 1.2e-7 and 1.9e-7, as it is
 // for numbers of one size (fp32 kernel 1.7e-7 and 2.8e-7).
@@ -300,7 +300,8 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     // (no store of this kernel meets the weights: a scalar load)
     const auto *const each = (const __attribute__((address_space(4))) float *)(uintptr_t)(a.wback + size_t(a.R) * J * D + r * J);
     auto together_of = [&](int s) { return each[s]; };
-    float together = together_of(BWD ? J - 1 : 0);            // of the stage whose product is next
+    // of the stage whose product is next and the one after, requested a stage ahead (a product's LDS reads would wait for it)
+    float together = together_of(BWD ? J - 1 : 0), together_next = together_of(BWD ? max(J - 2, 0) : min(1, J - 1));
     auto back_of = [&](int s, int col) { return *reinterpret_cast<const f32x4 *>(a.wback + size_t(r * J + s) * D + col); };
     // v[i] times the way back of four columns (a few at a time: registers), over 2^14 times f
     auto go_back = [&](int s, auto &v, auto col, float f) {
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     auto product = [&](int s) {
         const float own = together;
         inv_x = own != 0.f ? unscale[c] * (own * (BWD ? 1.f : TOP)) : unscale[c];
-        together = together_of(BWD ? max(s - 1, 0) : min(s + 1, J - 1));
+        together = together_next;
         uint4 xv[2][4];
         read_x(0, xv[0]);
         static_for<NBW>([&](auto n_c) {
@@ -336,6 +337,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
             __builtin_amdgcn_sched_barrier(0);
         });
         load_w(s, NBW - 1 + AHEAD);
+        together_next = together_of(BWD ? max(s - 2, 0) : min(s + 2, J - 1));
         if (BWD && own == 0.f) go_back(s, acc, own_col, 1.f);                   // uniform
     };
 
