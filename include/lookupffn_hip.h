@@ -716,7 +716,7 @@ int lffn_lookup_scatter_f32(const int32_t *code, const float *score, const float
 /*
  * The same sums without atomics on the accumulators, through a caller-provided workspace:
  * the inputs are transposed / copied slice-major, each table's tokens are sorted by code
- * (stable counting sort, (token, score) pairs, buckets padded to multiples of eight), and a
+ * (stable counting sort, (token, score) pairs), and a
  * last kernel walks the sorted lists and adds the rows of g in registers; rows of
  * grad_tables are written with plain stores and the order of additions is fixed (token order
  * inside a code), so results are reproducible from run to run, unlike the reference's

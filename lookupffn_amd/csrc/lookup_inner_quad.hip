@@ -53,8 +53,8 @@ constexpr int TOUCH_AHEAD = 3;              // steps between the one being read 
 
 struct InnerQuadArgs {
     const int32_t *code;   // [B, T]
-    const float *g;        // token b, slice s (32 columns) at g + b * g_token_stride + s * g_slice_stride
-    int64_t g_token_stride, g_slice_stride;     // floats: Do and 32 for [B, Do]; 32 and (B + 1) * 32 for [Do/32][B + 1][32]
+    const float *g;        // token b, slice s (32 columns) at g + b * g_token_stride + s / 2 * g_pair_stride + s % 2 * 32
+    int64_t g_token_stride, g_pair_stride;      // floats: Do and 64 for [B, Do]; 64 and (B + 1) * 64 for [Do/64][B + 1][64]
     const char *tables;    // [T, S, Do] fp32
     float *out;            // [B, T]
     int64_t B;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(WG) void lookup_inner_quad_kernel(InnerQuadArgs a) 
         // hoisted out of the slice loop the NP row pointers would cost 2*NP registers
         asm volatile("" : "+v"(tok_low));
         const int64_t tok = min(int64_t(tok_low) + int64_t(p) * 256, a.B - 1);
-        const float *gp = a.g + tok * a.g_token_stride + (size_t)slice * a.g_slice_stride + g_col;
+        const float *gp = a.g + tok * a.g_token_stride + (size_t)(slice >> 1) * a.g_pair_stride + ((slice & 1) * SLICE_COLS + g_col);
         gq[p][0] = *reinterpret_cast<const float4 *>(gp + half0 * 16);
         gq[p][1] = *reinterpret_cast<const float4 *>(gp + (half0 ^ 1) * 16);
     };
@@ -395,14 +395,14 @@ int launch_inner_quad(InnerQuadArgs a, hipStream_t stream) {
 // The caller has checked that the shape qualifies: S = 256 (a table pair fills an LDS buffer), T even,
 // Do a multiple of 32, 2*S*Do*4 < 2^32 (32-bit lane offsets from a table pair's base), 1 <= B < 2^31, code
 // aligned to 8 bytes, g to 16.  g: token b's 32 columns of slice s start at g + b * g_token_stride +
-// s * g_slice_stride floats (both multiples of 4).  256 * np tokens and c table pairs per workgroup.
-int lffn_internal_lookup_inner_quad(const int32_t *code, const float *g, int64_t g_token_stride, int64_t g_slice_stride,
+// s / 2 * g_pair_stride + s % 2 * 32 floats (the strides multiples of 4).  256 * np tokens and c table pairs per workgroup.
+int lffn_internal_lookup_inner_quad(const int32_t *code, const float *g, int64_t g_token_stride, int64_t g_pair_stride,
                                     const void *tables, float *grad_score, int64_t B, int64_t T, int64_t S, int64_t Do,
                                     int np, int c, void *stream) {
     if (S != MAX_S || T % 2 != 0 || T < 2 || Do % SLICE_COLS != 0 || B < 1) return LFFN_ERR_BAD_ARG;
     InnerQuadArgs a{};
     a.code = code; a.g = g; a.tables = static_cast<const char *>(tables); a.out = grad_score;
-    a.g_token_stride = g_token_stride; a.g_slice_stride = g_slice_stride;
+    a.g_token_stride = g_token_stride; a.g_pair_stride = g_pair_stride;
     a.B = B; a.T = (int)T; a.S = (int)S; a.Do = (int)Do;
     a.nslices = (int)(Do / SLICE_COLS);
     a.row_bytes = (int)(Do * 4);

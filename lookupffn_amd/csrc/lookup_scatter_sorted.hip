@@ -11,33 +11,43 @@
 //
 // lookup_sort_pack_kernel: two jobs in one launch, by workgroup number.  The sort occupies one
 // workgroup per table (128 of the 256 compute units at 128 tables) and is bound by latency; the
-// copy of g to a slice-major layout [Do/32][B + 1][32] (in which the 128-byte row pieces of a slice
-// are contiguous: with rows 4*Do bytes apart the pieces of one slice fall on a quarter of the L2
+// copy of g to a slice-major layout [ceil(Do / 64)][B + 1][64] (in which the 256-byte row pieces of a slice
+// are contiguous: with rows 4*Do bytes apart the pieces of one slice fall on a part of the L2
 // channels) is pure memory traffic and depends on nothing: its workgroups fill the rest of the
 // chip while the sort runs (23 + 25 us as two launches at 16384 tokens x 128 tables x 768).
 //
 // The sort: one workgroup per table sorts the tokens by their code for that
 // table (a stable counting sort: per-wavefront histograms over contiguous token ranges,
 // ranks inside a 64-token batch from ballots over the code bits) and writes (token, score)
-// pairs bucket by bucket: into LDS first (a 16-bit token and a score per entry: at most 18432
-// entries, 108 KB), from where the list goes to memory in whole lines; written straight
-// from the ranks, every wavefront store was 64 separate 8-byte requests.  Every bucket is padded to a multiple of eight entries,
-// so that eight consecutive entries always belong to one code, and the bucket boundaries are stored in units of eight entries.
-// The padding names token B, whose row of the copy of g is zero (a token of the bucket with weight 0 would make a row of an
-// infinite gradient NaN).
+// pairs bucket by bucket: into LDS first (a 16-bit token and a score per entry, 98 KB at most), from where the list goes to memory in
+// whole lines; written straight from the ranks, every wavefront store was 64 separate 8-byte requests.  More than SUB tokens are two
+// lists, each sorted by half of the wavefronts (a workgroup per list: 28 -> 34 us at 16384 tokens).  Nothing is padded.
 //
-// lookup_scatter_sorted_kernel: one workgroup per (table, 32-column slice).  The sorted
-// list is cut into equal pieces, one per wavefront, whatever the bucket sizes (a skewed code
-// distribution costs nothing).  A wavefront walks its piece eight tokens at a time: lane
-// group q = lane / 8 takes token q of the step, its eight lanes load the token's 128-byte
-// piece of g and multiply-add it into registers; at a bucket boundary (wave-uniform,
-// because of the padding) the eight partial sums are added across the lane groups and the
-// row is stored.  Buckets cut by a piece boundary go to LDS and one wavefront adds the
-// pieces in order after a barrier.  Every row of the slice is written exactly once with
-// plain stores: no zero-fill, no atomics, and the sum order is fixed (run-to-run
-// reproducible).  The slices are dealt to the XCDs so that the workgroups running on one
-// XCD read the same 32 columns of g (2 MB at 16384 tokens), which then stay in its L2.
+// lookup_scatter_sorted_kernel: one workgroup per (table, 64-column slice).  What bounds it is the compute unit's vector memory path: every
+// pair's 256 bytes of g come out of the L2, random rows of any length at 33 TB/s where nothing else is asked for (57 bytes a clock of a
+// compute unit), and it does so with the least beside them:
+//   * 64 columns, so that a list is read once per 256 bytes of a row.  A slice of 16384 rows is then 4 MB, as much as an XCD's L2, and
+//     its tokens are two lists whose rows are walked one after the other (as one list 275 -> 296 us at 16384 x 128 x 768); four lists
+//     cost more bucket ends than they give (300).
+//   * A list is cut into equal pieces, one per wavefront, whatever the bucket sizes (a skewed code distribution costs nothing).  A
+//     wavefront takes four entries a step: lane group q = lane / 16 has entry q and its sixteen lanes the 256 bytes.  Entries
+//     reach their lanes by DPP (through LDS, two permutes a step, it had 12.7 vector instructions a kilobyte for 9.3), and eight steps' loads are in flight all the
+//     time: the register of a step that is done is loaded for the step eight on.
+//   * A bucket ends between any two entries: then a step's lane groups are split by selects.  (Lists padded to whole steps cost 5 % of the
+//     reads at 64 pairs a row and 18 % at 16.)
+//   * A bucket's sum goes to LDS, where its row holds what earlier lists gave, and the rows are written at the end, whole: no store sits
+//     among the loads (the counter that loads are waited for with counts stores too), no zero-fill and no atomics.  Buckets cut by
+//     a piece boundary go to slots, and the wavefront in whose piece one ends adds its parts in order.  The sum order is fixed
+//     (run-to-run reproducible), and eight partial sums of a bucket (four lane groups, even and odd steps) keep its error where it was.
+// Eight wavefronts a workgroup, two of them a compute unit for their LDS; 12 or 16 wavefronts are slower (285, 310 us).  All launches,
+// before (padded lists of 16384 tokens, 32 columns, rows stored as they end) -> now: 16384 x 128 x 768 331 -> 305 us, x 512 221 -> 204; 32768 x 128 x 512
+// 446 -> 413; 8192 x 128 x 768 194 -> 152; 4096 x 128 x 768 140 -> 95, x 512 92 -> 73; 16384 x 512 x 1024 1507 -> 1514.  What is left at 16384 x 128 x 768, taken
+// apart: without bucket ends -12 us, with lists from the L2 -28, rows from the L1 -47, all three 228 of 285, of which 25 to 35 are starts and ends of workgroups in step
+// with each other.  Fetching the lists' lines or the next list's rows ahead through the scalar cache gives nothing, nor does a
+// workgroup that stays for several slices.
 #include "lffn_common.h"
+
+#include <climits>
 
 namespace {
 
@@ -45,12 +55,14 @@ constexpr int SORT_WG = 1024;
 constexpr int SORT_WAVES = SORT_WG / 64;
 constexpr int MAX_S = 512;
 constexpr int XCDS = 8;
-constexpr int SORT_DEPTH = 16;      // batches of 64 tokens whose loads are in flight per wavefront
+constexpr int64_t CHUNK = 16384;    // tokens of a launch
+constexpr int64_t SUB = 8192;       // tokens whose pairs are sorted together, at most
+constexpr int SORT_DEPTH = CHUNK / SORT_WG;    // batches of 64 tokens whose loads are in flight per wavefront
 
-constexpr int MWG = 512;             // main kernel: threads per workgroup
-constexpr int MWAVES = MWG / 64;
-constexpr int SC = 32;               // columns per slice: 8 lanes x float4
-constexpr int U = 8;                 // steps (of eight tokens) per batch = one 64-entry load of pairs
+constexpr int SC = 64;               // columns per slice: 16 lanes x float4
+constexpr int WAVES = 8;            // of the sums' workgroup
+constexpr int MWG = WAVES * 64;
+constexpr int RING = 8;              // loads in flight per wavefront
 
 struct PrepArgs {
     const int32_t *code;   // [B, T]
@@ -58,7 +70,7 @@ struct PrepArgs {
     const float *g;        // [B, Do]
     uint16_t *code_t;      // [T, Bp]
     float *score_t;        // [T, Bp]
-    float *g_packed;       // [Do / SC][B + 1][SC], the last row zero
+    float *g_packed;       // [ceil(Do / SC)][B + 1][SC], the last row zero
     float *sums;           // [ceil((B + 1) / PACK_TOKENS), Do] or null: column sums of the rows of g that a workgroup copies
     int64_t B, Bp;
     int T, S, Do, tiles_t;
@@ -103,7 +115,7 @@ __global__ __launch_bounds__(256) void lookup_prep_kernel(PrepArgs a) {
 constexpr int PACK_TOKENS = 32;      // rows of g per workgroup of the slice-major copy
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy); row B is the padding's.  A thread has four
+// PACK_TOKENS rows of g, copied to the slice-major layout (workgroup `blk` of the copy); row B is zeros.  A thread has four
 // columns of every G-th row, so that their sum (the output bias's gradient) is a few additions and a pass over LDS (a
 // launch of its own for them took 14 us at 16384 x 768, this one is no longer for it).  g is read nontemporally, since the copy is
 // what is read from here on: training step at 16384 x 768 745 -> 738 us.
@@ -154,30 +166,29 @@ __device__ __forceinline__ void pack_rows(const PrepArgs &a, int64_t blk) {
 struct SortArgs {
     const uint16_t *code;  // [T, Bp], masked
     const float *score;    // [T, Bp]
-    uint2 *pairs;          // [T, stride] (token, score bits)
-    int32_t *off8;         // [T, S + 1] bucket starts, in units of eight entries
-    int64_t B, Bp, stride;
-    int T, S, nbits;
-    int stage;             // the sorted list is collected in LDS and written out in whole lines (it fits: S <= 256)
+    uint2 *pairs;          // [subs, T, stride] (token, counted from the list's first on, and score bits)
+    int32_t *off;          // [subs, T, S + 2] bucket starts in a list and its length; where the list starts, in units of eight entries
+    int64_t B, Bp, sub_len, stride;      // list `sub` has the tokens [sub * sub_len, (sub + 1) * sub_len)
+    int T, S, nbits, subs;
 };
 
+// The lists of table t: one, or two, to each half of the wavefronts one.
 __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
     extern __shared__ int sm[];
-    const int S = a.S;
+    const int S = a.S, waves = SORT_WAVES / a.subs;      // of a list
     int *hist = sm;                    // [SORT_WAVES][S]: counts, then running write positions
-    int *count = hist + SORT_WAVES * S;
-    int *start = count + S;            // padded bucket starts (entries)
-    int *total = start + S;
-    float *sc_s = reinterpret_cast<float *>(total + 4);                       // [stride] scores of the sorted list
-    unsigned short *tok_s = reinterpret_cast<unsigned short *>(sc_s + a.stride);   // [stride] tokens
+    int *start = hist + SORT_WAVES * S;                                        // [subs][S] bucket starts (entries)
+    float *sc_s = reinterpret_cast<float *>(start + a.subs * S);                // [subs * stride] scores of the sorted lists
+    unsigned short *tok_s = reinterpret_cast<unsigned short *>(sc_s + a.subs * a.stride);   // [subs * stride] tokens
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int sub = wave / waves;
     const uint16_t *code = a.code + (size_t)t * a.Bp;
     const float *score = a.score + (size_t)t * a.Bp;
     for (int q = tid; q < SORT_WAVES * S; q += SORT_WG) hist[q] = 0;
     __syncthreads();
 
-    // A wavefront takes up to SORT_DEPTH batches of 64 consecutive tokens (the launch keeps B within 1024 * SORT_DEPTH).
+    // A wavefront takes up to SORT_DEPTH batches of 64 consecutive tokens (a list's length is a multiple of its wavefronts').
     // Their codes and scores are loaded once, all loads in flight together, and stay in registers through both
     // passes, as does every token's rank among the tokens of its batch with the same code (from ballots over
     // the code bits): the first pass counts a batch's codes once per code (the lowest lane of each adds the
@@ -214,23 +225,24 @@ __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
         if (live && rank == 0) myh[c] += cnt;
     }
     __syncthreads();
-    for (int c = tid; c < S; c += SORT_WG) {
+    for (int i = tid; i < a.subs * S; i += SORT_WG) {
+        const int w0 = i / S * waves, c = i % S;
         int sum = 0;
-        for (int w = 0; w < SORT_WAVES; ++w) {
+        for (int w = w0; w < w0 + waves; ++w) {
             const int v = hist[w * S + c];
             hist[w * S + c] = sum;
             sum += v;
         }
-        count[c] = sum;
-        start[c] = (sum + 7) & ~7;
+        start[i] = sum;
     }
     __syncthreads();
-    if (wave == 0) {                   // exclusive scan of the padded counts
+    if (wave % waves == 0) {           // exclusive scan of the counts
+        int *mine = start + sub * S;
         const int per_lane = (S + 63) / 64;
         int loc = 0;
         for (int k = 0; k < per_lane; ++k) {
             const int i = lane * per_lane + k;
-            if (i < S) loc += start[i];
+            if (i < S) loc += mine[i];
         }
         int inc = loc;
         for (int d = 1; d < 64; d <<= 1) {
@@ -241,54 +253,42 @@ __device__ __forceinline__ void sort_table(const SortArgs &a, const int t) {
         for (int k = 0; k < per_lane; ++k) {
             const int i = lane * per_lane + k;
             if (i < S) {
-                const int v = start[i];
-                start[i] = run;
+                const int v = mine[i];
+                mine[i] = run;
                 run += v;
             }
         }
-        if (lane == 63) *total = inc;
     }
     __syncthreads();
-    for (int c = tid; c < S; c += SORT_WG) {
-        const int o = start[c];
-        a.off8[(size_t)t * (S + 1) + c] = o >> 3;
-        for (int w = 0; w < SORT_WAVES; ++w) hist[w * S + c] += o;
+    for (int i = tid; i < a.subs * S; i += SORT_WG) {
+        const int q = i / S, c = i % S, o = start[i];
+        a.off[((size_t)q * a.T + t) * (S + 2) + c] = o;
+        for (int w = q * waves; w < (q + 1) * waves; ++w) hist[w * S + c] += q * (int)a.stride + o;
     }
-    if (tid == 0) a.off8[(size_t)t * (S + 1) + S] = *total >> 3;
+    if (tid < a.subs) {
+        const int64_t list = (int64_t)tid * a.T + t;
+        a.off[list * (S + 2) + S] = (int)min(a.B - tid * a.sub_len, a.sub_len);
+        a.off[list * (S + 2) + S + 1] = (int)(list * a.stride / 8);
+    }
     __syncthreads();
 
-    uint2 *out = a.pairs + (size_t)t * a.stride;
 #pragma unroll
     for (int k = 0; k < SORT_DEPTH; ++k) {
         if (lo + 64 * k >= hi) continue;                         // uniform
         if (cv[k] >= 0) {
             const int c = cv[k], rank = rk[k] & 0xff, cnt = rk[k] >> 8;
             const int base = myh[c];                              // all lanes of a code read before its last lane writes
-            if (a.stage) {                                        // uniform
-                tok_s[base + rank] = (unsigned short)(lo + 64 * k + lane);
-                sc_s[base + rank] = sv[k];
-            } else {
-                out[base + rank] = make_uint2((unsigned)(lo + 64 * k + lane), __float_as_uint(sv[k]));
-            }
+            tok_s[base + rank] = (unsigned short)(lo - sub * a.sub_len + 64 * k + lane);
+            sc_s[base + rank] = sv[k];
             if (rank == cnt - 1) myh[c] = base + cnt;
         }
     }
     __syncthreads();
-    for (int c = tid; c < S; c += SORT_WG) {
-        const int n = count[c], o = start[c];
-        for (int p = n; p < ((n + 7) & ~7); ++p) {
-            if (a.stage) {
-                tok_s[o + p] = (unsigned short)a.B;
-                sc_s[o + p] = 0.f;
-            } else {
-                out[o + p] = make_uint2((unsigned)a.B, 0u);
-            }
-        }
+    for (int q = 0; q < a.subs; ++q) {
+        const int n = (int)min(a.B - q * a.sub_len, a.sub_len), first = q * (int)a.stride;
+        uint2 *out = a.pairs + ((int64_t)q * a.T + t) * a.stride;
+        for (int i = tid; i < n; i += SORT_WG) out[i] = make_uint2((unsigned)tok_s[first + i], __float_as_uint(sc_s[first + i]));
     }
-    if (!a.stage) return;                                     // uniform
-    __syncthreads();
-    const int n_out = *total;
-    for (int i = tid; i < n_out; i += SORT_WG) out[i] = make_uint2((unsigned)tok_s[i], __float_as_uint(sc_s[i]));
 }
 
 // workgroups [0, nsort): the sort of one table each; the others: PACK_TOKENS rows of the copy of g each
@@ -298,210 +298,303 @@ __global__ __launch_bounds__(SORT_WG) void lookup_sort_pack_kernel(SortArgs sa, 
 }
 
 struct SortedArgs {
-    const uint2 *pairs;    // table t's list starts at t * stride
-    const int32_t *off8;   // [T, S + 1] bucket starts inside that list, in units of eight entries
-    const float *g;        // [Do / SC][B + 1][SC]
+    const uint2 *pairs;
+    const int32_t *off;    // [subs, T, S + 2] as in SortArgs
+    const float *g;        // [nslices][B + 1][SC], the last row zero
     float *out;            // [rows, Do]; table t's rows from t * S on
-    int64_t stride, rows;
-    unsigned last_token;   // B: the padding's
-    int T, S, Do, nslices, accumulate;
+    int64_t rows;
+    int B, sub_len;        // tokens, CHUNK at most, and those of a list
+    int T, S, Do, nslices, subs, per_xcd, accumulate;
     int more;              // a later launch adds to these rows
 };
 
 __device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
 
-// v + (v of the lane 16 / 32 positions away): gfx950's row and half-wave swaps, no LDS traffic
-__device__ __forceinline__ float add_xor16(float v) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+// Sum over the four lane groups of a float4 that every lane holds for its four columns: two values change places with each swap, so that
+// both sums take one addition, and a lane ends with one of its four (6 instructions; one value after the other takes 16).  Lane
+// 16 r + i has column 4 i + {0, 2, 1, 3}[r].
+__device__ __forceinline__ float sum_swapped32(float x, float y) {     // lanes 0-31: x of both halves, 32-63: y
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ float add_xor32(float v) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+__device__ __forceinline__ float sum_swapped16(float x, float y) {     // rows of 16: x of rows 0 and 1, y of both, x of rows 2 and 3, y of both
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-// v + (v of lane ^ 8): a DPP rotation by eight inside the 16-lane row
-__device__ __forceinline__ float add_xor8(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true));
+__device__ __forceinline__ float sum_groups(float4 v) { return sum_swapped16(sum_swapped32(v.x, v.y), sum_swapped32(v.z, v.w)); }
+
+// What lane u of a row of sixteen lanes holds, in all of them (a DPP operand of the instruction that uses it).
+__device__ __forceinline__ int row_pick(int v, int u) {
+#define LFFN_PICK(n) case n: return __builtin_amdgcn_mov_dpp(v, 0x150 + n, 0xF, 0xF, true)
+    switch (u) {
+        LFFN_PICK(0); LFFN_PICK(1); LFFN_PICK(2); LFFN_PICK(3); LFFN_PICK(4); LFFN_PICK(5); LFFN_PICK(6); LFFN_PICK(7);
+        LFFN_PICK(8); LFFN_PICK(9); LFFN_PICK(10); LFFN_PICK(11); LFFN_PICK(12); LFFN_PICK(13); LFFN_PICK(14);
+        default: return __builtin_amdgcn_mov_dpp(v, 0x15F, 0xF, 0xF, true);
+    }
+#undef LFFN_PICK
 }
 
-// sum over the eight lane groups; afterwards every lane holds the total of its column group
-__device__ __forceinline__ float4 sum_groups(float4 v) {
-    v.x = add_xor32(add_xor16(add_xor8(v.x)));
-    v.y = add_xor32(add_xor16(add_xor8(v.y)));
-    v.z = add_xor32(add_xor16(add_xor8(v.z)));
-    v.w = add_xor32(add_xor16(add_xor8(v.w)));
-    return v;
-}
-
-// ADD: the sums are added to what a.out holds.  They are kept in LDS, and the rows read, added to and written at the end, eight of a
-// thread's pieces in flight: read where a bucket ends, every row was waited for with all that was in flight behind it (the second
-// 16384 tokens of 128 tables of 512 columns 264 -> 214 us; requested when the bucket begins 255, as atomic additions 249).
+// ADD: the sums are added to what a.out holds.
 template <bool ADD>
-__global__ __launch_bounds__(MWG) void lookup_scatter_sorted_kernel(SortedArgs a) {
-    extern __shared__ int sm[];
-    int *off = sm;                                            // [S + 1]
-    int *flag = off + ((a.S + 1 + 3) & ~3);                     // [MWAVES][4]: head code, head closes, tail code
-    float *slot = reinterpret_cast<float *>(flag + MWAVES * 4);   // [MWAVES][2][SC]
-    float *row_s = slot + MWAVES * 2 * SC;                      // ADD: [S][SC]
+__global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(SortedArgs a) {
+    extern __shared__ float4 lds4[];
+    float *row_s = reinterpret_cast<float *>(lds4);             // [S][SC]: the rows' sums
+    float *slot = row_s + a.S * SC;                             // [WAVES][2][SC]
+    int *flag_s = reinterpret_cast<int *>(slot + WAVES * 2 * SC);    // [2][WAVES][4]: head bucket, it closes here, tail bucket
+    int *off_s = flag_s + 2 * WAVES * 4;                        // [2][S + 2]
 
-    const int xcd = blockIdx.x % XCDS, idx = blockIdx.x / XCDS;
-    const int slice = xcd + XCDS * (idx / a.T);
-    const int t = idx % a.T;
-    if (slice >= a.nslices) return;                           // uniform over the workgroup
-    const int S = (int)min<int64_t>(a.S, a.rows - (int64_t)t * a.S);      // the last table of a row count that a.S does not divide
+    // neighbouring tables of a slice on one XCD
+    const int unit = (int)(blockIdx.x % XCDS) * a.per_xcd + (int)(blockIdx.x / XCDS);
+    if (unit >= a.T * a.nslices) return;                      // uniform over the workgroup
+    const int slice = unit / a.T, t = unit % a.T;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int grp = lane >> 3, j = lane & 7;
-    for (int q = tid; q <= S; q += MWG) off[q] = a.off8[(size_t)t * (a.S + 1) + q];
-    if (tid < MWAVES * 4) flag[tid] = -1;
+    const int grp = lane >> 4, i16 = lane & 15;
+    const int my_col = i16 * 4 + (lane >> 5) + ((lane >> 3) & 2);
+    const int slot0 = (a.S + wave * 2) * SC + my_col;          // (a column's place in the LDS as a whole: one index serves rows and slots)
+
+    constexpr int OFFS = (MAX_S + 2 + MWG - 1) / MWG;
+    int next_off[OFFS];                                       // a thread's offsets of a list
+    auto load_offsets = [&](int sub) {
+#pragma unroll
+        for (int k = 0; k < OFFS; ++k)
+            if (tid + k * MWG < a.S + 2) next_off[k] = a.off[((size_t)sub * a.T + t) * (a.S + 2) + tid + k * MWG];
+    };
+    auto keep_offsets = [&](int *off) {
+#pragma unroll
+        for (int k = 0; k < OFFS; ++k)
+            if (tid + k * MWG < a.S + 2) off[tid + k * MWG] = next_off[k];
+    };
+    load_offsets(0);
+    for (int q = tid; q < a.S * (SC / 4); q += MWG) lds4[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    keep_offsets(off_s);
     __syncthreads();
 
-    float *orow = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC + j * 4;     // + code * Do
+    // What a wavefront knows of its piece of the list at hand, and its first pairs.
+    int sub = 0;
+    int e_lo, e_hi, cur, first_end, ends, head_bucket, tokens;
+    const uint2 *pp;
+    uint2 pr0, pr1;
+    // The ends of 64 buckets, one a lane, so that nothing waits for LDS at a bucket's end; those that the piece does not reach lie
+    // beyond every entry.
+    auto load_ends = [&]() {
+        int v = off_s[(sub & 1) * (a.S + 2) + min(first_end + lane, a.S)];
+        v = v < e_hi ? v : INT_MAX;
+        asm volatile("" : "+v"(v));                           // (waited for here, not where one is read)
+        return v;
+    };
+    // 64 pairs as they lie, past the piece's end weight 0 and the row of zeros
+    auto load_pairs = [&](int e) { return pp[min(e + lane, e_hi - 1)]; };
+    auto begin_list = [&]() {
+        const int *off = off_s + (sub & 1) * (a.S + 2);
+        const int n = __builtin_amdgcn_readfirstlane(off[a.S]), pieces = (n + 7) >> 3;
+        e_lo = (int)((int64_t)wave * pieces / WAVES) * 8;
+        e_hi = min((int)((int64_t)(wave + 1) * pieces / WAVES) * 8, n);
+        tokens = a.B - sub * a.sub_len;                       // the row of zeros, from the list's first token on
+        pp = a.pairs + (int64_t)__builtin_amdgcn_readfirstlane(off[a.S + 1]) * 8;
+        head_bucket = -1;
+        if (e_lo >= e_hi) return;                             // uniform
+        pr0 = load_pairs(e_lo);
+        pr1 = load_pairs(min(e_lo + 64, e_hi - 1));
+        // the bucket holding entry e_lo: the last c with off[c] <= e_lo
+        int lo = 0, hi = a.S;                                 // invariant: off[lo] <= e_lo < off[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (off[mid] <= e_lo) lo = mid; else hi = mid;
+        }
+        cur = __builtin_amdgcn_readfirstlane(lo);
+        first_end = cur + 1;
+        ends = load_ends();
+        head_bucket = __builtin_amdgcn_readfirstlane(off[cur] < e_lo ? cur : -1);
+    };
+    begin_list();
+
+    for (;;) {
+        const bool last_list = sub + 1 == a.subs;
+        if (!last_list) load_offsets(sub + 1);                // the next list's, on their way while this one is walked
+        int *flag = flag_s + (sub & 1) * WAVES * 4;
+        int closes = 0, goes_on = 0;
+        if (e_lo < e_hi) {
+            const int *off = off_s + (sub & 1) * (a.S + 2);
+            int next_b = __builtin_amdgcn_readlane(ends, 0);
+            closes = head_bucket >= 0 && __builtin_amdgcn_readfirstlane(off[cur + 1]) <= e_hi ? 1 : 0;
+            // where the sum of the bucket at hand goes: its row, or, if it began in an earlier piece, this wavefront's first slot
+            int dst = head_bucket >= 0 ? slot0 : cur * SC + my_col;
+            float before = head_bucket >= 0 ? 0.f : row_s[cur * SC + my_col];      // what the row holds: the sum over earlier lists
+            const char *gs = reinterpret_cast<const char *>(a.g + ((size_t)slice * (a.B + 1) + (size_t)sub * a.sub_len) * SC);
+            float acc[2][4];                                  // the even and the odd steps' sums
+            auto clear = [&]() {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[e >> 2][e & 3] = 0.f;
+            };
+            clear();
+            auto flush = [&]() {
+                const float v = sum_groups(make_float4(acc[0][0] + acc[1][0], acc[0][1] + acc[1][1], acc[0][2] + acc[1][2], acc[0][3] + acc[1][3]));
+                row_s[dst] = before + v;
+            };
+            // Lane i of group q gets the pair that the group takes in step i (loaded so, sixteen lanes would be sixteen lines).
+            auto turned = [&](unsigned v) { return __builtin_amdgcn_ds_bpermute((i16 * 4 + grp) * 4, (int)v); };
+            // (a launch's tokens: 32 bits hold the offset of a row in the slice)
+            auto rows_of = [&](uint2 v, int e) {
+                return turned((e + lane < e_hi ? min(v.x, (unsigned)tokens) : (unsigned)tokens) * unsigned(SC * 4));
+            };
+            auto weights_of = [&](uint2 v, int e) { return turned(e + lane < e_hi ? v.y : 0u); };
+            auto load_row = [&](int rows, int u) {
+                return *reinterpret_cast<const float4 *>(gs + (unsigned)(row_pick(rows, u) + i16 * 16));
+            };
+            auto add = [&](float (&to)[4], float w, float4 v, bool live) {
+                const float x = fmaf(w, v.x, to[0]), y = fmaf(w, v.y, to[1]), z = fmaf(w, v.z, to[2]), u = fmaf(w, v.w, to[3]);
+                to[0] = live ? x : to[0];
+                to[1] = live ? y : to[1];
+                to[2] = live ? z : to[2];
+                to[3] = live ? u : to[3];
+            };
+            // four entries from e on, one per lane group; a bucket may end before any of them
+            auto take = [&](int e, int odd, float w, float4 v) {
+                if (next_b >= e + 4) {                        // uniform
+                    add(acc[odd], w, v, true);
+                    return;
+                }
+                int from = 0;
+                do {
+                    const int to = next_b - e;
+                    add(acc[odd], w, v, grp >= from && grp < to);      // (selected, not branched on: all control flow is the wavefront's)
+                    flush();
+                    const int end = next_b;
+                    do {
+                        ++cur;
+                        if (cur + 1 - first_end == 64) {
+                            first_end = cur + 1;
+                            ends = load_ends();
+                        }
+                        next_b = __builtin_amdgcn_readlane(ends, cur + 1 - first_end);
+                    } while (next_b == end);                  // skip codes without tokens
+                    dst = cur * SC + my_col;
+                    before = row_s[dst];
+                    clear();
+                    from = to;
+                } while (next_b < e + 4);
+                add(acc[odd], w, v, grp >= from);
+            };
+
+            int rows = rows_of(pr0, e_lo), w = weights_of(pr0, e_lo);
+            float4 gv[RING];
+#pragma unroll
+            for (int u = 0; u < RING; ++u) gv[u] = load_row(rows, u);
+            int e = e_lo;
+            for (; e + 64 < e_hi; e += 64) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    take(e + 4 * u, u & 1, __int_as_float(row_pick(w, u)), gv[u]);
+                    gv[u] = load_row(rows, u + 8);
+                }
+                rows = rows_of(pr1, e + 64);
+                const int w_next = weights_of(pr1, e + 64);
+                pr1 = load_pairs(min(e + 128, e_hi - 1));
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    take(e + 32 + 4 * u, u & 1, __int_as_float(row_pick(w, u + 8)), gv[u]);
+                    gv[u] = load_row(rows, u);
+                }
+                w = w_next;
+            }
+            if (e + 32 < e_hi) {                              // uniform
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    take(e + 4 * u, u & 1, __int_as_float(row_pick(w, u)), gv[u]);
+                    gv[u] = load_row(rows, u + 8);
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (e + 32 + 4 * u < e_hi) take(e + 32 + 4 * u, u & 1, __int_as_float(row_pick(w, u + 8)), gv[u]);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (e + 4 * u < e_hi) take(e + 4 * u, u & 1, __int_as_float(row_pick(w, u)), gv[u]);
+            }
+            goes_on = cur != head_bucket && __builtin_amdgcn_readfirstlane(off[cur + 1]) > e_hi ? 1 : 0;      // in the next piece
+            dst = goes_on ? slot0 + SC : dst;
+            before = goes_on ? 0.f : before;
+            flush();
+        }
+        flag[wave * 4 + 0] = head_bucket;                     // (every lane the same)
+        flag[wave * 4 + 1] = closes;
+        flag[wave * 4 + 2] = goes_on ? cur : -1;
+        if (!last_list) keep_offsets(off_s + (~sub & 1) * (a.S + 2));
+        __syncthreads();
+        // a bucket cut by piece boundaries: the wavefront in whose piece it ends adds its parts
+        if (closes) {                                         // uniform
+            float sum = slot[wave * 2 * SC + lane];
+            for (int k = wave - 1; k >= 0; --k) {
+                if (__builtin_amdgcn_readfirstlane(flag[k * 4 + 2]) >= 0) {
+                    sum = slot[(k * 2 + 1) * SC + lane] + sum;
+                    break;
+                }
+                if (__builtin_amdgcn_readfirstlane(flag[k * 4 + 0]) >= 0) sum = slot[k * 2 * SC + lane] + sum;
+            }
+            row_s[head_bucket * SC + lane] += sum;
+        }
+        ++sub;
+        if (!last_list) begin_list();
+        __syncthreads();
+        if (last_list) break;
+    }
+
     // Rows that nothing adds to any more go out nontemporally: in the caches they would take the place of g.  Read again next, 32768 x 512,
     // that costs 7 us of 1490.  With a reader behind the pass, unlike the lists and the sums of few pairs (lffn_rows_written_past_caches), it
     // costs no more than it gives: a training step of 2500 tokens and more of 128 to 512 tables takes the same alone and with SGD, clipping
     // or Adam behind it; the operator's pass, plainly -> nontemporally, alone, with SGD, with Adam:
     //   4096 x 128 x 512  231 -> 226 (219 for 229 where the passes' results stay), 270 -> 264, 317 -> 318    3000 x 128 x 512  206 -> 204, 245 -> 239, 295 -> 298
     //   8192 x 64 x 512  217 -> 202, 232 -> 240, 283 -> 284    2500 x 128 x 768  266 -> 265, 332 -> 337, 462 -> 462    8192 x 256 x 512  601 -> 586, 671 -> 662
-    auto store_row = [&](float *p, float4 v) {
-        if (a.more) *reinterpret_cast<float4 *>(p) = v;                            // uniform
-        else __builtin_nontemporal_store((f32x4){v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4 *>(p));
-    };
-    if (!ADD)                                                 // rows no token points at
-        for (int q = tid; q < S * 8; q += MWG) {
-            const int c = q >> 3;
-            if (off[c + 1] == off[c])
-                *reinterpret_cast<float4 *>(a.out + ((size_t)t * a.S + c) * a.Do + (size_t)slice * SC + (q & 7) * 4) =
-                    make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-
-    const int n0 = off[0], n8 = off[S] - n0;
-    const int s_lo = n0 + (int)((int64_t)wave * n8 / MWAVES), s_hi = n0 + (int)((int64_t)(wave + 1) * n8 / MWAVES);
-    if (s_lo < s_hi) {
-        // the bucket holding step s_lo: the last c with off[c] <= s_lo
-        int lo = 0, hi = S;                                   // invariant: off[lo] <= s_lo < off[hi]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (off[mid] <= s_lo) lo = mid; else hi = mid;
-        }
-        int cur = __builtin_amdgcn_readfirstlane(lo);
-        int next_b = __builtin_amdgcn_readfirstlane(off[cur + 1]);
-        bool head = off[cur] < s_lo;                          // the bucket began in an earlier piece
-        const uint2 *pp = a.pairs + (size_t)t * a.stride;
-        const float *gcol = a.g + (size_t)slice * SC * (size_t(a.last_token) + 1) + j * 4;
-        const int64_t last_entry = (int64_t)s_hi * 8 - 1;
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-
-        auto flush = [&](bool continues) {
-            const float4 v = sum_groups(acc);
-            if (head) {
-                if (lane < 8) *reinterpret_cast<float4 *>(slot + (wave * 2 + 0) * SC + j * 4) = v;
-                if (lane == 0) { flag[wave * 4 + 0] = cur; flag[wave * 4 + 1] = continues ? 0 : 1; }
-            } else if (continues) {
-                if (lane < 8) *reinterpret_cast<float4 *>(slot + (wave * 2 + 1) * SC + j * 4) = v;
-                if (lane == 0) flag[wave * 4 + 2] = cur;
-            } else if (lane < 8) {
-                if (ADD) *reinterpret_cast<float4 *>(row_s + cur * SC + j * 4) = v;
-                else store_row(orow + (size_t)cur * a.Do, v);
-            }
-            head = false;
-            acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        };
-
-        uint2 pr = pp[min((int64_t)s_lo * 8 + lane, last_entry)];
-        for (int step0 = s_lo; step0 < s_hi; step0 += U) {
-            float4 gv[U];
-            float sc[U];
+    const int S = (int)min<int64_t>(a.S, a.rows - (int64_t)t * a.S);      // the last table of a row count that a.S does not divide
+    if (i16 * 4 >= a.Do - slice * SC) return;                 // (the last slice may be half a one)
+    constexpr int DEPTH = 4;
+    float *const first = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC + i16 * 4;
+    for (int r0 = tid >> 4; r0 < S; r0 += MWG / 16 * DEPTH) {
+        float4 v[DEPTH];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const unsigned tok = min(__shfl(pr.x, u * 8 + grp), a.last_token);
-                sc[u] = __uint_as_float(__shfl(pr.y, u * 8 + grp));
-                gv[u] = *reinterpret_cast<const float4 *>(gcol + (size_t)tok * SC);
-            }
-            if (step0 + U < s_hi) pr = pp[min((int64_t)(step0 + U) * 8 + lane, last_entry)];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int step = step0 + u;
-                if (step < s_hi) {                            // uniform
-                    if (step == next_b) {                     // uniform: the bucket ended with the step before
-                        flush(false);
-                        do {
-                            ++cur;
-                            next_b = __builtin_amdgcn_readfirstlane(off[cur + 1]);
-                        } while (next_b == step && cur < S - 1);   // skip codes without tokens
-                    }
-                    acc.x = fmaf(sc[u], gv[u].x, acc.x);
-                    acc.y = fmaf(sc[u], gv[u].y, acc.y);
-                    acc.z = fmaf(sc[u], gv[u].z, acc.z);
-                    acc.w = fmaf(sc[u], gv[u].w, acc.w);
-                }
-            }
+        for (int k = 0; k < DEPTH; ++k) {
+            const int row = r0 + k * (MWG / 16);
+            if (ADD && row < S) v[k] = *reinterpret_cast<const float4 *>(first + (size_t)row * a.Do);
         }
-        flush(next_b > s_hi);
-    }
-    __syncthreads();
-
-    // buckets cut by piece boundaries: add their parts in order
-    if (tid < 8) {
-        float4 pend = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int w = 0; w < MWAVES; ++w) {
-            const int hc = flag[w * 4 + 0];
-            if (hc >= 0) {
-                pend = add4(pend, *reinterpret_cast<const float4 *>(slot + (w * 2 + 0) * SC + j * 4));
-                if (flag[w * 4 + 1] == 1) {
-                    *reinterpret_cast<float4 *>(ADD ? row_s + hc * SC + j * 4 : orow + (size_t)hc * a.Do) = pend;
-                    pend = make_float4(0.f, 0.f, 0.f, 0.f);
-                }
-            }
-            if (flag[w * 4 + 2] >= 0) pend = *reinterpret_cast<const float4 *>(slot + (w * 2 + 1) * SC + j * 4);
-        }
-    }
-    if constexpr (ADD) {
-        __syncthreads();
-        constexpr int DEPTH = 8;
-        float *const first = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC;
-        for (int q0 = tid; q0 < S * 8; q0 += MWG * DEPTH) {
-            float4 v[DEPTH];
-            bool live[DEPTH];
 #pragma unroll
-            for (int i = 0; i < DEPTH; ++i) {
-                const int q = q0 + i * MWG, row = min(q >> 3, S - 1);
-                live[i] = q < S * 8 && off[row + 1] > off[row];          // rows no token points at stay as they are
-                if (live[i]) v[i] = *reinterpret_cast<const float4 *>(first + (size_t)row * a.Do + (q & 7) * 4);
-            }
-#pragma unroll
-            for (int i = 0; i < DEPTH; ++i) {
-                const int q = q0 + i * MWG;
-                if (live[i])
-                    store_row(first + (size_t)(q >> 3) * a.Do + (q & 7) * 4, add4(v[i], *reinterpret_cast<const float4 *>(row_s + q * 4)));
-            }
+        for (int k = 0; k < DEPTH; ++k) {
+            const int row = r0 + k * (MWG / 16);
+            if (row >= S) continue;
+            const float4 sum = lds4[row * (SC / 4) + i16];
+            v[k] = ADD ? add4(v[k], sum) : sum;
+            float *p = first + (size_t)row * a.Do;
+            if (a.more) *reinterpret_cast<float4 *>(p) = v[k];                     // uniform
+            else __builtin_nontemporal_store((f32x4){v[k].x, v[k].y, v[k].z, v[k].w}, reinterpret_cast<f32x4 *>(p));
         }
     }
 }
 
 // one workgroup per (table of a.S rows, slice)
-int launch_sorted(SortedArgs a, hipStream_t st) {
-    const int64_t per_xcd = (int64_t)((a.nslices + XCDS - 1) / XCDS) * a.T;
-    const size_t lds = (((a.S + 1 + 3) & ~3) + MWAVES * 4) * sizeof(int) + size_t(MWAVES) * 2 * SC * sizeof(float);
-    const dim3 grid((unsigned)(per_xcd * XCDS));
-    if (a.accumulate) {
-        const size_t add_lds = lds + size_t(a.S) * SC * sizeof(float);
-        static LdsGrant granted;
-        if (add_lds > 65000 && !lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<true>), add_lds, granted))
-            return LFFN_ERR_LAUNCH;
-        hipLaunchKernelGGL(lookup_scatter_sorted_kernel<true>, grid, dim3(MWG), add_lds, st, a);
-    } else {
-        hipLaunchKernelGGL(lookup_scatter_sorted_kernel<false>, grid, dim3(MWG), lds, st, a);
-    }
+template <bool ADD>
+int launch_sorted_form(SortedArgs a, hipStream_t st) {
+    const size_t lds = (size_t(a.S) + WAVES * 2) * SC * sizeof(float) + (2 * WAVES * 4 + size_t(2) * (a.S + 2)) * sizeof(int);
+    static LdsGrant granted;
+    if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD>), lds, granted)) return LFFN_ERR_LAUNCH;
+    a.per_xcd = (a.T * a.nslices + XCDS - 1) / XCDS;
+    hipLaunchKernelGGL(lookup_scatter_sorted_kernel<ADD>, dim3((unsigned)(a.per_xcd * XCDS)), dim3(MWG), lds, st, a);
     return lffn_launch_status();
 }
 
-inline int64_t pair_stride(int64_t B, int64_t S) { return ((B + 7) & ~int64_t(7)) + 8 * S; }
+int launch_sorted(const SortedArgs &a, hipStream_t st) {
+    return a.accumulate ? launch_sorted_form<true>(a, st) : launch_sorted_form<false>(a, st);
+}
+
+inline int64_t slices(int64_t Do) { return (Do + SC - 1) / SC; }
+// One list of a chunk's tokens, or two: then half of the sort's wavefronts have the first, and all of them as many batches of 64.
+inline int64_t sub_lists(int64_t Bc) { return Bc > SUB ? 2 : 1; }
+inline int64_t list_tokens(int64_t Bc) { return Bc > SUB ? (Bc + SORT_WG - 1) / SORT_WG * (SORT_WG / 2) : Bc; }
+inline int64_t pair_stride(int64_t Bc) { return (list_tokens(Bc) + 7) & ~int64_t(7); }
 
 inline bool sorted_supported(int64_t B, int64_t T, int64_t S, int64_t Do) {
-    return B >= 1 && T >= 1 && lffn_is_pow2(S) && S <= MAX_S && Do % SC == 0 && Do <= (1 << 20) &&
-           B <= (int64_t(1) << 31) - 1 && T <= (1 << 20) && T * ((Do / SC + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff;
+    return B >= 1 && T >= 1 && lffn_is_pow2(S) && S <= MAX_S && Do % 32 == 0 && Do <= (1 << 20) &&
+           B <= (int64_t(1) << 31) - 1 && T <= (1 << 20) && T * ((Do / 32 + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff;
 }
 
 inline int64_t pack_workgroups(int64_t Bc) { return (Bc + 1 + PACK_TOKENS - 1) / PACK_TOKENS; }
@@ -509,23 +602,23 @@ inline int64_t round16(int64_t v) { return (v + 15) & ~int64_t(15); }
 inline int64_t padded_tokens(int64_t B) { return (B + 63) & ~int64_t(63); }
 
 // Tokens are taken CHUNK at a time (later chunks add to the result of the earlier ones): a
-// 32-column slice of 16384 rows of g is 2 MB and stays in an XCD's 4 MB L2 while the
-// workgroups of that XCD walk it in 128 different orders; twice that no longer does.
-constexpr int64_t CHUNK = 16384;
+// list's 64 columns of 8192 rows of g are 2 MB and stay in an XCD's 4 MB L2 while the
+// workgroups of that XCD walk them in as many orders; twice that no longer does.
+static_assert(CHUNK <= 2 * SUB, "a chunk's tokens are one list or two");
 
 struct Workspace {
-    int64_t pairs, off8, code_t, score_t, g_packed, total;    // byte offsets
+    int64_t pairs, off, code_t, score_t, g_packed, total;    // byte offsets
 };
 
 inline Workspace workspace_layout(int64_t B, int64_t T, int64_t S, int64_t Do) {
     Workspace w{};
     const int64_t Bc = B < CHUNK ? B : CHUNK, Bp = padded_tokens(Bc);
     w.pairs = 0;
-    w.off8 = w.pairs + T * pair_stride(Bc, S) * 8;
-    w.code_t = w.off8 + round16(T * (S + 1) * 4);
+    w.off = w.pairs + sub_lists(Bc) * T * pair_stride(Bc) * 8;
+    w.code_t = w.off + round16(sub_lists(Bc) * T * (S + 2) * 4);
     w.score_t = w.code_t + round16(T * Bp * 2);
     w.g_packed = w.score_t + round16(T * Bp * 4);
-    w.total = w.g_packed + round16((Bc + 1) * Do * 4);
+    w.total = w.g_packed + (Bc + 1) * slices(Do) * SC * 4;
     return w;
 }
 
@@ -550,11 +643,11 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
     hipStream_t st = static_cast<hipStream_t>(stream);
     char *base = static_cast<char *>(workspace);
     uint2 *pairs = reinterpret_cast<uint2 *>(base + w.pairs);
-    int32_t *off8 = reinterpret_cast<int32_t *>(base + w.off8);
+    int32_t *off = reinterpret_cast<int32_t *>(base + w.off);
 
     for (int64_t c0 = 0; c0 < B; c0 += CHUNK) {
         const int64_t Bc = B - c0 < CHUNK ? B - c0 : CHUNK;
-        const int64_t stride = pair_stride(Bc, S), Bp = padded_tokens(Bc);
+        const int64_t stride = pair_stride(Bc), Bp = padded_tokens(Bc);
 
         PrepArgs pa{};
         pa.code = code + c0 * T; pa.score = score + c0 * T; pa.g = g + c0 * Do;
@@ -577,15 +670,12 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
             if (rc != LFFN_OK) return rc;
         }
         SortArgs sa{};
-        sa.code = pa.code_t; sa.score = pa.score_t; sa.pairs = pairs; sa.off8 = off8;
-        sa.B = Bc; sa.Bp = Bp; sa.stride = stride; sa.T = (int)T; sa.S = (int)S; sa.nbits = lffn_log2(S);
-        // histograms and bucket tables, then the sorted list itself (4 + 2 bytes per entry; tokens of a chunk fit 16 bits)
-        static_assert(CHUNK < 65536, "tokens of a chunk and the padding's are staged as 16-bit values");
-        static_assert(CHUNK <= int64_t(SORT_WG) * SORT_DEPTH, "a wavefront of the sort holds its tokens in registers");
-        const size_t tables_lds = (size_t(SORT_WAVES) * S + 2 * S + 4 + 4) * sizeof(int);
-        const size_t staged_lds = tables_lds + size_t(stride) * 6 + 16;
-        sa.stage = staged_lds <= 160 * 1024 ? 1 : 0;            // 512-row tables: the list goes straight to memory
-        size_t sort_lds = nsort ? (sa.stage ? staged_lds : tables_lds) : 0;
+        sa.code = pa.code_t; sa.score = pa.score_t; sa.pairs = pairs; sa.off = off;
+        sa.B = Bc; sa.Bp = Bp; sa.sub_len = list_tokens(Bc); sa.stride = stride;
+        sa.T = (int)T; sa.S = (int)S; sa.nbits = lffn_log2(S); sa.subs = (int)sub_lists(Bc);
+        // histograms and bucket starts, then the sorted lists themselves (4 + 2 bytes per entry)
+        static_assert(SUB <= 65536 && CHUNK % SORT_WG == 0, "a list's tokens are staged as 16-bit values, and held in registers");
+        size_t sort_lds = nsort ? size_t(SORT_WAVES + sa.subs) * S * sizeof(int) + size_t(sa.subs) * stride * 6 : 0;
         if (pa.sums && sort_lds < SORT_WG * sizeof(float4)) sort_lds = SORT_WG * sizeof(float4);
         static LdsGrant granted;
         if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_sort_pack_kernel), sort_lds, granted))
@@ -596,7 +686,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         if (rc != LFFN_OK) return rc;
 
         if (grad_score) {
-            // token b's 32 columns of slice s sit at g_packed + (s * (Bc + 1) + b) * 32
+            // token b's 64 columns of slice s sit at g_packed + (s * (Bc + 1) + b) * 64
             if (!lffn_internal_lookup_inner_quad_try(pa.code, pa.g_packed, SC, (Bc + 1) * SC, tables, grad_score + c0 * T, Bc, T, S,
                                                      Do, stream, &rc))
                 rc = lffn_lookup_inner_f32(pa.code, pa.g, tables, grad_score + c0 * T, Bc, T, S, Do, stream);
@@ -605,9 +695,9 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         if (!grad_tables) continue;
 
         SortedArgs ma{};
-        ma.pairs = pairs; ma.off8 = off8; ma.g = pa.g_packed; ma.out = grad_tables; ma.stride = stride; ma.rows = T * S;
-        ma.last_token = (unsigned)Bc;
-        ma.T = (int)T; ma.S = (int)S; ma.Do = (int)Do; ma.nslices = (int)(Do / SC);
+        ma.pairs = pairs; ma.off = off; ma.g = pa.g_packed; ma.out = grad_tables; ma.rows = T * S; ma.B = (int)Bc;
+        ma.T = (int)T; ma.S = (int)S; ma.Do = (int)Do; ma.nslices = (int)slices(Do); ma.subs = sa.subs;
+        ma.sub_len = (int)sa.sub_len;
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
         ma.more = c0 + CHUNK < B ? 1 : 0;
         rc = launch_sorted(ma, st);
@@ -671,9 +761,10 @@ extern "C" int lffn_lookup_backward_sums_rows(int64_t B, int64_t *rows) {
 // accumulation above needs the (token, weight) pairs listed row by row instead, which takes one integer atomic per pair:
 //   rows_rank_kernel    a pair's place among the pairs of its row: the value its atomic add on the row's counter returns, or a
 //                       workgroup's one such add for all its pairs of the row
-//   rows_claim_kernel   one workgroup per 256 rows (a "table" of the accumulation) scans their padded counts and takes that
-//                       much of the list; which table's part comes first does not matter
-//   rows_place_kernel   pairs into the list (and a row's padding, which names the zero row, by its first pair); other workgroups copy
+//   rows_claim_kernel   one workgroup per 256 rows (a "table" of the accumulation) scans their counts and takes that
+//                       much of the list; which table's part comes first does not matter (more than SUB tokens: as if each of their
+//                       two parts had rows of its own)
+//   rows_place_kernel   pairs into the list; other workgroups copy
 //                       g slice-major
 // The order inside a row is the order of arrival: sums differ from run to run in their last bit, as they did with
 // atomics.
@@ -685,19 +776,24 @@ struct RowsArgs {
     const int32_t *idx;    // [B, I]
     const float *w;        // [B, I]
     const void *g;         // [B, Dv] fp32 or half
-    int32_t *count;        // [tables * VT] pairs per row, then (one word) the list's end in units of eight entries
+    int32_t *count;        // [subs * tables * VT] pairs per row, then (one word) the lists' end in units of eight entries
     int32_t *rank;         // [B * I]
-    int32_t *off8;         // [tables, VT + 1]
+    int32_t *off;          // [subs * tables, VT + 2] as in SortArgs
     int32_t *flags;        // [TABLE_FLAGS] not zero where a row number lies outside its column's table, or null: not looked for
     uint2 *pairs;
     float *g_packed;       // [Dv / SC][B + 1][SC], the last row zero
     int64_t B, n, rows;
-    int I, Dv, tables, place_blocks;
+    int64_t sub_pairs;     // pairs of the tokens whose pairs are listed together (all of them or SUB tokens')
+    int I, Dv, tables, subs, place_blocks;
 };
 
 __device__ __forceinline__ int row_of(const RowsArgs &a, int64_t e) {
     const int64_t raw = a.idx[e], hi = a.rows - 1;
     return (int)(raw < 0 ? 0 : (raw > hi ? hi : raw));
+}
+// the place of pair e's counter: its row's, among those of its part of the tokens
+__device__ __forceinline__ int64_t counter_of(const RowsArgs &a, int64_t e) {
+    return (e >= a.sub_pairs ? (int64_t)a.tables * VT : 0) + row_of(a, e);
 }
 
 // The counters to zero; with flags, what table_form_kernel (gather.hip) leaves there for these row numbers.
@@ -726,7 +822,7 @@ __global__ __launch_bounds__(1024) void rows_zero_kernel(RowsArgs a, int64_t n4)
 
 __global__ __launch_bounds__(256) void rows_rank_kernel(RowsArgs a) {
     const int64_t stride = int64_t(gridDim.x) * 256;
-    for (int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) a.rank[e] = atomicAdd(a.count + row_of(a, e), 1);
+    for (int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) a.rank[e] = atomicAdd(a.count + counter_of(a, e), 1);
 }
 
 // The same for many tokens.  Row numbers as the layer forms them lie in table i in column i: then a workgroup has RANK_TOKENS tokens of
@@ -744,7 +840,7 @@ __global__ __launch_bounds__(RANK_WG) void rows_rank_tables_kernel(RowsArgs a, i
         for (int64_t e0 = int64_t(blockIdx.x) * RANK_WG + threadIdx.x; e0 < a.n; e0 += stride * EACH) {
             int rank[EACH];
 #pragma unroll
-            for (int k = 0; k < EACH; ++k) rank[k] = e0 + k * stride < a.n ? atomicAdd(a.count + row_of(a, e0 + k * stride), 1) : 0;
+            for (int k = 0; k < EACH; ++k) rank[k] = e0 + k * stride < a.n ? atomicAdd(a.count + counter_of(a, e0 + k * stride), 1) : 0;
 #pragma unroll
             for (int k = 0; k < EACH; ++k)
                 if (e0 + k * stride < a.n) a.rank[e0 + k * stride] = rank[k];
@@ -753,6 +849,8 @@ __global__ __launch_bounds__(RANK_WG) void rows_rank_tables_kernel(RowsArgs a, i
     }
     const int c = threadIdx.x % RANK_COLS, col0 = int(blockIdx.x % col_groups) * RANK_COLS, col = col0 + c;
     const int64_t b0 = int64_t(blockIdx.x / col_groups) * RANK_TOKENS + threadIdx.x / RANK_COLS;
+    static_assert(SUB % RANK_TOKENS == 0, "a workgroup's tokens are of one part");
+    int32_t *const count = a.count + (int64_t(blockIdx.x / col_groups) * RANK_TOKENS * a.I >= a.sub_pairs ? (size_t)a.tables * VT : 0);
     int row[EACH], rank[EACH];
 #pragma unroll
     for (int k = 0; k < EACH; ++k) {
@@ -765,10 +863,10 @@ __global__ __launch_bounds__(RANK_WG) void rows_rank_tables_kernel(RowsArgs a, i
     auto in_table = [&](int k) { return row[k] / VT == col; };            // (-1 / VT == 0, but such a thread writes nothing)
 #pragma unroll
     for (int k = 0; k < EACH; ++k)
-        if (row[k] >= 0) rank[k] = in_table(k) ? atomicAdd(&place[c * VT + row[k] % VT], 1) : atomicAdd(a.count + row[k], 1);
+        if (row[k] >= 0) rank[k] = in_table(k) ? atomicAdd(&place[c * VT + row[k] % VT], 1) : atomicAdd(count + row[k], 1);
     __syncthreads();
     const int n = place[threadIdx.x];             // row threadIdx.x % VT of table col0 + threadIdx.x / VT
-    if (n > 0) place[threadIdx.x] = atomicAdd(a.count + (size_t)col0 * VT + threadIdx.x, n);
+    if (n > 0) place[threadIdx.x] = atomicAdd(count + (size_t)col0 * VT + threadIdx.x, n);
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < EACH; ++k)
@@ -777,9 +875,9 @@ __global__ __launch_bounds__(RANK_WG) void rows_rank_tables_kernel(RowsArgs a, i
 }
 
 __global__ __launch_bounds__(VT) void rows_claim_kernel(RowsArgs a) {
-    __shared__ int wave_sum_s[VT / 64], base_s;
+    __shared__ int wave_sum_s[VT / 64];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int mine = (a.count[t * VT + tid] + 7) >> 3;
+    const int mine = a.count[(size_t)t * VT + tid];
     int inc = mine;
     for (int d = 1; d < 64; d <<= 1) {
         const int v = __shfl_up(inc, d);
@@ -793,11 +891,12 @@ __global__ __launch_bounds__(VT) void rows_claim_kernel(RowsArgs a) {
         before += w < wave ? wave_sum_s[w] : 0;
         total += wave_sum_s[w];
     }
-    if (tid == 0) base_s = atomicAdd(a.count + (size_t)a.tables * VT, total);
-    __syncthreads();
-    int32_t *off = a.off8 + (size_t)t * (VT + 1);
-    off[tid] = base_s + before + inc - mine;
-    if (tid == 0) off[VT] = base_s + total;
+    int32_t *off = a.off + (size_t)t * (VT + 2);
+    off[tid] = before + inc - mine;
+    if (tid == 0) {
+        off[VT] = total;
+        off[VT + 1] = atomicAdd(a.count + (size_t)a.subs * a.tables * VT, (total + 7) >> 3);
+    }
 }
 
 __device__ __forceinline__ float4 load4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
@@ -812,14 +911,10 @@ __global__ __launch_bounds__(256) void rows_place_kernel(RowsArgs a) {
     if ((int)blockIdx.x < a.place_blocks) {
         const int64_t stride = int64_t(a.place_blocks) * 256;
         for (int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) {
-            const int row = row_of(a, e), rank = a.rank[e];
-            const unsigned token = (unsigned)((uint32_t)e / (uint32_t)a.I);
-            uint2 *list = a.pairs + (int64_t)a.off8[(row / VT) * (VT + 1) + row % VT] * 8;
-            list[rank] = make_uint2(token, __float_as_uint(a.w[e]));
-            if (rank == 0) {
-                const int c = a.count[row];
-                for (int p = c; p < ((c + 7) & ~7); ++p) list[p] = make_uint2((unsigned)a.B, 0u);
-            }
+            const int64_t row = counter_of(a, e);
+            const unsigned token = (unsigned)((uint32_t)(e >= a.sub_pairs ? e - a.sub_pairs : e) / (uint32_t)a.I);
+            const int32_t *off = a.off + row / VT * (VT + 2);
+            a.pairs[(int64_t)off[VT + 1] * 8 + off[row % VT] + a.rank[e]] = make_uint2(token, __float_as_uint(a.w[e]));
         }
         return;
     }
@@ -893,8 +988,11 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(RowsArgs a, float *out, i
     const G *g = static_cast<const G *>(a.g);
     // counts and list positions of the workgroup's rows, a row per lane
     const int64_t my_row = first + min(lane, nrows - 1);
-    const int my_count = a.count[my_row], my_off = a.off8[(my_row / VT) * (VT + 1) + my_row % VT];
-    auto list_of = [&](int r) { return a.pairs + (int64_t)__builtin_amdgcn_readlane(my_off, r) * 8; };
+    const int32_t *const off = a.off + first / VT * (VT + 2);      // (a workgroup's rows are of one table)
+    static_assert(VT % ROW_GROUP == 0, "a workgroup's rows are of one table");
+    const int my_count = a.count[my_row], my_off = off[my_row % VT];
+    const uint2 *const pairs = a.pairs + (int64_t)off[VT + 1] * 8;
+    auto list_of = [&](int r) { return pairs + __builtin_amdgcn_readlane(my_off, r); };
     auto store = [&](int r, int col, float4 v) {
         float4 *dst = reinterpret_cast<float4 *>(out + (first + r) * a.Dv + col);
         if (accumulate) {
@@ -957,30 +1055,33 @@ int launch_rows_sum(const RowsArgs &a, float *out, int accumulate, hipStream_t s
 }
 
 struct RowsWorkspace {
-    int64_t count, rank, off8, pairs, g_packed, flags, total;
+    int64_t count, rank, off, pairs, g_packed, flags, total;
 };
+
+// The lists that a launch walks: of all its tokens where rows are summed from g as it lies (SPARSE_PAIRS), of SUB tokens each otherwise.
+inline bool rows_sparse(int64_t Bc, int64_t I, int64_t rows) { return Bc * I <= SPARSE_PAIRS * rows; }
 
 // Worth it from 3e6 products on (five launches, about 30 us of them whatever the size, against 79 G atomics/s; forward and backward at 512
 // tokens of 32 x 256, 4e6 products: fp32 75 -> 71 us, half 155 -> 99; at 128 x 512, 64 tokens 104 -> 73 and 219 -> 99) and while
 // the list that every slice reads is in proportion: at least one pair for every four rows of the output.
 bool rows_supported(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
-    if (B < 1 || I < 1 || rows < 1 || Dv < SC || Dv % SC != 0 || Dv > (1 << 20)) return false;
+    if (B < 1 || I < 1 || rows < 1 || Dv < 32 || Dv % 32 != 0 || Dv > (1 << 20)) return false;
     const int64_t Bc = B < CHUNK ? B : CHUNK, tables = (rows + VT - 1) / VT;
     return Bc * I < (int64_t(1) << 31) - 8 * 256 && rows <= (int64_t(1) << 30) && B * I * 4 >= rows &&
-           double(B) * double(I) * double(Dv) >= 3e6 && tables * ((Dv / SC + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff &&
+           double(B) * double(I) * double(Dv) >= 3e6 && tables * ((Dv / 32 + XCDS - 1) / XCDS) * XCDS <= 0x7fffffff &&
            (Bc + 1) * Dv / 1024 < (int64_t(1) << 30);
 }
 
 RowsWorkspace rows_layout(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
     RowsWorkspace w{};
     const int64_t Bc = B < CHUNK ? B : CHUNK, tables = (rows + VT - 1) / VT, n = Bc * I;
+    const int64_t lists = sub_lists(Bc) * tables;               // (a shorter last launch has no more of them)
     w.count = 0;
-    w.rank = round16((tables * VT + 1) * 4);
-    w.off8 = w.rank + round16(n * 4);
-    w.pairs = w.off8 + round16(tables * (VT + 1) * 4);
-    w.g_packed = w.pairs + (n + 7 * (n < rows ? n : rows)) * 8 + 8;
-    w.g_packed = round16(w.g_packed);
-    w.flags = w.g_packed + (Bc + 1) * Dv * 4;               // (a multiple of 128)
+    w.rank = round16((lists * VT + 1) * 4);
+    w.off = w.rank + round16(n * 4);
+    w.pairs = w.off + round16(lists * (VT + 2) * 4);
+    w.g_packed = w.pairs + round16((n + 7 * lists) * 8 + 8);
+    w.flags = w.g_packed + (Bc + 1) * slices(Dv) * SC * 4;
     w.total = w.flags + TABLE_FLAGS * 4;
     return w;
 }
@@ -1011,14 +1112,16 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         a.g = static_cast<const char *>(g) + c0 * Dv * (g_format == LFFN_ROWS_F16 ? 2 : 4);
         a.count = reinterpret_cast<int32_t *>(base + l.count);
         a.rank = reinterpret_cast<int32_t *>(base + l.rank);
-        a.off8 = reinterpret_cast<int32_t *>(base + l.off8);
+        a.off = reinterpret_cast<int32_t *>(base + l.off);
         a.pairs = reinterpret_cast<uint2 *>(base + l.pairs);
         a.g_packed = reinterpret_cast<float *>(base + l.g_packed);
         a.n = a.B * I; a.rows = out_size; a.I = (int)I; a.Dv = (int)Dv;
         a.tables = (int)((out_size + VT - 1) / VT);
         const int64_t blocks = (a.n + 255) / 256;
         a.place_blocks = (int)(blocks < 4096 ? blocks : 4096);
-        const bool sparse = a.n <= SPARSE_PAIRS * out_size;      // (no slice-major copy of g)
+        const bool sparse = rows_sparse(a.B, I, out_size);       // (no slice-major copy of g)
+        a.subs = sparse ? 1 : (int)sub_lists(a.B);
+        a.sub_pairs = a.subs > 1 ? SUB * I : a.n;
         const int64_t pack_blocks = sparse ? 0 : ((a.B + 1) * (Dv / 4) + 1023) / 1024;
         const int64_t zero4 = l.rank / 16;                      // the counters and the list's end
         a.flags = a.B >= RANK_TABLES_TOKENS ? reinterpret_cast<int32_t *>(base + l.flags) : nullptr;
@@ -1032,7 +1135,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         } else {
             hipLaunchKernelGGL(rows_rank_kernel, dim3((unsigned)a.place_blocks), dim3(256), 0, st, a);
         }
-        hipLaunchKernelGGL(rows_claim_kernel, dim3((unsigned)a.tables), dim3(VT), 0, st, a);
+        hipLaunchKernelGGL(rows_claim_kernel, dim3((unsigned)(a.subs * a.tables)), dim3(VT), 0, st, a);
         const dim3 grid((unsigned)(a.place_blocks + pack_blocks));
         if (g_format == LFFN_ROWS_F16) hipLaunchKernelGGL(rows_place_kernel<_Float16>, grid, dim3(256), 0, st, a);
         else hipLaunchKernelGGL(rows_place_kernel<float>, grid, dim3(256), 0, st, a);
@@ -1045,9 +1148,9 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
             continue;
         }
         SortedArgs ma{};
-        ma.pairs = a.pairs; ma.off8 = a.off8; ma.g = a.g_packed; ma.out = out; ma.stride = 0; ma.rows = out_size;
-        ma.last_token = (unsigned)a.B;
-        ma.T = a.tables; ma.S = VT; ma.Do = (int)Dv; ma.nslices = (int)(Dv / SC);
+        ma.pairs = a.pairs; ma.off = a.off; ma.g = a.g_packed; ma.out = out; ma.rows = out_size; ma.B = (int)a.B;
+        ma.T = a.tables; ma.S = VT; ma.Do = (int)Dv; ma.nslices = (int)slices(Dv); ma.subs = a.subs;
+        ma.sub_len = (int)(a.sub_pairs / I);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
         ma.more = c0 + CHUNK < B ? 1 : 0;
         rc = launch_sorted(ma, st);

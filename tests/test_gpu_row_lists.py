@@ -1,0 +1,85 @@
+"""The table gradient's row sums where their lists can go wrong: tokens around one list and two, a slice that is half a one,
+buckets that end at every entry of a step, pieces that one bucket cuts, 512 rows a table.
+
+Bound: an fp32 sum of n products is within n * 2^-24 of the sum of their magnitudes, which is the scale of every element here, and
+the result's own rounding 2^-23 of it."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from lookupffn_amd import _lib
+from tests import _cabi as cabi
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(code, w, g, S, accumulate=False):
+    B, T = code.shape
+    idx = code + (np.arange(T, dtype=np.int32) * S)[None]
+    want = oracle.scatter_add(idx, g.astype(np.float64), w.astype(np.float64), T * S).reshape(T, S, -1)
+    scale = oracle.scatter_add(idx, np.abs(g).astype(np.float64), np.abs(w).astype(np.float64), T * S).reshape(T, S, -1)
+    init = np.random.RandomState(1).randn(*want.shape).astype(np.float32) if accumulate else None
+    if accumulate:
+        want, scale = want + init, scale + np.abs(init)
+    got = cabi.lookup_scatter_sorted(code, w, g, S, accumulate=accumulate, init=init)
+    terms = np.bincount(code.ravel(), minlength=S).max() + 1
+    assert (np.abs(got - want) <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
+    return got
+
+
+@pytest.mark.parametrize("B,T,S,Do", [(8192, 3, 256, 64), (8193, 2, 256, 96), (8200, 3, 512, 32), (9217, 2, 16, 160), (15871, 2, 256, 64),
+                                      (16384, 9, 1, 32), (16384 + 8193, 2, 256, 96), (37, 3, 256, 32), (513, 2, 8, 608)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_tokens_around_one_list_and_two(B, T, S, Do, skew):
+    rng = np.random.RandomState(B + S + Do)
+    code = (rng.zipf(1.2, size=(B, T)) % S if skew else rng.randint(0, S, size=(B, T))).astype(np.int32)
+    w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    got = _check(code, w, g, S)
+    assert np.array_equal(got, cabi.lookup_scatter_sorted(code, w, g, S))        # fixed order of additions
+    _check(code, w, g, S, accumulate=True)
+
+
+@pytest.mark.parametrize("lengths", [(1, 2, 3, 4, 5, 6, 7, 8), (1, 1, 1, 1, 1, 1, 1, 60), (63, 64, 65, 0, 0, 1, 0, 3), (0, 0, 700, 0, 1, 0, 0, 0)])
+def test_bucket_ends_at_every_entry(lengths):
+    rng = np.random.RandomState(sum(lengths))
+    code = np.repeat(np.arange(8), lengths).astype(np.int32)[:, None]
+    code = np.concatenate([code, rng.permutation(code)], 1)
+    _check(code, rng.randn(*code.shape).astype(np.float32), rng.randn(len(code), 96).astype(np.float32), 8)
+
+
+def test_infinite_gradient_stays_in_its_row():
+    rng = np.random.RandomState(5)
+    B, T, S, Do = 9000, 2, 256, 96
+    code = rng.randint(0, S, size=(B, T)).astype(np.int32)
+    code[code == 17] = 18
+    code[8500, 0] = 17                                      # alone in its bucket, amid others in its step
+    w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    g[8500] = np.inf
+    got = cabi.lookup_scatter_sorted(code, w, g, S)
+    assert np.isinf(got[0, 17]).all() and np.isinf(got[1, code[8500, 1]]).all()
+    got[0, 17] = got[1, code[8500, 1]] = 0
+    assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("B,I,rows,in_tables", [(8193, 8, 1948, 1.0), (9300, 8, 1948, 0.9), (16384, 4, 924, 0.0), (24600, 4, 924, 1.0),
+                                                (9000, 4, 5000, 0.0)])      # the last: few pairs a row, one list
+def test_flat_rows_of_two_lists(B, I, rows, in_tables):
+    rng = np.random.RandomState(B)
+    Dv = 96
+    idx = rng.randint(0, 256, size=(B, I)) + 256 * np.arange(I)[None]
+    idx = np.where(rng.rand(B, I) < in_tables, idx, rng.randint(0, rows, size=(B, I))).clip(0, rows - 1).astype(np.int32)
+    w, g = rng.randn(B, I).astype(np.float32), rng.randn(B, Dv).astype(np.float32)
+    size = ctypes.c_int64()
+    assert _lib.load().lffn_scatter_rows_workspace_bytes(B, I, rows, Dv, ctypes.byref(size)) == 0 and size.value > 0
+    idd, gd, wd = (torch.from_numpy(v).cuda() for v in (idx, g, w))
+    ws, out = torch.full((size.value,), 0x7f, dtype=torch.uint8, device="cuda"), torch.full((rows, Dv), float("nan"), device="cuda")
+    assert _lib.load().lffn_scatter_rows(idd.data_ptr(), gd.data_ptr(), wd.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), B, I, rows, Dv,
+                                         0, 0, _lib.stream_of(gd)) == 0
+    got = out.cpu().numpy()
+    want = oracle.scatter_add(idx, g.astype(np.float64), w.astype(np.float64), rows)
+    scale = oracle.scatter_add(idx, np.abs(g).astype(np.float64), np.abs(w).astype(np.float64), rows)
+    terms = np.bincount(idx.ravel()).max()
+    assert (np.abs(got - want) <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
