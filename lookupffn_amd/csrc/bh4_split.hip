@@ -44,6 +44,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BS = 64;          // block size this file is built for
 constexpr int PAD = 4;          // floats of padding per row of the fp32 tile
+constexpr unsigned REPEAT_TILES = 128;      // tiles that one repeat after the other takes
 constexpr float TOP = 16384.f;  // what the largest of a row is scaled to at least (and less than twice that)
 
 // Largest and smallest over the wavefront.
@@ -247,22 +248,27 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     const int bg = wave >> 2;                     // group of blocks of this wavefront
     const int c = lane & 15;                      // A operand: output column; B operand and result: token
     const int kq = lane >> 4;                     // operands: columns 16*kq .. + 15 of the block; result: output columns 4*kq .. + 3
-    const int64_t tok_base = int64_t(blockIdx.x) * TOK;
+    // A workgroup takes one repeat of its tokens: few tokens with several repeats are as many workgroups more.  The repeats of
+    // REPEAT_TILES tiles come one after the other in the grid (on the same XCDs, as that is a multiple of their number), so that the
+    // second still finds the tokens' rows in the L2, and a stage's weights serve as many tiles in a row.  32768 tokens, D = 512,
+    // two repeats, all tiles of a repeat after all of the one before -> so: layer 259 -> 255 us, training step 1473 -> 1464 (groups of 32 to 512 the same).
+    const unsigned in_order = blockIdx.y * gridDim.x + blockIdx.x, group = in_order / (REPEAT_TILES * gridDim.y);
+    const unsigned group_tiles = min(REPEAT_TILES, gridDim.x - group * REPEAT_TILES), in_group = in_order - group * (REPEAT_TILES * gridDim.y);
+    const int r = __builtin_amdgcn_readfirstlane(in_group / group_tiles);
+    const unsigned tile_no = __builtin_amdgcn_readfirstlane(group * REPEAT_TILES + in_group % group_tiles);
+    const int64_t tok_base = int64_t(tile_no) * TOK;
     if (!BWD) {
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         for (int e = tid * 4; e < D; e += 256 * NWAVE) {
             const f32x4 one = {1.f, 1.f, 1.f, 1.f};
             *reinterpret_cast<f32x4 *>(lnw_s + e) = e >= H ? zero : a.ln_w ? *reinterpret_cast<const f32x4 *>(a.ln_w + e) : one;
             *reinterpret_cast<f32x4 *>(lnb_s + e) = e < H && a.ln_w ? *reinterpret_cast<const f32x4 *>(a.ln_b + e) : zero;
-            const int col = blockIdx.y * D + e;
+            const int col = r * D + e;
             *reinterpret_cast<f32x4 *>(pbias_s + e) = a.pbias && col < a.T * 8 ? *reinterpret_cast<const f32x4 *>(a.pbias + col) : zero;
         }
         __syncthreads();
     }
 
-    // A workgroup takes one repeat of its tokens, and the repeats come one after the other in the grid: their weights
-    // stay in the L2 for the launch's workgroups, and few tokens with several repeats are as many workgroups more.
-    const int r = blockIdx.y;
     f32x4 acc[NBW];
 
     // this wavefront's weights of a block: four fragments of 1 KB (hi, hi, lo, lo)
@@ -545,7 +551,7 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
                     float sum = 0.f;
 #pragma unroll
                     for (int t = 0; t < TOK; ++t) sum += rows32[t * LDR + e];
-                    a.bias_parts[size_t(blockIdx.x) * ncols + r * D + e] = sum;
+                    a.bias_parts[size_t(tile_no) * ncols + r * D + e] = sum;
                 }
             }
 #pragma unroll

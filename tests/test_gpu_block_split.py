@@ -267,3 +267,16 @@ def test_columns_against_their_inputs(B, D, kind):
     codes, scores = ops.bh4_block_front(x[:few], lw, lb, 1e-5, ops.bh4_fold_split(w, False), 1, J, D, None, T, 1.0, 0.0)
     got = ops.bh4_block_front_train(x, lw, lb, 1e-5, ops.bh4_fold_split(w, False), 1, J, D, None, T, 1.0, 0.0)
     assert torch.equal(codes, got[0][:few]) and torch.equal(scores, got[1][:few])
+
+
+# the repeats take turns at groups of 128 tiles of 16 tokens: the last group whole, a tile short or a tile over
+@pytest.mark.parametrize("B,D,R", [(2048, 512, 2), (2049, 256, 3), (4080, 512, 2), (4112, 64, 4)])
+def test_every_tile_of_every_repeat(B, D, R):
+    gen = torch.Generator(device=DEV).manual_seed(B)
+    J, T = 4, R * D // 8
+    x, w = _randn(gen, B, D), _randn(gen, R, J, D // 64, 64, 64) / math.sqrt(64 * D)
+    split = ops.bh4_fold_split(w, False)
+    front = lambda rows: ops.bh4_block_front(rows, None, None, 1e-5, split, R, J, D, None, T, 0.7, 0.3)
+    whole, parts = front(x), [front(x[i:i + 200]) for i in range(0, B, 200)]
+    for k in range(2):
+        assert torch.equal(whole[k], torch.cat([p[k] for p in parts]))
