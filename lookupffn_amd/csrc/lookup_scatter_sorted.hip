@@ -827,7 +827,7 @@ __global__ __launch_bounds__(256) void rows_rank_kernel(RowsArgs a) {
 
 // The same for many tokens.  Row numbers as the layer forms them lie in table i in column i: then a workgroup has RANK_TOKENS tokens of
 // RANK_COLS columns, counts them in LDS and takes their places from one add per row.  What bounds it is the adds that return something,
-// 24 G/s: 4096 x 128 pairs, 32768 rows, 22 -> 7 us, 16000 x 64 41 -> 9.5, 2500 x 256 27 -> 8.  For other row numbers an add for every pair, in
+// 24 G/s: 4096 x 128 pairs, 32768 rows, 22 -> 7 us, 16000 x 64 41 -> 9.5, 2500 x 256 27 -> 8 (neighbouring columns on one XCD: 7 -> 5.8).  For other row numbers an add for every pair, in
 // their order (in the order of the tables' form, sixteen bytes of a token's at a time, 22 -> 25 us, 45 -> 54).  From RANK_TABLES_TOKENS
 // on: at 1024 tokens a row has four pairs in a table, and there is nothing to win.
 constexpr int64_t RANK_TABLES_TOKENS = 2048;
@@ -847,10 +847,14 @@ __global__ __launch_bounds__(RANK_WG) void rows_rank_tables_kernel(RowsArgs a, i
         }
         return;
     }
-    const int c = threadIdx.x % RANK_COLS, col0 = int(blockIdx.x % col_groups) * RANK_COLS, col = col0 + c;
-    const int64_t b0 = int64_t(blockIdx.x / col_groups) * RANK_TOKENS + threadIdx.x / RANK_COLS;
+    // neighbouring groups of columns on one XCD, as rows_place_kernel has them
+    const int per_xcd = (col_groups + XCDS - 1) / XCDS, group = int(blockIdx.x % XCDS) * per_xcd + int(blockIdx.x / XCDS % per_xcd);
+    if (group >= col_groups) return;                          // uniform
+    const int64_t b_first = int64_t(blockIdx.x / XCDS / per_xcd) * RANK_TOKENS;
+    const int c = threadIdx.x % RANK_COLS, col0 = group * RANK_COLS, col = col0 + c;
+    const int64_t b0 = b_first + threadIdx.x / RANK_COLS;
     static_assert(SUB % RANK_TOKENS == 0, "a workgroup's tokens are of one part");
-    int32_t *const count = a.count + (int64_t(blockIdx.x / col_groups) * RANK_TOKENS * a.I >= a.sub_pairs ? (size_t)a.tables * VT : 0);
+    int32_t *const count = a.count + (b_first * a.I >= a.sub_pairs ? (size_t)a.tables * VT : 0);
     int row[EACH], rank[EACH];
 #pragma unroll
     for (int k = 0; k < EACH; ++k) {
@@ -906,13 +910,20 @@ __device__ __forceinline__ float4 load4(const _Float16 *p) {
     return make_float4((float)h.x, (float)h.y, (float)h.z, (float)h.w);
 }
 
+constexpr int PLACE_COLS = 32;
 template <typename G>
 __global__ __launch_bounds__(256) void rows_place_kernel(RowsArgs a) {
     if ((int)blockIdx.x < a.place_blocks) {
-        const int64_t stride = int64_t(a.place_blocks) * 256;
-        for (int64_t e = int64_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) {
+        // An XCD takes an eighth of the columns, from PLACE_COLS of them on: where column i's rows are of table i, what is written to a line
+        // of a list then meets in one L2 (4096 x 128 pairs 13.3 -> 8.4 us).
+        const unsigned xcds = a.I >= PLACE_COLS ? XCDS : 1, cols = (unsigned)(a.I + xcds - 1) / xcds, col0 = blockIdx.x % xcds * cols;
+        if (col0 >= (unsigned)a.I) return;                    // uniform
+        const unsigned mine = min(cols, a.I - col0), pairs = (unsigned)a.B * mine;
+        for (unsigned q = blockIdx.x / xcds * 256 + threadIdx.x; q < pairs; q += a.place_blocks / xcds * 256) {
+            const unsigned b = q / mine;
+            const int64_t e = (int64_t)b * a.I + col0 + (q - b * mine);
             const int64_t row = counter_of(a, e);
-            const unsigned token = (unsigned)((uint32_t)(e >= a.sub_pairs ? e - a.sub_pairs : e) / (uint32_t)a.I);
+            const unsigned token = e >= a.sub_pairs ? b - (unsigned)SUB : b;
             const int32_t *off = a.off + row / VT * (VT + 2);
             a.pairs[(int64_t)off[VT + 1] * 8 + off[row % VT] + a.rank[e]] = make_uint2(token, __float_as_uint(a.w[e]));
         }
@@ -1118,7 +1129,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         a.n = a.B * I; a.rows = out_size; a.I = (int)I; a.Dv = (int)Dv;
         a.tables = (int)((out_size + VT - 1) / VT);
         const int64_t blocks = (a.n + 255) / 256;
-        a.place_blocks = (int)(blocks < 4096 ? blocks : 4096);
+        a.place_blocks = (int)((blocks < 4096 ? blocks + XCDS - 1 : 4096) / XCDS * XCDS);
         const bool sparse = rows_sparse(a.B, I, out_size);       // (no slice-major copy of g)
         a.subs = sparse ? 1 : (int)sub_lists(a.B);
         a.sub_pairs = a.subs > 1 ? SUB * I : a.n;
@@ -1130,7 +1141,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
                            zero4);
         if (a.flags) {
             const int col_groups = (int)((I + RANK_COLS - 1) / RANK_COLS);      // (workgroups: fewer than pairs)
-            hipLaunchKernelGGL(rows_rank_tables_kernel, dim3((unsigned)((a.B + RANK_TOKENS - 1) / RANK_TOKENS * col_groups)), dim3(RANK_WG), 0,
+            hipLaunchKernelGGL(rows_rank_tables_kernel, dim3((unsigned)((a.B + RANK_TOKENS - 1) / RANK_TOKENS * ((col_groups + XCDS - 1) / XCDS * XCDS))), dim3(RANK_WG), 0,
                                st, a, col_groups);
         } else {
             hipLaunchKernelGGL(rows_rank_kernel, dim3((unsigned)a.place_blocks), dim3(256), 0, st, a);
