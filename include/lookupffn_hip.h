@@ -698,6 +698,11 @@ int lffn_scatter_add_f16(const int32_t *idx, const uint16_t *g, const float *w, 
 /* Tokens up to which lffn_lookup_scatter_f32 is faster than lffn_lookup_scatter_sorted_f32 (tables of at most 256 rows): up to
  * there it sums every row of the gradient from a list of its tokens, where that is faster than summing in LDS. */
 #define LFFN_SCATTER_LIST_TOKENS 2048
+/* Beyond, from this many products (B * T * Do) on lffn_lookup_scatter_sorted_f32 and lffn_lookup_backward_f32 are the faster ones; below
+ * the second number, for at most LFFN_SCATTER_CHUNK_TOKENS tokens, their sums are doubles as lffn_lookup_scatter_f32's are. */
+#define LFFN_SCATTER_SORTED_WORK 45000000
+#define LFFN_SCATTER_DOUBLE_WORK 400000000
+#define LFFN_SCATTER_CHUNK_TOKENS 16384
 
 /*
  * The scatter-add as the layer's backward issues it: table-local codes, the
@@ -722,7 +727,7 @@ int lffn_lookup_scatter_f32(const int32_t *code, const float *score, const float
  * inside a code), so results are reproducible from run to run, unlike the reference's
  * atomics.  Tokens are taken 16384 at a time (the workspace is sized for one such chunk).
  * About twice as fast as lffn_lookup_scatter_f32 at 16384 tokens x 128 tables x 768
- * columns; slower below about 4e8 multiply-adds (B * T * Do).
+ * columns; slower below LFFN_SCATTER_SORTED_WORK multiply-adds (B * T * Do).
  * lffn_lookup_scatter_workspace_bytes sets *bytes to the workspace this form needs for a
  * shape, or to 0 when the form does not cover it (S > 512, Do % 32 != 0, B == 0 or T == 0):
  * lffn_lookup_scatter_f32 covers those.  workspace: device memory, 16-byte aligned, at

@@ -378,7 +378,9 @@ struct LookupFFNBackward : public torch::autograd::Node {
         if (need_score || need[TABLES]) {
             int64_t ws_bytes = 0;
             CALL(lffn_lookup_scatter_workspace_bytes, B, T, S, Do, &ws_bytes);
-            if (B <= LFFN_SCATTER_LIST_TOKENS || B * T * Do < limits.sorted_min_work) ws_bytes = 0;
+            if (B <= LFFN_SCATTER_LIST_TOKENS || B * T * Do < limits.sorted_min_work ||
+                (B > LFFN_SCATTER_CHUNK_TOKENS && B * T * Do < LFFN_SCATTER_DOUBLE_WORK))
+                ws_bytes = 0;
             if (need[TABLES] && ws_bytes > 0) {
                 Tensor ws = empty_bytes(ws_bytes, dev);
                 if (need_score) {

@@ -321,7 +321,20 @@ __device__ __forceinline__ float sum_swapped16(float x, float y) {     // rows o
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ float sum_groups(float4 v) { return sum_swapped16(sum_swapped32(v.x, v.y), sum_swapped32(v.z, v.w)); }
+__device__ __forceinline__ float sum_groups(const float (&v)[4]) { return sum_swapped16(sum_swapped32(v[0], v[1]), sum_swapped32(v[2], v[3])); }
+// the same of doubles, the two words of each on the same ways
+template <bool HALVES>
+__device__ __forceinline__ double sum_swapped(double x, double y) {
+    const uint64_t a = __double_as_longlong(x), b = __double_as_longlong(y);
+    auto swap = [](unsigned p, unsigned q) {
+        return HALVES ? __builtin_amdgcn_permlane32_swap(p, q, false, false) : __builtin_amdgcn_permlane16_swap(p, q, false, false);
+    };
+    const auto lo = swap((unsigned)a, (unsigned)b), hi = swap((unsigned)(a >> 32), (unsigned)(b >> 32));
+    return __longlong_as_double((uint64_t)hi[0] << 32 | lo[0]) + __longlong_as_double((uint64_t)hi[1] << 32 | lo[1]);
+}
+__device__ __forceinline__ double sum_groups(const double (&v)[4]) {
+    return sum_swapped<false>(sum_swapped<true>(v[0], v[1]), sum_swapped<true>(v[2], v[3]));
+}
 
 // What lane u of a row of sixteen lanes holds, in all of them (a DPP operand of the instruction that uses it).
 __device__ __forceinline__ int row_pick(int v, int u) {
@@ -334,8 +347,8 @@ __device__ __forceinline__ int row_pick(int v, int u) {
 #undef LFFN_PICK
 }
 
-// ADD: the sums are added to what a.out holds.
-template <bool ADD>
+// ADD: the sums are added to what a.out holds.  Sum: float, or double (sums_in_doubles).
+template <bool ADD, typename Sum>
 __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(SortedArgs a) {
     extern __shared__ float4 lds4[];
     float *row_s = reinterpret_cast<float *>(lds4);             // [S][SC]: the rows' sums
@@ -423,14 +436,18 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
             int dst = head_bucket >= 0 ? slot0 : cur * SC + my_col;
             float before = head_bucket >= 0 ? 0.f : row_s[cur * SC + my_col];      // what the row holds: the sum over earlier lists
             const char *gs = reinterpret_cast<const char *>(a.g + ((size_t)slice * (a.B + 1) + (size_t)sub * a.sub_len) * SC);
-            float acc[2][4];                                  // the even and the odd steps' sums
+            constexpr int SUMS = sizeof(Sum) == 4 ? 2 : 1;    // the even and the odd steps', so that an fp32 sum is one of eight
+            Sum acc[SUMS][4];
             auto clear = [&]() {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e >> 2][e & 3] = 0.f;
+                for (int e = 0; e < 4 * SUMS; ++e) acc[e >> 2][e & 3] = 0;
             };
             clear();
             auto flush = [&]() {
-                const float v = sum_groups(make_float4(acc[0][0] + acc[1][0], acc[0][1] + acc[1][1], acc[0][2] + acc[1][2], acc[0][3] + acc[1][3]));
+                if constexpr (SUMS == 2)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[0][e] += acc[1][e];
+                const float v = (float)sum_groups(acc[0]);
                 row_s[dst] = before + v;
             };
             // Lane i of group q gets the pair that the group takes in step i (loaded so, sixteen lanes would be sixteen lines).
@@ -443,8 +460,10 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
             auto load_row = [&](int rows, int u) {
                 return *reinterpret_cast<const float4 *>(gs + (unsigned)(row_pick(rows, u) + i16 * 16));
             };
-            auto add = [&](float (&to)[4], float w, float4 v, bool live) {
-                const float x = fmaf(w, v.x, to[0]), y = fmaf(w, v.y, to[1]), z = fmaf(w, v.z, to[2]), u = fmaf(w, v.w, to[3]);
+            auto add = [&](int odd, float w, float4 v, bool live) {
+                Sum (&to)[4] = acc[odd % SUMS];
+                const Sum x = fma((Sum)w, (Sum)v.x, to[0]), y = fma((Sum)w, (Sum)v.y, to[1]), z = fma((Sum)w, (Sum)v.z, to[2]),
+                          u = fma((Sum)w, (Sum)v.w, to[3]);
                 to[0] = live ? x : to[0];
                 to[1] = live ? y : to[1];
                 to[2] = live ? z : to[2];
@@ -453,13 +472,13 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
             // four entries from e on, one per lane group; a bucket may end before any of them
             auto take = [&](int e, int odd, float w, float4 v) {
                 if (next_b >= e + 4) {                        // uniform
-                    add(acc[odd], w, v, true);
+                    add(odd, w, v, true);
                     return;
                 }
                 int from = 0;
                 do {
                     const int to = next_b - e;
-                    add(acc[odd], w, v, grp >= from && grp < to);      // (selected, not branched on: all control flow is the wavefront's)
+                    add(odd, w, v, grp >= from && grp < to);      // (selected, not branched on: all control flow is the wavefront's)
                     flush();
                     const int end = next_b;
                     do {
@@ -475,7 +494,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
                     clear();
                     from = to;
                 } while (next_b < e + 4);
-                add(acc[odd], w, v, grp >= from);
+                add(odd, w, v, grp >= from);
             };
 
             int rows = rows_of(pr0, e_lo), w = weights_of(pr0, e_lo);
@@ -572,25 +591,37 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
 }
 
 // one workgroup per (table of a.S rows, slice)
-template <bool ADD>
+template <bool ADD, typename Sum>
 int launch_sorted_form(SortedArgs a, hipStream_t st) {
     const size_t lds = (size_t(a.S) + WAVES * 2) * SC * sizeof(float) + (2 * WAVES * 4 + size_t(2) * (a.S + 2)) * sizeof(int);
     static LdsGrant granted;
-    if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD>), lds, granted)) return LFFN_ERR_LAUNCH;
+    if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD, Sum>), lds, granted)) return LFFN_ERR_LAUNCH;
     a.per_xcd = (a.T * a.nslices + XCDS - 1) / XCDS;
-    hipLaunchKernelGGL(lookup_scatter_sorted_kernel<ADD>, dim3((unsigned)(a.per_xcd * XCDS)), dim3(MWG), lds, st, a);
+    hipLaunchKernelGGL((lookup_scatter_sorted_kernel<ADD, Sum>), dim3((unsigned)(a.per_xcd * XCDS)), dim3(MWG), lds, st, a);
     return lffn_launch_status();
 }
 
-int launch_sorted(const SortedArgs &a, hipStream_t st) {
-    return a.accumulate ? launch_sorted_form<true>(a, st) : launch_sorted_form<false>(a, st);
+// Calls of fewer products than this and of at most CHUNK tokens have their sums in doubles: the LDS form (lookup_scatter.hip) has, which
+// served the layer there and takes longer from LFFN_SCATTER_SORTED_WORK products on.  They cost little beside the loads (3000 tokens of
+// 128 tables of 768 columns 81 -> 90 us, 4096 x 64 x 512 50 -> 53; the LDS form 192 and 64), and the error against 64 bits is 2.6e-8
+// (fp32 5.5e-8 to 5.7e-8, the LDS form's products rounded to fp32 3.6e-8).
+inline bool sums_in_doubles(int64_t B, int64_t T, int64_t Do) {
+    return B <= CHUNK && double(B) * double(T) * double(Do) < LFFN_SCATTER_DOUBLE_WORK;
+}
+
+int launch_sorted(const SortedArgs &a, bool doubles, hipStream_t st) {
+    if (doubles) return a.accumulate ? launch_sorted_form<true, double>(a, st) : launch_sorted_form<false, double>(a, st);
+    return a.accumulate ? launch_sorted_form<true, float>(a, st) : launch_sorted_form<false, float>(a, st);
 }
 
 inline int64_t slices(int64_t Do) { return (Do + SC - 1) / SC; }
 // One list of a chunk's tokens, or two: then half of the sort's wavefronts have the first, and all of them as many batches of 64.
-inline int64_t sub_lists(int64_t Bc) { return Bc > SUB ? 2 : 1; }
-inline int64_t list_tokens(int64_t Bc) { return Bc > SUB ? (Bc + SORT_WG - 1) / SORT_WG * (SORT_WG / 2) : Bc; }
-inline int64_t pair_stride(int64_t Bc) { return (list_tokens(Bc) + 7) & ~int64_t(7); }
+// Sums in doubles are not taken apart (kept in fp32 between two lists, the error is 3.8e-8 instead of 2.6e-8 at 12000 tokens).
+inline int64_t sub_lists(int64_t Bc, bool doubles = false) { return Bc > SUB && !doubles ? 2 : 1; }
+inline int64_t list_tokens(int64_t Bc, bool doubles = false) {
+    return sub_lists(Bc, doubles) > 1 ? (Bc + SORT_WG - 1) / SORT_WG * (SORT_WG / 2) : Bc;
+}
+inline int64_t pair_stride(int64_t Bc, bool doubles = false) { return (list_tokens(Bc, doubles) + 7) & ~int64_t(7); }      // (times their number: doubles' is no more)
 
 inline bool sorted_supported(int64_t B, int64_t T, int64_t S, int64_t Do) {
     return B >= 1 && T >= 1 && lffn_is_pow2(S) && S <= MAX_S && Do % 32 == 0 && Do <= (1 << 20) &&
@@ -644,10 +675,11 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
     char *base = static_cast<char *>(workspace);
     uint2 *pairs = reinterpret_cast<uint2 *>(base + w.pairs);
     int32_t *off = reinterpret_cast<int32_t *>(base + w.off);
+    const bool doubles = sums_in_doubles(B, T, Do);
 
     for (int64_t c0 = 0; c0 < B; c0 += CHUNK) {
         const int64_t Bc = B - c0 < CHUNK ? B - c0 : CHUNK;
-        const int64_t stride = pair_stride(Bc), Bp = padded_tokens(Bc);
+        const int64_t stride = pair_stride(Bc, doubles), Bp = padded_tokens(Bc);
 
         PrepArgs pa{};
         pa.code = code + c0 * T; pa.score = score + c0 * T; pa.g = g + c0 * Do;
@@ -671,10 +703,10 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         }
         SortArgs sa{};
         sa.code = pa.code_t; sa.score = pa.score_t; sa.pairs = pairs; sa.off = off;
-        sa.B = Bc; sa.Bp = Bp; sa.sub_len = list_tokens(Bc); sa.stride = stride;
-        sa.T = (int)T; sa.S = (int)S; sa.nbits = lffn_log2(S); sa.subs = (int)sub_lists(Bc);
+        sa.B = Bc; sa.Bp = Bp; sa.sub_len = list_tokens(Bc, doubles); sa.stride = stride;
+        sa.T = (int)T; sa.S = (int)S; sa.nbits = lffn_log2(S); sa.subs = (int)sub_lists(Bc, doubles);
         // histograms and bucket starts, then the sorted lists themselves (4 + 2 bytes per entry)
-        static_assert(SUB <= 65536 && CHUNK % SORT_WG == 0, "a list's tokens are staged as 16-bit values, and held in registers");
+        static_assert(CHUNK <= 65536 && CHUNK % SORT_WG == 0, "a list's tokens are staged as 16-bit values, and held in registers");
         size_t sort_lds = nsort ? size_t(SORT_WAVES + sa.subs) * S * sizeof(int) + size_t(sa.subs) * stride * 6 : 0;
         if (pa.sums && sort_lds < SORT_WG * sizeof(float4)) sort_lds = SORT_WG * sizeof(float4);
         static LdsGrant granted;
@@ -700,7 +732,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         ma.sub_len = (int)sa.sub_len;
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
         ma.more = c0 + CHUNK < B ? 1 : 0;
-        rc = launch_sorted(ma, st);
+        rc = launch_sorted(ma, doubles, st);
         if (rc != LFFN_OK) return rc;
     }
     return LFFN_OK;
@@ -1164,7 +1196,7 @@ extern "C" int lffn_scatter_rows(const int32_t *idx, const void *g, const float 
         ma.sub_len = (int)(a.sub_pairs / I);
         ma.accumulate = (accumulate || c0 > 0) ? 1 : 0;
         ma.more = c0 + CHUNK < B ? 1 : 0;
-        rc = launch_sorted(ma, st);
+        rc = launch_sorted(ma, false, st);
         if (rc != LFFN_OK) return rc;
     }
     return LFFN_OK;

@@ -1105,11 +1105,20 @@ def _(indexes, source, weights, output_size):
     return source.new_empty(output_size, source.shape[1], dtype=torch.float32)
 
 
-# Below this many multiply-adds (B * T * Do) the LDS-accumulating scatter is the faster one
-# (measured: 16384 x 32 x 768 and 16384 x 128 x 256 favour the sorted form, 2048 x 128 x 768 does not).
-SORTED_SCATTER_MIN_WORK = 4 * 10 ** 8
+# From this many multiply-adds (B * T * Do) on the sorted scatter is the faster one (LFFN_SCATTER_SORTED_WORK of the C header; both gradients,
+# by the LDS-accumulating scatter -> sorted, us: 4096 x 32 x 256 43 -> 50, 6000 x 32 x 256 65 -> 60, 2049 x 64 x 512 67 -> 68, 3000 x 64 x
+# 512 106 -> 86, 4096 x 128 x 512 168 -> 125, 3000 x 128 x 768 273 -> 163, 3000 x 256 x 512 322 -> 185)
+SORTED_SCATTER_MIN_WORK = 45 * 10 ** 6
+# below this many its sums are doubles as the other's are, for at most so many tokens (LFFN_SCATTER_DOUBLE_WORK, LFFN_SCATTER_CHUNK_TOKENS)
+DOUBLE_SCATTER_WORK, SCATTER_CHUNK_TOKENS = 4 * 10 ** 8, 16384
 # and up to this many tokens (LFFN_SCATTER_LIST_TOKENS of the C header) the one that sums rows from lists of their tokens is
 LIST_SCATTER_MAX_TOKENS = 2048
+
+
+def _sorted_scatter_pays(B, T, Do):
+    work = B * T * Do
+    return B > LIST_SCATTER_MAX_TOKENS and work >= SORTED_SCATTER_MIN_WORK and (B <= SCATTER_CHUNK_TOKENS or work >= DOUBLE_SCATTER_WORK)
+
 
 _L.define("lookup_scatter(Tensor code, Tensor score, Tensor g, int S) -> Tensor")
 
@@ -1128,7 +1137,7 @@ def _lookup_scatter_impl(code, score, g, S):
     ws_bytes = ctypes.c_int64(0)
     _lib.check(lib.lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)), "lffn_lookup_scatter_workspace_bytes")
     with _dev_guard(g):
-        if ws_bytes.value > 0 and B > LIST_SCATTER_MAX_TOKENS and B * T * Do >= SORTED_SCATTER_MIN_WORK:
+        if ws_bytes.value > 0 and _sorted_scatter_pays(B, T, Do):
             # sort the tokens of every table by code, then sum rows in registers: no atomics
             ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=g.device)
             rc = lib.lffn_lookup_scatter_sorted_f32(_lib.ptr(code), _lib.ptr(score), _lib.ptr(g), _lib.ptr(out), _lib.ptr(ws),
@@ -1155,7 +1164,7 @@ _L.define("lookup_backward(Tensor code, Tensor score, Tensor g, Tensor tables) -
 def lookup_backward_is_fused(B, T, S, Do):
     """Both gradients of the gather go through one call (lffn_lookup_backward_f32: the sorted scatter and the
     score gradient sharing one slice-major copy of g) for this shape."""
-    if B <= LIST_SCATTER_MAX_TOKENS or B * T * Do < SORTED_SCATTER_MIN_WORK or Do % 64 != 0:
+    if not _sorted_scatter_pays(B, T, Do) or Do % 64 != 0:
         return False
     ws_bytes = ctypes.c_int64(0)
     _lib.check(_lib.load().lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)),

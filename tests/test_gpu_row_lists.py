@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle
-from lookupffn_amd import _lib
+from lookupffn_amd import _lib, ops
 from tests import _cabi as cabi
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +83,25 @@ def test_flat_rows_of_two_lists(B, I, rows, in_tables):
     scale = oracle.scatter_add(idx, np.abs(g).astype(np.float64), np.abs(w).astype(np.float64), rows)
     terms = np.bincount(idx.ravel()).max()
     assert (np.abs(got - want) <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
+
+
+@pytest.mark.parametrize("B,T,Do", [(2049, 64, 384), (3001, 32, 512), (8193, 32, 256), (16384, 33, 128)])
+def test_calls_that_had_double_sums_keep_them(B, T, Do):
+    """Rounded once, a number is off by 2^-24 / 3^0.5 of its power of two, root mean square; the rows cut by pieces a few roundings more."""
+    assert ops.lookup_backward_is_fused(B, T, 256, Do) and B * T * Do < ops.DOUBLE_SCATTER_WORK
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    code = torch.randint(0, 256, (B, T), generator=gen, device="cuda", dtype=torch.int32)
+    score, g = torch.rand(B, T, generator=gen, device="cuda"), torch.randn(B, Do, generator=gen, device="cuda")
+    tables = torch.randn(T, 256, Do, generator=gen, device="cuda")
+    grad_score, grad = ops._lookup_backward_impl(code, score, g, tables)
+    for t in (0, T - 1):
+        want = torch.zeros(256, Do, dtype=torch.float64, device="cuda").index_add_(0, code[:, t].long(), score[:, t, None].double() * g.double())
+        assert (grad[t] - want).norm() <= 2.0 ** -24 / 3 ** 0.5 * 1.1 * want.norm()
+        want = (tables[t].double()[code[:, t].long()] * g.double()).sum(1)
+        assert ((grad_score[:, t] - want).abs() <= Do * 2.0 ** -24 * (tables[t].abs()[code[:, t].long()] * g.abs()).sum(1)).all()
+
+
+def test_which_calls_the_lists_serve():
+    assert not ops.lookup_backward_is_fused(2048, 128, 256, 512) and not ops.lookup_backward_is_fused(4096, 32, 256, 256)
+    assert ops.lookup_backward_is_fused(2049, 128, 256, 512) and ops.lookup_backward_is_fused(16384, 32, 256, 256)
+    assert not ops.lookup_backward_is_fused(16385, 32, 256, 512) and ops.lookup_backward_is_fused(32768, 128, 256, 512)
