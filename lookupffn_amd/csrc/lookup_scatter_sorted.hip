@@ -630,6 +630,7 @@ inline bool sorted_supported(int64_t B, int64_t T, int64_t S, int64_t Do) {
 
 inline int64_t pack_workgroups(int64_t Bc) { return (Bc + 1 + PACK_TOKENS - 1) / PACK_TOKENS; }
 inline int64_t round16(int64_t v) { return (v + 15) & ~int64_t(15); }
+inline int64_t whole_rows(int64_t v) { return (v + SC * 4 - 1) / (SC * 4) * (SC * 4); }      // rows of the copy of g on whole lines
 inline int64_t padded_tokens(int64_t B) { return (B + 63) & ~int64_t(63); }
 
 // Tokens are taken CHUNK at a time (later chunks add to the result of the earlier ones): a
@@ -648,7 +649,7 @@ inline Workspace workspace_layout(int64_t B, int64_t T, int64_t S, int64_t Do) {
     w.off = w.pairs + sub_lists(Bc) * T * pair_stride(Bc) * 8;
     w.code_t = w.off + round16(sub_lists(Bc) * T * (S + 2) * 4);
     w.score_t = w.code_t + round16(T * Bp * 2);
-    w.g_packed = w.score_t + round16(T * Bp * 4);
+    w.g_packed = whole_rows(w.score_t + T * Bp * 4);
     w.total = w.g_packed + (Bc + 1) * slices(Do) * SC * 4;
     return w;
 }
@@ -1123,7 +1124,7 @@ RowsWorkspace rows_layout(int64_t B, int64_t I, int64_t rows, int64_t Dv) {
     w.rank = round16((lists * VT + 1) * 4);
     w.off = w.rank + round16(n * 4);
     w.pairs = w.off + round16(lists * (VT + 2) * 4);
-    w.g_packed = w.pairs + round16((n + 7 * lists) * 8 + 8);
+    w.g_packed = whole_rows(w.pairs + (n + 7 * lists) * 8 + 8);
     w.flags = w.g_packed + (Bc + 1) * slices(Dv) * SC * 4;
     w.total = w.flags + TABLE_FLAGS * 4;
     return w;
