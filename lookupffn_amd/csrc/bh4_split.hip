@@ -44,7 +44,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BS = 64;          // block size this file is built for
 constexpr int PAD = 4;          // floats of padding per row of the fp32 tile
-constexpr unsigned REPEAT_TILES = 128;      // tiles that one repeat after the other takes
 constexpr float TOP = 16384.f;  // what the largest of a row is scaled to at least (and less than twice that)
 
 // Largest and smallest over the wavefront.
@@ -249,13 +248,20 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     const int c = lane & 15;                      // A operand: output column; B operand and result: token
     const int kq = lane >> 4;                     // operands: columns 16*kq .. + 15 of the block; result: output columns 4*kq .. + 3
     // A workgroup takes one repeat of its tokens: few tokens with several repeats are as many workgroups more.  The repeats of
-    // REPEAT_TILES tiles come one after the other in the grid (on the same XCDs, as that is a multiple of their number), so that the
-    // second still finds the tokens' rows in the L2, and a stage's weights serve as many tiles in a row.  32768 tokens, D = 512,
-    // two repeats, all tiles of a repeat after all of the one before -> so: layer 259 -> 255 us, training step 1473 -> 1464 (groups of 32 to 512 the same).
-    const unsigned in_order = blockIdx.y * gridDim.x + blockIdx.x, group = in_order / (REPEAT_TILES * gridDim.y);
-    const unsigned group_tiles = min(REPEAT_TILES, gridDim.x - group * REPEAT_TILES), in_group = in_order - group * (REPEAT_TILES * gridDim.y);
-    const int r = __builtin_amdgcn_readfirstlane(in_group / group_tiles);
-    const unsigned tile_no = __builtin_amdgcn_readfirstlane(group * REPEAT_TILES + in_group % group_tiles);
+    // GROUP tiles come one after the other in the grid (on the same XCDs, as that is a multiple of their number), so that the
+    // second still finds the tokens' rows in the L2.  32768 tokens, D = 512, two repeats, all tiles of a repeat after all of the one
+    // before -> groups of 128: hash 2 to 4 us of a layer's 259, backward 244 -> 231 us (32 to 512 the same); but the training form 168 -> 173, which keeps
+    // the old order.
+    constexpr unsigned GROUP = 128;
+    unsigned repeat = blockIdx.y, tile_no = blockIdx.x;
+    if constexpr (FORM != TRAIN) {
+        const unsigned in_order = blockIdx.y * gridDim.x + blockIdx.x, group = in_order / (GROUP * gridDim.y);
+        const unsigned group_tiles = min(GROUP, gridDim.x - group * GROUP), in_group = in_order - group * (GROUP * gridDim.y);
+        repeat = in_group / group_tiles;
+        tile_no = group * GROUP + in_group % group_tiles;
+    }
+    const int r = __builtin_amdgcn_readfirstlane(repeat);
+    tile_no = __builtin_amdgcn_readfirstlane(tile_no);
     const int64_t tok_base = int64_t(tile_no) * TOK;
     if (!BWD) {
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
