@@ -98,7 +98,7 @@ MEASURED_TRAFFIC = {
     "cfg3": {"bytes": 1072501827, "form": "record stream (four lanes per token), 2048 tokens per workgroup"},
     "cfg3bf16": {"bytes": 757701017, "form": "record stream (four lanes per token), 1024 tokens per workgroup"},
     "cfg3f16": {"bytes": 770419298, "form": "record stream (four lanes per token), 1024 tokens per workgroup"},
-    "cfg5": {"bytes": 942744083, "form": "sorted"},
+    "cfg5": {"bytes": 796624011, "form": "sorted, 64 columns"},
 }
 
 
@@ -365,7 +365,7 @@ def main_backward(args):
                      "achieved": row_bytes / (scatter_ms * 1e-3) / 1e9, "peak": L2_READ_PEAK_GBS, "unit": "GB/s",
                      "frac": row_bytes / (scatter_ms * 1e-3) / 1e9 / L2_READ_PEAK_GBS,
                      "peak_basis": "16 channels x 128 B/clk per XCD x 8 XCDs x 2.4 GHz",
-                     "traffic": measured_traffic("cfg5", "sorted"),
+                     "traffic": measured_traffic("cfg5", "sorted, 64 columns"),
                      "row_read_bytes": row_bytes, "avg_kernel_ms": scatter_ms,
                      "hbm": {"compulsory_bytes": compulsory, "frac_of_peak": compulsory / (scatter_ms * 1e-3) / 1e9 / HBM_PEAK_GBS},
                      "logical_gbps": achieved, "algorithmic_bytes": scatter_bytes},
