@@ -248,10 +248,10 @@ __global__ __launch_bounds__(256 * BG, BG > 1 || NB <= 8 ? 4 : 2) void bh4_split
     const int c = lane & 15;                      // A operand: output column; B operand and result: token
     const int kq = lane >> 4;                     // operands: columns 16*kq .. + 15 of the block; result: output columns 4*kq .. + 3
     // A workgroup takes one repeat of its tokens: few tokens with several repeats are as many workgroups more.  The repeats of
-    // GROUP tiles come one after the other in the grid (on the same XCDs, as that is a multiple of their number), so that the
-    // second still finds the tokens' rows in the L2.  32768 tokens, D = 512, two repeats, all tiles of a repeat after all of the one
-    // before -> groups of 128: hash 2 to 4 us of a layer's 259, backward 244 -> 231 us (32 to 512 the same); but the training form 168 -> 173, which keeps
-    // the old order.
+    // GROUP tiles come one after the other in the grid (on the same XCDs, as that is a multiple of their number), so that what they share, the
+    // tokens' rows forward, lines and pages of z and of the scores' gradient backward, is read close together.  32768 tokens, D = 512, two
+    // repeats, all tiles of a repeat after all of the one before -> groups of 128: backward 244 -> 231 us, hash 2 to 4 us of a layer's 259 (groups of 64
+    // the same, 256 241 of 238, 512 248); but the training form 168 -> 173, which keeps the old order.
     constexpr unsigned GROUP = 128;
     unsigned repeat = blockIdx.y, tile_no = blockIdx.x;
     if constexpr (FORM != TRAIN) {
