@@ -17,7 +17,7 @@
 //                                    and sums over its four lanes
 //
 // The sums of a (token, table) stay in a register of one lane across the slices and are stored once:
-// no atomics, no zero-fill, a fixed order of additions (slice by slice).  The four-lane sum transposes
+// no atomics, no zero-fill, a fixed order of additions (slice by slice, with few pairs a chunk from a slice of the XCD's on).  The four-lane sum transposes
 // as it goes: the two values of a pass (first and second table of the pair) end up in the even and the
 // odd lanes of the quad, three DPP operations and two selects for both.
 //
@@ -179,7 +179,13 @@ __global__ __launch_bounds__(WG) void lookup_inner_quad_kernel(InnerQuadArgs a) 
     const size_t table_bytes = (size_t)a.S * a.row_bytes;
     const size_t pair_stride = 2 * table_bytes;
     const char *chunk_base = a.tables + (size_t)k0 * pair_stride;
-    auto step_base = [&](int slice, int kk) { return chunk_base + (size_t)kk * pair_stride + (size_t)slice * 128; };
+    // With few pairs a chunk an XCD begins with a slice of its own and goes round: at the same one, all of them ask for the same columns of
+    // rows that are a power of two or little else apart, a part of the memory's channels.  g row-major, us: 4096 x 128 x 768 84 -> 74, 2048 x 128 x 768 83 ->
+    // 75, 2500 x 256 x 512 78 -> 67, 4096 x 128 x 512 in the operator's pass 53 -> 46 (the pass 192 -> 183); g slice-major the same either way.  With four
+    // pairs a chunk, where a slice takes four steps and g comes slice-major, a training step is 0.2 to 0.4 % longer so (16384 x 768, 32768 x 512).
+    const int first_slice = C < 4 ? xcd * a.nslices / XCDS : 0;
+    auto place = [&](int slice) { return slice + first_slice < a.nslices ? slice + first_slice : slice + first_slice - a.nslices; };
+    auto step_base = [&](int slice, int kk) { return chunk_base + (size_t)kk * pair_stride + (size_t)place(slice) * 128; };
     const size_t quarter = (size_t)(WG / 16) * a.row_bytes;
     const uint32_t copy_off = ((tid & 15) < 8 ? 0u : (uint32_t)table_bytes) + (uint32_t)(tid >> 4) * (uint32_t)a.row_bytes +
                               (uint32_t)(tid & 7) * 16u;
@@ -217,7 +223,8 @@ __global__ __launch_bounds__(WG) void lookup_inner_quad_kernel(InnerQuadArgs a) 
         // hoisted out of the slice loop the NP row pointers would cost 2*NP registers
         asm volatile("" : "+v"(tok_low));
         const int64_t tok = min(int64_t(tok_low) + int64_t(p) * 256, a.B - 1);
-        const float *gp = a.g + tok * a.g_token_stride + (size_t)(slice >> 1) * a.g_pair_stride + ((slice & 1) * SLICE_COLS + g_col);
+        const int at = place(slice);
+        const float *gp = a.g + tok * a.g_token_stride + (size_t)(at >> 1) * a.g_pair_stride + ((at & 1) * SLICE_COLS + g_col);
         gq[p][0] = *reinterpret_cast<const float4 *>(gp + half0 * 16);
         gq[p][1] = *reinterpret_cast<const float4 *>(gp + (half0 ^ 1) * 16);
     };

@@ -39,3 +39,16 @@ def test_inner_where_one_table_pair_a_workgroup_may_pay(B, T, Do):
         rows = tables[t, code[:, t]].astype(np.float64)
         want, bound = (rows * g).sum(1), (np.abs(rows) * np.abs(g)).sum(1) * Do * 2.0 ** -24
         assert (np.abs(got[:, t] - want) <= bound).all()
+
+
+# every XCD goes round the slices from one of its own: slices that are fewer than the XCDs, no multiple of them, more; one pair and two a workgroup
+@pytest.mark.parametrize("B,T,Do", [(8000, 64, 64), (7173, 64, 320), (4096, 128, 576), (2100, 200, 832), (3000, 250, 1088)])
+def test_inner_goes_round_every_slice(B, T, Do):
+    rng = np.random.RandomState(B + Do)
+    tables, g = rng.randn(T, 256, Do).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    code = rng.randint(0, 256, size=(B, T)).astype(np.int32)
+    got = cabi.lookup_inner(code, g, tables)
+    for t in range(0, T, 7):
+        rows = tables[t, code[:, t]].astype(np.float64)
+        want, bound = (rows * g).sum(1), (np.abs(rows) * np.abs(g)).sum(1) * Do * 2.0 ** -24
+        assert (np.abs(got[:, t] - want) <= bound).all()
