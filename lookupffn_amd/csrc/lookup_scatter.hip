@@ -142,8 +142,8 @@ __global__ __launch_bounds__(WG) void lookup_scatter_lds_kernel(ScatterArgs a) {
 // table, every groups-th: it lists the (token, score) pairs of each row, and a wavefront adds up a row's products in registers (in
 // fp64, as above) and writes the whole row: plain streaming stores from many wavefronts.  A row's pairs are listed in any order, which
 // fp64 sums do not show but for ties of the final rounding.  128 tables of 768 columns: 64 tokens 35.8 -> 18.2 us (100 MB
-// written: 5.5 TB/s), 1024 tokens 76.5 -> 35.5, 2048 112 -> 77 (the sorted form 102), 3072 131 against the sorted form's 112; 512
-// tables of 1024 columns: 64 tokens 179 -> 100, 2048 430 (sorted 453).
+// written: 5.5 TB/s), 1024 tokens 76.5 -> 35.5, 2048 112 -> 77 (the sorted form 79); 512
+// tables of 1024 columns: 64 tokens 179 -> 100, 1500 268 (sorted 261), 2048 409 (288).
 //
 // Rows of many pairs would leave that to one wavefront, a chain of loads (2048 tokens of which half fall on one row of 128 tables of
 // 768 columns: 264 us).  A row of more than LONG_ROW pairs, and of four times the average, is summed by all workgroups of its

@@ -40,7 +40,7 @@
 //     a piece boundary go to slots, and the wavefront in whose piece one ends adds its parts in order.  The sum order is fixed
 //     (run-to-run reproducible), and eight partial sums of a bucket (four lane groups, even and odd steps) keep its error where it was.
 // Eight wavefronts a workgroup, two of them a compute unit for their LDS; 12 or 16 wavefronts are slower (285, 310 us).  All launches,
-// before (padded lists of 16384 tokens, 32 columns, rows stored as they end) -> now: 16384 x 128 x 768 331 -> 305 us, x 512 221 -> 204; 32768 x 128 x 512
+// before (padded lists of 16384 tokens, 32 columns, rows stored as they end) -> now, sums in fp32: 16384 x 128 x 768 331 -> 305 us, x 512 221 -> 204; 32768 x 128 x 512
 // 446 -> 413; 8192 x 128 x 768 194 -> 152; 4096 x 128 x 768 140 -> 95, x 512 92 -> 73; 16384 x 512 x 1024 1507 -> 1514.  What is left at 16384 x 128 x 768, taken
 // apart: without bucket ends -12 us, with lists from the L2 -28, rows from the L1 -47, all three 228 of 285, of which 25 to 35 are starts and ends of workgroups in step
 // with each other.  Fetching the lists' lines or the next list's rows ahead through the scalar cache gives nothing, nor does a
@@ -56,7 +56,7 @@ constexpr int SORT_WAVES = SORT_WG / 64;
 constexpr int MAX_S = 512;
 constexpr int XCDS = 8;
 constexpr int64_t CHUNK = 16384;    // tokens of a launch
-constexpr int64_t SUB = 8192;       // tokens whose pairs are sorted together, at most
+constexpr int64_t SUB = 8192;       // tokens whose pairs are sorted together, at most (all of a launch for sums in doubles)
 constexpr int SORT_DEPTH = CHUNK / SORT_WG;    // batches of 64 tokens whose loads are in flight per wavefront
 
 constexpr int SC = 64;               // columns per slice: 16 lanes x float4
