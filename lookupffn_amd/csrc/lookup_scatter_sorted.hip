@@ -352,8 +352,8 @@ template <bool ADD, typename Sum>
 __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(SortedArgs a) {
     extern __shared__ float4 lds4[];
     float *row_s = reinterpret_cast<float *>(lds4);             // [S][SC]: the rows' sums
-    float *slot = row_s + a.S * SC;                             // [WAVES][2][SC]
-    int *flag_s = reinterpret_cast<int *>(slot + WAVES * 2 * SC);    // [2][WAVES][4]: head bucket, it closes here, tail bucket
+    Sum *slot = reinterpret_cast<Sum *>(row_s + a.S * SC);      // [WAVES][2][SC], and where sums go that belong in no slot
+    int *flag_s = reinterpret_cast<int *>(slot + (WAVES * 2 + 1) * SC);      // [2][WAVES][4]: head bucket, it closes here, tail bucket
     int *off_s = flag_s + 2 * WAVES * 4;                        // [2][S + 2]
 
     // neighbouring tables of a slice on one XCD
@@ -365,7 +365,8 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = lane >> 4, i16 = lane & 15;
     const int my_col = i16 * 4 + (lane >> 5) + ((lane >> 3) & 2);
-    const int slot0 = (a.S + wave * 2) * SC + my_col;          // (a column's place in the LDS as a whole: one index serves rows and slots)
+    // fp32: a column's place in the LDS as a whole, so that one index serves rows and slots; doubles: in the slots
+    const int slot0 = ((sizeof(Sum) == 4 ? a.S : 0) + wave * 2) * SC + my_col, no_slot = WAVES * 2 * SC + my_col;
 
     constexpr int OFFS = (MAX_S + 2 + MWG - 1) / MWG;
     int next_off[OFFS];                                       // a thread's offsets of a list
@@ -432,11 +433,13 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
             const int *off = off_s + (sub & 1) * (a.S + 2);
             int next_b = __builtin_amdgcn_readlane(ends, 0);
             closes = head_bucket >= 0 && __builtin_amdgcn_readfirstlane(off[cur + 1]) <= e_hi ? 1 : 0;
-            // where the sum of the bucket at hand goes: its row, or, if it began in an earlier piece, this wavefront's first slot
-            int dst = head_bucket >= 0 ? slot0 : cur * SC + my_col;
+            constexpr int SUMS = sizeof(Sum) == 4 ? 2 : 1;    // the even and the odd steps', so that an fp32 sum is one of eight
+            // where the sum of the bucket at hand goes: its row, or, if it began in an earlier piece, this wavefront's first slot.  Doubles,
+            // whose rows hold nothing before, are written to both, the row of a cut bucket once more by whoever closes it, others' slot nobody's: a
+            // branch here costs 3 to 8 % where codes have Zipf's distribution.
+            int dst = head_bucket >= 0 ? slot0 : SUMS == 2 ? cur * SC + my_col : no_slot;
             float before = head_bucket >= 0 ? 0.f : row_s[cur * SC + my_col];      // what the row holds: the sum over earlier lists
             const char *gs = reinterpret_cast<const char *>(a.g + ((size_t)slice * (a.B + 1) + (size_t)sub * a.sub_len) * SC);
-            constexpr int SUMS = sizeof(Sum) == 4 ? 2 : 1;    // the even and the odd steps', so that an fp32 sum is one of eight
             Sum acc[SUMS][4];
             auto clear = [&]() {
 #pragma unroll
@@ -447,8 +450,13 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
                 if constexpr (SUMS == 2)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[0][e] += acc[1][e];
-                const float v = (float)sum_groups(acc[0]);
-                row_s[dst] = before + v;
+                const Sum v = sum_groups(acc[0]);
+                if constexpr (SUMS == 2) {
+                    row_s[dst] = before + v;
+                } else {
+                    slot[dst] = v;
+                    row_s[cur * SC + my_col] = (float)v;
+                }
             };
             // Lane i of group q gets the pair that the group takes in step i (loaded so, sixteen lanes would be sixteen lines).
             auto turned = [&](unsigned v) { return __builtin_amdgcn_ds_bpermute((i16 * 4 + grp) * 4, (int)v); };
@@ -489,8 +497,8 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
                         }
                         next_b = __builtin_amdgcn_readlane(ends, cur + 1 - first_end);
                     } while (next_b == end);                  // skip codes without tokens
-                    dst = cur * SC + my_col;
-                    before = row_s[dst];
+                    dst = SUMS == 2 ? cur * SC + my_col : no_slot;
+                    if (SUMS == 2) before = row_s[dst];
                     clear();
                     from = to;
                 } while (next_b < e + 4);
@@ -544,7 +552,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         __syncthreads();
         // a bucket cut by piece boundaries: the wavefront in whose piece it ends adds its parts
         if (closes) {                                         // uniform
-            float sum = slot[wave * 2 * SC + lane];
+            Sum sum = slot[wave * 2 * SC + lane];
             for (int k = wave - 1; k >= 0; --k) {
                 if (__builtin_amdgcn_readfirstlane(flag[k * 4 + 2]) >= 0) {
                     sum = slot[(k * 2 + 1) * SC + lane] + sum;
@@ -552,7 +560,9 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
                 }
                 if (__builtin_amdgcn_readfirstlane(flag[k * 4 + 0]) >= 0) sum = slot[k * 2 * SC + lane] + sum;
             }
-            row_s[head_bucket * SC + lane] += sum;
+            float &row = row_s[head_bucket * SC + lane];
+            if constexpr (sizeof(Sum) == 4) row += sum;
+            else row = (float)sum;
         }
         ++sub;
         if (!last_list) begin_list();
@@ -593,7 +603,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
 // one workgroup per (table of a.S rows, slice)
 template <bool ADD, typename Sum>
 int launch_sorted_form(SortedArgs a, hipStream_t st) {
-    const size_t lds = (size_t(a.S) + WAVES * 2) * SC * sizeof(float) + (2 * WAVES * 4 + size_t(2) * (a.S + 2)) * sizeof(int);
+    const size_t lds = size_t(a.S) * SC * sizeof(float) + (WAVES * 2 + 1) * SC * sizeof(Sum) + (2 * WAVES * 4 + size_t(2) * (a.S + 2)) * sizeof(int);
     static LdsGrant granted;
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD, Sum>), lds, granted)) return LFFN_ERR_LAUNCH;
     a.per_xcd = (a.T * a.nslices + XCDS - 1) / XCDS;
@@ -604,7 +614,7 @@ int launch_sorted_form(SortedArgs a, hipStream_t st) {
 // Calls of fewer products than this and of at most CHUNK tokens have their sums in doubles: the LDS form (lookup_scatter.hip) has, which
 // served the layer there and takes longer from LFFN_SCATTER_SORTED_WORK products on.  They cost little beside the loads (3000 tokens of
 // 128 tables of 768 columns 81 -> 90 us, 4096 x 64 x 512 50 -> 53; the LDS form 192 and 64), and the error against 64 bits is 2.6e-8
-// (fp32 5.5e-8 to 5.7e-8, the LDS form's products rounded to fp32 3.6e-8).
+// (fp32 5.5e-8 to 5.7e-8, the LDS form's products rounded to fp32 3.6e-8), whatever pieces cut: a row's parts stay doubles and are rounded once.
 inline bool sums_in_doubles(int64_t B, int64_t T, int64_t Do) {
     return B <= CHUNK && double(B) * double(T) * double(Do) < LFFN_SCATTER_DOUBLE_WORK;
 }

@@ -105,3 +105,26 @@ def test_which_calls_the_lists_serve():
     assert not ops.lookup_backward_is_fused(2048, 128, 256, 512) and not ops.lookup_backward_is_fused(4096, 32, 256, 256)
     assert ops.lookup_backward_is_fused(2049, 128, 256, 512) and ops.lookup_backward_is_fused(16384, 32, 256, 256)
     assert not ops.lookup_backward_is_fused(16385, 32, 256, 512) and ops.lookup_backward_is_fused(32768, 128, 256, 512)
+
+
+@pytest.mark.parametrize("B,T,Do", [(2049, 2, 64), (4096, 2, 128), (9001, 2, 96), (16384, 1, 64)])
+@pytest.mark.parametrize("codes", ["one row", "a tenth", "zipf", "even"])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_double_sums_are_rounded_once(B, T, Do, codes, accumulate):
+    """However many pieces a row's tokens are in: products of two fp32 numbers are exact in a double, n additions are within n * 2^-53 of the
+    sum of magnitudes, and there is one rounding to fp32, or two with what is added to."""
+    rng = np.random.RandomState(B + len(codes))
+    code = {"one row": lambda: np.full((B, T), 77), "a tenth": lambda: np.where(rng.rand(B, T) < 0.1, 77, rng.randint(0, 256, (B, T))),
+            "zipf": lambda: (rng.zipf(1.1, (B, T)) - 1) % 256, "even": lambda: rng.randint(0, 256, (B, T))}[codes]().astype(np.int32)
+    w, g = rng.rand(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    init = rng.randn(T, 256, Do).astype(np.float32) if accumulate else None
+    got = cabi.lookup_scatter_sorted(code, w, g, 256, accumulate=accumulate, init=init).astype(np.float64)
+    for t in range(T):
+        rows = np.zeros((256, B))
+        rows[code[:, t], np.arange(B)] = w[:, t]
+        want, scale = rows @ g.astype(np.float64), rows @ np.abs(g).astype(np.float64)
+        bound = 2.0 ** -24 * np.abs(want) + np.bincount(code[:, t], minlength=256)[:, None] * 2.0 ** -52 * scale
+        if accumulate:
+            want = init[t] + want
+            bound += 2.0 ** -24 * (np.abs(want) + bound)
+        assert (np.abs(got[t] - want) <= bound).all()
