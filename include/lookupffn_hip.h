@@ -725,7 +725,8 @@ int lffn_lookup_scatter_f32(const int32_t *code, const float *score, const float
  * last kernel walks the sorted lists and adds the rows of g in registers; rows of
  * grad_tables are written with plain stores and the order of additions is fixed (token order
  * inside a code), so results are reproducible from run to run, unlike the reference's
- * atomics.  Tokens are taken 16384 at a time (the workspace is sized for one such chunk).
+ * atomics.  With accumulate != 0, rows that no token points at are neither read nor written.
+ * Tokens are taken 16384 at a time (the workspace is sized for one such chunk).
  * About twice as fast as lffn_lookup_scatter_f32 at 16384 tokens x 128 tables x 768
  * columns; slower below LFFN_SCATTER_SORTED_WORK multiply-adds (B * T * Do).
  * lffn_lookup_scatter_workspace_bytes sets *bytes to the workspace this form needs for a

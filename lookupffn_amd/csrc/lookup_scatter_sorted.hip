@@ -578,19 +578,29 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     //   8192 x 64 x 512  217 -> 202, 232 -> 240, 283 -> 284    2500 x 128 x 768  266 -> 265, 332 -> 337, 462 -> 462    8192 x 256 x 512  601 -> 586, 671 -> 662
     const int S = (int)min<int64_t>(a.S, a.rows - (int64_t)t * a.S);      // the last table of a row count that a.S does not divide
     if (i16 * 4 >= a.Do - slice * SC) return;                 // (the last slice may be half a one)
+    // ADD: rows that no token points at stay as they are, to the bit, and are not touched (somebody else may be adding to them).  The offsets of both
+    // lists are still there.
+    auto live = [&](int row) {
+        if (row >= S) return false;
+        if (!ADD) return true;
+        const int *const o = off_s + row, *const o2 = o + (a.subs - 1) * (a.S + 2);
+        return o[1] > o[0] || o2[1] > o2[0];
+    };
     constexpr int DEPTH = 4;
     float *const first = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC + i16 * 4;
     for (int r0 = tid >> 4; r0 < S; r0 += MWG / 16 * DEPTH) {
         float4 v[DEPTH];
+        bool mine[DEPTH];
 #pragma unroll
         for (int k = 0; k < DEPTH; ++k) {
             const int row = r0 + k * (MWG / 16);
-            if (ADD && row < S) v[k] = *reinterpret_cast<const float4 *>(first + (size_t)row * a.Do);
+            mine[k] = live(row);
+            if (ADD && mine[k]) v[k] = *reinterpret_cast<const float4 *>(first + (size_t)row * a.Do);
         }
 #pragma unroll
         for (int k = 0; k < DEPTH; ++k) {
             const int row = r0 + k * (MWG / 16);
-            if (row >= S) continue;
+            if (!mine[k]) continue;
             const float4 sum = lds4[row * (SC / 4) + i16];
             v[k] = ADD ? add4(v[k], sum) : sum;
             float *p = first + (size_t)row * a.Do;

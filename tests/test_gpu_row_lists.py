@@ -128,3 +128,34 @@ def test_double_sums_are_rounded_once(B, T, Do, codes, accumulate):
             want = init[t] + want
             bound += 2.0 ** -24 * (np.abs(want) + bound)
         assert (np.abs(got[t] - want) <= bound).all()
+
+
+@pytest.mark.parametrize("B,T,S,Do", [(40, 2, 256, 96), (3000, 2, 512, 64), (9000, 2, 256, 64), (16384 + 50, 2, 256, 32)])
+def test_rows_without_tokens_stay_as_they_are(B, T, S, Do):
+    """Added to, a row that no token of the call points at keeps its bits: negative zeros, and numbers that are none."""
+    rng = np.random.RandomState(B)
+    code = rng.randint(0, S // 4, (B, T)).astype(np.int32) * 4
+    code[B // 2:] = np.where(code[B // 2:] == 16, 20, code[B // 2:])       # row 16: in the first list only (row 24 is in no list of table 1)
+    code[:, 1] = np.where(code[:, 1] == 24, 28, code[:, 1])
+    w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    init = np.where(np.arange(S)[None, :, None] % 8 < 4, np.float32(-0.0), np.float32("nan")) * np.ones((T, S, Do), np.float32)
+    got = cabi.lookup_scatter_sorted(code, w, g, S, accumulate=True, init=init)
+    for t in range(T):
+        untouched = np.bincount(code[:, t], minlength=S) == 0
+        assert untouched.sum() >= S // 2 and np.array_equal(got[t, untouched].view(np.uint32), init[t, untouched].view(np.uint32))
+        assert not np.signbit(got[t, ~untouched]).all()
+
+
+def test_flat_rows_without_tokens_stay_as_they_are():
+    rng = np.random.RandomState(7)
+    B, I, rows, Dv = 9000, 4, 1500, 96
+    idx = (rng.randint(0, rows // 3, (B, I)) * 3).astype(np.int32)
+    idd, gd, wd = torch.from_numpy(idx).cuda(), torch.randn(B, Dv, device="cuda"), torch.rand(B, I, device="cuda")
+    size = ctypes.c_int64()
+    assert _lib.load().lffn_scatter_rows_workspace_bytes(B, I, rows, Dv, ctypes.byref(size)) == 0 and size.value > 0
+    ws, out = torch.full((size.value,), 0x7f, dtype=torch.uint8, device="cuda"), torch.full((rows, Dv), -0.0, device="cuda")
+    assert _lib.load().lffn_scatter_rows(idd.data_ptr(), gd.data_ptr(), wd.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), B, I, rows, Dv,
+                                         0, 1, _lib.stream_of(gd)) == 0
+    untouched = np.bincount(idx.ravel(), minlength=rows) == 0
+    got = out.cpu().numpy()
+    assert (got[untouched].view(np.uint32) == 0x80000000).all() and (got[~untouched] != 0).any(1).all()
