@@ -202,17 +202,18 @@ static inline bool lffn_record_layout_ok(int64_t B, int64_t record_stride, int64
            record_stride >= (B + tile_tokens - 1) / tile_tokens * tile_tokens;
 }
 
-// lookup_inner.hip: the four-lanes-per-token score gradient where the shape qualifies (not exported)
+// lookup_inner.hip: the four-lanes-per-token score gradient where the shape qualifies (not exported).  go_round: workgroups of few table pairs
+// may begin with other slices than the first
 __attribute__((visibility("hidden")))
 bool lffn_internal_lookup_inner_quad_try(const int32_t *code, const float *g, int64_t g_token_stride,
                                          int64_t g_pair_stride, const void *tables, float *grad_score, int64_t B,
-                                         int64_t T, int64_t S, int64_t Do, void *stream, int *rc);
+                                         int64_t T, int64_t S, int64_t Do, bool go_round, void *stream, int *rc);
 
 // lookup_inner_quad.hip: the score gradient with four lanes per token and one owner per (token, table) (not exported)
 __attribute__((visibility("hidden")))
 int lffn_internal_lookup_inner_quad(const int32_t *code, const float *g, int64_t g_token_stride, int64_t g_pair_stride,
                                     const void *tables, float *grad_score, int64_t B, int64_t T, int64_t S, int64_t Do,
-                                    int np, int c, void *stream);
+                                    int np, int c, bool go_round, void *stream);
 
 static inline int lffn_launch_status() {
     return hipGetLastError() == hipSuccess ? LFFN_OK : LFFN_ERR_LAUNCH;

@@ -289,17 +289,18 @@ static int quad_chunk(int64_t B, int64_t T, int64_t Do) {
 
 // The four-lanes-per-token kernel (lookup_inner_quad.hip) where the shape qualifies: S = 256, T even, tiles of
 // 1024 tokens x chunks of quad_chunk table pairs.  g: token b's 32 columns of slice s at g + b * g_token_stride + s / 2 * g_pair_stride +
-// s % 2 * 32 floats.  Returns
+// s % 2 * 32 floats.  go_round: workgroups of few pairs may begin with other slices than the first, which the calls with the promise of equal bits
+// (lffn_lookup_inner_f32 and lffn_lookup_backward_f32) do only up to the tokens of one launch, where both cut the batch the same way.  Returns
 // false when the shape does not qualify (nothing launched), true with the launch status in *rc otherwise.
 bool lffn_internal_lookup_inner_quad_try(const int32_t *code, const float *g, int64_t g_token_stride,
                                          int64_t g_pair_stride, const void *tables, float *grad_score, int64_t B,
-                                         int64_t T, int64_t S, int64_t Do, void *stream, int *rc) {
+                                         int64_t T, int64_t S, int64_t Do, bool go_round, void *stream, int *rc) {
     if (!(S == MAX_S && T % 2 == 0 && Do % 32 == 0 && B >= 1 && reinterpret_cast<uintptr_t>(code) % 8 == 0 &&
           2 * S * Do * 4 < (int64_t(1) << 32)))
         return false;
     const int c = quad_chunk(B, T, Do);
     if (!c || (B + 1023) / 1024 * ((T / 2 + c - 1) / c) > (int64_t(1) << 30)) return false;
-    *rc = lffn_internal_lookup_inner_quad(code, g, g_token_stride, g_pair_stride, tables, grad_score, B, T, S, Do, 4, c, stream);
+    *rc = lffn_internal_lookup_inner_quad(code, g, g_token_stride, g_pair_stride, tables, grad_score, B, T, S, Do, 4, c, go_round, stream);
     return true;
 }
 
@@ -319,7 +320,8 @@ extern "C" int lffn_lookup_inner_f32(const int32_t *code, const float *g, const 
     {
         int rc = LFFN_OK;
         if (lffn_internal_lookup_inner_tokens_try(code, g, tables, grad_score, B, T, S, Do, stream, &rc)) return rc;
-        if (lffn_internal_lookup_inner_quad_try(code, g, Do, 64, tables, grad_score, B, T, S, Do, stream, &rc)) return rc;
+        if (lffn_internal_lookup_inner_quad_try(code, g, Do, 64, tables, grad_score, B, T, S, Do, B <= LFFN_SCATTER_CHUNK_TOKENS, stream, &rc))
+            return rc;
     }
 
     if (S > MAX_S || !lds_form(B, T, Do)) return lffn_internal_lookup_inner_token_major(code, g, tables, grad_score, B, T, S, Do, stream);
@@ -392,7 +394,7 @@ extern "C" int lffn_indexed_inner_product_ws_f32(const int32_t *idx, const float
     {
         TableGuardScope scope(flags);
         int rc_quad = LFFN_OK;
-        taken = lffn_internal_lookup_inner_quad_try(idx, g, Dv, 64, src, out, B, I, MAX_S, Dv, stream, &rc_quad);
+        taken = lffn_internal_lookup_inner_quad_try(idx, g, Dv, 64, src, out, B, I, MAX_S, Dv, true, stream, &rc_quad);
         if (taken && rc_quad != LFFN_OK) return rc_quad;
     }
     return lffn_internal_inner_flat(idx, g, src, out, B, I, source_size, Dv, taken ? flags : nullptr, stream);

@@ -17,7 +17,7 @@
 //                                    and sums over its four lanes
 //
 // The sums of a (token, table) stay in a register of one lane across the slices and are stored once:
-// no atomics, no zero-fill, a fixed order of additions (slice by slice, with few pairs a chunk from a slice of the XCD's on).  The four-lane sum transposes
+// no atomics, no zero-fill, a fixed order of additions (slice by slice, with few pairs a chunk from a slice of the pair's own on).  The four-lane sum transposes
 // as it goes: the two values of a pass (first and second table of the pair) end up in the even and the
 // odd lanes of the quad, three DPP operations and two selects for both.
 //
@@ -34,8 +34,8 @@
 //     compiler, which places waits by the worst path, would then wait for everything (the copies just
 //     issued included) at the top of every step: measured, 30 % of the kernel's time.
 // Measured at 16384 tokens x 128 tables x 256 x 768 (MI355X, NP = 4, C = 4): 140-150 us against 234 us
-// for the form with atomics in lookup_inner.hip; 130-140 us with g slice-major ([Do/32][B][32]: a
-// tile's slice contiguous instead of one 128-byte line per 3 KB).  Without the g loads the loop runs
+// for the form with atomics in lookup_inner.hip; 130-140 us with g slice-major ([Do/64][B + 1][64]: a
+// tile's two slices contiguous instead of one 128-byte line per 3 KB).  Without the g loads the loop runs
 // in 113 us.  Pulling the next slice of g into L2 ahead of the loads (a share per step) and issuing a
 // step's four copies one per pass instead of together both cost more instructions on the vector
 // memory path than they saved in waiting (173 against 161 us; no change).  NP = 6 and 8 (fewer table
@@ -62,6 +62,7 @@ struct InnerQuadArgs {
     int ntiles, nchunks, nslices, per_xcd;
     int group_tiles;       // tiles per tile group (see the unit order in the kernel)
     int row_bytes;         // Do * 4
+    int sections;          // the pairs in as many parts, each beginning with another slice (chunks of few pairs; 1: all begin with the first)
     TableGuard guard;
 };
 
@@ -179,11 +180,13 @@ __global__ __launch_bounds__(WG) void lookup_inner_quad_kernel(InnerQuadArgs a) 
     const size_t table_bytes = (size_t)a.S * a.row_bytes;
     const size_t pair_stride = 2 * table_bytes;
     const char *chunk_base = a.tables + (size_t)k0 * pair_stride;
-    // With few pairs a chunk an XCD begins with a slice of its own and goes round: at the same one, all of them ask for the same columns of
-    // rows that are a power of two or little else apart, a part of the memory's channels.  g row-major, us: 4096 x 128 x 768 84 -> 74, 2048 x 128 x 768 83 ->
-    // 75, 2500 x 256 x 512 78 -> 67, 4096 x 128 x 512 in the operator's pass 53 -> 46 (the pass 192 -> 183); g slice-major the same either way.  With four
-    // pairs a chunk, where a slice takes four steps and g comes slice-major, a training step is 0.2 to 0.4 % longer so (16384 x 768, 32768 x 512).
-    const int first_slice = C < 4 ? xcd * a.nslices / XCDS : 0;
+    // With few pairs a chunk the pairs that one XCD has begin with a slice of their own and go round: at the same one, all workgroups ask for the
+    // same columns of rows that are a power of two or little else apart, a part of the memory's channels.  g row-major, us: 4096 x 128 x 768 84 -> 74, 2048 x 128 x 768
+    // 83 -> 75, 2500 x 256 x 512 78 -> 67, 4096 x 128 x 512 in the operator's pass 53 -> 46 (the pass 192 -> 183); g slice-major the same either way.
+    // Chunks of four pairs, where a slice takes four steps, don't: 16384 x 128 x 768 138 -> 144, a training step 0.9 % longer.  Which slice goes by
+    // the pair alone: a token's sums don't depend on the tile that it is in.
+    // (By the eighth of the pairs, where an XCD has pairs of several eighths of fewer tiles, 16384 x 32 x 512 41 -> 52, g coming from beyond the L2.)
+    const int first_slice = C < 4 ? k0 * a.sections / npairs * a.nslices / a.sections : 0;
     auto place = [&](int slice) { return slice + first_slice < a.nslices ? slice + first_slice : slice + first_slice - a.nslices; };
     auto step_base = [&](int slice, int kk) { return chunk_base + (size_t)kk * pair_stride + (size_t)place(slice) * 128; };
     const size_t quarter = (size_t)(WG / 16) * a.row_bytes;
@@ -387,6 +390,7 @@ int launch_inner_quad(InnerQuadArgs a, hipStream_t stream) {
         a.group_tiles = best;
     }
     const int groups = (a.ntiles + a.group_tiles - 1) / a.group_tiles;
+    if (a.sections > 1) a.sections = std::max(1, XCDS / groups);      // ranges of chunks that XCDs have
     const int units = groups * a.nchunks * a.group_tiles;       // the last group's missing tiles included
     a.per_xcd = (units + XCDS - 1) / XCDS;
     const size_t lds_bytes = size_t(2) * BUF_BYTES + TOUCH_SINK_BYTES;
@@ -405,11 +409,12 @@ int launch_inner_quad(InnerQuadArgs a, hipStream_t stream) {
 // s / 2 * g_pair_stride + s % 2 * 32 floats (the strides multiples of 4).  256 * np tokens and c table pairs per workgroup.
 int lffn_internal_lookup_inner_quad(const int32_t *code, const float *g, int64_t g_token_stride, int64_t g_pair_stride,
                                     const void *tables, float *grad_score, int64_t B, int64_t T, int64_t S, int64_t Do,
-                                    int np, int c, void *stream) {
+                                    int np, int c, bool go_round, void *stream) {
     if (S != MAX_S || T % 2 != 0 || T < 2 || Do % SLICE_COLS != 0 || B < 1) return LFFN_ERR_BAD_ARG;
     InnerQuadArgs a{};
     a.code = code; a.g = g; a.tables = static_cast<const char *>(tables); a.out = grad_score;
     a.g_token_stride = g_token_stride; a.g_pair_stride = g_pair_stride;
+    a.sections = go_round ? XCDS : 1;
     a.B = B; a.T = (int)T; a.S = (int)S; a.Do = (int)Do;
     a.nslices = (int)(Do / SLICE_COLS);
     a.row_bytes = (int)(Do * 4);

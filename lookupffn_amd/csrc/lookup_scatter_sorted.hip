@@ -55,7 +55,7 @@ constexpr int SORT_WG = 1024;
 constexpr int SORT_WAVES = SORT_WG / 64;
 constexpr int MAX_S = 512;
 constexpr int XCDS = 8;
-constexpr int64_t CHUNK = 16384;    // tokens of a launch
+constexpr int64_t CHUNK = LFFN_SCATTER_CHUNK_TOKENS;    // tokens of a launch: 16384
 constexpr int64_t SUB = 8192;       // tokens whose pairs are sorted together, at most (all of a launch for sums in doubles)
 constexpr int SORT_DEPTH = CHUNK / SORT_WG;    // batches of 64 tokens whose loads are in flight per wavefront
 
@@ -741,7 +741,7 @@ int sorted_backward(const int32_t *code, const float *score, const float *g, con
         if (grad_score) {
             // token b's 64 columns of slice s sit at g_packed + (s * (Bc + 1) + b) * 64
             if (!lffn_internal_lookup_inner_quad_try(pa.code, pa.g_packed, SC, (Bc + 1) * SC, tables, grad_score + c0 * T, Bc, T, S,
-                                                     Do, stream, &rc))
+                                                     Do, B <= CHUNK, stream, &rc))
                 rc = lffn_lookup_inner_f32(pa.code, pa.g, tables, grad_score + c0 * T, Bc, T, S, Do, stream);
             if (rc != LFFN_OK) return rc;
         }

@@ -2,6 +2,7 @@
 of their magnitudes."""
 import numpy as np
 import pytest
+import torch
 
 from tests import _cabi as cabi
 
@@ -41,7 +42,7 @@ def test_inner_where_one_table_pair_a_workgroup_may_pay(B, T, Do):
         assert (np.abs(got[:, t] - want) <= bound).all()
 
 
-# every XCD goes round the slices from one of its own: slices that are fewer than the XCDs, no multiple of them, more; one pair and two a workgroup
+# the pairs of an XCD go round the slices from one of their own: slices that are fewer than the XCDs, no multiple of them, more; one pair and two a workgroup
 @pytest.mark.parametrize("B,T,Do", [(8000, 64, 64), (7173, 64, 320), (4096, 128, 576), (2100, 200, 832), (3000, 250, 1088)])
 def test_inner_goes_round_every_slice(B, T, Do):
     rng = np.random.RandomState(B + Do)
@@ -52,3 +53,23 @@ def test_inner_goes_round_every_slice(B, T, Do):
         rows = tables[t, code[:, t]].astype(np.float64)
         want, bound = (rows * g).sum(1), (np.abs(rows) * np.abs(g)).sum(1) * Do * 2.0 ** -24
         assert (np.abs(got[:, t] - want) <= bound).all()
+
+
+# the batch cut into launches of 16384 tokens, whose chunks have other numbers of pairs than the whole has
+@pytest.mark.parametrize("B,T,Do", [(32768, 32, 512), (32768, 64, 128), (16384 + 4096, 128, 256), (16384, 32, 512), (4096, 128, 512), (3000, 130, 64)])
+def test_both_gradients_at_once_have_the_bits_of_the_separate_calls(B, T, Do):
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    code = torch.randint(0, 256, (B, T), generator=gen, device="cuda", dtype=torch.int32)
+    score, g, tables = (torch.randn(*n, generator=gen, device="cuda") for n in ((B, T), (B, Do), (T, 256, Do)))
+    code, score, g, tables = (v.cpu().numpy() for v in (code, score, g, tables))
+    assert np.array_equal(cabi.lookup_backward(code, score, g, tables, want=(True, False))[0], cabi.lookup_inner(code, g, tables))
+
+
+# one pair a workgroup and two; the same token everywhere.  Neighbours read the two halves of a row in different orders, by the token's number mod 4
+@pytest.mark.parametrize("B,T,Do", [(4096, 128, 512), (8192, 64, 320), (5000, 128, 768), (16384, 32, 256)])
+def test_a_token_has_the_same_bits_in_every_tile(B, T, Do):
+    rng = np.random.RandomState(T)
+    tables, g = rng.randn(T, 256, Do).astype(np.float32), rng.randn(1, Do).astype(np.float32)
+    code = rng.randint(0, 256, size=(1, T)).astype(np.int32)
+    got = cabi.lookup_inner(code.repeat(B, 0), g.repeat(B, 0), tables)
+    assert (got[4:] == got[:-4]).all()
