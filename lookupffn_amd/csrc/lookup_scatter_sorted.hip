@@ -29,7 +29,10 @@
 //   * 64 columns, so that a list is read once per 256 bytes of a row.  A slice of 16384 rows is then 4 MB, as much as an XCD's L2, and
 //     its tokens are two lists whose rows are walked one after the other (as one list 275 -> 296 us at 16384 x 128 x 768); four lists
 //     cost more bucket ends than they give (300).
-//   * A list is cut into equal pieces, one per wavefront, whatever the bucket sizes (a skewed code distribution costs nothing).  A
+//   * A list is cut into pieces of the same cost, one per wavefront, a bucket's end taken as END_COST entries: with the same number of entries, the
+//     wavefront with the shortest buckets was waited for by all.  us, same entries -> same cost, codes by Zipf's law from row 0 on: 16384 x 128 x 768 349 -> 301,
+//     16384 x 512 x 1024 1879 -> 1577, 4096 x 128 x 768 150 -> 101, 32768 x 32 x 512 249 -> 189; the same law, rows shuffled: 302 -> 298, 1555 -> 1530, 106 -> 97, 193 -> 177;
+//     spread evenly: 292 -> 293, 1521 -> 1530, 95 -> 95, 170 -> 170.  (END_COST 4: 308, 1598, 109, 204 and 300, 1533, 98, 182; 8: 301, 1555, 98, 178 but evenly 294, 1535.)  A
 //     wavefront takes four entries a step: lane group q = lane / 16 has entry q and its sixteen lanes the 256 bytes.  Entries
 //     reach their lanes by DPP (through LDS, two permutes a step, it had 12.7 vector instructions a kilobyte for 9.3), and eight steps' loads are in flight all the
 //     time: the register of a step that is done is loaded for the step eight on.
@@ -63,6 +66,7 @@ constexpr int SC = 64;               // columns per slice: 16 lanes x float4
 constexpr int WAVES = 8;            // of the sums' workgroup
 constexpr int MWG = WAVES * 64;
 constexpr int RING = 8;              // loads in flight per wavefront
+constexpr int END_COST = 6;          // what a bucket's end costs, in entries
 
 struct PrepArgs {
     const int32_t *code;   // [B, T]
@@ -354,7 +358,8 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     float *row_s = reinterpret_cast<float *>(lds4);             // [S][SC]: the rows' sums
     Sum *slot = reinterpret_cast<Sum *>(row_s + a.S * SC);      // [WAVES][2][SC], and where sums go that belong in no slot
     int *flag_s = reinterpret_cast<int *>(slot + (WAVES * 2 + 1) * SC);      // [2][WAVES][4]: head bucket, it closes here, tail bucket
-    int *off_s = flag_s + 2 * WAVES * 4;                        // [2][S + 2]
+    int *cut_s = flag_s + 2 * WAVES * 4;                        // [2][WAVES + 2]: where pieces begin, the last one's end, the list's first line
+    int *off_s = cut_s + 2 * (WAVES + 2);                       // [2][S + 1]
 
     // neighbouring tables of a slice on one XCD
     const int unit = (int)(blockIdx.x % XCDS) * a.per_xcd + (int)(blockIdx.x / XCDS);
@@ -368,21 +373,39 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     // fp32: a column's place in the LDS as a whole, so that one index serves rows and slots; doubles: in the slots
     const int slot0 = ((sizeof(Sum) == 4 ? a.S : 0) + wave * 2) * SC + my_col, no_slot = WAVES * 2 * SC + my_col;
 
-    constexpr int OFFS = (MAX_S + 2 + MWG - 1) / MWG;
-    int next_off[OFFS];                                       // a thread's offsets of a list
+    // A list's offsets: thread q has those of row q, where its bucket starts and ends.  A piece's cost is its entries and its buckets' ends, and
+    // all pieces' are the same: else the wavefront with the shortest buckets would be waited for by all.  A piece begins in the row
+    // that its share of the cost falls to, on a whole line of pairs.
+    static_assert(MAX_S <= MWG, "a row a thread");
+    int next_off = 0, next_end = 0, list_entries = 0, list_line = 0;
     auto load_offsets = [&](int sub) {
-#pragma unroll
-        for (int k = 0; k < OFFS; ++k)
-            if (tid + k * MWG < a.S + 2) next_off[k] = a.off[((size_t)sub * a.T + t) * (a.S + 2) + tid + k * MWG];
+        const int32_t *off = a.off + ((size_t)sub * a.T + t) * (a.S + 2), *mine = off + min(tid, a.S - 1);
+        next_off = mine[0];
+        next_end = mine[1];
+        list_entries = off[a.S];
+        list_line = off[a.S + 1];
     };
-    auto keep_offsets = [&](int *off) {
+    auto keep_offsets = [&](int sub) {
+        int *off = off_s + (sub & 1) * (a.S + 1), *cuts = cut_s + (sub & 1) * (WAVES + 2);
+        if (tid < a.S) {
+            off[tid] = next_off;
+            const int first = next_off + END_COST * tid, cost = next_end - next_off + END_COST;      // of the row
+            const int whole = __builtin_amdgcn_readfirstlane(list_entries) + END_COST * a.S;
 #pragma unroll
-        for (int k = 0; k < OFFS; ++k)
-            if (tid + k * MWG < a.S + 2) off[tid + k * MWG] = next_off[k];
+            for (int w = 1; w < WAVES; ++w) {
+                const int at = (int)((unsigned)(w * whole) / WAVES) - first;
+                if ((unsigned)at < (unsigned)cost) cuts[w] = min(next_off + at, next_end) & ~7;
+            }
+        }
+        if (tid == a.S - 1) off[a.S] = cuts[WAVES] = next_end;
+        if (tid == 0) {
+            cuts[0] = 0;
+            cuts[WAVES + 1] = list_line;
+        }
     };
     load_offsets(0);
     for (int q = tid; q < a.S * (SC / 4); q += MWG) lds4[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-    keep_offsets(off_s);
+    keep_offsets(0);
     __syncthreads();
 
     // What a wavefront knows of its piece of the list at hand, and its first pairs.
@@ -393,7 +416,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     // The ends of 64 buckets, one a lane, so that nothing waits for LDS at a bucket's end; those that the piece does not reach lie
     // beyond every entry.
     auto load_ends = [&]() {
-        int v = off_s[(sub & 1) * (a.S + 2) + min(first_end + lane, a.S)];
+        int v = off_s[(sub & 1) * (a.S + 1) + min(first_end + lane, a.S)];
         v = v < e_hi ? v : INT_MAX;
         asm volatile("" : "+v"(v));                           // (waited for here, not where one is read)
         return v;
@@ -401,12 +424,12 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     // 64 pairs as they lie, past the piece's end weight 0 and the row of zeros
     auto load_pairs = [&](int e) { return pp[min(e + lane, e_hi - 1)]; };
     auto begin_list = [&]() {
-        const int *off = off_s + (sub & 1) * (a.S + 2);
-        const int n = __builtin_amdgcn_readfirstlane(off[a.S]), pieces = (n + 7) >> 3;
-        e_lo = (int)((int64_t)wave * pieces / WAVES) * 8;
-        e_hi = min((int)((int64_t)(wave + 1) * pieces / WAVES) * 8, n);
+        const int *off = off_s + (sub & 1) * (a.S + 1);
+        const int *cuts = cut_s + (sub & 1) * (WAVES + 2) + wave;
+        e_lo = __builtin_amdgcn_readfirstlane(cuts[0]);
+        e_hi = __builtin_amdgcn_readfirstlane(cuts[1]);
         tokens = a.B - sub * a.sub_len;                       // the row of zeros, from the list's first token on
-        pp = a.pairs + (int64_t)__builtin_amdgcn_readfirstlane(off[a.S + 1]) * 8;
+        pp = a.pairs + (int64_t)__builtin_amdgcn_readfirstlane(cuts[WAVES + 1 - wave]) * 8;
         head_bucket = -1;
         if (e_lo >= e_hi) return;                             // uniform
         pr0 = load_pairs(e_lo);
@@ -430,7 +453,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         int *flag = flag_s + (sub & 1) * WAVES * 4;
         int closes = 0, goes_on = 0;
         if (e_lo < e_hi) {
-            const int *off = off_s + (sub & 1) * (a.S + 2);
+            const int *off = off_s + (sub & 1) * (a.S + 1);
             int next_b = __builtin_amdgcn_readlane(ends, 0);
             closes = head_bucket >= 0 && __builtin_amdgcn_readfirstlane(off[cur + 1]) <= e_hi ? 1 : 0;
             constexpr int SUMS = sizeof(Sum) == 4 ? 2 : 1;    // the even and the odd steps', so that an fp32 sum is one of eight
@@ -548,7 +571,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         flag[wave * 4 + 0] = head_bucket;                     // (every lane the same)
         flag[wave * 4 + 1] = closes;
         flag[wave * 4 + 2] = goes_on ? cur : -1;
-        if (!last_list) keep_offsets(off_s + (~sub & 1) * (a.S + 2));
+        if (!last_list) keep_offsets(sub + 1);
         __syncthreads();
         // a bucket cut by piece boundaries: the wavefront in whose piece it ends adds its parts
         if (closes) {                                         // uniform
@@ -583,7 +606,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     auto live = [&](int row) {
         if (row >= S) return false;
         if (!ADD) return true;
-        const int *const o = off_s + row, *const o2 = o + (a.subs - 1) * (a.S + 2);
+        const int *const o = off_s + row, *const o2 = o + (a.subs - 1) * (a.S + 1);
         return o[1] > o[0] || o2[1] > o2[0];
     };
     constexpr int DEPTH = 4;
@@ -613,7 +636,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
 // one workgroup per (table of a.S rows, slice)
 template <bool ADD, typename Sum>
 int launch_sorted_form(SortedArgs a, hipStream_t st) {
-    const size_t lds = size_t(a.S) * SC * sizeof(float) + (WAVES * 2 + 1) * SC * sizeof(Sum) + (2 * WAVES * 4 + size_t(2) * (a.S + 2)) * sizeof(int);
+    const size_t lds = size_t(a.S) * SC * sizeof(float) + (WAVES * 2 + 1) * SC * sizeof(Sum) + (2 * WAVES * 4 + 2 * (WAVES + 2) + size_t(2) * (a.S + 1)) * sizeof(int);
     static LdsGrant granted;
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD, Sum>), lds, granted)) return LFFN_ERR_LAUNCH;
     a.per_xcd = (a.T * a.nslices + XCDS - 1) / XCDS;

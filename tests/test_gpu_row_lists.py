@@ -159,3 +159,42 @@ def test_flat_rows_without_tokens_stay_as_they_are():
     untouched = np.bincount(idx.ravel(), minlength=rows) == 0
     got = out.cpu().numpy()
     assert (got[untouched].view(np.uint32) == 0x80000000).all() and (got[~untouched] != 0).any(1).all()
+
+
+def _rows_within(code, w, g, S, got, init=None, doubles=False):
+    """Every row of `got` against float64.  Doubles are rounded once, or twice with what is added to.  An fp32 sum goes through no longer chain than an eighth of its
+    row's tokens, or of those in a piece (an eighth of a list of at most 8192, by entries and six for every row), and some twenty additions of parts, lists and launches:
+    one lost or doubled pair of a row of 16384 is more than that."""
+    B, T = code.shape
+    code, w, g = (torch.from_numpy(v).cuda() for v in (code, w, g))
+    for t in range(T):
+        rows = code[:, t].long()
+        want, scale = (torch.zeros(S, g.shape[1], dtype=torch.float64, device="cuda").index_add_(0, rows, a.double()[:, t, None] * b.double())
+                       for a, b in ((w, g), (w.abs(), g.abs())))
+        n = torch.bincount(rows, minlength=S)[:, None].double()
+        if doubles:
+            bound = 2.0 ** -24 * want.abs() + n * 2.0 ** -52 * scale
+        else:
+            bound = (n.clamp(max=(8192 + 6 * S) / 8 + 8) / 8 + 20) * 2.0 ** -24 * scale
+        if init is not None:
+            want = want + torch.from_numpy(init[t]).cuda().double()
+            bound = bound + 2.0 ** -24 * (want.abs() + bound) * (1 if doubles else 4)
+        off = (torch.from_numpy(got[t]).cuda().double() - want).abs() - bound
+        assert off.max() <= 0, (t, off.argmax() // g.shape[1], off.max())
+
+
+# pieces are cut by what rows cost: rows of one token each, of none but one, shrinking ones, the many in the last row, fewer tokens than rows
+@pytest.mark.parametrize("n", [24, 200, 1000, 8192, 8193, 16384])
+@pytest.mark.parametrize("S", [2, 8, 256, 512])
+@pytest.mark.parametrize("doubles", [False, True])
+def test_pieces_of_skewed_rows(n, S, doubles):
+    rng = np.random.RandomState(n + S)
+    shrinking = np.minimum((rng.exponential(size=n) * S / 12).astype(int), S - 1)
+    spread = np.arange(n) % S
+    last = np.where(np.arange(n) < min(n // 4, S - 1), spread, S - 1)
+    one = np.full(n, S // 2)
+    code = np.stack([shrinking, S - 1 - shrinking, spread, rng.permutation(last), one], 1).astype(np.int32)
+    if not doubles:                                         # behind 16384 tokens, so that these are a launch of their own, in fp32
+        code = np.concatenate([rng.randint(0, S, (16384, 5)).astype(np.int32), code])
+    w, g = rng.randn(*code.shape).astype(np.float32), rng.randn(len(code), 96).astype(np.float32)
+    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S), doubles=doubles)
