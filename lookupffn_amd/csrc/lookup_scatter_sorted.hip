@@ -23,7 +23,9 @@
 // whole lines; written straight from the ranks, every wavefront store was 64 separate 8-byte requests.  More than SUB tokens are two
 // lists, each sorted by half of the wavefronts (a workgroup per list: 28 -> 34 us at 16384 tokens).  Nothing is padded.
 //
-// lookup_scatter_sorted_kernel: one workgroup per (table, 64-column slice).  What bounds it is the compute unit's vector memory path: every
+// lookup_scatter_sorted_kernel: one workgroup per (table, 64-column slice), or more of them, each for some of the table's rows, whose entries are a part of the
+// table's lists: more than 256 rows leave no room in LDS for a second workgroup on a compute unit, and few tables of few columns would leave compute
+// units idle (launch_sorted_form).  What bounds it is the compute unit's vector memory path: every
 // pair's 256 bytes of g come out of the L2, random rows of any length at 33 TB/s where nothing else is asked for (57 bytes a clock of a
 // compute unit), and it does so with the least beside them:
 //   * 64 columns, so that a list is read once per 256 bytes of a row.  A slice of 16384 rows is then 4 MB, as much as an XCD's L2, and
@@ -57,7 +59,7 @@ namespace {
 constexpr int SORT_WG = 1024;
 constexpr int SORT_WAVES = SORT_WG / 64;
 constexpr int MAX_S = 512;
-constexpr int XCDS = 8;
+constexpr int XCDS = 8, COMPUTE_UNITS = 256;
 constexpr int64_t CHUNK = LFFN_SCATTER_CHUNK_TOKENS;    // tokens of a launch: 16384
 constexpr int64_t SUB = 8192;       // tokens whose pairs are sorted together, at most (all of a launch for sums in doubles)
 constexpr int SORT_DEPTH = CHUNK / SORT_WG;    // batches of 64 tokens whose loads are in flight per wavefront
@@ -66,6 +68,7 @@ constexpr int SC = 64;               // columns per slice: 16 lanes x float4
 constexpr int WAVES = 8;            // of the sums' workgroup
 constexpr int MWG = WAVES * 64;
 constexpr int RING = 8;              // loads in flight per wavefront
+constexpr int MAX_BLOCK_ROWS = 256;  // rows of a table that lie together in LDS
 constexpr int END_COST = 6;          // what a bucket's end costs, in entries
 
 struct PrepArgs {
@@ -309,6 +312,8 @@ struct SortedArgs {
     int64_t rows;
     int B, sub_len;        // tokens, CHUNK at most, and those of a list
     int T, S, Do, nslices, subs, per_xcd, accumulate;
+    int block_rows, block_bits;       // rows of a table that lie together in LDS: S >> block_bits
+    int part_bits;         // and into how many parts their lists are cut, a workgroup each
     int more;              // a later launch adds to these rows
 };
 
@@ -355,56 +360,80 @@ __device__ __forceinline__ int row_pick(int v, int u) {
 template <bool ADD, typename Sum>
 __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(SortedArgs a) {
     extern __shared__ float4 lds4[];
-    float *row_s = reinterpret_cast<float *>(lds4);             // [S][SC]: the rows' sums
-    Sum *slot = reinterpret_cast<Sum *>(row_s + a.S * SC);      // [WAVES][2][SC], and where sums go that belong in no slot
+    const int R = a.block_rows;
+    float *row_s = reinterpret_cast<float *>(lds4);             // [R][SC]: the rows' sums
+    Sum *slot = reinterpret_cast<Sum *>(row_s + R * SC);        // [WAVES][2][SC], and where sums go that belong in no slot
     int *flag_s = reinterpret_cast<int *>(slot + (WAVES * 2 + 1) * SC);      // [2][WAVES][4]: head bucket, it closes here, tail bucket
     int *cut_s = flag_s + 2 * WAVES * 4;                        // [2][WAVES + 2]: where pieces begin, the last one's end, the list's first line
-    int *off_s = cut_s + 2 * (WAVES + 2);                       // [2][S + 1]
+    int *off_s = cut_s + 2 * (WAVES + 2);                       // [2][R + 1]
 
     // neighbouring tables of a slice on one XCD
-    const int unit = (int)(blockIdx.x % XCDS) * a.per_xcd + (int)(blockIdx.x / XCDS);
-    if (unit >= a.T * a.nslices) return;                      // uniform over the workgroup
-    const int slice = unit / a.T, t = unit % a.T;
+    const int unit = (int)(blockIdx.x % XCDS) * a.per_xcd + (int)(blockIdx.x / XCDS), slice_units = a.T << (a.block_bits + a.part_bits);
+    if (unit >= slice_units * a.nslices) return;              // uniform over the workgroup
+    const int slice = unit / slice_units, block = unit - slice * slice_units >> a.part_bits, part = unit & ((1 << a.part_bits) - 1);
+    const int t = block >> a.block_bits, row0 = (block - (t << a.block_bits)) * R;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = lane >> 4, i16 = lane & 15;
     const int my_col = i16 * 4 + (lane >> 5) + ((lane >> 3) & 2);
     // fp32: a column's place in the LDS as a whole, so that one index serves rows and slots; doubles: in the slots
-    const int slot0 = ((sizeof(Sum) == 4 ? a.S : 0) + wave * 2) * SC + my_col, no_slot = WAVES * 2 * SC + my_col;
+    const int slot0 = ((sizeof(Sum) == 4 ? R : 0) + wave * 2) * SC + my_col, no_slot = WAVES * 2 * SC + my_col;
 
-    // A list's offsets: thread q has those of row q, where its bucket starts and ends.  A piece's cost is its entries and its buckets' ends, and
-    // all pieces' are the same: else the wavefront with the shortest buckets would be waited for by all.  A piece begins in the row
-    // that its share of the cost falls to, on a whole line of pairs.
-    static_assert(MAX_S <= MWG, "a row a thread");
-    int next_off = 0, next_end = 0, list_entries = 0, list_line = 0;
+    static_assert(MAX_BLOCK_ROWS <= MWG, "a row a thread");
+    auto offsets = [&](int sub) { return a.off + ((size_t)sub * a.T + t) * (a.S + 2) + row0; };
+    // The rows [r0, r1) of the block are this workgroup's.  Parts are of the same cost, as near as whole rows allow: a row's entries and END_COST for
+    // its end.
+    int r0 = 0, r1 = R;
+    if (a.part_bits > 0) {                                    // uniform
+        const int q = min(tid, R - 1);
+        int first = END_COST * a.subs * q, next = first + END_COST * a.subs, whole = END_COST * a.subs * R;
+        for (int sub = 0; sub < a.subs; ++sub) {
+            const int32_t *off = offsets(sub);
+            first += off[q] - off[0];
+            next += off[q + 1] - off[0];
+            whole += off[R] - off[0];
+        }
+        const int from = part * whole >> a.part_bits, to = (part + 1) * whole >> a.part_bits;
+        if (tid < R && first < to && to <= next) flag_s[1] = tid + 1;
+        if (part == 0 ? tid == 0 : tid < R && first < from && from <= next) flag_s[0] = part == 0 ? 0 : tid + 1;
+        __syncthreads();
+        r0 = __builtin_amdgcn_readfirstlane(flag_s[0]);
+        r1 = __builtin_amdgcn_readfirstlane(flag_s[1]);
+    }
+    // A list's offsets: thread q has those of row q, where its bucket starts and ends.  Pieces, too, are of the same cost: else the wavefront with the
+    // shortest buckets would be waited for by all.  A piece begins in the row that its share of the cost falls to, on a whole line of pairs.
+    int next_off = 0, next_end = 0, list_begin = 0, list_end = 0, list_line = 0;
     auto load_offsets = [&](int sub) {
-        const int32_t *off = a.off + ((size_t)sub * a.T + t) * (a.S + 2), *mine = off + min(tid, a.S - 1);
+        const int32_t *off = offsets(sub), *mine = off + min(tid, R - 1);
         next_off = mine[0];
         next_end = mine[1];
-        list_entries = off[a.S];
-        list_line = off[a.S + 1];
+        list_begin = off[r0];
+        list_end = off[r1];
+        list_line = off[a.S + 1 - row0];
     };
     auto keep_offsets = [&](int sub) {
-        int *off = off_s + (sub & 1) * (a.S + 1), *cuts = cut_s + (sub & 1) * (WAVES + 2);
-        if (tid < a.S) {
-            off[tid] = next_off;
-            const int first = next_off + END_COST * tid, cost = next_end - next_off + END_COST;      // of the row
-            const int whole = __builtin_amdgcn_readfirstlane(list_entries) + END_COST * a.S;
+        int *off = off_s + (sub & 1) * (R + 1), *cuts = cut_s + (sub & 1) * (WAVES + 2);
+        if (tid < R) off[tid] = next_off;
+        if (tid == R - 1) off[R] = next_end;
+        if (tid >= r0 && tid < r1) {
+            const int first = next_off - list_begin + END_COST * (tid - r0), cost = next_end - next_off + END_COST;      // of the row
+            const int whole = __builtin_amdgcn_readfirstlane(list_end - list_begin) + END_COST * (r1 - r0);
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) {
                 const int at = (int)((unsigned)(w * whole) / WAVES) - first;
-                if ((unsigned)at < (unsigned)cost) cuts[w] = min(next_off + at, next_end) & ~7;
+                if ((unsigned)at < (unsigned)cost) cuts[w] = max(min(next_off + at, next_end) & ~7, list_begin);
             }
         }
-        if (tid == a.S - 1) off[a.S] = cuts[WAVES] = next_end;
         if (tid == 0) {
-            cuts[0] = 0;
+            cuts[0] = list_begin;
+            cuts[WAVES] = list_end;
             cuts[WAVES + 1] = list_line;
         }
+        if (r0 == r1 && tid > 0 && tid < WAVES) cuts[tid] = list_begin;      // no rows, no entries
     };
     load_offsets(0);
-    for (int q = tid; q < a.S * (SC / 4); q += MWG) lds4[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int q = tid; q < R * (SC / 4); q += MWG) lds4[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     keep_offsets(0);
     __syncthreads();
 
@@ -416,7 +445,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     // The ends of 64 buckets, one a lane, so that nothing waits for LDS at a bucket's end; those that the piece does not reach lie
     // beyond every entry.
     auto load_ends = [&]() {
-        int v = off_s[(sub & 1) * (a.S + 1) + min(first_end + lane, a.S)];
+        int v = off_s[(sub & 1) * (R + 1) + min(first_end + lane, R)];
         v = v < e_hi ? v : INT_MAX;
         asm volatile("" : "+v"(v));                           // (waited for here, not where one is read)
         return v;
@@ -424,7 +453,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     // 64 pairs as they lie, past the piece's end weight 0 and the row of zeros
     auto load_pairs = [&](int e) { return pp[min(e + lane, e_hi - 1)]; };
     auto begin_list = [&]() {
-        const int *off = off_s + (sub & 1) * (a.S + 1);
+        const int *off = off_s + (sub & 1) * (R + 1);
         const int *cuts = cut_s + (sub & 1) * (WAVES + 2) + wave;
         e_lo = __builtin_amdgcn_readfirstlane(cuts[0]);
         e_hi = __builtin_amdgcn_readfirstlane(cuts[1]);
@@ -435,7 +464,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         pr0 = load_pairs(e_lo);
         pr1 = load_pairs(min(e_lo + 64, e_hi - 1));
         // the bucket holding entry e_lo: the last c with off[c] <= e_lo
-        int lo = 0, hi = a.S;                                 // invariant: off[lo] <= e_lo < off[hi]
+        int lo = r0, hi = r1;                                 // invariant: off[lo] <= e_lo < off[hi]
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (off[mid] <= e_lo) lo = mid; else hi = mid;
@@ -453,7 +482,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         int *flag = flag_s + (sub & 1) * WAVES * 4;
         int closes = 0, goes_on = 0;
         if (e_lo < e_hi) {
-            const int *off = off_s + (sub & 1) * (a.S + 1);
+            const int *off = off_s + (sub & 1) * (R + 1);
             int next_b = __builtin_amdgcn_readlane(ends, 0);
             closes = head_bucket >= 0 && __builtin_amdgcn_readfirstlane(off[cur + 1]) <= e_hi ? 1 : 0;
             constexpr int SUMS = sizeof(Sum) == 4 ? 2 : 1;    // the even and the odd steps', so that an fp32 sum is one of eight
@@ -599,30 +628,31 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     // or Adam behind it; the operator's pass, plainly -> nontemporally, alone, with SGD, with Adam:
     //   4096 x 128 x 512  231 -> 226 (219 for 229 where the passes' results stay), 270 -> 264, 317 -> 318    3000 x 128 x 512  206 -> 204, 245 -> 239, 295 -> 298
     //   8192 x 64 x 512  217 -> 202, 232 -> 240, 283 -> 284    2500 x 128 x 768  266 -> 265, 332 -> 337, 462 -> 462    8192 x 256 x 512  601 -> 586, 671 -> 662
-    const int S = (int)min<int64_t>(a.S, a.rows - (int64_t)t * a.S);      // the last table of a row count that a.S does not divide
+    const int64_t first_row = (int64_t)t * a.S + row0;
+    const int rows = (int)min<int64_t>(r1, a.rows - first_row);      // the last table of a row count that a.S does not divide: fewer, or none
     if (i16 * 4 >= a.Do - slice * SC) return;                 // (the last slice may be half a one)
     // ADD: rows that no token points at stay as they are, to the bit, and are not touched (somebody else may be adding to them).  The offsets of both
     // lists are still there.
     auto live = [&](int row) {
-        if (row >= S) return false;
+        if (row >= rows) return false;
         if (!ADD) return true;
-        const int *const o = off_s + row, *const o2 = o + (a.subs - 1) * (a.S + 1);
+        const int *const o = off_s + row, *const o2 = o + (a.subs - 1) * (R + 1);
         return o[1] > o[0] || o2[1] > o2[0];
     };
     constexpr int DEPTH = 4;
-    float *const first = a.out + (size_t)t * a.S * a.Do + (size_t)slice * SC + i16 * 4;
-    for (int r0 = tid >> 4; r0 < S; r0 += MWG / 16 * DEPTH) {
+    float *const first = a.out + (size_t)first_row * a.Do + (size_t)slice * SC + i16 * 4;
+    for (int row_k = r0 + (tid >> 4); row_k < rows; row_k += MWG / 16 * DEPTH) {
         float4 v[DEPTH];
         bool mine[DEPTH];
 #pragma unroll
         for (int k = 0; k < DEPTH; ++k) {
-            const int row = r0 + k * (MWG / 16);
+            const int row = row_k + k * (MWG / 16);
             mine[k] = live(row);
             if (ADD && mine[k]) v[k] = *reinterpret_cast<const float4 *>(first + (size_t)row * a.Do);
         }
 #pragma unroll
         for (int k = 0; k < DEPTH; ++k) {
-            const int row = r0 + k * (MWG / 16);
+            const int row = row_k + k * (MWG / 16);
             if (!mine[k]) continue;
             const float4 sum = lds4[row * (SC / 4) + i16];
             v[k] = ADD ? add4(v[k], sum) : sum;
@@ -633,13 +663,28 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     }
 }
 
-// one workgroup per (table of a.S rows, slice)
 template <bool ADD, typename Sum>
 int launch_sorted_form(SortedArgs a, hipStream_t st) {
-    const size_t lds = size_t(a.S) * SC * sizeof(float) + (WAVES * 2 + 1) * SC * sizeof(Sum) + (2 * WAVES * 4 + 2 * (WAVES + 2) + size_t(2) * (a.S + 1)) * sizeof(int);
+    // 512 rows, whole -> two blocks, us, codes spread evenly, by Zipf's law in any order of the rows, in order from row 0 on: 16384 x 128 x 256 168 -> 132, 173 -> 151,
+    // 188 -> 199; x 768 437 -> 335, 447 -> 369, 494 -> 521; 8192 x 64 x 1024 170 -> 126, 172 -> 136, 187 -> 184.
+    a.block_rows = a.S < MAX_BLOCK_ROWS ? a.S : MAX_BLOCK_ROWS;
+    a.block_bits = lffn_log2(a.S / a.block_rows);
+    const int64_t blocks = (int64_t(a.T) << a.block_bits) * a.nslices;
+    // As many parts as give every compute unit a workgroup, and twice as many where most of them would otherwise wait for the others' second.  us, whole
+    // tables -> parts, codes as above: 65536 x 32 x 256 (128 workgroups) 335 -> 250, 346 -> 271, 371 -> 273; 16384 x 32 x 256 79 -> 60, 80 -> 67, 83 -> 62;
+    // 32768 x 32 x 576 (288) 255 -> 218, 260 -> 235, 266 -> 232; 16384 x 32 x 768 (384) 125 -> 103, 127 -> 114, 128 -> 112; but 16384 x 100 x 256 (400) 117 -> 122,
+    // 118 -> 127, 122 -> 136.
+    auto more_parts = [&](int64_t least, int64_t most) {
+        const int64_t units = blocks << a.part_bits;
+        return units >= least && units <= most && a.block_rows >> a.part_bits > 16;
+    };
+    while (more_parts(0, COMPUTE_UNITS - 1)) ++a.part_bits;
+    if (more_parts(COMPUTE_UNITS + 1, COMPUTE_UNITS * 3 / 2)) ++a.part_bits;
+    const size_t lds = size_t(a.block_rows) * SC * sizeof(float) + (WAVES * 2 + 1) * SC * sizeof(Sum) +
+                       (2 * WAVES * 4 + 2 * (WAVES + 2) + size_t(2) * (a.block_rows + 1)) * sizeof(int);
     static LdsGrant granted;
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD, Sum>), lds, granted)) return LFFN_ERR_LAUNCH;
-    a.per_xcd = (a.T * a.nslices + XCDS - 1) / XCDS;
+    a.per_xcd = (int)(((blocks << a.part_bits) + XCDS - 1) / XCDS);
     hipLaunchKernelGGL((lookup_scatter_sorted_kernel<ADD, Sum>), dim3((unsigned)(a.per_xcd * XCDS)), dim3(MWG), lds, st, a);
     return lffn_launch_status();
 }

@@ -198,3 +198,24 @@ def test_pieces_of_skewed_rows(n, S, doubles):
         code = np.concatenate([rng.randint(0, S, (16384, 5)).astype(np.int32), code])
     w, g = rng.randn(*code.shape).astype(np.float32), rng.randn(len(code), 96).astype(np.float32)
     _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S), doubles=doubles)
+
+
+# a table's rows are two workgroups' or more: 512 rows; fewer tables x columns than compute units, or up to one and a half times as many.  Either side of each line, and
+# rows with more tokens than a part's share, so that parts have one row or none
+@pytest.mark.parametrize("B,T,S,Do", [(3000, 65, 512, 256), (3000, 31, 512, 256), (2500, 31, 256, 512), (2500, 32, 256, 512), (2500, 33, 256, 512), (2500, 48, 256, 512),
+                                      (2500, 49, 256, 512), (2100, 5, 64, 96), (2100, 5, 32, 64), (16384 + 2500, 31, 256, 512), (16384 + 9000, 33, 256, 480),
+                                      (16384 + 700, 9, 512, 224)])
+def test_rows_of_several_workgroups(B, T, S, Do):
+    rng = np.random.RandomState(B + T + S)
+    code = rng.randint(0, S, (B, T))
+    code[:, 0] = S - 1                                      # one row has all
+    code[:, 1] = np.where(rng.rand(B) < 0.6, S // 2, code[:, 1])
+    code[:, 2] = np.minimum(rng.exponential(size=B) * S / 12, S - 1)
+    code[:, 3] = np.where(np.arange(B) < B // 2, 0, S - 1)      # and in either list another
+    code = code.astype(np.int32)
+    w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    got = cabi.lookup_scatter_sorted(code, w, g, S)
+    _rows_within(code, w, g, S, got, doubles=B <= 16384)
+    assert np.array_equal(got, cabi.lookup_scatter_sorted(code, w, g, S))
+    init = rng.randn(T, S, Do).astype(np.float32)
+    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S, accumulate=True, init=init), init=init, doubles=B <= 16384)
