@@ -41,7 +41,7 @@ extern "C" {
 #define LFFN_ERR_LAUNCH      -3   /* hipGetLastError() after the launch was not hipSuccess */
 #define LFFN_ERR_SCRATCH     -4   /* an entry point that allocates nothing: the shape exceeds its static scratch */
 
-#define LFFN_ABI_VERSION 14
+#define LFFN_ABI_VERSION 15
 
 /* ABI version of the loaded library (LFFN_ABI_VERSION at build time). */
 int lffn_version(void);
@@ -695,11 +695,12 @@ int lffn_indexed_inner_product_f16(const int32_t *idx, const uint16_t *g, const 
 int lffn_scatter_add_f16(const int32_t *idx, const uint16_t *g, const float *w, float *out,
                          int64_t B, int64_t I, int64_t out_size, int64_t Dv, void *stream);
 
-/* Tokens up to which lffn_lookup_scatter_f32 is faster than lffn_lookup_scatter_sorted_f32 (tables of at most 256 rows): up to
- * there it sums every row of the gradient from a list of its tokens, where that is faster than summing in LDS. */
+/* Which of the two forms of the table gradient a caller should use (lffn_lookup_scatter_plan), and which sums it then has.  Up to this
+ * many tokens lffn_lookup_scatter_f32, which there sums every row from a list of its tokens where that is faster than summing in LDS; tables of
+ * many columns would be faster sorted from fewer tokens on (2048 tokens of 512 tables of 1024 columns 409 us, sorted 288), but in fp32. */
 #define LFFN_SCATTER_LIST_TOKENS 2048
-/* Beyond, from this many products (B * T * Do) on lffn_lookup_scatter_sorted_f32 and lffn_lookup_backward_f32 are the faster ones; below
- * the second number, for at most LFFN_SCATTER_CHUNK_TOKENS tokens, their sums are doubles as lffn_lookup_scatter_f32's are. */
+/* Beyond, never below this many products (B * T * Do) sorted; below the second number lffn_lookup_scatter_sorted_f32 and lffn_lookup_backward_f32
+ * have their sums in doubles, as lffn_lookup_scatter_f32 has, for at most LFFN_SCATTER_CHUNK_TOKENS tokens, the tokens of one launch. */
 #define LFFN_SCATTER_SORTED_WORK 45000000
 #define LFFN_SCATTER_DOUBLE_WORK 400000000
 #define LFFN_SCATTER_CHUNK_TOKENS 16384
@@ -728,7 +729,7 @@ int lffn_lookup_scatter_f32(const int32_t *code, const float *score, const float
  * atomics.  With accumulate != 0, rows that no token points at are neither read nor written.
  * Tokens are taken 16384 at a time (the workspace is sized for one such chunk).
  * About twice as fast as lffn_lookup_scatter_f32 at 16384 tokens x 128 tables x 768
- * columns; slower below LFFN_SCATTER_SORTED_WORK multiply-adds (B * T * Do).
+ * columns; which calls it is the faster one for, lffn_lookup_scatter_plan says.
  * lffn_lookup_scatter_workspace_bytes sets *bytes to the workspace this form needs for a
  * shape, or to 0 when the form does not cover it (S > 512, Do % 32 != 0, B == 0 or T == 0):
  * lffn_lookup_scatter_f32 covers those.  workspace: device memory, 16-byte aligned, at
@@ -736,6 +737,9 @@ int lffn_lookup_scatter_f32(const int32_t *code, const float *score, const float
  * lffn_lookup_scatter_f32 (PL/gather/cuda/kernel.py:200, PL/lookup.py:126).
  */
 int lffn_lookup_scatter_workspace_bytes(int64_t B, int64_t T, int64_t S, int64_t Do, int64_t *bytes);
+/* *sorted: 1 where lffn_lookup_scatter_sorted_f32, and lffn_lookup_backward_f32 for both gradients, are the calls to use for a shape, 0 where
+ * lffn_lookup_scatter_f32 is.  A function of the sizes alone. */
+int lffn_lookup_scatter_plan(int64_t B, int64_t T, int64_t S, int64_t Do, int32_t *sorted);
 int lffn_lookup_scatter_sorted_f32(const int32_t *code, const float *score, const float *g, float *grad_tables,
                                    void *workspace, int64_t workspace_bytes, int64_t B, int64_t T, int64_t S,
                                    int64_t Do, int32_t accumulate, void *stream);

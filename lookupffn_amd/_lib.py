@@ -16,7 +16,7 @@ _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 # LOOKUPFFN_HIP_LIB points at another build of the same ABI (e.g. a tuning build)
 LIB_PATH = os.environ.get("LOOKUPFFN_HIP_LIB") or os.path.join(_PKG_DIR, "liblookupffn_hip.so")
 
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 LFFN_OK = 0
 LFFN_ERR_BAD_ARG = -1
@@ -99,6 +99,7 @@ SIGNATURES = {
     "lffn_scatter_add_f16": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp],
     "lffn_lookup_scatter_f32": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
     "lffn_lookup_scatter_workspace_bytes": [_i64, _i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64)],
+    "lffn_lookup_scatter_plan": [_i64, _i64, _i64, _i64, ctypes.POINTER(ctypes.c_int32)],
     "lffn_lookup_scatter_sorted_f32": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
     "lffn_lookup_backward_f32": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, ctypes.c_int32, _vp],
     "lffn_gather_add_workspace_bytes": [_i64, _i64, _i64, _i64, _i32, ctypes.POINTER(_i64)],
@@ -203,8 +204,7 @@ def _load_host():
         raise ImportError(f"{HOST_PATH} was built against torch {module.torch_version}, this is {torch.__version__}")
     from . import ops
     from .lookup import BH4
-    module.bind(LIB_PATH, torch.nn.LayerNorm, BH4, (ops.SORTED_SCATTER_MIN_WORK, ops.LN_BWD_PARTIALS,
-                                                   ops.PROJECT_BWD_PARTIALS, ops.COLUMN_SUM_CHUNK_ROWS))
+    module.bind(LIB_PATH, torch.nn.LayerNorm, BH4, (ops.LN_BWD_PARTIALS, ops.PROJECT_BWD_PARTIALS, ops.COLUMN_SUM_CHUNK_ROWS))
     return module
 
 

@@ -60,6 +60,7 @@ using torch::autograd::variable_list;
     X(lffn_bh4_fold_split_both_f32)         \
     X(lffn_bh4_fold_mode_f32)               \
     X(lffn_lookup_scatter_workspace_bytes)  \
+    X(lffn_lookup_scatter_plan)             \
     X(lffn_lookup_backward_sums_f32)        \
     X(lffn_lookup_backward_sums_rows)       \
     X(lffn_lookup_inner_f32)                \
@@ -92,7 +93,7 @@ struct Config {
 
 // The Python operators' own (bind).
 struct Thresholds {
-    int64_t sorted_min_work, ln_partials, project_partials, sum_chunk_rows;
+    int64_t ln_partials, project_partials, sum_chunk_rows;
 } limits;
 PyTypeObject *layer_norm_type, *bh4_type;
 
@@ -377,10 +378,9 @@ struct LookupFFNBackward : public torch::autograd::Node {
         if (need[TABLES]) out[TABLES] = at::empty_like(tab);
         if (need_score || need[TABLES]) {
             int64_t ws_bytes = 0;
-            CALL(lffn_lookup_scatter_workspace_bytes, B, T, S, Do, &ws_bytes);
-            if (B <= LFFN_SCATTER_LIST_TOKENS || B * T * Do < limits.sorted_min_work ||
-                (B > LFFN_SCATTER_CHUNK_TOKENS && B * T * Do < LFFN_SCATTER_DOUBLE_WORK))
-                ws_bytes = 0;
+            int32_t sorted = 0;
+            CALL(lffn_lookup_scatter_plan, B, T, S, Do, &sorted);
+            if (sorted) CALL(lffn_lookup_scatter_workspace_bytes, B, T, S, Do, &ws_bytes);
             if (need[TABLES] && ws_bytes > 0) {
                 Tensor ws = empty_bytes(ws_bytes, dev);
                 if (need_score) {
@@ -523,8 +523,8 @@ bool watched_over() {
 // bind(path of the kernel library, nn.LayerNorm, BH4, the operators' thresholds)
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    TORCH_CHECK(n == 4 && PyType_Check(args[1]) && PyType_Check(args[2]) && PyTuple_Check(args[3]) && PyTuple_GET_SIZE(args[3]) == 4,
-                "bind: a path, two types and four numbers");
+    TORCH_CHECK(n == 4 && PyType_Check(args[1]) && PyType_Check(args[2]) && PyTuple_Check(args[3]) && PyTuple_GET_SIZE(args[3]) == 3,
+                "bind: a path, two types and three numbers");
     const char *p = PyUnicode_AsUTF8(args[0]);
     if (!p) return nullptr;
     void *h = dlopen(p, RTLD_NOW | RTLD_NOLOAD);
@@ -537,8 +537,8 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
     LFFN_ENTRIES(X)
 #undef X
     Thresholds t{};
-    for (int i = 0; i < 4; ++i)
-        TORCH_CHECK(whole(PyTuple_GET_ITEM(args[3], i), (&t.sorted_min_work)[i]), "bind: a threshold is no integer");
+    for (int i = 0; i < 3; ++i)
+        TORCH_CHECK(whole(PyTuple_GET_ITEM(args[3], i), (&t.ln_partials)[i]), "bind: a threshold is no integer");
     Py_INCREF(args[1]);
     Py_INCREF(args[2]);
     lib = found;

@@ -1105,19 +1105,21 @@ def _(indexes, source, weights, output_size):
     return source.new_empty(output_size, source.shape[1], dtype=torch.float32)
 
 
-# From this many multiply-adds (B * T * Do) on the sorted scatter is the faster one (LFFN_SCATTER_SORTED_WORK of the C header; both gradients,
-# by the LDS-accumulating scatter -> sorted, us: 4096 x 32 x 256 43 -> 50, 6000 x 32 x 256 65 -> 60, 2049 x 64 x 512 67 -> 68, 3000 x 64 x
-# 512 106 -> 86, 4096 x 128 x 512 168 -> 125, 3000 x 128 x 768 273 -> 163, 3000 x 256 x 512 322 -> 185)
+# LFFN_SCATTER_SORTED_WORK, _DOUBLE_WORK, _CHUNK_TOKENS and _LIST_TOKENS of the C header, whose lffn_lookup_scatter_plan says where the sorted scatter is the
+# faster one: never below the first many multiply-adds (B * T * Do) and for no more tokens than the last; below the second many, for at most the
+# third many tokens, its sums are doubles.
 SORTED_SCATTER_MIN_WORK = 45 * 10 ** 6
-# below this many its sums are doubles as the other's are, for at most so many tokens (LFFN_SCATTER_DOUBLE_WORK, LFFN_SCATTER_CHUNK_TOKENS)
 DOUBLE_SCATTER_WORK, SCATTER_CHUNK_TOKENS = 4 * 10 ** 8, 16384
-# and up to this many tokens (LFFN_SCATTER_LIST_TOKENS of the C header) the one that sums rows from lists of their tokens is
 LIST_SCATTER_MAX_TOKENS = 2048
 
 
-def _sorted_scatter_pays(B, T, Do):
-    work = B * T * Do
-    return B > LIST_SCATTER_MAX_TOKENS and work >= SORTED_SCATTER_MIN_WORK and (B <= SCATTER_CHUNK_TOKENS or work >= DOUBLE_SCATTER_WORK)
+def _sorted_scatter_workspace(B, T, S, Do):
+    """Bytes of the sorted scatter's workspace where it is the form to use, else 0."""
+    lib, pays, ws_bytes = _lib.load(), ctypes.c_int32(0), ctypes.c_int64(0)
+    _lib.check(lib.lffn_lookup_scatter_plan(B, T, S, Do, ctypes.byref(pays)), "lffn_lookup_scatter_plan")
+    if pays.value:
+        _lib.check(lib.lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)), "lffn_lookup_scatter_workspace_bytes")
+    return ws_bytes.value
 
 
 _L.define("lookup_scatter(Tensor code, Tensor score, Tensor g, int S) -> Tensor")
@@ -1134,14 +1136,13 @@ def _lookup_scatter_impl(code, score, g, S):
     _check_gather_args(code, max(T * S, 1), Do)
     out = torch.empty(T, S, Do, dtype=torch.float32, device=g.device)     # fully overwritten by the kernel
     lib = _lib.load()
-    ws_bytes = ctypes.c_int64(0)
-    _lib.check(lib.lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)), "lffn_lookup_scatter_workspace_bytes")
+    ws_bytes = _sorted_scatter_workspace(B, T, S, Do)
     with _dev_guard(g):
-        if ws_bytes.value > 0 and _sorted_scatter_pays(B, T, Do):
+        if ws_bytes > 0:
             # sort the tokens of every table by code, then sum rows in registers: no atomics
-            ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=g.device)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=g.device)
             rc = lib.lffn_lookup_scatter_sorted_f32(_lib.ptr(code), _lib.ptr(score), _lib.ptr(g), _lib.ptr(out), _lib.ptr(ws),
-                                                    ws_bytes.value, B, T, S, Do, 0, _lib.stream_of(g))
+                                                    ws_bytes, B, T, S, Do, 0, _lib.stream_of(g))
             _lib.check(rc, f"lffn_lookup_scatter_sorted_f32(B={B}, T={T}, S={S}, Do={Do})")
         else:
             rc = lib.lffn_lookup_scatter_f32(_lib.ptr(code), _lib.ptr(score), _lib.ptr(g), _lib.ptr(out),
@@ -1164,12 +1165,7 @@ _L.define("lookup_backward(Tensor code, Tensor score, Tensor g, Tensor tables) -
 def lookup_backward_is_fused(B, T, S, Do):
     """Both gradients of the gather go through one call (lffn_lookup_backward_f32: the sorted scatter and the
     score gradient sharing one slice-major copy of g) for this shape."""
-    if not _sorted_scatter_pays(B, T, Do) or Do % 64 != 0:
-        return False
-    ws_bytes = ctypes.c_int64(0)
-    _lib.check(_lib.load().lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)),
-               "lffn_lookup_scatter_workspace_bytes")
-    return ws_bytes.value > 0
+    return Do % 64 == 0 and _sorted_scatter_workspace(B, T, S, Do) > 0
 
 
 def _lookup_backward_impl(code, score, g, tables):
@@ -1185,14 +1181,13 @@ def _lookup_backward_impl(code, score, g, tables):
     if not lookup_backward_is_fused(B, T, S, Do):
         return _lookup_inner_impl(code, g, tables), _lookup_scatter_impl(code, score, g, S)
     lib = _lib.load()
-    ws_bytes = ctypes.c_int64(0)
-    _lib.check(lib.lffn_lookup_scatter_workspace_bytes(B, T, S, Do, ctypes.byref(ws_bytes)), "lffn_lookup_scatter_workspace_bytes")
+    ws_bytes = _sorted_scatter_workspace(B, T, S, Do)
     grad_score = torch.empty(B, T, dtype=torch.float32, device=g.device)          # both fully overwritten
     grad_tables = torch.empty(T, S, Do, dtype=torch.float32, device=g.device)
-    ws = torch.empty(ws_bytes.value, dtype=torch.uint8, device=g.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=g.device)
     with _dev_guard(g):
         rc = lib.lffn_lookup_backward_f32(_lib.ptr(code), _lib.ptr(score), _lib.ptr(g), _lib.ptr(tables), _lib.ptr(grad_score),
-                                          _lib.ptr(grad_tables), _lib.ptr(ws), ws_bytes.value, B, T, S, Do, 0, _lib.stream_of(g))
+                                          _lib.ptr(grad_tables), _lib.ptr(ws), ws_bytes, B, T, S, Do, 0, _lib.stream_of(g))
     _lib.check(rc, f"lffn_lookup_backward_f32(B={B}, T={T}, S={S}, Do={Do})")
     return grad_score, grad_tables
 

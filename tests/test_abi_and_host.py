@@ -234,6 +234,37 @@ def test_workspace_queries_are_host_side_plans():
         assert scatter_ws(*shape) == 0, shape
 
 
+def test_which_calls_the_sorted_scatter_serves():
+    """lffn_lookup_scatter_plan, the operators' questions to it, and the header's numbers as the operators have them."""
+    from lookupffn_amd import ops
+    lib = _lib.load()
+
+    def plan(B, T, S, Do):
+        n = ctypes.c_int32(-1)
+        assert lib.lffn_lookup_scatter_plan(B, T, S, Do, ctypes.byref(n)) == 0
+        assert ops.lookup_backward_is_fused(B, T, S, Do) == (n.value == 1 and Do % 64 == 0)
+        return n.value
+
+    # from 45e6 products and 2049 tokens on where the form in LDS takes more than a round of 256 workgroups, or half a one
+    assert plan(2049, 128, 256, 512) == plan(3000, 128, 256, 768) == plan(2049, 64, 256, 384) == plan(16384, 32, 256, 256) == 1
+    assert plan(2048, 128, 256, 512) == plan(4096, 32, 256, 256) == plan(2048, 512, 256, 1024) == 0
+    # a round nearly full is the other form's, up to some thousand tokens
+    assert plan(4600, 64, 256, 256) == plan(11999, 48, 256, 320) == 0 and plan(12000, 48, 256, 320) == plan(4600, 65, 256, 256) == 1
+    # few tables of many columns do not repay the copy of the gradient
+    assert plan(16384, 1, 256, 4096) == plan(16384, 4, 256, 4096) == plan(8192, 8, 256, 4096) == plan(16384, 16, 256, 1024) == 0
+    assert plan(16384, 16, 256, 512) == plan(16384, 16, 256, 768) == plan(16384, 24, 256, 768) == 1
+    # from 4e8 products on always, below it only in one launch, where the sums are doubles
+    assert plan(16385, 32, 256, 512) == 0 and plan(32768, 32, 256, 512) == plan(16384, 8, 256, 4096) == plan(32768, 128, 256, 512) == 1
+    # what the other form has only atomics for, or does not take
+    assert plan(4600, 64, 512, 256) == plan(4600, 64, 256, 288) == 1 and plan(32768, 128, 1024, 512) == plan(32768, 128, 256, 520) == plan(0, 4, 16, 64) == 0
+    assert lib.lffn_lookup_scatter_plan(16, 4, 16, 64, None) == _lib.LFFN_ERR_BAD_ARG
+
+    hdr = open(os.path.join(ROOT, "include", "lookupffn_hip.h")).read()
+    number = {k: int(v) for k, v in re.findall(r"#define (LFFN_SCATTER_\w+) (\d+)", hdr)}
+    assert number == {"LFFN_SCATTER_LIST_TOKENS": ops.LIST_SCATTER_MAX_TOKENS, "LFFN_SCATTER_SORTED_WORK": ops.SORTED_SCATTER_MIN_WORK,
+                      "LFFN_SCATTER_DOUBLE_WORK": ops.DOUBLE_SCATTER_WORK, "LFFN_SCATTER_CHUNK_TOKENS": ops.SCATTER_CHUNK_TOKENS}
+
+
 def test_gather_plans_are_consistent_over_a_grid_of_shapes():
     """Host-side sweep of the three gather queries over 15 000 shapes (ragged token counts, odd table
     counts, every row format).  Whenever the workspace entry point would run the four-lanes-per-token

@@ -85,7 +85,7 @@ def test_flat_rows_of_two_lists(B, I, rows, in_tables):
     assert (np.abs(got - want) <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
 
 
-@pytest.mark.parametrize("B,T,Do", [(2049, 64, 384), (3001, 32, 512), (8193, 32, 256), (16384, 33, 128)])
+@pytest.mark.parametrize("B,T,Do", [(2049, 64, 384), (3001, 33, 512), (8193, 32, 256), (16384, 33, 128)])
 def test_calls_that_had_double_sums_keep_them(B, T, Do):
     """Rounded once, a number is off by 2^-24 / 3^0.5 of its power of two, root mean square; the rows cut by pieces a few roundings more."""
     assert ops.lookup_backward_is_fused(B, T, 256, Do) and B * T * Do < ops.DOUBLE_SCATTER_WORK
@@ -99,12 +99,6 @@ def test_calls_that_had_double_sums_keep_them(B, T, Do):
         assert (grad[t] - want).norm() <= 2.0 ** -24 / 3 ** 0.5 * 1.1 * want.norm()
         want = (tables[t].double()[code[:, t].long()] * g.double()).sum(1)
         assert ((grad_score[:, t] - want).abs() <= Do * 2.0 ** -24 * (tables[t].abs()[code[:, t].long()] * g.abs()).sum(1)).all()
-
-
-def test_which_calls_the_lists_serve():
-    assert not ops.lookup_backward_is_fused(2048, 128, 256, 512) and not ops.lookup_backward_is_fused(4096, 32, 256, 256)
-    assert ops.lookup_backward_is_fused(2049, 128, 256, 512) and ops.lookup_backward_is_fused(16384, 32, 256, 256)
-    assert not ops.lookup_backward_is_fused(16385, 32, 256, 512) and ops.lookup_backward_is_fused(32768, 128, 256, 512)
 
 
 @pytest.mark.parametrize("B,T,Do", [(2049, 2, 64), (4096, 2, 128), (9001, 2, 96), (16384, 1, 64)])
