@@ -70,6 +70,7 @@ constexpr int MWG = WAVES * 64;
 constexpr int RING = 8;              // loads in flight per wavefront
 constexpr int MAX_BLOCK_ROWS = 256;  // rows of a table that lie together in LDS
 constexpr int END_COST = 6;          // what a bucket's end costs, in entries
+constexpr int CUTS = 2 * WAVES + 2;  // words about a list's pieces
 
 struct PrepArgs {
     const int32_t *code;   // [B, T]
@@ -364,8 +365,8 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     float *row_s = reinterpret_cast<float *>(lds4);             // [R][SC]: the rows' sums
     Sum *slot = reinterpret_cast<Sum *>(row_s + R * SC);        // [WAVES][2][SC], and where sums go that belong in no slot
     int *flag_s = reinterpret_cast<int *>(slot + (WAVES * 2 + 1) * SC);      // [2][WAVES][4]: head bucket, it closes here, tail bucket
-    int *cut_s = flag_s + 2 * WAVES * 4;                        // [2][WAVES + 2]: where pieces begin, the last one's end, the list's first line
-    int *off_s = cut_s + 2 * (WAVES + 2);                       // [2][R + 1]
+    int *cut_s = flag_s + 2 * WAVES * 4;                        // [2][CUTS]: where pieces begin, the last one's end, the list's first line, rows that cuts fall to
+    int *off_s = cut_s + 2 * CUTS;                              // [2][R + 1]
 
     // neighbouring tables of a slice on one XCD
     const int unit = (int)(blockIdx.x % XCDS) * a.per_xcd + (int)(blockIdx.x / XCDS), slice_units = a.T << (a.block_bits + a.part_bits);
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         list_line = off[a.S + 1 - row0];
     };
     auto keep_offsets = [&](int sub) {
-        int *off = off_s + (sub & 1) * (R + 1), *cuts = cut_s + (sub & 1) * (WAVES + 2);
+        int *off = off_s + (sub & 1) * (R + 1), *cuts = cut_s + (sub & 1) * CUTS;
         if (tid < R) off[tid] = next_off;
         if (tid == R - 1) off[R] = next_end;
         if (tid >= r0 && tid < r1) {
@@ -422,13 +423,17 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) {
                 const int at = (int)((unsigned)(w * whole) / WAVES) - first;
-                if ((unsigned)at < (unsigned)cost) cuts[w] = max(min(next_off + at, next_end) & ~7, list_begin);
+                if ((unsigned)at < (unsigned)cost) {
+                    cuts[w] = max(min(next_off + at, next_end) & ~7, list_begin);
+                    cuts[WAVES + 2 + w] = tid;
+                }
             }
         }
         if (tid == 0) {
             cuts[0] = list_begin;
             cuts[WAVES] = list_end;
             cuts[WAVES + 1] = list_line;
+            cuts[WAVES + 2] = r0;
         }
         if (r0 == r1 && tid > 0 && tid < WAVES) cuts[tid] = list_begin;      // no rows, no entries
     };
@@ -454,7 +459,7 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
     auto load_pairs = [&](int e) { return pp[min(e + lane, e_hi - 1)]; };
     auto begin_list = [&]() {
         const int *off = off_s + (sub & 1) * (R + 1);
-        const int *cuts = cut_s + (sub & 1) * (WAVES + 2) + wave;
+        const int *cuts = cut_s + (sub & 1) * CUTS + wave;
         e_lo = __builtin_amdgcn_readfirstlane(cuts[0]);
         e_hi = __builtin_amdgcn_readfirstlane(cuts[1]);
         tokens = a.B - sub * a.sub_len;                       // the row of zeros, from the list's first token on
@@ -463,13 +468,22 @@ __global__ __launch_bounds__(MWG, WAVES / 2) void lookup_scatter_sorted_kernel(S
         if (e_lo >= e_hi) return;                             // uniform
         pr0 = load_pairs(e_lo);
         pr1 = load_pairs(min(e_lo + 64, e_hi - 1));
-        // the bucket holding entry e_lo: the last c with off[c] <= e_lo
-        int lo = r0, hi = r1;                                 // invariant: off[lo] <= e_lo < off[hi]
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (off[mid] <= e_lo) lo = mid; else hi = mid;
+        // the bucket holding entry e_lo, the last c with off[c] <= e_lo: the row that the cut fell to, a neighbour, or searched for
+        cur = __builtin_amdgcn_readfirstlane(cuts[WAVES + 2]);
+        int tries = 3;
+        for (; tries > 0; --tries) {
+            const int from = __builtin_amdgcn_readfirstlane(off[cur]), to = __builtin_amdgcn_readfirstlane(off[cur + 1]);
+            if (from <= e_lo && e_lo < to) break;
+            cur += from > e_lo ? -1 : 1;
         }
-        cur = __builtin_amdgcn_readfirstlane(lo);
+        if (tries == 0) {                                     // uniform
+            int lo = r0, hi = r1;                             // invariant: off[lo] <= e_lo < off[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (off[mid] <= e_lo) lo = mid; else hi = mid;
+            }
+            cur = __builtin_amdgcn_readfirstlane(lo);
+        }
         first_end = cur + 1;
         ends = load_ends();
         head_bucket = __builtin_amdgcn_readfirstlane(off[cur] < e_lo ? cur : -1);
@@ -681,7 +695,7 @@ int launch_sorted_form(SortedArgs a, hipStream_t st) {
     while (more_parts(0, COMPUTE_UNITS - 1)) ++a.part_bits;
     if (more_parts(COMPUTE_UNITS + 1, COMPUTE_UNITS * 3 / 2)) ++a.part_bits;
     const size_t lds = size_t(a.block_rows) * SC * sizeof(float) + (WAVES * 2 + 1) * SC * sizeof(Sum) +
-                       (2 * WAVES * 4 + 2 * (WAVES + 2) + size_t(2) * (a.block_rows + 1)) * sizeof(int);
+                       (2 * WAVES * 4 + 2 * CUTS + size_t(2) * (a.block_rows + 1)) * sizeof(int);
     static LdsGrant granted;
     if (!lffn_grant_dynamic_lds(reinterpret_cast<const void *>(lookup_scatter_sorted_kernel<ADD, Sum>), lds, granted)) return LFFN_ERR_LAUNCH;
     a.per_xcd = (int)(((blocks << a.part_bits) + XCDS - 1) / XCDS);
