@@ -1,8 +1,8 @@
 """The table gradient's row sums where their lists can go wrong: tokens around one list and two, a slice that is half a one,
-buckets that end at every entry of a step, pieces that one bucket cuts, 512 rows a table.
+buckets that end at every entry of a step, pieces that one bucket cuts, 512 rows a table, rows of several workgroups.
 
-Bound: an fp32 sum of n products is within n * 2^-24 of the sum of their magnitudes, which is the scale of every element here, and
-the result's own rounding 2^-23 of it."""
+Up to 16384 tokens and 4e8 products the sums are doubles and their tokens one list; of other calls every 16384 tokens are one list or two, in fp32.  Small calls
+in fp32 are the end of one of more than 16384 tokens, whose last launch has the tokens in question and adds to the rows of the first."""
 import ctypes
 
 import numpy as np
@@ -16,51 +16,91 @@ from tests import _cabi as cabi
 pytestmark = pytest.mark.gpu
 
 
-def _check(code, w, g, S, accumulate=False):
+def _in_doubles(B, T, Do):
+    return B <= ops.SCATTER_CHUNK_TOKENS and B * T * Do < ops.DOUBLE_SCATTER_WORK
+
+
+def _bound(want, scale, n, piece, doubles):
+    """How far a row of n tokens may be off.  Doubles are rounded once.  An fp32 sum goes through no longer chain than an eighth of its row's tokens, or of those in a
+    piece, and some twenty additions of parts, lists and launches: one lost or doubled pair of a row of 16384 is more than that."""
+    if doubles:
+        return 2.0 ** -24 * want.abs() + n * 2.0 ** -52 * scale
+    return (n.clamp(max=piece) / 8 + 20) * 2.0 ** -24 * scale
+
+
+def _rows_within(code, w, g, S, got, init=None, tables=None):
+    """Every row of `got`, or of some of its tables, against float64."""
     B, T = code.shape
-    idx = code + (np.arange(T, dtype=np.int32) * S)[None]
-    want = oracle.scatter_add(idx, g.astype(np.float64), w.astype(np.float64), T * S).reshape(T, S, -1)
-    scale = oracle.scatter_add(idx, np.abs(g).astype(np.float64), np.abs(w).astype(np.float64), T * S).reshape(T, S, -1)
-    init = np.random.RandomState(1).randn(*want.shape).astype(np.float32) if accumulate else None
-    if accumulate:
-        want, scale = want + init, scale + np.abs(init)
-    got = cabi.lookup_scatter_sorted(code, w, g, S, accumulate=accumulate, init=init)
-    terms = np.bincount(code.ravel(), minlength=S).max() + 1
-    assert (np.abs(got - want) <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
-    return got
+    doubles = _in_doubles(B, T, g.shape[1])
+    code, w, g = (torch.from_numpy(v).cuda() for v in (code, w, g))
+    for t in range(T) if tables is None else tables:
+        rows = code[:, t].long()
+        weights = torch.zeros(S, B, dtype=torch.float64, device="cuda")
+        weights[rows, torch.arange(B, device="cuda")] = w[:, t].double()
+        want, scale = weights @ g.double(), weights.abs() @ g.double().abs()
+        n = torch.bincount(rows, minlength=S)[:, None].double()
+        bound = _bound(want, scale, n, (8192 + 6 * S) / 8 + 8, doubles)      # a list of at most 8192 in eight pieces, by entries and six for every row
+        if init is not None:                                # each launch that adds rounds once more
+            want = want + torch.from_numpy(init[t]).cuda().double()
+            bound = bound + 2.0 ** -24 * (want.abs() + bound) + (0 if doubles else (B // 16384 + 1) * 2.0 ** -24 * (scale + want.abs()))
+        off = (torch.from_numpy(got[t]).cuda().double() - want).abs() - bound
+        assert off.max() <= 0, (t, off.argmax() // g.shape[1], off.max())
 
 
-@pytest.mark.parametrize("B,T,S,Do", [(8192, 3, 256, 64), (8193, 2, 256, 96), (8200, 3, 512, 32), (9217, 2, 16, 160), (15871, 2, 256, 64),
-                                      (16384, 9, 1, 32), (16384 + 8193, 2, 256, 96), (37, 3, 256, 32), (513, 2, 8, 608)])
+def _behind(rng, code, S, fp32):
+    """`code` alone, or behind 16384 tokens of a launch of their own."""
+    return np.concatenate([rng.randint(0, S, (16384, code.shape[1])), code]).astype(np.int32) if fp32 else code.astype(np.int32)
+
+
+@pytest.mark.parametrize("n,T,S,Do", [(4500, 2, 256, 96), (8192, 3, 256, 64), (8193, 2, 256, 96), (8200, 3, 512, 32), (9217, 2, 16, 160), (15871, 2, 256, 64),
+                                      (16384, 9, 1, 32), (37, 3, 256, 32), (513, 2, 8, 608)])
 @pytest.mark.parametrize("skew", [False, True])
-def test_tokens_around_one_list_and_two(B, T, S, Do, skew):
-    rng = np.random.RandomState(B + S + Do)
-    code = (rng.zipf(1.2, size=(B, T)) % S if skew else rng.randint(0, S, size=(B, T))).astype(np.int32)
-    w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
-    got = _check(code, w, g, S)
+@pytest.mark.parametrize("fp32", [False, True])
+def test_tokens_around_one_list_and_two(n, T, S, Do, skew, fp32):
+    rng = np.random.RandomState(n + S + Do)
+    code = _behind(rng, rng.zipf(1.2, size=(n, T)) % S if skew else rng.randint(0, S, size=(n, T)), S, fp32)
+    B = len(code)
+    assert _in_doubles(B, T, Do) != fp32
+    w, g, init = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32), rng.randn(T, S, Do).astype(np.float32)
+    got = cabi.lookup_scatter_sorted(code, w, g, S)
+    _rows_within(code, w, g, S, got)
     assert np.array_equal(got, cabi.lookup_scatter_sorted(code, w, g, S))        # fixed order of additions
-    _check(code, w, g, S, accumulate=True)
+    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S, accumulate=True, init=init), init=init)
+
+
+# one list and two in fp32 that overwrite, as a call's first launch does
+@pytest.mark.parametrize("B,T,S,Do", [(4500, 128, 256, 768), (8193, 64, 256, 768), (9217, 64, 512, 704), (15871, 64, 16, 416), (16384, 65, 1, 384)])
+def test_lists_of_a_first_launch_in_fp32(B, T, S, Do):
+    assert not _in_doubles(B, T, Do)
+    rng = np.random.RandomState(B)
+    code, w, g = rng.randint(0, S, (B, T)).astype(np.int32), rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
+    code[:, 1] = S - 1
+    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S), tables=(0, 1, T // 2, T - 1))
 
 
 @pytest.mark.parametrize("lengths", [(1, 2, 3, 4, 5, 6, 7, 8), (1, 1, 1, 1, 1, 1, 1, 60), (63, 64, 65, 0, 0, 1, 0, 3), (0, 0, 700, 0, 1, 0, 0, 0)])
-def test_bucket_ends_at_every_entry(lengths):
+@pytest.mark.parametrize("fp32", [False, True])
+def test_bucket_ends_at_every_entry(lengths, fp32):
     rng = np.random.RandomState(sum(lengths))
-    code = np.repeat(np.arange(8), lengths).astype(np.int32)[:, None]
-    code = np.concatenate([code, rng.permutation(code)], 1)
-    _check(code, rng.randn(*code.shape).astype(np.float32), rng.randn(len(code), 96).astype(np.float32), 8)
+    code = np.repeat(np.arange(8), lengths)[:, None]
+    code = _behind(rng, np.concatenate([code, rng.permutation(code)], 1), 8, fp32)
+    w, g = rng.randn(*code.shape).astype(np.float32), rng.randn(len(code), 96).astype(np.float32)
+    assert _in_doubles(len(code), 2, 96) != fp32
+    _rows_within(code, w, g, 8, cabi.lookup_scatter_sorted(code, w, g, 8))
 
 
-def test_infinite_gradient_stays_in_its_row():
+@pytest.mark.parametrize("B", [9000, 16384 + 9000])
+def test_infinite_gradient_stays_in_its_row(B):
     rng = np.random.RandomState(5)
-    B, T, S, Do = 9000, 2, 256, 96
+    T, S, Do = 2, 256, 96
     code = rng.randint(0, S, size=(B, T)).astype(np.int32)
     code[code == 17] = 18
-    code[8500, 0] = 17                                      # alone in its bucket, amid others in its step
+    code[B - 500, 0] = 17                                     # alone in its bucket, amid others in its step
     w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
-    g[8500] = np.inf
+    g[B - 500] = np.inf
     got = cabi.lookup_scatter_sorted(code, w, g, S)
-    assert np.isinf(got[0, 17]).all() and np.isinf(got[1, code[8500, 1]]).all()
-    got[0, 17] = got[1, code[8500, 1]] = 0
+    assert np.isinf(got[0, 17]).all() and np.isinf(got[1, code[B - 500, 1]]).all()
+    got[0, 17] = got[1, code[B - 500, 1]] = 0
     assert np.isfinite(got).all()
 
 
@@ -78,11 +118,9 @@ def test_flat_rows_of_two_lists(B, I, rows, in_tables):
     ws, out = torch.full((size.value,), 0x7f, dtype=torch.uint8, device="cuda"), torch.full((rows, Dv), float("nan"), device="cuda")
     assert _lib.load().lffn_scatter_rows(idd.data_ptr(), gd.data_ptr(), wd.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), B, I, rows, Dv,
                                          0, 0, _lib.stream_of(gd)) == 0
-    got = out.cpu().numpy()
-    want = oracle.scatter_add(idx, g.astype(np.float64), w.astype(np.float64), rows)
-    scale = oracle.scatter_add(idx, np.abs(g).astype(np.float64), np.abs(w).astype(np.float64), rows)
-    terms = np.bincount(idx.ravel()).max()
-    assert (np.abs(got - want) <= scale * (terms * 2.0 ** -24 + 2.0 ** -23)).all()
+    want, scale = (torch.from_numpy(oracle.scatter_add(idx, a.astype(np.float64), b.astype(np.float64), rows)) for a, b in ((g, w), (np.abs(g), np.abs(w))))
+    n = torch.from_numpy(np.bincount(idx.ravel(), minlength=rows))[:, None].double()
+    assert ((out.cpu().double() - want).abs() <= _bound(want, scale, n, B * I, False)).all()
 
 
 @pytest.mark.parametrize("B,T,Do", [(2049, 64, 384), (3001, 33, 512), (8193, 32, 256), (16384, 33, 128)])
@@ -155,43 +193,21 @@ def test_flat_rows_without_tokens_stay_as_they_are():
     assert (got[untouched].view(np.uint32) == 0x80000000).all() and (got[~untouched] != 0).any(1).all()
 
 
-def _rows_within(code, w, g, S, got, init=None, doubles=False):
-    """Every row of `got` against float64.  Doubles are rounded once, or twice with what is added to.  An fp32 sum goes through no longer chain than an eighth of its
-    row's tokens, or of those in a piece (an eighth of a list of at most 8192, by entries and six for every row), and some twenty additions of parts, lists and launches:
-    one lost or doubled pair of a row of 16384 is more than that."""
-    B, T = code.shape
-    code, w, g = (torch.from_numpy(v).cuda() for v in (code, w, g))
-    for t in range(T):
-        rows = code[:, t].long()
-        want, scale = (torch.zeros(S, g.shape[1], dtype=torch.float64, device="cuda").index_add_(0, rows, a.double()[:, t, None] * b.double())
-                       for a, b in ((w, g), (w.abs(), g.abs())))
-        n = torch.bincount(rows, minlength=S)[:, None].double()
-        if doubles:
-            bound = 2.0 ** -24 * want.abs() + n * 2.0 ** -52 * scale
-        else:
-            bound = (n.clamp(max=(8192 + 6 * S) / 8 + 8) / 8 + 20) * 2.0 ** -24 * scale
-        if init is not None:
-            want = want + torch.from_numpy(init[t]).cuda().double()
-            bound = bound + 2.0 ** -24 * (want.abs() + bound) * (1 if doubles else 4)
-        off = (torch.from_numpy(got[t]).cuda().double() - want).abs() - bound
-        assert off.max() <= 0, (t, off.argmax() // g.shape[1], off.max())
-
-
 # pieces are cut by what rows cost: rows of one token each, of none but one, shrinking ones, the many in the last row, fewer tokens than rows
 @pytest.mark.parametrize("n", [24, 200, 1000, 8192, 8193, 16384])
 @pytest.mark.parametrize("S", [2, 8, 256, 512])
-@pytest.mark.parametrize("doubles", [False, True])
-def test_pieces_of_skewed_rows(n, S, doubles):
+@pytest.mark.parametrize("fp32", [False, True])
+def test_pieces_of_skewed_rows(n, S, fp32):
     rng = np.random.RandomState(n + S)
     shrinking = np.minimum((rng.exponential(size=n) * S / 12).astype(int), S - 1)
     spread = np.arange(n) % S
     last = np.where(np.arange(n) < min(n // 4, S - 1), spread, S - 1)
     one = np.full(n, S // 2)
-    code = np.stack([shrinking, S - 1 - shrinking, spread, rng.permutation(last), one], 1).astype(np.int32)
-    if not doubles:                                         # behind 16384 tokens, so that these are a launch of their own, in fp32
-        code = np.concatenate([rng.randint(0, S, (16384, 5)).astype(np.int32), code])
+    code = np.stack([shrinking, S - 1 - shrinking, spread, rng.permutation(last), one], 1)
+    code = _behind(rng, code, S, fp32)
+    assert _in_doubles(len(code), 5, 96) != fp32
     w, g = rng.randn(*code.shape).astype(np.float32), rng.randn(len(code), 96).astype(np.float32)
-    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S), doubles=doubles)
+    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S))
 
 
 # a table's rows are two workgroups' or more: 512 rows; fewer tables x columns than compute units, or up to one and a half times as many.  Either side of each line, and
@@ -209,7 +225,7 @@ def test_rows_of_several_workgroups(B, T, S, Do):
     code = code.astype(np.int32)
     w, g = rng.randn(B, T).astype(np.float32), rng.randn(B, Do).astype(np.float32)
     got = cabi.lookup_scatter_sorted(code, w, g, S)
-    _rows_within(code, w, g, S, got, doubles=B <= 16384)
+    _rows_within(code, w, g, S, got)
     assert np.array_equal(got, cabi.lookup_scatter_sorted(code, w, g, S))
     init = rng.randn(T, S, Do).astype(np.float32)
-    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S, accumulate=True, init=init), init=init, doubles=B <= 16384)
+    _rows_within(code, w, g, S, cabi.lookup_scatter_sorted(code, w, g, S, accumulate=True, init=init), init=init)

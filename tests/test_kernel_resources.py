@@ -1,12 +1,14 @@
 """Compile-time guard for the hand-scheduled kernels (no GPU needed: hipcc cross-compiles).
 
 The table-major kernels issue global -> LDS copies as inline assembly and wait for them with
-hand-counted `s_waitcnt vmcnt(n)`.  Two things keep that sound and neither is visible in the source:
+hand-counted `s_waitcnt vmcnt(n)`.  What keeps that sound, and what keeps the loops fast, is not visible in the source:
 
   * the four-lanes-per-token gather (lookup_gather_quad.hip) and the score-gradient kernel
     (lookup_inner_quad.hip) must not spill: a spilling variant of the former once moved registers
     to scratch while loads into them were in flight and ended in a GPU memory fault, and the
     latter's wait leaves an exact number of compiler-visible loads in flight across a barrier;
+  * the row sums (lookup_scatter_sorted.hip) keep eight steps' loads in flight and let no store sit among them, which a spill
+    would be: it costs time, not correctness;
   * the older LDS kernels (lookup_gather.hip, lookup_gather_pair.hip, lookup_inner.hip) write no
     register from inline assembly and wait with vmcnt(0) / vmcnt(1) only, where an extra scratch
     access makes a wait stricter, never weaker; their largest tiles are known to spill a few
@@ -25,7 +27,7 @@ import pytest
 
 from lookupffn_amd import _build
 
-STRICT = ["lookup_gather_quad.hip", "lookup_inner_quad.hip"]
+STRICT = ["lookup_gather_quad.hip", "lookup_inner_quad.hip", "lookup_scatter_sorted.hip"]
 LDS_FORMS = ["lookup_gather.hip", "lookup_gather_pair.hip", "lookup_inner.hip"]
 # instantiations of the older kernels that are known to spill (fp32 rows, 13 and 16 passes)
 MAY_SPILL = re.compile(r"lookup_gather_lds_kernelILb0ELi1[36]E|lookup_gather_pair_kernelILb0ELi16E")
@@ -69,6 +71,7 @@ def test_remarks_are_parsed(usage):
             assert {"ScratchSize", "VGPRs Spill", "SGPRs Spill", "VGPRs", "Dynamic Stack"} <= set(k), (src, name, k)
     assert sum("lookup_gather_quad_kernel" in n for n in usage["lookup_gather_quad.hip"]) >= 4
     assert sum("lookup_inner_quad_kernel" in n for n in usage["lookup_inner_quad.hip"]) >= 2
+    assert sum("lookup_scatter_sorted_kernel" in n for n in usage["lookup_scatter_sorted.hip"]) >= 4
 
 
 @pytest.mark.parametrize("src", STRICT)
