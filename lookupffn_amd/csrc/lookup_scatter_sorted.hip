@@ -766,14 +766,15 @@ extern "C" int lffn_lookup_scatter_workspace_bytes(int64_t B, int64_t T, int64_t
 
 // Where the sorted form is the one to use.  From LFFN_SCATTER_DOUBLE_WORK products on it is; below, lffn_lookup_scatter_f32 sums in LDS, which
 // takes 6.1 us per thousand tokens for every round of one workgroup (64 columns of a table) on each compute unit, whatever the round has.  The sorted form
-// reads and writes g once more, which few tables of many columns don't repay.  Both gradients, us, LDS form and score gradient -> sorted, codes by Zipf's
-// law in any order of the rows:
-//   more than one round     3000 x 128 x 768 250 -> 149, 2100 x 128 x 256 69 -> 63, 16384 x 24 x 768 264 -> 191, 12000 x 32 x 704 207 -> 161; 4600 x 16 x 2048
-//                           107 -> 96, 8192 x 16 x 2048 164 -> 167, but 8192 x 8 x 4096 181 -> 245
-//   half a round or less    8192 x 32 x 256 71 -> 63, 16384 x 8 x 1024 134 -> 120, 16384 x 4 x 1024 123 -> 88; but 8192 x 4 x 2048 79 -> 90, 16384 x 1 x 4096 150 -> 225
-//   up to one round         16384 x 32 x 448 144 -> 139, 12000 x 48 x 256 109 -> 99, 16384 x 16 x 768 144 -> 133; 8192 x 48 x 320 86 -> 86, 8192 x 24 x 512
-//                           86 -> 90; but 4600 x 64 x 256 59 -> 64, 16384 x 16 x 1024 158 -> 174, 16384 x 12 x 1024 147 -> 154
-// With 512 rows lffn_lookup_scatter_f32 has only atomics (16384 x 32 x 256 1785 -> 124), and columns that are no multiple of 64 it does not take.
+// reads and writes g once more, which few tables of many columns don't repay.  Training step of the layer, us, LDS form -> sorted (whose copy of g gives the output
+// bias's gradient, too):
+//   more than one round     3000 x 48 x 384 157 -> 130, 16384 x 32 x 640 452 -> 349, 8192 x 128 x 256 303 -> 266; both gradients alone 4600 x 16 x 4096
+//                           200 -> 180, 8192 x 16 x 2048 163 -> 167, but 4600 x 8 x 4096 113 -> 137, 8192 x 8 x 4096 181 -> 245
+//   more than half a round  16384 x 48 x 256 282 -> 245, 4600 x 48 x 256 136 -> 132, 8192 x 32 x 448 186 -> 179, 16384 x 32 x 512 275 -> 249, 4600 x 64 x 256 149 -> 150,
+//                           4600 x 32 x 512 160 -> 163, 16384 x 12 x 768 312 -> 294, 4600 x 16 x 768 142 -> 141; but 3000 x 16 x 1024 124 -> 130, 16384 x 16 x 1024 369 -> 382
+//   half a round or less    8192 x 32 x 256 146 -> 132, 16384 x 8 x 1024 350 -> 330, 16384 x 4 x 1024 336 -> 293; but both gradients alone 8192 x 4 x 2048 78 -> 89,
+//                           16384 x 1 x 4096 161 -> 224
+// With 512 rows lffn_lookup_scatter_f32 has only atomics (both gradients of 16384 x 32 x 256 1785 -> 124), and columns that are no multiple of 64 it does not take.
 extern "C" int lffn_lookup_scatter_plan(int64_t B, int64_t T, int64_t S, int64_t Do, int32_t *sorted) {
     LFFN_REQUIRE(sorted, LFFN_ERR_BAD_ARG);
     const double work = double(B) * double(T) * double(Do);
@@ -782,7 +783,8 @@ extern "C" int lffn_lookup_scatter_plan(int64_t B, int64_t T, int64_t S, int64_t
     if (work >= LFFN_SCATTER_DOUBLE_WORK) {
         *sorted = 1;
     } else if (B <= CHUNK) {
-        const int64_t workgroups = T * (Do / 64), most_columns = workgroups > COMPUTE_UNITS || workgroups <= COMPUTE_UNITS / 2 ? 128 * T : B >= 12000 ? 48 * T : 0;
+        const int64_t workgroups = T * (Do / 64);
+        const int64_t most_columns = workgroups > COMPUTE_UNITS ? 256 * T : workgroups > COMPUTE_UNITS / 2 ? 768 : 1024;
         *sorted = S > 256 || Do % 64 != 0 || Do <= most_columns ? 1 : 0;
     }
     return LFFN_OK;

@@ -245,18 +245,16 @@ def test_which_calls_the_sorted_scatter_serves():
         assert ops.lookup_backward_is_fused(B, T, S, Do) == (n.value == 1 and Do % 64 == 0)
         return n.value
 
-    # from 45e6 products and 2049 tokens on where the form in LDS takes more than a round of 256 workgroups, or half a one
-    assert plan(2049, 128, 256, 512) == plan(3000, 128, 256, 768) == plan(2049, 64, 256, 384) == plan(16384, 32, 256, 256) == 1
+    # from 45e6 products and 2049 tokens on
+    assert plan(2049, 128, 256, 512) == plan(3000, 128, 256, 768) == plan(2049, 64, 256, 384) == plan(16384, 32, 256, 256) == plan(4600, 64, 256, 256) == 1
     assert plan(2048, 128, 256, 512) == plan(4096, 32, 256, 256) == plan(2048, 512, 256, 1024) == 0
-    # a round nearly full is the other form's, up to some thousand tokens
-    assert plan(4600, 64, 256, 256) == plan(11999, 48, 256, 320) == 0 and plan(12000, 48, 256, 320) == plan(4600, 65, 256, 256) == 1
-    # few tables of many columns do not repay the copy of the gradient
-    assert plan(16384, 1, 256, 4096) == plan(16384, 4, 256, 4096) == plan(8192, 8, 256, 4096) == plan(16384, 16, 256, 1024) == 0
-    assert plan(16384, 16, 256, 512) == plan(16384, 16, 256, 768) == plan(16384, 24, 256, 768) == 1
+    # but few tables of many columns do not repay the copy of the gradient: where the form in LDS takes half a round of 256 workgroups, a whole one, more
+    assert plan(16384, 4, 256, 1024) == plan(16384, 8, 256, 1024) == plan(16384, 16, 256, 768) == plan(4600, 16, 256, 2048) == plan(4600, 16, 256, 4096) == 1
+    assert plan(16384, 4, 256, 1088) == plan(16384, 9, 256, 1024) == plan(16384, 16, 256, 832) == plan(4600, 15, 256, 4096) == plan(8192, 8, 256, 4096) == 0
     # from 4e8 products on always, below it only in one launch, where the sums are doubles
     assert plan(16385, 32, 256, 512) == 0 and plan(32768, 32, 256, 512) == plan(16384, 8, 256, 4096) == plan(32768, 128, 256, 512) == 1
     # what the other form has only atomics for, or does not take
-    assert plan(4600, 64, 512, 256) == plan(4600, 64, 256, 288) == 1 and plan(32768, 128, 1024, 512) == plan(32768, 128, 256, 520) == plan(0, 4, 16, 64) == 0
+    assert plan(16384, 4, 512, 1088) == plan(16384, 4, 256, 1056) == 1 and plan(32768, 128, 1024, 512) == plan(32768, 128, 256, 520) == plan(0, 4, 16, 64) == 0
     assert lib.lffn_lookup_scatter_plan(16, 4, 16, 64, None) == _lib.LFFN_ERR_BAD_ARG
 
     hdr = open(os.path.join(ROOT, "include", "lookupffn_hip.h")).read()

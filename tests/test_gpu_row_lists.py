@@ -123,7 +123,7 @@ def test_flat_rows_of_two_lists(B, I, rows, in_tables):
     assert ((out.cpu().double() - want).abs() <= _bound(want, scale, n, B * I, False)).all()
 
 
-@pytest.mark.parametrize("B,T,Do", [(2049, 64, 384), (3001, 33, 512), (8193, 32, 256), (16384, 33, 128)])
+@pytest.mark.parametrize("B,T,Do", [(2049, 64, 384), (3001, 32, 512), (8193, 32, 256), (16384, 33, 128)])
 def test_calls_that_had_double_sums_keep_them(B, T, Do):
     """Rounded once, a number is off by 2^-24 / 3^0.5 of its power of two, root mean square; the rows cut by pieces a few roundings more."""
     assert ops.lookup_backward_is_fused(B, T, 256, Do) and B * T * Do < ops.DOUBLE_SCATTER_WORK
