@@ -724,9 +724,9 @@ int lffn_lookup_scatter_f32(const int32_t *code, const float *score, const float
  * the inputs are transposed / copied slice-major, each table's tokens are sorted by code
  * (stable counting sort, (token, score) pairs), and a
  * last kernel walks the sorted lists and adds the rows of g in registers; rows of
- * grad_tables are written with plain stores and the order of additions is fixed (token order
- * inside a code), so results are reproducible from run to run, unlike the reference's
- * atomics.  With accumulate != 0, rows that no token points at are neither read nor written.
+ * grad_tables are written with plain stores and the order of additions is fixed (not token order: a
+ * row's sum is that of several partial sums of its tokens), so results are reproducible from run to
+ * run, unlike the reference's atomics.  With accumulate != 0, rows that no token points at are neither read nor written.
  * Tokens are taken 16384 at a time (the workspace is sized for one such chunk).
  * About twice as fast as lffn_lookup_scatter_f32 at 16384 tokens x 128 tables x 768
  * columns; which calls it is the faster one for, lffn_lookup_scatter_plan says.
@@ -754,7 +754,7 @@ int lffn_lookup_scatter_sorted_f32(const int32_t *code, const float *score, cons
  * chunk of 16384 tokens one kernel transposes code and score and copies g slice-major, and the
  * score-gradient kernel and the sorted scatter both read that copy (for the score gradient, a token
  * tile's slice of g is then contiguous instead of one 128-byte line per row).  Results are bit-identical
- * to the two separate calls.  grad_score or grad_tables may be NULL (that gradient is not computed; tables
+ * to the two separate calls (grad_score where both calls give every (token, table) one owner, see there).  grad_score or grad_tables may be NULL (that gradient is not computed; tables
  * is needed for the former only, score for the latter only).  Do % 64 == 0, S <= 512.
  * Replaces WeightedVectorGatherAdd.backward (PL/gather/cuda/kernel.py:190-202: indexed_inner_product +
  * weighted_vector_scatter_add, kernels gather_kernel_fp32.cu:49-157) with the index offset of
@@ -779,7 +779,8 @@ int lffn_lookup_backward_sums_rows(int64_t B, int64_t *rows);
  * in LDS.  At the layer's shapes (S = 256, T even, Do a multiple of 32, a few thousand
  * tokens or more) every (token, table) sum has one owner that walks the column slices
  * itself: no atomics, a fixed order of additions, results bit-identical from run to
- * run.  The other shapes (S < 256, odd T, small batches) combine the partial sums of
+ * run (not from one place in the batch to another: neighbouring tokens read the halves of
+ * a row in different orders).  The other shapes (S < 256, odd T, small batches) combine the partial sums of
  * the 64-column slices of a row with global atomics, in no fixed order (as the partial
  * sums of the reference's kernel are, PL/gather/cuda/extension/gather_kernel_fp32.cu:141).
  * Replaces WeightedVectorGatherAdd.backward's indexed_inner_product call

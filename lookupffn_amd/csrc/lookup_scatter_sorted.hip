@@ -45,8 +45,9 @@
 //     a piece boundary go to slots, and the wavefront in whose piece one ends adds its parts in order.  The sum order is fixed
 //     (run-to-run reproducible), and eight partial sums of a bucket (four lane groups, even and odd steps) keep its error where it was.
 // Eight wavefronts a workgroup, two of them a compute unit for their LDS; 12 or 16 wavefronts are slower (285, 310 us).  All launches,
-// before (padded lists of 16384 tokens, 32 columns, rows stored as they end) -> now, sums in fp32: 16384 x 128 x 768 331 -> 305 us, x 512 221 -> 204; 32768 x 128 x 512
-// 446 -> 413; 8192 x 128 x 768 194 -> 152; 4096 x 128 x 768 140 -> 95, x 512 92 -> 73; 16384 x 512 x 1024 1507 -> 1514.  What is left at 16384 x 128 x 768, taken
+// before (padded lists of 16384 tokens, 32 columns, rows stored as they end) -> now, sums in fp32, codes spread evenly, by Zipf's law in any order of the rows:
+// 16384 x 128 x 768 317 -> 294 us, 322 -> 299; x 512 223 -> 204, 229 -> 206; 32768 x 128 x 512 445 -> 413, 457 -> 420; 8192 x 256 x 768 336 -> 279, 348 -> 283;
+// 16384 x 512 x 1024 1532 -> 1524, 1545 -> 1529; of 512 rows 16384 x 128 x 768 348 -> 335, 369 -> 369; sums in doubles (in fp32 before) 4096 x 128 x 768 123 -> 95, 137 -> 97.  What is left at 16384 x 128 x 768, taken
 // apart: without bucket ends -12 us, with lists from the L2 -28, rows from the L1 -47, all three 228 of 285, of which 25 to 35 are starts and ends of workgroups in step
 // with each other.  Fetching the lists' lines or the next list's rows ahead through the scalar cache gives nothing, nor does a
 // workgroup that stays for several slices.
@@ -1112,10 +1113,11 @@ __global__ __launch_bounds__(256) void rows_place_kernel(RowsArgs a) {
 }
 
 // The rows' sums where rows have few pairs or none (SPARSE_PAIRS on average or fewer): a wavefront adds up a row at a time over
-// all its columns from g as it lies and writes it whole.  The slice-by-slice accumulation above reads every row's list once per 32
-// columns, which for rows of a few pairs is most of its time.  All five launches, 64 tokens: 128 tables of 768 columns 55 -> 29 us,
-// 512 of 1024 217 -> 125 us (537 MB written: 4.3 TB/s); 8 pairs a row, 2048 tokens of 128 x 512: 92 -> 60 us; 16 pairs a row 128 us
-// either way, hence the limit.  A row of more than LONG_ROW pairs goes to the whole workgroup; with half of all pairs on one row a single
+// all its columns from g as it lies and writes it whole.  The slice-by-slice accumulation above reads every row's list once per 64
+// columns and copies g first, which for rows of a few pairs is most of its time.  All five launches, us, by slices -> so, rows by chance: 2 pairs a row 128 x 512
+// 45 -> 30, 512 x 1024 218 -> 128 (537 MB written: 4.2 TB/s); 4 pairs 53 -> 38, 260 -> 185, 32 x 256 22 -> 22; 6 pairs 58 -> 46, 297 -> 298, 128 x 768 74 -> 66; 8 pairs 58 -> 51,
+// 303 -> 399, 75 -> 84, 26 -> 29; 16 pairs 75 -> 111, 449 -> 1006; by Zipf's law in any order of the rows 2 pairs 41 -> 41, 4 pairs 51 -> 56, 8 pairs 58 -> 81.  So the limit, set by a
+// slower form by slices (16 pairs of 128 x 512 128 us either way), is some two pairs too high but for tables of few columns.  A row of more than LONG_ROW pairs goes to the whole workgroup; with half of all pairs on one row a single
 // compute unit's reads of g bound it (512 tokens of 128 x 768: 516 us by slices, 1275 so, 3437 by fp32 atomics; with a tenth 288 and 1174).
 constexpr int64_t SPARSE_PAIRS = 8;
 constexpr int LONG_ROW = 32;
